@@ -519,6 +519,25 @@ int m40llm_ext_batched_gemm_residual_onto_zero_f32xf16_async(M40llmCudaContext* 
 int m40llm_ext_batched_norm_gemm_f32xf16_async(M40llmCudaContext* ctx, const void* d_x_f32, const void* d_norm_w,
                                                uint32_t norm_weight_dtype, float eps, const void* d_w_f16, void* d_out_f32,
                                                uint32_t rows, int N, int K);
+/* The four calls above for up to 32 rows (K a multiple of 256, operands 16-byte aligned, head_dim a multiple of 16; -6 otherwise): the
+ * weights are read once for all rows, one launch a call.  d_clear_f32 / clear_floats as in the ..._clear call.  The result of
+ * ..._onto_zero HOLDS ZEROS stored by an earlier call on the decode stream; where it overlaps an operand it is overwritten
+ * instead of added to (a residual may be the result itself, element by element). */
+int m40llm_ext_batched_wide_norm_qkv_rope_append_async(
+    M40llmCudaContext* ctx, M40llmKVCache* kv, const uint32_t* seq_ids_dev, const uint32_t* seq_lens_dev, uint32_t rows,
+    const void* d_x_f32, const void* d_norm_w, uint32_t norm_weight_dtype, float eps, const void* d_wq_f16,
+    const void* d_wk_f16, const void* d_wv_f16, const void* d_bq_f32, const void* d_bk_f32, const void* d_bv_f32,
+    uint32_t d_model, uint32_t q_heads, float freq_base, float freq_scale, uint32_t rope_layout, void* d_q_out_f32,
+    void* d_clear_f32, uint32_t clear_floats);
+int m40llm_ext_batched_wide_norm_gate_up_swiglu_async(M40llmCudaContext* ctx, const void* d_x_f32, const void* d_norm_w,
+                                                      uint32_t norm_weight_dtype, float eps, const void* d_wgate_f16,
+                                                      const void* d_wup_f16, void* d_hid_f32, uint32_t rows, int ffn, int d_model,
+                                                      void* d_clear_f32, uint32_t clear_floats);
+int m40llm_ext_batched_wide_gemm_residual_onto_zero_async(M40llmCudaContext* ctx, const void* d_a_f32, const void* d_w_f16,
+                                                          const void* d_residual_f32, void* d_out_f32, uint32_t rows, int N, int K);
+int m40llm_ext_batched_wide_norm_gemm_async(M40llmCudaContext* ctx, const void* d_x_f32, const void* d_norm_w,
+                                            uint32_t norm_weight_dtype, float eps, const void* d_w_f16, void* d_out_f32,
+                                            uint32_t rows, int N, int K);
 /*   per row: first index of the maximum of logits[row][n] and the top-1/top-2 gap -> ids_dev/gaps_dev[row][step of the
  *   row] (row stride = capacity); seq_lens_dev[row] += 1; embedding row of the pick -> d_x_out_f32[row].
  *   state_dev = {unused, capacity, step of row 0, step of row 1, ...} */

@@ -149,6 +149,18 @@ int m40_rows_mfma_qkv(M40llmCudaContext* ctx, hipStream_t stream, const M40llmKV
                       const uint16_t* wq, const uint16_t* wk, const uint16_t* wv, const float* bq, const float* bk,
                       const float* bv, uint32_t d_model, uint32_t q_heads, float rope_base, float rope_scale,
                       uint32_t rope_layout, float* q_out);
+// the projections for 9 to 32 rows, K a multiple of 256 (rows_wide_mfma.hip); zero: zero_count floats cleared on the side
+bool m40_rows_wide_supported(int rows, int K);
+int m40_rows_wide_qkv(M40llmCudaContext* ctx, hipStream_t stream, const M40llmKVCache* kv, const uint32_t* ids_dev, const uint32_t* lens_dev,
+                      uint32_t rows, const float* x, const void* norm_w, uint32_t norm_dtype, float eps, const uint16_t* wq, const uint16_t* wk,
+                      const uint16_t* wv, const float* bq, const float* bk, const float* bv, uint32_t d_model, uint32_t q_heads, float rope_base,
+                      float rope_scale, uint32_t rope_layout, float* q_out, float* zero, int zero_count);
+int m40_rows_wide_swiglu(M40llmCudaContext* ctx, hipStream_t stream, const float* x, const void* norm_w, uint32_t norm_dtype, float eps,
+                         const uint16_t* wgate, const uint16_t* wup, float* out, int rows, int ffn, int K, float* zero, int zero_count);
+int m40_rows_wide_norm(M40llmCudaContext* ctx, hipStream_t stream, const float* x, const void* norm_w, uint32_t norm_dtype, float eps,
+                       const uint16_t* W, float* out, int rows, int N, int K);
+int m40_rows_wide_residual(M40llmCudaContext* ctx, hipStream_t stream, const float* x, const uint16_t* W, const float* residual, float* out, int rows,
+                           int N, int K, bool onto_zero);
 // many-row f32 x f16 GEMM on 128 x 128 tiles (gemm_tiled.hip): M > 32, K a multiple of 32, 16-byte aligned operands
 bool m40_gemm_tiled_supported(const void* A, const void* B, int M, int N, int K);
 int m40_launch_gemm_tiled(M40llmCudaContext* ctx, hipStream_t stream, uint32_t stream_kind, const float* A, const uint16_t* B,

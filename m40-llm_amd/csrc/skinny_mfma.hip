@@ -780,6 +780,13 @@ int m40llm_ext_batched_norm_qkv_rope_append_async(
                                  static_cast<const float*>(d_bq_f32), static_cast<const float*>(d_bk_f32),
                                  static_cast<const float*>(d_bv_f32), d_model, q_heads, freq_base, freq_scale, rope_layout,
                                  static_cast<float*>(d_q_out_f32));
+    // nine rows and more: one launch as well, K in chunks
+    if (rows > 8 && kv->head_dim % 16 == 0 && m40_aligned16(d_x_f32) && m40_aligned16(d_norm_w))
+        return m40_rows_wide_qkv(ctx, ctx->decode_stream, kv, seq_ids_dev, seq_lens_dev, rows, static_cast<const float*>(d_x_f32), d_norm_w,
+                                 norm_weight_dtype, eps, static_cast<const uint16_t*>(d_wq_f16), static_cast<const uint16_t*>(d_wk_f16),
+                                 static_cast<const uint16_t*>(d_wv_f16), static_cast<const float*>(d_bq_f32),
+                                 static_cast<const float*>(d_bk_f32), static_cast<const float*>(d_bv_f32), d_model, q_heads, freq_base,
+                                 freq_scale, rope_layout, static_cast<float*>(d_q_out_f32), nullptr, 0);
     // up to eight rows and K <= 2048: vector-ALU kernel with the whole epilogue inside (one launch instead of two)
     if (m40_rows_gemv_supported((int)rows, (int)d_model) && m40_aligned16(d_x_f32) && m40_aligned16(d_norm_w))
         return m40_rows_norm_qkv(ctx, ctx->decode_stream, kv, seq_ids_dev, seq_lens_dev, rows, static_cast<const float*>(d_x_f32),
@@ -819,6 +826,9 @@ int m40llm_ext_batched_gemm_residual_f32xf16_async(M40llmCudaContext* ctx, const
         return m40_rows_gemv_residual(ctx->decode_stream, static_cast<const float*>(d_a_f32),
                                       static_cast<const uint16_t*>(d_w_f16), static_cast<const float*>(d_residual_f32),
                                       static_cast<float*>(d_out_f32), (int)rows, N, K);
+    if (rows > 8 && m40_aligned16(d_a_f32))
+        return m40_rows_wide_residual(ctx, ctx->decode_stream, static_cast<const float*>(d_a_f32), static_cast<const uint16_t*>(d_w_f16),
+                                      static_cast<const float*>(d_residual_f32), static_cast<float*>(d_out_f32), (int)rows, N, K, false);
     PackSpec pk{static_cast<const float*>(d_a_f32), nullptr, nullptr, 0, 0.0f};
     const void* W[1] = {d_w_f16};
     const int Ns[1] = {N};
@@ -845,6 +855,12 @@ int m40llm_ext_batched_gemm_residual_onto_zero_f32xf16_async(M40llmCudaContext* 
         return m40_rows_khalf_residual(ctx, ctx->decode_stream, static_cast<const float*>(d_a_f32),
                                        static_cast<const uint16_t*>(d_w_f16), static_cast<const float*>(d_residual_f32),
                                        static_cast<float*>(d_out_f32), (int)rows, N, K);
+    }
+    if (rows > 8 && rows <= 16 && m40_rows_wide_supported((int)rows, K) && m40_aligned16(d_a_f32) && m40_aligned16(d_w_f16) &&
+        apart(d_a_f32, (size_t)rows * K * 4) && apart(d_residual_f32, (size_t)rows * N * 4)) {
+        (void)hipGetLastError();
+        return m40_rows_wide_residual(ctx, ctx->decode_stream, static_cast<const float*>(d_a_f32), static_cast<const uint16_t*>(d_w_f16),
+                                      static_cast<const float*>(d_residual_f32), static_cast<float*>(d_out_f32), (int)rows, N, K, true);
     }
     // any other shape: the form that overwrites its result
     return m40llm_ext_batched_gemm_residual_f32xf16_async(ctx, d_a_f32, d_w_f16, d_residual_f32, d_out_f32, rows, N, K);
@@ -874,6 +890,11 @@ int m40llm_ext_batched_norm_gate_up_swiglu_clear_async(M40llmCudaContext* ctx, c
                                     eps, static_cast<const uint16_t*>(d_wgate_f16), static_cast<const uint16_t*>(d_wup_f16),
                                     static_cast<float*>(d_hid_f32), (int)rows, ffn, d_model,
                                     clear_floats ? static_cast<float*>(d_clear_f32) : nullptr, (int)clear_floats);
+    if (rows > 8 && m40_aligned16(d_x_f32) && m40_aligned16(d_norm_w))
+        return m40_rows_wide_swiglu(ctx, ctx->decode_stream, static_cast<const float*>(d_x_f32), d_norm_w, norm_weight_dtype, eps,
+                                    static_cast<const uint16_t*>(d_wgate_f16), static_cast<const uint16_t*>(d_wup_f16),
+                                    static_cast<float*>(d_hid_f32), (int)rows, ffn, d_model,
+                                    clear_floats ? static_cast<float*>(d_clear_f32) : nullptr, (int)clear_floats);
     if (clear_floats && m40_zero_f32(ctx->decode_stream, static_cast<float*>(d_clear_f32), clear_floats) != 0) return -7;
     PackSpec pk{static_cast<const float*>(d_x_f32), nullptr, d_norm_w, norm_weight_dtype, eps};
     const void* W[2] = {d_wgate_f16, d_wup_f16};
@@ -896,6 +917,9 @@ int m40llm_ext_batched_norm_gemm_f32xf16_async(M40llmCudaContext* ctx, const voi
     if (m40_rows_mfma_supported((int)rows, K) && m40_aligned16(d_x_f32) && m40_aligned16(d_norm_w))
         return m40_rows_mfma_plain(ctx, ctx->decode_stream, static_cast<const float*>(d_x_f32), d_norm_w, norm_weight_dtype, eps,
                                    static_cast<const uint16_t*>(d_w_f16), static_cast<float*>(d_out_f32), (int)rows, N, K);
+    if (rows > 8 && m40_aligned16(d_x_f32) && m40_aligned16(d_norm_w))
+        return m40_rows_wide_norm(ctx, ctx->decode_stream, static_cast<const float*>(d_x_f32), d_norm_w, norm_weight_dtype, eps,
+                                  static_cast<const uint16_t*>(d_w_f16), static_cast<float*>(d_out_f32), (int)rows, N, K);
     PackSpec pk{static_cast<const float*>(d_x_f32), nullptr, d_norm_w, norm_weight_dtype, eps};
     const void* W[1] = {d_w_f16};
     const int Ns[1] = {N};

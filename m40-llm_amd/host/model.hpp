@@ -618,17 +618,36 @@ public:
         M40H_TRY(m40llm_memcpy_d2h(ctx_, host_logits, ws_.logits.ptr(), (size_t)rows * cfg_.vocab * 4));
     }
 
-    // ---- device-driven row-batched greedy loop (modes 1 and 2; rows <= 16, dense cache) -------------------------
+    // ---- device-driven row-batched greedy loop (modes 1 and 2; dense cache) -------------------------------------
     // Per step: every layer as five fused calls on the decode stream, output norm + lm_head, then the greedy pick,
-    // the length increment and the next embedding on the device.  Nothing is read back until the end.
+    // the length increment and the next embedding on the device.  Nothing is read back until the end.  More rows than the
+    // fused calls take go through the layers in equal groups.
+    static constexpr uint32_t kFusedRows = 32, kNarrowRows = 8;   // rows of one fused call; of the calls made for few rows
+    static uint32_t fused_group(uint32_t rows) {
+        const uint32_t groups = (rows + kFusedRows - 1) / kFusedRows;
+        return (rows + groups - 1) / groups;
+    }
     bool batched_fused_available(uint32_t rows) const {
-        return !kvcfg_.is_enabled() && rows >= 1 && rows <= 16 && cfg_.d_model % 256 == 0 && cfg_.ffn % 256 == 0 &&
+        return !kvcfg_.is_enabled() && rows >= 1 && cfg_.d_model % 256 == 0 && cfg_.ffn % 256 == 0 &&
                (cfg_.head_dim == 64 || cfg_.head_dim == 128);   // the lengths-on-device attention serves these two
     }
     void batched_layer_fused(uint32_t l, const uint32_t* slots_dev, const uint32_t* lens_dev, uint32_t rows, uint32_t hint,
                              const float* d_x, float* d_out) {
         const LayerWeights& w = layers_[l];
         const uint32_t D = cfg_.d_model, F = cfg_.ffn;
+        if (rows > kNarrowRows) {
+            // x1 and d_out are dead until the O and the down projection write them: the launches before clear them on the side
+            M40H_TRY(m40llm_ext_batched_wide_norm_qkv_rope_append_async(ctx_, kv_, slots_dev, lens_dev, rows, d_x, w.attn_norm, cfg_.norm_weight_dtype,
+                                                                        cfg_.rms_eps, w.wq, w.wk, w.wv, w.bq, w.bk, w.bv, D, cfg_.q_heads, cfg_.rope_base,
+                                                                        cfg_.rope_scale, cfg_.rope_layout, ws_.q.ptr(), ws_.x1.ptr(), rows * D));
+            M40H_TRY(m40llm_ext_attention_last_token_f32_gqa_batched_lens_dev_async(ctx_, kv_, slots_dev, lens_dev, 1, rows, hint, ws_.q.ptr(),
+                                                                                    cfg_.q_heads, ws_.ctx_out.ptr()));
+            M40H_TRY(m40llm_ext_batched_wide_gemm_residual_onto_zero_async(ctx_, ws_.ctx_out.ptr(), w.wo, d_x, ws_.x1.ptr(), rows, (int)D, (int)D));
+            M40H_TRY(m40llm_ext_batched_wide_norm_gate_up_swiglu_async(ctx_, ws_.x1.ptr(), w.ffn_norm, cfg_.norm_weight_dtype, cfg_.rms_eps, w.wgate,
+                                                                       w.wup, ws_.hid.ptr(), rows, (int)F, (int)D, d_out, rows * D));
+            M40H_TRY(m40llm_ext_batched_wide_gemm_residual_onto_zero_async(ctx_, ws_.hid.ptr(), w.wdown, ws_.x1.ptr(), d_out, rows, (int)D, (int)F));
+            return;
+        }
         M40H_TRY(m40llm_ext_batched_norm_qkv_rope_append_async(ctx_, kv_, slots_dev, lens_dev, rows, d_x, w.attn_norm,
                                                                cfg_.norm_weight_dtype, cfg_.rms_eps, w.wq, w.wk, w.wv, w.bq, w.bk,
                                                                w.bv, D, cfg_.q_heads, cfg_.rope_base, cfg_.rope_scale,
@@ -644,17 +663,29 @@ public:
         M40H_TRY(m40llm_ext_batched_gemm_residual_onto_zero_f32xf16_async(ctx_, ws_.hid.ptr(), w.wdown, ws_.x1.ptr(), d_out, rows,
                                                                           (int)D, (int)F));
     }
+    // output norm + lm_head of a group of rows
+    void batched_logits_fused(const float* d_x, uint32_t rows, float* d_logits) {
+        if (rows > kNarrowRows)
+            M40H_TRY(m40llm_ext_batched_wide_norm_gemm_async(ctx_, d_x, out_norm_, cfg_.norm_weight_dtype, cfg_.rms_eps, lm_head_, d_logits, rows,
+                                                             (int)cfg_.vocab, (int)cfg_.d_model));
+        else
+            M40H_TRY(m40llm_ext_batched_norm_gemm_f32xf16_async(ctx_, d_x, out_norm_, cfg_.norm_weight_dtype, cfg_.rms_eps, lm_head_, d_logits, rows,
+                                                                (int)cfg_.vocab, (int)cfg_.d_model));
+    }
     void enqueue_batched_step(uint32_t rows, uint32_t hint, float* hidden, float* other) {
         const uint32_t* slots = static_cast<const uint32_t*>(bslots_.ptr());
         uint32_t* lens = static_cast<uint32_t*>(blens_.ptr());
-        float* a = hidden;
-        float* b = other;
-        for (uint32_t l = 0; l < cfg_.n_layers; ++l) {
-            batched_layer_fused(l, slots + (size_t)l * rows, lens, rows, hint, a, b);
-            std::swap(a, b);
+        const uint32_t group = fused_group(rows);
+        for (uint32_t r0 = 0; r0 < rows; r0 += group) {
+            const uint32_t n = rows - r0 < group ? rows - r0 : group;
+            float* a = hidden + (size_t)r0 * cfg_.d_model;
+            float* b = other + (size_t)r0 * cfg_.d_model;
+            for (uint32_t l = 0; l < cfg_.n_layers; ++l) {
+                batched_layer_fused(l, slots + (size_t)l * rows + r0, lens + r0, n, hint, a, b);
+                std::swap(a, b);
+            }
+            batched_logits_fused(a, n, ws_.logits.f32((size_t)r0 * cfg_.vocab));
         }
-        M40H_TRY(m40llm_ext_batched_norm_gemm_f32xf16_async(ctx_, a, out_norm_, cfg_.norm_weight_dtype, cfg_.rms_eps, lm_head_,
-                                                            ws_.logits.ptr(), rows, (int)cfg_.vocab, (int)cfg_.d_model));
         M40H_TRY(m40llm_ext_batched_greedy_step_async(ctx_, ws_.logits.ptr(), rows, cfg_.vocab,
                                                       static_cast<uint32_t*>(bstate_.ptr()), lens,
                                                       static_cast<uint32_t*>(bids_.ptr()), static_cast<float*>(bgaps_.ptr()),
@@ -663,7 +694,7 @@ public:
     // One decode step for `rows` sequences (token r at position kv_lens[r] of sequence seq_ids[r]) with the logits of
     // every row brought to the host: what a serving loop that samples on the host needs per tick
     // (forward_one_token_all_layers_batched_for_sequences + logits_after_batched_forward, src/server.rs:664-711).
-    // Fused kernels in groups of up to 16 rows when the host mode allows them, the reference's sequence otherwise.
+    // Fused kernels in groups of up to 32 rows when the host mode allows them, the reference's sequence otherwise.
     // greedy / picks / picked (all null, or all given): rows marked greedy get their token picked on the device (first
     // index of the maximum, as a top_k = 1 sampler picks) when the top-1 / top-2 logit gap clears the tie guard; such
     // rows set picked[r] = 1 and their logits are not copied.  Every other row receives its logits.
@@ -687,13 +718,14 @@ public:
             }
             return;
         }
-        if (!(mode_ >= 1 && batched_fused_available(rows < 16 ? rows : 16))) {
+        if (!(mode_ >= 1 && batched_fused_available(rows))) {
             const float* hidden = forward_batched(seq_ids, kv_lens, tokens, rows);
             logits_from_hidden_rows(hidden, rows, host_logits);
             return;
         }
-        for (uint32_t r0 = 0; r0 < rows; r0 += 16) {
-            const uint32_t n = rows - r0 < 16 ? rows - r0 : 16;
+        const uint32_t group = fused_group(rows);
+        for (uint32_t r0 = 0; r0 < rows; r0 += group) {
+            const uint32_t n = rows - r0 < group ? rows - r0 : group;
             ensure_workspace(n);
             std::vector<uint32_t> table((size_t)cfg_.n_layers * n + 2 * n);   // slots per layer, then lengths, then tokens
             uint32_t longest = 0;
@@ -721,8 +753,7 @@ public:
                 batched_layer_fused(l, slots + (size_t)l * n, lens, n, hint, a, b);
                 std::swap(a, b);
             }
-            M40H_TRY(m40llm_ext_batched_norm_gemm_f32xf16_async(ctx_, a, out_norm_, cfg_.norm_weight_dtype, cfg_.rms_eps, lm_head_,
-                                                                ws_.logits.ptr(), n, (int)cfg_.vocab, (int)cfg_.d_model));
+            batched_logits_fused(a, n, ws_.logits.f32());
             bool any_greedy = false;
             for (uint32_t r = 0; r < n && greedy && picks && picked; ++r) any_greedy = any_greedy || greedy[r0 + r];
             std::vector<uint32_t> idx(n);
