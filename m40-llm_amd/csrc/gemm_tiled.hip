@@ -2,20 +2,14 @@
 // matrix cores.  Same contract as the reference's gemm_f32xf16_gguf_f32 (cuda/kernels.cu:5037-5052); used when M is
 // beyond what the skinny kernels serve in one pass, where they would stream the weights once per 16 rows.
 //
-// Tiling: a workgroup of 4 waves owns a 128 x 128 tile of C and walks K in steps of 32.  Per step the 128 x 32 block
-// of A, split into an f16 high part and an f16 low part under a per-row power-of-two scale (a = scale (hi + lo) up to
-// 2^-22 relative; the scale multiplies the row of C at the end), is written to
-// LDS with the 128 x 32 block of B; each wave then computes its 64 x 64 quarter with
-// v_mfma_f32_16x16x32_f16, once with the high and once with the low part, so the products carry the f32 activations'
-// precision.  The global loads of the next three steps are in flight (three rotating register sets) while a step
-// computes from one LDS buffer and the following step's data moves into the other: one barrier per step.
-//
-// Larger grids (from 9/16 of a 128 x 256 tile per CU) take a second kernel built the same way round a wider tile and the
-// direct global-to-LDS loads of gfx950 (gemm_tiled_wide_kernel, below): what bounded the 128 x 128 kernel was not
-// arithmetic but the issue of its memory instructions, all of them between the barrier and the first matrix instruction.
+// Tiling: a workgroup of 4 waves owns a tile of C and walks K in steps of 32.  The rows of A are split into an f16 high part and an f16
+// low part under a per-row power-of-two scale (a = scale (hi + lo) up to 2^-22 relative; the scale multiplies the row of C at the end);
+// v_mfma_f32_16x16x32_f16 runs once with the high and once with the low part, so the products carry the f32 activations' precision.
+// Four tile shapes, from 128 x 256 (most products per byte of LDS traffic) to 64 x 64 (most workgroups for few rows), and parts of K where
+// even those leave CUs idle; pick_tile() weighs them.
 //
 // The split is done once per call by a packing pass (A -> two f16 planes in a per-stream buffer that grows on
-// demand), so the 128 x 128 tiles along N do not each repeat it.  When the buffer cannot be grown (the stream is being
+// demand), so the tiles along N do not each repeat it.  When the buffer cannot be grown (the stream is being
 // captured) the launch is declined and the caller falls back to the skinny kernels.  Several weight matrices that
 // share A (Q/K/V, gate/up) can be served by one packing pass and one launch.
 #include "common.hpp"
@@ -27,12 +21,7 @@ namespace {
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-
-constexpr int kBM = 128, kBN = 128, kBK = 32;
-constexpr int kStride = kBK;                     // halves per LDS row: 64 B, no padding; 16-byte chunks are swizzled (below)
-constexpr int kTileHalves = kBM * kStride;       // one 128 x 32 operand block
-constexpr int kBufHalves = 3 * kTileHalves;      // A high, A low, B
+constexpr int kBK = 32;
 constexpr int kThreads = 256;
 constexpr int kMaxMats = 3;
 
@@ -57,10 +46,6 @@ struct PackSource {
     float eps;
 };
 enum { kPackPlain = 0, kPackNorm = 1, kPackSwiglu = 2 };
-
-struct StepRegs {   // one K step of one thread: rows lrow and lrow + 64, 16 bytes (8 halves) of each
-    uint4 ah[2], al[2], b[2];
-};
 
 // A [M][K] f32 -> hi, lo [M][K] f16 planes and one scale per row: a = scale * (hi + lo) up to 2^-22 relative.  The scale is
 // the power of two that brings the row's largest magnitude into [2^10, 2^11) -- any finite f32 row fits the f16 planes,
@@ -214,172 +199,269 @@ __global__ __launch_bounds__(256) void pack_hilo_planes_kernel(PackSource src_ar
     }
 }
 
-__global__ __launch_bounds__(kThreads, 2) void gemm_tiled_f32xf16_gguf_kernel(const _Float16* __restrict__ A_hi,
-                                                                              const _Float16* __restrict__ A_lo,
-                                                                              const float* __restrict__ row_scale,
-                                                                              TiledMats mats, int M, int K, int k_splits) {
-    extern __shared__ __align__(16) _Float16 lds[];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int tiles_n = mats.tile_start[mats.n];
-    // Workgroups are dealt to the eight dies in turn.  Renumbered so that each die owns a contiguous band of tile
-    // rows: its L2 then holds one eighth of A (and streams B) instead of every die reading all of A.
-    const int per_die = (int)gridDim.x / 8;
+// ---- tiles of 32 MT x 32 NT per workgroup of four waves (2 x 2, wave tile 16 MT x 16 NT) -----------------------------------
+//
+// Measured on a 128 x 128 kernel that staged through registers with parts of it switched off (M 4096, N 2048, K 2048): arithmetic alone
+// 46 us, loads + LDS traffic + barriers alone 45 us, everything 87 us -- the two did not overlap.  A wave issues in order, and a
+// memory instruction holds the issue slot until its unit accepts it; with the four waves of a CU in step behind the
+// barrier, sixteen fragment reads, eight LDS writes and eight global loads each queue for ~500 cycles before the first
+// matrix instruction of the step can go.  Here:
+//  * every memory instruction of a step is issued under the step's matrix instructions (sched_group_barrier), so it waits for its unit
+//    while the matrix pipe works;
+//  * the fragments of step s + 1 are read from LDS during the arithmetic of step s (two fragment sets in registers);
+//  * global data goes straight into LDS (global_load_lds_dwordx4: no registers, no LDS write instruction, no wait
+//    before one), kBufs buffers deep -- a lane fetches the 16-byte chunk that belongs at its place in the swizzled
+//    row layout, so a wave's instruction fills one contiguous kilobyte; the workgroup waits only for the step after
+//    next (vmcnt) ahead of the barrier that publishes it;
+//  * in the 128 x 256 tile the wave tile is 64 x 128: per matrix instruction two thirds of the fragment bytes of a 64 x 64 tile (the
+//    activation rows, read twice -- high and low part -- are the short side).
+// M 4096, N 2048, K 2048: 79 (128 x 128, through registers) -> 63 us; N 11264: 479 -> 338 us; K 5632: 232 -> 155 us.  Under this load the part lowers
+// its clock (1.4-1.9 GHz measured inside the kernel, against 2.0-2.2 GHz in short or memory-bound launches), and a form
+// with fewer issue cycles (32 x 32 x 16 instructions: 1370 instead of 1500 cycles per step) ran at a lower clock
+// still and took the same time: what is left is energy per product, of which the exact hi + lo split is half.
+struct TileWalk {          // which tile (and part of K) a workgroup owns
+    int m0, n0, mat, split;
+};
+// Workgroups are dealt to the eight dies in turn.  Each die gets a contiguous run of tiles, walked in blocks of `band` tile rows, column
+// after column: what runs on a die at one time is then a roughly square block of tiles, which shares the steps of both operands in its L2.
+__device__ __forceinline__ TileWalk tile_walk(const TiledMats& mats, int tiles_m, int k_splits, int band, int bm, int bn) {
+    const int tiles_n = mats.tile_start[mats.n], per_die = (int)gridDim.x / 8;
     int logical = (int)blockIdx.x < per_die * 8 ? ((int)blockIdx.x % 8) * per_die + (int)blockIdx.x / 8 : (int)blockIdx.x;
-    // K split (few tiles, long K): split s of a tile walks its share of the K steps and writes its partial sums to
-    // plane s of the output buffer (a reduction launch adds the planes in order)
-    const int tiles_all = (int)gridDim.x / k_splits;
-    const int split = logical / tiles_all;
-    logical -= split * tiles_all;
-    const int tile_m = logical / tiles_n;
-    int tile_n = logical % tiles_n;
-    int mat = 0;
+    TileWalk w;
+    w.split = logical / (tiles_m * tiles_n);
+    logical -= w.split * tiles_m * tiles_n;
+    const int group = logical / (band * tiles_n), in_group = logical - group * band * tiles_n;
+    const int rows = tiles_m - group * band < band ? tiles_m - group * band : band;
+    w.m0 = (group * band + in_group % rows) * bm;
+    int tile_n = in_group / rows;
+    w.mat = 0;
 #pragma unroll
     for (int i = 1; i < kMaxMats; ++i)
-        if (i < mats.n && tile_n >= mats.tile_start[i]) mat = i;
-    tile_n -= mats.tile_start[mat];
-    const uint16_t* __restrict__ B = mats.B[mat];
-    float* __restrict__ C = mats.C[mat];
-    const int N = mats.N[mat];
-    const int m0 = tile_m * kBM, n0 = tile_n * kBN;
-    // loader role: four lanes cover the 64 bytes one row contributes to a step, so a wave's load instruction touches
-    // 16 rows (16 cache lines) instead of 32; each thread serves rows lrow and lrow + 64
-    const int lrow = tid >> 2, lchunk = tid & 3;
-    size_t a_off[2], b_off[2];
+        if (i < mats.n && tile_n >= mats.tile_start[i]) w.mat = i;
+    w.n0 = (tile_n - mats.tile_start[w.mat]) * bn;
+    return w;
+}
+
+// s_waitcnt for vector-memory operations only: at most n of them may still be outstanding
+__device__ __forceinline__ constexpr int vmcnt_only(int n) { return 0x0f70 | (n & 15) | ((n >> 4) << 14); }
+
+template <int... I, class F>
+__device__ __forceinline__ void tiled_unrolled(std::integer_sequence<int, I...>, F&& f) { (f(std::integral_constant<int, I>{}), ...); }
+
+// KS: k steps of 32 a stage (what is loaded together, between two barriers); kBufs: LDS buffers of a stage each (one
+// workgroup is resident per CU).  Two steps a stage read whole 128-byte lines of a column: with weights that no cache holds 64 x 64 tiles of N 2048,
+// K 2048 take 15.5 us that way and 21.3 us in stages of one step, 64 x 128 tiles 21.0 and 24.6 us (60 rows).
+template <int MT, int NT, int KS, int kBufs>
+__global__ __launch_bounds__(kThreads, 1) void gemm_tiled_kernel(const _Float16* __restrict__ A_hi, const _Float16* __restrict__ A_lo,
+                                                                      const float* __restrict__ row_scale, TiledMats mats, int M, int K,
+                                                                      int k_splits, int band) {
+    typedef __attribute__((address_space(3))) void* lds_dst_t;
+    typedef const __attribute__((address_space(1))) void* global_src_t;
+    constexpr int BM = 32 * MT, BN = 32 * NT;
+    constexpr int kRow = 64 * KS, kLoadRows = kThreads / (4 * KS);           // bytes of a row in a stage; rows the workgroup loads at a time
+    constexpr int kPlane = BM * kRow, kBuf = 2 * kPlane + BN * kRow;         // bytes of a stage: A high, A low, B
+    constexpr int AL = BM / kLoadRows, BL = BN / kLoadRows, kLoads = 2 * AL + BL;      // 16-byte loads per thread: rows lrow + kLoadRows i
+    extern __shared__ __align__(16) uint8_t tile_lds[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    TileWalk at = tile_walk(mats, (M + BM - 1) / BM, k_splits, band, BM, BN);
+    at.m0 = __builtin_amdgcn_readfirstlane(at.m0); at.n0 = __builtin_amdgcn_readfirstlane(at.n0);      // the same in every lane: divisions leave them in vector registers
+    at.mat = __builtin_amdgcn_readfirstlane(at.mat); at.split = __builtin_amdgcn_readfirstlane(at.split);
+    const uint16_t* __restrict__ B = mats.B[at.mat];
+    const int N = mats.N[at.mat], m0 = at.m0, n0 = at.n0;
+    // loader: thread -> row lrow (+ kLoadRows i) of a plane and a 16-byte place in that row's bytes, which holds the row's chunk of that number
+    // xor-ed with bits of the row: the fragment reads of rows that share banks fall into different ones
+    auto swizzle = [](int row) { return KS == 1 ? (row >> 2) & 3 : row & 7; };
+    const int lrow = tid / (4 * KS), gchunk = tid % (4 * KS) ^ swizzle(lrow);
+    const int stages_all = K / (kBK * KS), per_split = __builtin_amdgcn_readfirstlane((stages_all + k_splits - 1) / k_splits), stage0 = at.split * per_split;
+    const int stages = stage0 + per_split <= stages_all ? per_split : stages_all - stage0;     // >= 1 by the host's choice of k_splits
+    // a scalar address that walks K, and per lane a 32-bit offset from it that does not change
+    const uint8_t* hi_base = reinterpret_cast<const uint8_t*>(A_hi + (size_t)m0 * K + (size_t)stage0 * (kBK * KS));
+    const uint8_t* lo_base = reinterpret_cast<const uint8_t*>(A_lo + (size_t)m0 * K + (size_t)stage0 * (kBK * KS));
+    const uint8_t* b_base = reinterpret_cast<const uint8_t*>(B + (size_t)n0 * K + (size_t)stage0 * (kBK * KS));
+    uint32_t a_off[AL], b_off[BL];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int ar = m0 + lrow + 64 * i < M ? m0 + lrow + 64 * i : M - 1;   // clamped: computed, never stored
-        const int bc = n0 + lrow + 64 * i < N ? n0 + lrow + 64 * i : N - 1;
-        a_off[i] = (size_t)ar * K + lchunk * 8;
-        b_off[i] = (size_t)bc * K + lchunk * 8;
+    for (int i = 0; i < AL; ++i) {
+        const int r = lrow + kLoadRows * i;
+        a_off[i] = (uint32_t)(m0 + r < M ? r : M - 1 - m0) * (uint32_t)K * 2u + gchunk * 16u;     // clamped: computed, never stored
     }
-    const int steps_all = K / kBK, per_split = (steps_all + k_splits - 1) / k_splits;
-    const int step0 = split * per_split;
-    const int steps = step0 + per_split <= steps_all ? per_split : steps_all - step0;     // >= 1 by the host's choice of k_splits
-
-    auto issue = [&](StepRegs& r, int step) {
-        const size_t k = (size_t)(step0 + step) * kBK;
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            r.ah[i] = *reinterpret_cast<const uint4*>(A_hi + a_off[i] + k);
-            r.al[i] = *reinterpret_cast<const uint4*>(A_lo + a_off[i] + k);
-            r.b[i] = *reinterpret_cast<const uint4*>(B + b_off[i] + k);
+    for (int i = 0; i < BL; ++i) {
+        const int c = lrow + kLoadRows * i;
+        b_off[i] = (uint32_t)(n0 + c < N ? c : N - 1 - n0) * (uint32_t)K * 2u + gchunk * 16u;
+    }
+    // one instruction of a wave fills a contiguous kilobyte of a plane, lane by lane
+    auto issue = [&](int buf, int stage) __attribute__((always_inline)) {
+        int k = (stage < stages ? stage : stages - 1) * kRow;          // past the end: the last stage again (no branch around loads)
+        asm("" : "+s"(k));                                                      // keeps it out of the lanes' addresses
+        uint8_t* dst = tile_lds + buf * kBuf + wave * 1024;
+#pragma unroll
+        for (int i = 0; i < AL; ++i) {
+            __builtin_amdgcn_global_load_lds((global_src_t)(hi_base + k + a_off[i]), (lds_dst_t)(dst + i * 4096), 16, 0, 0);
+            __builtin_amdgcn_global_load_lds((global_src_t)(lo_base + k + a_off[i]), (lds_dst_t)(dst + kPlane + i * 4096), 16, 0, 0);
+        }
+#pragma unroll
+        for (int i = 0; i < BL; ++i)
+            __builtin_amdgcn_global_load_lds((global_src_t)(b_base + k + b_off[i]), (lds_dst_t)(dst + 2 * kPlane + i * 4096), 16, 0, 0);
+    };
+    const int wm = wave >> 1, wn = wave & 1, frag_row = lane & 15;
+    float scale[MT];                   // of the rows this lane will store, requested ahead of everything else
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+        const int row = m0 + (wm * MT + mt) * 16 + frag_row;
+        scale[mt] = row_scale[row < M ? row : M - 1];
+    }
+    struct Frags { half8 hi[MT], lo[MT], b[NT]; } f[2];
+    auto read_frags = [&](Frags& f, int buf, auto sub_c) __attribute__((always_inline)) {
+        const uint8_t* base = tile_lds + buf * kBuf + frag_row * kRow + (((lane >> 4) + 4 * decltype(sub_c)::value) ^ swizzle(frag_row)) * 16;
+        const uint8_t* a = base + wm * MT * 16 * kRow;
+        const uint8_t* b = base + 2 * kPlane + wn * NT * 16 * kRow;
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+            f.hi[mt] = *reinterpret_cast<const half8*>(a + mt * 16 * kRow);
+            f.lo[mt] = *reinterpret_cast<const half8*>(a + kPlane + mt * 16 * kRow);
+        }
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) f.b[nt] = *reinterpret_cast<const half8*>(b + nt * 16 * kRow);
+    };
+    floatx4 acc[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+    // Per accumulator step by step, high part then low part: the two large tiles give the same bits.  The weights are the instruction's first
+    // operand, so a lane's four sums are four neighbouring columns of one row and a store is 16 bytes.
+    auto compute = [&](const Frags& f) __attribute__((always_inline)) {
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(f.b[nt], f.hi[mt], acc[mt][nt], 0, 0, 0);
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(f.b[nt], f.lo[mt], acc[mt][nt], 0, 0, 0);
         }
     };
-    // LDS rows are 64 bytes = four 16-byte chunks; chunk c of row r is stored at position c ^ ((r / 4) % 4), so that
-    // the 16-byte fragment reads of rows r and r + 4 (same banks without the swizzle) fall into different banks, with
-    // no padding: 48 KB per workgroup
-    auto to_lds = [&](const StepRegs& r, int buf) {
-        _Float16* base = lds + buf * kBufHalves + lrow * kStride + ((lchunk ^ ((lrow >> 2) & 3)) * 8);
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            _Float16* p = base + i * 64 * kStride;
-            *reinterpret_cast<u32x4*>(p) = u32x4{r.ah[i].x, r.ah[i].y, r.ah[i].z, r.ah[i].w};
-            *reinterpret_cast<u32x4*>(p + kTileHalves) = u32x4{r.al[i].x, r.al[i].y, r.al[i].z, r.al[i].w};
-            *reinterpret_cast<u32x4*>(p + 2 * kTileHalves) = u32x4{r.b[i].x, r.b[i].y, r.b[i].z, r.b[i].w};
-        }
+    // The barriers are bare s_barrier instructions with the vector-memory wait written out: __syncthreads() would wait for every
+    // outstanding load (its fence covers LDS).
+    auto wait_and_meet = [&](auto n) __attribute__((always_inline)) {
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_waitcnt(vmcnt_only(decltype(n)::value));
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
     };
-
-    floatx4 acc[4][4];
+    constexpr int kInFlight = (kBufs - 3) * kLoads;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < kBufs - 1; ++i) issue(i, i);
+    wait_and_meet(std::integral_constant<int, kInFlight>());               // stages 0 and 1 have landed
+    read_frags(f[0], 0, std::integral_constant<int, 0>());
+    // Step u of a stage: the next step's fragments are read (the next stage's first ones behind its last step: buffer s + 1 is complete and
+    // visible), then its products.  Stage s refills the buffer of stage s - 1 -- whose fragments every wave had in registers before
+    // the last barrier -- with stage s + kBufs - 1, and ends with stage s + 2 landed.  ph: the stage's number in a period, after which buffers
+    // and fragment sets are back in their order: written out so that their addresses are constants and sums stay in their registers (a loop of
+    // two stages moved 200 accumulation registers a turn: 169 against 161 us at M 4096, N 2048, K 5632).
+    constexpr int kPeriod = KS == 2 || kBufs % 2 == 0 ? kBufs : 2 * kBufs;
+    auto sub_step = [&](auto ph_c, auto sub_c, int s) __attribute__((always_inline)) {
+        constexpr int ph = decltype(ph_c)::value, sub = decltype(sub_c)::value, buf = ph % kBufs, set = (ph * KS + sub) & 1;
+        read_frags(f[set ^ 1], sub + 1 < KS ? buf : (buf + 1) % kBufs, std::integral_constant<int, (sub + 1) % KS>());
+        if constexpr (sub == 0) issue((buf + kBufs - 1) % kBufs, s + kBufs - 1);
+        compute(f[set]);
+        constexpr int kReads = 2 * MT + NT, kProducts = 2 * MT * NT, kPerRead = NT == 8 ? 2 : 1;
+        constexpr int kPerLoad = (kProducts - kPerRead * kReads) / kLoads > 0 ? (kProducts - kPerRead * kReads) / kLoads : 1;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-
-    const int wm = wave >> 1, wn = wave & 1;
-    // the scales of the rows this lane will store, requested now: at the end they would be 16 dependent round trips
-    // (a load behind a store to memory it might alias waits for the store)
-    float sc_all[4][4];
-#pragma unroll
-    for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int row = m0 + wm * 64 + mt * 16 + (lane >> 4) * 4 + r;
-            sc_all[mt][r] = row_scale[row < M ? row : M - 1];
+        for (int i = 0; i < kReads; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x008, kPerRead, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
         }
-    const int frag_row = lane & 15, frag_k = ((lane >> 4) ^ ((frag_row >> 2) & 3)) * 8;   // swizzled chunk of this lane's k group
-    auto compute = [&](int buf) {
-        const _Float16* base = lds + buf * kBufHalves;
-        const _Float16* ah = base + (wm * 64 + frag_row) * kStride + frag_k;
-        const _Float16* bb = base + 2 * kTileHalves + (wn * 64 + frag_row) * kStride + frag_k;
-        half8 bf[4];
+        if constexpr (sub == 0) {
 #pragma unroll
-        for (int nt = 0; nt < 4; ++nt) bf[nt] = *reinterpret_cast<const half8*>(bb + nt * 16 * kStride);
-#pragma unroll
-        for (int mt = 0; mt < 4; ++mt) {
-            const half8 hi = *reinterpret_cast<const half8*>(ah + mt * 16 * kStride);
-            const half8 lo = *reinterpret_cast<const half8*>(ah + kTileHalves + mt * 16 * kStride);
-            // the four high-part products first, then the four low-part ones: two instructions on one accumulator are
-            // four instructions apart instead of back to back
-#pragma unroll
-            for (int nt = 0; nt < 4; ++nt) acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi, bf[nt], acc[mt][nt], 0, 0, 0);
-#pragma unroll
-            for (int nt = 0; nt < 4; ++nt) acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(lo, bf[nt], acc[mt][nt], 0, 0, 0);
+            for (int i = 0; i < kLoads; ++i) {
+                __builtin_amdgcn_sched_group_barrier(0x008, kPerLoad, 0);
+                __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+            }
         }
+        __builtin_amdgcn_sched_barrier(0);
     };
-
-    // Three register sets keep the loads of the next three steps in flight (a step's arithmetic is several times
-    // shorter than the memory latency); the sets rotate with the step, so the loop is unrolled by three.  (Two sets and
-    // three workgroups per CU measured the same on large shapes and slower on small grids.)
-    StepRegs r0, r1, r2;
-    const int last = steps - 1;
-    issue(r0, 0);
-    issue(r1, 1 < last ? 1 : last);
-    issue(r2, 2 < last ? 2 : last);
-    to_lds(r0, 0);
-    __syncthreads();
-    // step s: reload the set that step s consumed with step s + 3 (clamped: no branch around loads), compute from the
-    // current LDS buffer, move step s + 1 into the other buffer
-    auto step = [&](StepRegs& reload, const StepRegs& next, int s) {
-        issue(reload, s + 3 < last ? s + 3 : last);
-        compute(s & 1);
-        to_lds(next, (s + 1) & 1);
-        __syncthreads();
+    auto stage = [&](auto ph_c, int s) __attribute__((always_inline)) {
+        sub_step(ph_c, std::integral_constant<int, 0>(), s);
+        if constexpr (KS == 2) sub_step(ph_c, std::integral_constant<int, 1>(), s);
+        wait_and_meet(std::integral_constant<int, kInFlight>());
     };
+    // Small tiles have registers to keep the sums of a period (10 or 12 steps) apart from those before: a fraction of the chain of roundings
+    // that all of K would be (as short as the parts of K that small grids are otherwise cut into).
+    constexpr bool kBlocked = MT * NT <= 8;
+    floatx4 total[kBlocked ? MT : 1][kBlocked ? NT : 1];
+    if (kBlocked) {
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int j = 0; j < NT; ++j) total[kBlocked ? i : 0][kBlocked ? j : 0] = floatx4{0.f, 0.f, 0.f, 0.f};
+    }
     int s = 0;
-    for (; s + 3 <= steps; s += 3) {
-        step(r0, r1, s);
-        step(r1, r2, s + 1);
-        step(r2, r0, s + 2);
-    }
-    if (s < steps) step(r0, r1, s);
-    if (s + 1 < steps) step(r1, r2, s + 1);
-
-    // D fragment: lane holds rows 4 * (lane / 16) + r, column lane % 16 of each 16 x 16 tile
-    const int out_col = lane & 15, out_row = (lane >> 4) * 4;
-    const float* R = k_splits == 1 ? mats.R[mat] : nullptr;      // a K split adds the residual when it adds the planes
-    // Two forms of the last step, chosen once per workgroup.  With a residual: per group of 16 rows its values first --
-    // unconditional loads from clamped addresses, no branch and no wait between them -- then the stores; a load that
-    // follows a store to memory it might alias is not moved ahead of it, and a load under a per-lane branch is awaited at
-    // the branch's end (measured with both mistakes in place: +10 us on a 65 us launch).
-    auto store_tile = [&](auto with_residual) {
+    for (; s + kPeriod <= stages; s += kPeriod) {
+        tiled_unrolled(std::make_integer_sequence<int, kPeriod>(),
+                       [&](auto ph_c) __attribute__((always_inline)) { stage(ph_c, s + decltype(ph_c)::value); });
+        if (kBlocked) {
 #pragma unroll
-        for (int mt = 0; mt < 4; ++mt) {
-            float res[4][4];
+            for (int i = 0; i < MT; ++i)
+#pragma unroll
+                for (int j = 0; j < NT; ++j) {
+                    total[kBlocked ? i : 0][kBlocked ? j : 0] += acc[i][j];
+                    acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+                }
+        }
+    }
+    tiled_unrolled(std::make_integer_sequence<int, kPeriod - 1>(), [&](auto ph_c) __attribute__((always_inline)) {
+        if (s + decltype(ph_c)::value < stages) stage(ph_c, s + decltype(ph_c)::value);
+    });
+    if (kBlocked) {
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int j = 0; j < NT; ++j) acc[i][j] += total[kBlocked ? i : 0][kBlocked ? j : 0];
+    }
+    __builtin_amdgcn_s_waitcnt(vmcnt_only(0));      // no write into LDS may be outstanding when the workgroup ends
+
+    // lane: row lane % 16, columns 4 (lane / 16) .. + 3 of each 16 x 16 tile
+    float* __restrict__ C = mats.C[at.mat] + (size_t)at.split * M * N;
+    const float* R = k_splits == 1 ? mats.R[at.mat] : nullptr;      // a K split adds the residual when it adds the planes
+    const bool whole = N % 4 == 0 && m40_aligned16(mats.C[at.mat]) && m40_aligned16(R);
+    const int col0 = n0 + wn * NT * 16 + 4 * (lane >> 4);
+    // With a residual: per group of 16 rows its values first -- unconditional loads from clamped addresses, no branch and no wait between
+    // them -- then the stores; a load that follows a store to memory it might alias is not moved ahead of it, and a load under a
+    // per-lane branch is awaited at the branch's end (measured with both mistakes in place: +10 us on a 65 us launch).
+    auto store_tile = [&](auto with_residual) __attribute__((always_inline)) {
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+            const int row = m0 + (wm * MT + mt) * 16 + frag_row;
+            const size_t row_off = (size_t)(row < M ? row : M - 1) * N;
+            floatx4 res[NT];
             if (decltype(with_residual)::value) {
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int row = m0 + wm * 64 + mt * 16 + out_row + r;
-                    const size_t row_off = (size_t)(row < M ? row : M - 1) * N;
+                for (int nt = 0; nt < NT; ++nt) {
+                    const int col = col0 + nt * 16;
+                    if (whole) {
+                        res[nt] = *reinterpret_cast<const floatx4*>(R + row_off + (col < N ? col : 0));
+                    } else {
 #pragma unroll
-                    for (int nt = 0; nt < 4; ++nt) {
-                        const int col = n0 + wn * 64 + nt * 16 + out_col;
-                        res[r][nt] = R[row_off + (col < N ? col : N - 1)];
+                        for (int r = 0; r < 4; ++r) res[nt][r] = R[row_off + (col + r < N ? col + r : N - 1)];
                     }
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
+            if (row >= M) continue;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int row = m0 + wm * 64 + mt * 16 + out_row + r;
-                if (row >= M) continue;
-                const float sc = sc_all[mt][r];       // a power of two: exact, also on the partial sums of a K split
+            for (int nt = 0; nt < NT; ++nt) {
+                const int col = col0 + nt * 16;
+                floatx4 v = acc[mt][nt];
 #pragma unroll
-                for (int nt = 0; nt < 4; ++nt) {
-                    const int col = n0 + wn * 64 + nt * 16 + out_col;
-                    if (col < N) {
-                        const float v = acc[mt][nt][r] * sc;
-                        C[((size_t)split * M + row) * N + col] = decltype(with_residual)::value ? res[r][nt] + v : v;
-                    }
+                for (int r = 0; r < 4; ++r) {
+                    v[r] *= scale[mt];       // a power of two: exact, also on the partial sums of a K split
+                    if (decltype(with_residual)::value) v[r] = res[nt][r] + v[r];
+                }
+                if (whole) {
+                    if (col < N) *reinterpret_cast<floatx4*>(C + row_off + col) = v;
+                } else {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        if (col + r < N) C[row_off + col + r] = v[r];
                 }
             }
         }
@@ -388,219 +470,61 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_tiled_f32xf16_gguf_kernel(co
     else store_tile(std::false_type{});
 }
 
-// ---- wide tile: 128 x 256 per workgroup of four waves (wave tile 64 x 128), one workgroup per CU ---------------------------
-//
-// Measured on the 128 x 128 kernel above with parts of it switched off (M 4096, N 2048, K 2048): arithmetic alone 46 us,
-// loads + LDS traffic + barriers alone 45 us, everything 87 us -- the two did not overlap.  A wave issues in order, and a
-// memory instruction holds the issue slot until its unit accepts it; with the four waves of a CU in step behind the
-// barrier, sixteen fragment reads, eight LDS writes and eight global loads each queue for ~500 cycles before the first
-// matrix instruction of the step can go.  Here:
-//  * every memory instruction of a step is issued under the step's matrix instructions, one per two of them
-//    (sched_group_barrier), so it waits for its unit while the matrix pipe works;
-//  * the fragments of step s + 1 are read from LDS during the arithmetic of step s (two fragment sets in registers);
-//  * global data goes straight into LDS (global_load_lds_dwordx4: no registers, no LDS write instruction, no wait
-//    before one), five 32 KB buffers deep -- a lane fetches the 16-byte chunk that belongs at its place in the swizzled
-//    row layout, so a wave's instruction fills one contiguous kilobyte; the workgroup waits only for the step after
-//    next (vmcnt) ahead of the barrier that publishes it;
-//  * the wave tile is 64 x 128: per matrix instruction two thirds of the fragment bytes of a 64 x 64 tile (the activation
-//    rows, read twice -- high and low part -- are the short side).
-// M 4096, N 2048, K 2048: 79 -> 60 us; N 11264: 479 -> 404 us; K 5632: 232 -> 173 us.  Under this load the part lowers
-// its clock (1.4-1.9 GHz measured inside the kernel, against 2.0-2.2 GHz in short or memory-bound launches), and a form
-// with fewer issue cycles (32 x 32 x 16 instructions: 1370 instead of 1500 cycles per step) ran at a lower clock
-// still and took the same time: what is left is energy per product, of which the exact hi + lo split is half.
-constexpr int kWideBN = 256;
-constexpr int kWideWM = 64, kWideWN = 128;                   // wave tile, waves 2 x 2
-constexpr int kWideMT = kWideWM / 16, kWideNT = kWideWN / 16;
-constexpr int kWidePlane = kBM * 64;                          // bytes of a 128-row operand block (32 k)
-constexpr int kWideBuf = 2 * kWidePlane + kWideBN * 64;      // A high, A low, B: 32 KB
-constexpr int kWideBufs = 5;
-constexpr int kWideLds = kWideBufs * kWideBuf;               // 160 KB: the whole LDS of a CU
-constexpr int kWideAL = kBM / 64, kWideBL = kWideBN / 64;    // 16-byte loads per thread: rows lrow + 64 i of a plane
-constexpr int kWideLoads = 2 * kWideAL + kWideBL;
-
-struct WideFrags { half8 hi[kWideMT], lo[kWideMT], b[kWideNT]; };
-
-template <int... I, class F>
-__device__ __forceinline__ void tiled_unrolled(std::integer_sequence<int, I...>, F&& f) { (f(std::integral_constant<int, I>{}), ...); }
-
-// s_waitcnt for vector-memory operations only: at most n of them may still be outstanding
-__device__ __forceinline__ constexpr int vmcnt_only(int n) { return 0x0f70 | (n & 15) | ((n >> 4) << 14); }
-
-__global__ __launch_bounds__(kThreads, 1) void gemm_tiled_wide_kernel(const _Float16* __restrict__ A_hi,
-                                                                      const _Float16* __restrict__ A_lo,
-                                                                      const float* __restrict__ row_scale, TiledMats mats,
-                                                                      int M, int K) {
-    typedef __attribute__((address_space(3))) void* lds_dst_t;
-    typedef const __attribute__((address_space(1))) void* global_src_t;
-    extern __shared__ __align__(16) uint8_t wide_lds[];
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int tiles_n = mats.tile_start[mats.n];
-    // each die owns a contiguous band of tile rows, as above
-    const int per_die = (int)gridDim.x / 8;
-    const int logical = (int)blockIdx.x < per_die * 8 ? ((int)blockIdx.x % 8) * per_die + (int)blockIdx.x / 8 : (int)blockIdx.x;
-    const int tile_m = logical / tiles_n;
-    int tile_n = logical % tiles_n;
-    int mat = 0;
-#pragma unroll
-    for (int i = 1; i < kMaxMats; ++i)
-        if (i < mats.n && tile_n >= mats.tile_start[i]) mat = i;
-    tile_n -= mats.tile_start[mat];
-    const uint16_t* __restrict__ B = mats.B[mat];
-    float* __restrict__ C = mats.C[mat];
-    const int N = mats.N[mat];
-    const int m0 = tile_m * kBM, n0 = tile_n * kWideBN;
-    // loader: thread -> row lrow (+ 64 i) of a plane and the place tid % 4 in that row's 64 bytes, which holds chunk
-    // (tid % 4) ^ ((lrow / 4) % 4) of the row; the host guarantees that M * K and N * K fit 31 bits
-    const int lrow = tid >> 2, gchunk = (tid & 3) ^ ((lrow >> 2) & 3);
-    uint32_t a_off[kWideAL], b_off[kWideBL];     // in halves
-#pragma unroll
-    for (int i = 0; i < kWideAL; ++i) {
-        const int ar = m0 + lrow + 64 * i < M ? m0 + lrow + 64 * i : M - 1;     // clamped: computed, never stored
-        a_off[i] = (uint32_t)ar * (uint32_t)K + gchunk * 8;
+template <int MT, int NT, int KS, int kBufs>
+int launch_tiles(hipStream_t stream, const _Float16* hi, const _Float16* lo, const float* row_scale, TiledMats mats, int M, int K, int k_splits) {
+    constexpr int BM = 32 * MT, BN = 32 * NT, bytes = kBufs * (2 * BM + BN) * 64 * KS;
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_tiled_kernel<MT, NT, KS, kBufs>),
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    if (attr != hipSuccess) return -2;
+    const int tiles_m = (M + BM - 1) / BM;
+    long long tiles_n = 0;
+    for (int i = 0; i < mats.n; ++i) {
+        mats.tile_start[i] = (int)tiles_n;
+        tiles_n += (mats.N[i] + BN - 1) / BN;
     }
-#pragma unroll
-    for (int i = 0; i < kWideBL; ++i) {
-        const int bc = n0 + lrow + 64 * i < N ? n0 + lrow + 64 * i : N - 1;
-        b_off[i] = (uint32_t)bc * (uint32_t)K + gchunk * 8;
+    mats.tile_start[mats.n] = (int)tiles_n;
+    // M 4096, N 11264, K 2048 on the 128 x 256 tile (32 tile rows), bands of 4 / 6 rows: 357 / 338 us (bands of 2, 4, 8 and 16 are all slower than 5, 6
+    // and 7); M 522, N 2048, K 5632 on 64 x 128 (9 tile rows), bands of 1 / 3 / 5 / 9: 54.2 / 48.1 / 46.7 / 44.4 us
+    const int band = tiles_m <= 9 ? tiles_m : 6;
+    gemm_tiled_kernel<MT, NT, KS, kBufs><<<(unsigned)(tiles_m * tiles_n * k_splits), kThreads, bytes, stream>>>(hi, lo, row_scale, mats, M, K, k_splits, band);
+    return hipGetLastError() == hipSuccess ? 0 : -2;
+}
+
+// Which tile, and into how many parts to cut K.  A launch of t workgroups on c CUs takes, per step of 32 k, about
+// max(least, start * ceil(t / c) + load * t / c): a workgroup alone on its CU is bound by the round trips of a step, more of them by the step's
+// products and LDS traffic, and by caches and clock when the other CUs work too.  Fitted to 50 shapes with weights that no cache holds (M 60 ..
+// 4096 of N 2048, 2560, 11264, K 2048 and 5632), most within 10 %, e.g. N 2048, K 2048 (128 x 256 / 128 x 128 / 64 x 128 / 64 x 64):
+//   60 rows 43.6 / 28.5 / 21.0 / 15.5 us, 522 rows 43.3 / 28.0 / 18.2 / 23.4, 1030 rows 44.1 / 30.4 / 35.0 / 35.6, 4096 rows 62 / 82 / 84 / 110
+// (a 128 x 128 tile staged through registers and cut into four parts of K up to 128 tiles, with the launch that adds them: 23 / 32 / 42.7 / 80).
+// Parts of K cost the launch that adds their sums; K 5632 at 256 rows: 35.9 us whole, 24.7 us in two.
+struct TileChoice { int shape, k_splits; };
+constexpr struct { int bm, bn; float least, start, load; } kShapes[4] = {
+    {128, 256, 0.66f, 0.64f, 0.28f}, {128, 128, 0.44f, 0.42f, 0.10f}, {64, 128, 0.28f, 0.25f, 0.05f}, {64, 64, 0.235f, 0.17f, 0.03f}};
+// The two large tiles add up all of their part of K in one chain: where small grids are cut (may_split) they are taken for four parts only (K 2048 is
+// where a chain's error shows: 64 steps and more).  The two small tiles, which add up blocks of k, are for small grids and for one row of tiles; past
+// that the larger ones are faster (above, 1030 rows), and a row's sums do not depend on how many rows come with it.
+TileChoice pick_tile(int M, int n_mats, const int* N, int steps, int num_cus, bool small_grid, bool may_split) {
+    TileChoice best{1, may_split && steps >= 64 ? 4 : 1};        // what is left for a small grid of an odd number of steps
+    float best_us = 3.0e38f;
+    float out_mb = 0.0f;
+    for (int i = 0; i < n_mats; ++i) out_mb += (float)M * (float)N[i] * 4e-6f;
+    for (int c = 0; c < 4; ++c) {
+        if (c >= 2 && (steps % 2 != 0 || !(small_grid || M <= 128))) break;            // the small tiles take two steps a stage
+        long long tiles = 0;
+        for (int i = 0; i < n_mats; ++i) tiles += (N[i] + kShapes[c].bn - 1) / kShapes[c].bn;
+        tiles *= (M + kShapes[c].bm - 1) / kShapes[c].bm;
+        for (int s = 1; s <= 8; ++s) {
+            const int stage = c >= 2 ? 2 : 1, per = (steps / stage + s - 1) / s * stage;
+            if (s > 1 && (!may_split || per < 16 || (long long)per * (s - 1) >= steps || tiles * (s - 1) >= num_cus)) break;
+            if (c < 2 && may_split && s < 4 && per >= 32) continue;
+            const long long units = (tiles * s + num_cus - 1) / num_cus;
+            const float a = kShapes[c].start * (float)units + kShapes[c].load * (float)(tiles * s) / (float)num_cus;
+            float us = (float)per * (a > kShapes[c].least ? a : kShapes[c].least);
+            if (s > 1) us += 6.0f + (float)(s + 1) * out_mb / 5.0f;       // MB over TB/s are us
+            if (us < best_us) { best_us = us; best = {c, s}; }
+        }
     }
-    const int steps = K / kBK, last = steps - 1;
-    // one instruction of a wave fills rows 16 wave .. 16 wave + 15 (+ 64 i) of a plane: a contiguous kilobyte, lane by lane
-    auto issue = [&](int buf, int step) {
-        step = step < last ? step : last;          // past the end: the last step again (no branch around loads)
-        const _Float16* ah = A_hi + (size_t)step * kBK;
-        const _Float16* al = A_lo + (size_t)step * kBK;
-        const uint16_t* bb = B + (size_t)step * kBK;
-        uint8_t* dst = wide_lds + buf * kWideBuf + wave * 1024;
-#pragma unroll
-        for (int i = 0; i < kWideAL; ++i) {
-            __builtin_amdgcn_global_load_lds((global_src_t)(ah + a_off[i]), (lds_dst_t)(dst + i * 4096), 16, 0, 0);
-            __builtin_amdgcn_global_load_lds((global_src_t)(al + a_off[i]), (lds_dst_t)(dst + kWidePlane + i * 4096), 16, 0, 0);
-        }
-#pragma unroll
-        for (int i = 0; i < kWideBL; ++i)
-            __builtin_amdgcn_global_load_lds((global_src_t)(bb + b_off[i]), (lds_dst_t)(dst + 2 * kWidePlane + i * 4096), 16, 0, 0);
-    };
-    const int wm = wave >> 1, wn = wave & 1;
-    float sc_all[kWideMT][4];          // the scales of the rows this lane will store, requested ahead of everything else
-#pragma unroll
-    for (int mt = 0; mt < kWideMT; ++mt)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int row = m0 + wm * kWideWM + mt * 16 + (lane >> 4) * 4 + r;
-            sc_all[mt][r] = row_scale[row < M ? row : M - 1];
-        }
-    const int frag_row = lane & 15;
-    const int fr_off = frag_row * 64 + (((lane >> 4) ^ ((frag_row >> 2) & 3)) * 16);
-    auto read_frags = [&](WideFrags& f, int buf) {
-        const uint8_t* base = wide_lds + buf * kWideBuf + fr_off;
-        const uint8_t* a = base + wm * kWideWM * 64;
-        const uint8_t* b = base + 2 * kWidePlane + wn * kWideWN * 64;
-#pragma unroll
-        for (int mt = 0; mt < kWideMT; ++mt) {
-            f.hi[mt] = *reinterpret_cast<const half8*>(a + mt * 16 * 64);
-            f.lo[mt] = *reinterpret_cast<const half8*>(a + kWidePlane + mt * 16 * 64);
-        }
-#pragma unroll
-        for (int nt = 0; nt < kWideNT; ++nt) f.b[nt] = *reinterpret_cast<const half8*>(b + nt * 16 * 64);
-    };
-    floatx4 acc[kWideMT][kWideNT];
-#pragma unroll
-    for (int i = 0; i < kWideMT; ++i)
-#pragma unroll
-        for (int j = 0; j < kWideNT; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-    // per accumulator the same order as the 128 x 128 kernel (step by step, high part then low part): the same bits
-    auto compute = [&](const WideFrags& f) {
-#pragma unroll
-        for (int mt = 0; mt < kWideMT; ++mt) {
-#pragma unroll
-            for (int nt = 0; nt < kWideNT; ++nt) acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(f.hi[mt], f.b[nt], acc[mt][nt], 0, 0, 0);
-#pragma unroll
-            for (int nt = 0; nt < kWideNT; ++nt) acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(f.lo[mt], f.b[nt], acc[mt][nt], 0, 0, 0);
-        }
-    };
-
-    WideFrags f[2];
-    // steps 0 .. 4 requested, one per buffer; steps 0 and 1 awaited.  The barriers are bare s_barrier instructions with
-    // the vector-memory wait written out: __syncthreads() would wait for every outstanding load (its fence covers LDS).
-#pragma unroll
-    for (int i = 0; i < kWideBufs; ++i) issue(i, i);
-    __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_waitcnt(vmcnt_only((kWideBufs - 2) * kWideLoads));
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_sched_barrier(0);
-    read_frags(f[0], 0);
-    // Before step s: the fragments of step s are requested into f[s % 2]; buffer (s + 1) % 5 is complete and visible;
-    // steps s + 2 .. s + 3 are in flight.  Step s refills the buffer of step s - 1 -- whose fragments every wave had in
-    // registers before the last barrier -- with step s + 4, and waits for step s + 2 ahead of its barrier.  (Step 0
-    // requests step 4 a second time: buffer 0 is still being read then.)
-    constexpr int kPeriod = 2 * kWideBufs;
-    auto step = [&](auto ph_c, int s) __attribute__((always_inline)) {
-        constexpr int ph = decltype(ph_c)::value;
-        read_frags(f[(ph + 1) & 1], (ph + 1) % kWideBufs);
-        issue((ph + kWideBufs - 1) % kWideBufs, s - 1 + kWideBufs);
-        compute(f[ph & 1]);
-        // issue order: two matrix instructions, one LDS read (16 times), then two matrix instructions, one load (8 times)
-#pragma unroll
-        for (int i = 0; i < 2 * kWideMT + kWideNT; ++i) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
-            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-        }
-#pragma unroll
-        for (int i = 0; i < kWideLoads; ++i) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
-            __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        __builtin_amdgcn_s_waitcnt(vmcnt_only((kWideBufs - 3) * kWideLoads));
-        __builtin_amdgcn_s_barrier();
-        __builtin_amdgcn_sched_barrier(0);
-    };
-    int s = 0;
-    for (; s + kPeriod <= steps; s += kPeriod)
-        tiled_unrolled(std::make_integer_sequence<int, kPeriod>(),
-                       [&](auto ph_c) __attribute__((always_inline)) { step(ph_c, s + decltype(ph_c)::value); });
-    tiled_unrolled(std::make_integer_sequence<int, kPeriod - 1>(), [&](auto ph_c) __attribute__((always_inline)) {
-        if (s + decltype(ph_c)::value < steps) step(ph_c, s + decltype(ph_c)::value);
-    });
-    __builtin_amdgcn_s_waitcnt(vmcnt_only(0));      // no write into LDS may be outstanding when the workgroup ends
-
-    const int out_col = lane & 15, out_row = (lane >> 4) * 4;
-    const float* R = mats.R[mat];
-    auto store_tile = [&](auto with_residual) {          // two forms, as in the kernel above
-#pragma unroll
-        for (int mt = 0; mt < kWideMT; ++mt) {
-            float res[4][kWideNT];
-            if (decltype(with_residual)::value) {
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int row = m0 + wm * kWideWM + mt * 16 + out_row + r;
-                    const size_t row_off = (size_t)(row < M ? row : M - 1) * N;
-#pragma unroll
-                    for (int nt = 0; nt < kWideNT; ++nt) {
-                        const int col = n0 + wn * kWideWN + nt * 16 + out_col;
-                        res[r][nt] = R[row_off + (col < N ? col : N - 1)];
-                    }
-                }
-                __builtin_amdgcn_sched_barrier(0);
-            }
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int row = m0 + wm * kWideWM + mt * 16 + out_row + r;
-                if (row >= M) continue;
-                const float sc = sc_all[mt][r];
-#pragma unroll
-                for (int nt = 0; nt < kWideNT; ++nt) {
-                    const int col = n0 + wn * kWideWN + nt * 16 + out_col;
-                    if (col < N) {
-                        const float v = acc[mt][nt][r] * sc;
-                        C[(size_t)row * N + col] = decltype(with_residual)::value ? res[r][nt] + v : v;
-                    }
-                }
-            }
-        }
-    };
-    if (R) store_tile(std::true_type{});
-    else store_tile(std::false_type{});
+    return best;
 }
 
 // out[i] = planes[0][i] + planes[1][i] + ... in that order (n4 float4 per plane), then residual[i] + that (residual may be
@@ -633,7 +557,7 @@ __global__ __launch_bounds__(256) void add_k_planes_kernel(KPlaneSet set, int k_
 
 bool m40_gemm_tiled_supported(const void* A, const void* B, int M, int N, int K) {
     return M > 32 && N >= 16 && K >= kBK && K % kBK == 0 && m40_aligned16(A) && m40_aligned16(B) &&
-           ((long long)((M + kBM - 1) / kBM) * ((N + kBN - 1) / kBN)) <= 0x3fffffffll;
+           ((long long)((M + 127) / 128) * ((N + 127) / 128)) <= 0x3fffffffll;
 }
 
 // Returns 1 when the activations' packing buffer cannot be provided (the stream is being captured and the buffer is
@@ -646,40 +570,31 @@ int m40_launch_gemm_tiled_fused(M40llmCudaContext* ctx, hipStream_t stream, uint
     if (source_kind == kPackNorm && (!norm_w || norm_dtype > 1u || !m40_aligned16(norm_w))) return -2;
     TiledMats mats{};
     mats.n = n_mats;
-    long long tiles_n = 0;
+    long long tiles_128 = 0;
     for (int i = 0; i < n_mats; ++i) {
         if (!m40_gemm_tiled_supported(A, B[i], M, N[i], K) || !C[i]) return -2;
         mats.B[i] = B[i];
         mats.C[i] = C[i];
         mats.R[i] = R ? R[i] : nullptr;
         mats.N[i] = N[i];
-        mats.tile_start[i] = (int)tiles_n;
-        tiles_n += (N[i] + kBN - 1) / kBN;
+        tiles_128 += (N[i] + 127) / 128;
     }
-    mats.tile_start[n_mats] = (int)tiles_n;
-    const long long tiles_m = (M + kBM - 1) / kBM;
-    if (tiles_m * tiles_n > 0x7fffffffll) return -2;
-    constexpr size_t lds_bytes = 2 * kBufHalves * sizeof(_Float16);   // 49152
+    if ((long long)((M + 127) / 128) * tiles_128 > 0x7fffffffll / 8) return -2;
     // two f16 planes of A (and the partial sums of a K split) in the stream's packing buffer, grown on demand (never while
     // the stream is being captured)
     M40StreamScratch& sc = ctx->scratch[stream_kind];
-    // Few tiles and many K steps (short prompts, the down projection): split K so that the chip is covered and a
-    // workgroup's chain of dependent steps is shorter; partial sums go to planes behind the packed activations and are
-    // added in a fixed order by a second launch (every N a multiple of 4 for its float4 accesses).
-    const int steps = K / kBK;
-    int k_splits = 1;
-    const long long tiles = tiles_m * tiles_n;
+    // Parts of K: partial sums go to planes behind the packed activations and are added in a fixed order by a second launch (every N a
+    // multiple of 4 for its float4 accesses).  From half a 128 x 128 tile per CU on a split only adds a pass over the sums (1030 rows of N 2048,
+    // K 5632, 144 tiles: 77.7 us whole, 78.5 us in the best parts).
     bool n4_ok = true;
     size_t out_floats = 0;
     for (int i = 0; i < n_mats; ++i) {
         n4_ok = n4_ok && N[i] % 4 == 0 && m40_aligned16(C[i]) && m40_aligned16(mats.R[i]);
         out_floats += (size_t)M * N[i];
     }
-    if (n4_ok && tiles <= 128) {   // above that a split only adds a partial-sum pass (measured at 176 tiles)
-        k_splits = (int)(512 / tiles);
-        if (k_splits > 4) k_splits = 4;
-        while (k_splits > 1 && (steps / k_splits < 16 || (steps + k_splits - 1) / k_splits * (k_splits - 1) >= steps)) --k_splits;
-    }
+    const bool small_grid = (M + 127) / 128 * tiles_128 <= ctx->num_cus / 2;
+    const TileChoice choice = pick_tile(M, n_mats, N, K / kBK, ctx->num_cus, small_grid, small_grid && n4_ok);
+    const int k_splits = choice.k_splits;
     const size_t scale_bytes = ((size_t)M * 4 + 15) & ~(size_t)15;
     const size_t need = (size_t)M * K * 4 + scale_bytes + (k_splits > 1 ? (size_t)k_splits * out_floats * 4 : 0);
     if (sc.tiled_pack_bytes < need) {
@@ -721,28 +636,14 @@ int m40_launch_gemm_tiled_fused(M40llmCudaContext* ctx, hipStream_t stream, uint
             at += (size_t)k_splits * M * N[i];
         }
     }
-    // the wide tile from 9/16 of a tile per CU on (measured at K 2048: 144 tiles 52 against 68 us for the 128 x 128 kernel, 180
-    // tiles 54 against 72 us; 120 tiles 51 against 48 us, 96 tiles 49 against 46 us), element offsets fitting its 32-bit arithmetic
-    long long wide_tiles_n = 0;
-    TiledMats wide = mats;
-    bool wide_ok = k_splits == 1 && (long long)M * K < 0x7fffffffll;
-    for (int i = 0; i < n_mats; ++i) {
-        wide.tile_start[i] = (int)wide_tiles_n;
-        wide_tiles_n += (N[i] + kWideBN - 1) / kWideBN;
-        wide_ok = wide_ok && (long long)N[i] * K < 0x7fffffffll;
+    int rc = -2;
+    switch (choice.shape) {
+        case 0: rc = launch_tiles<4, 8, 1, 5>(stream, hi, lo, row_scale, launch, M, K, k_splits); break;
+        case 1: rc = launch_tiles<4, 4, 1, 6>(stream, hi, lo, row_scale, launch, M, K, k_splits); break;
+        case 2: rc = launch_tiles<2, 4, 2, 5>(stream, hi, lo, row_scale, launch, M, K, k_splits); break;
+        case 3: rc = launch_tiles<2, 2, 2, 6>(stream, hi, lo, row_scale, launch, M, K, k_splits); break;
     }
-    wide.tile_start[n_mats] = (int)wide_tiles_n;
-    if (wide_ok && 16 * tiles_m * wide_tiles_n >= 9ll * ctx->num_cus) {
-        static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_tiled_wide_kernel),
-                                                           hipFuncAttributeMaxDynamicSharedMemorySize, kWideLds);
-        wide_ok = attr == hipSuccess;
-    } else {
-        wide_ok = false;
-    }
-    if (wide_ok)
-        gemm_tiled_wide_kernel<<<(unsigned)(tiles_m * wide_tiles_n), kThreads, kWideLds, stream>>>(hi, lo, row_scale, wide, M, K);
-    else
-        gemm_tiled_f32xf16_gguf_kernel<<<(unsigned)(tiles * k_splits), kThreads, lds_bytes, stream>>>(hi, lo, row_scale, launch, M, K, k_splits);
+    if (rc != 0) return rc;
     if (k_splits > 1) {
         KPlaneSet set{};
         size_t blocks = 0;
