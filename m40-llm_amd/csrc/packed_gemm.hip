@@ -4,8 +4,8 @@
 //                      straight from memory into the matrix instruction's operand registers, one contiguous kilobyte a
 //                      load, each tile read once per 64 rows; the waves' sums meet in LDS.  Decode steps and short
 //                      portions, and every product in f32.
-// tile_packed_kernel   bf16, more rows: 128 x (128 or 256) tiles of C, both operands staged through LDS by direct
-//                      global-to-LDS loads, five or six steps of 32 k deep with one barrier a step.  The buffers hold
+// tile_packed_kernel   bf16, more rows: tiles of C of 64 x 64 to 128 x 256, both operands staged through LDS by direct
+//                      global-to-LDS loads, five or six stages deep with one barrier a stage.  The buffers hold
 //                      operands in instruction order, so LDS reads are contiguous kilobytes as well.
 //
 // Products per expert: both kernels take a list of jobs (expert, rows of the list sorted by expert) made on the device; the rows are
@@ -13,6 +13,7 @@
 #include "packed_gemm.hpp"
 
 #include <type_traits>
+#include <utility>
 
 namespace {
 
@@ -154,88 +155,108 @@ int launch_rows_any(hipStream_t stream, const PackedArgs& g, const M40Epilogue<T
 }
 
 // ---- many rows, bf16 ---------------------------------------------------------------------------------------------------
-// Workgroup of four waves (2 x 2), wave tile 64 x (16 NTW): C tile 128 x 32 NTW.  A step is one k tile of every operand
-// tile: (8 + 2 NTW) KB, filled by global_load_lds (a wave's instruction moves one 16 x 32 operand tile, a contiguous kilobyte).
+// Workgroup of four waves (2 x 2), wave tile 16 MTW x 16 NTW: C tile 32 MTW x 32 NTW.  A stage is KS k tiles of every operand
+// tile: 2 (MTW + NTW) KS KB, filled by global_load_lds (a wave's instruction moves one 16 x 32 operand tile, a contiguous kilobyte).
 //
-// Memory instructions are issued under matrix instructions: the fragments of the next step and the loads of a step kBufs - 1
+// Memory instructions are issued under matrix instructions: the fragments of the next step and the loads of a stage kBufs - 1
 // ahead go out one at a time between the current step's products (sched_group_barrier), so that no wave waits for an address
-// or LDS unit with the matrix pipe idle.  Step t refills the buffer of step t - 1, whose fragments every wave had in registers
-// before the barrier behind that step, and ends with step t + 2 landed.
+// or LDS unit with the matrix pipe idle.  Stage s refills the buffer of stage s - 1, whose fragments every wave had in registers
+// before the barrier behind that stage, and ends with stage s + 2 landed.
 enum { kPlainRows = 0, kPageKeys = 1, kPageValues = 2, kSlots = 3 };
-constexpr int tile_bufs(int ntw) { return ntw == 8 ? 6 : 5; }       // one or two workgroups a CU
 
-template <int NTW, int FORM>
-__global__ __launch_bounds__(256, 1) void tile_packed_kernel(PackedArgs g, M40Epilogue<m40_bf16> e) {
+// s_waitcnt for vector-memory operations only, then the barrier: reads of LDS need no wait of their own here
+template <int VM>
+__device__ __forceinline__ void landed_and_meet() {
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(0x0f70 | (VM & 15) | ((VM >> 4) << 14));
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+}
+template <int... I, class F>
+__device__ __forceinline__ void unrolled(std::integer_sequence<int, I...>, F&& f) { (f(std::integral_constant<int, I>{}), ...); }
+
+// rows of tiles of a wave whose sums fit into the buffers at a time
+constexpr int tile_part(int mtw, int ntw, int ks, int bufs) {
+    int part = mtw;
+    while (4 * part * ntw > 2 * (mtw + ntw) * ks * bufs) part /= 2;
+    return part;
+}
+
+template <int MTW, int NTW, int KS, int kBufs, int FORM>
+__global__ __launch_bounds__(256, 1) void tile_packed_kernel(PackedArgs g, M40Epilogue<m40_bf16> e, int band) {
     typedef __attribute__((address_space(3))) void* lds_dst_t;
     typedef const __attribute__((address_space(1))) void* global_src_t;
     extern __shared__ __align__(16) uint8_t stage_lds[];
-    constexpr int kATiles = 8, kBTiles = 2 * NTW;                    // 16-row operand tiles of the workgroup
-    constexpr int kBufs = tile_bufs(NTW), kStepBytes = (kATiles + kBTiles) * 1024;
-    constexpr int kLoads = (kATiles + kBTiles) / 4;                  // per wave and step
+    constexpr int kATiles = 2 * MTW, kBTiles = 2 * NTW, kRows = 16 * kATiles;      // 16-row operand tiles of the workgroup
+    constexpr int kStageBytes = (kATiles + kBTiles) * KS * 1024;
+    constexpr int kALoads = kATiles * KS / 4, kLoads = (kATiles + kBTiles) * KS / 4;      // per wave and stage
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    constexpr bool kJobs = FORM == kSlots;
-    const int tiles_n = (g.n_tiles + kBTiles - 1) / kBTiles, tiles_m = kJobs ? (int)g.jobs[0] : (g.rows + 127) / 128;
+    constexpr bool kJobs = FORM == kSlots, kPaged = FORM == kPageKeys || FORM == kPageValues;
+    const int tiles_n = (g.n_tiles + kBTiles - 1) / kBTiles, tiles_m = kJobs ? (int)g.jobs[0] : (g.rows + kRows - 1) / kRows;
     const int workgroups = kJobs ? tiles_m * tiles_n : (int)gridDim.x;       // the grid is as large as the list of jobs can be
     if (kJobs && (int)blockIdx.x >= workgroups) return;
-    // workgroups are dealt to the eight dies in turn: each die gets a contiguous band of tiles, walked in blocks of four row
+    // workgroups are dealt to the eight dies in turn: each die gets a contiguous run of tiles, walked in blocks of `band` row
     // tiles so that what runs on a die at one time shares both operands
     const int per_die = workgroups / 8;
     const int logical = (int)blockIdx.x < per_die * 8 ? ((int)blockIdx.x % 8) * per_die + (int)blockIdx.x / 8 : (int)blockIdx.x;
-    const int group = logical / (4 * tiles_n), in_group = logical - group * 4 * tiles_n, gm = tiles_m - group * 4 < 4 ? tiles_m - group * 4 : 4;
-    const int t0 = in_group / gm * kBTiles;
-    int m0 = (group * 4 + in_group % gm) * 128, batch = blockIdx.z;
+    const int group = logical / (band * tiles_n), in_group = logical - group * band * tiles_n, gm = tiles_m - group * band < band ? tiles_m - group * band : band;
+    const int t0 = __builtin_amdgcn_readfirstlane(in_group / gm * kBTiles), row_tile = group * band + in_group % gm;
+    int m0 = __builtin_amdgcn_readfirstlane(row_tile * kRows), batch = blockIdx.z;
     if (kJobs) {
-        const uint32_t* job = g.jobs + 4 + 4 * (group * 4 + in_group % gm);
+        const uint32_t* job = g.jobs + 4 + 4 * row_tile;
         batch = __builtin_amdgcn_readfirstlane((int)job[0]);
         m0 = __builtin_amdgcn_readfirstlane((int)job[1]);
         g.rows = e.rows = m0 + __builtin_amdgcn_readfirstlane((int)job[2]);
     }
-    const m40_bf16* A = static_cast<const m40_bf16*>(g.a) + (kJobs ? 0 : (g.segment ? t0 / g.segment : batch) * g.a_batch);
-    const m40_bf16* W = g.w + batch * g.w_batch;
-    const int k_tiles = g.k_count(batch);
-    // this wave's pieces of a step: operand tiles wave, wave + 4, ... of the A tiles, then of the W tiles
-    const m40_bf16* src[kLoads];
+    const int stages = g.k_count(batch) / KS;
+    // A scalar address that walks k, and per lane a 32-bit offset from it that does not change (cache pages lie anywhere: whole addresses).
+    // This wave's pieces of a stage: operand tiles' k tiles wave, wave + 4, ... of A, then of the weights.
+    const uint8_t* a_base = static_cast<const uint8_t*>(g.a) + ((kJobs ? 0 : (g.segment ? t0 / g.segment : batch) * g.a_batch) + (long)m0 * g.lda) * 2;
+    const uint8_t* w_base = reinterpret_cast<const uint8_t*>(g.w + batch * g.w_batch + (long)t0 * g.k_stride * kM40Tile);
+    const uint8_t* page[kPaged ? kALoads : 1];
+    uint32_t off[kLoads];
 #pragma unroll
     for (int i = 0; i < kLoads; ++i) {
-        const int t = wave + 4 * i;
-        if (i < kATiles / 4) {
-            if (FORM == kPageKeys || FORM == kPageValues) {
-                const int rt = m0 / 16 + t, tiles = g.rows / 16, c = rt < tiles ? rt : tiles - 1;
-                src[i] = A + ((long)g.pages[c >> 2] * 4 + (c & 3)) * g.page_k_tiles * kM40Tile + lane * 8;
-            } else {
-                const int rt = m0 / 16 + t, last = (g.rows - 1) / 16;
-                src[i] = A + (long)(rt < last ? rt : last) * 16 * g.lda + lane * 8;
-            }
-        } else {
+        const int piece = wave + 4 * i, sub = piece % KS, t = piece / KS;
+        if (i >= kALoads) {
             const int n = t0 + t - kATiles;
-            src[i] = W + (long)(n < g.n_tiles ? n : g.n_tiles - 1) * g.k_stride * kM40Tile + lane * 8;
+            off[i] = (uint32_t)((n < g.n_tiles ? n : g.n_tiles - 1) - t0) * (uint32_t)g.k_stride * 1024u + sub * 1024u + lane * 16u;
+        } else if (kPaged) {
+            const int rt = m0 / 16 + t, tiles = g.rows / 16, c = rt < tiles ? rt : tiles - 1;
+            page[kPaged ? i : 0] = static_cast<const uint8_t*>(g.a) + (((long)g.pages[c >> 2] * 4 + (c & 3)) * g.page_k_tiles + sub) * 1024 + lane * 16;
+        } else {
+            const int last = (g.rows - 1 - m0) / 16;
+            off[i] = (uint32_t)(t < last ? t : last) * (uint32_t)g.lda * 32u + sub * 1024u + lane * 16u;
         }
     }
-    auto issue = [&](int buf, int t) __attribute__((always_inline)) {
-        uint8_t* base = stage_lds + buf * kStepBytes + wave * 1024;
-        const int k = t < k_tiles ? t : k_tiles - 1;                 // past the end: loaded again, not used
+    auto issue = [&](int buf, int s) __attribute__((always_inline)) {
+        uint8_t* base = stage_lds + buf * kStageBytes + wave * 1024;
+        int k = (s < stages ? s : stages - 1) * KS * 1024;               // past the end: loaded again, not used
+        asm("" : "+s"(k));                                               // keeps it out of the lanes' addresses
 #pragma unroll
-        for (int i = 0; i < kLoads; ++i)
-            __builtin_amdgcn_global_load_lds((global_src_t)(src[i] + (long)k * kM40Tile), (lds_dst_t)(base + i * 4096), 16, 0, 0);
+        for (int i = 0; i < kLoads; ++i) {
+            const uint8_t* src = i >= kALoads ? w_base + k + off[i] : kPaged ? page[kPaged ? i : 0] + k : a_base + k + off[i];
+            __builtin_amdgcn_global_load_lds((global_src_t)src, (lds_dst_t)(base + i * 4096), 16, 0, 0);
+        }
     };
     const int wm = wave >> 1, wn = wave & 1;
-    m40_float4 acc[4][NTW];
+    m40_float4 acc[MTW][NTW];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < MTW; ++i)
 #pragma unroll
         for (int j = 0; j < NTW; ++j) acc[i][j] = m40_float4{0.f, 0.f, 0.f, 0.f};
-    struct Frags { m40_bf16x8 a[4], b[NTW]; } f[2];
-    auto read_frags = [&](Frags& f, int buf) __attribute__((always_inline)) {
-        const uint8_t* a = stage_lds + buf * kStepBytes + wm * 4096 + lane * 16;
-        const uint8_t* b = stage_lds + buf * kStepBytes + (kATiles + wn * NTW) * 1024 + lane * 16;
+    struct Frags { m40_bf16x8 a[MTW], b[NTW]; } f[2];
+    auto read_frags = [&](Frags& f, int buf, int sub) __attribute__((always_inline)) {
+        const uint8_t* a = stage_lds + buf * kStageBytes + (wm * MTW * KS + sub) * 1024 + lane * 16;
+        const uint8_t* b = stage_lds + buf * kStageBytes + ((kATiles + wn * NTW) * KS + sub) * 1024 + lane * 16;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) f.a[i] = *reinterpret_cast<const m40_bf16x8*>(a + i * 1024);
+        for (int i = 0; i < MTW; ++i) f.a[i] = *reinterpret_cast<const m40_bf16x8*>(a + i * KS * 1024);
 #pragma unroll
-        for (int j = 0; j < NTW; ++j) f.b[j] = *reinterpret_cast<const m40_bf16x8*>(b + j * 1024);
+        for (int j = 0; j < NTW; ++j) f.b[j] = *reinterpret_cast<const m40_bf16x8*>(b + j * KS * 1024);
     };
     auto compute = [&](const Frags& f) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < MTW; ++i)
 #pragma unroll
             for (int j = 0; j < NTW; ++j)
                 acc[i][j] = FORM == kPageValues ? __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.a[i], f.b[j], acc[i][j], 0, 0, 0)
@@ -243,99 +264,159 @@ __global__ __launch_bounds__(256, 1) void tile_packed_kernel(PackedArgs g, M40Ep
     };
 #pragma unroll
     for (int i = 0; i < kBufs - 1; ++i) issue(i, i);
-    m40_wait_and_meet<(kBufs - 3) * kLoads>();                       // steps 0 and 1 have landed
-    read_frags(f[0], 0);
-    int buf = 0;
-    auto step = [&](auto parity, int t) __attribute__((always_inline)) {
-        constexpr int ph = decltype(parity)::value;
-        const int next = buf == kBufs - 1 ? 0 : buf + 1;
-        read_frags(f[ph ^ 1], next);
-        issue(buf == 0 ? kBufs - 1 : buf - 1, t + kBufs - 1);
-        compute(f[ph]);
+    landed_and_meet<(kBufs - 3) * kLoads>();                         // stages 0 and 1 have landed
+    read_frags(f[0], 0, 0);
+    // ph: the stage's number in a period, after which buffers and fragment sets are back in their order; periods are written out so that
+    // addresses are constants and sums stay in their registers
+    constexpr int kPeriod = KS == 2 || kBufs % 2 == 0 ? kBufs : 2 * kBufs;
+    auto sub_step = [&](auto ph_c, auto sub_c, int s) __attribute__((always_inline)) {
+        constexpr int ph = decltype(ph_c)::value, sub = decltype(sub_c)::value, buf = ph % kBufs, set = (ph * KS + sub) & 1;
+        read_frags(f[set ^ 1], sub + 1 < KS ? buf : (buf + 1) % kBufs, (sub + 1) % KS);
+        if constexpr (sub == 0) issue((buf + kBufs - 1) % kBufs, s + kBufs - 1);
+        compute(f[set]);
         // products between two fragment reads, and between two loads
-        constexpr int kPerRead = NTW == 8 ? 2 : 1, kPerLoad = (4 * NTW - kPerRead * (4 + NTW)) / kLoads;
+        constexpr int kReads = MTW + NTW, kProducts = MTW * NTW, kPerRead = kProducts >= 2 * kReads + kLoads ? 2 : 1;
+        constexpr int kPerLoad = (kProducts - kPerRead * kReads) / kLoads > 0 ? (kProducts - kPerRead * kReads) / kLoads : 1;
 #pragma unroll
-        for (int i = 0; i < 4 + NTW; ++i) {
+        for (int i = 0; i < kReads; ++i) {
             __builtin_amdgcn_sched_group_barrier(0x008, kPerRead, 0);
             __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
         }
+        if constexpr (sub == 0) {
 #pragma unroll
-        for (int i = 0; i < kLoads; ++i) {
-            __builtin_amdgcn_sched_group_barrier(0x008, kPerLoad, 0);
-            __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+            for (int i = 0; i < kLoads; ++i) {
+                __builtin_amdgcn_sched_group_barrier(0x008, kPerLoad, 0);
+                __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+            }
         }
-        m40_wait_and_meet<(kBufs - 3) * kLoads>();
-        buf = next;
+        __builtin_amdgcn_sched_barrier(0);
     };
-    int t = 0;
-    for (; t + 2 <= k_tiles; t += 2) {
-        step(std::integral_constant<int, 0>(), t);
-        step(std::integral_constant<int, 1>(), t + 1);
-    }
-    if (t < k_tiles) compute(f[0]);
+    auto stage = [&](auto ph_c, int s) __attribute__((always_inline)) {
+        sub_step(ph_c, std::integral_constant<int, 0>(), s);
+        if constexpr (KS == 2) sub_step(ph_c, std::integral_constant<int, 1>(), s);
+        landed_and_meet<(kBufs - 3) * kLoads>();
+    };
+    int s = 0;
+    for (; s + kPeriod <= stages; s += kPeriod)
+        unrolled(std::make_integer_sequence<int, kPeriod>(), [&](auto ph_c) __attribute__((always_inline)) { stage(ph_c, s + decltype(ph_c)::value); });
+    unrolled(std::make_integer_sequence<int, kPeriod - 1>(), [&](auto ph_c) __attribute__((always_inline)) {
+        if (s + decltype(ph_c)::value < stages) stage(ph_c, s + decltype(ph_c)::value);
+    });
     m40_wait_and_meet<0>();                                          // every load has landed: the buffers are free
-    // The sums go through LDS (each wave its own) so that the last step is a loop of a few instructions and not 4 NTW copies of it:
-    // run once per workgroup, those would be fetched cold.
-    m40_float4* mine = reinterpret_cast<m40_float4*>(stage_lds) + wave * 4 * NTW * 64 + lane;
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < NTW; ++j) mine[(i * NTW + j) * 64] = acc[i][j];
     if (FORM == kPlainRows && e.kind == M40LLM_PACKED_ADD && e.vec_out && e.cols % 16 == 0) {
-        // the old values of four tiles are requested together, under clamped addresses: loads behind a branch would be awaited one by one
-#pragma unroll 1
-        for (int i = 0; i < NTW; ++i) {
-            const int row = m0 + (wm * 4 + i * 4 / NTW) * 16 + (lane & 15), j0 = i * 4 % NTW;
-            float* o = e.out_f32 + batch * e.out_batch + (long)(row < e.rows ? row : e.rows - 1) * e.ld_out + 4 * (lane >> 4);
-            m40_float4 old[4];
+        // The old values of a row of tiles are requested together, under clamped addresses and ahead of the stores of the row before: loads
+        // behind a branch or behind a store that they might alias would be awaited one by one.
+        float* o[NTW];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int col = (t0 + wn * NTW + j0 + j) * 16;
-                old[j] = *reinterpret_cast<const m40_float4*>(o + (col < e.cols ? col : 0));
-            }
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int col = (t0 + wn * NTW + j0 + j) * 16;
-                if (row < e.rows && col < e.cols) *reinterpret_cast<m40_float4*>(o + col) = old[j] + mine[(i * 4 + j) * 64];
-            }
+        for (int j = 0; j < NTW; ++j) {
+            const int col = (t0 + wn * NTW + j) * 16;
+            o[j] = e.out_f32 + batch * e.out_batch + (col < e.cols ? col : 0) + 4 * (lane >> 4);
         }
+        m40_float4 old[2][NTW];
+        auto request = [&](auto i_c) __attribute__((always_inline)) {
+            constexpr int i = decltype(i_c)::value;
+            const int row = m0 + (wm * MTW + i) * 16 + (lane & 15);
+            const long at = (long)(row < e.rows ? row : e.rows - 1) * e.ld_out;
+#pragma unroll
+            for (int j = 0; j < NTW; ++j) old[i & 1][j] = *reinterpret_cast<const m40_float4*>(o[j] + at);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        request(std::integral_constant<int, 0>());
+        unrolled(std::make_integer_sequence<int, MTW>(), [&](auto i_c) __attribute__((always_inline)) {
+            constexpr int i = decltype(i_c)::value;
+            if constexpr (i + 1 < MTW) request(std::integral_constant<int, i + 1>());
+            const int row = m0 + (wm * MTW + i) * 16 + (lane & 15);
+            if (row >= e.rows) return;
+#pragma unroll
+            for (int j = 0; j < NTW; ++j)
+                if ((t0 + wn * NTW + j) * 16 < e.cols) *reinterpret_cast<m40_float4*>(o[j] + (long)row * e.ld_out) = old[i & 1][j] + acc[i][j];
+        });
         return;
     }
+    // The sums go through LDS (each wave its own, as many rows of tiles at a time as fit) so that the last step is a loop of a few instructions
+    // and not MTW NTW copies of it: run once per workgroup, those would be fetched cold.
+    constexpr int kPart = tile_part(MTW, NTW, KS, kBufs);
+    m40_float4* mine = reinterpret_cast<m40_float4*>(stage_lds) + wave * kPart * NTW * 64 + lane;
 #pragma unroll 1
-    for (int p = 0; p < 2 * NTW; ++p) {
-        const int i = p / (NTW / 2), j = p % (NTW / 2) * 2, row0 = m0 + (wm * 4 + i) * 16, tile = t0 + wn * NTW + j;
-        if (row0 >= g.rows || tile >= g.n_tiles) continue;
-        const m40_float4 v0 = mine[(2 * p) * 64], v1 = mine[(2 * p + 1) * 64];
-        const bool second = tile + 1 < g.n_tiles;
-        if (FORM == kPageValues) {
-            m40_epilogue_values(e, row0, tile, lane, v0);
-            if (second) m40_epilogue_values(e, row0, tile + 1, lane, v1);
-        } else if (e.kind == M40LLM_PACKED_PROJECT && tile >= e.plain_tiles) {
-            if (second) m40_epilogue_pair(e, row0, (tile - e.plain_tiles) / 2, lane, v0, v1);
-        } else {
+    for (int part = 0; part < MTW / kPart; ++part) {
+        unrolled(std::make_integer_sequence<int, MTW / kPart>(), [&](auto p_c) __attribute__((always_inline)) {
+            if (part != decltype(p_c)::value) return;
+#pragma unroll
+            for (int i = 0; i < kPart; ++i)
+#pragma unroll
+                for (int j = 0; j < NTW; ++j) mine[(i * NTW + j) * 64] = acc[decltype(p_c)::value * kPart + i][j];
+        });
+        const int part_row = m0 + (wm * MTW + part * kPart) * 16;
 #pragma unroll 1
-            for (int k = 0; k < (second ? 2 : 1); ++k) m40_epilogue_tile(e, kJobs ? 0 : batch, row0, tile + k, lane, k ? v1 : v0);
+        for (int p = 0; p < kPart * NTW / 2; ++p) {
+            const int i = p / (NTW / 2), j = p % (NTW / 2) * 2, row0 = part_row + i * 16, tile = t0 + wn * NTW + j;
+            if (row0 >= g.rows || tile >= g.n_tiles) continue;
+            const m40_float4 v0 = mine[(2 * p) * 64], v1 = mine[(2 * p + 1) * 64];
+            const bool second = tile + 1 < g.n_tiles;
+            if (FORM == kPageValues) {
+                m40_epilogue_values(e, row0, tile, lane, v0);
+                if (second) m40_epilogue_values(e, row0, tile + 1, lane, v1);
+            } else if (e.kind == M40LLM_PACKED_PROJECT && tile >= e.plain_tiles) {
+                if (second) m40_epilogue_pair(e, row0, (tile - e.plain_tiles) / 2, lane, v0, v1);
+            } else {
+#pragma unroll 1
+                for (int k = 0; k < (second ? 2 : 1); ++k) m40_epilogue_tile(e, kJobs ? 0 : batch, row0, tile + k, lane, k ? v1 : v0);
+            }
         }
     }
 }
 
-template <int NTW, int FORM>
+template <int MTW, int NTW, int KS, int kBufs, int FORM>
 int launch_tile(hipStream_t stream, const PackedArgs& g, const M40Epilogue<m40_bf16>& e, int batches) {
-    constexpr int lds = (8 + 2 * NTW) * 1024 * tile_bufs(NTW);
-    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(tile_packed_kernel<NTW, FORM>),
+    constexpr int lds = 2 * (MTW + NTW) * KS * 1024 * kBufs;
+    static_assert(lds <= 160 * 1024);
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(tile_packed_kernel<MTW, NTW, KS, kBufs, FORM>),
                                                        hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     if (attr != hipSuccess) return -2;
     constexpr bool kJobs = FORM == kSlots;        // g.rows: the most jobs there can be
-    const long long tiles = (long long)(kJobs ? g.rows : (g.rows + 127) / 128) * ((g.n_tiles + 2 * NTW - 1) / (2 * NTW));
-    tile_packed_kernel<NTW, FORM><<<dim3((unsigned)tiles, 1, (unsigned)batches), 256, lds, stream>>>(g, e);
+    const long long tiles_m = kJobs ? g.rows : (g.rows + 32 * MTW - 1) / (32 * MTW), tiles = tiles_m * ((g.n_tiles + 2 * NTW - 1) / (2 * NTW));
+    // blocks of 5 to 7 rows of tiles measure alike, larger and smaller ones up to a tenth slower (4096 rows, K 2048, N 11264, 128 x 128 tiles, blocks of
+    // 4 / 6 / 8 / 16 / 32: 188 / 178 / 185 / 187 / 214 us); few rows are one block
+    const int band = kJobs ? 4 : tiles_m <= 9 ? (int)tiles_m : 6;
+    tile_packed_kernel<MTW, NTW, KS, kBufs, FORM><<<dim3((unsigned)tiles, 1, (unsigned)batches), 256, lds, stream>>>(g, e, band);
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }
+// Which tile: sums are the same whichever it is.  A launch of t workgroups on c CUs takes, per k tile, about max(least, start + load * t / c): one
+// workgroup alone waits for the round trips of a stage, the second on its CU fills those waits.  Measured with weights that no cache holds, bf16, K 2048 (128 x 256 / 128 x 128 / 64 x 128 / 64 x 64, us):
+//   N 2048:  77 rows 31 / 17.3 / 12.0 / 8.3, 300 rows 31 / 17.7 / 12.0 / 9.2, 700 rows 31 / 18.2 / 13.5 / 15.0, 4096 rows 39.7 / 38.5 / - / -
+//   N 11264: 77 rows 36 / 24 / 17.7 / 18.2, 300 rows 35 / 30 / 29 / 33, 1300 rows 73 / 71 / 82 / 95, 2600 rows 139 / 125 / - / -, 4096 rows 212 / 178 / - / -
+//   N 2048, K 5632: 77 rows 77 / 51 / 36 / 21, 700 rows 75 / 51 / 38 / 41, 4096 rows 85 / 91 / - / -
+// (4096 rows before, with the first tile alone on its CU and addresses and buffers worked out at run time: 230 us at N 11264, 121 at K 5632.)
+constexpr struct { int rows, cols; float least, start, load; } kTileShapes[4] = {
+    {128, 256, 0.48f, 0.50f, 0.0f}, {128, 128, 0.28f, 0.13f, 0.245f}, {64, 128, 0.20f, 0.10f, 0.165f}, {64, 64, 0.13f, 0.10f, 0.10f}};
+
 template <int FORM>
 int launch_tile_any(hipStream_t stream, const PackedArgs& g, const M40Epilogue<m40_bf16>& e, int batches, int num_cus) {
-    const long long wide = (long long)(FORM == kSlots ? g.rows : (g.rows + 127) / 128) * ((g.n_tiles + 15) / 16) * batches;
-    // a short sum is mostly a workgroup's start and end: two narrower workgroups a CU cover each other's
-    if (wide * 16 >= 9ll * num_cus && g.k_tiles > (FORM == kSlots && e.kind == M40LLM_PACKED_STORE_ACT ? 64 : 32)) return launch_tile<8, FORM>(stream, g, e, batches);
-    return launch_tile<4, FORM>(stream, g, e, batches);
+    if constexpr (FORM == kSlots) {
+        return launch_tile<4, 4, 1, 5, FORM>(stream, g, e, batches);          // a job is one row of tiles
+    } else {
+        const bool pairs = g.k_tiles % 2 == 0 && g.k_total % 2 == 0;          // two k tiles a stage
+        int best = 1;
+        float best_cost = 3.0e38f;
+        long long t[4];
+        for (int c = 0; c < 4; ++c) {
+            t[c] = (long long)((g.rows + kTileShapes[c].rows - 1) / kTileShapes[c].rows) * ((g.n_tiles * 16 + kTileShapes[c].cols - 1) / kTileShapes[c].cols) * batches;
+            // the largest tile pays where a long sum's tiles fill the CUs just once
+            if ((c == 0 && (g.k_tiles <= 64 || t[0] > num_cus)) || (c == 3 && !pairs)) continue;
+            const float u = (float)t[c] / (float)num_cus, cost = kTileShapes[c].start + kTileShapes[c].load * u;
+            const float at_least = cost > kTileShapes[c].least ? cost : kTileShapes[c].least;
+            if (at_least < best_cost) { best_cost = at_least; best = c; }
+        }
+        // alone on its CU a workgroup takes the memory of two for deeper buffers: N 2048, K 5632 at 77 rows 21.2 us (64 x 64) against 24.4, at
+        // 1300 rows 43.6 us (128 x 128) against 50.7
+        const bool alone = pairs && t[best] <= num_cus;
+        switch (best) {
+            case 0: return launch_tile<4, 8, 1, 6, FORM>(stream, g, e, batches);
+            case 1: return alone ? launch_tile<4, 4, 2, 5, FORM>(stream, g, e, batches) : launch_tile<4, 4, 1, 5, FORM>(stream, g, e, batches);
+            case 2: return launch_tile<2, 4, 1, 6, FORM>(stream, g, e, batches);
+            default: return alone ? launch_tile<2, 2, 2, 6, FORM>(stream, g, e, batches) : launch_tile<2, 2, 2, 5, FORM>(stream, g, e, batches);
+        }
+    }
 }
 
 template <class T>

@@ -1,0 +1,49 @@
+"""Products of many packed bf16 rows over the tile sizes that row, column and k counts choose, at their edges."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+from pimosun_common import close_to, ld, m40, unpack_tiles, up32  # noqa: E402
+from test_gpu_layer_kernels import ADD, PROJECT, STORE, bf16w, gemm, rounded  # noqa: E402
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    yield m40.Context(0)
+
+
+# 64 x 64 tiles alone on their CU (65 .. 500 rows of few columns) and two to a CU, 64 x 128 (odd number of k tiles, or rows between), 128 x 128, 128 x 256
+# (whole rounds of them); k of one tile, of fewer stages than buffers, of one stage more than a period; rows and columns that fill no tile
+@pytest.mark.parametrize("rows,n,k", [(65, 144, 32), (65, 150, 64), (127, 2048, 384), (200, 500, 352), (300, 1040, 2112), (500, 2048, 256), (700, 2050, 320), (700, 2048, 992),
+                                      (1300, 1504, 96), (1300, 2050, 160), (2049, 3000, 352), (4096, 2048, 192), (4000, 2040, 224)])
+def test_tiles_store_and_add(ctx, rows, n, k):
+    rng = np.random.default_rng(rows + n + k)
+    A, W = rng.standard_normal((rows, k)), bf16w(rng, n, k)
+    want = rounded(A, "bfloat16") @ W.T.astype(np.float64)
+    for ld_out in (n, (n + 3) // 4 * 4 + 4):
+        old = rng.standard_normal((rows, ld_out)).astype(np.float32)
+        got = gemm(ctx, "bfloat16", STORE, A, W, out_f32=old, ld_out=ld_out, cols=n)["out_f32"]
+        close_to(got[:, :n], want, "float32", factor=2)
+        assert np.array_equal(got[:, n:], old[:, n:])
+        added = gemm(ctx, "bfloat16", ADD, A, W, out_f32=old, ld_out=ld_out, cols=n)["out_f32"]
+        assert np.array_equal(added[:, :n], old[:, :n] + got[:, :n])       # one addition, whichever way the results are written
+        assert np.array_equal(added[:, n:], old[:, n:])
+
+
+@pytest.mark.parametrize("rows,ff,k", [(65, 64, 64), (129, 1024, 352), (300, 72, 128), (700, 1024, 96), (1300, 1504, 160), (4096, 1024, 64)])
+def test_tiles_gated_pairs(ctx, rows, ff, k):
+    """The first 32 columns plain, then pairs of tiles of gate and up."""
+    rng = np.random.default_rng(rows + ff)
+    tiles = (ff + 15) // 16
+    gate, up, plain = (bf16w(rng, m, k, 2.0) for m in (tiles * 16, tiles * 16, 32))
+    W = np.concatenate([plain] + [np.concatenate([gate[i * 16:i * 16 + 16], up[i * 16:i * 16 + 16]]) for i in range(tiles)])
+    A = rng.standard_normal((rows, k))
+    a = rounded(A, "bfloat16")
+    want = ld.gelu_tanh(a @ gate.T.astype(np.float64)) * (a @ up.T.astype(np.float64))
+    ld_act = up32(tiles * 16)
+    out = gemm(ctx, "bfloat16", PROJECT, A, W, out_f32=np.zeros((rows, 32), np.float32), ld_out=32, out_act=np.zeros((rows + 15) // 16 * 16 * ld_act, np.uint16), ld_act=ld_act,
+               plain_tiles=2, cols=W.shape[0])
+    close_to(out["out_f32"], a @ plain.T.astype(np.float64), "float32", factor=2)
+    got = (unpack_tiles(out["out_act"], rows, ld_act).astype(np.uint32) << 16).view(np.float32)[:, :tiles * 16]
+    assert (np.abs(got - want) <= 2.0 ** -8 * np.abs(want) + 1e-5 * np.abs(want).max()).all()      # one rounding to 8 bits, and f32 sums
