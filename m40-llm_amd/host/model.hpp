@@ -18,6 +18,7 @@
 //   mode 1 "fused": single decode stream, fused entry points (m40llm_ext_*), device-side greedy.
 #pragma once
 
+#include <algorithm>
 #include <chrono>
 #include <cmath>
 #include <cstdint>
@@ -672,9 +673,15 @@ public:
             M40H_TRY(m40llm_ext_batched_norm_gemm_f32xf16_async(ctx_, d_x, out_norm_, cfg_.norm_weight_dtype, cfg_.rms_eps, lm_head_, d_logits, rows,
                                                                 (int)cfg_.vocab, (int)cfg_.d_model));
     }
+    // device state of a batched run, one buffer (in u32s): slot ids per layer, lengths, {0, steps} and per-row step counters, first tokens
+    struct BatchTable {
+        size_t slots, lens, state, tokens, size;
+        BatchTable(uint32_t layers, uint32_t rows) : slots(0), lens((size_t)layers * rows), state(lens + rows), tokens(state + 2 + rows), size(tokens + rows) {}
+    };
     void enqueue_batched_step(uint32_t rows, uint32_t hint, float* hidden, float* other) {
-        const uint32_t* slots = static_cast<const uint32_t*>(bslots_.ptr());
-        uint32_t* lens = static_cast<uint32_t*>(blens_.ptr());
+        const BatchTable t(cfg_.n_layers, rows);
+        const uint32_t* slots = btable_.u32(t.slots);
+        uint32_t* lens = btable_.u32(t.lens);
         const uint32_t group = fused_group(rows);
         for (uint32_t r0 = 0; r0 < rows; r0 += group) {
             const uint32_t n = rows - r0 < group ? rows - r0 : group;
@@ -687,8 +694,7 @@ public:
             batched_logits_fused(a, n, ws_.logits.f32((size_t)r0 * cfg_.vocab));
         }
         M40H_TRY(m40llm_ext_batched_greedy_step_async(ctx_, ws_.logits.ptr(), rows, cfg_.vocab,
-                                                      static_cast<uint32_t*>(bstate_.ptr()), lens,
-                                                      static_cast<uint32_t*>(bids_.ptr()), static_cast<float*>(bgaps_.ptr()),
+                                                      btable_.u32(t.state), lens, bpicks_.u32(), bpicks_.f32((size_t)rows * bpicks_steps_),
                                                       tok_emb_, cfg_.d_model, hidden));
     }
     // One decode step for `rows` sequences (token r at position kv_lens[r] of sequence seq_ids[r]) with the logits of
@@ -789,25 +795,28 @@ public:
             if (seq_ids[r] >= cfg_.max_sequences) throw std::out_of_range("sequence id out of range");
             max_len = kv_lens[r] > max_len ? kv_lens[r] : max_len;
         }
+        for (uint32_t r = 0; r < rows; ++r)
+            if (first_tokens[r] >= cfg_.vocab) throw std::out_of_range("token id out of range");
         ensure_workspace(rows);
-        // device state: slot ids per layer, lengths, per-row step counters, picks and gaps
-        std::vector<uint32_t> slots((size_t)cfg_.n_layers * rows);
+        const BatchTable t(cfg_.n_layers, rows);
+        std::vector<uint32_t> table(t.size, 0);
         for (uint32_t l = 0; l < cfg_.n_layers; ++l)
-            for (uint32_t r = 0; r < rows; ++r) slots[(size_t)l * rows + r] = kv_slot(seq_ids[r], l);
-        std::vector<uint32_t> state(2 + rows, 0);
-        state[1] = total;
+            for (uint32_t r = 0; r < rows; ++r) table[t.slots + (size_t)l * rows + r] = kv_slot(seq_ids[r], l);
+        std::copy(kv_lens, kv_lens + rows, table.begin() + t.lens);
+        table[t.state + 1] = total;
+        std::copy(first_tokens, first_tokens + rows, table.begin() + t.tokens);
         sync_all();
-        drop_batch_graph();
-        bslots_ = DeviceBuf(ctx_, slots.size() * 4); blens_ = DeviceBuf(ctx_, (size_t)rows * 4);
-        bstate_ = DeviceBuf(ctx_, state.size() * 4);
-        bids_ = DeviceBuf(ctx_, (size_t)rows * total * 4); bgaps_ = DeviceBuf(ctx_, (size_t)rows * total * 4);
-        M40H_TRY(m40llm_memcpy_h2d(ctx_, bslots_.ptr(), slots.data(), slots.size() * 4));
-        M40H_TRY(m40llm_memcpy_h2d(ctx_, blens_.ptr(), kv_lens, (size_t)rows * 4));
-        M40H_TRY(m40llm_memcpy_h2d(ctx_, bstate_.ptr(), state.data(), state.size() * 4));
+        drop_batch_graph();       // it holds pointers into the buffers below
+        const size_t picks = (size_t)rows * total;        // ids, then gaps
+        if (btable_.bytes() < t.size * 4) btable_ = DeviceBuf(ctx_, t.size * 4);
+        if (bpicks_.bytes() < picks * 8) bpicks_ = DeviceBuf(ctx_, picks * 8);
+        bpicks_steps_ = total;
+        M40H_TRY(m40llm_memcpy_h2d(ctx_, btable_.ptr(), table.data(), t.size * 4));
         float* hidden = ws_.scratch_a.f32();
         float* other = ws_.scratch_b.f32();
-        for (uint32_t r = 0; r < rows; ++r) embed(first_tokens[r], hidden + (size_t)r * cfg_.d_model);
-        M40H_TRY(m40llm_stream_wait_for_stream(ctx_, M40LLM_STREAM_DECODE, M40LLM_STREAM_PREFILL));
+        for (uint32_t r = 0; r < rows; r += 65535u)
+            M40H_TRY(m40llm_ext_embed_rows_async(ctx_, tok_emb_, btable_.u32(t.tokens + r), std::min(rows - r, 65535u), cfg_.vocab, cfg_.d_model,
+                                                 hidden + (size_t)r * cfg_.d_model));
         auto run = [&](uint32_t first_step, uint32_t n_steps) {
             uint32_t done = 0;
             while (done < n_steps) {
@@ -815,10 +824,14 @@ public:
                 const uint32_t hint = len_hint_for(longest);                // >= longest + 1
                 uint32_t n = n_steps - done;
                 if (hint < cfg_.max_seq_len && longest + n > hint) n = hint - longest;
-                if (mode_ >= 2) {
-                    if (!bgraph_ || bgraph_rows_ != rows || bgraph_hint_ != hint || bgraph_ws_generation_ != ws_.generation) {
-                        drop_batch_graph();
-                        M40H_TRY(m40llm_stream_synchronize(ctx_, M40LLM_STREAM_DECODE));
+                uint32_t i = 0;
+                if (mode_ >= 2 && (!bgraph_ || bgraph_rows_ != rows || bgraph_hint_ != hint || bgraph_ws_generation_ != ws_.generation)) {
+                    if (bgraph_) M40H_TRY(m40llm_stream_synchronize(ctx_, M40LLM_STREAM_DECODE));
+                    drop_batch_graph();
+                    // the first step goes out launch by launch: the GPU works on it while the host records the graph for those after it
+                    enqueue_batched_step(rows, hint, hidden, other);
+                    i = 1;
+                    if (n > 1) {
                         M40H_TRY(m40llm_cuda_graph_begin_capture(ctx_, M40LLM_STREAM_DECODE));
                         try {
                             enqueue_batched_step(rows, hint, hidden, other);
@@ -829,9 +842,10 @@ public:
                         M40H_TRY(m40llm_cuda_graph_end_capture(ctx_, M40LLM_STREAM_DECODE, &bgraph_));
                         bgraph_rows_ = rows; bgraph_hint_ = hint; bgraph_ws_generation_ = ws_.generation;
                     }
-                    for (uint32_t i = 0; i < n; ++i) M40H_TRY(m40llm_cuda_graph_launch(ctx_, bgraph_, M40LLM_STREAM_DECODE));
-                } else {
-                    for (uint32_t i = 0; i < n; ++i) enqueue_batched_step(rows, hint, hidden, other);
+                }
+                for (; i < n; ++i) {
+                    if (mode_ >= 2) M40H_TRY(m40llm_cuda_graph_launch(ctx_, bgraph_, M40LLM_STREAM_DECODE));
+                    else enqueue_batched_step(rows, hint, hidden, other);
                 }
                 done += n;
             }
@@ -843,10 +857,12 @@ public:
         sync_all();
         const auto t1 = std::chrono::steady_clock::now();
         if (elapsed_ms) *elapsed_ms = std::chrono::duration<double, std::milli>(t1 - t0).count();
-        std::vector<float> gaps((size_t)rows * total);
-        M40H_TRY(m40llm_memcpy_d2h(ctx_, ids_out, bids_.ptr(), (size_t)rows * total * 4));
-        M40H_TRY(m40llm_memcpy_d2h(ctx_, gaps.data(), bgaps_.ptr(), gaps.size() * 4));
-        drop_batch_graph();       // the graph holds pointers into the per-call state buffers
+        std::vector<uint32_t> out(2 * picks);
+        M40H_TRY(m40llm_memcpy_d2h(ctx_, out.data(), bpicks_.ptr(), out.size() * 4));
+        drop_batch_graph();
+        std::copy(out.begin(), out.begin() + picks, ids_out);
+        std::vector<float> gaps(picks);
+        if (picks) std::memcpy(gaps.data(), out.data() + picks, picks * 4);
         bool ok = true;
         for (size_t i = 0; i < gaps.size(); ++i) {
             if (gaps_out) gaps_out[i] = gaps[i];
@@ -1079,7 +1095,8 @@ private:
     DeviceBuf top2_;
     static constexpr uint32_t kTop2Capacity = 1u << 16;
     uint32_t state_cap_ = 0;
-    DeviceBuf bslots_, blens_, bstate_, bids_, bgaps_;
+    DeviceBuf btable_, bpicks_;      // of a batched run (BatchTable; ids and gaps, bpicks_steps_ a row); grown, and kept for the next run
+    uint32_t bpicks_steps_ = 0;
     DeviceBuf tick_table_;
     size_t tick_table_cap_ = 0;
     M40llmCudaGraphExec* bgraph_ = nullptr;
