@@ -410,6 +410,12 @@ int m40llm_ext_prefill_gemm_fused_async(M40llmCudaContext* ctx, uint32_t source_
                                         int n_mats, const void* d_B0_f16, int N0, void* d_C0_f32, const void* d_R0_f32,
                                         const void* d_B1_f16, int N1, void* d_C1_f32, const void* d_B2_f16, int N2,
                                         void* d_C2_f32, uint32_t stream_kind);
+/* Gate and up projection of the packed prefill with the norm before and SwiGLU after them: d_hid_f32 [M][N] has the bits that
+ * m40llm_ext_prefill_gemm_fused_async (source_kind 1, the two matrices, f16 GGUF [N][K]) and m40llm_swiglu_f32 over its results give where
+ * both take the same tiles and parts of K; the two products are never written out.  Returns as that call (1 also when N is not a multiple of 16). */
+int m40llm_ext_prefill_norm_gate_up_swiglu_async(M40llmCudaContext* ctx, const void* d_a_f32, const void* d_norm_weight, uint32_t norm_weight_dtype,
+                                                 float eps, int M, int K, const void* d_gate_f16, const void* d_up_f16, int N, void* d_hid_f32,
+                                                 uint32_t stream_kind);
 /* embedding rows of `rows` (<= 65535) token ids held on the device (f16 table [vocab][d_model]) -> f32 [rows][d_model];
  * the row form of m40llm_ext_embed_token_dev_async (src/infer/forward.rs:2241-2250 loads them one blocking call per
  * token).  Decode stream. */

@@ -658,7 +658,24 @@ int m40llm_ext_prefill_gemm_fused_async(M40llmCudaContext* ctx, uint32_t source_
     if (source_kind == 2u) tiled = tiled && m40_aligned16(d_a2_f32);
     if (!tiled) return 1;
     return m40_launch_gemm_tiled_fused(ctx, stream, stream_kind, (int)source_kind, A, static_cast<const float*>(d_a2_f32),
-                                       d_norm_weight, norm_weight_dtype, eps, M, K, n_mats, B, N, C, R);
+                                       d_norm_weight, norm_weight_dtype, eps, M, K, n_mats, B, N, C, R, false);
+}
+
+int m40llm_ext_prefill_norm_gate_up_swiglu_async(M40llmCudaContext* ctx, const void* d_a_f32, const void* d_norm_weight, uint32_t norm_weight_dtype,
+                                                 float eps, int M, int K, const void* d_gate_f16, const void* d_up_f16, int N, void* d_hid_f32,
+                                                 uint32_t stream_kind) {
+    if (!ctx || !d_a_f32 || !d_norm_weight || !d_gate_f16 || !d_up_f16 || !d_hid_f32) return -1;
+    if (M <= 0 || K <= 0 || N <= 0 || norm_weight_dtype > 1u) return -2;
+    if (m40_ensure_device(ctx) != 0) return -2;
+    hipStream_t stream = m40_select_stream(ctx, stream_kind);
+    if (!stream) return -3;
+    const float* A = static_cast<const float*>(d_a_f32);
+    const uint16_t* B[2] = {static_cast<const uint16_t*>(d_gate_f16), static_cast<const uint16_t*>(d_up_f16)};
+    const int Ns[2] = {N, N};
+    float* const C[2] = {static_cast<float*>(d_hid_f32), nullptr};
+    if (N % 16 != 0 || N > 0x3fffffff || !m40_aligned16(d_norm_weight) || !m40_gemm_tiled_supported(A, B[0], M, N, K) || !m40_gemm_tiled_supported(A, B[1], M, N, K))
+        return 1;
+    return m40_launch_gemm_tiled_fused(ctx, stream, stream_kind, 1, A, nullptr, d_norm_weight, norm_weight_dtype, eps, M, K, 2, B, Ns, C, nullptr, true);
 }
 
 int m40llm_ext_gemm_f32xf16_gguf_f32_async(M40llmCudaContext* ctx, const void* d_A_f32, const void* d_B_f16,

@@ -33,6 +33,9 @@ struct TiledMats {
     const float* R[kMaxMats];       // not null: C = R + product (R may be C itself)
     int N[kMaxMats];
     int tile_start[kMaxMats + 1];   // first column tile of each matrix; [n] = total
+    // B[0] and B[1] are gate and up of N[0] / 2 columns each (a multiple of 16), taken 16 columns at a time in turn as one matrix of N[0];
+    // C[0], half as wide, gets SwiGLU of the two: [M][N[0] / 2]
+    int pair;
 };
 
 // Where the rows of A come from: as they are, RMSNorm of the rows (what m40llm_rms_norm_f32_weighted writes: the same
@@ -266,8 +269,9 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_tiled_kernel(const _Float16*
     TileWalk at = tile_walk(mats, (M + BM - 1) / BM, k_splits, band, BM, BN);
     at.m0 = __builtin_amdgcn_readfirstlane(at.m0); at.n0 = __builtin_amdgcn_readfirstlane(at.n0);      // the same in every lane: divisions leave them in vector registers
     at.mat = __builtin_amdgcn_readfirstlane(at.mat); at.split = __builtin_amdgcn_readfirstlane(at.split);
-    const uint16_t* __restrict__ B = mats.B[at.mat];
     const int N = mats.N[at.mat], m0 = at.m0, n0 = at.n0;
+    // in a pair a wave's rows of a load are one matrix's: 16 rows of 64 bytes or 8 of 128, four times as far on with the next load
+    const uint16_t* __restrict__ B = mats.B[mats.pair ? (wave >> (KS - 1)) & 1 : at.mat];
     // loader: thread -> row lrow (+ kLoadRows i) of a plane and a 16-byte place in that row's bytes, which holds the row's chunk of that number
     // xor-ed with bits of the row: the fragment reads of rows that share banks fall into different ones
     auto swizzle = [](int row) { return KS == 1 ? (row >> 2) & 3 : row & 7; };
@@ -277,7 +281,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_tiled_kernel(const _Float16*
     // a scalar address that walks K, and per lane a 32-bit offset from it that does not change
     const uint8_t* hi_base = reinterpret_cast<const uint8_t*>(A_hi + (size_t)m0 * K + (size_t)stage0 * (kBK * KS));
     const uint8_t* lo_base = reinterpret_cast<const uint8_t*>(A_lo + (size_t)m0 * K + (size_t)stage0 * (kBK * KS));
-    const uint8_t* b_base = reinterpret_cast<const uint8_t*>(B + (size_t)n0 * K + (size_t)stage0 * (kBK * KS));
+    const uint8_t* b_base = reinterpret_cast<const uint8_t*>(B + (size_t)(mats.pair ? n0 / 2 : n0) * K + (size_t)stage0 * (kBK * KS));
     uint32_t a_off[AL], b_off[BL];
 #pragma unroll
     for (int i = 0; i < AL; ++i) {
@@ -286,8 +290,8 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_tiled_kernel(const _Float16*
     }
 #pragma unroll
     for (int i = 0; i < BL; ++i) {
-        const int c = lrow + kLoadRows * i;
-        b_off[i] = (uint32_t)(n0 + c < N ? c : N - 1 - n0) * (uint32_t)K * 2u + gchunk * 16u;
+        const int c = lrow + kLoadRows * i, last = mats.pair ? N / 2 - 1 - n0 / 2 : N - 1 - n0, col = mats.pair ? c / 32 * 16 + c % 16 : c;
+        b_off[i] = (uint32_t)(col < last ? col : last) * (uint32_t)K * 2u + gchunk * 16u;
     }
     // one instruction of a wave fills a contiguous kilobyte of a plane, lane by lane
     auto issue = [&](int buf, int stage) __attribute__((always_inline)) {
@@ -466,6 +470,31 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_tiled_kernel(const _Float16*
             }
         }
     };
+    if (mats.pair) {
+        const int half = N / 2, pair_col0 = (n0 + wn * NT * 16) / 2 + 4 * (lane >> 4);
+        const bool whole_pair = m40_aligned16(C);
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+            const int row = m0 + (wm * MT + mt) * 16 + frag_row;
+            if (row >= M) continue;
+#pragma unroll
+            for (int nt = 0; nt < NT; nt += 2) {
+                const int col = pair_col0 + nt * 8;
+                if (col >= half) continue;
+                floatx4 v;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) v[r] = tiled_swiglu(acc[mt][nt][r] * scale[mt], acc[mt][nt + 1][r] * scale[mt]);
+                float* o = C + (size_t)row * half + col;
+                if (whole_pair) {
+                    *reinterpret_cast<floatx4*>(o) = v;
+                } else {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) o[r] = v[r];
+                }
+            }
+        }
+        return;
+    }
     if (R) store_tile(std::true_type{});
     else store_tile(std::false_type{});
 }
@@ -499,9 +528,9 @@ int launch_tiles(hipStream_t stream, const _Float16* hi, const _Float16* lo, con
 // Parts of K cost the launch that adds their sums; K 5632 at 256 rows: 35.9 us whole, 24.7 us in two.
 struct TileChoice { int shape, k_splits; };
 constexpr struct { int bm, bn; float least, start, load; } kShapes[4] = {
-    {128, 256, 0.66f, 0.64f, 0.28f}, {128, 128, 0.44f, 0.42f, 0.10f}, {64, 128, 0.28f, 0.25f, 0.05f}, {64, 64, 0.235f, 0.17f, 0.03f}};
-// The two large tiles add up all of their part of K in one chain: where small grids are cut (may_split) they are taken for four parts only (K 2048 is
-// where a chain's error shows: 64 steps and more).  The two small tiles, which add up blocks of k, are for small grids and for one row of tiles; past
+    {128, 256, 0.66f, 0.62f, 0.28f}, {128, 128, 0.44f, 0.38f, 0.20f}, {64, 128, 0.28f, 0.25f, 0.05f}, {64, 64, 0.235f, 0.17f, 0.03f}};
+// The two large tiles add up all of their part of K in one chain: in small grids they are taken for four parts only (K 2048 is where a chain's error
+// shows: 64 steps and more).  The two small tiles, which add up blocks of k, are for small grids and for one row of tiles; past
 // that the larger ones are faster (above, 1030 rows), and a row's sums do not depend on how many rows come with it.
 TileChoice pick_tile(int M, int n_mats, const int* N, int steps, int num_cus, bool small_grid, bool may_split) {
     TileChoice best{1, may_split && steps >= 64 ? 4 : 1};        // what is left for a small grid of an odd number of steps
@@ -517,6 +546,7 @@ TileChoice pick_tile(int M, int n_mats, const int* N, int steps, int num_cus, bo
             const int stage = c >= 2 ? 2 : 1, per = (steps / stage + s - 1) / s * stage;
             if (s > 1 && (!may_split || per < 16 || (long long)per * (s - 1) >= steps || tiles * (s - 1) >= num_cus)) break;
             if (c < 2 && may_split && s < 4 && per >= 32) continue;
+            if (c < 2 && small_grid && !may_split && steps >= 64 && steps % 2 == 0) continue;
             const long long units = (tiles * s + num_cus - 1) / num_cus;
             const float a = kShapes[c].start * (float)units + kShapes[c].load * (float)(tiles * s) / (float)num_cus;
             float us = (float)per * (a > kShapes[c].least ? a : kShapes[c].least);
@@ -564,15 +594,15 @@ bool m40_gemm_tiled_supported(const void* A, const void* B, int M, int N, int K)
 // too small, or the allocation fails): the caller then uses another kernel.
 int m40_launch_gemm_tiled_fused(M40llmCudaContext* ctx, hipStream_t stream, uint32_t stream_kind, int source_kind, const float* A,
                                 const float* A2, const void* norm_w, uint32_t norm_dtype, float eps, int M, int K, int n_mats,
-                                const uint16_t* const* B, const int* N, float* const* C, const float* const* R) {
-    if (!ctx || stream_kind > 1u || n_mats < 1 || n_mats > kMaxMats || source_kind < kPackPlain || source_kind > kPackSwiglu) return -2;
+                                const uint16_t* const* B, const int* N, float* const* C, const float* const* R, bool pair) {
+    if (!ctx || (pair && (n_mats != 2 || N[0] != N[1] || N[0] % 16 != 0 || N[0] > 0x3fffffff || R)) || stream_kind > 1u || n_mats < 1 || n_mats > kMaxMats || source_kind < kPackPlain || source_kind > kPackSwiglu) return -2;
     if (source_kind == kPackSwiglu && (!A2 || !m40_aligned16(A2))) return -2;
     if (source_kind == kPackNorm && (!norm_w || norm_dtype > 1u || !m40_aligned16(norm_w))) return -2;
     TiledMats mats{};
     mats.n = n_mats;
     long long tiles_128 = 0;
     for (int i = 0; i < n_mats; ++i) {
-        if (!m40_gemm_tiled_supported(A, B[i], M, N[i], K) || !C[i]) return -2;
+        if (!m40_gemm_tiled_supported(A, B[i], M, N[i], K) || !(C[i] || (pair && i == 1))) return -2;
         mats.B[i] = B[i];
         mats.C[i] = C[i];
         mats.R[i] = R ? R[i] : nullptr;
@@ -593,7 +623,10 @@ int m40_launch_gemm_tiled_fused(M40llmCudaContext* ctx, hipStream_t stream, uint
         out_floats += (size_t)M * N[i];
     }
     const bool small_grid = (M + 127) / 128 * tiles_128 <= ctx->num_cus / 2;
-    const TileChoice choice = pick_tile(M, n_mats, N, K / kBK, ctx->num_cus, small_grid, small_grid && n4_ok);
+    const int pair_n = pair ? 2 * N[0] : 0;
+    if (pair && small_grid && K / kBK % 2 != 0) return 1;
+    if (pair) { mats.pair = 1; mats.n = 1; mats.N[0] = pair_n; }
+    const TileChoice choice = pick_tile(M, mats.n, pair ? &pair_n : N, K / kBK, ctx->num_cus, small_grid, small_grid && n4_ok && !pair);
     const int k_splits = choice.k_splits;
     const size_t scale_bytes = ((size_t)M * 4 + 15) & ~(size_t)15;
     const size_t need = (size_t)M * K * 4 + scale_bytes + (k_splits > 1 ? (size_t)k_splits * out_floats * 4 : 0);
@@ -661,7 +694,7 @@ int m40_launch_gemm_tiled_fused(M40llmCudaContext* ctx, hipStream_t stream, uint
 
 int m40_launch_gemm_tiled_multi(M40llmCudaContext* ctx, hipStream_t stream, uint32_t stream_kind, const float* A, int M, int K,
                                 int n_mats, const uint16_t* const* B, const int* N, float* const* C) {
-    return m40_launch_gemm_tiled_fused(ctx, stream, stream_kind, kPackPlain, A, nullptr, nullptr, 0u, 0.0f, M, K, n_mats, B, N, C, nullptr);
+    return m40_launch_gemm_tiled_fused(ctx, stream, stream_kind, kPackPlain, A, nullptr, nullptr, 0u, 0.0f, M, K, n_mats, B, N, C, nullptr, false);
 }
 
 int m40_launch_gemm_tiled(M40llmCudaContext* ctx, hipStream_t stream, uint32_t stream_kind, const float* A, const uint16_t* B,

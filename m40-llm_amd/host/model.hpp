@@ -451,8 +451,8 @@ public:
         std::vector<uint32_t> slots(batch);
         const uint32_t* d_off = pws_.offsets.u32();
         const uint32_t* d_len = pws_.lens.u32();
-        // Every launch of a layer goes to the prefill stream: RMSNorm and SwiGLU are produced inside the GEMMs' packing
-        // pass and the residual adds inside their last step (m40llm_ext_prefill_gemm_fused_async), so a layer is four
+        // Every launch of a layer goes to the prefill stream: RMSNorm is produced inside the GEMMs' packing pass, SwiGLU and the
+        // residual adds inside their last step (m40llm_ext_prefill_gemm_fused_async), so a layer is four
         // projections, the RoPE + append launch and the attention, with no hop between streams.
         for (uint32_t l = 0; l < cfg_.n_layers; ++l) {
             const LayerWeights& w = layers_[l];
@@ -470,10 +470,18 @@ public:
                                                                                    pws_.att.ptr()));
             prefill_project(0, pws_.att.f32(), nullptr, nullptr, nullptr, rows, D, 1, w.wo, D, pws_.x1.f32(), nullptr, 0, nullptr, nullptr, 0,
                             nullptr, a);
-            prefill_project(1, pws_.x1.f32(), nullptr, w.ffn_norm, pws_.xn.f32(), rows, D, 2, w.wgate, F, pws_.gate.f32(), w.wup, F,
-                            pws_.up.f32(), nullptr, 0, nullptr, nullptr);
-            prefill_project(2, pws_.gate.f32(), pws_.up.f32(), nullptr, pws_.hid.f32(), rows, F, 1, w.wdown, D, b, nullptr, 0, nullptr, nullptr,
-                            0, nullptr, pws_.x1.f32());
+            const int gated = m40llm_ext_prefill_norm_gate_up_swiglu_async(ctx_, pws_.x1.ptr(), w.ffn_norm, cfg_.norm_weight_dtype, cfg_.rms_eps, (int)rows,
+                                                                           (int)D, w.wgate, w.wup, (int)F, pws_.hid.ptr(), PRE);
+            if (gated == 0) {
+                prefill_project(0, pws_.hid.f32(), nullptr, nullptr, nullptr, rows, F, 1, w.wdown, D, b, nullptr, 0, nullptr, nullptr, 0, nullptr,
+                                pws_.x1.f32());
+            } else {
+                if (gated != 1) M40H_TRY(gated);
+                prefill_project(1, pws_.x1.f32(), nullptr, w.ffn_norm, pws_.xn.f32(), rows, D, 2, w.wgate, F, pws_.gate.f32(), w.wup, F,
+                                pws_.up.f32(), nullptr, 0, nullptr, nullptr);
+                prefill_project(2, pws_.gate.f32(), pws_.up.f32(), nullptr, pws_.hid.f32(), rows, F, 1, w.wdown, D, b, nullptr, 0, nullptr, nullptr,
+                                0, nullptr, pws_.x1.f32());
+            }
             std::swap(a, b);
         }
         M40H_TRY(m40llm_stream_synchronize(ctx_, PRE));

@@ -33,3 +33,38 @@ def test_many_rows_tiles_vs_float64(dev, M, N, K):
     err = np.abs(got - A.astype(np.float64) @ B64.T)
     i = int(np.argmax(err / bound))
     assert (err <= bound).all(), (i // N, i % N, float(err.flat[i]), float(bound.flat[i]))
+
+
+@pytest.mark.parametrize("norm_dtype", [0, 1])
+@pytest.mark.parametrize("M,F,K", [(33, 16, 64), (65, 48, 128), (100, 5632, 2048), (129, 1024, 320), (300, 5632, 256), (522, 272, 2048), (1030, 2816, 96), (2049, 1040, 160)])
+def test_gate_up_swiglu_equals_separate_calls(dev, M, F, K, norm_dtype):
+    rng = np.random.default_rng(M + F + K)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    x[2] *= 1e-4
+    w = (1.0 + 0.1 * rng.standard_normal(K)).astype(np.float32)
+    dw, dx = dev.up(w if norm_dtype else f16bits(w)), dev.up(x)
+    gate, up = (f16bits(rng.standard_normal((F, K)) * 0.05) for _ in range(2))
+    dg, du = dev.up(gate), dev.up(up)
+    g, u, want, got = (dev.zeros(M * F * 4) for _ in range(4))
+    dev.call("m40llm_ext_prefill_gemm_fused_async", 1, dx.ptr, None, dw.ptr, norm_dtype, 1e-5, M, K, 2, dg.ptr, F, g.ptr, None, du.ptr, F, u.ptr, None, 0, None, 0)
+    dev.sync()
+    dev.call("m40llm_swiglu_f32_async", g.ptr, u.ptr, want.ptr, M * F)
+    dev.sync()
+    dev.call("m40llm_ext_prefill_norm_gate_up_swiglu_async", dx.ptr, dw.ptr, norm_dtype, 1e-5, M, K, dg.ptr, du.ptr, F, got.ptr, 0)
+    dev.sync()
+    want, got = want.download(np.float32, (M, F)), got.download(np.float32, (M, F))
+    if (M + 127) // 128 * ((F + 127) // 128) * 2 > 128:        # larger grids are cut nowhere: the same sums
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+    # otherwise the two may add k in other blocks: two products of about sqrt(K) roundings each, relative to their own size
+    assert (np.abs(got - want) <= 2.0 ** -22 * np.sqrt(K) * (np.abs(want) + np.abs(want).max())).all()
+
+
+def test_gate_up_swiglu_declines_and_checks(dev):
+    M, K, F = 64, 64, 48
+    x, w, b, o = dev.zeros(M * K * 4), dev.zeros(K * 4), dev.zeros(F * K * 2), dev.zeros(M * F * 4)
+    name = "m40llm_ext_prefill_norm_gate_up_swiglu_async"
+    dev.call(name, x.ptr, w.ptr, 1, 1e-5, 32, K, b.ptr, b.ptr, F, o.ptr, 0, expect=1)           # few rows
+    dev.call(name, x.ptr, w.ptr, 1, 1e-5, M, K, b.ptr, b.ptr, 40, o.ptr, 0, expect=1)           # columns in no groups of 16
+    dev.call(name, x.ptr, w.ptr, 1, 1e-5, M, 32, b.ptr, b.ptr, F, o.ptr, 0, expect=1)           # a small grid, an odd number of steps
+    dev.call(name, x.ptr, None, 1, 1e-5, M, K, b.ptr, b.ptr, F, o.ptr, 0, expect=-1)
+    dev.call(name, x.ptr, w.ptr, 2, 1e-5, M, K, b.ptr, b.ptr, F, o.ptr, 0, expect=-2)
