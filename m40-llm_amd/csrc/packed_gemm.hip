@@ -38,7 +38,7 @@ template <class T, int MT, int NT, int WAVES, int JOBS>
 __global__ __launch_bounds__(WAVES * 64) void rows_packed_kernel(PackedArgs g, M40Epilogue<T> e) {
     extern __shared__ __align__(16) float red[];       // [WAVES][MT][NT][64][4]
     typedef typename M40Act<T>::vec8 vec8;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int tile0 = (int)blockIdx.x * NT;
     int row0 = (int)blockIdx.y * 16 * MT, batch = blockIdx.z;
     if (JOBS != kAllRows) {
@@ -68,35 +68,28 @@ __global__ __launch_bounds__(WAVES * 64) void rows_packed_kernel(PackedArgs g, M
     for (int m = 0; m < MT; ++m)
 #pragma unroll
         for (int n = 0; n < NT; ++n) acc[m][n] = m40_float4{0.f, 0.f, 0.f, 0.f};
+    // A wave's next U k tiles are requested together, also where fewer are left (K 2048 over 16 waves is four): one by one each would cost a
+    // round trip to memory.
     constexpr int U = sizeof(T) == 2 ? (MT * NT <= 2 ? 8 : 4) : 1;
-    int k = wave;
-    for (; k + (U - 1) * WAVES < k_tiles; k += U * WAVES) {
+    for (int k = wave; k < k_tiles; k += U * WAVES) {
         uint4 wf[U][NT];
         vec8 af[U][MT];
+        const int left = (k_tiles - k + WAVES - 1) / WAVES;
 #pragma unroll
-        for (int u = 0; u < U; ++u)
+        for (int u = 0; u < U; ++u) {
+            if (u >= left) break;
 #pragma unroll
             for (int n = 0; n < NT; ++n) wf[u][n] = m40_load_stream(reinterpret_cast<const uint4*>(w[n] + (long)(k + u * WAVES) * kM40Tile));
 #pragma unroll
-        for (int u = 0; u < U; ++u)
-#pragma unroll
             for (int m = 0; m < MT; ++m) af[u][m] = M40Act<T>::load8(a[m] + (long)(k + u * WAVES) * kStep);
+        }
 #pragma unroll
-        for (int u = 0; u < U; ++u)
+        for (int u = 0; u < U; ++u) {
+            if (u >= left) break;
 #pragma unroll
             for (int m = 0; m < MT; ++m)
 #pragma unroll
                 for (int n = 0; n < NT; ++n) acc[m][n] = M40Act<T>::mma(__builtin_bit_cast(m40_bf16x8, wf[u][n]), af[u][m], acc[m][n]);
-    }
-    for (; k < k_tiles; k += WAVES) {
-        uint4 wf[NT];
-#pragma unroll
-        for (int n = 0; n < NT; ++n) wf[n] = *reinterpret_cast<const uint4*>(w[n] + (long)k * kM40Tile);
-#pragma unroll
-        for (int m = 0; m < MT; ++m) {
-            const vec8 af = M40Act<T>::load8(a[m] + (long)k * kStep);
-#pragma unroll
-            for (int n = 0; n < NT; ++n) acc[m][n] = M40Act<T>::mma(__builtin_bit_cast(m40_bf16x8, wf[n]), af, acc[m][n]);
         }
     }
     m40_float4* r4 = reinterpret_cast<m40_float4*>(red);
@@ -136,11 +129,36 @@ int launch_rows(hipStream_t stream, const PackedArgs& g, const M40Epilogue<T>& e
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 
+// Waves and column tiles of a workgroup, bf16: a launch is mostly the round trips of its requests, so as many waves share out K as let every
+// workgroup have its place at once (32 waves a CU).  From four single tiles a CU on (two rows' worth of tiles: from one), tiles go in pairs, which
+// read the rows once.  Weights that no cache holds, one row, 16 / 8 / 4 waves of one tile, 8 / 4 of two, us:
+//   K 2048: 128 tiles 5.0 / 5.7 / 7.6 / - / -, 256 tiles 5.3 / 6.0 / 8.0 / 6.9 / 8.6, 384 tiles 8.1 / 7.4 / 8.8 / 7.5 / 9.1, 644 tiles
+//   11.4 / 12.3 / 10.0 / 11.2 / 10.7, 1024 tiles 16.1 / 14.6 / 13.2 / 13.3 / 12.7, 2000 tiles 29.1 / 26.2 / 25.0 / 22.3 / 22.2
+//   K 1408: 256 tiles 4.4 / 5.1 / 6.3, 768 tiles 9.8 / 10.1 / 8.2;  gate and up in pairs, 352 of them: 16 / 8 / 4 waves 13.2 / 11.3 / 10.9
+// and 64 rows: 192 tiles 8.5 / 8.7 / 9.1 / 10.4 / 11.2, 384 tiles 15.0 / 14.0 / 14.1 / 11.1 / 11.7, 2000 tiles 56 / 48 / 47 / 37 / 33.
 template <class T, int MT, int JOBS>
-int launch_rows_m(hipStream_t stream, const PackedArgs& g, const M40Epilogue<T>& e, int batches) {
+int launch_rows_m(hipStream_t stream, const PackedArgs& g, const M40Epilogue<T>& e, int batches, int num_cus) {
+    // jobs: as many as there can be
+    const long long tiles = (long long)g.n_tiles * (JOBS == kAllRows ? (long long)((g.rows + 16 * MT - 1) / (16 * MT)) * batches : g.rows);
     if constexpr (JOBS != kJobSlots)
-        if (e.kind == M40LLM_PACKED_PROJECT) return launch_rows<T, MT, 2, 8, JOBS>(stream, g, e, batches);
+        if (e.kind == M40LLM_PACKED_PROJECT) {
+            if constexpr (sizeof(T) == 2)
+                if (tiles > 2ll * num_cus) return launch_rows<T, MT, 2, 4, JOBS>(stream, g, e, batches);
+            return launch_rows<T, MT, 2, 8, JOBS>(stream, g, e, batches);
+        }
     if constexpr (JOBS != kJobGather) {
+        if constexpr (sizeof(T) == 2) {
+            if (g.k_tiles >= 16) {
+                if (tiles <= num_cus) return launch_rows<T, MT, 1, 16, JOBS>(stream, g, e, batches);
+                if constexpr (JOBS == kAllRows)
+                    if (tiles >= (MT == 1 ? 4ll : 1ll) * num_cus) {
+                        if (tiles <= 2ll * num_cus) return launch_rows<T, MT, 2, 8, JOBS>(stream, g, e, batches);
+                        return launch_rows<T, MT, 2, 4, JOBS>(stream, g, e, batches);
+                    }
+                if (tiles <= 2ll * num_cus) return launch_rows<T, MT, 1, 8, JOBS>(stream, g, e, batches);
+                return launch_rows<T, MT, 1, 4, JOBS>(stream, g, e, batches);
+            }
+        }
         if (g.k_tiles >= 64) return launch_rows<T, MT, 1, 16, JOBS>(stream, g, e, batches);
         if (g.k_tiles >= 16) return launch_rows<T, MT, 1, 8, JOBS>(stream, g, e, batches);
         return launch_rows<T, MT, 1, 4, JOBS>(stream, g, e, batches);
@@ -148,10 +166,10 @@ int launch_rows_m(hipStream_t stream, const PackedArgs& g, const M40Epilogue<T>&
     return -3;
 }
 template <class T, int JOBS>
-int launch_rows_any(hipStream_t stream, const PackedArgs& g, const M40Epilogue<T>& e, int batches, int rows) {
-    if (rows <= 16) return launch_rows_m<T, 1, JOBS>(stream, g, e, batches);
-    if (rows <= 32) return launch_rows_m<T, 2, JOBS>(stream, g, e, batches);
-    return launch_rows_m<T, 4, JOBS>(stream, g, e, batches);
+int launch_rows_any(hipStream_t stream, const PackedArgs& g, const M40Epilogue<T>& e, int batches, int rows, int num_cus) {
+    if (rows <= 16) return launch_rows_m<T, 1, JOBS>(stream, g, e, batches, num_cus);
+    if (rows <= 32) return launch_rows_m<T, 2, JOBS>(stream, g, e, batches, num_cus);
+    return launch_rows_m<T, 4, JOBS>(stream, g, e, batches, num_cus);
 }
 
 // ---- many rows, bf16 ---------------------------------------------------------------------------------------------------
@@ -591,21 +609,21 @@ int m40llm_ext_packed_gemm_async(M40llmCudaContext* ctx, const M40llmPackedGemm*
         const int rows = (int)p->job_rows;
         if (p->act_dtype == M40LLM_ACT_F32) {
             const M40Epilogue<float> e = make_epilogue<float>(*p);
-            return p->gather ? launch_rows_any<float, kJobGather>(stream, g, e, 1, rows) : launch_rows_any<float, kJobSlots>(stream, g, e, 1, rows);
+            return p->gather ? launch_rows_any<float, kJobGather>(stream, g, e, 1, rows, ctx->num_cus) : launch_rows_any<float, kJobSlots>(stream, g, e, 1, rows, ctx->num_cus);
         }
         const M40Epilogue<m40_bf16> e = make_epilogue<m40_bf16>(*p);
         if (rows == 128) return launch_tile_any<kSlots>(stream, g, e, 1, ctx->num_cus);
-        return p->gather ? launch_rows_any<m40_bf16, kJobGather>(stream, g, e, 1, rows) : launch_rows_any<m40_bf16, kJobSlots>(stream, g, e, 1, rows);
+        return p->gather ? launch_rows_any<m40_bf16, kJobGather>(stream, g, e, 1, rows, ctx->num_cus) : launch_rows_any<m40_bf16, kJobSlots>(stream, g, e, 1, rows, ctx->num_cus);
     }
     if (p->act_dtype == M40LLM_ACT_F32) {
         if ((g.rows + 63) / 64 > 65535) return -3;
-        return launch_rows_any<float, kAllRows>(stream, g, make_epilogue<float>(*p), batches, g.rows);
+        return launch_rows_any<float, kAllRows>(stream, g, make_epilogue<float>(*p), batches, g.rows, ctx->num_cus);
     }
     const M40Epilogue<m40_bf16> e = make_epilogue<m40_bf16>(*p);
     if (p->epilogue == M40LLM_PACKED_KEYS) return launch_tile_any<kPageKeys>(stream, g, e, batches, ctx->num_cus);
     if (p->epilogue == M40LLM_PACKED_VALUES) return launch_tile_any<kPageValues>(stream, g, e, batches, ctx->num_cus);
     // few columns leave most CUs without a wide tile
-    if (g.rows <= 64 || (g.n_tiles <= 8 && batches == 1 && g.rows <= 65535 * 16 && p->epilogue != M40LLM_PACKED_PROJECT)) return launch_rows_any<m40_bf16, kAllRows>(stream, g, e, batches, g.rows);
+    if (g.rows <= 64 || (g.n_tiles <= 8 && batches == 1 && g.rows <= 65535 * 16 && p->epilogue != M40LLM_PACKED_PROJECT)) return launch_rows_any<m40_bf16, kAllRows>(stream, g, e, batches, g.rows, ctx->num_cus);
     return launch_tile_any<kPlainRows>(stream, g, e, batches, ctx->num_cus);
 }
 

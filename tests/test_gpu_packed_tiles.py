@@ -31,7 +31,21 @@ def test_tiles_store_and_add(ctx, rows, n, k):
         assert np.array_equal(added[:, n:], old[:, n:])
 
 
-@pytest.mark.parametrize("rows,ff,k", [(65, 64, 64), (129, 1024, 352), (300, 72, 128), (700, 1024, 96), (1300, 1504, 160), (4096, 1024, 64)])
+# few rows: 16, 8 and 4 waves a tile and pairs of tiles (an odd last one); k tiles that no wave count divides, fewer than a wave's batch, more than one
+@pytest.mark.parametrize("rows,n,k", [(1, 4096, 544), (3, 4100, 512), (5, 8200, 2080), (16, 16390, 512), (16, 16400, 1408), (17, 4000, 2048), (30, 4112, 608), (32, 8230, 992),
+                                      (33, 4097, 3000), (64, 8210, 1100), (2, 2048, 5632), (1, 12304, 768)])
+def test_few_rows_waves_and_pairs(ctx, rows, n, k):
+    rng = np.random.default_rng(rows + n + k)
+    A, W = rng.standard_normal((rows, k)), bf16w(rng, n, k)
+    want = rounded(A, "bfloat16") @ W.T.astype(np.float64)
+    ld_out = (n + 3) // 4 * 4 + 4
+    old = rng.standard_normal((rows, ld_out)).astype(np.float32)
+    got = gemm(ctx, "bfloat16", STORE, A, W, out_f32=old, ld_out=ld_out, cols=n)["out_f32"]
+    close_to(got[:, :n], want, "float32", factor=2)
+    assert np.array_equal(got[:, n:], old[:, n:])
+
+
+@pytest.mark.parametrize("rows,ff,k", [(1, 4112, 512), (20, 4200, 352), (65, 64, 64), (129, 1024, 352), (300, 72, 128), (700, 1024, 96), (1300, 1504, 160), (4096, 1024, 64)])
 def test_tiles_gated_pairs(ctx, rows, ff, k):
     """The first 32 columns plain, then pairs of tiles of gate and up."""
     rng = np.random.default_rng(rows + ff)
