@@ -421,6 +421,10 @@ int m40llm_ext_prefill_norm_gate_up_swiglu_async(M40llmCudaContext* ctx, const v
  * token).  Decode stream. */
 int m40llm_ext_embed_rows_async(M40llmCudaContext* ctx, const void* d_table_f16, const uint32_t* tokens_dev, uint32_t rows,
                                 uint32_t vocab, uint32_t d_model, void* d_out_f32);
+/* the last rows of `rows` (<= 65535) packed sequences: d_out_f32 [i] = d_x_f32 [offsets_dev[i] + lens_dev[i] - 1] (lens >= 1), f32 rows of `cols`.
+ * Decode stream. */
+int m40llm_ext_last_rows_f32_async(M40llmCudaContext* ctx, const void* d_x_f32, const uint32_t* offsets_dev, const uint32_t* lens_dev, uint32_t rows,
+                                   uint32_t cols, void* d_out_f32);
 /* Weight-file ingestion: `num_bytes` of the file at `path`, from byte `file_offset`, into one new device allocation
  * (*out_device_ptr, released with m40llm_device_free).  Replaces read-the-file + m40llm_upload_weights
  * (src/infer/load.rs:27-40, kernels.cu:1264-1290): positional reads into two pinned staging buffers overlap the

@@ -437,6 +437,13 @@ __global__ __launch_bounds__(1024) void greedy_step_kernel(const float* __restri
 
 bool fast_ok(const void* a, const void* b, int K) { return K % 8 == 0 && m40_aligned16(a) && m40_aligned16(b); }
 
+// rows offsets[i] + lens[i] - 1 of x, in order (bound: the launch)
+__global__ __launch_bounds__(kThreads) void last_rows_kernel(const float* __restrict__ x, const uint32_t* __restrict__ offsets, const uint32_t* __restrict__ lens,
+                                                             uint32_t cols, float* __restrict__ out) {
+    const uint32_t i = blockIdx.y, c = blockIdx.x * kThreads + threadIdx.x;
+    if (c < cols) out[(size_t)i * cols + c] = x[((size_t)offsets[i] + lens[i] - 1u) * cols + c];
+}
+
 }  // namespace
 
 extern "C" {
@@ -568,6 +575,16 @@ int m40llm_ext_embed_rows_async(M40llmCudaContext* ctx, const void* d_table_f16,
     (void)hipGetLastError();
     embed_token_dev_kernel<<<dim3((d_model + kThreads - 1) / kThreads, rows), kThreads, 0, ctx->decode_stream>>>(
         static_cast<const uint16_t*>(d_table_f16), tokens_dev, vocab, d_model, static_cast<float*>(d_out_f32));
+    return hipGetLastError() == hipSuccess ? 0 : -3;
+}
+
+int m40llm_ext_last_rows_f32_async(M40llmCudaContext* ctx, const void* d_x_f32, const uint32_t* offsets_dev, const uint32_t* lens_dev, uint32_t rows,
+                                   uint32_t cols, void* d_out_f32) {
+    if (!ctx || !d_x_f32 || !offsets_dev || !lens_dev || !d_out_f32) return -1;
+    if (rows == 0 || rows > 65535u || cols == 0) return -2;
+    (void)hipGetLastError();
+    last_rows_kernel<<<dim3((cols + kThreads - 1) / kThreads, rows), kThreads, 0, ctx->decode_stream>>>(static_cast<const float*>(d_x_f32), offsets_dev, lens_dev, cols,
+                                                                                                        static_cast<float*>(d_out_f32));
     return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 

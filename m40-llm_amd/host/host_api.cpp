@@ -426,14 +426,7 @@ int m40host_model_forward_prefill(M40HostModel* m, const uint32_t* seq_ids, cons
             if (!m || !seq_ids || !lens || !tokens) throw std::invalid_argument("null argument");
             DecodeModel& d = m->dense();
             const float* h = d.forward_prefill(seq_ids, lens, tokens, batch);
-            const size_t D = d.config().d_model, V = d.config().vocab;
-            size_t row = 0;
-            for (uint32_t i = 0; i < batch; ++i) {
-                row += lens[i];
-                const float* last = h + (row - 1) * D;
-                if (hidden_last_host) M40H_TRY(m40llm_memcpy_d2h(d.ctx(), hidden_last_host + i * D, last, D * 4));
-                if (logits_last_host) d.logits_from_hidden(last, logits_last_host + i * V);
-            }
+            d.last_rows(h, lens, batch, hidden_last_host, logits_last_host);
             return 0;
         },
         -100);

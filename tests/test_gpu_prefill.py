@@ -156,6 +156,33 @@ def test_forward_prefill_matches_token_by_token_oracle_and_decode_continues(dev,
     dm.close()
 
 
+@pytest.mark.parametrize("n", [2, 8, 9, 32, 33])
+def test_last_rows_of_many_prompts_equal_each_prompt_alone(dev, n):
+    """Logits of n prompts through the output norm and lm_head together (groups of up to 32 rows, kernels for up to 8) against one by one."""
+    cfg = dict(n_layers=1, d_model=256, q_heads=4, kv_heads=2, head_dim=64, ffn=512, vocab=1003, rms_eps=1e-5, rope_base=10000.0, rope_scale=1.0, rope_layout=0, qkv_bias=False)
+    dm = syn.DeviceModel(dev.ctx, cfg, syn.make_weights(cfg, seed=2, std=0.08, emb_std=1.0), max_seq_len=48, max_sequences=n)
+    rng = np.random.default_rng(n)
+    prompts = [rng.integers(0, 1003, size=1 + (7 * i + n) % 40).tolist() for i in range(n)]
+    apart = dm.forward_prefill(list(range(n)), prompts)             # mode 0: row by row
+    dm.set_mode(2)
+    hid, log = dm.forward_prefill(list(range(n)), prompts)
+    assert np.array_equal(np.asarray(hid), np.asarray(apart[0]))
+    # 256 products a logit: exact splits to 2^-22 and f32 sums
+    close(log, apart[1], 1e-5, 1e-5 * float(np.abs(apart[1]).max()))
+    dm.close()
+
+
+def test_last_rows_gather(dev):
+    rng = np.random.default_rng(3)
+    x = rng.standard_normal((50, 333)).astype(np.float32)
+    lens, offsets = u32([5, 1, 30, 14]), u32([0, 5, 6, 36])
+    dx, dl, do, out = dev.up(x), dev.up(lens), dev.up(offsets), dev.zeros(4 * 333 * 4)
+    dev.call("m40llm_ext_last_rows_f32_async", dx.ptr, do.ptr, dl.ptr, 4, 333, out.ptr)
+    dev.sync()
+    assert np.array_equal(out.download(np.float32, (4, 333)), x[offsets + lens - 1])
+    dev.call("m40llm_ext_last_rows_f32_async", dx.ptr, do.ptr, dl.ptr, 0, 333, out.ptr, expect=-2)
+
+
 def _f16(a):
     return np.ascontiguousarray(np.asarray(a, dtype=np.float32).astype(np.float16).view(np.uint16))
 
