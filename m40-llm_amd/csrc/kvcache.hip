@@ -99,37 +99,67 @@ __global__ __launch_bounds__(kThreads) void prefill_rope_append_kernel(
     const size_t ept = (size_t)kv_heads * head_dim;
     uint16_t* k_out = k_base + ((size_t)slot * max_seq_len + position) * ept;
     uint16_t* v_out = v_base + ((size_t)slot * max_seq_len + position) * ept;
-    for (uint32_t idx = threadIdx.x; idx < q_pairs + kv_pairs; idx += kThreads) {
-        const bool is_q = idx < q_pairs;
-        const uint32_t p = is_q ? idx : idx - q_pairs;
-        const uint32_t off = p % half_dim, head = p / half_dim;
-        size_t i0, i1;
-        m40_rope_pair(head, off, head_dim, layout, &i0, &i1);
+    // A row's angles are the same for every head: worked out once.  A thread's elements are requested together, ahead of the angles (bound: the
+    // round trips at few rows, the stream of q at many; 36 heads of 64, 522 rows: 6.2 us; 7.3 us with the angles and the
+    // requests one pair at a time).
+    __shared__ float2 angles[kThreads];
+    auto angle = [&](uint32_t off) {
         const float f = inv_freq_table ? inv_freq_table[off] : m40_rope_inv_freq(off, head_dim, freq_base);
-        const float2 cs = m40_rope_cos_sin_freq(position, f, freq_scale);
-        float* x = is_q ? q_row : k_row;
-        const float* bias = is_q ? bq : bk;
-        float x0 = x[i0], x1 = x[i1];
-        if (bias) {   // the bias add of the per-row sequence (forward.rs:149-160), before the rotation
-            x0 = x0 + bias[i0];
-            x1 = x1 + bias[i1];
-        }
-        float y0, y1;
-        m40_rope_apply(cs, x0, x1, &y0, &y1);
-        x[i0] = y0;
-        x[i1] = y1;
-        if (!is_q) {
-            float v0 = v_row[i0], v1 = v_row[i1];
-            if (bv) {
-                v0 = v0 + bv[i0];
-                v1 = v1 + bv[i1];
-                v_row[i0] = v0;
-                v_row[i1] = v1;
+        return m40_rope_cos_sin_freq(position, f, freq_scale);
+    };
+    const bool tabled = half_dim <= kThreads;
+    constexpr uint32_t kBatch = 5;
+    for (uint32_t base = 0; base < q_pairs + kv_pairs; base += kBatch * kThreads) {
+        float x0[kBatch], x1[kBatch], v0[kBatch], v1[kBatch];
+        size_t i0[kBatch], i1[kBatch];
+#pragma unroll
+        for (uint32_t u = 0; u < kBatch; ++u) {
+            const uint32_t idx = base + u * kThreads + threadIdx.x;
+            if (idx >= q_pairs + kv_pairs) continue;
+            const bool is_q = idx < q_pairs;
+            const uint32_t p = is_q ? idx : idx - q_pairs;
+            m40_rope_pair(p / half_dim, p % half_dim, head_dim, layout, &i0[u], &i1[u]);
+            const float* x = is_q ? q_row : k_row;
+            x0[u] = x[i0[u]];
+            x1[u] = x[i1[u]];
+            if (!is_q) {
+                v0[u] = v_row[i0[u]];
+                v1[u] = v_row[i1[u]];
             }
-            k_out[i0] = m40_f2h(y0);
-            k_out[i1] = m40_f2h(y1);
-            v_out[i0] = m40_f2h(v0);
-            v_out[i1] = m40_f2h(v1);
+        }
+        if (base == 0 && tabled) {
+            if (threadIdx.x < half_dim) angles[threadIdx.x] = angle(threadIdx.x);
+            __syncthreads();
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < kBatch; ++u) {
+            const uint32_t idx = base + u * kThreads + threadIdx.x;
+            if (idx >= q_pairs + kv_pairs) continue;
+            const bool is_q = idx < q_pairs;
+            const uint32_t off = (is_q ? idx : idx - q_pairs) % half_dim;
+            const float2 cs = tabled ? angles[off] : angle(off);
+            float* x = is_q ? q_row : k_row;
+            const float* bias = is_q ? bq : bk;
+            if (bias) {   // the bias add of the per-row sequence (forward.rs:149-160), before the rotation
+                x0[u] = x0[u] + bias[i0[u]];
+                x1[u] = x1[u] + bias[i1[u]];
+            }
+            float y0, y1;
+            m40_rope_apply(cs, x0[u], x1[u], &y0, &y1);
+            x[i0[u]] = y0;
+            x[i1[u]] = y1;
+            if (!is_q) {
+                if (bv) {
+                    v0[u] = v0[u] + bv[i0[u]];
+                    v1[u] = v1[u] + bv[i1[u]];
+                    v_row[i0[u]] = v0[u];
+                    v_row[i1[u]] = v1[u];
+                }
+                k_out[i0[u]] = m40_f2h(y0);
+                k_out[i1[u]] = m40_f2h(y1);
+                v_out[i0[u]] = m40_f2h(v0[u]);
+                v_out[i1[u]] = m40_f2h(v1[u]);
+            }
         }
     }
     if (threadIdx.x == 0 && local + 1u == t.len[s]) seq_map[slot] = position + 1u;

