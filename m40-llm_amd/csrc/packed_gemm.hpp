@@ -65,6 +65,18 @@ __device__ __forceinline__ void m40_wait_and_meet() {
     __builtin_amdgcn_sched_barrier(0);
     asm volatile("" ::: "memory");
 }
+// Issue order of a phase of READS operand reads from LDS, each for PER matrix instructions: the reads run four ahead of their instructions
+// (left to itself the compiler waits for each).  No branch may stand inside the phase.
+template <int READS, int PER>
+__device__ __forceinline__ void m40_fragments_ahead() {
+    __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+#pragma unroll
+    for (int i = 0; i < READS - 4; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, PER, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x008, 4 * PER, 0);
+}
 // Workgroup b of a launch over rows: workgroups are dealt to the eight dies in turn, and the rows of a 16-row tile go to one die so
 // that its L2 puts their pieces of the tile's lines together.
 __device__ __forceinline__ uint32_t m40_tile_row(uint32_t b, uint32_t rows) {
