@@ -34,9 +34,14 @@ struct PackedArgs {
 
 enum { kAllRows = 0, kJobSlots = 1, kJobGather = 2 };
 
-template <class T, int MT, int NT, int WAVES, int JOBS>
+constexpr int rows_at_once(int mt, int nt, int waves, int parts) { return parts * mt * nt <= 16 ? parts / waves : 1; }
+
+// The k tiles of a product are added up as PARTS sums (k tile i in sum i % PARTS, the sums in order), PARTS following from K alone: WAVES, which
+// follows from the launch's size, divides it and changes no bit of the result.
+template <class T, int MT, int NT, int WAVES, int PARTS, int JOBS>
 __global__ __launch_bounds__(WAVES * 64) void rows_packed_kernel(PackedArgs g, M40Epilogue<T> e) {
-    extern __shared__ __align__(16) float red[];       // [WAVES][MT][NT][64][4]
+    extern __shared__ __align__(16) float red[];       // [sums at once][MT][NT][64][4]
+    constexpr int kOwn = PARTS / WAVES;                // sums a wave keeps
     typedef typename M40Act<T>::vec8 vec8;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int tile0 = (int)blockIdx.x * NT;
@@ -63,14 +68,17 @@ __global__ __launch_bounds__(WAVES * 64) void rows_packed_kernel(PackedArgs g, M
         w[n] = g.w + batch * g.w_batch + (long)t * g.k_stride * kM40Tile + lane * 8;
     }
     const int k_tiles = g.k_count(batch);
-    m40_float4 acc[MT][NT];
+    m40_float4 acc[kOwn][MT][NT];
 #pragma unroll
-    for (int m = 0; m < MT; ++m)
+    for (int q = 0; q < kOwn; ++q)
 #pragma unroll
-        for (int n = 0; n < NT; ++n) acc[m][n] = m40_float4{0.f, 0.f, 0.f, 0.f};
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (int n = 0; n < NT; ++n) acc[q][m][n] = m40_float4{0.f, 0.f, 0.f, 0.f};
     // A wave's next U k tiles are requested together, also where fewer are left (K 2048 over 16 waves is four): one by one each would cost a
     // round trip to memory.
     constexpr int U = sizeof(T) == 2 ? (MT * NT <= 2 ? 8 : 4) : 1;
+    static_assert(PARTS % WAVES == 0 && U % kOwn == 0);
     for (int k = wave; k < k_tiles; k += U * WAVES) {
         uint4 wf[U][NT];
         vec8 af[U][MT];
@@ -89,53 +97,77 @@ __global__ __launch_bounds__(WAVES * 64) void rows_packed_kernel(PackedArgs g, M
 #pragma unroll
             for (int m = 0; m < MT; ++m)
 #pragma unroll
-                for (int n = 0; n < NT; ++n) acc[m][n] = M40Act<T>::mma(__builtin_bit_cast(m40_bf16x8, wf[u][n]), af[u][m], acc[m][n]);
+                for (int n = 0; n < NT; ++n) acc[u % kOwn][m][n] = M40Act<T>::mma(__builtin_bit_cast(m40_bf16x8, wf[u][n]), af[u][m], acc[u % kOwn][m][n]);
         }
     }
     m40_float4* r4 = reinterpret_cast<m40_float4*>(red);
+    static_assert(MT <= WAVES, "a wave adds up one row tile");
+    const int mine = wave < MT ? wave : 0;
+    m40_float4 s[NT];
+    // all sums at once where they take no more memory than eight workgroups a CU have, else a wave's sums one after the other
+    constexpr int kAtOnce = rows_at_once(MT, NT, WAVES, PARTS);
 #pragma unroll
-    for (int m = 0; m < MT; ++m)
+    for (int q = 0; q < kOwn; q += kAtOnce) {
+        if (q > 0) __syncthreads();
 #pragma unroll
-        for (int n = 0; n < NT; ++n) r4[((wave * MT + m) * NT + n) * 64 + lane] = acc[m][n];
-    __syncthreads();
-    for (int m = wave; m < MT; m += WAVES) {
-        if (row0 + m * 16 >= g.rows) continue;
-        m40_float4 s[NT];
+        for (int i = 0; i < kAtOnce; ++i)
 #pragma unroll
-        for (int n = 0; n < NT; ++n) {
-            s[n] = r4[(m * NT + n) * 64 + lane];
+            for (int m = 0; m < MT; ++m)
 #pragma unroll
-            for (int i = 1; i < WAVES; ++i) s[n] += r4[((i * MT + m) * NT + n) * 64 + lane];
-        }
-        if (NT == 2 && e.kind == M40LLM_PACKED_PROJECT && tile0 >= e.plain_tiles) {
-            m40_epilogue_pair(e, row0 + m * 16, (tile0 - e.plain_tiles) / 2, lane, s[0], s[NT - 1]);
-        } else {
+                for (int n = 0; n < NT; ++n) r4[(((i * WAVES + wave) * MT + m) * NT + n) * 64 + lane] = acc[q + i][m][n];
+        __syncthreads();
+        if (wave < MT) {
 #pragma unroll
             for (int n = 0; n < NT; ++n)
-                if (tile0 + n < g.n_tiles) m40_epilogue_tile(e, JOBS == kAllRows ? batch : 0, row0 + m * 16, tile0 + n, lane, s[n]);
+#pragma unroll
+                for (int i = 0; i < kAtOnce * WAVES; ++i) {
+                    const m40_float4 v = r4[((i * MT + mine) * NT + n) * 64 + lane];
+                    s[n] = q == 0 && i == 0 ? v : s[n] + v;
+                }
         }
+    }
+    if (wave >= MT || row0 + mine * 16 >= g.rows) return;
+    if (NT == 2 && e.kind == M40LLM_PACKED_PROJECT && tile0 >= e.plain_tiles) {
+        m40_epilogue_pair(e, row0 + mine * 16, (tile0 - e.plain_tiles) / 2, lane, s[0], s[NT - 1]);
+    } else {
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+            if (tile0 + n < g.n_tiles) m40_epilogue_tile(e, JOBS == kAllRows ? batch : 0, row0 + mine * 16, tile0 + n, lane, s[n]);
     }
 }
 
-template <class T, int MT, int NT, int WAVES, int JOBS>
+template <class T, int MT, int NT, int WAVES, int PARTS, int JOBS>
 int launch_rows(hipStream_t stream, const PackedArgs& g, const M40Epilogue<T>& e, int batches) {
     // g.rows: with jobs, the most jobs there can be
     const dim3 grid((unsigned)((g.n_tiles + NT - 1) / NT), (unsigned)(JOBS == kAllRows ? (g.rows + 16 * MT - 1) / (16 * MT) : g.rows), (unsigned)batches);
-    constexpr size_t lds = (size_t)WAVES * MT * NT * 1024;
-    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(rows_packed_kernel<T, MT, NT, WAVES, JOBS>),
+    constexpr size_t lds = (size_t)rows_at_once(MT, NT, WAVES, PARTS) * WAVES * MT * NT * 1024;
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(rows_packed_kernel<T, MT, NT, WAVES, PARTS, JOBS>),
                                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (attr != hipSuccess) return -2;
-    rows_packed_kernel<T, MT, NT, WAVES, JOBS><<<grid, WAVES * 64, lds, stream>>>(g, e);
+    rows_packed_kernel<T, MT, NT, WAVES, PARTS, JOBS><<<grid, WAVES * 64, lds, stream>>>(g, e);
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 
 // Waves and column tiles of a workgroup, bf16: a launch is mostly the round trips of its requests, so as many waves share out K as let every
-// workgroup have its place at once (32 waves a CU).  From four single tiles a CU on (two rows' worth of tiles: from one), tiles go in pairs, which
-// read the rows once.  Weights that no cache holds, one row, 16 / 8 / 4 waves of one tile, 8 / 4 of two, us:
-//   K 2048: 128 tiles 5.0 / 5.7 / 7.6 / - / -, 256 tiles 5.3 / 6.0 / 8.0 / 6.9 / 8.6, 384 tiles 8.1 / 7.4 / 8.8 / 7.5 / 9.1, 644 tiles
-//   11.4 / 12.3 / 10.0 / 11.2 / 10.7, 1024 tiles 16.1 / 14.6 / 13.2 / 13.3 / 12.7, 2000 tiles 29.1 / 26.2 / 25.0 / 22.3 / 22.2
-//   K 1408: 256 tiles 4.4 / 5.1 / 6.3, 768 tiles 9.8 / 10.1 / 8.2;  gate and up in pairs, 352 of them: 16 / 8 / 4 waves 13.2 / 11.3 / 10.9
-// and 64 rows: 192 tiles 8.5 / 8.7 / 9.1 / 10.4 / 11.2, 384 tiles 15.0 / 14.0 / 14.1 / 11.1 / 11.7, 2000 tiles 56 / 48 / 47 / 37 / 33.
+// workgroup have its place at once (32 waves a CU); more than 16 rows take tiles in pairs, which read the rows once.  K 2048, weights that no cache
+// holds, us:
+//   8 rows, 16 / 8 / 4 waves: 192 tiles 5.7 / 6.5 / 8.3, 384 tiles 8.2 / 7.5 / 8.9, 528 tiles 11.3 / 11.7 / 10.3, 644 tiles 11.7 / 13.1 / 10.6, 2000 tiles
+//   29.8 / 27.7 / 25.1;  gate and up in pairs, 352 of them: 13.1 / 13.1 / 11.6
+//   64 rows, 16 waves / pairs and 8 waves / pairs and 4: 192 tiles 8.5 / 11.0 / 12.4, 384 tiles 15.0 / 11.1 / 11.7, 644 tiles 21.8 / 21.1 / 18.8, 2000 tiles
+//   57 / 43 / 36
+template <class T, int MT, int PARTS, int JOBS>
+int launch_rows_parts(hipStream_t stream, const PackedArgs& g, const M40Epilogue<T>& e, int batches, long long tiles, int num_cus) {
+    if constexpr (sizeof(T) == 2) {
+        if constexpr (JOBS == kAllRows)
+            if (MT > 1 && tiles > num_cus) {
+                if (tiles <= 2ll * num_cus) return launch_rows<T, MT, 2, 8, PARTS, JOBS>(stream, g, e, batches);
+                return launch_rows<T, MT, 2, 4, PARTS, JOBS>(stream, g, e, batches);
+            }
+        if (tiles > 2ll * num_cus) return launch_rows<T, MT, 1, 4, PARTS, JOBS>(stream, g, e, batches);
+        if (tiles > num_cus) return launch_rows<T, MT, 1, 8, PARTS, JOBS>(stream, g, e, batches);
+    }
+    return launch_rows<T, MT, 1, PARTS, PARTS, JOBS>(stream, g, e, batches);
+}
 template <class T, int MT, int JOBS>
 int launch_rows_m(hipStream_t stream, const PackedArgs& g, const M40Epilogue<T>& e, int batches, int num_cus) {
     // jobs: as many as there can be
@@ -143,25 +175,13 @@ int launch_rows_m(hipStream_t stream, const PackedArgs& g, const M40Epilogue<T>&
     if constexpr (JOBS != kJobSlots)
         if (e.kind == M40LLM_PACKED_PROJECT) {
             if constexpr (sizeof(T) == 2)
-                if (tiles > 2ll * num_cus) return launch_rows<T, MT, 2, 4, JOBS>(stream, g, e, batches);
-            return launch_rows<T, MT, 2, 8, JOBS>(stream, g, e, batches);
+                if (tiles > 2ll * num_cus) return launch_rows<T, MT, 2, 4, 8, JOBS>(stream, g, e, batches);
+            return launch_rows<T, MT, 2, 8, 8, JOBS>(stream, g, e, batches);
         }
     if constexpr (JOBS != kJobGather) {
-        if constexpr (sizeof(T) == 2) {
-            if (g.k_tiles >= 16) {
-                if (tiles <= num_cus) return launch_rows<T, MT, 1, 16, JOBS>(stream, g, e, batches);
-                if constexpr (JOBS == kAllRows)
-                    if (tiles >= (MT == 1 ? 4ll : 1ll) * num_cus) {
-                        if (tiles <= 2ll * num_cus) return launch_rows<T, MT, 2, 8, JOBS>(stream, g, e, batches);
-                        return launch_rows<T, MT, 2, 4, JOBS>(stream, g, e, batches);
-                    }
-                if (tiles <= 2ll * num_cus) return launch_rows<T, MT, 1, 8, JOBS>(stream, g, e, batches);
-                return launch_rows<T, MT, 1, 4, JOBS>(stream, g, e, batches);
-            }
-        }
-        if (g.k_tiles >= 64) return launch_rows<T, MT, 1, 16, JOBS>(stream, g, e, batches);
-        if (g.k_tiles >= 16) return launch_rows<T, MT, 1, 8, JOBS>(stream, g, e, batches);
-        return launch_rows<T, MT, 1, 4, JOBS>(stream, g, e, batches);
+        if (g.k_tiles >= 64) return launch_rows_parts<T, MT, 16, JOBS>(stream, g, e, batches, tiles, num_cus);
+        if (g.k_tiles >= 16) return launch_rows_parts<T, MT, 8, JOBS>(stream, g, e, batches, tiles, num_cus);
+        return launch_rows<T, MT, 1, 4, 4, JOBS>(stream, g, e, batches);
     }
     return -3;
 }
