@@ -416,6 +416,14 @@ int m40llm_ext_prefill_gemm_fused_async(M40llmCudaContext* ctx, uint32_t source_
 int m40llm_ext_prefill_norm_gate_up_swiglu_async(M40llmCudaContext* ctx, const void* d_a_f32, const void* d_norm_weight, uint32_t norm_weight_dtype,
                                                  float eps, int M, int K, const void* d_gate_f16, const void* d_up_f16, int N, void* d_hid_f32,
                                                  uint32_t stream_kind);
+/* A projection with its residual, and the projections of the norm of its result: d_C0_f32 [M][N0] = R0 + a . B0 (d_a_f32 [M][K0]), then C_i of
+ * RMSNorm(C_0) with one to three matrices [N_i][N0], or with gated = 1 and two matrices SwiGLU of the two into C_1.  The bits are those of
+ * m40llm_ext_prefill_gemm_fused_async (source_kind 0 with R0) followed by the same call with source_kind 1, or by
+ * m40llm_ext_prefill_norm_gate_up_swiglu_async.  Returns as those calls (1: nothing was enqueued). */
+int m40llm_ext_prefill_project_norm_project_async(M40llmCudaContext* ctx, const void* d_a_f32, int M, int K0, const void* d_B0_f16, int N0, const void* d_R0_f32,
+                                                  void* d_C0_f32, const void* d_norm_weight, uint32_t norm_weight_dtype, float eps, uint32_t gated, int n_mats,
+                                                  const void* d_B1_f16, int N1, void* d_C1_f32, const void* d_B2_f16, int N2, void* d_C2_f32,
+                                                  const void* d_B3_f16, int N3, void* d_C3_f32, uint32_t stream_kind);
 /* embedding rows of `rows` (<= 65535) token ids held on the device (f16 table [vocab][d_model]) -> f32 [rows][d_model];
  * the row form of m40llm_ext_embed_token_dev_async (src/infer/forward.rs:2241-2250 loads them one blocking call per
  * token).  Decode stream. */

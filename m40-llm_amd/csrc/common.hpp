@@ -174,6 +174,10 @@ int m40_launch_gemm_tiled_multi(M40llmCudaContext* ctx, hipStream_t stream, uint
 int m40_launch_gemm_tiled_fused(M40llmCudaContext* ctx, hipStream_t stream, uint32_t stream_kind, int source_kind, const float* A,
                                 const float* A2, const void* norm_w, uint32_t norm_dtype, float eps, int M, int K, int n_mats,
                                 const uint16_t* const* B, const int* N, float* const* C, const float* const* R, bool pair);
+// C0 [M][N0] = R0 + A [M][K0] . B0, and the products of RMSNorm(C0) with one to three matrices (pair: as above); 1 as above, nothing enqueued
+int m40_launch_gemm_tiled_chain(M40llmCudaContext* ctx, hipStream_t stream, uint32_t stream_kind, const float* A, int M, int K0, const uint16_t* B0, int N0,
+                                const float* R0, float* C0, const void* norm_w, uint32_t norm_dtype, float eps, int n_mats, const uint16_t* const* B,
+                                const int* N, float* const* C, bool pair);
 bool m40_skinny_supported(const M40llmCudaContext* ctx, uint32_t stream_kind, int M, int N, int K, int fmt);
 int m40_launch_skinny(M40llmCudaContext* ctx, hipStream_t stream, uint32_t stream_kind, int fmt, const float* A,
                       const float* up, const void* W0, float* C0, const void* W1, float* C1, int M, int N, int K);

@@ -678,6 +678,32 @@ int m40llm_ext_prefill_norm_gate_up_swiglu_async(M40llmCudaContext* ctx, const v
     return m40_launch_gemm_tiled_fused(ctx, stream, stream_kind, 1, A, nullptr, d_norm_weight, norm_weight_dtype, eps, M, K, 2, B, Ns, C, nullptr, true);
 }
 
+int m40llm_ext_prefill_project_norm_project_async(M40llmCudaContext* ctx, const void* d_a_f32, int M, int K0, const void* d_B0_f16, int N0, const void* d_R0_f32,
+                                                  void* d_C0_f32, const void* d_norm_weight, uint32_t norm_weight_dtype, float eps, uint32_t gated, int n_mats,
+                                                  const void* d_B1_f16, int N1, void* d_C1_f32, const void* d_B2_f16, int N2, void* d_C2_f32,
+                                                  const void* d_B3_f16, int N3, void* d_C3_f32, uint32_t stream_kind) {
+    if (!ctx || !d_a_f32 || !d_B0_f16 || !d_R0_f32 || !d_C0_f32 || !d_norm_weight) return -1;
+    if (M <= 0 || K0 <= 0 || N0 <= 0 || n_mats < 1 || n_mats > 3 || norm_weight_dtype > 1u || gated > 1u || (gated && (n_mats != 2 || N1 != N2))) return -2;
+    const uint16_t* B[3] = {static_cast<const uint16_t*>(d_B1_f16), static_cast<const uint16_t*>(d_B2_f16), static_cast<const uint16_t*>(d_B3_f16)};
+    float* C[3] = {static_cast<float*>(d_C1_f32), static_cast<float*>(d_C2_f32), static_cast<float*>(d_C3_f32)};
+    const int N[3] = {N1, N2, N3};
+    for (int i = 0; i < n_mats; ++i) {
+        if (!B[i] || (!C[i] && !(gated && i == 1))) return -1;
+        if (N[i] <= 0) return -2;
+    }
+    if (m40_ensure_device(ctx) != 0) return -2;
+    hipStream_t stream = m40_select_stream(ctx, stream_kind);
+    if (!stream) return -3;
+    const float* A = static_cast<const float*>(d_a_f32);
+    const uint16_t* B0 = static_cast<const uint16_t*>(d_B0_f16);
+    float* C0 = static_cast<float*>(d_C0_f32);
+    bool tiled = m40_gemm_tiled_supported(A, B0, M, N0, K0) && m40_aligned16(d_norm_weight) && (!gated || (N1 % 16 == 0 && N1 <= 0x3fffffff));
+    for (int i = 0; i < n_mats && tiled; ++i) tiled = m40_gemm_tiled_supported(C0, B[i], M, N[i], N0);
+    if (!tiled) return 1;
+    return m40_launch_gemm_tiled_chain(ctx, stream, stream_kind, A, M, K0, B0, N0, static_cast<const float*>(d_R0_f32), C0, d_norm_weight, norm_weight_dtype, eps,
+                                       n_mats, B, N, C, gated != 0u);
+}
+
 int m40llm_ext_gemm_f32xf16_gguf_f32_async(M40llmCudaContext* ctx, const void* d_A_f32, const void* d_B_f16,
                                            void* d_C_f32, int M, int N, int K, uint32_t stream_kind) {
     if (!ctx || !d_A_f32 || !d_B_f16 || !d_C_f32) return -1;

@@ -454,11 +454,13 @@ public:
         // Every launch of a layer goes to the prefill stream: RMSNorm is produced inside the GEMMs' packing pass, SwiGLU and the
         // residual adds inside their last step (m40llm_ext_prefill_gemm_fused_async), so a layer is four
         // projections, the RoPE + append launch and the attention, with no hop between streams.
+        bool have_qkv = false;
         for (uint32_t l = 0; l < cfg_.n_layers; ++l) {
             const LayerWeights& w = layers_[l];
             for (uint32_t i = 0; i < batch; ++i) slots[i] = kv_slot(seq_ids[i], l);
-            prefill_project(1, a, nullptr, w.attn_norm, pws_.xn.f32(), rows, D, 3, w.wq, D, pws_.q.f32(), w.wk, KV, pws_.k.f32(), w.wv, KV,
-                            pws_.v.f32(), nullptr);
+            if (!have_qkv)
+                prefill_project(1, a, nullptr, w.attn_norm, pws_.xn.f32(), rows, D, 3, w.wq, D, pws_.q.f32(), w.wk, KV, pws_.k.f32(), w.wv, KV,
+                                pws_.v.f32(), nullptr);
             M40H_TRY(m40llm_ext_prefill_rope_append_on_stream_async(ctx_, kv_, pws_.q.ptr(), pws_.k.ptr(), pws_.v.ptr(), batch, slots.data(),
                                                                     lens, nullptr, cfg_.q_heads, cfg_.rope_base, cfg_.rope_scale,
                                                                     cfg_.rope_layout, cfg_.has_qkv_bias ? w.bq : nullptr,
@@ -468,15 +470,31 @@ public:
                                                                                    d_len, d_len, offsets.data(), lens, lens, batch,
                                                                                    cfg_.q_heads, cfg_.kv_heads, cfg_.head_dim,
                                                                                    pws_.att.ptr()));
-            prefill_project(0, pws_.att.f32(), nullptr, nullptr, nullptr, rows, D, 1, w.wo, D, pws_.x1.f32(), nullptr, 0, nullptr, nullptr, 0,
-                            nullptr, a);
-            const int gated = m40llm_ext_prefill_norm_gate_up_swiglu_async(ctx_, pws_.x1.ptr(), w.ffn_norm, cfg_.norm_weight_dtype, cfg_.rms_eps, (int)rows,
-                                                                           (int)D, w.wgate, w.wup, (int)F, pws_.hid.ptr(), PRE);
-            if (gated == 0) {
+            // O projection, norm, gate and up in one call; the down projection, the next layer's norm and Q/K/V likewise
+            int gated = m40llm_ext_prefill_project_norm_project_async(ctx_, pws_.att.ptr(), (int)rows, (int)D, w.wo, (int)D, a, pws_.x1.ptr(), w.ffn_norm,
+                                                                      cfg_.norm_weight_dtype, cfg_.rms_eps, 1u, 2, w.wgate, (int)F, pws_.hid.ptr(), w.wup, (int)F,
+                                                                      nullptr, nullptr, 0, nullptr, PRE);
+            if (gated != 0) {
+                if (gated != 1) M40H_TRY(gated);
+                prefill_project(0, pws_.att.f32(), nullptr, nullptr, nullptr, rows, D, 1, w.wo, D, pws_.x1.f32(), nullptr, 0, nullptr, nullptr, 0,
+                                nullptr, a);
+                gated = m40llm_ext_prefill_norm_gate_up_swiglu_async(ctx_, pws_.x1.ptr(), w.ffn_norm, cfg_.norm_weight_dtype, cfg_.rms_eps, (int)rows, (int)D,
+                                                                     w.wgate, w.wup, (int)F, pws_.hid.ptr(), PRE);
+                if (gated != 0 && gated != 1) M40H_TRY(gated);
+            }
+            have_qkv = false;
+            if (gated == 0 && l + 1 < cfg_.n_layers) {
+                const LayerWeights& next = layers_[l + 1];
+                const int rc = m40llm_ext_prefill_project_norm_project_async(ctx_, pws_.hid.ptr(), (int)rows, (int)F, w.wdown, (int)D, pws_.x1.ptr(), b,
+                                                                             next.attn_norm, cfg_.norm_weight_dtype, cfg_.rms_eps, 0u, 3, next.wq, (int)D,
+                                                                             pws_.q.ptr(), next.wk, (int)KV, pws_.k.ptr(), next.wv, (int)KV, pws_.v.ptr(), PRE);
+                if (rc != 0 && rc != 1) M40H_TRY(rc);
+                have_qkv = rc == 0;
+            }
+            if (gated == 0 && !have_qkv) {
                 prefill_project(0, pws_.hid.f32(), nullptr, nullptr, nullptr, rows, F, 1, w.wdown, D, b, nullptr, 0, nullptr, nullptr, 0, nullptr,
                                 pws_.x1.f32());
-            } else {
-                if (gated != 1) M40H_TRY(gated);
+            } else if (gated != 0) {
                 prefill_project(1, pws_.x1.f32(), nullptr, w.ffn_norm, pws_.xn.f32(), rows, D, 2, w.wgate, F, pws_.gate.f32(), w.wup, F,
                                 pws_.up.f32(), nullptr, 0, nullptr, nullptr);
                 prefill_project(2, pws_.gate.f32(), pws_.up.f32(), nullptr, pws_.hid.f32(), rows, F, 1, w.wdown, D, b, nullptr, 0, nullptr, nullptr,

@@ -68,3 +68,37 @@ def test_gate_up_swiglu_declines_and_checks(dev):
     dev.call(name, x.ptr, w.ptr, 1, 1e-5, M, 32, b.ptr, b.ptr, F, o.ptr, 0, expect=1)           # a small grid, an odd number of steps
     dev.call(name, x.ptr, None, 1, 1e-5, M, K, b.ptr, b.ptr, F, o.ptr, 0, expect=-1)
     dev.call(name, x.ptr, w.ptr, 2, 1e-5, M, K, b.ptr, b.ptr, F, o.ptr, 0, expect=-2)
+
+
+# the first product whole, in two and in more parts of K; fewer k than columns (the parts would lie under the next product's rows); as gate and up and as Q/K/V
+@pytest.mark.parametrize("M,K0,D,Ns,gated", [(33, 2048, 2048, (1024, 1024), 1), (101, 2048, 2048, (5632, 5632), 1), (101, 5632, 2048, (2048, 256, 256), 0), (250, 11008, 2048, (2048, 256, 256), 0),
+                                             (522, 5632, 2048, (2048, 256, 256), 0), (522, 512, 2048, (272, 272), 1), (1030, 2048, 2048, (2816, 2816), 1), (65, 96, 160, (50,), 0),
+                                             (300, 1024, 64, (48, 33), 0), (40, 4096, 260, (16,), 0)])
+def test_project_norm_project_equals_separate_calls(dev, M, K0, D, Ns, gated):
+    rng = np.random.default_rng(M + K0 + D)
+    x, r = rng.standard_normal((M, K0)).astype(np.float32), rng.standard_normal((M, D)).astype(np.float32)
+    w = (1.0 + 0.1 * rng.standard_normal(D)).astype(np.float32)
+    dx, dr, dw, dB0 = dev.up(x), dev.up(r), dev.up(w), dev.up(f16bits(rng.standard_normal((D, K0)) * 0.05))
+    dB = [dev.up(f16bits(rng.standard_normal((n, D)) * 0.05)) for n in Ns]
+    none = [None, 0, None]
+    supported = K0 % 32 == 0 and D % 32 == 0
+    name = "m40llm_ext_prefill_project_norm_project_async"
+    c0, got = dev.zeros(M * D * 4), [dev.zeros(M * n * 4) for n in Ns]
+    args = sum([[b.ptr, n, o.ptr] for b, n, o in zip(dB, Ns, got)], []) + none * (3 - len(Ns))
+    dev.call(name, dx.ptr, M, K0, dB0.ptr, D, dr.ptr, c0.ptr, dw.ptr, 1, 1e-5, gated, len(Ns), *args, 0, expect=0 if supported else 1)
+    dev.sync()
+    if not supported:
+        return
+    want0, want = dev.zeros(M * D * 4), [dev.zeros(M * n * 4) for n in Ns]
+    fused = "m40llm_ext_prefill_gemm_fused_async"
+    dev.call(fused, 0, dx.ptr, None, None, 0, 1e-5, M, K0, 1, dB0.ptr, D, want0.ptr, dr.ptr, None, 0, None, None, 0, None, 0)
+    if gated:
+        dev.call("m40llm_ext_prefill_norm_gate_up_swiglu_async", want0.ptr, dw.ptr, 1, 1e-5, M, D, dB[0].ptr, dB[1].ptr, Ns[0], want[0].ptr, 0)
+    else:
+        a = sum([[b.ptr, n, o.ptr] + ([None] if i == 0 else []) for i, (b, n, o) in enumerate(zip(dB, Ns, want))], []) + none * (3 - len(Ns))
+        dev.call(fused, 1, want0.ptr, None, dw.ptr, 1, 1e-5, M, D, len(Ns), *a, 0)
+    dev.sync()
+    for n, g, o in [(D, c0, want0)] + list(zip(Ns, got, want)):
+        assert np.array_equal(g.download(np.uint32, (M, n)), o.download(np.uint32, (M, n))), n
+    dev.call(name, dx.ptr, M, K0, dB0.ptr, D, None, c0.ptr, dw.ptr, 1, 1e-5, gated, len(Ns), *args, 0, expect=-1)
+    dev.call(name, dx.ptr, M, K0, dB0.ptr, D, dr.ptr, c0.ptr, dw.ptr, 1, 1e-5, gated, 0, *args, 0, expect=-2)
