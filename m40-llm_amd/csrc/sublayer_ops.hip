@@ -61,7 +61,13 @@ __global__ __launch_bounds__(kThreads) void norm_add_rows_kernel(M40llmNormAdd a
             }
         }
     };
-    float keep[kGroups][8];
+    // a row's old values and the weights, requested ahead of the sums
+    auto old_and_weights = [&](uint32_t g, float (&v)[8], float (&u)[8]) __attribute__((always_inline)) {
+        const uint32_t c = g * 8u < width ? g * 8u : 0u;
+        load_group<float, VEC>(x, c, width, v);
+        load_group<float, VEC>(w, c, width, u);
+    };
+    float keep[kGroups][8], keep_x[kGroups][8], keep_w[kGroups][8];
     float q = 0.0f;
     auto sq8 = [&](const float (&y)[8]) __attribute__((always_inline)) {
 #pragma unroll
@@ -69,6 +75,7 @@ __global__ __launch_bounds__(kThreads) void norm_add_rows_kernel(M40llmNormAdd a
     };
 #pragma unroll
     for (uint32_t j = 0; j < kGroups; ++j) {
+        old_and_weights(threadIdx.x + j * kThreads, keep_x[j], keep_w[j]);
         value(threadIdx.x + j * kThreads, keep[j]);
         sq8(keep[j]);
     }
@@ -78,12 +85,11 @@ __global__ __launch_bounds__(kThreads) void norm_add_rows_kernel(M40llmNormAdd a
         sq8(y);
     }
     const float f = a.mult / sqrtf(block_sum(q, scratch) / (float)width + a.eps);
-    auto finish = [&](uint32_t g, const float (&y)[8]) __attribute__((always_inline)) {
+    auto finish = [&](uint32_t g, const float (&y)[8], const float (&old)[8], const float (&u)[8]) __attribute__((always_inline)) {
         float v[8];
         if (g * 8u < width) {
-            load_group<float, VEC>(x, g * 8u, width, v);
 #pragma unroll
-            for (uint32_t i = 0; i < 8; ++i) v[i] = VEC || g * 8u + i < width ? fmaf(y[i] * f, w[g * 8u + i], v[i]) : 0.0f;
+            for (uint32_t i = 0; i < 8; ++i) v[i] = VEC || g * 8u + i < width ? fmaf(y[i] * f, u[i], old[i]) : 0.0f;
             if (VEC) {
                 reinterpret_cast<float4*>(x + g * 8u)[0] = make_float4(v[0], v[1], v[2], v[3]);
                 reinterpret_cast<float4*>(x + g * 8u)[1] = make_float4(v[4], v[5], v[6], v[7]);
@@ -97,24 +103,19 @@ __global__ __launch_bounds__(kThreads) void norm_add_rows_kernel(M40llmNormAdd a
             for (int i = 0; i < 8; ++i) v[i] = 0.0f;
         }
         const m40_float4 lo = {v[0], v[1], v[2], v[3]}, hi = {v[4], v[5], v[6], v[7]};
-        T* o = static_cast<T*>(a.h) + m40_packed_at(row, g * 8u, a.ld_h >> 5);
-        m40_store4<T>(o, lo);
-        m40_store4<T>(o + 4, hi);
-        if (a.h_rows) {
-            T* r = static_cast<T*>(a.h_rows) + (size_t)row * a.ld_h + g * 8u;
-            m40_store4<T>(r, lo);
-            m40_store4<T>(r + 4, hi);
-        }
+        m40_store8<T>(static_cast<T*>(a.h) + m40_packed_at(row, g * 8u, a.ld_h >> 5), lo, hi);
+        if (a.h_rows) m40_store8<T>(static_cast<T*>(a.h_rows) + (size_t)row * a.ld_h + g * 8u, lo, hi);
     };
 #pragma unroll
     for (uint32_t j = 0; j < kGroups; ++j) {
         const uint32_t g = threadIdx.x + j * kThreads;
-        if (g < groups) finish(g, keep[j]);
+        if (g < groups) finish(g, keep[j], keep_x[j], keep_w[j]);
     }
     for (uint32_t g = threadIdx.x + kGroups * kThreads; g < groups; g += kThreads) {
-        float y[8];
+        float y[8], v[8], u[8];
+        old_and_weights(g, v, u);
         value(g, y);
-        finish(g, y);
+        finish(g, y, v, u);
     }
 }
 
@@ -138,15 +139,14 @@ __global__ __launch_bounds__(kThreads) void norm_gate_rows_kernel(const float* _
 #pragma unroll
         for (int i = 0; i < 8; ++i) v[i] = 0.0f;
         if (g * 8u < cols) {
-            float z[8];
+            float z[8], u[8];
             load_group<float, VEC>(src, g * 8u, cols, v);
             load_group<float, VEC>(gt, g * 8u, cols, z);
+            load_group<float, VEC>(w, g * 8u, cols, u);
 #pragma unroll
-            for (uint32_t i = 0; i < 8; ++i) v[i] = VEC || g * 8u + i < cols ? v[i] * inv * w[g * 8u + i] * m40_sigmoid(z[i]) : 0.0f;
+            for (uint32_t i = 0; i < 8; ++i) v[i] = VEC || g * 8u + i < cols ? v[i] * inv * u[i] * m40_sigmoid(z[i]) : 0.0f;
         }
-        T* o = out + m40_packed_at(row, g * 8u, ld_out >> 5);
-        m40_store4<T>(o, m40_float4{v[0], v[1], v[2], v[3]});
-        m40_store4<T>(o + 4, m40_float4{v[4], v[5], v[6], v[7]});
+        m40_store8<T>(out + m40_packed_at(row, g * 8u, ld_out >> 5), m40_float4{v[0], v[1], v[2], v[3]}, m40_float4{v[4], v[5], v[6], v[7]});
     }
 }
 
@@ -239,7 +239,7 @@ int m40llm_ext_norm_add_rows_async(M40llmCudaContext* ctx, const M40llmNormAdd* 
     if (!stream || m40_ensure_device(ctx) != 0) return -2;
     if (n->rows == 0 || n->width == 0 || n->ld_h < n->width || n->ld_h % 32u != 0 || n->act_dtype > 1u || !m40_aligned16(n->h) || (n->h_rows && !m40_aligned16(n->h_rows)))
         return -3;
-    const bool vec = n->width % 8u == 0 && m40_aligned16(n->x) && (n->place ? n->ld_expert % 8u == 0 && m40_aligned16(n->expert_out) : n->plane_stride % 4u == 0 && m40_aligned16(n->planes));
+    const bool vec = n->width % 8u == 0 && m40_aligned16(n->x) && m40_aligned16(n->w) && (n->place ? n->ld_expert % 8u == 0 && m40_aligned16(n->expert_out) : n->plane_stride % 4u == 0 && m40_aligned16(n->planes));
     if (n->act_dtype == M40LLM_ACT_F32) {
         if (vec) norm_add_rows_kernel<float, true><<<n->rows, kThreads, 0, stream>>>(*n);
         else norm_add_rows_kernel<float, false><<<n->rows, kThreads, 0, stream>>>(*n);
@@ -257,7 +257,7 @@ int m40llm_ext_norm_gate_rows_async(M40llmCudaContext* ctx, const void* d_y, uin
     if (!stream || m40_ensure_device(ctx) != 0) return -2;
     if (rows == 0 || cols == 0 || ld_out < cols || ld_out % 32u != 0 || ld_y < cols || ld_gate < cols || act_dtype > 1u || !m40_aligned16(d_out)) return -3;
     const float *y = static_cast<const float*>(d_y), *w = static_cast<const float*>(d_w), *g = static_cast<const float*>(d_gate);
-    const bool vec = cols % 8u == 0 && ld_y % 4u == 0 && ld_gate % 4u == 0 && m40_aligned16(d_y) && m40_aligned16(d_gate);
+    const bool vec = cols % 8u == 0 && ld_y % 4u == 0 && ld_gate % 4u == 0 && m40_aligned16(d_y) && m40_aligned16(d_gate) && m40_aligned16(d_w);
     auto go = [&](auto kernel, auto* out) { kernel<<<rows, kThreads, 0, stream>>>(y, (size_t)ld_y, w, g, (size_t)ld_gate, rows, cols, eps, out, ld_out); };
     if (act_dtype == M40LLM_ACT_F32) {
         if (vec) go(norm_gate_rows_kernel<float, true>, static_cast<float*>(d_out));

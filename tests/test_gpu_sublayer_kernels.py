@@ -12,8 +12,8 @@ from gulidra_common import od  # noqa: E402
 from pimosun_common import as_act, c_struct, close_to, from_act, ld, m40, pack_tiles, unpack_tiles, up32  # noqa: E402
 from test_gpu_layer_kernels import ACT, DTYPES, PROJECT, STORE_ACT, act_type, bf16w, call, gemm, rounded  # noqa: E402
 
-Embed, NormAdd, Route, Split, Attn, Light, Gemm = (c_struct("M40llm" + n) for n in ("EmbedTokens", "NormAdd", "Route", "PairSplit", "PairAttention",
-                                                                                   "Lightning", "PackedGemm"))
+Embed, NormAdd, Route, Split, Attn, Light, Gemm, Update = (c_struct("M40llm" + n) for n in ("EmbedTokens", "NormAdd", "Route", "PairSplit", "PairAttention",
+                                                                                           "Lightning", "PackedGemm", "StreamUpdate"))
 SILU_KIND, SILU, INPUT, RMS = 8, 1, 0xffffffff, 1
 LONE = 0x80000000
 
@@ -111,6 +111,39 @@ def test_norm_times_gate(ctx, rows, cols, dtype):
     got = from_act(unpack_tiles(out.download(act_type(dtype), ((rows + 15) // 16 * 16 * ldo,)), rows, ldo), dtype)
     close_to(got[:, :cols], od.rms_norm(y, w, 1e-3) * od.sigmoid(z[:, :cols]), dtype)
     assert np.all(got[:, cols:] == 0)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("width", [8, 2048, 4104])
+def test_norm_weights_that_are_not_16_byte_aligned(ctx, width, dtype):
+    """The weights of the row norms are read 16 bytes a load only where they lie so: one element further on, each kernel gives the same."""
+    rng, keep, rows, eps = np.random.default_rng(width), [], 5, 1e-3
+    x, y, w, z = (rng.standard_normal(s).astype(np.float32) for s in ((rows, width), (rows, width), width, (rows, width)))
+    aligned, after_one = dev(ctx, keep, w), dev(ctx, keep, np.concatenate([[np.float32(7.0)], w])) + 4
+    ldh, packed = up32(width), (rows + 15) // 16 * 16 * up32(width)
+    py, pz, one = dev(ctx, keep, y), dev(ctx, keep, z), dev(ctx, keep, np.ones(1, np.float32))
+
+    def outputs(pw):
+        found = []
+        for kind in range(4):
+            dx, h = ctx.to_device(x), ctx.to_device(filled(packed, dtype))
+            if kind == 0:
+                call(ctx, "m40llm_ext_norm_rows_async", RMS, dx.ptr, py, 1, rows * width, pw, None, rows, width, C.c_float(eps), h.ptr, ldh, ACT[dtype], 1)
+            elif kind == 1:
+                n = NormAdd(act_dtype=ACT[dtype], rows=rows, width=width, eps=eps, mult=0.5, x=dx.ptr, w=pw, h=h.ptr, ld_h=ldh, planes=py, n_planes=1, plane_stride=rows * width)
+                call(ctx, "m40llm_ext_norm_add_rows_async", C.byref(n), 1)
+            elif kind == 2:
+                call(ctx, "m40llm_ext_norm_gate_rows_async", py, C.c_uint64(width), pw, pz, C.c_uint64(width), rows, width, C.c_float(eps), h.ptr, ldh, ACT[dtype], 1)
+            else:
+                n = Update(act_dtype=ACT[dtype], rows=rows, width=width, streams=1, eps=eps, mult=0.5, streams_x=dx.ptr, stream_stride=rows * width, mix=one, share=one, take=one,
+                           planes=py, n_planes=1, plane_stride=rows * width, w=pw, h=h.ptr, ld_h=ldh)
+                call(ctx, "m40llm_ext_stream_update_async", C.byref(n), 1)
+            found.append((dx.download(np.float32, (rows, width)), from_act(unpack_tiles(h.download(act_type(dtype), (packed,)), rows, ldh), dtype)))
+        return found
+    for (xa, ha), (xb, hb) in zip(outputs(aligned), outputs(after_one)):
+        close_to(xb, xa, "float32")
+        close_to(hb, ha, dtype)
+        assert np.abs(ha[:, :width]).max() > 0.1 and np.all(hb[:, width:] == 0)
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
