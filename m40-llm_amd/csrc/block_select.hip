@@ -10,7 +10,7 @@
 //   2. rank   : per q head, blocks ordered by (score descending, block id ascending): the order the reference's
 //               strict-'>' insertion into a list initialised to -1e30 produces (cuda/kernels.cu:2913-2927); the
 //               first min(top_blocks, old_blocks) valid ones are kept.  A block's rank is the number of blocks above
-//               it, counted 64 blocks at a time with one compare and a wave-wide ballot.
+//               it, counted by a lane of its own.
 //   3. attend : per q head, softmax attention over [tokens of the selected blocks] ++ [recent window], one block per
 //               wave.  Old V is unpacked from 4 bits in registers (value = nibble * scale, rounded through f16 as
 //               the reference does).
@@ -188,22 +188,26 @@ __global__ __launch_bounds__(128) void bs_score_kernel(BsMulti multi) {
 // ---- 2. ranking ---------------------------------------------------------------------------------------------------
 // Block b is at rank #{o : score[o] > score[b] or (== and o < b)}: the order the reference's strict-'>' insertion
 // into a list initialised to -1e30 produces (cuda/kernels.cu:2913-2927); scores that are NaN or not above -1e30 never
-// enter the list.  Grid (q head, 16 candidate blocks, slot), four waves of 4 candidates each.  A wave holds the order
-// keys of all blocks 64 at a time, one per lane, and counts the blocks above a candidate with one compare and a
-// wave-wide ballot per 64 blocks.  sel[rank] = block for rank < top_n; the first workgroup of a head also writes the
-// list length and the unused tail of the list.
+// enter the list.  Grid (q head, 64 candidate blocks, slot): a lane holds one candidate, and each of the eight waves counts an eighth of the
+// head's keys, which all lanes read together from LDS (a compare and an add with carry for 64 pairs).  Instructions bound it once several
+// slots share a launch: with a wave's lanes over the keys and a ballot and a scalar count per candidate it took 8.9 us for four slots of
+// 504 blocks (16.8 us for eight, 4.6 us for one) against 6.0 us (10.4, 4.1) here.  Sixteen keys a step in four waves: 6.7 us (9.0, 5.1).  One
+// wave per head that finds the last key to enter bit by bit: 8.4 us whatever the slots, a chain of 32 counts.  sel[rank] = block for
+// rank < top_n; the first workgroup of a head also writes the list length and the unused tail of the list.
 __device__ __forceinline__ uint32_t bs_order_key(float s) {
     const uint32_t u = __float_as_uint(s);
     const uint32_t k = (u & 0x80000000u) ? ~u : (u | 0x80000000u);      // monotone in s
     return (s > -1e30f) ? k : 0u;                                       // invalid (and NaN): below every valid key
 }
-constexpr int kBsRankThreads = 256, kBsRankCand = 16;
+constexpr int kBsRankThreads = 512, kBsRankCand = 64;
 __global__ __launch_bounds__(kBsRankThreads) void bs_rank_kernel(BsMulti multi) {
     const BsParams& p = multi.slot[blockIdx.z];
-    extern __shared__ uint32_t s_keys[];            // order keys of the head's blocks, padded with zeros to 64 words
-    __shared__ uint32_t s_valid[kBsRankThreads / 64];
+    extern __shared__ uint4 s_keys4[];              // order keys of the head's blocks, padded with zeros to 64 words
+    uint32_t* s_keys = reinterpret_cast<uint32_t*>(s_keys4);
+    constexpr uint32_t kWaves = kBsRankThreads / 64, kStep = 64 / kWaves;
+    __shared__ uint32_t s_valid[kWaves], s_above[kWaves][64];
     const uint32_t qh = blockIdx.x, y = blockIdx.y;
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     if (p.nblk == 0) {
         if (y == 0) {
             if (tid < 64) { p.sel[qh * 64 + tid] = 0xffffffffu; p.sel_scores[qh * 64 + tid] = -1e30f; }
@@ -224,40 +228,47 @@ __global__ __launch_bounds__(kBsRankThreads) void bs_rank_kernel(BsMulti multi) 
     for (int o = 1; o < 64; o <<= 1) valid += __shfl_xor(valid, o, 64);
     if (lane == 0) s_valid[wave] = valid;
     __syncthreads();
-    constexpr int CPW = kBsRankCand / (kBsRankThreads / 64);     // candidates per wave
-    const uint32_t cand0 = y * kBsRankCand + (uint32_t)wave * CPW;
-    uint32_t kb[CPW], above[CPW];
+    const uint32_t cand = y * kBsRankCand + (uint32_t)lane, key = s_keys[cand];
+    // blocks before a candidate count when they score at least as high, blocks after it when higher: one limit for all keys of a step
+    // but in the 64 blocks that the candidates are
+    uint32_t above = 0;
+    const auto step = [&](uint32_t u, uint32_t limit) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < CPW; ++i) {
-        const uint32_t b = cand0 + i;
-        kb[i] = b < p.nblk ? s_keys[b] : 0u;      // wave-uniform
-        above[i] = 0;
-    }
-    for (uint32_t ch = 0; ch < n64; ++ch) {
-        const uint32_t o = ch * 64u + (uint32_t)lane;
-        const uint32_t ko = s_keys[o];
-#pragma unroll
-        for (int i = 0; i < CPW; ++i) {
-            // blocks before the candidate count when they score at least as high, blocks after it when higher
-            const uint32_t thr = kb[i] + (o >= cand0 + i ? 1u : 0u);
-            above[i] += (uint32_t)__popcll(__ballot(ko >= thr));
+        for (uint32_t i = 0; i < kStep / 4u; ++i) {
+            const uint4 k = s_keys4[u * (kStep / 4u) + i];
+            above += k.x >= limit ? 1u : 0u;
+            above += k.y >= limit ? 1u : 0u;
+            above += k.z >= limit ? 1u : 0u;
+            above += k.w >= limit ? 1u : 0u;
         }
-    }
-    if (lane == 0) {
+    };
+    const uint32_t end = ((uint32_t)wave + 1u) * n64, own = y * kWaves;
+    uint32_t u = (uint32_t)wave * n64;              // a step is kStep keys, a wave's share n64 steps
+#pragma unroll 4
+    for (const uint32_t stop = end < own ? end : own; u < stop; ++u) step(u, key);
+    for (const uint32_t stop = end < own + kWaves ? end : own + kWaves; u < stop; ++u)
 #pragma unroll
-        for (int i = 0; i < CPW; ++i) {
-            if (kb[i] != 0u && above[i] < p.top_n) {
-                p.sel[qh * 64 + above[i]] = cand0 + i;
-                p.sel_scores[qh * 64 + above[i]] = scores[cand0 + i];
-            }
+        for (uint32_t i = 0; i < kStep; ++i) {
+            const uint32_t o = u * kStep + i;
+            above += s_keys[o] >= key + (o >= cand ? 1u : 0u) ? 1u : 0u;
         }
+#pragma unroll 4
+    for (; u < end; ++u) step(u, key + 1u);
+    s_above[wave][lane] = above;
+    __syncthreads();
+    if (wave != 0) return;
+#pragma unroll
+    for (uint32_t w = 1; w < kWaves; ++w) above += s_above[w][lane];
+    if (key != 0u && above < p.top_n) {
+        p.sel[qh * 64 + above] = cand;
+        p.sel_scores[qh * 64 + above] = scores[cand];
     }
-    if (y == 0 && tid < 64) {
+    if (y == 0) {
         uint32_t total = 0;
-        for (int w = 0; w < kBsRankThreads / 64; ++w) total += s_valid[w];
+        for (uint32_t w = 0; w < kWaves; ++w) total += s_valid[w];
         const uint32_t count = total < p.top_n ? total : p.top_n;
-        if ((uint32_t)tid >= count) { p.sel[qh * 64 + tid] = 0xffffffffu; p.sel_scores[qh * 64 + tid] = -1e30f; }
-        if (tid == 0) p.counts[qh] = count;
+        if ((uint32_t)lane >= count) { p.sel[qh * 64 + lane] = 0xffffffffu; p.sel_scores[qh * 64 + lane] = -1e30f; }
+        if (lane == 0) p.counts[qh] = count;
     }
 }
 

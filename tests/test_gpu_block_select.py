@@ -183,6 +183,30 @@ def _block_select_case(dev, orc, qh, kvh, hd, L, W, bs, top, S=None, seed=0, sca
     return dict(got=got, want=want, sel=sel, cnt=cnt, ssc=ssc, wsel=wsel, wcnt=wcnt, c=c, q=q, kv=kv, k16=k16, v16=v16)
 
 
+@pytest.mark.parametrize("nblk,top", [(1, 64), (63, 5), (64, 64), (65, 64), (130, 64), (513, 33)])
+def test_rank_of_tied_and_infinite_scores(dev, orc, nblk, top):
+    """Few distinct blocks, so that most scores tie (the lower block id is first), and some infinite ones (-inf and NaN never enter)."""
+    qh, kvh, hd, W, bs = 4, 2, 64, 16, 4
+    L = W + nblk * bs - 1
+    rng = np.random.default_rng(nblk)
+    rows = rng.standard_normal((3, kvh, hd))
+    k = np.repeat(rows[rng.integers(0, 3, nblk)], bs, axis=0)[:L - W]
+    for b in rng.integers(0, nblk, 4):
+        k[b * bs:(b + 1) * bs, :, 0] = np.inf
+    k16, v16 = f16bits(np.concatenate([k, rng.standard_normal((W, kvh, hd))])), f16bits(rng.standard_normal((L, kvh, hd)))
+    q = rng.standard_normal((qh, hd)).astype(np.float32)
+    kv = m40.KVCache(dev.ctx, L, 1, kvh, hd, dict(recent_window=W, block_size=bs, top_blocks=top, exact_old_backing=2))
+    dk, dv = dev.up(k16), dev.up(v16)
+    dev.call("m40llm_ext_kvcache_bulk_fill_f16", kv.h, 0, dk.ptr, dv.ptr, L)
+    c = orc.CompressedKV(L, 1, kvh, hd, W, bs)
+    c.bulk_fill(0, k16, v16)
+    sel, cnt, ssc = np.zeros((qh, 64), np.uint32), np.zeros(qh, np.uint32), np.zeros((qh, 64), np.float32)
+    dq = dev.up(q)
+    dev.call("m40llm_ext_block_select_read_selection", kv.h, 0, dq.ptr, qh, L, W, bs, top, sel.ctypes.data, cnt.ctypes.data, ssc.ctypes.data)
+    rc, _, wsel, wcnt = c.attention(0, q, qh, L, top, score_order=0)
+    assert rc == 0 and np.array_equal(cnt, wcnt) and np.array_equal(sel, wsel)
+
+
 @pytest.mark.parametrize("qh,kvh,hd,L,W,bs,top", [
     (4, 2, 128, 16, 4, 4, 3),          # tests/attention_parity_cuda_grid.rs:726-843
     (4, 2, 128, 5, 4, 32, 8),          # :608-723, one partial old block
