@@ -431,7 +431,10 @@ constexpr struct { int rows, cols; float least, start, load; } kTileShapes[4] = 
 template <int FORM>
 int launch_tile_any(hipStream_t stream, const PackedArgs& g, const M40Epilogue<m40_bf16>& e, int batches, int num_cus) {
     if constexpr (FORM == kSlots) {
-        return launch_tile<4, 4, 1, 5, FORM>(stream, g, e, batches);          // a job is one row of tiles
+        // a job is one row of tiles; long sums take the wider tile, which reads a job's rows half as often (32 experts of 4096 x 5504, 512 rows of four
+        // choices: 302 us against 316; of 2048 x 2816 the narrow one's two workgroups a CU are faster)
+        if (g.k_tiles > 64) return launch_tile<4, 8, 1, 6, FORM>(stream, g, e, batches);
+        return launch_tile<4, 4, 1, 5, FORM>(stream, g, e, batches);
     } else {
         const bool pairs = g.k_tiles % 2 == 0 && g.k_total % 2 == 0;          // two k tiles a stage
         int best = 1;
@@ -439,11 +442,17 @@ int launch_tile_any(hipStream_t stream, const PackedArgs& g, const M40Epilogue<m
         long long t[4];
         for (int c = 0; c < 4; ++c) {
             t[c] = (long long)((g.rows + kTileShapes[c].rows - 1) / kTileShapes[c].rows) * ((g.n_tiles * 16 + kTileShapes[c].cols - 1) / kTileShapes[c].cols) * batches;
-            // the largest tile pays where a long sum's tiles fill the CUs just once
+            // the largest tile pays for long sums, where its tiles fill the CUs just once or their rounds better (below)
             if ((c == 0 && (g.k_tiles <= 64 || t[0] > num_cus)) || (c == 3 && !pairs)) continue;
             const float u = (float)t[c] / (float)num_cus, cost = kTileShapes[c].start + kTileShapes[c].load * u;
             const float at_least = cost > kTileShapes[c].least ? cost : kTileShapes[c].least;
             if (at_least < best_cost) { best_cost = at_least; best = c; }
+        }
+        // long sums over more tiles than CUs: what counts is how many the fullest CU has (K 4096, 128 x 256 / 128 x 128: 512 rows, N 26752 131 / 147 us;
+        // 1500 rows, N 4096 67 / 78, N 6144 116 / 102, N 12800 188 / 174)
+        if (best == 1 && g.k_tiles > 64 && t[1] > num_cus) {
+            const auto most = [&](int c) { return (float)((t[c] + num_cus - 1) / num_cus); };
+            if (kTileShapes[0].start * most(0) < kTileShapes[1].start + kTileShapes[1].load * most(1)) best = 0;
         }
         // alone on its CU a workgroup takes the memory of two for deeper buffers: N 2048, K 5632 at 77 rows 21.2 us (64 x 64) against 24.4, at
         // 1300 rows 43.6 us (128 x 128) against 50.7

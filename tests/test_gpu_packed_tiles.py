@@ -1,11 +1,15 @@
 """Products of many packed bf16 rows over the tile sizes that row, column and k counts choose, at their edges."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
 pytestmark = pytest.mark.gpu
 
-from pimosun_common import close_to, ld, m40, unpack_tiles, up32  # noqa: E402
-from test_gpu_layer_kernels import ADD, PROJECT, STORE, bf16w, gemm, rounded  # noqa: E402
+from pimosun_common import c_struct, close_to, from_act, ld, m40, pack_tiles, unpack_tiles, up32  # noqa: E402
+from test_gpu_layer_kernels import ACT, ADD, PROJECT, STORE, STORE_ACT, bf16w, call, gemm, rounded  # noqa: E402
+
+Gemm = c_struct("M40llmPackedGemm")
 
 
 @pytest.fixture(scope="module")
@@ -16,7 +20,7 @@ def ctx():
 # 64 x 64 tiles alone on their CU (65 .. 500 rows of few columns) and two to a CU, 64 x 128 (odd number of k tiles, or rows between), 128 x 128, 128 x 256
 # (whole rounds of them); k of one tile, of fewer stages than buffers, of one stage more than a period; rows and columns that fill no tile
 @pytest.mark.parametrize("rows,n,k", [(65, 144, 32), (65, 150, 64), (127, 2048, 384), (200, 500, 352), (300, 1040, 2112), (500, 2048, 256), (700, 2050, 320), (700, 2048, 992),
-                                      (1300, 1504, 96), (1300, 2050, 160), (2049, 3000, 352), (4096, 2048, 192), (4000, 2040, 224)])
+                                      (1300, 1504, 96), (1300, 2050, 160), (1700, 2310, 2112), (2049, 3000, 352), (4096, 2048, 192), (4000, 2040, 224)])
 def test_tiles_store_and_add(ctx, rows, n, k):
     rng = np.random.default_rng(rows + n + k)
     A, W = rng.standard_normal((rows, k)), bf16w(rng, n, k)
@@ -61,3 +65,24 @@ def test_tiles_gated_pairs(ctx, rows, ff, k):
     close_to(out["out_f32"], a @ plain.T.astype(np.float64), "float32", factor=2)
     got = (unpack_tiles(out["out_act"], rows, ld_act).astype(np.uint32) << 16).view(np.float32)[:, :tiles * 16]
     assert (np.abs(got - want) <= 2.0 ** -8 * np.abs(want) + 1e-5 * np.abs(want).max()).all()      # one rounding to 8 bits, and f32 sums
+
+
+@pytest.mark.parametrize("k", [2048, 2080])
+@pytest.mark.parametrize("n", [304, 1280])
+def test_expert_jobs_of_short_and_long_sums(ctx, n, k):
+    """Jobs of up to 128 rows take 128-column tiles up to 64 k tiles and 256-column ones beyond; an unused expert, ragged rows, a ragged last tile."""
+    counts, rng, keep = [130, 0, 17, 128], np.random.default_rng(n + k), []
+    W, jobs, slots = [bf16w(rng, n, k) for _ in counts], [], 0
+    for e, m in enumerate(counts):
+        jobs += [(e, slots + j, min(128, m - j), 0) for j in range(0, m, 128)]
+        slots += (m + 15) // 16 * 16
+    A = rng.standard_normal((slots, k))
+    dev = lambda a: keep.append(ctx.to_device(np.ascontiguousarray(a))) or keep[-1].ptr
+    out = ctx.to_device(np.full(slots * n, 0x4b4b, np.uint16))
+    g = Gemm(act_dtype=ACT["bfloat16"], epilogue=STORE_ACT, lda=k, a=dev(pack_tiles(ld.f32_to_bf16(A))), w=dev(np.concatenate([pack_tiles(ld.f32_to_bf16(w)).reshape(-1) for w in W])),
+             n_tiles=n // 16, k_tiles=k // 32, w_batch=n // 16 * (k // 32) * 512, rows=slots, batches=1, out_act=out.ptr, ld_act=n, cols=n,
+             jobs=dev(np.concatenate([[len(jobs), slots, 0, 0], np.array(jobs).reshape(-1)]).astype(np.uint32)), max_jobs=len(jobs) + 2, job_rows=128)
+    call(ctx, "m40llm_ext_packed_gemm_async", C.byref(g), 1)
+    got = from_act(out.download(np.uint16, (slots, n)), "bfloat16")
+    for e, first, m, _ in jobs:
+        close_to(got[first:first + m], rounded(A[first:first + m], "bfloat16") @ W[e].T.astype(np.float64), "bfloat16")
