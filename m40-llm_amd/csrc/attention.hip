@@ -346,8 +346,10 @@ int launch_hd(M40llmCudaContext* ctx, hipStream_t stream, float* partial, size_t
         uint64_t chunk = (((uint64_t)span * groups / ctx->num_cus) + 64) / 128 * 128;
         // Around half a thousand tokens a chunk two workgroups a CU are better: a wave's tiles follow one another, and two is as many as are worth
         // waiting for (32 rows of up to 1021 tokens, 4 kv heads of 64: chunks of 512 9.0 us, of 256 7.8 us; 8 rows of up to 4093, 2 kv heads of 128:
-        // chunks of 256 8.8 us, of 128 9.2 us).
-        if (chunk > 256 && chunk <= 512) chunk = 256;
+        // chunks of 256 8.8 us, of 128 9.2 us).  One sequence keeps the larger ones where its partials of 256 tokens would not fit the fixed buffer:
+        // with the context's arena and with that buffer the chunks are the same.
+        const size_t need_256 = (size_t)p.q_heads * ((span + 255u) / 256u) * (HD + 2) * sizeof(float);
+        if (chunk > 256 && chunk <= 512 && (batch > 1 || need_256 <= kStaticScratchBytes)) chunk = 256;
         if (chunk < 128) chunk = 128;
         while (groups * ((span + chunk - 1) / chunk) > 2ull * ctx->num_cus) chunk += 128;
         if (chunk > 2048) chunk = 2048;

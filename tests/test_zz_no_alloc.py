@@ -47,6 +47,11 @@ def test_static_scratch_two_calls_second_smaller(dev, orc):
     _case(dev, orc, 32, 4, 64, [4096, 700], seed=1)
 
 
+def test_static_scratch_takes_rows_whose_smaller_chunks_would_not_fit(dev, orc):
+    # 128 chunks of 256 tokens for 32 heads of 128 are 2.03 MiB; 64 of 512 fit
+    _case(dev, orc, 32, 4, 128, [32768], seed=2)
+
+
 def test_static_scratch_argument_codes_and_size_limit(dev):
     qh, kvh, hd = 32, 4, 64
     kv = m40.KVCache(dev.ctx, 64, 1, kvh, hd)
