@@ -286,6 +286,34 @@ def test_split_norm_rotate_append(ctx, dtype):
         close_to(unpack_tiles(pages[p], 64, ew), want[p], dtype, scale=np.abs(lat_want).max(), factor=1 if dtype == "bfloat16" else 2)
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("qr,kr,rd", [(1, 1, 2), (1536, 512, 256), (1540, 530, 300)])
+def test_split_norm_rotate_at_the_edges_of_a_threads_registers(ctx, dtype, qr, kr, rd):
+    rng, rows, eps = np.random.default_rng(qr), 18, 5e-3
+    kv_off, rot_off, lat, half = up32(qr), up32(qr) + up32(kr), up32(kr), up32(rd) // 2
+    ldp, ew = rot_off + up32(rd), lat + up32(rd)
+    proj = rng.standard_normal((rows, ldp)).astype(np.float32)
+    qn, kn = rng.standard_normal(qr).astype(np.float32), rng.standard_normal(kr).astype(np.float32)
+    spec, pos = dict(dims=rd, base=50.0), np.arange(3, 3 + rows).astype(np.uint32)
+    ang = angles(ctx, pos, spec, half)
+    bufs = {k: ctx.to_device(v) for k, v in dict(proj=proj, q_norm=qn, kv_norm=kn, cache=np.zeros(64 * ew, act_type(dtype)), cq=np.zeros(32 * up32(qr), act_type(dtype)), angles=ang,
+                                                 row_slot=np.zeros(rows, np.uint32), row_pos=pos, page_table=np.zeros(1, np.uint32)).items()}
+    p64 = proj.astype(np.float64)
+    q_want, k_want, r_want = ld.rms_norm(p64[:, :qr], qn, eps), ld.rms_norm(p64[:, kv_off:kv_off + kr], kn, eps), ld.rotate(p64[:, rot_off:rot_off + rd], pos, spec)
+    for with_cache in (True, False):
+        given = {k: b.ptr for k, b in bufs.items() if with_cache or k != "cache"}
+        s = Split(act_dtype=ACT[dtype], rows=rows, ld_proj=ldp, q_rank=qr, kv_offset=kv_off, kv_rank=kr, rot_offset=rot_off, rot_dim=rd, eps=eps, ld_cq=up32(qr), latent_pad=lat,
+                  entry_width=ew, rot_half=half, max_pages=1, **given)
+        call(ctx, "m40llm_ext_latent_split_append_async", C.byref(s), 1)
+        got = from_act(unpack_tiles(bufs["cq"].download(act_type(dtype), (32 * up32(qr),)), rows, up32(qr)), dtype)
+        close_to(got[:, :qr], q_want, dtype)
+        assert np.all(got[:, qr:] == 0)
+    entries = unpack_tiles(from_act(bufs["cache"].download(act_type(dtype), (64 * ew,)), dtype), 64, ew)[3:3 + rows]
+    close_to(entries[:, :kr], k_want, dtype)
+    close_to(entries[:, lat:lat + rd], r_want, dtype)
+    assert np.all(entries[:, kr:lat] == 0) and np.all(entries[:, lat + rd:] == 0)
+
+
 # ---- attention -------------------------------------------------------------------------------------------------------------
 
 
