@@ -539,8 +539,8 @@ int m40llm_ext_batched_norm_gemm_f32xf16_async(M40llmCudaContext* ctx, const voi
                                                uint32_t rows, int N, int K);
 /* The four calls above for up to 32 rows (K a multiple of 256, operands 16-byte aligned, head_dim a multiple of 16; -6 otherwise): the
  * weights are read once for all rows, one launch a call.  d_clear_f32 / clear_floats as in the ..._clear call.  The result of
- * ..._onto_zero HOLDS ZEROS stored by an earlier call on the decode stream; where it overlaps an operand it is overwritten
- * instead of added to (a residual may be the result itself, element by element). */
+ * ..._onto_zero HOLDS ZEROS stored by an earlier call on the decode stream, or is the residual itself, which is then overwritten.  Results and
+ * what is cleared overlap neither the rows nor each other, nor a result its residual in part: -6, nothing enqueued. */
 int m40llm_ext_batched_wide_norm_qkv_rope_append_async(
     M40llmCudaContext* ctx, M40llmKVCache* kv, const uint32_t* seq_ids_dev, const uint32_t* seq_lens_dev, uint32_t rows,
     const void* d_x_f32, const void* d_norm_w, uint32_t norm_weight_dtype, float eps, const void* d_wq_f16,

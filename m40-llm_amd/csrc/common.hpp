@@ -112,6 +112,11 @@ static inline hipStream_t m40_select_stream(M40llmCudaContext* ctx, uint32_t str
 #define M40_HD
 #endif
 M40_HD static inline bool m40_aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
+// no byte in common (a null range has none)
+static inline bool m40_apart(const void* a, size_t a_bytes, const void* b, size_t b_bytes) {
+    const char *p = static_cast<const char*>(a), *q = static_cast<const char*>(b);
+    return !p || !q || p + a_bytes <= q || q + b_bytes <= p;
+}
 
 // Internal launch entry points shared between translation units ------------------
 // GEMM family (gemm.hip)
@@ -149,7 +154,8 @@ int m40_rows_mfma_qkv(M40llmCudaContext* ctx, hipStream_t stream, const M40llmKV
                       const uint16_t* wq, const uint16_t* wk, const uint16_t* wv, const float* bq, const float* bk,
                       const float* bv, uint32_t d_model, uint32_t q_heads, float rope_base, float rope_scale,
                       uint32_t rope_layout, float* q_out);
-// the projections for 9 to 32 rows, K a multiple of 256 (rows_wide_mfma.hip); zero: zero_count floats cleared on the side
+// the projections for 9 to 32 rows, K a multiple of 256 (rows_wide_mfma.hip); zero: zero_count floats cleared on the side.  -6 also where
+// what a launch writes overlaps rows that it reads (a residual may be the result itself)
 bool m40_rows_wide_supported(int rows, int K);
 int m40_rows_wide_qkv(M40llmCudaContext* ctx, hipStream_t stream, const M40llmKVCache* kv, const uint32_t* ids_dev, const uint32_t* lens_dev,
                       uint32_t rows, const float* x, const void* norm_w, uint32_t norm_dtype, float eps, const uint16_t* wq, const uint16_t* wk,

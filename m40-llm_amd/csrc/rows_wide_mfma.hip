@@ -412,6 +412,17 @@ int launch(M40llmCudaContext* ctx, hipStream_t stream, WideArgs& a, int k_parts 
 
 }  // namespace
 
+namespace {
+
+// Every workgroup reads all rows while others already store their columns and clear their share: what is written must lie apart from the rows
+// and from each other.
+bool rows_untouched(const WideArgs& a, const float* out, size_t out_cols) {
+    const size_t x_bytes = (size_t)a.rows * a.K * 4, out_bytes = (size_t)a.rows * out_cols * 4, zero_bytes = (size_t)a.zero_count * 4;
+    return m40_apart(a.x, x_bytes, out, out_bytes) && m40_apart(a.x, x_bytes, a.zero, zero_bytes) && m40_apart(out, out_bytes, a.zero, zero_bytes);
+}
+
+}  // namespace
+
 // 9 .. 32 rows: fewer rows have faster kernels (rows_mfma.hip, rows_gemv.hip); the operands 16-byte aligned, K whole steps of 256.
 bool m40_rows_wide_supported(int rows, int K) { return rows >= 1 && rows <= 32 && K >= 256 && K % 256 == 0; }
 
@@ -430,6 +441,7 @@ int m40_rows_wide_qkv(M40llmCudaContext* ctx, hipStream_t stream, const M40llmKV
     a.head_dim = kv->head_dim; a.rope_layout = rope_layout; a.rope_base = rope_base; a.rope_scale = rope_scale;
     a.rows = (int)rows; a.K = (int)d_model; a.N = (int)((q_heads + 2u * kv->num_heads) * kv->head_dim);
     a.tiles = a.N / 16; a.zero = zero; a.zero_count = zero_count;
+    if (!rows_untouched(a, q_out, (size_t)q_heads * kv->head_dim)) return -6;
     return launch<kQkv>(ctx, stream, a);
 }
 
@@ -440,6 +452,7 @@ int m40_rows_wide_swiglu(M40llmCudaContext* ctx, hipStream_t stream, const float
     WideArgs a{};
     a.x = x; a.norm_w = norm_w; a.norm_dtype = norm_dtype; a.eps = eps; a.W0 = wgate; a.W1 = wup; a.out = out;
     a.rows = rows; a.N = ffn; a.K = K; a.tiles = (ffn + 7) / 8; a.zero = zero; a.zero_count = zero_count;
+    if (!rows_untouched(a, out, ffn)) return -6;
     return launch<kSwiglu>(ctx, stream, a);
 }
 
@@ -449,26 +462,22 @@ int m40_rows_wide_norm(M40llmCudaContext* ctx, hipStream_t stream, const float* 
     if (!m40_aligned16(x) || !m40_aligned16(norm_w) || !m40_aligned16(W)) return -6;
     WideArgs a{};
     a.x = x; a.norm_w = norm_w; a.norm_dtype = norm_dtype; a.eps = eps; a.W0 = W; a.out = out; a.rows = rows; a.N = N; a.K = K; a.tiles = (N + 15) / 16;
+    if (!rows_untouched(a, out, N)) return -6;
     return launch<kNorm>(ctx, stream, a);
 }
 
-// onto_zero: out holds zeros and overlaps neither operand, so that two halves of K may be added into it where one tile a workgroup would
-// leave half of the CUs idle.
+// onto_zero: out holds zeros, so that two halves of K may be added into it where one tile a workgroup would leave half of the CUs idle; a
+// residual that is out itself is read before each element is stored, in one part.
 int m40_rows_wide_residual(M40llmCudaContext* ctx, hipStream_t stream, const float* x, const uint16_t* W, const float* residual, float* out, int rows,
                            int N, int K, bool onto_zero) {
     if (!m40_rows_wide_supported(rows, K) || N <= 0) return -6;
     if (!m40_aligned16(x) || !m40_aligned16(W)) return -6;
     WideArgs a{};
     a.x = x; a.W0 = W; a.residual = residual; a.out = out; a.rows = rows; a.N = N; a.K = K; a.tiles = (N + 15) / 16;
-    return launch<kResidual>(ctx, stream, a, onto_zero && K >= 2 * kChunk && 2 * a.tiles <= ctx->num_cus ? 2 : 1);
+    const size_t out_bytes = (size_t)rows * N * 4;
+    if (!rows_untouched(a, out, N) || (residual != out && !m40_apart(residual, out_bytes, out, out_bytes))) return -6;
+    return launch<kResidual>(ctx, stream, a, onto_zero && residual != out && K >= 2 * kChunk && 2 * a.tiles <= ctx->num_cus ? 2 : 1);
 }
-
-namespace {
-bool apart(const void* a, size_t a_bytes, const void* b, size_t b_bytes) {
-    const char *p = static_cast<const char*>(a), *q = static_cast<const char*>(b);
-    return !p || !q || p + a_bytes <= q || q + b_bytes <= p;
-}
-}  // namespace
 
 extern "C" {
 
@@ -506,10 +515,8 @@ int m40llm_ext_batched_wide_gemm_residual_onto_zero_async(M40llmCudaContext* ctx
     if (!ctx || !d_a_f32 || !d_w_f16 || !d_out_f32) return -1;
     if (N <= 0 || K <= 0) return -2;
     (void)hipGetLastError();
-    const size_t out_bytes = (size_t)rows * N * 4;
     return m40_rows_wide_residual(ctx, ctx->decode_stream, static_cast<const float*>(d_a_f32), static_cast<const uint16_t*>(d_w_f16),
-                                  static_cast<const float*>(d_residual_f32), static_cast<float*>(d_out_f32), (int)rows, N, K,
-                                  apart(d_a_f32, (size_t)rows * K * 4, d_out_f32, out_bytes) && apart(d_residual_f32, out_bytes, d_out_f32, out_bytes));
+                                  static_cast<const float*>(d_residual_f32), static_cast<float*>(d_out_f32), (int)rows, N, K, true);
 }
 
 int m40llm_ext_batched_wide_norm_gemm_async(M40llmCudaContext* ctx, const void* d_x_f32, const void* d_norm_w, uint32_t norm_weight_dtype, float eps,

@@ -780,8 +780,9 @@ int m40llm_ext_batched_norm_qkv_rope_append_async(
                                  static_cast<const float*>(d_bq_f32), static_cast<const float*>(d_bk_f32),
                                  static_cast<const float*>(d_bv_f32), d_model, q_heads, freq_base, freq_scale, rope_layout,
                                  static_cast<float*>(d_q_out_f32));
-    // nine rows and more: one launch as well, K in chunks
-    if (rows > 8 && kv->head_dim % 16 == 0 && m40_aligned16(d_x_f32) && m40_aligned16(d_norm_w))
+    // nine rows and more: one launch as well, K in chunks; a result that overlaps the rows takes the two launches below, here and in the other calls
+    if (rows > 8 && kv->head_dim % 16 == 0 && m40_aligned16(d_x_f32) && m40_aligned16(d_norm_w) &&
+        m40_apart(d_x_f32, (size_t)rows * d_model * 4, d_q_out_f32, (size_t)rows * q_heads * kv->head_dim * 4))
         return m40_rows_wide_qkv(ctx, ctx->decode_stream, kv, seq_ids_dev, seq_lens_dev, rows, static_cast<const float*>(d_x_f32), d_norm_w,
                                  norm_weight_dtype, eps, static_cast<const uint16_t*>(d_wq_f16), static_cast<const uint16_t*>(d_wk_f16),
                                  static_cast<const uint16_t*>(d_wv_f16), static_cast<const float*>(d_bq_f32),
@@ -826,7 +827,9 @@ int m40llm_ext_batched_gemm_residual_f32xf16_async(M40llmCudaContext* ctx, const
         return m40_rows_gemv_residual(ctx->decode_stream, static_cast<const float*>(d_a_f32),
                                       static_cast<const uint16_t*>(d_w_f16), static_cast<const float*>(d_residual_f32),
                                       static_cast<float*>(d_out_f32), (int)rows, N, K);
-    if (rows > 8 && m40_aligned16(d_a_f32))
+    const size_t out_bytes = (size_t)rows * N * 4;
+    if (rows > 8 && m40_aligned16(d_a_f32) && m40_apart(d_a_f32, (size_t)rows * K * 4, d_out_f32, out_bytes) &&
+        (d_residual_f32 == d_out_f32 || m40_apart(d_residual_f32, out_bytes, d_out_f32, out_bytes)))
         return m40_rows_wide_residual(ctx, ctx->decode_stream, static_cast<const float*>(d_a_f32), static_cast<const uint16_t*>(d_w_f16),
                                       static_cast<const float*>(d_residual_f32), static_cast<float*>(d_out_f32), (int)rows, N, K, false);
     PackSpec pk{static_cast<const float*>(d_a_f32), nullptr, nullptr, 0, 0.0f};
@@ -844,11 +847,7 @@ int m40llm_ext_batched_gemm_residual_onto_zero_f32xf16_async(M40llmCudaContext* 
                                                              int K) {
     if (!ctx || !d_a_f32 || !d_w_f16 || !d_out_f32) return -1;
     if (N <= 0 || K <= 0) return -2;
-    const char* o = static_cast<const char*>(d_out_f32);
-    auto apart = [&](const void* q, size_t bytes) {
-        const char* c = static_cast<const char*>(q);
-        return !c || c + bytes <= o || o + (size_t)rows * N * 4 <= c;
-    };
+    auto apart = [&](const void* q, size_t bytes) { return m40_apart(q, bytes, d_out_f32, (size_t)rows * N * 4); };
     if (m40_rows_khalf_supported(ctx, (int)rows, N, K) && m40_aligned16(d_a_f32) && m40_aligned16(d_w_f16) &&
         apart(d_a_f32, (size_t)rows * K * 4) && apart(d_residual_f32, (size_t)rows * N * 4)) {
         (void)hipGetLastError();
@@ -890,7 +889,9 @@ int m40llm_ext_batched_norm_gate_up_swiglu_clear_async(M40llmCudaContext* ctx, c
                                     eps, static_cast<const uint16_t*>(d_wgate_f16), static_cast<const uint16_t*>(d_wup_f16),
                                     static_cast<float*>(d_hid_f32), (int)rows, ffn, d_model,
                                     clear_floats ? static_cast<float*>(d_clear_f32) : nullptr, (int)clear_floats);
-    if (rows > 8 && m40_aligned16(d_x_f32) && m40_aligned16(d_norm_w))
+    const size_t x_bytes = (size_t)rows * d_model * 4, hid_bytes = (size_t)rows * ffn * 4, clear_bytes = (size_t)clear_floats * 4;
+    if (rows > 8 && m40_aligned16(d_x_f32) && m40_aligned16(d_norm_w) && m40_apart(d_x_f32, x_bytes, d_hid_f32, hid_bytes) &&
+        (!clear_floats || (m40_apart(d_x_f32, x_bytes, d_clear_f32, clear_bytes) && m40_apart(d_hid_f32, hid_bytes, d_clear_f32, clear_bytes))))
         return m40_rows_wide_swiglu(ctx, ctx->decode_stream, static_cast<const float*>(d_x_f32), d_norm_w, norm_weight_dtype, eps,
                                     static_cast<const uint16_t*>(d_wgate_f16), static_cast<const uint16_t*>(d_wup_f16),
                                     static_cast<float*>(d_hid_f32), (int)rows, ffn, d_model,
@@ -917,7 +918,7 @@ int m40llm_ext_batched_norm_gemm_f32xf16_async(M40llmCudaContext* ctx, const voi
     if (m40_rows_mfma_supported((int)rows, K) && m40_aligned16(d_x_f32) && m40_aligned16(d_norm_w))
         return m40_rows_mfma_plain(ctx, ctx->decode_stream, static_cast<const float*>(d_x_f32), d_norm_w, norm_weight_dtype, eps,
                                    static_cast<const uint16_t*>(d_w_f16), static_cast<float*>(d_out_f32), (int)rows, N, K);
-    if (rows > 8 && m40_aligned16(d_x_f32) && m40_aligned16(d_norm_w))
+    if (rows > 8 && m40_aligned16(d_x_f32) && m40_aligned16(d_norm_w) && m40_apart(d_x_f32, (size_t)rows * K * 4, d_out_f32, (size_t)rows * N * 4))
         return m40_rows_wide_norm(ctx, ctx->decode_stream, static_cast<const float*>(d_x_f32), d_norm_w, norm_weight_dtype, eps,
                                   static_cast<const uint16_t*>(d_w_f16), static_cast<float*>(d_out_f32), (int)rows, N, K);
     PackSpec pk{static_cast<const float*>(d_x_f32), nullptr, d_norm_w, norm_weight_dtype, eps};

@@ -113,3 +113,34 @@ def test_norm_qkv_rope_append(dev, rows, qh, kvh, hd, K, layout, bias):
             close(bits.view(np.float16) / np.abs(want).max(), want / np.abs(want).max(), 1e-3, 1e-4)
     assert np.array_equal(clear.download(np.float32, (77,)), [0.0] * 76 + [5.0])
     kv.destroy()
+
+
+def test_results_that_overlap_the_rows(dev):
+    """One launch reads all rows in every workgroup: results (and what is cleared) in them are refused, a result that is its own residual is not.  The calls for
+    up to 16 rows take a result in place of the rows as before, in two launches."""
+    rng, rows, K, D = np.random.default_rng(4), 12, 1024, 1024
+    a, w = _rows(rng, rows, K), f16bits(rng.standard_normal((D, K)) * 0.03)
+    res, ones = rng.standard_normal((rows, D)).astype(np.float32), np.ones(K, np.float32)
+    da, dw, dn, dres, out = dev.up(a), dev.up(w), dev.up(ones), dev.up(np.concatenate([res.ravel(), np.zeros(4, np.float32)])), dev.zeros(rows * D * 4 + 64)
+    last = da.ptr + rows * K * 4 - 16                  # the rows' last 16 bytes
+    onto, wide = "m40llm_ext_batched_wide_gemm_residual_onto_zero_async", "m40llm_ext_batched_wide_norm_gate_up_swiglu_async"
+    for to in (da.ptr, last, da.ptr - rows * D * 4 + 16):
+        dev.call(onto, da.ptr, dw.ptr, dres.ptr, to, rows, D, K, expect=-6)
+        dev.call("m40llm_ext_batched_wide_norm_gemm_async", da.ptr, dn.ptr, 1, 1e-5, dw.ptr, to, rows, D, K, expect=-6)
+        dev.call(wide, da.ptr, dn.ptr, 1, 1e-5, dw.ptr, dw.ptr, to, rows, D, K, None, 0, expect=-6)
+    dev.call(onto, da.ptr, dw.ptr, dres.ptr, dres.ptr + 16, rows, D, K, expect=-6)          # a residual half under the result
+    dev.call(wide, da.ptr, dn.ptr, 1, 1e-5, dw.ptr, dw.ptr, out.ptr, rows, D, K, last, 4, expect=-6)
+    dev.call(wide, da.ptr, dn.ptr, 1, 1e-5, dw.ptr, dw.ptr, out.ptr, rows, D, K, out.ptr + rows * D * 4 - 16, 8, expect=-6)
+    kv = m40.KVCache(dev.ctx, 64, rows, 2, 64)
+    ids, lens = dev.up(np.arange(rows, dtype=np.uint32)), dev.zeros(rows * 4)
+    dev.call("m40llm_ext_batched_wide_norm_qkv_rope_append_async", kv.h, ids.ptr, lens.ptr, rows, da.ptr, dn.ptr, 1, 1e-5, dw.ptr, dw.ptr, dw.ptr, None, None, None, K, 8, 1e4, 1.0, 0,
+             last, None, 0, expect=-6)
+    dev.sync()
+    assert np.array_equal(da.download(np.float32, (rows, K)), a)                            # nothing was enqueued
+    want = a.astype(np.float64) @ _f64(w).T + res
+    for name in ("m40llm_ext_batched_gemm_residual_f32xf16_async", "m40llm_ext_batched_gemm_residual_onto_zero_f32xf16_async"):
+        dev.call(name, da.ptr, dw.ptr, dres.ptr, da.ptr, rows, D, K)
+        dev.sync()
+        _same(da.download(np.float32, (rows, D)), want)
+        da = dev.up(a)
+    kv.destroy()
