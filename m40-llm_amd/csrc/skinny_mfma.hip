@@ -855,12 +855,6 @@ int m40llm_ext_batched_gemm_residual_onto_zero_f32xf16_async(M40llmCudaContext* 
                                        static_cast<const uint16_t*>(d_w_f16), static_cast<const float*>(d_residual_f32),
                                        static_cast<float*>(d_out_f32), (int)rows, N, K);
     }
-    if (rows > 8 && rows <= 16 && m40_rows_wide_supported((int)rows, K) && m40_aligned16(d_a_f32) && m40_aligned16(d_w_f16) &&
-        apart(d_a_f32, (size_t)rows * K * 4) && apart(d_residual_f32, (size_t)rows * N * 4)) {
-        (void)hipGetLastError();
-        return m40_rows_wide_residual(ctx, ctx->decode_stream, static_cast<const float*>(d_a_f32), static_cast<const uint16_t*>(d_w_f16),
-                                      static_cast<const float*>(d_residual_f32), static_cast<float*>(d_out_f32), (int)rows, N, K, true);
-    }
     // any other shape: the form that overwrites its result
     return m40llm_ext_batched_gemm_residual_f32xf16_async(ctx, d_a_f32, d_w_f16, d_residual_f32, d_out_f32, rows, N, K);
 }

@@ -144,3 +144,16 @@ def test_results_that_overlap_the_rows(dev):
         _same(da.download(np.float32, (rows, D)), want)
         da = dev.up(a)
     kv.destroy()
+
+
+@pytest.mark.parametrize("rows,N,K", [(9, 2048, 1024), (16, 512, 5632), (16, 4097, 2048)])
+def test_results_of_nine_and_more_rows_are_overwritten(dev, rows, N, K):
+    """Only up to eight rows are added onto zeros by the call for up to 16: whatever the result holds before, more rows overwrite it."""
+    rng = np.random.default_rng(rows + N)
+    a, w, res = _rows(rng, rows, K), f16bits(rng.standard_normal((N, K)) * 0.03), rng.standard_normal((rows, N)).astype(np.float32)
+    da, dw, dres, out = dev.up(a), dev.up(w), dev.up(res), dev.up(np.full((rows, N), 7.0, np.float32))
+    want = a.astype(np.float64) @ _f64(w).T + res
+    for _ in range(2):
+        dev.call("m40llm_ext_batched_gemm_residual_onto_zero_f32xf16_async", da.ptr, dw.ptr, dres.ptr, out.ptr, rows, N, K)
+        dev.sync()
+        _same(out.download(np.float32, (rows, N)), want)
