@@ -13,8 +13,8 @@
 // every workgroup as many bytes as two columns of weights; they come from L2 and are requested a chunk ahead.  One workgroup is
 // resident per CU (82 or 148 KB of LDS), which T is chosen for.  Weight loads are whole 128-byte lines
 // (eight lanes a column) and pass through a wave-private LDS tile into operand order, as in rows_mfma.hip; about 64 KB of them per CU
-// are in flight (one, two or four chunks ahead).  A product of few columns onto zeros is cut into two halves of K
-// whose sums are added atomically: two terms onto zero, the same bits in either order.
+// are in flight (one, two or four chunks ahead).  A product of few columns onto zeros is cut into two halves of K, which meet
+// in the result element by element: two terms, the same bits in either order.
 #include "common.hpp"
 
 #include <type_traits>
@@ -167,13 +167,18 @@ __global__ __launch_bounds__(kThreads, 1) void rows_wide_kernel(WideArgs p) {
     for (int u = 0; u < kAhead * T; ++u) issue(b[u], c_begin + u / T, u % T);
     __builtin_amdgcn_sched_barrier(0);
 
-    // what a thread's Q/K/V element needs besides the product (one tile a workgroup), asked for early
+    // what a thread's element needs besides the product (one tile a workgroup), asked for early
     const int e_j = tid & 15, e_row = (tid >> 4) & (16 * RT - 1);
     int q_which = 0, q_col = 0, q_partner = 0;
     bool q_second = false;
     uint32_t q_position = 0, q_seq = 0;
     float bias_own = 0.0f, bias_other = 0.0f;
     float2 q_cs = make_float2(1.0f, 0.0f);
+    float residual_own = 0.0f;
+    if (MODE == kResidual && T == 1 && p.residual) {
+        const int col = 16 * tile0 + e_j;
+        residual_own = p.residual[(size_t)(e_row < p.rows ? e_row : 0) * p.N + (col < p.N ? col : 0)];
+    }
     if (MODE == kQkv) {
         const QkvTile t = qkv_tile(p, tile0);
         const int e_rowc = e_row < p.rows ? e_row : 0;
@@ -360,11 +365,19 @@ __global__ __launch_bounds__(kThreads, 1) void rows_wide_kernel(WideArgs p) {
             }
             float* dst = p.out + (size_t)r * p.N + col;
             if (MODE == kResidual) {
-                if (blockIdx.y == 0 && p.residual) y = p.residual[(size_t)r * p.N + col] + y;
+                const float old = T > 1 && p.residual ? p.residual[(size_t)r * p.N + col] : residual_own;
                 if (gridDim.y > 1) {
-                    atomicAdd(dst, y);
+                    // dst holds +0: the half that comes first leaves its sum there (a zero as -0), the other finds it and adds the residual to the
+                    // whole product, which rounds on the residual's scale once (adding the halves to it one by one rounds there twice: a residual of
+                    // ten times the product, errors of 3.8e-8 instead of 2.8e-8 against 64 bits).  Both see each other past their dies' caches.
+                    const uint32_t left = __float_as_uint(y == 0.0f ? -0.0f : y);
+                    const uint32_t found = __hip_atomic_exchange(reinterpret_cast<uint32_t*>(dst), left, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    if (found == 0u) continue;
+                    y = __uint_as_float(found) + y;
+                    __hip_atomic_store(dst, p.residual ? old + y : y, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                     continue;
                 }
+                if (p.residual) y = old + y;
             }
             *dst = y;
         }
@@ -466,7 +479,7 @@ int m40_rows_wide_norm(M40llmCudaContext* ctx, hipStream_t stream, const float* 
     return launch<kNorm>(ctx, stream, a);
 }
 
-// onto_zero: out holds zeros, so that two halves of K may be added into it where one tile a workgroup would leave half of the CUs idle; a
+// onto_zero: out holds zeros (+0), so that two halves of K can meet in it where one tile a workgroup would leave half of the CUs idle; a
 // residual that is out itself is read before each element is stored, in one part.
 int m40_rows_wide_residual(M40llmCudaContext* ctx, hipStream_t stream, const float* x, const uint16_t* W, const float* residual, float* out, int rows,
                            int N, int K, bool onto_zero) {

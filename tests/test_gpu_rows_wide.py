@@ -157,3 +157,29 @@ def test_results_of_nine_and_more_rows_are_overwritten(dev, rows, N, K):
         dev.call("m40llm_ext_batched_gemm_residual_onto_zero_f32xf16_async", da.ptr, dw.ptr, dres.ptr, out.ptr, rows, N, K)
         dev.sync()
         _same(out.download(np.float32, (rows, N)), want)
+
+
+@pytest.mark.parametrize("rows,N,K", [(9, 2048, 2048), (32, 2048, 5632), (17, 333, 1024), (32, 16000, 768)])
+def test_residual_is_rounded_once(dev, rows, N, K):
+    """The product is finished before a residual of a hundred times its size is added: half a unit in the last place of the result, and the product's own
+    error, at most a third of that here."""
+    rng = np.random.default_rng(rows + K)
+    a, w = rng.standard_normal((rows, K)).astype(np.float32), f16bits(rng.standard_normal((N, K)) / np.sqrt(K))
+    res = (100.0 + 27.0 * rng.random((rows, N))).astype(np.float32) * rng.choice([-1.0, 1.0], (rows, N)).astype(np.float32)
+    a[0] = 0.0                                        # a product of zeros: the residual itself
+    da, dw, dres = dev.up(a), dev.up(w), dev.up(res)
+    want = a.astype(np.float64) @ _f64(w).T + res
+    for _ in range(3):
+        out = dev.zeros(rows * N * 4)
+        dev.call("m40llm_ext_batched_wide_gemm_residual_onto_zero_async", da.ptr, dw.ptr, dres.ptr, out.ptr, rows, N, K)
+        dev.sync()
+        got = out.download(np.float32, (rows, N))
+        assert np.array_equal(got[0], res[0])
+        ulp = np.spacing(np.abs(got)).astype(np.float64)
+        assert (np.abs(got - want) <= 0.5 * ulp + 5.0 * 2.0 ** -22).all()           # products of up to five, their error 1e-7 of that
+    out = dev.zeros(rows * N * 4)
+    dev.call("m40llm_ext_batched_wide_gemm_residual_onto_zero_async", da.ptr, dw.ptr, None, out.ptr, rows, N, K)
+    dev.sync()
+    got = out.download(np.float32, (rows, N))
+    assert not got[0].any()
+    _same(got[1:], (want - res)[1:])
