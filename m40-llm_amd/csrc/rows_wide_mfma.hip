@@ -6,7 +6,7 @@
 // workgroup of eight waves owns T column tiles and walks K in chunks of 512: the chunk's rows become f16 hi + lo fragments
 // (32 or 64 KB, two buffers: the next chunk is converted while this one is multiplied; one power-of-two scale per row and chunk,
 // RMSNorm weights folded in, the RMS factor applied to the sums), the eight waves take 64 k of the chunk each, and their sums meet in
-// LDS once, after the last chunk, in wave order.  So the weights are read once for all rows, every result is written once, nothing is
+// LDS once, after the last chunk, pair by pair.  So the weights are read once for all rows, every result is written once, nothing is
 // left for a second launch and no result depends on timing.
 //
 // Bound: the weight stream, and at one or two tiles a workgroup the chain rows -> fragments -> products of each chunk.  A row costs
@@ -268,16 +268,19 @@ __global__ __launch_bounds__(kThreads, 1) void rows_wide_kernel(WideArgs p) {
         m40_float4 acc[RT];
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) acc[rt] = {0.f, 0.f, 0.f, 0.f};
+        uint4 bw[kSteps];
 #pragma unroll
-        for (int i = 0; i < kSteps; ++i) {
-            const uint4 bw = *reinterpret_cast<const uint4*>(stage + j * kStageRow + 64 * i + 16 * g);
-            const int e = frag_slot((kSteps * wave + i) * 64 + lane);
+        for (int i = 0; i < kSteps; ++i) bw[i] = *reinterpret_cast<const uint4*>(stage + j * kStageRow + 64 * i + 16 * g);
+        // Low parts first, while the sum is small: a chunk's sums then round on the high parts' scale twice, not four times (K 2048 with the norm,
+        // against 64 bits: 1.30e-7 -> 1.17e-7, and 1.12e-7 with the waves' sums added pair by pair instead of one after the other)
 #pragma unroll
-            for (int rt = 0; rt < RT; ++rt) {
-                acc[rt] = mfma16x16x32(planes[(2 * rt) * kPlane + e], bw, acc[rt]);
-                acc[rt] = mfma16x16x32(planes[(2 * rt + 1) * kPlane + e], bw, acc[rt]);
+        for (int part = 1; part >= 0; --part)
+#pragma unroll
+            for (int i = 0; i < kSteps; ++i) {
+                const int e = frag_slot((kSteps * wave + i) * 64 + lane);
+#pragma unroll
+                for (int rt = 0; rt < RT; ++rt) acc[rt] = mfma16x16x32(planes[(2 * rt + part) * kPlane + e], bw[i], acc[rt]);
             }
-        }
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
             const float4 s = *reinterpret_cast<const float4*>(&scale_s[c & 1][16 * rt + 4 * g]);
@@ -311,7 +314,7 @@ __global__ __launch_bounds__(kThreads, 1) void rows_wide_kernel(WideArgs p) {
         }
     }
 
-    // ---- the waves' sums in wave order, and what follows the product
+    // ---- the waves' sums, and what follows the product
     if (NORM) {
         sq = m40_sum16(sq);
         if (kRowLanes == 32) sq = m40_add_xor16(sq);
@@ -327,10 +330,14 @@ __global__ __launch_bounds__(kThreads, 1) void rows_wide_kernel(WideArgs p) {
     __syncthreads();
     auto sum = [&](int t, int r, int col) {              // element (row r, column col) of tile t
         const float* at = red + ((size_t)t * kWaves * RT * 4 + (r >> 4) * 4 + (r & 3)) * 64 + 16 * ((r >> 2) & 3) + col;
-        float s = at[0];
+        float s[kWaves];
 #pragma unroll
-        for (int k = 1; k < kWaves; ++k) s += at[k * RT * 4 * 64];
-        return s;
+        for (int k = 0; k < kWaves; ++k) s[k] = at[k * RT * 4 * 64];
+#pragma unroll
+        for (int n = kWaves / 2; n >= 1; n /= 2)
+#pragma unroll
+            for (int k = 0; k < n; ++k) s[k] += s[k + n];
+        return s[0];
     };
     if (MODE == kQkv) {
         if (tid < 256 * RT && e_row < p.rows && q_position < p.max_seq_len && q_seq < p.max_batch) {

@@ -508,11 +508,14 @@ public:
     }
 
     // What a packed prefill is asked for: the last token's hidden row and logits of every prompt (either may be null), `h` and `lens` being those
-    // of the forward_prefill call before.  Several prompts go through the output norm and lm_head together: one launch reads the head once where
-    // a launch, two copies and a wait for each prompt took 0.1 ms more apiece.
+    // of the forward_prefill call before.  Several prompts go through the output norm and lm_head together (one launch reads the head once where
+    // a launch, two copies and a wait for each prompt took 0.1 ms more apiece) where the logits are no further from 64-bit ones than row by row: errors
+    // in units of 1e-7, together / row by row, rows with and without a few large columns: d_model 256 1.0-1.1 / 0.9-1.0, 768 1.1 / 1.1-1.2, 2048
+    // 1.1-1.2 / 1.3-1.4, 3072 1.2-1.3 / 1.5-1.6, 4096 1.2-1.3 / 1.2 (a row alone takes another kernel there).
+    static constexpr uint32_t kHeadTogetherFrom = 768, kHeadTogetherTo = 3072;
     void last_rows(const float* h, const uint32_t* lens, uint32_t batch, float* hidden_host, float* logits_host) {
         const size_t D = cfg_.d_model, V = cfg_.vocab;
-        if (batch == 1 || mode_ == 0 || !batched_fused_available(batch)) {
+        if (batch == 1 || mode_ == 0 || !batched_fused_available(batch) || D < kHeadTogetherFrom || D > kHeadTogetherTo) {
             size_t row = 0;
             for (uint32_t i = 0; i < batch; ++i) {
                 row += lens[i];
@@ -527,7 +530,9 @@ public:
         for (uint32_t r0 = 0; r0 < batch; r0 += group) {
             const uint32_t n = std::min(group, batch - r0);
             M40H_TRY(m40llm_ext_last_rows_f32_async(ctx_, h, pws_.offsets.u32(r0), pws_.lens.u32(r0), n, cfg_.d_model, ws_.scratch_a.ptr()));
-            if (logits_host) batched_logits_fused(ws_.scratch_a.f32(), n, ws_.logits.f32());
+            if (logits_host)
+                M40H_TRY(m40llm_ext_batched_wide_norm_gemm_async(ctx_, ws_.scratch_a.ptr(), out_norm_, cfg_.norm_weight_dtype, cfg_.rms_eps, lm_head_,
+                                                                 ws_.logits.ptr(), n, (int)V, (int)D));
             M40H_TRY(m40llm_stream_synchronize(ctx_, M40LLM_STREAM_DECODE));
             if (hidden_host) M40H_TRY(m40llm_memcpy_d2h(ctx_, hidden_host + r0 * D, ws_.scratch_a.ptr(), n * D * 4));
             if (logits_host) M40H_TRY(m40llm_memcpy_d2h(ctx_, logits_host + r0 * V, ws_.logits.ptr(), n * V * 4));

@@ -172,6 +172,30 @@ def test_last_rows_of_many_prompts_equal_each_prompt_alone(dev, n):
     dm.close()
 
 
+@pytest.mark.parametrize("n", [2, 5, 8, 9, 33])
+@pytest.mark.parametrize("D", [768, 1024, 2048, 4096])
+def test_logits_of_many_prompts_lose_nothing(dev, D, n):
+    """From 768 to 3072 columns the head takes the prompts together; either way the logits are as near to those in 64 bits as each prompt's alone."""
+    cfg = dict(n_layers=1, d_model=D, q_heads=D // 64, kv_heads=2, head_dim=64, ffn=512, vocab=4003, rms_eps=1e-5, rope_base=10000.0, rope_scale=1.0, rope_layout=0, qkv_bias=False)
+    W = syn.make_weights(cfg, seed=D, std=0.03, emb_std=1.0)
+    W["out_norm"] = (1 + 0.1 * np.random.default_rng(D).standard_normal(D)).astype(np.float32)
+    dm = syn.DeviceModel(dev.ctx, cfg, W, max_seq_len=48, max_sequences=n)
+    rng = np.random.default_rng(n)
+    prompts = [rng.integers(0, 4003, size=1 + (7 * i + n) % 40).tolist() for i in range(n)]
+    found = []
+    for mode in (0, 2):                                             # mode 0: row by row
+        dm.set_mode(mode)
+        hid, log = dm.forward_prefill(list(range(n)), prompts)
+        x = np.asarray(hid).astype(np.float64)
+        want = (x / np.sqrt((x * x).mean(axis=1, keepdims=True) + 1e-5) * W["out_norm"]) @ W["lm_head"].view(np.float16).astype(np.float64).T
+        close(log, want, 1e-5, 1e-6 * float(np.abs(want).max()))
+        found.append(np.sqrt(((log - want) ** 2).sum(axis=1) / (want ** 2).sum(axis=1)))
+    dm.close()
+    # a prompt's error varies with the rounding of its norm's factor, up to 2^-24 on all of its logits: their mean over n prompts, within that over sqrt(n)
+    apart, together = (float(np.sqrt((e * e).mean())) for e in found)
+    assert together <= apart + 2.0 ** -25 / np.sqrt(n), (apart, together)
+
+
 def test_last_rows_gather(dev):
     rng = np.random.default_rng(3)
     x = rng.standard_normal((50, 333)).astype(np.float32)
