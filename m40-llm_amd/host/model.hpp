@@ -148,6 +148,12 @@ public:
             kv_ = m40llm_kvcache_create(ctx, cfg.max_seq_len, slots, cfg.kv_heads, cfg.head_dim);
         }
         if (!kv_) throw std::runtime_error("KV cache allocation failed");
+        auto aligned = [](std::initializer_list<const void*> ps) {
+            return std::all_of(ps.begin(), ps.end(), [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; });
+        };
+        weights_aligned_ = aligned({lm_head, out_norm}) && std::all_of(layers_.begin(), layers_.end(), [&](const LayerWeights& w) {
+            return aligned({w.wq, w.wk, w.wv, w.wo, w.wgate, w.wup, w.wdown, w.attn_norm, w.ffn_norm});
+        });
         ws_.ensure(ctx, cfg, 1);
     }
     ~DecodeModel() override {
@@ -686,9 +692,11 @@ public:
         const uint32_t groups = (rows + kFusedRows - 1) / kFusedRows;
         return (rows + groups - 1) / groups;
     }
+    // The fused calls read weights 16 bytes a load (tensors of a file lie as its alignment says, a caller's pointers anywhere); the
+    // lengths-on-device attention serves two head sizes.
     bool batched_fused_available(uint32_t rows) const {
         return !kvcfg_.is_enabled() && rows >= 1 && cfg_.d_model % 256 == 0 && cfg_.ffn % 256 == 0 &&
-               (cfg_.head_dim == 64 || cfg_.head_dim == 128);   // the lengths-on-device attention serves these two
+               (cfg_.head_dim == 64 || cfg_.head_dim == 128) && weights_aligned_;
     }
     void batched_layer_fused(uint32_t l, const uint32_t* slots_dev, const uint32_t* lens_dev, uint32_t rows, uint32_t hint,
                              const float* d_x, float* d_out) {
@@ -1139,6 +1147,7 @@ private:
     const void* lm_head_;
     const void* tok_emb_;
     KvCompressionConfig kvcfg_;
+    bool weights_aligned_ = false;      // matrices and norms' weights, each to 16 bytes
     M40llmKVCache* kv_ = nullptr;
     ForwardWorkspace ws_;
     PrefillWorkspace pws_;

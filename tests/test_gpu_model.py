@@ -1,5 +1,6 @@
 """Whole decode step through the host layer on the GPU vs the CPU oracle: hidden states and logits within the
 float tolerance, greedy token ids exactly equal (with the smallest top-1/top-2 logit gap reported)."""
+import ctypes as C
 import importlib
 
 import numpy as np
@@ -261,6 +262,53 @@ def test_batched_fused_path_matches_oracle(ctx, orc, rows):
             assert np.array_equal(ids[r], want[int(s)]), (mode, r, ids[r], want[int(s)], gaps[r])
         assert (gaps > 0).all()
         dm.close()
+
+
+class _UploadsOffAlignment:
+    """The library, with uploads of more (or of no more) than `norm_bytes` bytes placed eight bytes past an allocation's start."""
+
+    def __init__(self, lib, norm_bytes, norms):
+        self.lib, self.norm_bytes, self.norms, self.moved = lib, norm_bytes, norms, set()
+
+    def __getattr__(self, name):
+        return getattr(self.lib, name)
+
+    def m40llm_upload_weights(self, h, src, n, out):
+        if (n <= self.norm_bytes) != self.norms:
+            return self.lib.m40llm_upload_weights(h, src, n, out)
+        padded = C.create_string_buffer(n + 8)
+        C.memmove(C.addressof(padded) + 8, src, n)
+        rc = self.lib.m40llm_upload_weights(h, padded, n + 8, out)
+        out._obj.value += 8
+        self.moved.add(out._obj.value)
+        return rc
+
+    def m40llm_device_free(self, h, p):
+        return self.lib.m40llm_device_free(h, p - 8 if p in self.moved else p)
+
+
+@pytest.mark.parametrize("norms", [False, True])
+def test_batches_and_prompts_with_weights_off_alignment(ctx, norms):
+    """Weights (or norms' weights only) that no 16-byte load may read: batched decode and the logits of several prompts take the reference's calls."""
+    cfg = dict(_toy_cfg(0, False, 64), d_model=768, q_heads=12, kv_heads=2, ffn=512, n_layers=1)
+    W = syn.make_weights(cfg, seed=11, std=0.05, emb_std=1.0)
+    n, rng = 20, np.random.default_rng(5)
+    prompts = [rng.integers(0, cfg["vocab"], size=1 + 3 * i % 11).tolist() for i in range(n)]
+    real = ctx.lib
+    try:
+        ctx.lib = _UploadsOffAlignment(real, 768 * 4, norms)
+        dm = syn.DeviceModel(ctx, cfg, W, max_seq_len=32, max_sequences=n)
+        found = []
+        for mode in (0, 2):
+            dm.set_mode(mode)
+            hid, log = dm.forward_prefill(list(range(n)), prompts)
+            lens, toks = np.array([len(p) for p in prompts], np.uint32), np.argmax(log, axis=1).astype(np.uint32)
+            found.append((hid, log, dm.decode_batch_greedy(np.arange(n), lens, toks, 6)[0], dm.decode_batch_greedy(np.arange(12), lens[:12], toks[:12], 6)[0]))
+        dm.close()
+    finally:
+        ctx.lib = real
+    for got, want in zip(found[1], found[0]):
+        assert np.array_equal(got, want)
 
 
 @pytest.mark.parametrize("layout,bias,hd", [(0, False, 64), (1, True, 128)])
