@@ -945,7 +945,7 @@ public:
     // first_tokens[r] is the input of step 0.  ids_out: [rows][steps], gaps_out (optional) likewise.
     void decode_batch_greedy(const uint32_t* seq_ids, const uint32_t* kv_lens, const uint32_t* first_tokens,
                              uint32_t rows, uint32_t steps, uint32_t* ids_out, float* gaps_out) override {
-        if (mode_ >= 1 && batched_fused_available(rows)) {
+        if (mode_ >= 1 && steps > 0 && batched_fused_available(rows)) {
             if (decode_batch_device(seq_ids, kv_lens, first_tokens, rows, 0, steps, ids_out, gaps_out, nullptr)) return;
             // near-tie somewhere: redo on the host-sampled path (same cache rows are rewritten)
         }
@@ -1004,7 +1004,7 @@ public:
     void decode_batch_timed(const uint32_t* seq_ids, const uint32_t* kv_lens, const uint32_t* first_tokens, uint32_t rows,
                             uint32_t warmup, uint32_t steps, uint32_t* ids_out, double* elapsed_ms) override {
         last_timed_host_fallback_ = false;
-        if (mode_ >= 1 && batched_fused_available(rows)) {
+        if (mode_ >= 1 && warmup + steps > 0 && batched_fused_available(rows)) {
             if (decode_batch_device(seq_ids, kv_lens, first_tokens, rows, warmup, steps, ids_out, nullptr, elapsed_ms)) return;
             last_timed_host_fallback_ = true;   // as in decode_timed: redo everything on the host-sampled path
         }

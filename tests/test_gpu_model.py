@@ -311,6 +311,18 @@ def test_batches_and_prompts_with_weights_off_alignment(ctx, norms):
         assert np.array_equal(got, want)
 
 
+@pytest.mark.parametrize("rows", [3, 20])
+def test_batched_decode_of_no_steps(ctx, rows):
+    cfg = dict(_toy_cfg(0, False, 64), ffn=512, n_layers=1)
+    dm = syn.DeviceModel(ctx, cfg, syn.make_weights(cfg, seed=1, std=0.08, emb_std=1.0), max_seq_len=16, max_sequences=rows)
+    for mode in (0, 1, 2):
+        dm.set_mode(mode)
+        ids, gaps = dm.decode_batch_greedy(np.arange(rows), np.ones(rows, np.uint32), np.ones(rows, np.uint32), 0)
+        assert ids.shape == gaps.shape == (rows, 0)
+        dm.decode_batch_timed(np.arange(rows), np.ones(rows, np.uint32), np.ones(rows, np.uint32), 0, 0)
+    dm.close()
+
+
 @pytest.mark.parametrize("layout,bias,hd", [(0, False, 64), (1, True, 128)])
 def test_fused_and_graph_paths_equal_reference_call_sequence(ctx, orc, layout, bias, hd):
     """The fused single-stream path (mode 1) and its graph replay (mode 2) run the same arithmetic as the
