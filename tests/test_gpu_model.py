@@ -229,9 +229,9 @@ def test_qwen_shape_reduced_depth_batched_greedy_ids(ctx, orc):
         dm.close()
 
 
-@pytest.mark.parametrize("rows", [1, 4, 11])
+@pytest.mark.parametrize("rows", [1, 4, 11, 16, 17, 32, 33, 65, 70])
 def test_batched_fused_path_matches_oracle(ctx, orc, rows):
-    """Fused row-batched step (modes 1 and 2; stacked MFMA rows up to 8, two fragment sets above): greedy ids equal to
+    """Fused row-batched step (modes 1 and 2; up to 8 rows, one or two tiles of 16 rows up to 32, equal groups of those beyond): greedy ids equal to
     the oracle's per-sequence decode and to the reference call sequence, across a 512-token length bucket boundary."""
     cfg = _toy_cfg(1, True, 128); cfg["ffn"] = 512
     W = syn.make_weights(cfg, seed=7, std=0.08, emb_std=1.0)

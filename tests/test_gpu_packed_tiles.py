@@ -49,6 +49,34 @@ def test_few_rows_waves_and_pairs(ctx, rows, n, k):
     assert np.array_equal(got[:, n:], old[:, n:])
 
 
+# up to 4, 8 and 16 sums of k tiles (fewer than 16, fewer than 64, more), each kept by one wave, or by 8 or 4 waves that keep two or four of them
+@pytest.mark.parametrize("k", [480, 512, 2016, 2048, 2080])
+@pytest.mark.parametrize("rows", [1, 16, 20, 64])
+def test_waves_and_pairs_change_no_bit(ctx, rows, k):
+    rng = np.random.default_rng(rows + k)
+    tiles = [4, 400, 600]                              # times up to one tile of rows: up to a CU each, up to two, more
+    A, W = rng.standard_normal((rows, k)), bf16w(rng, 16 * tiles[-1], k)
+    got = [gemm(ctx, "bfloat16", STORE, A, W[:16 * t], out_f32=np.zeros((rows, 16 * t), np.float32), ld_out=16 * t, cols=16 * t)["out_f32"] for t in tiles]
+    assert np.abs(got[0]).max(axis=1).min() > 0
+    for g in got[1:]:
+        assert np.array_equal(g[:, :64].view(np.uint32), got[0].view(np.uint32))
+    assert np.array_equal(got[1].view(np.uint32), got[2][:, :16 * tiles[1]].view(np.uint32))
+    last = 16 * tiles[-1] - 64                         # and the wide product's last columns by a narrow one
+    tail = gemm(ctx, "bfloat16", STORE, A, W[last:], out_f32=np.zeros((rows, 64), np.float32), ld_out=64, cols=64)["out_f32"]
+    assert np.array_equal(got[2][:, last:].view(np.uint32), tail.view(np.uint32))
+
+
+# 64 x 64 tiles (two k tiles a stage), 64 x 128, 128 x 128 (one and two a stage), 128 x 256 (long sums)
+@pytest.mark.parametrize("k", [992, 2048, 2112])
+def test_tile_shapes_change_no_bit(ctx, k):
+    rng, n = np.random.default_rng(k), 2048
+    A, W = rng.standard_normal((4096, k)), bf16w(rng, n, k)
+    product = lambda first, rows: gemm(ctx, "bfloat16", STORE, A[first:first + rows], W, out_f32=np.zeros((rows, n), np.float32), ld_out=n, cols=n)["out_f32"].view(np.uint32)
+    whole = product(0, 4096)
+    for first, rows in ((0, 65), (4000, 77), (100, 300), (2048, 700), (1000, 1300), (16, 2500)):
+        assert np.array_equal(product(first, rows), whole[first:first + rows]), (first, rows)
+
+
 @pytest.mark.parametrize("rows,ff,k", [(1, 4112, 512), (20, 4200, 352), (65, 64, 64), (129, 1024, 352), (300, 72, 128), (700, 1024, 96), (1300, 1504, 160), (4096, 1024, 64)])
 def test_tiles_gated_pairs(ctx, rows, ff, k):
     """The first 32 columns plain, then pairs of tiles of gate and up."""

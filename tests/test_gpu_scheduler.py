@@ -53,6 +53,40 @@ def test_scheduler_outputs_equal_oracle_greedy_per_request(ctx, orc, mode, hd):
     dm.close()
 
 
+def test_steps_of_more_rows_than_a_group_equal_each_request_alone(ctx, orc):
+    """70 requests, up to 70 rows a step in groups of up to 32: greedy rows, picked on the device, equal the oracle; rows in between that are sampled from
+    their logits equal the same request alone."""
+    n = 70
+    cfg = dict(n_layers=2, d_model=256, q_heads=4, kv_heads=2, head_dim=64, ffn=512, vocab=300, rms_eps=1e-5, rope_base=10000.0, rope_scale=1.0, rope_layout=0, qkv_bias=False)
+    W = syn.make_weights(cfg, seed=12, std=0.08, emb_std=1.0)
+    dm = syn.DeviceModel(ctx, cfg, W, max_seq_len=64, max_sequences=n)
+    dm.set_mode(2)
+    om = orc.Model(cfg, W)
+    rng = np.random.default_rng(9)
+    specs = [(rng.integers(0, 300, size=1 + 5 * i % 23).tolist(), dict(max_tokens=3 + i % 6, **(dict(temperature=0.8, top_k=40, seed=i) if i % 3 == 1 else {}))) for i in range(n)]
+    s = sch.Scheduler.for_model(dm)
+    rids = [s.submit(p, **kw) for p, kw in specs[:40]]
+    s.tick()
+    s.tick()
+    rids += [s.submit(p, **kw) for p, kw in specs[40:]]             # slots and rows in an order of their own
+    s.run_until_idle(200)
+    found = [s.generated(r) for r in rids]
+    assert all(s.state(r) == "complete" for r in rids)
+    s.close()
+    alone = sch.Scheduler.for_model(dm)
+    for i, (prompt, kw) in enumerate(specs):
+        if "seed" in kw:
+            rid = alone.submit(prompt, **kw)
+            alone.run_until_idle(200)
+            want = alone.generated(rid)
+        else:
+            om.alloc_kv(64, 1)
+            want = om.decode_greedy(0, prompt, kw["max_tokens"])[0][len(prompt):].tolist()
+        assert found[i] == want, i
+    alone.close()
+    dm.close()
+
+
 def test_scheduler_full_depth_tinyllama_requests_equal_oracle(ctx, orc, heartbeat):
     """The scheduler at the full BASELINE config-2 shape (22 layers): six requests with prompts of 40-150 tokens on four
     slots, arrivals spread over the ticks, so that packed prefills of one to three prompts, batched decode steps of one to
