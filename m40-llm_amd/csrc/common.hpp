@@ -167,7 +167,7 @@ int m40_rows_wide_norm(M40llmCudaContext* ctx, hipStream_t stream, const float* 
                        const uint16_t* W, float* out, int rows, int N, int K);
 int m40_rows_wide_residual(M40llmCudaContext* ctx, hipStream_t stream, const float* x, const uint16_t* W, const float* residual, float* out, int rows,
                            int N, int K, bool onto_zero);
-// many-row f32 x f16 GEMM on 128 x 128 tiles (gemm_tiled.hip): M > 32, K a multiple of 32, 16-byte aligned operands
+// many-row f32 x f16 GEMM on tiles of 64 x 64 to 128 x 256 (gemm_tiled.hip): M > 32, K a multiple of 32, 16-byte aligned operands
 bool m40_gemm_tiled_supported(const void* A, const void* B, int M, int N, int K);
 int m40_launch_gemm_tiled(M40llmCudaContext* ctx, hipStream_t stream, uint32_t stream_kind, const float* A, const uint16_t* B,
                           float* C, int M, int N, int K);
