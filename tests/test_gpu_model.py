@@ -229,11 +229,12 @@ def test_qwen_shape_reduced_depth_batched_greedy_ids(ctx, orc):
         dm.close()
 
 
-@pytest.mark.parametrize("rows", [1, 4, 11, 16, 17, 32, 33, 65, 70])
-def test_batched_fused_path_matches_oracle(ctx, orc, rows):
-    """Fused row-batched step (modes 1 and 2; up to 8 rows, one or two tiles of 16 rows up to 32, equal groups of those beyond): greedy ids equal to
+@pytest.mark.parametrize("rows,heads,ffn", [(rows, 4, 512) for rows in (1, 4, 11, 16, 17, 32, 33, 65, 70)] + [(rows, 8, 1280) for rows in (9, 16, 32, 33, 70)])
+def test_batched_fused_path_matches_oracle(ctx, orc, rows, heads, ffn):
+    """Fused row-batched step (modes 1 and 2; up to 8 rows, one or two tiles of 16 rows up to 32, equal groups of those beyond; from 1024 columns on O and
+    down in two halves of K that meet in a result cleared by the launch before): greedy ids equal to
     the oracle's per-sequence decode and to the reference call sequence, across a 512-token length bucket boundary."""
-    cfg = _toy_cfg(1, True, 128); cfg["ffn"] = 512
+    cfg = dict(_toy_cfg(1, True, 128), q_heads=heads, d_model=128 * heads, ffn=ffn)
     W = syn.make_weights(cfg, seed=7, std=0.08, emb_std=1.0)
     S, steps = 560, 8
     rng = np.random.default_rng(rows)
