@@ -3,18 +3,21 @@
 //
 // rows_mfma.hip keeps eight whole rows as operand fragments in LDS, which more rows do not fit; skinny_mfma.hip converts every step
 // of the rows once per 64 columns and adds its K slices in a second launch, and reads the weights once per sixteen rows.  Here a
-// workgroup of eight waves owns T column tiles and walks K in chunks of 512: the chunk's rows become f16 hi + lo fragments
-// (32 or 64 KB, two buffers: the next chunk is converted while this one is multiplied; one power-of-two scale per row and chunk,
-// RMSNorm weights folded in, the RMS factor applied to the sums), the eight waves take 64 k of the chunk each, and their sums meet in
-// LDS once, after the last chunk, pair by pair.  So the weights are read once for all rows, every result is written once, nothing is
-// left for a second launch and no result depends on timing.
+// workgroup of eight waves owns T column tiles, and a wave walks blocks of 64 k, every eighth: it turns its block of the rows into f16 hi + lo
+// operands (one power-of-two scale per row and block, RMSNorm weights folded in, the RMS factor applied to the sums) and multiplies them
+// with its block of every tile.  The waves share nothing until their sums meet in LDS once, after the last block, pair by pair.  So the weights
+// are read once for all rows, every result is written once, nothing is left for a second launch and no result depends on timing.
 //
-// Bound: the weight stream, and at one or two tiles a workgroup the chain rows -> fragments -> products of each chunk.  A row costs
-// every workgroup as many bytes as two columns of weights; they come from L2 and are requested a chunk ahead.  One workgroup is
-// resident per CU (82 or 148 KB of LDS), which T is chosen for.  Weight loads are whole 128-byte lines
-// (eight lanes a column) and pass through a wave-private LDS tile into operand order, as in rows_mfma.hip; about 64 KB of them per CU
-// are in flight (one, two or four chunks ahead).  A product of few columns onto zeros is cut into two halves of K, which meet
-// in the result element by element: two terms, the same bits in either order.
+// Bound: a launch of one tile a workgroup has about 5 us that no block takes part in (launch, arguments and first requests 2.5, sums and results
+// 2), and a block then costs a wave 1.3 us: rows in (8 KB from L2), two passes through LDS, about 200 vector instructions, and two waves a
+// SIMD to hide them.  The rows are asked for a quarter of a kilobyte of four rows at a time, whole lines: in operand order (16 rows of 64 bytes an
+// instruction) every workgroup reading 32 rows of 2048 takes 11.5 us instead of 4.7.  Requests go out one block ahead and no further: two or
+// four blocks of weights or rows on their way (more code, more registers, waits for what was asked for later) take 0.6 to 1.4 us more a launch.
+// 32 rows, width 2048, feed-forward 5632, against the form that converted chunks of 512 k for all waves between barriers: Q/K/V 13.9 -> 11.5 us, O
+// 7.6 -> 6.7, gate/up 19.0 -> 15.7, down 14.6 -> 11.8, vocabulary of 32000 39.4 -> 35.2; 16 rows 10.1 -> 8.3, 6.2 -> 5.4, 14.6 -> 13.8, 11.4 -> 10.0,
+// 31.4 -> 30.5.  Weight loads are whole 128-byte lines (eight lanes a column) and pass through a wave-private LDS tile into operand order, as in
+// rows_mfma.hip.  A product of few columns onto zeros is cut into two halves of K, which meet in the result element by element: two terms, the
+// same bits in either order.
 #include "common.hpp"
 
 #include <type_traits>
@@ -22,29 +25,26 @@
 namespace {
 
 constexpr int kWaves = 8, kThreads = 64 * kWaves;
-constexpr int kChunk = 512;                             // k per chunk
-constexpr int kShare = kChunk / kWaves;                 // k per wave and chunk
+constexpr int kShare = 64;                              // k of a block: what one wave converts and multiplies at a time
 constexpr int kSteps = kShare / 32;                     // matrix instructions deep
-constexpr int kRunLanes = kShare * 2 / 16;              // lanes that cover a column's share with 16 bytes each
+constexpr int kRunLanes = kShare * 2 / 16;              // lanes that cover a column's block with 16 bytes each
 constexpr int kColsPerLoad = 64 / kRunLanes;
 constexpr int kLoads = 16 / kColsPerLoad;
 constexpr int kStageRow = kShare * 2 + 16;              // LDS bytes per column: +16 spreads the columns over the banks
-constexpr int kStageBytes = 16 * kStageRow;             // per wave
-constexpr int kPlane = kChunk / 32 * 64;                // 16-byte entries of one 16-row operand plane of a chunk
+constexpr int kStageBytes = 16 * kStageRow;             // of one column tile
+constexpr int kRowBytes = kShare * 4 + 16;              // LDS bytes per row
+
+constexpr int wide_stages(int t) { return t > 1 ? 2 : 1; }      // column tiles a wave has in LDS
 
 enum Mode { kResidual = 0, kSwiglu = 1, kQkv = 2, kNorm = 3 };
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 
 __device__ __forceinline__ m40_float4 mfma16x16x32(const uint4& a, const uint4& b, m40_float4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(m40_half8, a), __builtin_bit_cast(m40_half8, b), c, 0, 0, 0);
 }
-
-// Where entry e of an operand plane ([k-step][lane]) lies: the row (low four bits) xor-ed with the four bits above, so that the lanes of
-// the conversion, which hold one row at consecutive eights of k, spread over the banks.
-__device__ __forceinline__ int frag_slot(int e) { return e ^ ((e >> 4) & 15); }
 
 struct WideArgs {
     const float* x;               // [rows][K]
@@ -54,7 +54,7 @@ struct WideArgs {
     const uint16_t *W0, *W1, *W2; // kSwiglu: gate, up; kQkv: q, k, v
     float* out;                   // [rows][N]
     const float* residual;        // kResidual: added to the product, or null
-    int rows, N, K, tiles, chunks;
+    int rows, N, K, tiles, blocks;
     float* zero;                  // cleared on the side, or null
     int zero_count;
     const float *bq, *bk, *bv;
@@ -92,89 +92,24 @@ __device__ __forceinline__ int qkv_col(const WideArgs& p, const QkvTile& t, int 
 template <int MODE, int RT, int T>
 __global__ __launch_bounds__(kThreads, 1) void rows_wide_kernel(WideArgs p) {
     constexpr bool NORM = MODE != kResidual;
-    constexpr int kRowLanes = 32 / RT;                  // lanes that convert one row
-    constexpr int kEights = kChunk / 8 / kRowLanes;     // eights of k per lane and chunk
-    constexpr int kAhead = T >= 3 ? 1 : 4 / T;          // chunks between a weight request and its use
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-    uint4* frag = reinterpret_cast<uint4*>(lds);        // [2 buffers][RT][hi, lo][kPlane]
-    uint8_t* stage = lds + 2 * RT * 2 * kPlane * 16 + (threadIdx.x >> 6) * kStageBytes;
-    __shared__ __attribute__((aligned(16))) float scale_s[2][16 * RT];      // undoes the chunk's scaling of each row
-    __shared__ float factor_s[16 * RT];                                     // RMSNorm factor of each row
+    __shared__ __attribute__((aligned(16))) float scale_s[kWaves][16 * RT];      // undoes the scaling of each row's block
+    __shared__ float square_s[kWaves][16 * RT];
+    __shared__ float factor_s[16 * RT];                                          // RMSNorm factor of each row
 
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, j = lane & 15, g = lane >> 4;
-    const int c_begin = p.chunks * (int)blockIdx.y / (int)gridDim.y, c_end = p.chunks * ((int)blockIdx.y + 1) / (int)gridDim.y;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, j = lane & 15, g = lane >> 4;
+    const int b_begin = p.blocks * (int)blockIdx.y / (int)gridDim.y, b_end = p.blocks * ((int)blockIdx.y + 1) / (int)gridDim.y;
     const int tile0 = (int)blockIdx.x * T;
+    constexpr int kStages = wide_stages(T);
+    uint8_t* stage = lds + wave * (kStages * kStageBytes + 16 * kRowBytes);
+    uint8_t* rows_lds = stage + kStages * kStageBytes;
 
-    // ---- rows of a chunk, requested ahead: 8-element pieces l, l + kRowLanes, ... of the thread's row
-    const int row = tid / kRowLanes, l = tid % kRowLanes;
-    const bool live = row < p.rows;
-    const float* xr = p.x + (size_t)(live ? row : 0) * p.K;
-    const int eights = p.K / 8;
-    float4 v[2 * kEights];
-    uint4 w[NORM ? 2 * kEights : 1];
-    const bool norm16 = NORM && p.norm_dtype == 0u;
-    const int w_mul = norm16 ? 1 : 2, w_second = norm16 ? 0 : 1;
-    auto load_rows = [&](int c) {
-#pragma unroll
-        for (int i = 0; i < kEights; ++i) {
-            int at = c * (kChunk / 8) + l + kRowLanes * i;
-            at = at < eights ? at : 0;
-            v[2 * i] = reinterpret_cast<const float4*>(xr)[2 * at];
-            v[2 * i + 1] = reinterpret_cast<const float4*>(xr)[2 * at + 1];
-            if (NORM) {      // f16 weights are 16 bytes an eight, requested twice: no load under a branch
-                w[2 * i] = static_cast<const uint4*>(p.norm_w)[w_mul * at];
-                w[2 * i + 1] = static_cast<const uint4*>(p.norm_w)[w_mul * at + w_second];
-            }
-        }
-    };
-    load_rows(c_begin);
-    __builtin_amdgcn_sched_barrier(0);
-
-    // ---- weights: instruction li of a wave reads its 64 k of columns 8 li .. 8 li + 7 of a tile
-    const int run_lane = lane % kRunLanes, run_col = lane / kRunLanes;
-    const uint16_t* col_ptr[T][kLoads];
-#pragma unroll
-    for (int t = 0; t < T; ++t) {
-        const int tile = tile0 + t < p.tiles ? tile0 + t : p.tiles - 1;
-#pragma unroll
-        for (int li = 0; li < kLoads; ++li) {
-            const int i = li * kColsPerLoad + run_col;
-            const uint16_t* W = p.W0;
-            int col;
-            if (MODE == kSwiglu) {
-                col = 8 * tile + (i & 7);
-                if (li * kColsPerLoad & 8) W = p.W1;
-                col = col < p.N ? col : p.N - 1;
-            } else if (MODE == kQkv) {
-                const QkvTile q = qkv_tile(p, tile);
-                col = qkv_col(p, q, i);
-                W = q.which == 0 ? p.W0 : (q.which == 1 ? p.W1 : p.W2);
-            } else {
-                col = 16 * tile + i;
-                col = col < p.N ? col : p.N - 1;
-            }
-            col_ptr[t][li] = W + (size_t)col * p.K;
-        }
-    }
-    uint4 b[kAhead * T][kLoads];
-    auto issue = [&](uint4 (&dst)[kLoads], int c, int t) {
-        const int k = c * kChunk + wave * kShare + 8 * run_lane;
-        const int at = c < c_end && k < p.K ? k : 0;       // past the end: a valid address, the value is not used
-#pragma unroll
-        for (int li = 0; li < kLoads; ++li) dst[li] = *reinterpret_cast<const uint4*>(col_ptr[t][li] + at);
-    };
-#pragma unroll
-    for (int u = 0; u < kAhead * T; ++u) issue(b[u], c_begin + u / T, u % T);
-    __builtin_amdgcn_sched_barrier(0);
-
-    // what a thread's element needs besides the product (one tile a workgroup), asked for early
+    // ---- what a thread's element needs besides the product (one tile a workgroup), asked for before anything else
     const int e_j = tid & 15, e_row = (tid >> 4) & (16 * RT - 1);
     int q_which = 0, q_col = 0, q_partner = 0;
     bool q_second = false;
-    uint32_t q_position = 0, q_seq = 0;
-    float bias_own = 0.0f, bias_other = 0.0f;
-    float2 q_cs = make_float2(1.0f, 0.0f);
-    float residual_own = 0.0f;
+    uint32_t q_position = 0, q_seq = 0, q_off = 0;
+    float bias_own = 0.0f, bias_other = 0.0f, residual_own = 0.0f;
     if (MODE == kResidual && T == 1 && p.residual) {
         const int col = 16 * tile0 + e_j;
         residual_own = p.residual[(size_t)(e_row < p.rows ? e_row : 0) * p.N + (col < p.N ? col : 0)];
@@ -186,141 +121,191 @@ __global__ __launch_bounds__(kThreads, 1) void rows_wide_kernel(WideArgs p) {
         q_col = qkv_col(p, t, e_j);
         q_partner = t.split ? e_j ^ 8 : e_j ^ 1;
         q_second = t.split ? (e_j & 8) != 0 : (e_j & 1) != 0;
-        const uint32_t off = t.split ? (uint32_t)(8 * t.tt + (e_j & 7)) : (uint32_t)((16 * t.tt + e_j) >> 1);
+        q_off = t.split ? (uint32_t)(8 * t.tt + (e_j & 7)) : (uint32_t)((16 * t.tt + e_j) >> 1);
         const float* bias = t.which == 0 ? p.bq : (t.which == 1 ? p.bk : p.bv);
         q_position = p.lens_dev[e_rowc];
         q_seq = p.ids_dev[e_rowc];
         bias_own = bias ? bias[q_col] : 0.0f;
         bias_other = bias ? bias[qkv_col(p, t, q_partner)] : 0.0f;
-        const float freq = p.rope_table ? p.rope_table[off] : m40_rope_inv_freq(off, p.head_dim, p.rope_base);
-        if (t.which != 2) q_cs = m40_rope_cos_sin_freq(q_position, freq, p.rope_scale);
     }
+    __builtin_amdgcn_sched_barrier(0);
 
-    // ---- rows of chunk c -> f16 hi + lo fragments of buffer c & 1
-    float sq = 0.0f;
-    auto convert = [&](int c) {
-        float x[kEights][8];
-        float mx = 0.0f;
+    // ---- rows of a block, one ahead: lane (j, g) asks for the elements 4 j .. 4 j + 3 of rows g, 4 + g, 8 + g, ...
+    constexpr int kRowLoads = 4 * RT;
+    uint32_t x_at[kRowLoads];
 #pragma unroll
-        for (int i = 0; i < kEights; ++i) {
-            const float4 a0 = v[2 * i], a1 = v[2 * i + 1];
-            const float a[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
-            const bool in = live && c * (kChunk / 8) + l + kRowLanes * i < eights;
-            float f[8] = {1.0f, 1.0f, 1.0f, 1.0f, 1.0f, 1.0f, 1.0f, 1.0f};
-            if (NORM) {
-                if (norm16) {
-                    m40_unpack8(w[2 * i], f);
-                } else {
-                    const uint4 f0 = w[2 * i], f1 = w[2 * i + 1];
-                    const uint32_t u[8] = {f0.x, f0.y, f0.z, f0.w, f1.x, f1.y, f1.z, f1.w};
+    for (int u = 0; u < kRowLoads; ++u) x_at[u] = (uint32_t)(4 * u + g < p.rows ? 4 * u + g : 0) * (uint32_t)p.K + 4u * j;
+    float4 x[kRowLoads];
+    uint4 nw;
+    const bool norm16 = NORM && p.norm_dtype == 0u;
+    auto load_rows = [&](int kb) {
+        kb = kb < b_end ? kb : 0;         // past the end: a valid address, the values are not used
+        const float* from = p.x + (size_t)kb * kShare;
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) f[e] = __uint_as_float(u[e]);
-                }
-            }
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const float y = in ? a[e] : 0.0f;
-                if (NORM) sq = fmaf(y, y, sq);
-                x[i][e] = NORM ? (in ? y * f[e] : 0.0f) : y;
-                mx = fmaxf(mx, fabsf(x[i][e]));
-            }
-        }
-        mx = m40_max16(mx);
-        if (kRowLanes == 32) mx = m40_max_xor16(mx);
-        float scale = 1.0f, inv_scale = 1.0f;
-        if (mx > 0.0f && mx < INFINITY) {
-            int ex;
-            (void)frexpf(mx, &ex);        // mx = f * 2^ex, f in [0.5, 1)
-            ex -= 11;                     // scaled maximum in [2^10, 2^11)
-            ex = ex < -100 ? -100 : (ex > 100 ? 100 : ex);
-            scale = ldexpf(1.0f, ex);
-            inv_scale = ldexpf(1.0f, -ex);
-        }
-        uint4* plane = frag + (size_t)(((c & 1) * RT + (row >> 4)) * 2) * kPlane;
-#pragma unroll
-        for (int i = 0; i < kEights; ++i) {
-            uint32_t hi[4], lo[4];
-#pragma unroll
-            for (int e = 0; e < 8; e += 2) {
-                const f32x2 s2 = {x[i][e] * inv_scale, x[i][e + 1] * inv_scale};
-                const f16x2 h2 = __builtin_convertvector(s2, f16x2);
-                const f16x2 l2 = __builtin_convertvector(s2 - __builtin_convertvector(h2, f32x2), f16x2);
-                hi[e / 2] = __builtin_bit_cast(uint32_t, h2);
-                lo[e / 2] = __builtin_bit_cast(uint32_t, l2);
-            }
-            const int eight = l + kRowLanes * i;
-            const int entry = frag_slot((eight >> 2) * 64 + (eight & 3) * 16 + (row & 15));
-            plane[entry] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
-            plane[kPlane + entry] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
-        }
-        if (l == 0) scale_s[c & 1][row] = scale;
+        for (int u = 0; u < kRowLoads; ++u) x[u] = *reinterpret_cast<const float4*>(from + x_at[u]);
+        // f16 weights: the sixteen bytes that hold the lane's four
+        if (NORM) nw = *(static_cast<const uint4*>(p.norm_w) + (norm16 ? kb * (kShare / 8) : kb * (kShare / 4)) + (norm16 ? j >> 1 : j));
     };
-    convert(c_begin);
-    __syncthreads();
+    load_rows(b_begin + wave);
+    __builtin_amdgcn_sched_barrier(0);
+
+    // ---- weights: instruction li of a wave reads its 64 k of columns 8 li .. 8 li + 7 of a tile
+    const int run_lane = lane % kRunLanes, run_col = lane / kRunLanes;
+    const uint16_t* tile_w[T][kLoads];
+    uint32_t w_at[T][kLoads];
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+        const int tile = tile0 + t < p.tiles ? tile0 + t : p.tiles - 1;
+        if (MODE == kQkv) {
+            const QkvTile q = qkv_tile(p, tile);
+            const int first = qkv_col(p, q, 0);
+#pragma unroll
+            for (int li = 0; li < kLoads; ++li) {
+                tile_w[t][li] = (q.which == 0 ? p.W0 : (q.which == 1 ? p.W1 : p.W2)) + (size_t)first * p.K;
+                w_at[t][li] = (uint32_t)(qkv_col(p, q, li * kColsPerLoad + run_col) - first) * (uint32_t)p.K + 8u * run_lane;
+            }
+        } else {
+            constexpr int kCols = MODE == kSwiglu ? 8 : 16;
+#pragma unroll
+            for (int li = 0; li < kLoads; ++li) {
+                const int c = MODE == kSwiglu ? run_col : li * kColsPerLoad + run_col, left = p.N - 1 - kCols * tile;
+                tile_w[t][li] = (MODE == kSwiglu && li * kColsPerLoad >= 8 ? p.W1 : p.W0) + (size_t)(kCols * tile) * p.K;
+                w_at[t][li] = (uint32_t)(c < left ? c : left) * (uint32_t)p.K + 8u * run_lane;
+            }
+        }
+    }
+    uint4 b[T][kLoads];
+    auto issue = [&](int kb, int t) {
+        kb = kb < b_end ? kb : 0;       // past the end: a valid address, the value is not used
+#pragma unroll
+        for (int li = 0; li < kLoads; ++li) b[t][li] = *reinterpret_cast<const uint4*>(tile_w[t][li] + (size_t)kb * kShare + w_at[t][li]);
+    };
+#pragma unroll
+    for (int t = 0; t < T; ++t) issue(b_begin + wave, t);
+    __builtin_amdgcn_sched_barrier(0);
+
+    // ---- rows of a block -> f16 hi + lo operands, through an LDS tile of the wave's own: lane (j, g) takes the elements k = 32 i + 8 g .. + 7
+    // of rows j and 16 + j
+    float sq[kRowLoads];
+    uint4 hi[RT][kSteps], lo[RT][kSteps];
+#pragma unroll
+    for (int u = 0; u < kRowLoads; ++u) sq[u] = 0.0f;
+    auto convert = [&]() {
+        float m[4] = {1.0f, 1.0f, 1.0f, 1.0f};
+        if (NORM) {
+            const uint4 w = nw;
+            const uint32_t w0 = j & 1 ? w.z : w.x, w1 = j & 1 ? w.w : w.y;
+            m[0] = norm16 ? m40_h2f((uint16_t)(w0 & 0xffffu)) : __uint_as_float(w.x);
+            m[1] = norm16 ? m40_h2f((uint16_t)(w0 >> 16)) : __uint_as_float(w.y);
+            m[2] = norm16 ? m40_h2f((uint16_t)(w1 & 0xffffu)) : __uint_as_float(w.z);
+            m[3] = norm16 ? m40_h2f((uint16_t)(w1 >> 16)) : __uint_as_float(w.w);
+        }
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+#pragma unroll
+            for (int u = 4 * rt; u < 4 * rt + 4; ++u) {
+                const float4 a = x[u];
+                if (NORM) sq[u] = fmaf(a.x, a.x, fmaf(a.y, a.y, fmaf(a.z, a.z, fmaf(a.w, a.w, sq[u]))));
+                *reinterpret_cast<f32x4*>(rows_lds + (4 * (u & 3) + g) * kRowBytes + 16 * j) = NORM ? f32x4{a.x * m[0], a.y * m[1], a.z * m[2], a.w * m[3]} : f32x4{a.x, a.y, a.z, a.w};
+            }
+            __builtin_amdgcn_wave_barrier();
+            f32x4 v[kSteps][2];
+#pragma unroll
+            for (int i = 0; i < kSteps; ++i)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) v[i][h] = *reinterpret_cast<const f32x4*>(rows_lds + j * kRowBytes + 128 * i + 32 * g + 16 * h);
+            __builtin_amdgcn_wave_barrier();
+            float mx = 0.0f;
+#pragma unroll
+            for (int i = 0; i < kSteps; ++i)
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+#pragma unroll
+                    for (int e = 0; e < 4; e += 2) mx = fmaxf(fmaxf(mx, fabsf(v[i][h][e])), fabsf(v[i][h][e + 1]));
+            mx = m40_max_xor32(m40_max_xor16(mx));      // over the row's block
+            float scale = 1.0f, inv_scale = 1.0f;
+            if (mx > 0.0f && mx < INFINITY) {
+                int ex;
+                (void)frexpf(mx, &ex);            // mx = f * 2^ex, f in [0.5, 1)
+                ex -= 11;                         // scaled maximum in [2^10, 2^11)
+                ex = ex < -100 ? -100 : (ex > 100 ? 100 : ex);
+                scale = ldexpf(1.0f, ex);
+                inv_scale = ldexpf(1.0f, -ex);
+            }
+            if (g == 0) scale_s[wave][16 * rt + j] = scale;
+#pragma unroll
+            for (int i = 0; i < kSteps; ++i) {
+                // hi = f16(v / scale), lo = f16(v / scale - hi): an instruction each (a multiply-add of mixed widths, rounded to f16)
+                f16x2 h2[4], l2[4];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const float y = v[i][e >> 2][e & 3];
+                    h2[e >> 1][e & 1] = static_cast<_Float16>(fmaf(y, inv_scale, -0.0f));
+                    l2[e >> 1][e & 1] = static_cast<_Float16>(fmaf(y, inv_scale, -static_cast<float>(h2[e >> 1][e & 1])));
+                }
+                hi[rt][i] = make_uint4(__builtin_bit_cast(uint32_t, h2[0]), __builtin_bit_cast(uint32_t, h2[1]), __builtin_bit_cast(uint32_t, h2[2]), __builtin_bit_cast(uint32_t, h2[3]));
+                lo[rt][i] = make_uint4(__builtin_bit_cast(uint32_t, l2[0]), __builtin_bit_cast(uint32_t, l2[1]), __builtin_bit_cast(uint32_t, l2[2]), __builtin_bit_cast(uint32_t, l2[3]));
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+    };
 
     m40_float4 total[T][RT];
 #pragma unroll
     for (int t = 0; t < T; ++t)
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) total[t][rt] = {0.f, 0.f, 0.f, 0.f};
-    auto multiply = [&](int c, int t) {
-        const uint4* planes = frag + (size_t)((c & 1) * RT * 2) * kPlane;
+    auto multiply = [&](const uint8_t* from, int t) {
         m40_float4 acc[RT];
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) acc[rt] = {0.f, 0.f, 0.f, 0.f};
         uint4 bw[kSteps];
 #pragma unroll
-        for (int i = 0; i < kSteps; ++i) bw[i] = *reinterpret_cast<const uint4*>(stage + j * kStageRow + 64 * i + 16 * g);
-        // Low parts first, while the sum is small: a chunk's sums then round on the high parts' scale twice, not four times (K 2048 with the norm,
-        // against 64 bits: 1.30e-7 -> 1.17e-7, and 1.12e-7 with the waves' sums added pair by pair instead of one after the other)
+        for (int i = 0; i < kSteps; ++i) bw[i] = *reinterpret_cast<const uint4*>(from + j * kStageRow + 64 * i + 16 * g);
+        // Low parts first, while the sum is small: a block's sums then round on the high parts' scale twice, not four times
 #pragma unroll
-        for (int part = 1; part >= 0; --part)
+        for (int i = 0; i < kSteps; ++i)
 #pragma unroll
-            for (int i = 0; i < kSteps; ++i) {
-                const int e = frag_slot((kSteps * wave + i) * 64 + lane);
+            for (int rt = 0; rt < RT; ++rt) acc[rt] = mfma16x16x32(lo[rt][i], bw[i], acc[rt]);
 #pragma unroll
-                for (int rt = 0; rt < RT; ++rt) acc[rt] = mfma16x16x32(planes[(2 * rt + part) * kPlane + e], bw[i], acc[rt]);
-            }
+        for (int i = 0; i < kSteps; ++i)
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) acc[rt] = mfma16x16x32(hi[rt][i], bw[i], acc[rt]);
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
-            const float4 s = *reinterpret_cast<const float4*>(&scale_s[c & 1][16 * rt + 4 * g]);
+            const float4 s = *reinterpret_cast<const float4*>(&scale_s[wave][16 * rt + 4 * g]);
             total[t][rt][0] = fmaf(s.x, acc[rt][0], total[t][rt][0]);
             total[t][rt][1] = fmaf(s.y, acc[rt][1], total[t][rt][1]);
             total[t][rt][2] = fmaf(s.z, acc[rt][2], total[t][rt][2]);
             total[t][rt][3] = fmaf(s.w, acc[rt][3], total[t][rt][3]);
         }
     };
-    for (int c0 = c_begin; c0 < c_end; c0 += kAhead) {
+    for (int kb = b_begin + wave; kb < b_end; kb += kWaves) {
+        convert();
+        load_rows(kb + kWaves);
 #pragma unroll
-        for (int a = 0; a < kAhead; ++a) {
-            const int c = c0 + a;
-            if (c >= c_end) break;
-            load_rows(c + 1 < c_end ? c + 1 : c);
-            const bool mine = c * kChunk + wave * kShare < p.K;       // the last chunk may end in its middle
+        for (int t = 0; t < T; ++t) {
+            uint8_t* to = stage + (t % kStages) * kStageBytes;
 #pragma unroll
-            for (int t = 0; t < T; ++t) {
-                uint4 (&set)[kLoads] = b[a * T + t];
-#pragma unroll
-                for (int li = 0; li < kLoads; ++li)      // built from the elements: a whole-struct copy would keep the array in scratch memory
-                    *reinterpret_cast<u32x4*>(stage + (li * kColsPerLoad + run_col) * kStageRow + 16 * run_lane) =
-                        u32x4{set[li].x, set[li].y, set[li].z, set[li].w};
-                __builtin_amdgcn_wave_barrier();
-                issue(set, c + kAhead, t);
-                if (mine) multiply(c, t);
-                __builtin_amdgcn_wave_barrier();
-            }
-            if (c + 1 < c_end) convert(c + 1);
-            __syncthreads();
+            for (int li = 0; li < kLoads; ++li)      // built from the elements: a whole-struct copy would keep the array in scratch memory
+                *reinterpret_cast<u32x4*>(to + (li * kColsPerLoad + run_col) * kStageRow + 16 * run_lane) = u32x4{b[t][li].x, b[t][li].y, b[t][li].z, b[t][li].w};
+            __builtin_amdgcn_wave_barrier();
+            issue(kb + kWaves, t);
+            multiply(to, t);
+            __builtin_amdgcn_wave_barrier();
         }
     }
+    __syncthreads();
 
     // ---- the waves' sums, and what follows the product
     if (NORM) {
-        sq = m40_sum16(sq);
-        if (kRowLanes == 32) sq = m40_add_xor16(sq);
-        if (l == 0) factor_s[row] = rsqrtf(sq / (float)p.K + p.eps);
+#pragma unroll
+        for (int u = 0; u < kRowLoads; ++u) {
+            const float sum = m40_sum16(sq[u]);
+            if (j == 0) square_s[wave][4 * u + g] = sum;
+        }
     }
-    float* red = reinterpret_cast<float*>(lds);          // [T][waves][RT * 4][64]: nobody reads the fragments any more
+    float* red = reinterpret_cast<float*>(lds);          // [T][waves][RT * 4][64]: nobody reads the staged weights any more
 #pragma unroll
     for (int t = 0; t < T; ++t)
 #pragma unroll
@@ -328,6 +313,19 @@ __global__ __launch_bounds__(kThreads, 1) void rows_wide_kernel(WideArgs p) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) red[((t * kWaves + wave) * RT * 4 + rt * 4 + r) * 64 + lane] = total[t][rt][r];
     __syncthreads();
+    if (NORM) {
+        if (tid < 16 * RT) {
+            float q[kWaves];
+#pragma unroll
+            for (int k = 0; k < kWaves; ++k) q[k] = square_s[k][tid];
+#pragma unroll
+            for (int n = kWaves / 2; n >= 1; n /= 2)
+#pragma unroll
+                for (int k = 0; k < n; ++k) q[k] += q[k + n];
+            factor_s[tid] = rsqrtf(q[0] / (float)p.K + p.eps);
+        }
+        __syncthreads();
+    }
     auto sum = [&](int t, int r, int col) {              // element (row r, column col) of tile t
         const float* at = red + ((size_t)t * kWaves * RT * 4 + (r >> 4) * 4 + (r & 3)) * 64 + 16 * ((r >> 2) & 3) + col;
         float s[kWaves];
@@ -345,6 +343,7 @@ __global__ __launch_bounds__(kThreads, 1) void rows_wide_kernel(WideArgs p) {
             float own = sum(0, e_row, e_j) * f + bias_own;
             const float other = sum(0, e_row, q_partner) * f + bias_other;
             if (q_which != 2) {
+                const float2 q_cs = m40_rope_cos_sin_freq(q_position, p.rope_table ? p.rope_table[q_off] : m40_rope_inv_freq(q_off, p.head_dim, p.rope_base), p.rope_scale);
                 float r0, r1;
                 m40_rope_apply(q_cs, q_second ? other : own, q_second ? own : other, &r0, &r1);
                 own = q_second ? r1 : r0;
@@ -395,7 +394,7 @@ __global__ __launch_bounds__(kThreads, 1) void rows_wide_kernel(WideArgs p) {
 
 template <int MODE, int RT, int T>
 int launch_t(hipStream_t stream, const WideArgs& a, int k_parts) {
-    constexpr int bytes = 2 * RT * 2 * kPlane * 16 + kWaves * kStageBytes;
+    constexpr int staged = kWaves * (wide_stages(T) * kStageBytes + 16 * kRowBytes), sums = T * kWaves * RT * 4 * 64 * 4, bytes = staged > sums ? staged : sums;
     static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(rows_wide_kernel<MODE, RT, T>),
                                                        hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
     if (attr != hipSuccess) return -7;
@@ -426,7 +425,7 @@ int launch_rt(M40llmCudaContext* ctx, hipStream_t stream, const WideArgs& a, int
 }
 template <int MODE>
 int launch(M40llmCudaContext* ctx, hipStream_t stream, WideArgs& a, int k_parts = 1) {
-    a.chunks = (a.K + kChunk - 1) / kChunk;
+    a.blocks = a.K / kShare;
     return a.rows <= 16 ? launch_rt<MODE, 1>(ctx, stream, a, k_parts) : launch_rt<MODE, 2>(ctx, stream, a, k_parts);
 }
 
@@ -496,7 +495,7 @@ int m40_rows_wide_residual(M40llmCudaContext* ctx, hipStream_t stream, const flo
     a.x = x; a.W0 = W; a.residual = residual; a.out = out; a.rows = rows; a.N = N; a.K = K; a.tiles = (N + 15) / 16;
     const size_t out_bytes = (size_t)rows * N * 4;
     if (!rows_untouched(a, out, N) || (residual != out && !m40_apart(residual, out_bytes, out, out_bytes))) return -6;
-    return launch<kResidual>(ctx, stream, a, onto_zero && residual != out && K >= 2 * kChunk && 2 * a.tiles <= ctx->num_cus ? 2 : 1);
+    return launch<kResidual>(ctx, stream, a, onto_zero && residual != out && K >= 1024 && 2 * a.tiles <= ctx->num_cus ? 2 : 1);
 }
 
 extern "C" {
