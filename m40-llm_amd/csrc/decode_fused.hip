@@ -143,20 +143,22 @@ struct QkvArgs {
 };
 
 // One wave per PAIRS consecutive rotation pairs (two output columns each).  Pair space: Q pairs, then K pairs, then
-// V pairs.
+// V pairs.  What the first requests need is passed on its own: such arguments lie in registers when a wave starts (a structure is read from memory first).
 template <int PAIRS>
-__global__ __launch_bounds__(kThreads) void norm_qkv_rope_append_kernel(QkvArgs p) {
+__global__ __launch_bounds__(kThreads) void norm_qkv_rope_append_kernel(const float* x, const void* norm_w, const uint16_t* wq, const uint32_t* position_dev,
+                                                                        uint32_t d_model, uint32_t q_heads, uint32_t kv_heads, uint32_t head_dim,
+                                                                        uint32_t rope_layout, uint32_t norm_dtype, QkvArgs p) {
     extern __shared__ float a_lds[];
     __shared__ float wave_sums[kWavesPerBlock];
-    const int K = (int)p.d_model;
+    const int K = (int)d_model;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     // x and the norm weights are requested before anything else is computed, then (below) the position and the pair's
     // rotation entry, then the GEMV weights; the norm prologue runs while the weights stream in
     StageRegs xr;
-    stage_load(p.x, p.norm_w, p.norm_dtype, K, 0, xr);
+    stage_load(x, norm_w, norm_dtype, K, 0, xr);
     __builtin_amdgcn_sched_barrier(0);
-    const uint32_t half = p.head_dim / 2u;
-    const uint32_t q_pairs = p.q_heads * half, kv_pairs = p.kv_heads * half;
+    const uint32_t half = head_dim / 2u;
+    const uint32_t q_pairs = q_heads * half, kv_pairs = kv_heads * half;
     const uint32_t pair0 = (blockIdx.x * kWavesPerBlock + wave) * PAIRS;
     bool live[PAIRS];
     int which[PAIRS];       // 0 Q, 1 K, 2 V
@@ -173,23 +175,23 @@ __global__ __launch_bounds__(kThreads) void norm_qkv_rope_append_kernel(QkvArgs 
         else { which[q] = 2; local[q] = pair - q_pairs - kv_pairs; }
         const uint32_t head = local[q] / half;
         off[q] = local[q] % half;
-        m40_rope_pair(head, off[q], p.head_dim, which[q] == 2 ? M40LLM_ROPE_LAYOUT_ADJACENT : p.rope_layout, &i0[q], &i1[q]);
-        const uint16_t* W = which[q] == 0 ? p.wq : (which[q] == 1 ? p.wk : p.wv);
+        m40_rope_pair(head, off[q], head_dim, which[q] == 2 ? M40LLM_ROPE_LAYOUT_ADJACENT : rope_layout, &i0[q], &i1[q]);
+        const uint16_t* W = which[q] == 0 ? wq : (which[q] == 1 ? p.wk : p.wv);
         bp[2 * q] = reinterpret_cast<const uint4*>(W + i0[q] * (size_t)K);
         bp[2 * q + 1] = reinterpret_cast<const uint4*>(W + i1[q] * (size_t)K);
     }
     // position and pair frequencies are requested with x, ahead of the weights.  Unconditionally: a load under a branch
     // costs a wait for everything in flight at the branch's join, which here held the weight requests back until x, the
     // norm weights and the position had arrived.  An absent input reads the first bytes of Wq and is ignored.
-    const uint32_t position_loaded = *(p.position_dev ? p.position_dev : reinterpret_cast<const uint32_t*>(p.wq));
+    const uint32_t position_loaded = *(position_dev ? position_dev : reinterpret_cast<const uint32_t*>(wq));
     float inv_freq[PAIRS];
     float4 kept[PAIRS];        // the pair's rotation as left by an earlier launch (the step's first layer)
 #pragma unroll
     for (int q = 0; q < PAIRS; ++q) {
-        inv_freq[q] = *(p.rope_table ? p.rope_table + off[q] : reinterpret_cast<const float*>(p.wq));
-        kept[q] = *(p.rope_cs ? p.rope_cs + off[q] : reinterpret_cast<const float4*>(p.wq));
+        inv_freq[q] = *(p.rope_table ? p.rope_table + off[q] : reinterpret_cast<const float*>(wq));
+        kept[q] = *(p.rope_cs ? p.rope_cs + off[q] : reinterpret_cast<const float4*>(wq));
     }
-    const uint32_t position = p.position_dev ? position_loaded : p.position;
+    const uint32_t position = position_dev ? position_loaded : p.position;
     __builtin_amdgcn_sched_barrier(0);
     GemvRegs<2 * PAIRS> regs;
     gemv_prefetch<2 * PAIRS>(bp, 0, K >> 3, lane, regs);
@@ -209,14 +211,14 @@ __global__ __launch_bounds__(kThreads) void norm_qkv_rope_append_kernel(QkvArgs 
             if (hit) {
                 cs[q] = make_float2(kept[q].y, kept[q].z);
             } else {
-                if (!p.rope_table) inv_freq[q] = m40_rope_inv_freq(off[q], p.head_dim, p.rope_base);      // replaces the ignored bytes
+                if (!p.rope_table) inv_freq[q] = m40_rope_inv_freq(off[q], head_dim, p.rope_base);      // replaces the ignored bytes
                 cs[q] = m40_rope_cos_sin_freq(position, inv_freq[q], p.rope_scale);
                 if (p.rope_cs && which[q] == 0 && local[q] < half && lane == 0)      // the waves of q head 0 keep it
                     p.rope_cs[off[q]] = make_float4(__uint_as_float(position), cs[q].x, cs[q].y, __uint_as_float(tag));
             }
         }
     }
-    stage_finish(xr, p.x, p.norm_w, p.norm_dtype, p.eps, K, a_lds, wave_sums);
+    stage_finish(xr, x, norm_w, norm_dtype, p.eps, K, a_lds, wave_sums);
     float d[2 * PAIRS];
     gemv_accumulate<2 * PAIRS>(bp, a_lds, 0, K >> 3, lane, regs, d);
     gemv_finish<2 * PAIRS, 1>(d, nullptr, wave, lane);
@@ -232,7 +234,7 @@ __global__ __launch_bounds__(kThreads) void norm_qkv_rope_append_kernel(QkvArgs 
             p.q_out[i0[q]] = y0;
             p.q_out[i1[q]] = y1;
         } else {
-            uint16_t* dst = (which[q] == 1 ? p.k_cache : p.v_cache) + (size_t)position * p.kv_heads * p.head_dim;
+            uint16_t* dst = (which[q] == 1 ? p.k_cache : p.v_cache) + (size_t)position * kv_heads * head_dim;
             dst[i0[q]] = m40_f2h(y0);
             dst[i1[q]] = m40_f2h(y1);
             if (which[q] == 1 && local[q] == 0) *p.seq_map_entry = position + 1u;
@@ -489,7 +491,8 @@ int m40llm_ext_fused_norm_qkv_rope_append_async(
     const uint32_t pairs = (q_heads + 2u * kv->num_heads) * (kv->head_dim / 2u);
     (void)hipGetLastError();
     // one pair per wave: two per wave measured 3 % slower on the whole token at 1280 pairs
-    norm_qkv_rope_append_kernel<1><<<(pairs + kWavesPerBlock - 1) / kWavesPerBlock, kThreads, (size_t)D * 4, ctx->decode_stream>>>(p);
+    norm_qkv_rope_append_kernel<1><<<(pairs + kWavesPerBlock - 1) / kWavesPerBlock, kThreads, (size_t)D * 4, ctx->decode_stream>>>(
+        p.x, p.norm_w, p.wq, p.position_dev, p.d_model, p.q_heads, p.kv_heads, p.head_dim, p.rope_layout, p.norm_dtype, p);
     return hipGetLastError() == hipSuccess ? 0 : -7;
 }
 

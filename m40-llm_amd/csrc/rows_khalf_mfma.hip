@@ -48,20 +48,13 @@ typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-struct KHalfArgs {
-    const float* A;            // [rows][K]
-    const uint16_t* W;         // [N][K] f16
-    const float* residual;     // [rows][N] or null
-    float* out;                // [rows][N], holds zeros when the launch starts
-    int rows, N, K;
-};
-
 // value of the partner lane (lane ^ 8) within a row of 16 lanes
 __device__ __forceinline__ uint32_t from_partner8(uint32_t v) {
     return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x128 /* row_ror:8 */, 0xf, 0xf, false);
 }
 
-__global__ __launch_bounds__(kThreads, 1) void rows_khalf_kernel(KHalfArgs p) {
+// A [rows][K], W [N][K] f16, residual [rows][N] or null, out [rows][N] that holds zeros when the launch starts
+__global__ __launch_bounds__(kThreads, 1) void rows_khalf_kernel(const float* A, const uint16_t* W, const float* residual, float* out, int rows, int N, int K) {
     extern __shared__ __attribute__((aligned(16))) uint8_t khalf_lds[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -74,12 +67,12 @@ __global__ __launch_bounds__(kThreads, 1) void rows_khalf_kernel(KHalfArgs p) {
     // residual value, requested ahead of everything else: one unconditional load from a clamped address -- at the end it
     // would be a round trip to memory with the whole workgroup waiting.
     const int e_row = (tid >> 4) & 7, e_j = tid & 15;
-    const size_t e_off = (size_t)(e_row < p.rows ? e_row : 0) * p.N + (n0 + e_j < p.N ? n0 + e_j : p.N - 1);
-    const float e_res = *(p.residual ? p.residual + e_off : p.A);
+    const size_t e_off = (size_t)(e_row < rows ? e_row : 0) * N + (n0 + e_j < N ? n0 + e_j : N - 1);
+    const float e_res = *(residual ? residual + e_off : A);
     __builtin_amdgcn_sched_barrier(0);
 
     // this wave's k-steps [ws0, ws1)
-    const int KS = p.K >> 5;
+    const int KS = K >> 5;
     const int hs0 = (int)((long long)KS * half / 2), hs1 = (int)((long long)KS * (half + 1) / 2);
     const int ws0 = hs0 + (int)((long long)(hs1 - hs0) * wave / kWaves);
     const int ws1 = hs0 + (int)((long long)(hs1 - hs0) * (wave + 1) / kWaves);
@@ -87,8 +80,8 @@ __global__ __launch_bounds__(kThreads, 1) void rows_khalf_kernel(KHalfArgs p) {
 
     // activations: lane (kg = g, r16 = j) -> row j & 7, elements 8 kg + 4 (j >> 3) .. + 3 of a k-step
     const int row = j & 7, part = j >> 3;
-    const bool row_live = row < p.rows;
-    const uint32_t a_voff = (uint32_t)(((size_t)(row_live ? row : 0) * p.K + 8 * g + 4 * part) * 4);   // bytes from a k-step's start in row 0
+    const bool row_live = row < rows;
+    const uint32_t a_voff = (uint32_t)(((size_t)(row_live ? row : 0) * K + 8 * g + 4 * part) * 4);   // bytes from a k-step's start in row 0
     // weights: instruction li of a batch covers kColsPerLoad columns, lane -> (column, 16-byte piece of its run)
     const int w_col = lane / kRunLanes, w_piece = lane % kRunLanes;
     const int w_step = w_piece >> 2;                                  // k-step of the piece inside its batch
@@ -100,18 +93,18 @@ __global__ __launch_bounds__(kThreads, 1) void rows_khalf_kernel(KHalfArgs p) {
 #pragma unroll
         for (int i = 0; i < kBatchSteps; ++i) {
             const int s = s0 + i < ws1 ? s0 + i : ws1 - 1;
-            a[i] = *reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(p.A + (size_t)s * 32) + a_voff);
+            a[i] = *reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(A + (size_t)s * 32) + a_voff);
         }
         __builtin_amdgcn_sched_barrier(0);
     };
     auto issue_w = [&](uint4 (&w)[kWLoads], int s0) {
         const int live = ws1 - s0;
         const int st = w_step < live ? w_step : (live > 0 ? live - 1 : 0);
-        const uint32_t voff = (uint32_t)(((size_t)w_col * p.K + 32 * st + 8 * (lane & 3)) * 2);
+        const uint32_t voff = (uint32_t)(((size_t)w_col * K + 32 * st + 8 * (lane & 3)) * 2);
         const int sb = s0 < ws1 ? s0 : ws1 - 1;
 #pragma unroll
         for (int li = 0; li < kWLoads; ++li) {
-            w[li] = *reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(p.W + (size_t)(n0 + kColsPerLoad * li) * p.K + (size_t)sb * 32) + voff);
+            w[li] = *reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(W + (size_t)(n0 + kColsPerLoad * li) * K + (size_t)sb * 32) + voff);
         }
         __builtin_amdgcn_sched_barrier(0);
     };
@@ -202,9 +195,9 @@ __global__ __launch_bounds__(kThreads, 1) void rows_khalf_kernel(KHalfArgs p) {
 #pragma unroll
         for (int w = 1; w < kWaves; ++w) v += red[(w * 4 + e_r) * 64 + e_lane];
         const int col = n0 + e_j;
-        if (e_row < p.rows && col < p.N) {
-            if (half == 0 && p.residual) v = e_res + v;
-            atomicAdd(p.out + (size_t)e_row * p.N + col, v);
+        if (e_row < rows && col < N) {
+            if (half == 0 && residual) v = e_res + v;
+            atomicAdd(out + (size_t)e_row * N + col, v);
         }
     }
 }
@@ -229,8 +222,7 @@ int m40_rows_khalf_residual(M40llmCudaContext* ctx, hipStream_t stream, const fl
     static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(rows_khalf_kernel),
                                                        hipFuncAttributeMaxDynamicSharedMemorySize, kDynamicLds);
     if (attr != hipSuccess) return -7;
-    KHalfArgs p{a, W, residual, out_zeroed, rows, N, K};
-    rows_khalf_kernel<<<2 * ((N + 15) / 16), kThreads, kDynamicLds, stream>>>(p);
+    rows_khalf_kernel<<<2 * ((N + 15) / 16), kThreads, kDynamicLds, stream>>>(a, W, residual, out_zeroed, rows, N, K);
     return hipGetLastError() == hipSuccess ? 0 : -7;
 }
 

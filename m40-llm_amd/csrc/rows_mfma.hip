@@ -108,9 +108,11 @@ __device__ __forceinline__ int qkv_col(const RowsMfmaArgs& p, const QkvTile& t, 
     return t.split ? t.head * hd + (i & 8 ? hd / 2 : 0) + 8 * t.tt + (i & 7) : t.head * hd + 16 * t.tt + i;
 }
 
-// MODE 0: out = x W^T; 1: SwiGLU of gate and up; 2: Q/K/V with bias, RoPE and cache append
+// MODE 0: out = x W^T; 1: SwiGLU of gate and up; 2: Q/K/V with bias, RoPE and cache append.  What the first requests need is passed on its own, in registers
+// when a wave starts; the structure is read from memory meanwhile.
 template <int MODE, int WAVES>
-__global__ __launch_bounds__(64 * WAVES, 1) void rows_mfma_kernel(RowsMfmaArgs p) {
+__global__ __launch_bounds__(64 * WAVES, 1) void rows_mfma_kernel(const float* x, const void* norm_w, const uint16_t* W0, const uint16_t* W1, int rows, uint32_t norm_dtype,
+                                                                  int units, int N, RowsMfmaArgs p) {
     using S = Shape<WAVES>;
     constexpr int kWaves = WAVES, kSteps = S::kSteps, kLoads = S::kLoads, kStageRow = S::kStageRow,
                   kStageBytes = S::kStageBytes, kRunLanes = S::kRunLanes, kColsPerLoad = S::kColsPerLoad,
@@ -128,8 +130,8 @@ __global__ __launch_bounds__(64 * WAVES, 1) void rows_mfma_kernel(RowsMfmaArgs p
     // The activation rows and the norm weights are requested before anything else is computed: they head the longest
     // dependent chain of the kernel (rows -> scale -> fragments -> first matrix instruction).
     const int row = tid / kRowThreads, l = tid % kRowThreads;
-    const bool live = row < p.rows;
-    const float* xr = p.x + (size_t)(live ? row : 0) * kK;
+    const bool live = row < rows;
+    const float* xr = x + (size_t)(live ? row : 0) * kK;
     float v[kChunks][8];
     float sq = 0.0f;            // sum of squares of the raw row (RMSNorm only)
 #pragma unroll
@@ -142,13 +144,13 @@ __global__ __launch_bounds__(64 * WAVES, 1) void rows_mfma_kernel(RowsMfmaArgs p
     // Everything the prologue needs goes out first, the weight tiles behind it: loads return in issue order, so the
     // rows and the norm weights (cache hits or a short fetch) are not kept waiting behind 64 KB of weights per
     // workgroup, and both tiles are on their way while the rows are converted.
-    const bool norm16 = p.norm_w && p.norm_dtype == 0u;
+    const bool norm16 = norm_w && norm_dtype == 0u;
     uint4 wraw[2 * kChunks];
     {
         // one unconditional batch of loads whatever the weights are (a branch around loads costs a full wait at
         // its join): f32 weights are 32 bytes per chunk; f16 weights 16 bytes, requested twice; without a norm the
         // row itself is read again and ignored
-        const uint4* wp = p.norm_w ? static_cast<const uint4*>(p.norm_w) : reinterpret_cast<const uint4*>(xr);
+        const uint4* wp = norm_w ? static_cast<const uint4*>(norm_w) : reinterpret_cast<const uint4*>(xr);
         const int mul = norm16 ? 1 : 2, second = norm16 ? 0 : 1;
 #pragma unroll
         for (int c = 0; c < kChunks; ++c) {
@@ -159,8 +161,8 @@ __global__ __launch_bounds__(64 * WAVES, 1) void rows_mfma_kernel(RowsMfmaArgs p
     __builtin_amdgcn_sched_barrier(0);
     // consecutive, nearly equal runs of tiles (a finer split of the last tile was measured and gains nothing: the
     // launch is bound by the memory system, and the workgroups still running share what the finished ones leave)
-    const int u_begin = (int)((uint32_t)blockIdx.x * (uint32_t)p.units / gridDim.x);          // units < 2^20, workgroups <= 2^10
-    const int n_units = (int)(((uint32_t)blockIdx.x + 1u) * (uint32_t)p.units / gridDim.x) - u_begin;
+    const int u_begin = (int)((uint32_t)blockIdx.x * (uint32_t)units / gridDim.x);          // units < 2^20, workgroups <= 2^10
+    const int n_units = (int)(((uint32_t)blockIdx.x + 1u) * (uint32_t)units / gridDim.x) - u_begin;
 
     // Weight loads are whole runs: an instruction of a wave reads the wave's share of K of one column (four waves) or
     // two columns (eight) of the tile, 16 bytes per lane.  (Reading the MFMA operand layout straight from memory -- 16 columns x 64 bytes per
@@ -180,18 +182,18 @@ __global__ __launch_bounds__(64 * WAVES, 1) void rows_mfma_kernel(RowsMfmaArgs p
             if (li < l_begin || li >= l_end) continue;
             const int i = li * kColsPerLoad + run_col;      // column of the tile (i & 8 is the same for the whole instruction)
             int col;
-            const uint16_t* W = p.W0;
+            const uint16_t* W = W0;
             if (SWIGLU) {
                 col = 8 * unit + (i & 7);
-                if (li * kColsPerLoad & 8) W = p.W1;
-                col = col < p.N ? col : p.N - 1;
+                if (li * kColsPerLoad & 8) W = W1;
+                col = col < N ? col : N - 1;
             } else if (QKV) {
                 const QkvTile t = qkv_tile(p, unit);
                 col = qkv_col(p, t, i);
-                W = t.which == 0 ? p.W0 : (t.which == 1 ? p.W1 : p.W2);
+                W = t.which == 0 ? W0 : (t.which == 1 ? W1 : p.W2);
             } else {
                 col = 16 * unit + i;
-                col = col < p.N ? col : p.N - 1;
+                col = col < N ? col : N - 1;
             }
             b[li] = *reinterpret_cast<const uint4*>(W + (size_t)col * kK + wave * (kK / kWaves) + lane_off);
         }
@@ -200,7 +202,7 @@ __global__ __launch_bounds__(64 * WAVES, 1) void rows_mfma_kernel(RowsMfmaArgs p
     __builtin_amdgcn_sched_barrier(0);
     // the tile element this thread writes (see `finish`)
     constexpr int kTileCols = SWIGLU ? 8 : 16;      // output columns of a tile
-    const int n_out = kTileCols * p.rows;
+    const int n_out = kTileCols * rows;
     const int e_out = tid % n_out, e_row = e_out / kTileCols, e_j = e_out % kTileCols;
     const int e_lane = 16 * (e_row >> 2) + e_j, e_r = e_row & 3;
 
@@ -247,7 +249,7 @@ __global__ __launch_bounds__(64 * WAVES, 1) void rows_mfma_kernel(RowsMfmaArgs p
                 for (int e = 0; e < 8; ++e) { sq0 = fmaf(v[c][e], v[c][e], sq0); v[c][e] *= w[e]; }
             }
             sq = sq0;
-        } else if (p.norm_w) {
+        } else if (norm_w) {
             float sq0 = 0.0f;
 #pragma unroll
             for (int c = 0; c < kChunks; ++c) {
@@ -298,7 +300,7 @@ __global__ __launch_bounds__(64 * WAVES, 1) void rows_mfma_kernel(RowsMfmaArgs p
             a_frag[frag_slot(entry)] = make_uint4(hi[0], hi[1], hi[2], hi[3]);          // rows 0..7: hi parts
             a_frag[frag_slot(entry + 8)] = make_uint4(lo[0], lo[1], lo[2], lo[3]);      // rows 8..15: lo parts
         }
-        if (l == 0) row_scale_s[row] = scale * (p.norm_w ? rsqrtf(sq / (float)kK + p.eps) : 1.0f);
+        if (l == 0) row_scale_s[row] = scale * (norm_w ? rsqrtf(sq / (float)kK + p.eps) : 1.0f);
     }
     if (QKV && first_ops.which != 2) first_cs = m40_rope_cos_sin_freq(first_ops.position, first_ops.inv_freq, p.rope_scale);
     __syncthreads();
@@ -360,13 +362,13 @@ __global__ __launch_bounds__(64 * WAVES, 1) void rows_mfma_kernel(RowsMfmaArgs p
             return;
         }
         int col = kTileCols * unit + e_j;
-        col = col < p.N ? col : p.N - 1;          // a column past the end was computed from the last column's weights
+        col = col < N ? col : N - 1;          // a column past the end was computed from the last column's weights
         float v = tile_sum(parity, e_lane) * s;
         if (SWIGLU) {
             const float up = tile_sum(parity, e_lane + 8) * s;
             v = v / (1.0f + expf(-v)) * up;
         }
-        p.out[(size_t)e_row * p.N + col] = v;
+        p.out[(size_t)e_row * N + col] = v;
     };
     // One tile from register set b; PREFETCH: tile local + 1 exists and is requested into the same set.
     auto tile = [&](uint4 (&b)[kLoads], auto prefetch_c, int local, int parity) {
@@ -401,7 +403,7 @@ int launch_w(M40llmCudaContext* ctx, hipStream_t stream, const RowsMfmaArgs& a) 
     if (attr != hipSuccess) return -7;
     int grid = ctx->num_cus;           // one workgroup per CU: most of its LDS
     if (grid > a.units) grid = a.units;
-    rows_mfma_kernel<MODE, WAVES><<<grid, S::kThreads, S::kDynamicLds, stream>>>(a);
+    rows_mfma_kernel<MODE, WAVES><<<grid, S::kThreads, S::kDynamicLds, stream>>>(a.x, a.norm_w, a.W0, a.W1, a.rows, a.norm_dtype, a.units, a.N, a);
     return hipGetLastError() == hipSuccess ? 0 : -7;
 }
 template <int MODE>
