@@ -250,6 +250,12 @@ __device__ __forceinline__ uint4 m40_load_stream(const uint4* p) {
     return make_uint4(v.x, v.y, v.z, v.w);
 }
 
+// Workgroup b of a launch over rows: workgroups are dealt to the eight dies in turn, and the rows of a 16-row tile go to one die so
+// that its L2 puts their pieces of the tile's lines together.
+__device__ __forceinline__ uint32_t m40_tile_row(uint32_t b, uint32_t rows) {
+    return (b | 127u) < rows ? (b & ~127u) + (b & 7u) * 16u + ((b & 127u) >> 3) : b;
+}
+
 // 8 halves packed in a uint4 -> 8 floats
 __device__ __forceinline__ void m40_unpack8(const uint4& w, float (&f)[8]) {
     const uint32_t u[4] = {w.x, w.y, w.z, w.w};

@@ -14,6 +14,7 @@
 // share A (Q/K/V, gate/up) can be served by one packing pass and one launch.
 #include "common.hpp"
 
+#include <numeric>
 #include <type_traits>
 #include <utility>
 
@@ -99,6 +100,12 @@ __device__ __forceinline__ float4 sum_planes(const float4* planes, int k_splits,
     return residual ? make_float4(r.x + a.x, r.y + a.y, r.z + a.z, r.w + a.w) : a;
 }
 
+// The planes lie in tiles of 16 rows x 32 k, a kilobyte each, all k of sixteen rows one after the other: what an instruction of the tiled kernel
+// loads is contiguous.  A row's stores are half lines, which the L2 of the die that has the tile's sixteen rows puts together (4096 rows of 5632: 32.0
+// us as whole rows, 35.1 this way, 39.2 with the rows dealt to the dies in turn).  16-byte chunk of a row's first k, and how far on its chunk c is:
+__device__ __forceinline__ size_t plane_chunk(int row, int K) { return (size_t)(row >> 4) * (K / kBK) * 64 + (row & 15) * 4; }
+__device__ __forceinline__ size_t plane_step(int c) { return (size_t)(c >> 2) * 64 + (c & 3); }
+
 // ROW_THREADS = 64: a wave per row, four rows per workgroup, no barrier (K <= 4096 keeps the row in registers);
 // 256: a workgroup per row (always for the RMSNorm source, whose sum of squares is formed with the thread layout and
 // order of rms_norm_kernel so that the fused form gives the bits of the two-launch form).
@@ -111,7 +118,10 @@ __global__ __launch_bounds__(256) void pack_hilo_planes_kernel(PackSource src_ar
     __shared__ float wave_max[4];
     __shared__ float wave_sums[4];
     constexpr int kRowsPerGroup = 256 / ROW_THREADS;
-    const int row = (int)blockIdx.x * kRowsPerGroup + (int)threadIdx.x / ROW_THREADS, tid = (int)threadIdx.x % ROW_THREADS;
+    // the rows of a tile on one die (m40_tile_row; a workgroup of four rows: four workgroups a tile)
+    const uint32_t b = blockIdx.x, groups = gridDim.x;
+    const uint32_t group = ROW_THREADS == 256 ? m40_tile_row(b, groups) : ((b | 31u) < groups ? (b & ~31u) + (b & 7u) * 4u + ((b & 31u) >> 3) : b);
+    const int row = (int)group * kRowsPerGroup + (int)threadIdx.x / ROW_THREADS, tid = (int)threadIdx.x % ROW_THREADS;
     if (ROW_THREADS == 64 && row >= M) return;          // whole waves: no barrier in this form
     const float4* src = reinterpret_cast<const float4*>(src_args.a + (size_t)row * K);
     const float4* src2 = KIND == kPackSwiglu ? reinterpret_cast<const float4*>(src_args.a2 + (size_t)row * K) : nullptr;
@@ -204,8 +214,8 @@ __global__ __launch_bounds__(256) void pack_hilo_planes_kernel(PackSource src_ar
         inv_scale = ldexpf(1.0f, -ex);
     }
     if (tid == 0) row_scale[row] = scale;
-    half8* hp = reinterpret_cast<half8*>(hi + (size_t)row * K);
-    half8* lp = reinterpret_cast<half8*>(lo + (size_t)row * K);
+    half8* hp = reinterpret_cast<half8*>(hi) + plane_chunk(row, K);
+    half8* lp = reinterpret_cast<half8*>(lo) + plane_chunk(row, K);
     if (in_regs) {
 #pragma unroll
         for (int i = 0; i < kPackChunks; ++i) {
@@ -213,8 +223,8 @@ __global__ __launch_bounds__(256) void pack_hilo_planes_kernel(PackSource src_ar
             if (c < chunks) {
                 half8 h, l;
                 pack_split8(x0[i], x1[i], inv_scale, h, l);
-                hp[c] = h;
-                lp[c] = l;
+                hp[plane_step(c)] = h;
+                lp[plane_step(c)] = l;
             }
         }
     } else {
@@ -223,8 +233,8 @@ __global__ __launch_bounds__(256) void pack_hilo_planes_kernel(PackSource src_ar
             load_chunk(c, a, b);
             half8 h, l;
             pack_split8(a, b, inv_scale, h, l);
-            hp[c] = h;
-            lp[c] = l;
+            hp[plane_step(c)] = h;
+            lp[plane_step(c)] = l;
         }
     }
 }
@@ -243,9 +253,13 @@ __global__ __launch_bounds__(256) void pack_hilo_planes_kernel(PackSource src_ar
 //    before one), kBufs buffers deep -- a lane fetches the 16-byte chunk that belongs at its place in the swizzled
 //    row layout, so a wave's instruction fills one contiguous kilobyte; the workgroup waits only for the step after
 //    next (vmcnt) ahead of the barrier that publishes it;
+//  * an instruction loads whole lines: of A a kilobyte of the packed planes, of B eight columns of 128 bytes, two steps at a time (kBBufs
+//    buffers of those, asked for in every second step).  With 16 rows of 64 bytes an instruction, half lines of both, the launches below took, on
+//    one card, 378 us (N 11264), 175 (K 5632) and 112 (N 2560); with both as they are 351, 162 and 105 (whole lines of A alone: 1 to 2 % more than
+//    that);
 //  * in the 128 x 256 tile the wave tile is 64 x 128: per matrix instruction two thirds of the fragment bytes of a 64 x 64 tile (the
 //    activation rows, read twice -- high and low part -- are the short side).
-// M 4096, N 2048, K 2048: 79 (128 x 128, through registers) -> 63 us; N 11264: 479 -> 338 us; K 5632: 232 -> 155 us.  Under this load the part lowers
+// M 4096, N 2048, K 2048: 79 (128 x 128, through registers) -> 63 us; N 11264: 479 -> 338 us; K 5632: 232 -> 155 us (before the whole lines).  Under this load the part lowers
 // its clock (1.4-1.9 GHz measured inside the kernel, against 2.0-2.2 GHz in short or memory-bound launches), and a form
 // with fewer issue cycles (32 x 32 x 16 instructions: 1370 instead of 1500 cycles per step) ran at a lower clock
 // still and took the same time: what is left is energy per product, of which the exact hi + lo split is half.
@@ -275,54 +289,63 @@ __device__ __forceinline__ TileWalk tile_walk(const TiledMats& mats, int tiles_m
 // s_waitcnt for vector-memory operations only: at most n of them may still be outstanding
 __device__ __forceinline__ constexpr int vmcnt_only(int n) { return 0x0f70 | (n & 15) | ((n >> 4) << 14); }
 
+// stages of a part of K
+template <int KS>
+__host__ __device__ constexpr int split_stages(int stages, int k_splits) {
+    const int per = (stages + k_splits - 1) / k_splits;
+    return KS == 1 && k_splits > 1 ? (per + 1) & ~1 : per;
+}
+
 template <int... I, class F>
 __device__ __forceinline__ void tiled_unrolled(std::integer_sequence<int, I...>, F&& f) { (f(std::integral_constant<int, I>{}), ...); }
 
 // KS: k steps of 32 a stage (what is loaded together, between two barriers); kBufs: LDS buffers of a stage each (one
 // workgroup is resident per CU).  Two steps a stage read whole 128-byte lines of a column: with weights that no cache holds 64 x 64 tiles of N 2048,
 // K 2048 take 15.5 us that way and 21.3 us in stages of one step, 64 x 128 tiles 21.0 and 24.6 us (60 rows).
-template <int MT, int NT, int KS, int kBufs>
+template <int MT, int NT, int KS, int kBufs, int kBBufs>
 __global__ __launch_bounds__(kThreads, 1) void gemm_tiled_kernel(const _Float16* __restrict__ A_hi, const _Float16* __restrict__ A_lo,
                                                                       const float* __restrict__ row_scale, TiledMats mats, int M, int K,
                                                                       int k_splits, int band) {
     typedef __attribute__((address_space(3))) void* lds_dst_t;
     typedef const __attribute__((address_space(1))) void* global_src_t;
     constexpr int BM = 32 * MT, BN = 32 * NT;
-    constexpr int kRow = 64 * KS, kLoadRows = kThreads / (4 * KS);           // bytes of a row in a stage; rows the workgroup loads at a time
-    constexpr int kPlane = BM * kRow, kBuf = 2 * kPlane + BN * kRow;         // bytes of a stage: A high, A low, B
-    constexpr int AL = BM / kLoadRows, BL = BN / kLoadRows, kLoads = 2 * AL + BL;      // 16-byte loads per thread: rows lrow + kLoadRows i
+    constexpr int kRow = 64 * KS, kLoadRows = kThreads / (4 * KS);           // bytes of a row of A in a stage; rows the workgroup loads at a time
+    constexpr int kRowB = 128, kLoadRowsB = kThreads / 8;                    // of B, always two steps
+    constexpr int kPlane = BM * kRow, kBuf = 2 * kPlane, kBufB = BN * kRowB, kB0 = kBufs * kBuf;      // bytes: a plane of a stage, both, B of two steps; where B starts
+    constexpr int AL = BM / kLoadRows, BL = BN / kLoadRowsB;                 // 16-byte loads per thread: rows lrow + kLoadRows i
     extern __shared__ __align__(16) uint8_t tile_lds[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     TileWalk at = tile_walk(mats, (M + BM - 1) / BM, k_splits, band, BM, BN);
     at.m0 = __builtin_amdgcn_readfirstlane(at.m0); at.n0 = __builtin_amdgcn_readfirstlane(at.n0);      // the same in every lane: divisions leave them in vector registers
     at.mat = __builtin_amdgcn_readfirstlane(at.mat); at.split = __builtin_amdgcn_readfirstlane(at.split);
     const int N = mats.N[at.mat], m0 = at.m0, n0 = at.n0;
-    // in a pair a wave's rows of a load are one matrix's: 16 rows of 64 bytes or 8 of 128, four times as far on with the next load
-    const uint16_t* __restrict__ B = mats.B[mats.pair ? (wave >> (KS - 1)) & 1 : at.mat];
+    // in a pair a wave's eight rows of a load are one matrix's
+    const uint16_t* __restrict__ B = mats.B[mats.pair ? (wave >> 1) & 1 : at.mat];
     // loader: thread -> row lrow (+ kLoadRows i) of a plane and a 16-byte place in that row's bytes, which holds the row's chunk of that number
     // xor-ed with bits of the row: the fragment reads of rows that share banks fall into different ones
     auto swizzle = [](int row) { return KS == 1 ? (row >> 2) & 3 : row & 7; };
-    const int lrow = tid / (4 * KS), gchunk = tid % (4 * KS) ^ swizzle(lrow);
-    const int stages_all = K / (kBK * KS), per_split = __builtin_amdgcn_readfirstlane((stages_all + k_splits - 1) / k_splits), stage0 = at.split * per_split;
+    const int lrow = tid / (4 * KS), gchunk = tid % (4 * KS) ^ swizzle(lrow), lrow_b = tid / 8, gchunk_b = tid % 8 ^ (lrow_b & 7);
+    // (stages of one step: an even number of them to a part of K)
+    const int stages_all = K / (kBK * KS), per_split = __builtin_amdgcn_readfirstlane(split_stages<KS>(stages_all, k_splits)), stage0 = at.split * per_split;
     const int stages = stage0 + per_split <= stages_all ? per_split : stages_all - stage0;     // >= 1 by the host's choice of k_splits
     // a scalar address that walks K, and per lane a 32-bit offset from it that does not change
-    const uint8_t* hi_base = reinterpret_cast<const uint8_t*>(A_hi + (size_t)m0 * K + (size_t)stage0 * (kBK * KS));
-    const uint8_t* lo_base = reinterpret_cast<const uint8_t*>(A_lo + (size_t)m0 * K + (size_t)stage0 * (kBK * KS));
+    const uint8_t* hi_base = reinterpret_cast<const uint8_t*>(A_hi + (size_t)m0 * K) + (size_t)stage0 * (KS * 1024);
+    const uint8_t* lo_base = reinterpret_cast<const uint8_t*>(A_lo + (size_t)m0 * K) + (size_t)stage0 * (KS * 1024);
     const uint8_t* b_base = reinterpret_cast<const uint8_t*>(B + (size_t)(mats.pair ? n0 / 2 : n0) * K + (size_t)stage0 * (kBK * KS));
     uint32_t a_off[AL], b_off[BL];
 #pragma unroll
     for (int i = 0; i < AL; ++i) {
-        const int r = lrow + kLoadRows * i;
-        a_off[i] = (uint32_t)(m0 + r < M ? r : M - 1 - m0) * (uint32_t)K * 2u + gchunk * 16u;     // clamped: computed, never stored
+        const int r = m0 + lrow + kLoadRows * i < M ? lrow + kLoadRows * i : M - 1 - m0;      // clamped: computed, never stored
+        a_off[i] = (uint32_t)(r >> 4) * (uint32_t)K * 32u + (gchunk >> 2) * 1024u + (r & 15) * 64u + (gchunk & 3) * 16u;
     }
 #pragma unroll
     for (int i = 0; i < BL; ++i) {
-        const int c = lrow + kLoadRows * i, last = mats.pair ? N / 2 - 1 - n0 / 2 : N - 1 - n0, col = mats.pair ? c / 32 * 16 + c % 16 : c;
-        b_off[i] = (uint32_t)(col < last ? col : last) * (uint32_t)K * 2u + gchunk * 16u;
+        const int c = lrow_b + kLoadRowsB * i, last = mats.pair ? N / 2 - 1 - n0 / 2 : N - 1 - n0, col = mats.pair ? c / 32 * 16 + c % 16 : c;
+        b_off[i] = (uint32_t)(col < last ? col : last) * (uint32_t)K * 2u + gchunk_b * 16u;
     }
-    // one instruction of a wave fills a contiguous kilobyte of a plane, lane by lane
-    auto issue = [&](int buf, int stage) __attribute__((always_inline)) {
-        int k = (stage < stages ? stage : stages - 1) * kRow;          // past the end: the last stage again (no branch around loads)
+    // one instruction of a wave fills a contiguous kilobyte of a buffer, lane by lane; past the end: the last stage again (no branch around loads)
+    auto issue_a = [&](int buf, int stage) __attribute__((always_inline)) {
+        int k = (stage < stages ? stage : stages - 1) * (KS * 1024);
         asm("" : "+s"(k));                                                      // keeps it out of the lanes' addresses
         uint8_t* dst = tile_lds + buf * kBuf + wave * 1024;
 #pragma unroll
@@ -330,9 +353,20 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_tiled_kernel(const _Float16*
             __builtin_amdgcn_global_load_lds((global_src_t)(hi_base + k + a_off[i]), (lds_dst_t)(dst + i * 4096), 16, 0, 0);
             __builtin_amdgcn_global_load_lds((global_src_t)(lo_base + k + a_off[i]), (lds_dst_t)(dst + kPlane + i * 4096), 16, 0, 0);
         }
+    };
+    // B of the steps 2 pair and 2 pair + 1 (one stage where a stage is two steps); of an odd number of steps the last one is read twice
+    const int pairs = KS == 2 ? stages : (stages + 1) / 2;
+    const bool odd = KS == 1 && stages % 2 != 0;
+    const uint32_t second = gchunk_b >= 4 ? 64u : 0u;
+    auto issue_b = [&](int buf, int pair) __attribute__((always_inline)) {
+        const int p = pair < pairs ? pair : pairs - 1;
+        int k = p * kRowB;
+        asm("" : "+s"(k));
+        const uint32_t back = odd && p == pairs - 1 ? second : 0u;
+        uint8_t* dst = tile_lds + kB0 + buf * kBufB + wave * 1024;
 #pragma unroll
         for (int i = 0; i < BL; ++i)
-            __builtin_amdgcn_global_load_lds((global_src_t)(b_base + k + b_off[i]), (lds_dst_t)(dst + 2 * kPlane + i * 4096), 16, 0, 0);
+            __builtin_amdgcn_global_load_lds((global_src_t)(b_base + k + (KS == 1 ? b_off[i] - back : b_off[i])), (lds_dst_t)(dst + i * 4096), 16, 0, 0);
     };
     const int wm = wave >> 1, wn = wave & 1, frag_row = lane & 15;
     float scale[MT];                   // of the rows this lane will store, requested ahead of everything else
@@ -342,17 +376,17 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_tiled_kernel(const _Float16*
         scale[mt] = row_scale[row < M ? row : M - 1];
     }
     struct Frags { half8 hi[MT], lo[MT], b[NT]; } f[2];
-    auto read_frags = [&](Frags& f, int buf, auto sub_c) __attribute__((always_inline)) {
-        const uint8_t* base = tile_lds + buf * kBuf + frag_row * kRow + (((lane >> 4) + 4 * decltype(sub_c)::value) ^ swizzle(frag_row)) * 16;
-        const uint8_t* a = base + wm * MT * 16 * kRow;
-        const uint8_t* b = base + 2 * kPlane + wn * NT * 16 * kRow;
+    // fragments of a step: which buffers, and which of a buffer's steps
+    auto read_frags = [&](Frags& f, int buf, int sub, int buf_b, int sub_b) __attribute__((always_inline)) {
+        const uint8_t* a = tile_lds + buf * kBuf + (wm * MT * 16 + frag_row) * kRow + (((lane >> 4) + 4 * sub) ^ swizzle(frag_row)) * 16;
+        const uint8_t* b = tile_lds + kB0 + buf_b * kBufB + (wn * NT * 16 + frag_row) * kRowB + (((lane >> 4) + 4 * sub_b) ^ (frag_row & 7)) * 16;
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
             f.hi[mt] = *reinterpret_cast<const half8*>(a + mt * 16 * kRow);
             f.lo[mt] = *reinterpret_cast<const half8*>(a + kPlane + mt * 16 * kRow);
         }
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) f.b[nt] = *reinterpret_cast<const half8*>(b + nt * 16 * kRow);
+        for (int nt = 0; nt < NT; ++nt) f.b[nt] = *reinterpret_cast<const half8*>(b + nt * 16 * kRowB);
     };
     floatx4 acc[MT][NT];
 #pragma unroll
@@ -378,30 +412,53 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_tiled_kernel(const _Float16*
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_sched_barrier(0);
     };
-    constexpr int kInFlight = (kBufs - 3) * kLoads;
+    // What stage s asks for: A of stage s + kBufs - 1, then B: with two steps a stage that of the same stage, else in every second step the pair whose
+    // buffer the step before last was the last to read (fragments are in registers one barrier later).  `at`: how many loads may be outstanding at
+    // the end of stage s, behind which the fragments of stage s + 2 are read.
+    struct Flight {
+        static constexpr bool asks_b(int s) { return KS == 2 || s % 2 == 0; }
+        static constexpr int pair(int s) { return KS == 2 ? s + kBBufs - 1 : s / 2 - 1 + kBBufs; }
+        static constexpr int of(int s) { return 2 * AL + (asks_b(s) ? BL : 0); }
+        static constexpr int at(int s) {
+            int behind_a = asks_b(s + 3 - kBufs) ? BL : 0, behind_b = 0;
+            for (int t = s + 4 - kBufs; t <= s; ++t) behind_a += of(t);
+            for (int t = KS == 2 ? s + 4 - kBBufs : s / 2 * 2 + 5 - 2 * kBBufs; t <= s; ++t) behind_b += of(t);
+            return behind_a < behind_b ? behind_a : behind_b;
+        }
+    };
+    constexpr int kEven = 64;           // of the stages before the first, counted from here
+    static_assert(kBBufs >= 3 && kBufs >= 4 && (KS == 1 || kBufs == kBBufs));
 #pragma unroll
-    for (int i = 0; i < kBufs - 1; ++i) issue(i, i);
-    wait_and_meet(std::integral_constant<int, kInFlight>());               // stages 0 and 1 have landed
-    read_frags(f[0], 0, std::integral_constant<int, 0>());
-    // Step u of a stage: the next step's fragments are read (the next stage's first ones behind its last step: buffer s + 1 is complete and
+    for (int t = kEven - 2 * kBBufs - kBufs; t < kEven; ++t) {
+        if (t + kBufs - 1 >= kEven) issue_a(t + kBufs - 1 - kEven, t + kBufs - 1 - kEven);
+        const int pair = KS == 2 ? t - kEven + kBBufs - 1 : t / 2 - kEven / 2 - 1 + kBBufs;
+        if (Flight::asks_b(t) && pair >= 0) issue_b(pair, pair);
+    }
+    wait_and_meet(std::integral_constant<int, Flight::at(kEven - 1)>());               // stages 0 and 1 have landed
+    read_frags(f[0], 0, 0, 0, 0);
+    // Step u of a stage: the next step's fragments are read (the next stage's first ones behind its last step: its buffers are complete and
     // visible), then its products.  Stage s refills the buffer of stage s - 1 -- whose fragments every wave had in registers before
     // the last barrier -- with stage s + kBufs - 1, and ends with stage s + 2 landed.  ph: the stage's number in a period, after which buffers
     // and fragment sets are back in their order: written out so that their addresses are constants and sums stay in their registers (a loop of
     // two stages moved 200 accumulation registers a turn: 169 against 161 us at M 4096, N 2048, K 5632).
-    constexpr int kPeriod = KS == 2 || kBufs % 2 == 0 ? kBufs : 2 * kBufs;
+    constexpr int kPeriod = KS == 2 ? kBufs : std::lcm(kBufs, 2 * kBBufs);
     auto sub_step = [&](auto ph_c, auto sub_c, int s) __attribute__((always_inline)) {
-        constexpr int ph = decltype(ph_c)::value, sub = decltype(sub_c)::value, buf = ph % kBufs, set = (ph * KS + sub) & 1;
-        read_frags(f[set ^ 1], sub + 1 < KS ? buf : (buf + 1) % kBufs, std::integral_constant<int, (sub + 1) % KS>());
-        if constexpr (sub == 0) issue((buf + kBufs - 1) % kBufs, s + kBufs - 1);
+        constexpr int ph = decltype(ph_c)::value, sub = decltype(sub_c)::value, set = (ph * KS + sub) & 1;
+        constexpr int next = ph + (KS == 1 || sub == 1);          // the next step's stage
+        if constexpr (KS == 2) read_frags(f[set ^ 1], next % kBufs, sub ^ 1, next % kBBufs, sub ^ 1);
+        else read_frags(f[set ^ 1], next % kBufs, 0, next / 2 % kBBufs, next % 2);
+        constexpr bool loads_b = sub == 0 && Flight::asks_b(ph);
+        if constexpr (sub == 0) issue_a((ph + kBufs - 1) % kBufs, s + kBufs - 1);
+        if constexpr (loads_b) issue_b(Flight::pair(ph) % kBBufs, Flight::pair(s));
         compute(f[set]);
-        constexpr int kReads = 2 * MT + NT, kProducts = 2 * MT * NT, kPerRead = NT == 8 ? 2 : 1;
-        constexpr int kPerLoad = (kProducts - kPerRead * kReads) / kLoads > 0 ? (kProducts - kPerRead * kReads) / kLoads : 1;
+        constexpr int kReads = 2 * MT + NT, kProducts = 2 * MT * NT, kPerRead = NT == 8 ? 2 : 1, kLoads = (sub == 0 ? 2 * AL : 0) + (loads_b ? BL : 0);
 #pragma unroll
         for (int i = 0; i < kReads; ++i) {
             __builtin_amdgcn_sched_group_barrier(0x008, kPerRead, 0);
             __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
         }
-        if constexpr (sub == 0) {
+        if constexpr (kLoads > 0) {
+            constexpr int kPerLoad = (kProducts - kPerRead * kReads) / kLoads > 0 ? (kProducts - kPerRead * kReads) / kLoads : 1;
 #pragma unroll
             for (int i = 0; i < kLoads; ++i) {
                 __builtin_amdgcn_sched_group_barrier(0x008, kPerLoad, 0);
@@ -413,7 +470,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_tiled_kernel(const _Float16*
     auto stage = [&](auto ph_c, int s) __attribute__((always_inline)) {
         sub_step(ph_c, std::integral_constant<int, 0>(), s);
         if constexpr (KS == 2) sub_step(ph_c, std::integral_constant<int, 1>(), s);
-        wait_and_meet(std::integral_constant<int, kInFlight>());
+        wait_and_meet(std::integral_constant<int, Flight::at(kEven + decltype(ph_c)::value)>());
     };
     // Small tiles have registers to keep the sums of a period (10 or 12 steps) apart from those before: a fraction of the chain of roundings
     // that all of K would be (as short as the parts of K that small grids are otherwise cut into).
@@ -526,10 +583,11 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_tiled_kernel(const _Float16*
     else store_tile(std::false_type{});
 }
 
-template <int MT, int NT, int KS, int kBufs>
+template <int MT, int NT, int KS, int kBufs, int kBBufs = kBufs>
 int launch_tiles(hipStream_t stream, const _Float16* hi, const _Float16* lo, const float* row_scale, TiledMats mats, int M, int K, int k_splits) {
-    constexpr int BM = 32 * MT, BN = 32 * NT, bytes = kBufs * (2 * BM + BN) * 64 * KS;
-    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_tiled_kernel<MT, NT, KS, kBufs>),
+    constexpr int BM = 32 * MT, BN = 32 * NT, bytes = kBufs * 2 * BM * 64 * KS + kBBufs * BN * 128;
+    static_assert(bytes <= 160 * 1024);
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_tiled_kernel<MT, NT, KS, kBufs, kBBufs>),
                                                        hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
     if (attr != hipSuccess) return -2;
     const int tiles_m = (M + BM - 1) / BM;
@@ -542,7 +600,7 @@ int launch_tiles(hipStream_t stream, const _Float16* hi, const _Float16* lo, con
     // M 4096, N 11264, K 2048 on the 128 x 256 tile (32 tile rows), bands of 4 / 6 rows: 357 / 338 us (bands of 2, 4, 8 and 16 are all slower than 5, 6
     // and 7); M 522, N 2048, K 5632 on 64 x 128 (9 tile rows), bands of 1 / 3 / 5 / 9: 54.2 / 48.1 / 46.7 / 44.4 us
     const int band = tiles_m <= 9 ? tiles_m : 6;
-    gemm_tiled_kernel<MT, NT, KS, kBufs><<<(unsigned)(tiles_m * tiles_n * k_splits), kThreads, bytes, stream>>>(hi, lo, row_scale, mats, M, K, k_splits, band);
+    gemm_tiled_kernel<MT, NT, KS, kBufs, kBBufs><<<(unsigned)(tiles_m * tiles_n * k_splits), kThreads, bytes, stream>>>(hi, lo, row_scale, mats, M, K, k_splits, band);
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 
@@ -570,7 +628,7 @@ TileChoice pick_tile(int M, int n_mats, const int* N, int steps, int num_cus, bo
         for (int i = 0; i < n_mats; ++i) tiles += (N[i] + kShapes[c].bn - 1) / kShapes[c].bn;
         tiles *= (M + kShapes[c].bm - 1) / kShapes[c].bm;
         for (int s = 1; s <= kMaxSplits; ++s) {
-            const int stage = c >= 2 ? 2 : 1, per = (steps / stage + s - 1) / s * stage;
+            const int per = s == 1 ? steps : ((steps + s - 1) / s + 1) & ~1;
             if (s > 1 && (!may_split || per < 16 || (long long)per * (s - 1) >= steps || tiles * (s - 1) >= num_cus)) break;
             if (c < 2 && may_split && s < 4 && per >= 32) continue;
             if (c < 2 && small_grid && !may_split && steps >= 64 && steps % 2 == 0) continue;
@@ -608,6 +666,8 @@ bool m40_gemm_tiled_supported(const void* A, const void* B, int M, int N, int K)
 }
 
 namespace {
+
+int padded_rows(int M) { return (M + 15) / 16 * 16; }
 
 struct TiledCall {
     int source_kind;
@@ -658,7 +718,7 @@ int plan_tiled(const M40llmCudaContext* ctx, const TiledCall& c, TiledPlan& plan
     if (c.pair) { mats.pair = 1; mats.n = 1; mats.N[0] = pair_n; }
     plan.choice = pick_tile(c.M, mats.n, c.pair ? &pair_n : c.N, c.K / kBK, ctx->num_cus, small_grid, small_grid && n4_ok && !c.pair);
     plan.scale_bytes = ((size_t)c.M * 4 + 15) & ~(size_t)15;
-    plan.need = (size_t)c.M * c.K * 4 + plan.scale_bytes + (plan.choice.k_splits > 1 ? (size_t)plan.choice.k_splits * out_floats * 4 : 0);
+    plan.need = (size_t)padded_rows(c.M) * c.K * 4 + plan.scale_bytes + (plan.choice.k_splits > 1 ? (size_t)plan.choice.k_splits * out_floats * 4 : 0);
     return 0;
 }
 
@@ -687,8 +747,8 @@ int provide_pack(M40StreamScratch& sc, hipStream_t stream, size_t need) {
 int enqueue_tiled(const M40StreamScratch& sc, hipStream_t stream, const TiledCall& c, const TiledPlan& plan, PackSource* leave) {
     const int M = c.M, K = c.K, k_splits = plan.choice.k_splits;
     _Float16* hi = static_cast<_Float16*>(sc.tiled_pack);
-    _Float16* lo = hi + (size_t)M * K;
-    float* row_scale = reinterpret_cast<float*>(static_cast<char*>(sc.tiled_pack) + (size_t)M * K * 4);
+    _Float16* lo = hi + (size_t)padded_rows(M) * K;
+    float* row_scale = reinterpret_cast<float*>(static_cast<char*>(sc.tiled_pack) + (size_t)padded_rows(M) * K * 4);
     const PackSource& source = c.source;
     const bool wave_rows = K <= kPackChunks * 64 * 8;
     if (c.source_kind == kPackNorm && source.planes)
@@ -703,7 +763,7 @@ int enqueue_tiled(const M40StreamScratch& sc, hipStream_t stream, const TiledCal
         pack_hilo_planes_kernel<64, kPackPlain><<<(unsigned)((M + 3) / 4), 256, 0, stream>>>(source, hi, lo, row_scale, M, K);
     else
         pack_hilo_planes_kernel<256, kPackPlain><<<(unsigned)M, 256, 0, stream>>>(source, hi, lo, row_scale, M, K);
-    float* partial = reinterpret_cast<float*>(static_cast<char*>(sc.tiled_pack) + (size_t)M * K * 4 + plan.scale_bytes);
+    float* partial = reinterpret_cast<float*>(static_cast<char*>(sc.tiled_pack) + (size_t)padded_rows(M) * K * 4 + plan.scale_bytes);
     TiledMats launch = plan.mats;
     if (k_splits > 1) {
         size_t at = 0;
@@ -714,8 +774,8 @@ int enqueue_tiled(const M40StreamScratch& sc, hipStream_t stream, const TiledCal
     }
     int rc = -2;
     switch (plan.choice.shape) {
-        case 0: rc = launch_tiles<4, 8, 1, 5>(stream, hi, lo, row_scale, launch, M, K, k_splits); break;
-        case 1: rc = launch_tiles<4, 4, 1, 6>(stream, hi, lo, row_scale, launch, M, K, k_splits); break;
+        case 0: rc = launch_tiles<4, 8, 1, 4, 3>(stream, hi, lo, row_scale, launch, M, K, k_splits); break;
+        case 1: rc = launch_tiles<4, 4, 1, 6, 3>(stream, hi, lo, row_scale, launch, M, K, k_splits); break;
         case 2: rc = launch_tiles<2, 4, 2, 5>(stream, hi, lo, row_scale, launch, M, K, k_splits); break;
         case 3: rc = launch_tiles<2, 2, 2, 6>(stream, hi, lo, row_scale, launch, M, K, k_splits); break;
     }

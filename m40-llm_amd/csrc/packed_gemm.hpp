@@ -77,11 +77,6 @@ __device__ __forceinline__ void m40_fragments_ahead() {
     }
     __builtin_amdgcn_sched_group_barrier(0x008, 4 * PER, 0);
 }
-// Workgroup b of a launch over rows: workgroups are dealt to the eight dies in turn, and the rows of a 16-row tile go to one die so
-// that its L2 puts their pieces of the tile's lines together.
-__device__ __forceinline__ uint32_t m40_tile_row(uint32_t b, uint32_t rows) {
-    return (b | 127u) < rows ? (b & ~127u) + (b & 7u) * 16u + ((b & 127u) >> 3) : b;
-}
 __device__ __forceinline__ float m40_sigmoid(float z) { return 1.0f / (1.0f + expf(-z)); }
 __device__ __forceinline__ float m40_silu(float z) { return z / (1.0f + expf(-z)); }
 // 0.5 z (1 + tanh(u)) = z / (1 + exp(-2 u)), u = sqrt(2 / pi) (z + 0.044715 z^3)

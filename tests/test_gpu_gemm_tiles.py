@@ -16,7 +16,7 @@ def dev():
 # 32, one step, fewer steps than buffers, columns that no float4 divides, more than one round of tiles
 @pytest.mark.parametrize("M,N,K", [(33, 16, 32), (33, 17, 64), (64, 64, 2048), (65, 130, 2112), (127, 1030, 5632), (129, 2048, 320), (200, 2560, 2080), (257, 2048, 5632),
                                    (257, 2049, 2048), (385, 2044, 1984), (522, 2048, 2048), (522, 2560, 2048), (522, 2050, 5600), (640, 2048, 2016), (1030, 2048, 2048),
-                                   (1030, 5640, 96), (1301, 3001, 352), (2049, 2300, 160)])
+                                   (1030, 5640, 96), (1301, 3001, 352), (2049, 2300, 160), (1030, 5640, 864), (2065, 2300, 800)])
 def test_many_rows_tiles_vs_float64(dev, M, N, K):
     rng = np.random.default_rng(M * 7 + N * 3 + K)
     A = rng.standard_normal((M, K)).astype(np.float32)
