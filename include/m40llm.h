@@ -587,6 +587,11 @@ int m40llm_ext_pack_tiles_async(M40llmCudaContext* ctx, const void* d_src_bf16, 
 /* n bf16 values, uniform with mean 0 and the given standard deviation, from a counter-based generator */
 int m40llm_ext_fill_random_bf16_async(M40llmCudaContext* ctx, void* d_dst, uint64_t n, uint64_t seed, float std_dev,
                                       uint32_t stream_kind);
+/* Pinned host memory that kernels reach, and a copy of n 32-bit words by a kernel of the stream: between device memory and such memory it needs no
+ * blocking call (the host reads what was copied once it has waited for the stream). */
+int m40llm_ext_pinned_malloc(M40llmCudaContext* ctx, size_t bytes, void** out_ptr);
+int m40llm_ext_pinned_free(M40llmCudaContext* ctx, void* ptr);
+int m40llm_ext_copy_words_async(M40llmCudaContext* ctx, void* dst, const void* src, size_t n_words, uint32_t stream_kind);
 /* clears n 32-bit words with a kernel */
 int m40llm_ext_clear_u32_async(M40llmCudaContext* ctx, void* d_dst, size_t n, uint32_t stream_kind);
 

@@ -46,6 +46,13 @@ __global__ void rope_table_kernel(float* table, uint32_t head_dim, float base) {
     if (i < head_dim / 2u) table[i] = m40_rope_inv_freq(i, head_dim, base);
 }
 
+// 32-bit words between device memory and pinned host memory (or any two places a kernel can reach), 16 bytes a lane where both ends allow it
+__global__ __launch_bounds__(256) void copy_words_kernel(uint32_t* __restrict__ dst, const uint32_t* __restrict__ src, size_t n, size_t quads) {
+    const size_t first = (size_t)blockIdx.x * 256 + threadIdx.x, step = (size_t)gridDim.x * 256;
+    for (size_t i = first; i < quads; i += step) reinterpret_cast<uint4*>(dst)[i] = reinterpret_cast<const uint4*>(src)[i];
+    for (size_t i = 4 * quads + first; i < n; i += step) dst[i] = src[i];
+}
+
 }  // namespace
 
 float4* m40_rope_cs_cache(M40llmCudaContext* ctx, const float* table) {
@@ -204,6 +211,34 @@ int m40llm_memcpy_d2h(M40llmCudaContext* ctx, void* dst_host, const void* src_de
     if (m40_ensure_device(ctx) != 0) return -3;
     if (hipMemcpy(dst_host, src_device, bytes, hipMemcpyDeviceToHost) != hipSuccess) return -2;
     return 0;
+}
+
+int m40llm_ext_pinned_malloc(M40llmCudaContext* ctx, size_t bytes, void** out_ptr) {
+    if (!ctx || !out_ptr) return -1;
+    if (m40_ensure_device(ctx) != 0) return -2;
+    void* p = nullptr;
+    if (hipHostMalloc(&p, bytes ? bytes : 4, hipHostMallocDefault) != hipSuccess) return -3;
+    *out_ptr = p;
+    return 0;
+}
+
+int m40llm_ext_pinned_free(M40llmCudaContext* ctx, void* ptr) {
+    if (!ctx || !ptr) return -1;
+    if (m40_ensure_device(ctx) != 0) return -2;
+    return hipHostFree(ptr) == hipSuccess ? 0 : -3;
+}
+
+int m40llm_ext_copy_words_async(M40llmCudaContext* ctx, void* dst, const void* src, size_t n_words, uint32_t stream_kind) {
+    if (!ctx || !dst || !src) return -1;
+    if (m40_ensure_device(ctx) != 0) return -2;
+    hipStream_t stream = m40_select_stream(ctx, stream_kind);
+    if (!stream) return -2;
+    if (reinterpret_cast<uintptr_t>(dst) % 4 != 0 || reinterpret_cast<uintptr_t>(src) % 4 != 0) return -3;
+    if (n_words == 0) return 0;
+    const size_t quads = m40_aligned16(dst) && m40_aligned16(src) ? n_words / 4 : 0, items = quads ? quads : n_words, blocks = (items + 255) / 256;
+    (void)hipGetLastError();
+    copy_words_kernel<<<(unsigned)(blocks < 512 ? blocks : 512), 256, 0, stream>>>(static_cast<uint32_t*>(dst), static_cast<const uint32_t*>(src), n_words, quads);
+    return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 
 int m40llm_memcpy_d2d_async(M40llmCudaContext* ctx, void* dst_device, const void* src_device,

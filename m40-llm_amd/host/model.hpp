@@ -85,6 +85,33 @@ private:
     size_t bytes_ = 0;
 };
 
+// Host memory that kernels read and write.
+class PinnedBuf {
+public:
+    PinnedBuf() = default;
+    PinnedBuf(M40llmCudaContext* ctx, size_t bytes) : ctx_(ctx), bytes_(bytes) {
+        if (m40llm_ext_pinned_malloc(ctx, bytes, &p_) != 0) throw std::runtime_error("pinned_malloc failed");
+    }
+    PinnedBuf(PinnedBuf&& o) noexcept : ctx_(o.ctx_), p_(o.p_), bytes_(o.bytes_) { o.p_ = nullptr; o.bytes_ = 0; }
+    PinnedBuf& operator=(PinnedBuf&& o) noexcept {
+        reset();
+        ctx_ = o.ctx_; p_ = o.p_; bytes_ = o.bytes_; o.p_ = nullptr; o.bytes_ = 0;
+        return *this;
+    }
+    PinnedBuf(const PinnedBuf&) = delete;
+    PinnedBuf& operator=(const PinnedBuf&) = delete;
+    ~PinnedBuf() { reset(); }
+    void reset() { if (p_) m40llm_ext_pinned_free(ctx_, p_); p_ = nullptr; bytes_ = 0; }
+    uint32_t* u32() const { return static_cast<uint32_t*>(p_); }
+    float* f32(size_t off = 0) const { return static_cast<float*>(p_) + off; }
+    size_t bytes() const { return bytes_; }
+
+private:
+    M40llmCudaContext* ctx_ = nullptr;
+    void* p_ = nullptr;
+    size_t bytes_ = 0;
+};
+
 // Named f32 scratch buffers sized by row count (src/infer/workspace.rs:60-126).
 struct ForwardWorkspace {
     uint32_t rows = 0;

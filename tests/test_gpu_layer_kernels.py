@@ -489,3 +489,24 @@ def test_greedy_pick_ties_and_gap(ctx, vocab):
         assert np.array_equal(gaps[:, 0], srt[:, -1] - srt[:, -2])
     assert np.array_equal(b[0].download(np.uint32, (rows,)), ids[:, 0]) and np.array_equal(b[1].download(np.uint32, (rows,)), ids[:, 0])
     assert np.all(b[2].download(np.uint32, (rows,)) == 11) and b[3].download(np.uint32, (4,))[0] == 2
+
+
+@pytest.mark.parametrize("at", [0, 4, 16])
+@pytest.mark.parametrize("n", [1, 3, 4, 1027, 600001])       # one workgroup's quads and words, and more than the grid's widest step
+def test_copy_words(ctx, n, at):
+    """Device words to pinned host memory and back, from offsets that allow 16 bytes a lane and that do not: the same words, none beside them."""
+    rng = np.random.default_rng(n)
+    src = rng.integers(0, 2 ** 32, n + 4, dtype=np.uint32)
+    d, back = ctx.to_device(np.concatenate([np.zeros(at // 4, np.uint32), src])), ctx.to_device(np.zeros(n + 4, np.uint32))
+    host = C.c_void_p()
+    call(ctx, "m40llm_ext_pinned_malloc", 4 * n + 16, C.byref(host))
+    view = np.ctypeslib.as_array(C.cast(host, C.POINTER(C.c_uint32)), (n + 4,))
+    view[:] = 7
+    call(ctx, "m40llm_ext_copy_words_async", host, d.ptr + at, n, 1)
+    assert np.array_equal(view[:n], src[:n]) and (view[n:] == 7).all()
+    call(ctx, "m40llm_ext_copy_words_async", back.ptr, host, n, 1)
+    got = back.download(np.uint32, (n + 4,))
+    assert np.array_equal(got[:n], src[:n]) and not got[n:].any()
+    call(ctx, "m40llm_ext_copy_words_async", host.value + 2, d.ptr, n, 1, rc=-3)
+    call(ctx, "m40llm_ext_copy_words_async", host, d.ptr, 0, 1)
+    call(ctx, "m40llm_ext_pinned_free", host)
