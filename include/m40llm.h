@@ -393,6 +393,18 @@ int m40llm_ext_prefill_rope_append_on_stream_async(M40llmCudaContext* ctx, M40ll
                                                    uint32_t q_heads, float freq_base, float freq_scale, uint32_t rope_layout,
                                                    const void* d_bq_f32, const void* d_bk_f32, const void* d_bv_f32,
                                                    uint32_t stream_kind);
+/* Rotation, cache append and attention of whole prompts (rows from position 0 on) without rotated rows in memory: Q, K and V as the projections
+ * left them (nothing is written back), the rows' rotations from m40llm_ext_prefill_angles_async ([rows][head_dim / 2] (cos, sin), one call for
+ * all layers), offsets and lengths on the device and on the host, the same values.  Out and cache are bit for bit what
+ * m40llm_ext_prefill_rope_append_on_stream_async and m40llm_ext_attention_prefill_f32_gqa_varlen_host_tables_async leave.  Prefill stream.  -1 null, -2
+ * batch / slot / layout / biases, -4 alignment, -5 past max_seq_len, -6 not a dense cache, -8 a slot named twice, otherwise as the attention call. */
+int m40llm_ext_prefill_attention_rope_append_async(M40llmCudaContext* ctx, M40llmKVCache* kv, const void* q_dev_f32, const void* k_dev_f32,
+                                                   const void* v_dev_f32, const uint32_t* offsets_dev, const uint32_t* lens_dev, uint32_t batch,
+                                                   const uint32_t* seq_slots_host, const uint32_t* offsets_host, const uint32_t* lens_host, uint32_t q_heads,
+                                                   uint32_t rope_layout, const void* d_angles, const void* d_bq_f32, const void* d_bk_f32,
+                                                   const void* d_bv_f32, void* out_dev_f32);
+int m40llm_ext_prefill_angles_async(M40llmCudaContext* ctx, uint32_t batch, const uint32_t* lens_host, uint32_t head_dim, float freq_base, float freq_scale,
+                                    void* d_angles, uint32_t stream_kind);
 /* Many-row projections of the packed prefill with the element-wise step before them and the residual add after them
  * folded in (src/infer/forward.rs:2300-2345, 2440-2530 issue these as rms_norm / swiglu, the GEMMs and residual_add, one
  * launch each).  The rows that enter the product are, by source_kind,

@@ -53,6 +53,7 @@ struct M40llmCudaContext {
     struct { float base; uint32_t head_dim; uint32_t ready; } rope_slots[2][4];
 };
 constexpr int kM40HostStagingWords = 2048;
+constexpr int kM40PrefillSeqs = 64;       // sequences of a packed prefill's by-value tables
 constexpr uint32_t kM40OldStoreSlackRows = 64;
 constexpr int kM40RopeSlots = 4;
 constexpr int kM40RopeTableLen = 256;

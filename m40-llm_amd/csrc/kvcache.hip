@@ -72,7 +72,7 @@ __global__ __launch_bounds__(kThreads) void dense_append_f16_kernel(
 // is found in the by-value table (at most kPrefillSeqs sequences).  Same rotation function and the same inverse
 // frequencies as the per-token appends and the standalone RoPE, so the bits agree with the per-token call sequence
 // (reference: src/infer/forward.rs:2349-2396, three launches per token and layer).
-constexpr int kPrefillSeqs = 64;
+constexpr int kPrefillSeqs = kM40PrefillSeqs;
 struct PrefillSeqTable {
     uint32_t n;
     uint32_t slot[kPrefillSeqs], q_off[kPrefillSeqs], len[kPrefillSeqs], start[kPrefillSeqs];
@@ -163,6 +163,17 @@ __global__ __launch_bounds__(kThreads) void prefill_rope_append_kernel(
         }
     }
     if (threadIdx.x == 0 && local + 1u == t.len[s]) seq_map[slot] = position + 1u;
+}
+
+// The rotations of a packed batch's rows, once for all layers and heads: [row][head_dim / 2] (cos, sin)
+__global__ __launch_bounds__(kThreads) void prefill_angles_kernel(float2* __restrict__ out, PrefillSeqTable t, uint32_t rows, uint32_t head_dim,
+                                                                  const float* __restrict__ inv_freq_table, float freq_base, float freq_scale) {
+    const uint32_t half_dim = head_dim / 2u, i = blockIdx.x * kThreads + threadIdx.x, row = i / half_dim, off = i % half_dim;
+    if (row >= rows) return;
+    uint32_t s = 0;
+    for (uint32_t j = 1; j < t.n; ++j)
+        if (row >= t.q_off[j]) s = j;
+    out[i] = m40_rope_cos_sin_freq(t.start[s] + row - t.q_off[s], inv_freq_table ? inv_freq_table[off] : m40_rope_inv_freq(off, head_dim, freq_base), freq_scale);
 }
 
 // Compressed append: one wave per kv head.  Phase 1 reads the ring row that is about to be
@@ -632,6 +643,29 @@ int m40llm_ext_prefill_rope_append_on_stream_async(M40llmCudaContext* ctx, M40ll
         static_cast<float*>(d_q_f32), static_cast<float*>(d_k_f32), static_cast<float*>(d_v_f32), kv->d_k, kv->d_v,
         kv->d_seq_map, t, q_heads, kv->num_heads, kv->head_dim, kv->max_seq_len, table, freq_base, freq_scale, rope_layout,
         static_cast<const float*>(d_bq_f32), static_cast<const float*>(d_bk_f32), static_cast<const float*>(d_bv_f32));
+    return hipGetLastError() == hipSuccess ? 0 : -6;
+}
+
+int m40llm_ext_prefill_angles_async(M40llmCudaContext* ctx, uint32_t batch, const uint32_t* lens_host, uint32_t head_dim, float freq_base, float freq_scale,
+                                    void* d_angles, uint32_t stream_kind) {
+    if (!ctx || !lens_host || !d_angles) return -1;
+    if (stream_kind > 1u || batch == 0 || batch > (uint32_t)kPrefillSeqs) return -2;
+    if (head_dim == 0 || head_dim % 2 != 0) return -3;
+    PrefillSeqTable t{};
+    t.n = batch;
+    uint64_t rows = 0;
+    for (uint32_t i = 0; i < batch; ++i) {
+        if (lens_host[i] == 0) return -7;
+        t.q_off[i] = (uint32_t)rows;
+        t.len[i] = lens_host[i];
+        rows += lens_host[i];
+        if (rows * (head_dim / 2u) > 0x7fffffffull) return -2;
+    }
+    hipStream_t stream = stream_kind == M40LLM_STREAM_PREFILL ? ctx->prefill_stream : ctx->decode_stream;
+    const float* table = m40_rope_inv_freq_table(ctx, stream_kind, stream, head_dim, freq_base);
+    (void)hipGetLastError();
+    prefill_angles_kernel<<<(unsigned)((rows * (head_dim / 2u) + kThreads - 1) / kThreads), kThreads, 0, stream>>>(static_cast<float2*>(d_angles), t, (uint32_t)rows, head_dim,
+                                                                                                                 table, freq_base, freq_scale);
     return hipGetLastError() == hipSuccess ? 0 : -6;
 }
 

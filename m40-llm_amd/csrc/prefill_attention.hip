@@ -29,6 +29,8 @@
 // (lengths are read back to the host and validated before the launch, also in the _async form).
 #include "common.hpp"
 
+#include <type_traits>
+
 #include <vector>
 
 namespace {
@@ -68,6 +70,8 @@ __device__ __forceinline__ void fragment_pipeline() {
         __builtin_amdgcn_sched_group_barrier(0x008, PER, 0);
     }
 }
+// The rotated value itself goes into the split: without this the compiler folds rotation and conversion into one multiply-add rounded to f16 (m40_f2h)
+__device__ __forceinline__ void rounded(float& x) { asm volatile("" : "+v"(x)); }
 // x = hi + lo with both parts f16: exact to about 2^-22 relative for values inside the f16 range
 __device__ __forceinline__ void split(float x, _Float16* hi, _Float16* lo) {
     const _Float16 h = static_cast<_Float16>(x);
@@ -82,6 +86,18 @@ struct PrefillArgs {
     const uint32_t* q_offsets; const uint32_t* kv_offsets; const uint32_t* q_lens; const uint32_t* kv_lens;
     uint32_t q_heads, kv_heads;
 };
+
+// Prompts that go in unrotated: rows 0 .. of sequence b are its positions 0 ..; queries are rotated where they are loaded, keys where they are
+// packed, which also appends them to the dense cache.
+struct PrefillRope {
+    const float2* angles;       // [row of the packed batch][HD / 2] (cos, sin)
+    const float *bq, *bk, *bv;  // added before the rotation, or null
+    uint32_t layout, max_seq_len;
+    uint16_t *k_cache, *v_cache;
+    uint32_t* seq_map;
+    uint32_t slot[kM40PrefillSeqs];
+};
+struct NoRope {};
 
 // Order of a tile's 32 keys along the k dimension of the P . V product: k-slot 8 g + i holds key 4 g + i (i < 4) or
 // key 16 + 4 g + (i - 4): exactly the eight keys whose scores lane group g holds after the two score products, so the
@@ -98,8 +114,12 @@ __device__ __forceinline__ uint32_t first_tile_of(uint32_t kv_offset, uint32_t b
 // K and V of one 32-key tile and kv head -> two f16 planes each, V transposed, in the order the attention kernel copies
 // them to LDS.  Done once per call so that the 64-query workgroups (and the q heads of a group) do not each repeat the
 // split.  Keys past the sequence end are written as zeros (they are masked anyway).
-template <int HD>
-__global__ __launch_bounds__(kThreads) void prefill_pack_kv_kernel(PrefillArgs p) {
+// With a PrefillRope the keys are rotated here and both go to the cache as well: the pass that rotated Q and K in place and appended K and V was a
+// launch of its own that read and wrote all of Q (4096 rows, 32 + 4 heads of 64: 21.2 us and 5.7 for the packing; one launch).  A thread holds
+// quads of columns that rotate with each other.
+template <int HD, class ROPE>
+__global__ __launch_bounds__(kThreads) void prefill_pack_kv_kernel(PrefillArgs p, ROPE rope) {
+    constexpr bool kRope = std::is_same<ROPE, PrefillRope>::value;
     constexpr int kKTile = key_tile_of(HD);
     __shared__ float vt[kKTile][HD + 1];
     const uint32_t b = blockIdx.z, kvh = blockIdx.y, tile = blockIdx.x;
@@ -112,22 +132,74 @@ __global__ __launch_bounds__(kThreads) void prefill_pack_kv_kernel(PrefillArgs p
     _Float16* kh = out, *kl = out + kKTile * HD, *vh = out + 2 * kKTile * HD, *vl = out + 3 * kKTile * HD;
     // All of a thread's elements are requested together, four a load where K and V are aligned for it, and stored four and eight at a time: a tile
     // is one round trip, not one per element (60 tiles of 64 keys x 64: 9.9 us one by one, 4.7 us now)
-    constexpr int kQuads = kKTile * HD / 4 / kThreads;
-    float4 kx[kQuads], vx[kQuads];
+    constexpr int kQuads = kKTile * HD / 4 / kThreads, kHalf = HD / 2;
+    static_assert(kQuads % 2 == 0, "quads come in pairs");
+    // where quad u of the thread lies in the tile: quads 2 i and 2 i + 1 hold columns that rotate with each other
+    int at[kQuads];
+    bool neox = true;
+    if constexpr (kRope) neox = rope.layout == M40LLM_ROPE_LAYOUT_NEOX;
+#pragma unroll
+    for (int u = 0; u < kQuads; ++u) {
+        const int pair = (int)threadIdx.x + u / 2 * kThreads, key_in = pair / (HD / 8), c = pair % (HD / 8);
+        at[u] = kRope ? key_in * HD + (neox ? 4 * c + u % 2 * kHalf : 8 * c + 4 * (u % 2)) : ((int)threadIdx.x + u * kThreads) * 4;
+    }
+    float4 kx[kQuads], vx[kQuads], cs[kRope ? kQuads : 1];
     auto load = [&](auto quad) {
 #pragma unroll
         for (int u = 0; u < kQuads; ++u) {
-            const int e = ((int)threadIdx.x + u * kThreads) * 4, key_in = e / HD, d = e % HD;
+            const int key_in = at[u] / HD, d = at[u] % HD;
             const uint32_t key = tile * kKTile + key_in, row = key < kv_len ? key : kv_len - 1;
+            // the four angles of a pair of quads, two by each
+            if constexpr (kRope) {
+                const int off = (neox ? at[u & ~1] : at[u & ~1] / 2) % kHalf + 2 * (u % 2);
+                cs[u] = *reinterpret_cast<const float4*>(rope.angles + ((size_t)p.kv_offsets[b] + row) * kHalf + off);
+            }
             kx[u] = quad(Kb + (size_t)row * row_stride + d);
             vx[u] = quad(Vb + (size_t)row * row_stride + d);
         }
     };
     if (m40_aligned16(Kb) && m40_aligned16(Vb)) load([](const float* x) { return *reinterpret_cast<const float4*>(x); });
     else load([](const float* x) { return make_float4(x[0], x[1], x[2], x[3]); });
+    if constexpr (kRope) {
+        auto add = [](float4& x, const float* bias) { x = make_float4(x.x + bias[0], x.y + bias[1], x.z + bias[2], x.w + bias[3]); };
+#pragma unroll
+        for (int u = 0; u < kQuads; ++u) {
+            const int d = at[u] % HD;
+            if (rope.bk) add(kx[u], rope.bk + kvh * HD + d);
+            if (rope.bv) add(vx[u], rope.bv + kvh * HD + d);
+        }
+        const size_t slot_row = (size_t)rope.slot[b] * rope.max_seq_len;
+#pragma unroll
+        for (int u = 0; u < kQuads; u += 2) {
+            float4 &x = kx[u], &y = kx[u + 1];
+            const float4 c0 = cs[u], c1 = cs[u + 1];
+            if (neox) {
+                m40_rope_apply(make_float2(c0.x, c0.y), x.x, y.x, &x.x, &y.x);
+                m40_rope_apply(make_float2(c0.z, c0.w), x.y, y.y, &x.y, &y.y);
+                m40_rope_apply(make_float2(c1.x, c1.y), x.z, y.z, &x.z, &y.z);
+                m40_rope_apply(make_float2(c1.z, c1.w), x.w, y.w, &x.w, &y.w);
+            } else {
+                m40_rope_apply(make_float2(c0.x, c0.y), x.x, x.y, &x.x, &x.y);
+                m40_rope_apply(make_float2(c0.z, c0.w), x.z, x.w, &x.z, &x.w);
+                m40_rope_apply(make_float2(c1.x, c1.y), y.x, y.y, &y.x, &y.y);
+                m40_rope_apply(make_float2(c1.z, c1.w), y.z, y.w, &y.z, &y.w);
+            }
+            rounded(x.x); rounded(x.y); rounded(x.z); rounded(x.w);
+            rounded(y.x); rounded(y.y); rounded(y.z); rounded(y.w);
+        }
+#pragma unroll
+        for (int u = 0; u < kQuads; ++u) {
+            const uint32_t key = tile * kKTile + at[u] / HD;
+            if (key >= kv_len) continue;
+            const size_t to = (slot_row + key) * row_stride + (size_t)kvh * HD + at[u] % HD;
+            *reinterpret_cast<ushort4*>(rope.k_cache + to) = make_ushort4(m40_f2h(kx[u].x), m40_f2h(kx[u].y), m40_f2h(kx[u].z), m40_f2h(kx[u].w));
+            *reinterpret_cast<ushort4*>(rope.v_cache + to) = make_ushort4(m40_f2h(vx[u].x), m40_f2h(vx[u].y), m40_f2h(vx[u].z), m40_f2h(vx[u].w));
+        }
+        if (tile == 0 && kvh == 0 && threadIdx.x == 0) rope.seq_map[rope.slot[b]] = kv_len;
+    }
 #pragma unroll
     for (int u = 0; u < kQuads; ++u) {
-        const int e = ((int)threadIdx.x + u * kThreads) * 4, key_in = e / HD, d = e % HD;
+        const int e = at[u], key_in = e / HD, d = e % HD;
         const bool live = tile * kKTile + key_in < kv_len;
         const float k4[4] = {kx[u].x, kx[u].y, kx[u].z, kx[u].w}, v4[4] = {vx[u].x, vx[u].y, vx[u].z, vx[u].w};
         half4 hi, lo;
@@ -161,8 +233,9 @@ __global__ __launch_bounds__(kThreads) void prefill_pack_kv_kernel(PrefillArgs p
 
 // QB: 16-query blocks per wave.  With two, every K and V fragment a wave reads from LDS serves 32 queries instead of 16:
 // the kernel's LDS traffic (each wave reads the whole K and V tile) was what it spent most of its time on.
-template <int HD, int QB>
-__global__ __launch_bounds__(kThreads) void prefill_attn_kernel(PrefillArgs p) {
+template <int HD, int QB, class ROPE>
+__global__ __launch_bounds__(kThreads) void prefill_attn_kernel(PrefillArgs p, ROPE rope) {
+    constexpr bool kRope = std::is_same<ROPE, PrefillRope>::value;
     constexpr int kKTile = key_tile_of(HD);
     constexpr int KB = kKTile / 16;        // 16-key score blocks of a tile
     constexpr int KS = HD / 32;            // matrix-instruction k-steps of a score tile
@@ -212,14 +285,54 @@ __global__ __launch_bounds__(kThreads) void prefill_attn_kernel(PrefillArgs p) {
         row_end[qb] = shift + my_q;
         blk_end[qb] = shift + (bq0 + 15u < q_len ? bq0 + 15u : q_len - 1);
         const float* qp = p.Q + ((size_t)(p.q_offsets[b] + my_q) * p.q_heads + h) * HD + 8 * g;
+        float x[KS][8];
 #pragma unroll
         for (int s = 0; s < KS; ++s) {
             const float4 x0 = *reinterpret_cast<const float4*>(qp + 32 * s), x1 = *reinterpret_cast<const float4*>(qp + 32 * s + 4);
-            const float x[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+            x[s][0] = x0.x; x[s][1] = x0.y; x[s][2] = x0.z; x[s][3] = x0.w; x[s][4] = x1.x; x[s][5] = x1.y; x[s][6] = x1.z; x[s][7] = x1.w;
+        }
+        if constexpr (kRope) {
+            // a lane holds both columns of its pairs: neighbours, or 32 s + 8 g + i and half a head further on
+            constexpr int kHalf = HD / 2, HS = KS / 2;
+            const bool neox = rope.layout == M40LLM_ROPE_LAYOUT_NEOX;
+            const float2* angles = rope.angles + ((size_t)p.q_offsets[b] + my_q) * kHalf + (neox ? 8 * g : 4 * g);
+            float4 cs[HS][4];
+#pragma unroll
+            for (int s = 0; s < HS; ++s)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)      // layout of neighbours: two angles of step s, two of step s + HS at a time
+                    cs[s][i] = *reinterpret_cast<const float4*>(angles + (neox ? 32 * s + 2 * i : 16 * (s + HS * (i >> 1)) + 2 * (i & 1)));
+            if (rope.bq) {
+#pragma unroll
+                for (int s = 0; s < KS; ++s)
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) x[s][i] += rope.bq[(size_t)h * HD + 32 * s + 8 * g + i];
+            }
+#pragma unroll
+            for (int s = 0; s < HS; ++s)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float2 c0 = make_float2(cs[s][i].x, cs[s][i].y), c1 = make_float2(cs[s][i].z, cs[s][i].w);
+                    if (neox) {
+                        m40_rope_apply(c0, x[s][2 * i], x[s + HS][2 * i], &x[s][2 * i], &x[s + HS][2 * i]);
+                        m40_rope_apply(c1, x[s][2 * i + 1], x[s + HS][2 * i + 1], &x[s][2 * i + 1], &x[s + HS][2 * i + 1]);
+                    } else {
+                        float(&y)[8] = x[s + HS * (i >> 1)];
+                        m40_rope_apply(c0, y[4 * (i & 1)], y[4 * (i & 1) + 1], &y[4 * (i & 1)], &y[4 * (i & 1) + 1]);
+                        m40_rope_apply(c1, y[4 * (i & 1) + 2], y[4 * (i & 1) + 3], &y[4 * (i & 1) + 2], &y[4 * (i & 1) + 3]);
+                    }
+                }
+#pragma unroll
+            for (int s = 0; s < KS; ++s)
+#pragma unroll
+                for (int i = 0; i < 8; ++i) rounded(x[s][i]);
+        }
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
                 _Float16 a, c;
-                split(x[i], &a, &c);
+                split(x[s][i], &a, &c);
                 qh[qb][s][i] = a;
                 ql[qb][s][i] = c;
             }
@@ -416,7 +529,7 @@ int prefill_impl(M40llmCudaContext* ctx, const void* q, const void* k, const voi
                  const uint32_t* kv_offsets, const uint32_t* q_lens, const uint32_t* kv_lens, uint32_t batch,
                  uint32_t q_heads, uint32_t kv_heads, uint32_t head_dim, void* out, bool synchronize,
                  const uint32_t* kv_offsets_host = nullptr, const uint32_t* q_lens_host = nullptr,
-                 const uint32_t* kv_lens_host = nullptr) {
+                 const uint32_t* kv_lens_host = nullptr, const PrefillRope* rope = nullptr) {
     if (!ctx || !q || !k || !v || !q_offsets || !kv_offsets || !q_lens || !kv_lens || !out) return -1;
     if (batch == 0) return -2;
     if (q_heads == 0 || kv_heads == 0 || q_heads % kv_heads != 0) return -3;
@@ -480,15 +593,16 @@ int prefill_impl(M40llmCudaContext* ctx, const void* q, const void* k, const voi
     const uint32_t blocks = long_groups >= (uint64_t)kTwoBlockMinGroupsPerCu * (uint64_t)ctx->num_cus ? 2u : 1u;
     const uint32_t q_group = 16u * kWaves * blocks;     // queries per workgroup
     const dim3 grid(q_heads, (max_q + q_group - 1) / q_group, batch);
-    if (head_dim == 64) {
-        prefill_pack_kv_kernel<64><<<pack_grid, kThreads, 0, ctx->prefill_stream>>>(a);
-        if (blocks == 2) prefill_attn_kernel<64, 2><<<grid, kThreads, 0, ctx->prefill_stream>>>(a);
-        else prefill_attn_kernel<64, 1><<<grid, kThreads, 0, ctx->prefill_stream>>>(a);
-    } else {
-        prefill_pack_kv_kernel<128><<<pack_grid, kThreads, 0, ctx->prefill_stream>>>(a);
-        if (blocks == 2) prefill_attn_kernel<128, 2><<<grid, kThreads, 0, ctx->prefill_stream>>>(a);
-        else prefill_attn_kernel<128, 1><<<grid, kThreads, 0, ctx->prefill_stream>>>(a);
-    }
+    const auto launch = [&](auto hd, auto r) {
+        constexpr int HD = decltype(hd)::value;
+        using R = decltype(r);
+        prefill_pack_kv_kernel<HD, R><<<pack_grid, kThreads, 0, ctx->prefill_stream>>>(a, r);
+        if (blocks == 2) prefill_attn_kernel<HD, 2, R><<<grid, kThreads, 0, ctx->prefill_stream>>>(a, r);
+        else prefill_attn_kernel<HD, 1, R><<<grid, kThreads, 0, ctx->prefill_stream>>>(a, r);
+    };
+    const auto launch_rope = [&](auto hd) { rope ? launch(hd, *rope) : launch(hd, NoRope{}); };
+    if (head_dim == 64) launch_rope(std::integral_constant<int, 64>());
+    else launch_rope(std::integral_constant<int, 128>());
     if (hipGetLastError() != hipSuccess) return -4;
     if (synchronize && hipStreamSynchronize(ctx->prefill_stream) != hipSuccess) return -5;
     return 0;
@@ -527,6 +641,33 @@ int m40llm_ext_attention_prefill_f32_gqa_varlen_host_tables_async(M40llmCudaCont
     if (!kv_offsets_host || !q_lens_host || !kv_lens_host) return -1;
     return prefill_impl(ctx, q_dev_f32, k_dev_f32, v_dev_f32, q_offsets_dev, kv_offsets_dev, q_lens_dev, kv_lens_dev,
                         batch_size, q_heads, kv_heads, head_dim, out_dev_f32, false, kv_offsets_host, q_lens_host, kv_lens_host);
+}
+
+int m40llm_ext_prefill_attention_rope_append_async(M40llmCudaContext* ctx, M40llmKVCache* kv, const void* q_dev_f32, const void* k_dev_f32,
+                                                   const void* v_dev_f32, const uint32_t* offsets_dev, const uint32_t* lens_dev, uint32_t batch,
+                                                   const uint32_t* seq_slots_host, const uint32_t* offsets_host, const uint32_t* lens_host, uint32_t q_heads,
+                                                   uint32_t rope_layout, const void* d_angles, const void* d_bq_f32, const void* d_bk_f32,
+                                                   const void* d_bv_f32, void* out_dev_f32) {
+    if (!ctx || !kv || !q_dev_f32 || !k_dev_f32 || !v_dev_f32 || !offsets_dev || !lens_dev || !seq_slots_host || !offsets_host || !lens_host || !d_angles || !out_dev_f32)
+        return -1;
+    const int n_bias = (d_bq_f32 != nullptr) + (d_bk_f32 != nullptr) + (d_bv_f32 != nullptr);
+    if (batch == 0 || batch > (uint32_t)kM40PrefillSeqs || (n_bias != 0 && n_bias != 3) || rope_layout > M40LLM_ROPE_LAYOUT_NEOX) return -2;
+    if (kv->compressed || !kv->d_k || !kv->d_v) return -6;
+    PrefillRope r{};
+    for (uint32_t i = 0; i < batch; ++i) {
+        if (seq_slots_host[i] >= kv->max_batch_size) return -2;
+        if (lens_host[i] > kv->max_seq_len) return -5;
+        for (uint32_t j = 0; j < i; ++j)
+            if (seq_slots_host[j] == seq_slots_host[i]) return -8;   // two sequences of one call would race on a slot
+        r.slot[i] = seq_slots_host[i];
+    }
+    if (!m40_aligned16(d_angles)) return -4;
+    r.angles = static_cast<const float2*>(d_angles);
+    r.bq = static_cast<const float*>(d_bq_f32); r.bk = static_cast<const float*>(d_bk_f32); r.bv = static_cast<const float*>(d_bv_f32);
+    r.layout = rope_layout; r.max_seq_len = kv->max_seq_len;
+    r.k_cache = kv->d_k; r.v_cache = kv->d_v; r.seq_map = kv->d_seq_map;
+    return prefill_impl(ctx, q_dev_f32, k_dev_f32, v_dev_f32, offsets_dev, offsets_dev, lens_dev, lens_dev, batch, q_heads, kv->num_heads, kv->head_dim, out_dev_f32,
+                        false, offsets_host, lens_host, lens_host, &r);
 }
 
 }  // extern "C"

@@ -135,7 +135,7 @@ struct ForwardWorkspace {
 
 struct PrefillWorkspace {   // activations of a packed prefill: no per-row logits
     uint32_t rows = 0, batch = 0;
-    DeviceBuf xn, q, k, v, att, y, x1, gate, up, hid, a, b, tokens, offsets, lens;
+    DeviceBuf xn, q, k, v, att, y, x1, gate, up, hid, a, b, tokens, offsets, lens, angles;
     void ensure(M40llmCudaContext* c, const ModelConfig& m, uint32_t want_rows, uint32_t want_batch) {
         if (want_rows > rows) {
             const size_t D = m.d_model, KV = (size_t)m.kv_heads * m.head_dim, F = m.ffn, R = want_rows;
@@ -144,6 +144,7 @@ struct PrefillWorkspace {   // activations of a packed prefill: no per-row logit
             gate = DeviceBuf(c, R * F * 4); up = DeviceBuf(c, R * F * 4); hid = DeviceBuf(c, R * F * 4);
             a = DeviceBuf(c, R * D * 4); b = DeviceBuf(c, R * D * 4);
             tokens = DeviceBuf(c, R * 4);
+            angles = DeviceBuf(c, R * (m.head_dim / 2) * 8);
             rows = want_rows;
         }
         if (want_batch > batch) {
@@ -481,12 +482,13 @@ public:
         float* b = pws_.b.f32();
         M40H_TRY(m40llm_ext_embed_rows_async(ctx_, tok_emb_, pws_.tokens.u32(), rows, cfg_.vocab, D, a));
         M40H_TRY(m40llm_stream_wait_for_stream(ctx_, PRE, DEC));
+        M40H_TRY(m40llm_ext_prefill_angles_async(ctx_, batch, lens, cfg_.head_dim, cfg_.rope_base, cfg_.rope_scale, pws_.angles.ptr(), PRE));
         std::vector<uint32_t> slots(batch);
         const uint32_t* d_off = pws_.offsets.u32();
         const uint32_t* d_len = pws_.lens.u32();
         // Every launch of a layer goes to the prefill stream: RMSNorm is produced inside the GEMMs' packing pass, SwiGLU and the
         // residual adds inside their last step (m40llm_ext_prefill_gemm_fused_async), so a layer is four
-        // projections, the RoPE + append launch and the attention, with no hop between streams.
+        // projections and the two launches of the attention (rotation and append inside), with no hop between streams.
         bool have_qkv = false;
         for (uint32_t l = 0; l < cfg_.n_layers; ++l) {
             const LayerWeights& w = layers_[l];
@@ -494,15 +496,10 @@ public:
             if (!have_qkv)
                 prefill_project(1, a, nullptr, w.attn_norm, pws_.xn.f32(), rows, D, 3, w.wq, D, pws_.q.f32(), w.wk, KV, pws_.k.f32(), w.wv, KV,
                                 pws_.v.f32(), nullptr);
-            M40H_TRY(m40llm_ext_prefill_rope_append_on_stream_async(ctx_, kv_, pws_.q.ptr(), pws_.k.ptr(), pws_.v.ptr(), batch, slots.data(),
-                                                                    lens, nullptr, cfg_.q_heads, cfg_.rope_base, cfg_.rope_scale,
-                                                                    cfg_.rope_layout, cfg_.has_qkv_bias ? w.bq : nullptr,
-                                                                    cfg_.has_qkv_bias ? w.bk : nullptr, cfg_.has_qkv_bias ? w.bv : nullptr,
-                                                                    PRE));
-            M40H_TRY(m40llm_ext_attention_prefill_f32_gqa_varlen_host_tables_async(ctx_, pws_.q.ptr(), pws_.k.ptr(), pws_.v.ptr(), d_off, d_off,
-                                                                                   d_len, d_len, offsets.data(), lens, lens, batch,
-                                                                                   cfg_.q_heads, cfg_.kv_heads, cfg_.head_dim,
-                                                                                   pws_.att.ptr()));
+            M40H_TRY(m40llm_ext_prefill_attention_rope_append_async(ctx_, kv_, pws_.q.ptr(), pws_.k.ptr(), pws_.v.ptr(), d_off, d_len, batch, slots.data(),
+                                                                    offsets.data(), lens, cfg_.q_heads, cfg_.rope_layout, pws_.angles.ptr(),
+                                                                    cfg_.has_qkv_bias ? w.bq : nullptr, cfg_.has_qkv_bias ? w.bk : nullptr,
+                                                                    cfg_.has_qkv_bias ? w.bv : nullptr, pws_.att.ptr()));
             // O projection, norm, gate and up in one call; the down projection, the next layer's norm and Q/K/V likewise
             int gated = m40llm_ext_prefill_project_norm_project_async(ctx_, pws_.att.ptr(), (int)rows, (int)D, w.wo, (int)D, a, pws_.x1.ptr(), w.ffn_norm,
                                                                       cfg_.norm_weight_dtype, cfg_.rms_eps, 1u, 2, w.wgate, (int)F, pws_.hid.ptr(), w.wup, (int)F,

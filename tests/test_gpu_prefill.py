@@ -75,6 +75,52 @@ def test_prefill_rope_append_equals_per_token_calls(dev, layout, bias, hd, q_hea
     close(np.linalg.norm(q_a, axis=1), np.linalg.norm(q + (bq if bias else 0), axis=1), 1e-5, 1e-5)
 
 
+@pytest.mark.parametrize("layout", [0, 1])
+@pytest.mark.parametrize("bias,hd,q_heads,kv_heads,lens", [(False, 64, 4, 1, [1, 63, 64, 65]), (True, 64, 8, 2, [200]), (True, 128, 4, 2, [31, 33, 1]), (False, 64, 32, 4, [4096]),
+                                                           (True, 128, 16, 2, [2100, 2049])])
+def test_prefill_attention_with_rotation_and_append_inside(dev, layout, bias, hd, q_heads, kv_heads, lens):
+    """Lengths around the key tiles of both head sizes, and long ones (two query blocks a wave): output and cache are the bits of the two calls, and Q, K and
+    V stay as they were."""
+    rng = np.random.default_rng(sum(lens) + hd)
+    rows, D, KV, base, n = sum(lens), q_heads * hd, kv_heads * hd, 1e6 if layout else 1e4, len(lens)
+    qkv = [rng.standard_normal((rows, w)).astype(np.float32) for w in (D, KV, KV)]
+    biases = [dev.up(rng.standard_normal(w).astype(np.float32)) for w in (D, KV, KV)]
+    bp = [b.ptr if bias else None for b in biases]
+    slots, h_lens, offs = u32(range(n, 0, -1)), u32(lens), u32(np.concatenate([[0], np.cumsum(lens)[:-1]]))
+    d_lens, d_offs = dev.up(h_lens), dev.up(offs)
+    got = []
+    for inside in (False, True):
+        kv = m40.KVCache(dev.ctx, max(lens) + 3, n + 1, kv_heads, hd)
+        d = [dev.up(a) for a in qkv]
+        out = dev.up(np.full((rows, D), 7, np.float32))
+        if inside:
+            angles = dev.zeros(rows * hd // 2 * 8)
+            dev.call("m40llm_ext_prefill_angles_async", n, h_lens.ctypes.data, hd, base, 1.0, angles.ptr, 0)
+            args = [kv.h, *(a.ptr for a in d), d_offs.ptr, d_lens.ptr, n, slots.ctypes.data, offs.ctypes.data, h_lens.ctypes.data, q_heads, layout, angles.ptr, *bp, out.ptr]
+            dev.call("m40llm_ext_prefill_attention_rope_append_async", *args)
+        else:
+            dev.call("m40llm_ext_prefill_rope_append_on_stream_async", kv.h, *(a.ptr for a in d), n, slots.ctypes.data, h_lens.ctypes.data, None, q_heads, base, 1.0, layout, *bp, 0)
+            dev.call("m40llm_ext_attention_prefill_f32_gqa_varlen_host_tables_async", *(a.ptr for a in d), d_offs.ptr, d_offs.ptr, d_lens.ptr, d_lens.ptr, offs.ctypes.data,
+                     h_lens.ctypes.data, h_lens.ctypes.data, n, q_heads, kv_heads, hd, out.ptr)
+        dev.sync()
+        cache = [kv.read_token(int(s), t) for s, l in zip(slots, lens) for t in {0, l // 2, l - 1}]
+        got.append((out.download(np.uint32, (rows, D)), cache, kv.read_raw(5, np.uint32, n + 1)))
+        if inside:
+            for a, b in zip(d, qkv):
+                assert np.array_equal(a.download(np.uint32, b.shape), b.view(np.uint32))
+            for i, v, rc in ((0, None, -1), (1, None, -1), (6, 0, -2), (6, 65, -2), (11, 2, -2), (12, angles.ptr + 4, -4)):
+                dev.call("m40llm_ext_prefill_attention_rope_append_async", *(args[:i] + [v] + args[i + 1:]), expect=rc)
+            long = u32([max(lens) + 4] * n)
+            dev.call("m40llm_ext_prefill_attention_rope_append_async", *(args[:9] + [long.ctypes.data] + args[10:]), expect=-5)
+            if n > 1:
+                same = u32([1] * n)
+                dev.call("m40llm_ext_prefill_attention_rope_append_async", *(args[:7] + [same.ctypes.data] + args[8:]), expect=-8)
+    assert np.array_equal(got[0][0], got[1][0])
+    for x, y in zip(got[0][1], got[1][1]):
+        assert np.array_equal(x[0], y[0]) and np.array_equal(x[1], y[1])
+    assert np.array_equal(got[0][2], got[1][2])
+
+
 def test_prefill_rope_append_argument_checks(dev):
     kv = m40.KVCache(dev.ctx, 8, 2, 2, 64)
     z = dev.zeros(16 * 4 * 64 * 4)
