@@ -62,7 +62,8 @@ enum { kPackPlain = 0, kPackNorm = 1, kPackSwiglu = 2, kPackSumNorm = 3 };
 // infinity or a NaN is packed unscaled with those elements as they are (their low parts zero), so that its products come
 // out non-finite as the f32 arithmetic of the reference would give them (cuda/kernels.cu:5037-5052), never as a finite
 // value.
-constexpr int kPackChunks = 8;       // 8-element chunks a thread keeps in registers
+constexpr int kPackChunks = 8;       // most 8-element chunks that a thread keeps in registers
+constexpr int kPackStaged = 4096;    // longest row that a norm stages
 
 // SwiGLU of one element, the expression of swiglu_kernel (cuda/kernels.cu:869-880)
 __device__ __forceinline__ float tiled_swiglu(float g, float u) {
@@ -109,7 +110,10 @@ __device__ __forceinline__ size_t plane_step(int c) { return (size_t)(c >> 2) * 
 // ROW_THREADS = 64: a wave per row, four rows per workgroup, no barrier (K <= 4096 keeps the row in registers);
 // 256: a workgroup per row (always for the RMSNorm source, whose sum of squares is formed with the thread layout and
 // order of rms_norm_kernel so that the fused form gives the bits of the two-launch form).
-template <int ROW_THREADS, int KIND>
+// CHUNKS: what a thread keeps.  Registers decide how many rows a CU has in flight: a staged norm needs two chunks, not eight (with the staging 4096 rows of
+// 2048 20.8 -> 14.6 us, 4.6 TB/s; 522 rows 7.8 -> 7.5, as parts of K 9.8 -> 9.2), a wave to a row of 2048 four (13.3 -> 12.9).  A workgroup to
+// a row keeps eight also where four would do: 4096 rows of 5632 take 34.9 us that way and 38.1 with more rows in flight, which write half lines.
+template <int ROW_THREADS, int KIND, int CHUNKS>
 __global__ __launch_bounds__(256) void pack_hilo_planes_kernel(PackSource src_args, _Float16* __restrict__ hi,
                                                                _Float16* __restrict__ lo, float* __restrict__ row_scale,
                                                                int M, int K) {
@@ -117,6 +121,9 @@ __global__ __launch_bounds__(256) void pack_hilo_planes_kernel(PackSource src_ar
     static_assert(!kNorm || ROW_THREADS == 256, "the norm's sums follow rms_norm_kernel's layout");
     __shared__ float wave_max[4];
     __shared__ float wave_sums[4];
+    // A row that is normed passes through LDS from the order of its sums to that of its chunks, and its weights are asked for ahead of the sums: read again
+    // behind the barrier, both cost another round trip, and the row a second pass through the caches
+    __shared__ __attribute__((aligned(16))) float4 staged[kNorm ? kPackStaged / 4 : 1];
     constexpr int kRowsPerGroup = 256 / ROW_THREADS;
     // the rows of a tile on one die (m40_tile_row; a workgroup of four rows: four workgroups a tile)
     const uint32_t b = blockIdx.x, groups = gridDim.x;
@@ -127,6 +134,21 @@ __global__ __launch_bounds__(256) void pack_hilo_planes_kernel(PackSource src_ar
     const float4* src2 = KIND == kPackSwiglu ? reinterpret_cast<const float4*>(src_args.a2 + (size_t)row * K) : nullptr;
     const int chunks = K >> 3;                     // K is a multiple of 32
     float norm_scale = 1.0f;
+    constexpr int kStagedChunks = kPackStaged / 8 / 256;
+    static_assert(kStagedChunks <= CHUNKS);
+    const bool stage = kNorm && K <= kPackStaged;
+    uint4 nw[kNorm ? kStagedChunks : 1][2];
+    if (kNorm && stage) {
+        // f16 weights: the chunk's sixteen bytes, asked for twice (no load under a branch)
+        const uint4* w = static_cast<const uint4*>(src_args.norm_w);
+        const int step = src_args.norm_dtype == 0u ? 1 : 2, second = src_args.norm_dtype == 0u ? 0 : 1;
+#pragma unroll
+        for (int i = 0; i < kStagedChunks; ++i) {
+            const int c = tid + 256 * i < chunks ? tid + 256 * i : 0;
+            nw[kNorm ? i : 0][0] = w[step * c];
+            nw[kNorm ? i : 0][1] = w[step * c + second];
+        }
+    }
     if (kNorm) {
         float ss = 0.0f;
         const size_t row4 = (size_t)row * (K / 4);
@@ -134,10 +156,11 @@ __global__ __launch_bounds__(256) void pack_hilo_planes_kernel(PackSource src_ar
             float4 v;
             if (KIND == kPackSumNorm) {
                 v = sum_planes(src_args.planes, src_args.k_splits, (size_t)M * (K / 4), row4 + i, src_args.residual);
-                src_args.sum[row4 + i] = v;       // read again behind the barrier below
+                src_args.sum[row4 + i] = v;       // long rows: read again behind the barrier below
             } else {
                 v = src[i];
             }
+            if (stage) staged[kNorm ? i : 0] = v;
             ss = fmaf(v.x, v.x, ss);
             ss = fmaf(v.y, v.y, ss);
             ss = fmaf(v.z, v.z, ss);
@@ -151,6 +174,11 @@ __global__ __launch_bounds__(256) void pack_hilo_planes_kernel(PackSource src_ar
         for (int w = 0; w < 4; ++w) total += wave_sums[w];
         norm_scale = 1.0f / sqrtf(total / static_cast<float>(K) + src_args.eps);
     }
+    // x * scale, then * weight: two roundings, as rms_norm_kernel has them
+    auto scale_chunk = [&](const float4 a, const float4 b, const float (&w)[8], float4& o0, float4& o1) {
+        o0 = make_float4(a.x * norm_scale * w[0], a.y * norm_scale * w[1], a.z * norm_scale * w[2], a.w * norm_scale * w[3]);
+        o1 = make_float4(b.x * norm_scale * w[4], b.y * norm_scale * w[5], b.z * norm_scale * w[6], b.w * norm_scale * w[7]);
+    };
     // the eight source values of chunk c
     auto load_chunk = [&](int c, float4& o0, float4& o1) {
         o0 = src[2 * c];
@@ -168,22 +196,33 @@ __global__ __launch_bounds__(256) void pack_hilo_planes_kernel(PackSource src_ar
                 const float4 w0 = reinterpret_cast<const float4*>(src_args.norm_w)[2 * c], w1 = reinterpret_cast<const float4*>(src_args.norm_w)[2 * c + 1];
                 w[0] = w0.x; w[1] = w0.y; w[2] = w0.z; w[3] = w0.w; w[4] = w1.x; w[5] = w1.y; w[6] = w1.z; w[7] = w1.w;
             }
-            // x * scale, then * weight: two roundings, as rms_norm_kernel has them
-            o0 = make_float4(o0.x * norm_scale * w[0], o0.y * norm_scale * w[1], o0.z * norm_scale * w[2], o0.w * norm_scale * w[3]);
-            o1 = make_float4(o1.x * norm_scale * w[4], o1.y * norm_scale * w[5], o1.z * norm_scale * w[6], o1.w * norm_scale * w[7]);
+            scale_chunk(o0, o1, w, o0, o1);
         }
     };
-    const bool in_regs = chunks <= kPackChunks * ROW_THREADS;
-    float4 x0[kPackChunks], x1[kPackChunks];
+    const bool in_regs = chunks <= CHUNKS * ROW_THREADS;
+    float4 x0[CHUNKS], x1[CHUNKS];
     float mx = 0.0f;
     if (in_regs) {
+        if (kNorm && stage) {
 #pragma unroll
-        for (int i = 0; i < kPackChunks; ++i) {
-            const int c = tid + ROW_THREADS * i;
-            if (c < chunks) load_chunk(c, x0[i], x1[i]);
+            for (int i = 0; i < kStagedChunks; ++i) {
+                const int c = tid + 256 * i;
+                if (c >= chunks) continue;
+                const uint4 a = nw[kNorm ? i : 0][0], b = nw[kNorm ? i : 0][1];
+                float w[8] = {__uint_as_float(a.x), __uint_as_float(a.y), __uint_as_float(a.z), __uint_as_float(a.w),
+                              __uint_as_float(b.x), __uint_as_float(b.y), __uint_as_float(b.z), __uint_as_float(b.w)};
+                if (src_args.norm_dtype == 0u) m40_unpack8(a, w);
+                scale_chunk(staged[kNorm ? 2 * c : 0], staged[kNorm ? 2 * c + 1 : 0], w, x0[i], x1[i]);
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < CHUNKS; ++i) {
+                const int c = tid + ROW_THREADS * i;
+                if (c < chunks) load_chunk(c, x0[i], x1[i]);
+            }
         }
 #pragma unroll
-        for (int i = 0; i < kPackChunks; ++i) {
+        for (int i = 0; i < CHUNKS; ++i) {
             if (tid + ROW_THREADS * i < chunks) {
                 mx = fmaxf(mx, fmaxf(fmaxf(pack_abs_or_inf(x0[i].x), pack_abs_or_inf(x0[i].y)), fmaxf(pack_abs_or_inf(x0[i].z), pack_abs_or_inf(x0[i].w))));
                 mx = fmaxf(mx, fmaxf(fmaxf(pack_abs_or_inf(x1[i].x), pack_abs_or_inf(x1[i].y)), fmaxf(pack_abs_or_inf(x1[i].z), pack_abs_or_inf(x1[i].w))));
@@ -197,8 +236,7 @@ __global__ __launch_bounds__(256) void pack_hilo_planes_kernel(PackSource src_ar
             mx = fmaxf(mx, fmaxf(fmaxf(pack_abs_or_inf(b.x), pack_abs_or_inf(b.y)), fmaxf(pack_abs_or_inf(b.z), pack_abs_or_inf(b.w))));
         }
     }
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+    mx = m40_max64(mx);
     if (ROW_THREADS == 256) {
         if ((tid & 63) == 0) wave_max[tid >> 6] = mx;
         __syncthreads();
@@ -218,7 +256,7 @@ __global__ __launch_bounds__(256) void pack_hilo_planes_kernel(PackSource src_ar
     half8* lp = reinterpret_cast<half8*>(lo) + plane_chunk(row, K);
     if (in_regs) {
 #pragma unroll
-        for (int i = 0; i < kPackChunks; ++i) {
+        for (int i = 0; i < CHUNKS; ++i) {
             const int c = tid + ROW_THREADS * i;
             if (c < chunks) {
                 half8 h, l;
@@ -751,18 +789,24 @@ int enqueue_tiled(const M40StreamScratch& sc, hipStream_t stream, const TiledCal
     float* row_scale = reinterpret_cast<float*>(static_cast<char*>(sc.tiled_pack) + (size_t)padded_rows(M) * K * 4);
     const PackSource& source = c.source;
     const bool wave_rows = K <= kPackChunks * 64 * 8;
-    if (c.source_kind == kPackNorm && source.planes)
-        pack_hilo_planes_kernel<256, kPackSumNorm><<<(unsigned)M, 256, 0, stream>>>(source, hi, lo, row_scale, M, K);
-    else if (c.source_kind == kPackNorm)
-        pack_hilo_planes_kernel<256, kPackNorm><<<(unsigned)M, 256, 0, stream>>>(source, hi, lo, row_scale, M, K);
-    else if (c.source_kind == kPackSwiglu && wave_rows)
-        pack_hilo_planes_kernel<64, kPackSwiglu><<<(unsigned)((M + 3) / 4), 256, 0, stream>>>(source, hi, lo, row_scale, M, K);
-    else if (c.source_kind == kPackSwiglu)
-        pack_hilo_planes_kernel<256, kPackSwiglu><<<(unsigned)M, 256, 0, stream>>>(source, hi, lo, row_scale, M, K);
-    else if (wave_rows)
-        pack_hilo_planes_kernel<64, kPackPlain><<<(unsigned)((M + 3) / 4), 256, 0, stream>>>(source, hi, lo, row_scale, M, K);
-    else
-        pack_hilo_planes_kernel<256, kPackPlain><<<(unsigned)M, 256, 0, stream>>>(source, hi, lo, row_scale, M, K);
+    const auto pack = [&](auto row_threads, auto kind, auto chunks) {
+        constexpr int kRowThreads = decltype(row_threads)::value;
+        pack_hilo_planes_kernel<kRowThreads, decltype(kind)::value, decltype(chunks)::value>
+            <<<(unsigned)(kRowThreads == 64 ? (M + 3) / 4 : M), 256, 0, stream>>>(source, hi, lo, row_scale, M, K);
+    };
+    const auto pack_norm = [&](auto kind) {
+        if (K <= kPackStaged) pack(std::integral_constant<int, 256>(), kind, std::integral_constant<int, kPackStaged / 8 / 256>());
+        else pack(std::integral_constant<int, 256>(), kind, std::integral_constant<int, kPackChunks>());
+    };
+    const auto pack_either = [&](auto kind) {
+        if (wave_rows && K <= 4 * 8 * 64) pack(std::integral_constant<int, 64>(), kind, std::integral_constant<int, 4>());
+        else if (wave_rows) pack(std::integral_constant<int, 64>(), kind, std::integral_constant<int, kPackChunks>());
+        else pack(std::integral_constant<int, 256>(), kind, std::integral_constant<int, kPackChunks>());
+    };
+    if (c.source_kind == kPackNorm && source.planes) pack_norm(std::integral_constant<int, kPackSumNorm>());
+    else if (c.source_kind == kPackNorm) pack_norm(std::integral_constant<int, kPackNorm>());
+    else if (c.source_kind == kPackSwiglu) pack_either(std::integral_constant<int, kPackSwiglu>());
+    else pack_either(std::integral_constant<int, kPackPlain>());
     float* partial = reinterpret_cast<float*>(static_cast<char*>(sc.tiled_pack) + (size_t)padded_rows(M) * K * 4 + plan.scale_bytes);
     TiledMats launch = plan.mats;
     if (k_splits > 1) {

@@ -325,6 +325,12 @@ def test_prefill_gemm_fused_equals_separate_calls(dev, kind, M, K, Ns, residual,
         assert np.array_equal(dR.download(np.float32, (M, Ns[0])).view(np.uint32), want[0].view(np.uint32))
 
 
+@pytest.mark.parametrize("kind,K", [(1, 32), (1, 2080), (1, 4096), (1, 4128), (0, 2048), (0, 2080), (0, 8192), (0, 8224)])
+def test_packed_rows_around_what_a_thread_keeps(dev, kind, K):
+    """Rows up to and past what the packing passes stage (norm: 4096) and keep a thread (four or eight chunks)."""
+    test_prefill_gemm_fused_equals_separate_calls(dev, kind, 50, K, (64,), False, K // 32 % 2)
+
+
 def test_prefill_gemm_fused_declines_and_checks(dev):
     rng = np.random.default_rng(3)
     M, K, N = 8, 256, 64
