@@ -38,6 +38,7 @@ struct LatentTiles : PassTable {
         return t;
     }
     uint64_t partial_floats(const Rows& r) const override { return m40llm_ext_latent_attention_partial_floats(r.short_rows * heads, latent_pad, splits); }
+    std::vector<uint32_t> shape() const override { return {n, m_tiles, splits}; }
     uint32_t act_dtype, heads, max_m_tiles, latent_pad, n = 0, m_tiles = 1, splits = 1;
 };
 
@@ -46,6 +47,7 @@ struct LatentJobs : PassTable {
     bool same() const { return true; }
     uint32_t fewest_heads = 0xffffffffu, n_jobs = 0, job_rows = 128, n_pages = 0;
     const uint32_t* list() const { return at + 4 * n_jobs; }
+    std::vector<uint32_t> shape() const override { return {n_jobs, job_rows, n_pages}; }
     std::vector<uint32_t> build(const PassPlan& plan, const SequencePages& pages, uint32_t) override {
         uint32_t blocks = 0;
         for (const Portion& p : plan.portions) blocks += p.is_long ? (p.n + 127) / 128 : 0;

@@ -47,6 +47,8 @@ class PassTable {
 public:
     virtual ~PassTable() = default;
     virtual std::vector<uint32_t> build(const PassPlan& plan, const SequencePages& pages, uint32_t longest) = 0;    // longest: most tokens a short portion sees
+    // what a layer's launches take from the table on the host, beside its place: passes with the same shapes make the same launches
+    virtual std::vector<uint32_t> shape() const = 0;
     virtual uint64_t partial_floats(const Rows&) const { return 0; }
     virtual void enqueue(const Rows&) {}                // what the device makes itself, at the start of a pass
     const uint32_t* at = nullptr;
@@ -56,6 +58,7 @@ public:
 class PortionTable : public PassTable {
 public:
     uint32_t n = 0, singles = 0, n_chunks = 0;
+    std::vector<uint32_t> shape() const override { return {n, singles, n_chunks}; }
     const uint32_t* multi() const { return at + 4 * singles; }
     const uint32_t* chunk_base() const { return at + 4 * n; }
     const uint32_t* chunks() const { return at + 4 * n + (n - singles); }
@@ -255,6 +258,7 @@ struct RotationAngles : PassTable {
     }
     bool same(LayerRuntime*, const RotationSpec& s, uint32_t h) const { return spec == s && half == h; }
     std::vector<uint32_t> build(const PassPlan&, const SequencePages&, uint32_t) override { return {}; }
+    std::vector<uint32_t> shape() const override { return {}; }
     void enqueue(const Rows& r) override {
         M40H_TRY(m40llm_ext_rotation_angles_async(rt_->ctx, r.pos, r.rows, static_cast<const double*>(freq_.ptr()), spec.dims / 2, half,
                                                   (float)spec.magnitude(), angles.ptr(), LayerRuntime::kStream));

@@ -52,6 +52,7 @@ public:
     ~LayeredDecoder() override {
         (void)m40llm_stream_synchronize(ctx_, kStream);
         drop_graph();
+        drop_steps();
     }
     LayeredDecoder(const LayeredDecoder&) = delete;
     LayeredDecoder& operator=(const LayeredDecoder&) = delete;
@@ -67,7 +68,12 @@ public:
         return spec_.positions ? std::min(pool, spec_.positions) : pool;
     }
     uint32_t max_sequences() const override { return opt_.max_sequences; }
-    void set_mode(uint32_t mode) override { mode_ = mode; drop_graph(); }
+    void set_mode(uint32_t mode) override {
+        (void)m40llm_stream_synchronize(ctx_, kStream);
+        mode_ = mode;
+        drop_graph();
+        drop_steps();
+    }
     void set_tie_guard(float g) override { tie_guard_ = g; }
     bool last_timed_host_fallback() const override { return timed_fallback_; }
 
@@ -372,14 +378,16 @@ private:
         for (uint32_t s = 0; s < opt_.max_sequences; ++s) std::copy(seqs_.pages(s).begin(), seqs_.pages(s).end(), t.begin() + (size_t)s * rt_.max_pages);
         return t;
     }
-    // Uploads a plan's tables and gives their device addresses.  Nothing of the stream is pending here: the pinned copy is free to be written.
-    Rows upload(const PassPlan& plan, DeviceBuf& buf, uint32_t longest, const uint32_t** want) {
+    // Lays a plan's tables out in pinned memory and gives their device addresses.  Nothing of the stream is pending here: the pinned copy is free to be
+    // written.  key: all that the pass's launches take from the plan besides the tables' contents.
+    struct Upload { void* to; size_t words; };
+    Rows lay_out(const PassPlan& plan, DeviceBuf& buf, uint32_t longest, const uint32_t** want, Upload& up, std::vector<uint32_t>* key = nullptr) {
         Rows r;
         r.rows = plan.rows();
         r.short_rows = plan.short_rows;
         for (const Portion& p : plan.portions) r.multi_row_portions += p.n > 1;
-        std::vector<uint32_t> all;
-        auto put = [&](const std::vector<uint32_t>& v) { const size_t at = all.size(); all.insert(all.end(), v.begin(), v.end()); return at; };
+        std::vector<uint32_t> all, places;
+        auto put = [&](const std::vector<uint32_t>& v) { const size_t at = all.size(); all.insert(all.end(), v.begin(), v.end()); places.push_back((uint32_t)at); return at; };
         const size_t tok = put(plan.tokens), prev = put(plan.prev), slot = put(plan.slot), pos = put(plan.pos), back = put(plan.back), w = put(plan.want),
                      table = put(page_table());
         std::vector<size_t> tables_at;
@@ -387,12 +395,21 @@ private:
         if (buf.bytes() < all.size() * 4) buf = DeviceBuf(ctx_, all.size() * 4 + all.size());
         if (tables_host_.bytes() < all.size() * 4) tables_host_ = PinnedBuf(ctx_, all.size() * 4 + all.size());
         std::copy(all.begin(), all.end(), tables_host_.u32());
-        M40H_TRY(m40llm_ext_copy_words_async(ctx_, buf.ptr(), tables_host_.u32(), all.size(), kStream));
+        up = {buf.ptr(), all.size()};
         r.tokens = buf.u32(tok); r.prev = buf.u32(prev); r.slot = buf.u32(slot); r.pos = buf.u32(pos); r.back = buf.u32(back); r.page_table = buf.u32(table);
         for (size_t i = 0; i < tables_at.size(); ++i) rt_.tables[i]->at = buf.u32(tables_at[i]);
         if (want) *want = buf.u32(w);
+        if (key) {
+            *key = {r.rows, r.short_rows, r.multi_row_portions, (uint32_t)plan.want.size(), (uint32_t)all.size()};
+            key->insert(key->end(), places.begin(), places.end());
+            for (auto& t : rt_.tables) {
+                const std::vector<uint32_t> shape = t->shape();
+                key->insert(key->end(), shape.begin(), shape.end());
+            }
+        }
         return r;
     }
+    void enqueue_upload(const Upload& up) { M40H_TRY(m40llm_ext_copy_words_async(ctx_, up.to, tables_host_.u32(), up.words, kStream)); }
 
     void enqueue_embedding(const Rows& r) {
         rt_.pending = 0;
@@ -430,20 +447,37 @@ private:
             if (!p.is_long) longest = std::max(longest, p.length);
         M40H_TRY(m40llm_stream_synchronize(ctx_, kStream));           // the tables of the pass before may still be read
         const uint32_t* want = nullptr;
-        Rows r = upload(plan, tables_, longest, &want);
+        Upload up;
+        std::vector<uint32_t> key;
+        Rows r = lay_out(plan, tables_, longest, &want, up, &key);
         r.in_place = (bool)on_layer;
         ensure_scratch(r);
-        enqueue_embedding(r);
-        for (size_t i = 0; i < layers_.size(); ++i) {
-            layers_[i]->enqueue(r);
-            if (on_layer) {
-                M40H_TRY(m40llm_stream_synchronize(ctx_, kStream));
-                on_layer((uint32_t)i, r.rows, rt_.x.f32());
+        // The rows of a step of single tokens come through pinned memory, which a kernel behind the head writes: a blocking copy begins when the
+        // host has seen the head's end, and takes 16 us a row and 66 us for eight of 32000 against 10 and 35 with the wait for the stream.
+        const auto pinned = [&](uint32_t n) { return !picks && (size_t)n * spec_.vocab * 4 <= logits_host_.bytes(); };
+        const auto first_logits = [&] {
+            const uint32_t n = (uint32_t)std::min<size_t>(logits_rows_, plan.want.size());
+            enqueue_logits(want, n, r.rows);
+            if (pinned(n)) M40H_TRY(m40llm_ext_copy_words_async(ctx_, logits_host_.f32(), logits_.ptr(), (size_t)n * spec_.vocab, kStream));
+        };
+        const auto layers = [&] {
+            enqueue_upload(up);
+            enqueue_embedding(r);
+            for (size_t i = 0; i < layers_.size(); ++i) {
+                layers_[i]->enqueue(r);
+                if (on_layer) {
+                    M40H_TRY(m40llm_stream_synchronize(ctx_, kStream));
+                    on_layer((uint32_t)i, r.rows, rt_.x.f32());
+                }
             }
-        }
+            if (!plan.want.empty()) first_logits();
+        };
+        key.push_back(picks ? 1u : 0u);
+        if (mode_ < 2 || on_layer || r.short_rows != r.rows || r.multi_row_portions) layers();
+        else enqueue_repeated(key, layers);
         for (size_t i = 0; i < plan.want.size(); i += logits_rows_) {
             const uint32_t n = (uint32_t)std::min<size_t>(logits_rows_, plan.want.size() - i);
-            enqueue_logits(want + i, n, r.rows);
+            if (i > 0) enqueue_logits(want + i, n, r.rows);
             std::vector<uint8_t> decided(n, 0);
             if (picks) {
                 M40H_TRY(m40llm_ext_top2_parts_async(ctx_, logits_.ptr(), n, spec_.vocab, pick_parts_.ptr(), kStream));
@@ -465,10 +499,6 @@ private:
                     picks->picks[out] = top.at;
                 }
             }
-            // The rows of a step of single tokens come through pinned memory, which a kernel behind the head writes: a blocking copy begins when the
-            // host has seen the head's end, and takes 16 us a row and 66 us for eight of 32000 against 10 and 35 with the wait for the stream.
-            const bool pinned = !picks && (size_t)n * spec_.vocab * 4 <= logits_host_.bytes();
-            if (pinned) M40H_TRY(m40llm_ext_copy_words_async(ctx_, logits_host_.f32(), logits_.ptr(), (size_t)n * spec_.vocab, kStream));
             // A result that nothing has written yet gets its pages now, while the device works, and not when its rows arrive
             for (uint32_t k = 0; !picks && k < n; ++k) {
                 volatile char* row = reinterpret_cast<volatile char*>(logits_out + plan.want_out[i + k] * spec_.vocab);
@@ -483,11 +513,48 @@ private:
                 uint32_t m = 1;
                 while (k + m < n && !decided[k + m] && plan.want_out[i + k + m] == plan.want_out[i + k] + m) ++m;
                 float* to = logits_out + plan.want_out[i + k] * spec_.vocab;
-                if (pinned) std::memcpy(to, logits_host_.f32((size_t)k * spec_.vocab), (size_t)m * spec_.vocab * 4);
+                if (i == 0 && pinned(n)) std::memcpy(to, logits_host_.f32((size_t)k * spec_.vocab), (size_t)m * spec_.vocab * 4);
                 else M40H_TRY(m40llm_memcpy_d2h(ctx_, to, logits_.f32((size_t)k * spec_.vocab), (size_t)m * spec_.vocab * 4));
                 k += m;
             }
         }
+    }
+
+    // The launches of a pass of single tokens: the next steps of the same sequences make the same ones, with other tables, until some sequence has
+    // grown past what a launch was split for.  From the third time on they are replayed from a graph: a launch of its own leaves about a
+    // microsecond to the next where a graph's nodes follow one another (45 of them: one sequence 320 -> 297 us a step, eight 415 -> 410), and the recording
+    // takes about 150 us.  The graphs of the latest kKeptSteps forms of step are kept, while no buffer has been replaced.
+    template <class F>
+    void enqueue_repeated(const std::vector<uint32_t>& key, const F& launches) {
+        auto it = std::find_if(steps_.begin(), steps_.end(), [&](const StepForm& f) { return f.key == key; });
+        if (it == steps_.end()) {
+            if (steps_.size() == kKeptSteps) {
+                drop(steps_.back());
+                steps_.pop_back();
+            }
+            steps_.insert(steps_.begin(), StepForm{key, nullptr, 0, 0});
+        } else {
+            std::rotate(steps_.begin(), it, it + 1);
+        }
+        StepForm& f = steps_.front();
+        if (f.graph && f.buffers != buffers_made()) {
+            drop(f);
+            f.seen = 0;
+        }
+        if (!f.graph && ++f.seen == kRecordAt) {
+            if (m40llm_cuda_graph_begin_capture(ctx_, kStream) == 0) {
+                try {
+                    launches();
+                } catch (...) {
+                    m40llm_cuda_graph_cancel_capture(ctx_, kStream);
+                    throw;
+                }
+                if (m40llm_cuda_graph_end_capture(ctx_, kStream, &f.graph) != 0) f.graph = nullptr;      // launched one by one from here on
+                f.buffers = buffers_made();
+            }
+        }
+        if (f.graph) M40H_TRY(m40llm_cuda_graph_launch(ctx_, f.graph, kStream));
+        else launches();
     }
 
     void run_items(const std::vector<SchedulerStepItem>& items, float* logits_out, const StepPicks* picks = nullptr) {
@@ -543,7 +610,9 @@ private:
         }
         M40H_TRY(m40llm_stream_synchronize(ctx_, kStream));
         drop_graph();
-        Rows r = upload(plan, loop_tables_, longest, nullptr);
+        Upload up;
+        Rows r = lay_out(plan, loop_tables_, longest, nullptr, up);
+        enqueue_upload(up);
         ensure_scratch(r);
         if (state_bytes_) {
             if (state_copy_.bytes() < state_bytes_ * rows) state_copy_ = DeviceBuf(ctx_, state_bytes_ * rows);
@@ -625,6 +694,20 @@ private:
         if (graph_) m40llm_cuda_graph_destroy(graph_);
         graph_ = nullptr;
     }
+    struct StepForm {
+        std::vector<uint32_t> key;
+        M40llmCudaGraphExec* graph;
+        uint32_t seen;
+        uint64_t buffers;             // buffers_made() when it was recorded
+    };
+    static void drop(StepForm& f) {
+        if (f.graph) m40llm_cuda_graph_destroy(f.graph);
+        f.graph = nullptr;
+    }
+    void drop_steps() {
+        for (StepForm& f : steps_) drop(f);
+        steps_.clear();
+    }
 
     M40llmCudaContext* ctx_;
     DecoderSpec spec_;
@@ -642,6 +725,9 @@ private:
     PinnedBuf tables_host_, logits_host_;
     DeviceBuf loop_tables_, loop_state_, loop_ids_, loop_gaps_, state_copy_;
     M40llmCudaGraphExec* graph_ = nullptr;
+    static constexpr size_t kKeptSteps = 8;
+    static constexpr uint32_t kRecordAt = 3;
+    std::vector<StepForm> steps_;                     // the latest first
 };
 
 // A folder with config.json and model.safetensors.

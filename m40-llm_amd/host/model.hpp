@@ -19,6 +19,7 @@
 #pragma once
 
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <cmath>
 #include <cstdint>
@@ -58,11 +59,17 @@ struct LayerWeights {   // device pointers; f16 GGUF layout [N cols][K]
         if (rc__ != 0) throw std::runtime_error(std::string(#expr) + " -> " + std::to_string(rc__)); \
     } while (0)
 
+// Buffers made so far, of all models: whoever keeps addresses of buffers can tell that none has been replaced since.
+inline std::atomic<uint64_t>& buffers_made() {
+    static std::atomic<uint64_t> n{0};
+    return n;
+}
 class DeviceBuf {
 public:
     DeviceBuf() = default;
     DeviceBuf(M40llmCudaContext* ctx, size_t bytes) : ctx_(ctx), bytes_(bytes) {
         if (m40llm_device_malloc(ctx, bytes ? bytes : 4, &p_) != 0) throw std::runtime_error("device_malloc failed");
+        ++buffers_made();
     }
     DeviceBuf(DeviceBuf&& o) noexcept : ctx_(o.ctx_), p_(o.p_), bytes_(o.bytes_) { o.p_ = nullptr; }
     DeviceBuf& operator=(DeviceBuf&& o) noexcept {
@@ -91,6 +98,7 @@ public:
     PinnedBuf() = default;
     PinnedBuf(M40llmCudaContext* ctx, size_t bytes) : ctx_(ctx), bytes_(bytes) {
         if (m40llm_ext_pinned_malloc(ctx, bytes, &p_) != 0) throw std::runtime_error("pinned_malloc failed");
+        ++buffers_made();
     }
     PinnedBuf(PinnedBuf&& o) noexcept : ctx_(o.ctx_), p_(o.p_), bytes_(o.bytes_) { o.p_ = nullptr; o.bytes_ = 0; }
     PinnedBuf& operator=(PinnedBuf&& o) noexcept {

@@ -25,6 +25,7 @@ struct PairTiles : PassTable {
     bool even = false;                    // long tiles see about equally many keys
     uint64_t floats_a_row = 0;            // of a split's partial sums, the largest layer's
     const uint32_t* long_tiles() const { return at + 2 * n_short; }
+    std::vector<uint32_t> shape() const override { return {n_short, n_long, long_queries, splits, even ? 1u : 0u}; }
     std::vector<uint32_t> build(const PassPlan& plan, const SequencePages&, uint32_t longest) override {
         std::vector<uint32_t> t;
         uint64_t blocks = 0;

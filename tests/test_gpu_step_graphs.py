@@ -1,0 +1,62 @@
+"""Steps of single tokens that a layered decoder replays from a graph: every step's logits are the bits of the launches one by one, with prompts, other
+forms of step, released sequences and replaced buffers in between."""
+import importlib
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+from gpu_common import m40  # noqa: E402
+
+layered = importlib.import_module("m40-llm_amd.layered")
+bench = importlib.import_module("m40-llm_amd.layered_bench")
+
+
+def config(design):
+    s = dict(bench.SHAPES["2k"], layers=4)
+    cfg = bench.pimosun_config(s) if design == "pimosun" else getattr(bench, design + "_config")("2k")
+    cfg["layers"] = cfg["layers"][:4]
+    return dict(cfg, vocab=1000)
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    yield m40.Context(0)
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
+@pytest.mark.parametrize("design", ["pimosun", "gulidra", "natatar", "fomunex"])
+def test_replayed_steps_equal_launched_steps(ctx, design, dtype):
+    models = [layered.LayeredModel.random(ctx, config(design), seed=3, std=0.05, dtype=dtype, max_tokens=2048, max_sequences=4, max_rows=256) for _ in range(2)]
+    models[1].set_mode(0)
+    rng = np.random.default_rng(1)
+
+    def step(entries):
+        entries = [(s, rng.integers(0, 1000, n), want) for s, n, want in entries]
+        a, b = (m.step(entries) for m in models)
+        assert a.shape == b.shape and np.array_equal(a.view(np.uint32), b.view(np.uint32)), (design, entries)
+        assert np.isfinite(a).all()
+
+    def singles(n, seqs, want=lambda s: [0]):
+        for _ in range(n):
+            step([(s, 1, want(s)) for s in seqs])
+    step([(0, 5, [4]), (1, 58, [0, 57]), (2, 130, [129])])
+    singles(12, (0, 1, 2))                                   # one sequence grows past its first page
+    singles(6, (2, 0), lambda s: [0] if s else [])           # another form, one place wanted
+    step([(3, 90, [89]), (0, 1, [0])])                       # a prompt beside a token: buffers may be made anew
+    singles(5, (0, 1, 2))
+    singles(5, (3, 1, 0, 2))
+    for m in models:
+        m.release(1)
+    singles(4, (0, 2, 3), lambda s: [])                      # no logits at all
+    step([(1, 1, [0])])
+    singles(5, (1, 0, 2))
+    models[0].set_mode(2)
+    singles(5, (1, 0, 2))
+    for n in range(10):                                      # more forms than are kept, and back to the first
+        singles(4, [(0, 1, 2, 3)[i] for i in range(4) if n + 1 >> i & 1])
+    singles(4, (1, 0, 2))
+    ids = [m.decode_batch_timed([0, 2], [m.length(0), m.length(2)], [5, 6], 2, 4)[0] for m in models]
+    assert np.array_equal(*ids)
+    singles(5, (0, 2))
