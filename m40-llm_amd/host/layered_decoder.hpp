@@ -381,7 +381,7 @@ private:
     // Lays a plan's tables out in pinned memory and gives their device addresses.  Nothing of the stream is pending here: the pinned copy is free to be
     // written.  key: all that the pass's launches take from the plan besides the tables' contents.
     struct Upload { void* to; size_t words; };
-    Rows lay_out(const PassPlan& plan, DeviceBuf& buf, uint32_t longest, const uint32_t** want, Upload& up, std::vector<uint32_t>* key = nullptr) {
+    Rows lay_out(const PassPlan& plan, DeviceBuf& buf, uint32_t longest, const uint32_t** want, Upload& up, std::vector<uint32_t>* key) {
         Rows r;
         r.rows = plan.rows();
         r.short_rows = plan.short_rows;
@@ -407,6 +407,18 @@ private:
                 key->insert(key->end(), shape.begin(), shape.end());
             }
         }
+        return r;
+    }
+    // The tables and the scratch of a pass.  Where that replaced a buffer (also if it then failed), the recorded steps, which hold addresses, go.
+    Rows provide(const PassPlan& plan, DeviceBuf& buf, uint32_t longest, const uint32_t** want, Upload& up, std::vector<uint32_t>* key = nullptr, bool in_place = false) {
+        struct Watch {
+            LayeredDecoder& d;
+            uint64_t made;
+            ~Watch() { if (buffers_made() != made) d.drop_steps(); }
+        } watch{*this, buffers_made()};
+        Rows r = lay_out(plan, buf, longest, want, up, key);
+        r.in_place = in_place;
+        ensure_scratch(r);
         return r;
     }
     void enqueue_upload(const Upload& up) { M40H_TRY(m40llm_ext_copy_words_async(ctx_, up.to, tables_host_.u32(), up.words, kStream)); }
@@ -449,9 +461,7 @@ private:
         const uint32_t* want = nullptr;
         Upload up;
         std::vector<uint32_t> key;
-        Rows r = lay_out(plan, tables_, longest, &want, up, &key);
-        r.in_place = (bool)on_layer;
-        ensure_scratch(r);
+        const Rows r = provide(plan, tables_, longest, &want, up, &key, (bool)on_layer);
         // The rows of a step of single tokens come through pinned memory, which a kernel behind the head writes: a blocking copy begins when the
         // host has seen the head's end, and takes 16 us a row and 66 us for eight of 32000 against 10 and 35 with the wait for the stream.
         const auto pinned = [&](uint32_t n) { return !picks && (size_t)n * spec_.vocab * 4 <= logits_host_.bytes(); };
@@ -523,7 +533,7 @@ private:
     // The launches of a pass of single tokens: the next steps of the same sequences make the same ones, with other tables, until some sequence has
     // grown past what a launch was split for.  From the third time on they are replayed from a graph: a launch of its own leaves about a
     // microsecond to the next where a graph's nodes follow one another (45 of them: one sequence 320 -> 297 us a step, eight 415 -> 410), and the recording
-    // takes about 150 us.  The graphs of the latest kKeptSteps forms of step are kept, while no buffer has been replaced.
+    // takes about 150 us.  The graphs of the latest kKeptSteps forms of step are kept, until a buffer of the model is replaced (drop_steps).
     template <class F>
     void enqueue_repeated(const std::vector<uint32_t>& key, const F& launches) {
         auto it = std::find_if(steps_.begin(), steps_.end(), [&](const StepForm& f) { return f.key == key; });
@@ -532,15 +542,11 @@ private:
                 drop(steps_.back());
                 steps_.pop_back();
             }
-            steps_.insert(steps_.begin(), StepForm{key, nullptr, 0, 0});
+            steps_.insert(steps_.begin(), StepForm{key, nullptr, 0});
         } else {
             std::rotate(steps_.begin(), it, it + 1);
         }
         StepForm& f = steps_.front();
-        if (f.graph && f.buffers != buffers_made()) {
-            drop(f);
-            f.seen = 0;
-        }
         if (!f.graph && ++f.seen == kRecordAt) {
             if (m40llm_cuda_graph_begin_capture(ctx_, kStream) == 0) {
                 try {
@@ -550,7 +556,6 @@ private:
                     throw;
                 }
                 if (m40llm_cuda_graph_end_capture(ctx_, kStream, &f.graph) != 0) f.graph = nullptr;      // launched one by one from here on
-                f.buffers = buffers_made();
             }
         }
         if (f.graph) M40H_TRY(m40llm_cuda_graph_launch(ctx_, f.graph, kStream));
@@ -611,9 +616,8 @@ private:
         M40H_TRY(m40llm_stream_synchronize(ctx_, kStream));
         drop_graph();
         Upload up;
-        Rows r = lay_out(plan, loop_tables_, longest, nullptr, up);
+        const Rows r = provide(plan, loop_tables_, longest, nullptr, up);
         enqueue_upload(up);
-        ensure_scratch(r);
         if (state_bytes_) {
             if (state_copy_.bytes() < state_bytes_ * rows) state_copy_ = DeviceBuf(ctx_, state_bytes_ * rows);
             copy_states(seq_ids, rows, false);
@@ -698,7 +702,6 @@ private:
         std::vector<uint32_t> key;
         M40llmCudaGraphExec* graph;
         uint32_t seen;
-        uint64_t buffers;             // buffers_made() when it was recorded
     };
     static void drop(StepForm& f) {
         if (f.graph) m40llm_cuda_graph_destroy(f.graph);

@@ -19,7 +19,6 @@
 #pragma once
 
 #include <algorithm>
-#include <atomic>
 #include <chrono>
 #include <cmath>
 #include <cstdint>
@@ -59,9 +58,9 @@ struct LayerWeights {   // device pointers; f16 GGUF layout [N cols][K]
         if (rc__ != 0) throw std::runtime_error(std::string(#expr) + " -> " + std::to_string(rc__)); \
     } while (0)
 
-// Buffers made so far, of all models: whoever keeps addresses of buffers can tell that none has been replaced since.
-inline std::atomic<uint64_t>& buffers_made() {
-    static std::atomic<uint64_t> n{0};
+// Buffers that this thread has made so far: whoever keeps addresses of buffers can tell that none was replaced in between.
+inline uint64_t& buffers_made() {
+    thread_local uint64_t n = 0;
     return n;
 }
 class DeviceBuf {
