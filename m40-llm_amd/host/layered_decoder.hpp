@@ -483,7 +483,9 @@ private:
             if (!plan.want.empty()) first_logits();
         };
         key.push_back(picks ? 1u : 0u);
-        if (mode_ < 2 || on_layer || r.short_rows != r.rows || r.multi_row_portions) layers();
+        // A replay leaves the host's side of the layers (the planes that the head is still to add, the streams' last sublayer) as the pass before had
+        // it, so a pass whose head takes more than one launch of its kernels is launched.
+        if (mode_ < 2 || on_layer || r.short_rows != r.rows || r.multi_row_portions || plan.want.size() > logits_rows_) layers();
         else enqueue_repeated(key, layers);
         for (size_t i = 0; i < plan.want.size(); i += logits_rows_) {
             const uint32_t n = (uint32_t)std::min<size_t>(logits_rows_, plan.want.size() - i);

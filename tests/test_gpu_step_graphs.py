@@ -60,3 +60,23 @@ def test_replayed_steps_equal_launched_steps(ctx, design, dtype):
     ids = [m.decode_batch_timed([0, 2], [m.length(0), m.length(2)], [5, 6], 2, 4)[0] for m in models]
     assert np.array_equal(*ids)
     singles(5, (0, 2))
+
+
+@pytest.mark.parametrize("design", ["pimosun", "gulidra", "natatar", "fomunex"])
+def test_more_logits_than_one_head_takes(ctx, design):
+    """Single tokens whose places are wanted 300 times (the head takes 256 rows at once), with a prompt of another row count in between."""
+    models = [layered.LayeredModel.random(ctx, config(design), seed=3, std=0.05, max_tokens=2048, max_sequences=4, max_rows=256) for _ in range(2)]
+    models[1].set_mode(0)
+    rng = np.random.default_rng(2)
+
+    def step(entries):
+        entries = [(s, rng.integers(0, 1000, n), want) for s, n, want in entries]
+        a, b = (m.step(entries) for m in models)
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32)), (design, entries)
+    step([(1, 70, [69])])
+    for _ in range(5):
+        step([(0, 1, [0] * 300)])
+    step([(2, 70, [69])])
+    for _ in range(2):
+        step([(0, 1, [0] * 300), (1, 1, [0])])
+        step([(0, 1, [0] * 300)])

@@ -1,0 +1,50 @@
+"""What a layered decoder's steps ask of the device, with the device calls stubbed (tests/layered_steps_check.cpp): launches, recordings and replays."""
+import json
+import os
+import subprocess
+
+import pytest
+
+import fomunex_common
+import gulidra_common
+import natatar_common
+import pimosun_common
+from pimosun_common import layer, mixer
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+# Pimosun so wide that products of one row and of 70 are cut into different numbers of parts
+WIDE = dict(pimosun_common.config_even(), width=2048, layers=[layer(mixer(4, 64, 32, 64, 256, 128), 4096)])
+DESIGNS = dict(pimosun=WIDE, gulidra=gulidra_common.config_even(), natatar=natatar_common.config_wide(),     # these two end with a mixer, whose product the head adds
+               fomunex=fomunex_common.config_wide())
+
+
+@pytest.fixture(scope="module")
+def run(tmp_path_factory):
+    at = tmp_path_factory.mktemp("steps")
+    exe = str(at / "check")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-Wall", "-I", os.path.join(HERE, "..", "include"), os.path.join(HERE, "layered_steps_check.cpp"), "-o", exe, "-lpthread"],
+                   check=True)
+
+    def call(design, mode, steps, max_sequences=4, max_rows=256):
+        """steps: lists of (sequence, tokens, copies of the last place wanted)"""
+        path = at / (design + ".json")
+        path.write_text(json.dumps(DESIGNS[design]))
+        words = ["steps", path, mode, max_sequences, max_rows]
+        for s in steps:
+            words += ["s", len(s), *(w for e in s for w in e)]
+        out = subprocess.run([exe], input=" ".join(str(w) for w in words) + "\n", capture_output=True, text=True, check=True, timeout=60).stdout
+        got = json.loads(out)
+        assert "error" not in got, got
+        return got
+    return call
+
+
+@pytest.mark.parametrize("design", list(DESIGNS))
+@pytest.mark.parametrize("singles", [[(0, 1, 300)], [(i, 1, 1) for i in range(300)]], ids=["places wanted more than once", "many sequences"])
+def test_more_logits_than_one_head_takes(run, design, singles):
+    """The head of rows past the first 256 reads the planes and streams of its own pass, whatever ran before."""
+    steps = [[(300, 70, 1)]] + [singles] * 5 + [[(301, 70, 1)]] + [singles] * 2      # a prompt first, so that the second one replaces no buffer
+    want, got = (run(design, mode, steps, 302, 320)["steps"] for mode in (0, 2))
+    for w, g in zip(want, got):
+        assert g["head"] == w["head"][-len(g["head"]):]
