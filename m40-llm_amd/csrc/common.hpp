@@ -51,6 +51,7 @@ struct M40llmCudaContext {
     float4* rope_cs;
     uint32_t* host_staging;        // pinned, kM40HostStagingWords words: device metadata read back for validation
     struct { float base; uint32_t head_dim; uint32_t ready; } rope_slots[2][4];
+    M40llmCudaContext* recorder_of;    // the context whose scratch, tables and staging these are, or null: this context's own
 };
 constexpr int kM40HostStagingWords = 2048;
 constexpr int kM40PrefillSeqs = 64;       // sequences of a packed prefill's by-value tables

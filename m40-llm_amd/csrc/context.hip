@@ -148,16 +148,35 @@ void m40llm_destroy_context(M40llmCudaContext* ctx) {
     (void)hipSetDevice(ctx->device_id);
     if (ctx->decode_stream) (void)hipStreamSynchronize(ctx->decode_stream);
     if (ctx->prefill_stream) (void)hipStreamSynchronize(ctx->prefill_stream);
-    free_scratch(ctx->scratch[0]);
-    free_scratch(ctx->scratch[1]);
-    if (ctx->rope_tables) (void)hipFree(ctx->rope_tables);
-    if (ctx->rope_cs) (void)hipFree(ctx->rope_cs);
-    if (ctx->host_staging) (void)hipHostFree(ctx->host_staging);
+    if (!ctx->recorder_of) {
+        free_scratch(ctx->scratch[0]);
+        free_scratch(ctx->scratch[1]);
+        if (ctx->rope_tables) (void)hipFree(ctx->rope_tables);
+        if (ctx->rope_cs) (void)hipFree(ctx->rope_cs);
+        if (ctx->host_staging) (void)hipHostFree(ctx->host_staging);
+    }
     if (ctx->prefill_waits_decode_event) (void)hipEventDestroy(ctx->prefill_waits_decode_event);
     if (ctx->decode_waits_prefill_event) (void)hipEventDestroy(ctx->decode_waits_prefill_event);
     if (ctx->prefill_stream) (void)hipStreamDestroy(ctx->prefill_stream);
     if (ctx->decode_stream) (void)hipStreamDestroy(ctx->decode_stream);
     delete ctx;
+}
+
+M40llmCudaContext* m40llm_ext_create_recorder(M40llmCudaContext* ctx) {
+    if (!ctx || ctx->recorder_of || m40_ensure_device(ctx) != 0) return nullptr;
+    M40llmCudaContext* rec = new (std::nothrow) M40llmCudaContext(*ctx);
+    if (!rec) return nullptr;
+    rec->recorder_of = ctx;
+    rec->prefill_stream = rec->decode_stream = nullptr;
+    rec->prefill_waits_decode_event = rec->decode_waits_prefill_event = nullptr;
+    if (hipStreamCreateWithFlags(&rec->prefill_stream, hipStreamNonBlocking) != hipSuccess || hipStreamCreateWithFlags(&rec->decode_stream, hipStreamNonBlocking) != hipSuccess ||
+        hipEventCreateWithFlags(&rec->prefill_waits_decode_event, hipEventDisableTiming) != hipSuccess ||
+        hipEventCreateWithFlags(&rec->decode_waits_prefill_event, hipEventDisableTiming) != hipSuccess) {
+        (void)hipGetLastError();
+        m40llm_destroy_context(rec);
+        return nullptr;
+    }
+    return rec;
 }
 
 int m40llm_current_device_props(char* name_buf, size_t buf_len, int* major, int* minor, int* device_id) {
@@ -446,6 +465,11 @@ int m40llm_cuda_graph_begin_capture(M40llmCudaContext* ctx, uint32_t stream_kind
     if (m40_ensure_device(ctx) != 0) return -2;
     hipStream_t stream = m40_select_stream(ctx, stream_kind);
     if (!stream) return -3;
+    if (const M40llmCudaContext* of = ctx->recorder_of) {      // buffers that grow on demand may have been replaced
+        ctx->scratch[0] = of->scratch[0];
+        ctx->scratch[1] = of->scratch[1];
+        std::memcpy(ctx->rope_slots, of->rope_slots, sizeof(ctx->rope_slots));
+    }
     return hipStreamBeginCapture(stream, hipStreamCaptureModeRelaxed) == hipSuccess ? 0 : -4;
 }
 

@@ -105,7 +105,7 @@ public:
         : ctx(c), spec(s), opt(o), es(o.act_dtype == M40LLM_ACT_F32 ? 4u : 2u), max_pages(pages), d_pad(round_up(s.width, 32)),
           rows_pad(round_up(std::max(o.max_rows, o.max_sequences), 64)) {}
 
-    M40llmCudaContext* ctx;
+    M40llmCudaContext* ctx;            // that launches go to
     const DecoderSpec& spec;
     LayeredOptions opt;
     uint32_t es, max_pages, d_pad, rows_pad;

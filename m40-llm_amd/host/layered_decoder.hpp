@@ -53,6 +53,7 @@ public:
         (void)m40llm_stream_synchronize(ctx_, kStream);
         drop_graph();
         drop_steps();
+        if (recorder_) m40llm_destroy_context(recorder_);
     }
     LayeredDecoder(const LayeredDecoder&) = delete;
     LayeredDecoder& operator=(const LayeredDecoder&) = delete;
@@ -421,7 +422,7 @@ private:
         ensure_scratch(r);
         return r;
     }
-    void enqueue_upload(const Upload& up) { M40H_TRY(m40llm_ext_copy_words_async(ctx_, up.to, tables_host_.u32(), up.words, kStream)); }
+    void enqueue_upload(const Upload& up) { M40H_TRY(m40llm_ext_copy_words_async(rt_.ctx, up.to, tables_host_.u32(), up.words, kStream)); }
 
     void enqueue_embedding(const Rows& r) {
         rt_.pending = 0;
@@ -434,14 +435,14 @@ private:
         e.scale = spec_.embedding_scale;
         e.x = rt_.x.ptr();
         if (spec_.block == BlockKind::OutputNorm) { e.h = rt_.h.ptr(); e.ld_h = rt_.d_pad; }
-        M40H_TRY(m40llm_ext_embed_tokens_async(ctx_, &e, kStream));
+        M40H_TRY(m40llm_ext_embed_tokens_async(rt_.ctx, &e, kStream));
         if (streams_) streams_->begin();
         for (auto& t : rt_.tables) t->enqueue(r);
     }
     // final norm and head of n of a pass's rows (row_index NULL = all of them)
     void enqueue_logits(const uint32_t* row_index, uint32_t n, uint32_t rows) {
         if (streams_) streams_->last_sum(row_index, n);
-        M40H_TRY(m40llm_ext_norm_rows_async(ctx_, spec_.norm == NormKind::Rms ? M40LLM_NORM_RMS : M40LLM_NORM_LAYER, rt_.x.ptr(), rt_.planes.ptr(), rt_.pending,
+        M40H_TRY(m40llm_ext_norm_rows_async(rt_.ctx, spec_.norm == NormKind::Rms ? M40LLM_NORM_RMS : M40LLM_NORM_LAYER, rt_.x.ptr(), rt_.planes.ptr(), rt_.pending,
                                             (uint64_t)rows * spec_.width, final_norm_.ptr(), row_index, n, spec_.width, spec_.eps, hn_.ptr(), rt_.d_pad,
                                             opt_.act_dtype, kStream));
         M40llmPackedGemm g = rt_.product(hn_.ptr(), rt_.d_pad, head_, round_up(spec_.vocab, 16) / 16, rt_.d_pad / 32, n, M40LLM_PACKED_STORE);
@@ -468,7 +469,7 @@ private:
         const auto first_logits = [&] {
             const uint32_t n = (uint32_t)std::min<size_t>(logits_rows_, plan.want.size());
             enqueue_logits(want, n, r.rows);
-            if (pinned(n)) M40H_TRY(m40llm_ext_copy_words_async(ctx_, logits_host_.f32(), logits_.ptr(), (size_t)n * spec_.vocab, kStream));
+            if (pinned(n)) M40H_TRY(m40llm_ext_copy_words_async(rt_.ctx, logits_host_.f32(), logits_.ptr(), (size_t)n * spec_.vocab, kStream));
         };
         const auto layers = [&] {
             enqueue_upload(up);
@@ -532,6 +533,25 @@ private:
         }
     }
 
+    // A graph of launches, or null.  They are recorded on a stream of the model's own: the context's is shared with whoever else uses the context, and what
+    // another thread enqueues there meanwhile has to run now, and once.
+    template <class F>
+    M40llmCudaGraphExec* recorded(const F& launches) {
+        if (!recorder_ && !(recorder_ = m40llm_ext_create_recorder(ctx_))) return nullptr;
+        if (m40llm_cuda_graph_begin_capture(recorder_, kStream) != 0) return nullptr;
+        rt_.ctx = recorder_;
+        try {
+            launches();
+        } catch (...) {
+            rt_.ctx = ctx_;
+            m40llm_cuda_graph_cancel_capture(recorder_, kStream);
+            throw;
+        }
+        rt_.ctx = ctx_;
+        M40llmCudaGraphExec* graph = nullptr;
+        return m40llm_cuda_graph_end_capture(recorder_, kStream, &graph) == 0 ? graph : nullptr;
+    }
+
     // The launches of a pass of single tokens: the next steps of the same sequences make the same ones, with other tables, until some sequence has
     // grown past what a launch was split for.  From the third time on they are replayed from a graph: a launch of its own leaves about a
     // microsecond to the next where a graph's nodes follow one another (45 of them: one sequence 320 -> 297 us a step, eight 415 -> 410), and the recording
@@ -549,17 +569,7 @@ private:
             std::rotate(steps_.begin(), it, it + 1);
         }
         StepForm& f = steps_.front();
-        if (!f.graph && ++f.seen == kRecordAt) {
-            if (m40llm_cuda_graph_begin_capture(ctx_, kStream) == 0) {
-                try {
-                    launches();
-                } catch (...) {
-                    m40llm_cuda_graph_cancel_capture(ctx_, kStream);
-                    throw;
-                }
-                if (m40llm_cuda_graph_end_capture(ctx_, kStream, &f.graph) != 0) f.graph = nullptr;      // launched one by one from here on
-            }
-        }
+        if (!f.graph && ++f.seen == kRecordAt) f.graph = recorded(launches);      // none: launched one by one from here on
         if (f.graph) M40H_TRY(m40llm_cuda_graph_launch(ctx_, f.graph, kStream));
         else launches();
     }
@@ -631,23 +641,13 @@ private:
             enqueue_embedding(r);
             for (auto& l : layers_) l->enqueue(r);
             enqueue_logits(nullptr, rows, rows);
-            M40H_TRY(m40llm_ext_top2_parts_async(ctx_, logits_.ptr(), rows, spec_.vocab, pick_parts_.ptr(), kStream));
-            M40H_TRY(m40llm_ext_advance_rows_async(ctx_, pick_parts_.ptr(), rows, r.tokens, r.prev, r.pos, loop_state_.u32(), loop_ids_.u32(),
+            M40H_TRY(m40llm_ext_top2_parts_async(rt_.ctx, logits_.ptr(), rows, spec_.vocab, pick_parts_.ptr(), kStream));
+            M40H_TRY(m40llm_ext_advance_rows_async(rt_.ctx, pick_parts_.ptr(), rows, r.tokens, r.prev, r.pos, loop_state_.u32(), loop_ids_.u32(),
                                                    loop_gaps_.f32(), total, kStream));
         };
         auto run = [&](uint32_t n) {
             if (mode_ >= 2 && n > 0) {
-                if (!graph_) {
-                    M40H_TRY(m40llm_stream_synchronize(ctx_, kStream));
-                    M40H_TRY(m40llm_cuda_graph_begin_capture(ctx_, kStream));
-                    try {
-                        enqueue();
-                    } catch (...) {
-                        m40llm_cuda_graph_cancel_capture(ctx_, kStream);
-                        throw;
-                    }
-                    M40H_TRY(m40llm_cuda_graph_end_capture(ctx_, kStream, &graph_));
-                }
+                if (!graph_ && !(graph_ = recorded(enqueue))) throw std::runtime_error("a step could not be recorded");
                 for (uint32_t i = 0; i < n; ++i) M40H_TRY(m40llm_cuda_graph_launch(ctx_, graph_, kStream));
             } else {
                 for (uint32_t i = 0; i < n; ++i) enqueue();
@@ -715,6 +715,7 @@ private:
     }
 
     M40llmCudaContext* ctx_;
+    M40llmCudaContext* recorder_ = nullptr;           // made for the first recording
     DecoderSpec spec_;
     LayeredOptions opt_;
     SequencePages seqs_;

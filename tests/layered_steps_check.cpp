@@ -63,6 +63,9 @@ int m40llm_ext_stream_update_async(M40llmCudaContext* ctx, const M40llmStreamUpd
                              ", experts " + std::to_string(u->expert_out != nullptr) + ", fresh " + std::to_string(u->x0 != nullptr) + ", rows " + std::to_string(u->rows));
     return 0;
 }
+static char recorder;
+M40llmCudaContext* m40llm_ext_create_recorder(M40llmCudaContext* ctx) { return ctx == world.own ? reinterpret_cast<M40llmCudaContext*>(&recorder) : nullptr; }
+void m40llm_destroy_context(M40llmCudaContext*) {}
 int m40llm_cuda_graph_begin_capture(M40llmCudaContext* ctx, uint32_t) {
     if (ctx == world.own) world.captured_shared = true;
     world.capturing = ctx;

@@ -1,5 +1,6 @@
 """Steps of single tokens that a layered decoder replays from a graph: every step's logits are the bits of the launches one by one, with prompts, other
 forms of step, released sequences and replaced buffers in between."""
+import ctypes as C
 import importlib
 
 import numpy as np
@@ -80,3 +81,31 @@ def test_more_logits_than_one_head_takes(ctx, design):
     for _ in range(2):
         step([(0, 1, [0] * 300), (1, 1, [0])])
         step([(0, 1, [0] * 300)])
+
+
+def test_a_recording_leaves_the_contexts_stream_alone(ctx):
+    """Between a recorder's begin and end the context's stream runs what it is given; the graph holds what the recorder was given, replay after replay."""
+    lib = ctx.lib
+    rec = C.c_void_p(lib.m40llm_ext_create_recorder(ctx.h))
+    assert rec.value and not lib.m40llm_ext_create_recorder(rec) and not lib.m40llm_ext_create_recorder(None)
+    src, mine, theirs = ctx.to_device(np.arange(64, dtype=np.uint32)), ctx.to_device(np.zeros(64, np.uint32)), ctx.to_device(np.zeros(64, np.uint32))
+    for _ in range(2):                                       # a recorder records more than once
+        m40.check(lib.m40llm_cuda_graph_begin_capture(rec, 1), "begin")
+        m40.check(lib.m40llm_ext_copy_words_async(rec, mine.ptr, src.ptr, 64, 1), "recorded")
+        m40.check(lib.m40llm_ext_copy_words_async(ctx.h, theirs.ptr, src.ptr, 64, 1), "launched")
+        ctx.sync(1)
+        graph = C.c_void_p()
+        m40.check(lib.m40llm_cuda_graph_end_capture(rec, 1, C.byref(graph)), "end")
+        assert np.array_equal(theirs.download(np.uint32, (64,)), np.arange(64)) and not mine.download(np.uint32, (64,)).any()
+        for _ in range(3):
+            m40.check(lib.m40llm_ext_clear_u32_async(ctx.h, mine.ptr, 64, 1), "clear")
+            m40.check(lib.m40llm_ext_clear_u32_async(ctx.h, theirs.ptr, 64, 1), "clear")
+            m40.check(lib.m40llm_cuda_graph_launch(ctx.h, graph, 1), "replay")
+            ctx.sync(1)
+            assert np.array_equal(mine.download(np.uint32, (64,)), np.arange(64)) and not theirs.download(np.uint32, (64,)).any()
+        m40.check(lib.m40llm_ext_clear_u32_async(ctx.h, mine.ptr, 64, 1), "clear")
+        ctx.sync(1)
+        lib.m40llm_cuda_graph_destroy(graph)
+    lib.m40llm_destroy_context(rec)
+    m40.check(lib.m40llm_ext_copy_words_async(ctx.h, theirs.ptr, src.ptr, 64, 1), "after the recorder is gone")
+    ctx.sync(1)

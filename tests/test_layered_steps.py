@@ -48,3 +48,13 @@ def test_more_logits_than_one_head_takes(run, design, singles):
     want, got = (run(design, mode, steps, 302, 320)["steps"] for mode in (0, 2))
     for w, g in zip(want, got):
         assert g["head"] == w["head"][-len(g["head"]):]
+
+
+@pytest.mark.parametrize("design", list(DESIGNS))
+def test_steps_are_recorded_beside_the_contexts_stream(run, design):
+    """What another thread enqueues on the context's stream while a step is recorded has to run, so nothing of a recording goes there."""
+    got = run(design, 2, [[(0, 1, 1), (1, 1, 1)]] * 6)
+    assert not got["captured_shared"]
+    assert sum(s["recordings"] for s in got["steps"]) == 1 and sum(s["replays"] for s in got["steps"]) >= 3
+    for s in got["steps"]:
+        assert ("BRE" in s["order"]) == (s["recordings"] == 1) and s["order"].count("R") == s["recordings"], s["order"]
