@@ -553,12 +553,21 @@ private:
     }
 
     // The launches of a pass of single tokens: the next steps of the same sequences make the same ones, with other tables, until some sequence has
-    // grown past what a launch was split for.  From the third time on they are replayed from a graph: a launch of its own leaves about a
-    // microsecond to the next where a graph's nodes follow one another (45 of them: one sequence 320 -> 297 us a step, eight 415 -> 410), and the recording
-    // takes about 150 us.  The graphs of the latest kKeptSteps forms of step are kept, until a buffer of the model is replaced (drop_steps).
+    // grown past what a launch was split for.  Behind its third time such a pass is recorded, and from the fourth on replayed from the graph: a launch of its
+    // own leaves about a microsecond to the next where a graph's nodes follow one another (2048 wide, eight layers: one sequence 482-552 -> 440-520 us a step,
+    // eight 550-1090 -> 513-1055).  The recording takes the host 300 to 400 us with the device idle (third step 550 -> 970), so it is made while the device
+    // runs the launched step (third and fourth step together 20 to 50 us more than launched ones): two replays pay for it.  The graphs of the latest
+    // kKeptSteps forms of step are kept, until a buffer of the model is replaced (drop_steps).
     template <class F>
     void enqueue_repeated(const std::vector<uint32_t>& key, const F& launches) {
-        auto it = std::find_if(steps_.begin(), steps_.end(), [&](const StepForm& f) { return f.key == key; });
+        const auto it = std::find_if(steps_.begin(), steps_.end(), [&](const StepForm& f) { return f.key == key; });
+        if (it != steps_.end() && it->graph) {
+            std::rotate(steps_.begin(), it, it + 1);
+            M40H_TRY(m40llm_cuda_graph_launch(ctx_, steps_.front().graph, kStream));
+            return;
+        }
+        launches();
+        // what follows is the host's alone, while the device runs the step
         if (it == steps_.end()) {
             if (steps_.size() == kKeptSteps) {
                 drop(steps_.back());
@@ -569,9 +578,7 @@ private:
             std::rotate(steps_.begin(), it, it + 1);
         }
         StepForm& f = steps_.front();
-        if (!f.graph && ++f.seen == kRecordAt) f.graph = recorded(launches);      // none: launched one by one from here on
-        if (f.graph) M40H_TRY(m40llm_cuda_graph_launch(ctx_, f.graph, kStream));
-        else launches();
+        if (++f.seen == kRecordAt) f.graph = recorded(launches);      // none: launched one by one from here on
     }
 
     void run_items(const std::vector<SchedulerStepItem>& items, float* logits_out, const StepPicks* picks = nullptr) {

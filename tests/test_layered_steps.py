@@ -58,3 +58,10 @@ def test_steps_are_recorded_beside_the_contexts_stream(run, design):
     assert sum(s["recordings"] for s in got["steps"]) == 1 and sum(s["replays"] for s in got["steps"]) >= 3
     for s in got["steps"]:
         assert ("BRE" in s["order"]) == (s["recordings"] == 1) and s["order"].count("R") == s["recordings"], s["order"]
+
+
+@pytest.mark.parametrize("design", list(DESIGNS))
+def test_a_step_is_recorded_behind_its_launches(run, design):
+    """The step that is recorded runs from its own launches, which come first, so that nothing waits for the recording; the next one is the first replay."""
+    orders = [s["order"] for s in run(design, 2, [[(0, 1, 1)]] * 6)["steps"]]
+    assert orders == ["L", "L", "LBRE", "G", "G", "G"]
