@@ -578,7 +578,10 @@ private:
             std::rotate(steps_.begin(), it, it + 1);
         }
         StepForm& f = steps_.front();
-        if (++f.seen == kRecordAt) f.graph = recorded(launches);      // none: launched one by one from here on
+        if (++f.seen != kRecordAt) return;
+        try {
+            f.graph = recorded(launches);
+        } catch (const std::exception&) {}                // the step itself is launched; so are the next ones
     }
 
     void run_items(const std::vector<SchedulerStepItem>& items, float* logits_out, const StepPicks* picks = nullptr) {

@@ -1,6 +1,6 @@
 // Driver for test_layered_steps.py: a layered decoder whose device calls are stubs, so that what a step asks of the device can be looked at without one.
 // One command a line on standard input, one JSON line out:
-//     steps <config.json> <mode> <max sequences> <max rows>  then per step  s <entries>  and per entry  <sequence> <tokens> <copies of the last place wanted>
+//     steps <config.json> <mode> <max sequences> <max rows>  then per step  s <entries>  and per entry  <sequence> <tokens> <copies of the last place wanted>;  f  recordings fail from here on
 #include <iostream>
 #include <sstream>
 
@@ -17,7 +17,7 @@ struct World {
     int launched = 0, recorded = 0, replays = 0, recordings = 0, destroyed = 0;
     bool captured_shared = false, fail_recording = false;
     std::vector<std::string> head;         // what the head's norms and the last sums of the streams were given, launches only
-    std::string order;                     // L a launch, R a recorded one, G a replay, B / E a recording's begin and end
+    std::string order;                     // L a launch, R a recorded one, G a replay, B / E a recording's begin and end, X given up
     bool call(const void* ctx) {           // whether it is a launch
         const bool records = ctx == capturing;
         ++(records ? recorded : launched);
@@ -30,7 +30,7 @@ World world;
 }  // namespace
 
 #define STUB(name, result) extern "C" long long stub_##name(const void* ctx) asm(#name); long long stub_##name(const void* ctx) { (void)ctx; return result; }
-#define LAUNCH(name) STUB(name, (world.call(ctx), 0))
+#define LAUNCH(name) STUB(name, (!world.call(ctx) && world.fail_recording ? -1 : 0))
 LAUNCH(m40llm_ext_advance_rows_async) LAUNCH(m40llm_ext_channel_delta_async) LAUNCH(m40llm_ext_clear_u32_async) LAUNCH(m40llm_ext_conv_state_async)
 LAUNCH(m40llm_ext_copy_words_async) LAUNCH(m40llm_ext_delta_split_async) LAUNCH(m40llm_ext_embed_tokens_async) LAUNCH(m40llm_ext_gate_group_norm_rows_async)
 LAUNCH(m40llm_ext_gather_rows_async) LAUNCH(m40llm_ext_head_attention_async) LAUNCH(m40llm_ext_latent_attention_async) LAUNCH(m40llm_ext_latent_split_append_async)
@@ -77,11 +77,10 @@ int m40llm_cuda_graph_end_capture(M40llmCudaContext* ctx, uint32_t, M40llmCudaGr
     if (ctx != world.capturing) return -1;
     world.capturing = nullptr;
     world.order += 'E';
-    if (world.fail_recording) return -4;
     *out = reinterpret_cast<M40llmCudaGraphExec*>(new char);
     return 0;
 }
-int m40llm_cuda_graph_cancel_capture(M40llmCudaContext*, uint32_t) { world.capturing = nullptr; return 0; }
+int m40llm_cuda_graph_cancel_capture(M40llmCudaContext*, uint32_t) { world.capturing = nullptr; world.order += 'X'; return 0; }
 int m40llm_cuda_graph_launch(M40llmCudaContext* ctx, M40llmCudaGraphExec*, uint32_t) {
     if (ctx != world.own || world.capturing) return -1;
     world.order += 'G';
@@ -109,6 +108,10 @@ static void steps(std::istream& in) {
         d.set_mode(mode);
         bool first = true;
         while (in >> op) {
+            if (op == "f") {
+                world.fail_recording = true;
+                continue;
+            }
             uint32_t n;
             in >> n;
             std::vector<std::vector<uint32_t>> tokens(n), want(n);

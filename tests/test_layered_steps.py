@@ -27,12 +27,12 @@ def run(tmp_path_factory):
                    check=True)
 
     def call(design, mode, steps, max_sequences=4, max_rows=256):
-        """steps: lists of (sequence, tokens, copies of the last place wanted)"""
+        """steps: lists of (sequence, tokens, copies of the last place wanted), or "f": recordings fail from there on"""
         path = at / (design + ".json")
         path.write_text(json.dumps(DESIGNS[design]))
         words = ["steps", path, mode, max_sequences, max_rows]
         for s in steps:
-            words += ["s", len(s), *(w for e in s for w in e)]
+            words += [s] if s == "f" else ["s", len(s), *(w for e in s for w in e)]
         out = subprocess.run([exe], input=" ".join(str(w) for w in words) + "\n", capture_output=True, text=True, check=True, timeout=60).stdout
         got = json.loads(out)
         assert "error" not in got, got
@@ -65,3 +65,9 @@ def test_a_step_is_recorded_behind_its_launches(run, design):
     """The step that is recorded runs from its own launches, which come first, so that nothing waits for the recording; the next one is the first replay."""
     orders = [s["order"] for s in run(design, 2, [[(0, 1, 1)]] * 6)["steps"]]
     assert orders == ["L", "L", "LBRE", "G", "G", "G"]
+
+
+@pytest.mark.parametrize("design", list(DESIGNS))
+def test_a_step_whose_recording_fails_is_a_launched_one(run, design):
+    orders = [s["order"] for s in run(design, 2, ["f"] + [[(0, 1, 1)]] * 5)["steps"]]
+    assert orders == ["L", "L", "LBRX", "L", "L"]
