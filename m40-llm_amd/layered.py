@@ -4,6 +4,7 @@ from __future__ import annotations
 
 import ctypes as C
 import json
+from operator import index
 
 import numpy as np
 
@@ -66,18 +67,25 @@ class LayeredModel:
     def step(self, entries):
         # All tokens and all places in one array each: the device waits while the entries are made, and addresses of an array an entry take
         # three times as long (eight entries: 74 -> 27 us)
-        lists, places, seqs, n_tokens, wants = [], [], [], [], []
+        lists, want_lists, places, seqs, n_tokens, wants = [], [], [], [], [], []
         for seq, tokens, want in entries:
             t = np.ascontiguousarray(tokens, dtype=np.uint32)
             n = len(t)
             want = list(want)
-            lists.append(t if t.ndim == 1 else t.reshape(-1)[:n])
+            lists.append(t if t.ndim == 1 else t.reshape(-1)[:n])       # of several dimensions: as many elements as there are rows
+            want_lists.append(want)
             places += want
-            seqs.append(int(seq) & 0xffffffff)
+            seqs.append(index(seq) & 0xffffffff)
             n_tokens.append(n)
             wants.append(len(want))
         t = np.concatenate(lists) if lists else np.empty(0, dtype=np.uint32)
-        w = np.ascontiguousarray(places, dtype=np.uint32)
+        n_want = len(places)
+        try:
+            w = np.array(places, dtype=np.uint32)
+        except ValueError:     # rows of one entry beside numbers of another
+            w = np.empty(n_want + 1)
+        if w.shape != (n_want,):
+            w = np.concatenate([np.ascontiguousarray(want, dtype=np.uint32).reshape(-1)[:len(want)] for want in want_lists])
         at_t, at_w = t.__array_interface__["data"][0], w.__array_interface__["data"][0]
         rows = []
         for seq, n, m in zip(seqs, n_tokens, wants):
@@ -85,8 +93,8 @@ class LayeredModel:
             at_t += 4 * n
             at_w += 4 * m
         arr = np.array(rows, dtype=_ENTRY)
-        out = np.empty((len(places), self.vocab), dtype=np.float32)
-        self._ok(self.H.m40host_model_step(self.h, arr.ctypes.data, len(rows), out.ctypes.data if places else None), "m40host_model_step")
+        out = np.empty((n_want, self.vocab), dtype=np.float32)
+        self._ok(self.H.m40host_model_step(self.h, arr.ctypes.data, len(rows), out.ctypes.data if n_want else None), "m40host_model_step")
         return out
 
     def step_layers(self, seq, tokens, n_layers, width):
