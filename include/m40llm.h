@@ -394,8 +394,9 @@ int m40llm_ext_prefill_rope_append_on_stream_async(M40llmCudaContext* ctx, M40ll
                                                    const void* d_bq_f32, const void* d_bk_f32, const void* d_bv_f32,
                                                    uint32_t stream_kind);
 /* Rotation, cache append and attention of whole prompts (rows from position 0 on) without rotated rows in memory: Q, K and V as the projections
- * left them (nothing is written back), the rows' rotations from m40llm_ext_prefill_angles_async ([rows][head_dim / 2] (cos, sin), one call for
- * all layers), offsets and lengths on the device and on the host, the same values.  Out and cache are bit for bit what
+ * left them (nothing is written back), the rows' rotations from m40llm_ext_prefill_angles_async for the same lengths ([rows][head_dim / 2] (cos, sin), the
+ * sequences' rows one behind the other also where the offsets leave gaps; one call for all layers), offsets and lengths on the device and on the host, the same
+ * values.  Out and cache are bit for bit what
  * m40llm_ext_prefill_rope_append_on_stream_async and m40llm_ext_attention_prefill_f32_gqa_varlen_host_tables_async leave.  Prefill stream.  -1 null, -2
  * batch / slot / layout / biases, -4 alignment, -5 past max_seq_len, -6 not a dense cache, -8 a slot named twice, otherwise as the attention call. */
 int m40llm_ext_prefill_attention_rope_append_async(M40llmCudaContext* ctx, M40llmKVCache* kv, const void* q_dev_f32, const void* k_dev_f32,

@@ -90,12 +90,13 @@ struct PrefillArgs {
 // Prompts that go in unrotated: rows 0 .. of sequence b are its positions 0 ..; queries are rotated where they are loaded, keys where they are
 // packed, which also appends them to the dense cache.
 struct PrefillRope {
-    const float2* angles;       // [row of the packed batch][HD / 2] (cos, sin)
+    const float2* angles;       // [rows of the sequences one behind the other][HD / 2] (cos, sin)
     const float *bq, *bk, *bv;  // added before the rotation, or null
     uint32_t layout, max_seq_len;
     uint16_t *k_cache, *v_cache;
     uint32_t* seq_map;
     uint32_t slot[kM40PrefillSeqs];
+    uint32_t first[kM40PrefillSeqs];      // row of the angles of a sequence's first row; its rows may lie further on, the offsets may have gaps
 };
 struct NoRope {};
 
@@ -152,7 +153,7 @@ __global__ __launch_bounds__(kThreads) void prefill_pack_kv_kernel(PrefillArgs p
             // the four angles of a pair of quads, two by each
             if constexpr (kRope) {
                 const int off = (neox ? at[u & ~1] : at[u & ~1] / 2) % kHalf + 2 * (u % 2);
-                cs[u] = *reinterpret_cast<const float4*>(rope.angles + ((size_t)p.kv_offsets[b] + row) * kHalf + off);
+                cs[u] = *reinterpret_cast<const float4*>(rope.angles + ((size_t)rope.first[b] + row) * kHalf + off);
             }
             kx[u] = quad(Kb + (size_t)row * row_stride + d);
             vx[u] = quad(Vb + (size_t)row * row_stride + d);
@@ -295,7 +296,7 @@ __global__ __launch_bounds__(kThreads) void prefill_attn_kernel(PrefillArgs p, R
             // a lane holds both columns of its pairs: neighbours, or 32 s + 8 g + i and half a head further on
             constexpr int kHalf = HD / 2, HS = KS / 2;
             const bool neox = rope.layout == M40LLM_ROPE_LAYOUT_NEOX;
-            const float2* angles = rope.angles + ((size_t)p.q_offsets[b] + my_q) * kHalf + (neox ? 8 * g : 4 * g);
+            const float2* angles = rope.angles + ((size_t)rope.first[b] + my_q) * kHalf + (neox ? 8 * g : 4 * g);
             float4 cs[HS][4];
 #pragma unroll
             for (int s = 0; s < HS; ++s)
@@ -654,12 +655,15 @@ int m40llm_ext_prefill_attention_rope_append_async(M40llmCudaContext* ctx, M40ll
     if (batch == 0 || batch > (uint32_t)kM40PrefillSeqs || (n_bias != 0 && n_bias != 3) || rope_layout > M40LLM_ROPE_LAYOUT_NEOX) return -2;
     if (kv->compressed || !kv->d_k || !kv->d_v) return -6;
     PrefillRope r{};
+    uint32_t rows = 0;
     for (uint32_t i = 0; i < batch; ++i) {
         if (seq_slots_host[i] >= kv->max_batch_size) return -2;
         if (lens_host[i] > kv->max_seq_len) return -5;
         for (uint32_t j = 0; j < i; ++j)
             if (seq_slots_host[j] == seq_slots_host[i]) return -8;   // two sequences of one call would race on a slot
         r.slot[i] = seq_slots_host[i];
+        r.first[i] = rows;
+        rows += lens_host[i];              // at most 64 lengths, which the attention refuses above 8192
     }
     if (!m40_aligned16(d_angles)) return -4;
     r.angles = static_cast<const float2*>(d_angles);

@@ -121,6 +121,39 @@ def test_prefill_attention_with_rotation_and_append_inside(dev, layout, bias, hd
     assert np.array_equal(got[0][2], got[1][2])
 
 
+@pytest.mark.parametrize("layout,hd", [(0, 64), (1, 128)])
+def test_prefill_attention_with_rotation_where_offsets_leave_gaps(dev, layout, hd):
+    """Rows in front of, between and behind the sequences: the same output rows, cache and lengths as without them, from the same angles (whose buffer ends with
+    the last sequence's last row); the rows between keep what they held."""
+    lens, gaps, q_heads, kv_heads = [33, 1, 70], [5, 64, 17, 3], 4, 2
+    rng = np.random.default_rng(hd)
+    D, KV, n, rows = q_heads * hd, kv_heads * hd, len(lens), sum(lens)
+    qkv = [rng.standard_normal((rows, w)).astype(np.float32) for w in (D, KV, KV)]
+    h_lens, slots, first = u32(lens), u32([2, 0, 1]), np.concatenate([[0], np.cumsum(lens)[:-1]])
+    got = []
+    for gap in ([0] * (n + 1), gaps):
+        offs = u32(first + np.cumsum(gap)[:n])
+        at = np.concatenate([np.arange(o, o + l) for o, l in zip(offs, lens)])
+        total = rows + sum(gap)
+        spread = []
+        for a in qkv:
+            b = np.full((total, a.shape[1]), np.nan, np.float32)
+            b[at] = a
+            spread.append(dev.up(b))
+        kv = m40.KVCache(dev.ctx, 80, n, kv_heads, hd)
+        out, angles, d_offs, d_lens = dev.up(np.full((total, D), 7, np.float32)), dev.zeros(rows * hd // 2 * 8), dev.up(offs), dev.up(h_lens)
+        dev.call("m40llm_ext_prefill_angles_async", n, h_lens.ctypes.data, hd, 1e4, 1.0, angles.ptr, 0)
+        dev.call("m40llm_ext_prefill_attention_rope_append_async", kv.h, *(a.ptr for a in spread), d_offs.ptr, d_lens.ptr, n, slots.ctypes.data, offs.ctypes.data,
+                 h_lens.ctypes.data, q_heads, layout, angles.ptr, None, None, None, out.ptr)
+        dev.sync()
+        o = out.download(np.float32, (total, D))
+        assert np.isfinite(o).all() and (np.delete(o, at, axis=0) == 7).all()
+        got.append((o[at].view(np.uint32), [kv.read_token(int(s), t) for s, l in zip(slots, lens) for t in range(l)], kv.read_raw(5, np.uint32, n)))
+    assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][2], got[1][2])
+    for x, y in zip(got[0][1], got[1][1]):
+        assert np.array_equal(x[0], y[0]) and np.array_equal(x[1], y[1])
+
+
 def test_prefill_rope_append_argument_checks(dev):
     kv = m40.KVCache(dev.ctx, 8, 2, 2, 64)
     z = dev.zeros(16 * 4 * 64 * 4)
