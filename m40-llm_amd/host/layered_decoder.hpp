@@ -349,7 +349,8 @@ private:
         hn_ = rt_.cleared((size_t)round_up(logits_rows_, 16) * rt_.d_pad * rt_.es);
         logits_ = DeviceBuf(ctx_, (size_t)logits_rows_ * spec_.vocab * 4);
         pick_parts_ = DeviceBuf(ctx_, (size_t)logits_rows_ * M40LLM_TOP2_PARTS * 16);
-        if (const size_t bytes = (size_t)std::min(logits_rows_, opt_.max_sequences) * spec_.vocab * 4; bytes <= kMostPinned) logits_host_ = PinnedBuf(ctx_, bytes);
+        const size_t row = (size_t)spec_.vocab * 4;
+        if (const size_t n = std::min<size_t>(std::min(logits_rows_, opt_.max_sequences), kMostPinned / row); n > 0) logits_host_ = PinnedBuf(ctx_, n * row);
         for (const SlotState& s : rt_.states) state_bytes_ += s.slot_bytes;
         M40H_TRY(m40llm_stream_synchronize(ctx_, kStream));
     }

@@ -14,7 +14,7 @@ namespace {
 struct World {
     const void* own = nullptr;
     const void* capturing = nullptr;
-    int launched = 0, recorded = 0, replays = 0, recordings = 0, destroyed = 0;
+    int launched = 0, recorded = 0, replays = 0, recordings = 0, destroyed = 0, blocking_copies = 0;
     bool captured_shared = false, fail_recording = false;
     std::vector<std::string> head;         // what the head's norms and the last sums of the streams were given, launches only
     std::string order;                     // L a launch, R a recorded one, G a replay, B / E a recording's begin and end, X given up
@@ -51,7 +51,7 @@ int m40llm_device_free(M40llmCudaContext*, void* p) { std::free(p); return 0; }
 int m40llm_ext_pinned_malloc(M40llmCudaContext* ctx, size_t bytes, void** out) { return m40llm_device_malloc(ctx, bytes, out); }
 int m40llm_ext_pinned_free(M40llmCudaContext* ctx, void* p) { return m40llm_device_free(ctx, p); }
 int m40llm_memcpy_h2d(M40llmCudaContext*, void* dst, const void* src, size_t n) { std::memcpy(dst, src, n); return 0; }
-int m40llm_memcpy_d2h(M40llmCudaContext*, void* dst, const void* src, size_t n) { std::memcpy(dst, src, n); return 0; }
+int m40llm_memcpy_d2h(M40llmCudaContext*, void* dst, const void* src, size_t n) { std::memcpy(dst, src, n); ++world.blocking_copies; return 0; }
 int m40llm_ext_norm_rows_async(M40llmCudaContext* ctx, uint32_t, void*, const void*, uint32_t n_planes, uint64_t plane_stride, const void*, const uint32_t* index, uint32_t rows,
                                uint32_t, float, void*, uint32_t, uint32_t, uint32_t) {
     if (world.call(ctx) && index) world.head.push_back("norm " + std::to_string(n_planes) + " planes " + std::to_string(plane_stride) + " apart, rows " + std::to_string(rows));
@@ -131,7 +131,7 @@ static void steps(std::istream& in) {
             world.order.clear();
             d.step(entries, logits.data());
             log << (first ? "" : ", ") << "{\"replays\": " << world.replays - before.replays << ", \"recordings\": " << world.recordings - before.recordings
-                << ", \"destroyed\": " << world.destroyed - before.destroyed << ", \"order\": " << quoted(world.order) << ", \"head\": [";
+                << ", \"destroyed\": " << world.destroyed - before.destroyed << ", \"blocking_copies\": " << world.blocking_copies - before.blocking_copies << ", \"order\": " << quoted(world.order) << ", \"head\": [";
             for (size_t i = 0; i < world.head.size(); ++i) log << (i ? ", " : "") << quoted(world.head[i]);
             log << "]}";
             first = false;

@@ -17,6 +17,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 WIDE = dict(pimosun_common.config_even(), width=2048, layers=[layer(mixer(4, 64, 32, 64, 256, 128), 4096)])
 DESIGNS = dict(pimosun=WIDE, gulidra=gulidra_common.config_even(), natatar=natatar_common.config_wide(),     # these two end with a mixer, whose product the head adds
                fomunex=fomunex_common.config_wide())
+MANY_WORDS = dict(pimosun_common.config_one(), vocab=1 << 18)         # a row of logits is a megabyte
 
 
 @pytest.fixture(scope="module")
@@ -29,7 +30,7 @@ def run(tmp_path_factory):
     def call(design, mode, steps, max_sequences=4, max_rows=256):
         """steps: lists of (sequence, tokens, copies of the last place wanted), or "f": recordings fail from there on"""
         path = at / (design + ".json")
-        path.write_text(json.dumps(DESIGNS[design]))
+        path.write_text(json.dumps(MANY_WORDS if design == "many_words" else DESIGNS[design]))
         words = ["steps", path, mode, max_sequences, max_rows]
         for s in steps:
             words += [s] if s == "f" else ["s", len(s), *(w for e in s for w in e)]
@@ -71,3 +72,9 @@ def test_a_step_is_recorded_behind_its_launches(run, design):
 def test_a_step_whose_recording_fails_is_a_launched_one(run, design):
     orders = [s["order"] for s in run(design, 2, ["f"] + [[(0, 1, 1)]] * 5)["steps"]]
     assert orders == ["L", "L", "LBRX", "L", "L"]
+
+
+def test_rows_that_fit_come_through_pinned_memory(run):
+    """16 megabytes of logits have a place in host memory that kernels write, whatever rows all sequences together would take."""
+    steps = [[(i, 1, 1) for i in range(n)] for n in (1, 16, 17, 1)]
+    assert [s["blocking_copies"] for s in run("many_words", 2, steps, 40, 64)["steps"]] == [0, 0, 1, 0]
