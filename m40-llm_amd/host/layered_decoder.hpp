@@ -95,6 +95,7 @@ public:
             for (uint32_t i = 0; i < e.n_want; ++i)
                 if (e.want[i] >= e.n) throw std::out_of_range("a wanted place lies outside the entry's tokens");
             check_positions(e.sequence, e.n);
+            if (e.n_want && !logits_out && !picks) throw std::invalid_argument("no place for the logits");
         }
         for (const auto& e : entries) seqs_.grow(e.sequence, (uint64_t)seqs_.length(e.sequence) + e.n);
         // passes of at most max_rows rows; an entry's rows stay in order

@@ -1,6 +1,7 @@
 // Driver for test_layered_steps.py: a layered decoder whose device calls are stubs, so that what a step asks of the device can be looked at without one.
 // One command a line on standard input, one JSON line out:
-//     steps <config.json> <mode> <max sequences> <max rows>  then per step  s <entries>  and per entry  <sequence> <tokens> <copies of the last place wanted>;  f  recordings fail from here on
+//     steps <config.json> <mode> <max sequences> <max rows>  then per step  s <entries>  and per entry  <sequence> <tokens> <copies of the last place wanted>;  f  recordings fail from here on;  n  no
+//     place for logits is given from here on
 #include <iostream>
 #include <sstream>
 
@@ -51,7 +52,12 @@ int m40llm_device_free(M40llmCudaContext*, void* p) { std::free(p); return 0; }
 int m40llm_ext_pinned_malloc(M40llmCudaContext* ctx, size_t bytes, void** out) { return m40llm_device_malloc(ctx, bytes, out); }
 int m40llm_ext_pinned_free(M40llmCudaContext* ctx, void* p) { return m40llm_device_free(ctx, p); }
 int m40llm_memcpy_h2d(M40llmCudaContext*, void* dst, const void* src, size_t n) { std::memcpy(dst, src, n); return 0; }
-int m40llm_memcpy_d2h(M40llmCudaContext*, void* dst, const void* src, size_t n) { std::memcpy(dst, src, n); ++world.blocking_copies; return 0; }
+int m40llm_memcpy_d2h(M40llmCudaContext*, void* dst, const void* src, size_t n) {
+    if (!dst) return -1;
+    std::memcpy(dst, src, n);
+    ++world.blocking_copies;
+    return 0;
+}
 int m40llm_ext_norm_rows_async(M40llmCudaContext* ctx, uint32_t, void*, const void*, uint32_t n_planes, uint64_t plane_stride, const void*, const uint32_t* index, uint32_t rows,
                                uint32_t, float, void*, uint32_t, uint32_t, uint32_t) {
     if (world.call(ctx) && index) world.head.push_back("norm " + std::to_string(n_planes) + " planes " + std::to_string(plane_stride) + " apart, rows " + std::to_string(rows));
@@ -106,8 +112,12 @@ static void steps(std::istream& in) {
     {
         LayeredDecoder d(reinterpret_cast<M40llmCudaContext*>(&own), read_decoder_spec(read_text_file(path)), tensors, opt);
         d.set_mode(mode);
-        bool first = true;
+        bool first = true, place = true;
         while (in >> op) {
+            if (op == "n") {
+                place = false;
+                continue;
+            }
             if (op == "f") {
                 world.fail_recording = true;
                 continue;
@@ -129,7 +139,7 @@ static void steps(std::istream& in) {
             const World before = world;
             world.head.clear();
             world.order.clear();
-            d.step(entries, logits.data());
+            d.step(entries, place ? logits.data() : nullptr);
             log << (first ? "" : ", ") << "{\"replays\": " << world.replays - before.replays << ", \"recordings\": " << world.recordings - before.recordings
                 << ", \"destroyed\": " << world.destroyed - before.destroyed << ", \"blocking_copies\": " << world.blocking_copies - before.blocking_copies << ", \"order\": " << quoted(world.order) << ", \"head\": [";
             for (size_t i = 0; i < world.head.size(); ++i) log << (i ? ", " : "") << quoted(world.head[i]);

@@ -27,16 +27,16 @@ def run(tmp_path_factory):
     subprocess.run(["g++", "-O1", "-std=c++17", "-Wall", "-I", os.path.join(HERE, "..", "include"), os.path.join(HERE, "layered_steps_check.cpp"), "-o", exe, "-lpthread"],
                    check=True)
 
-    def call(design, mode, steps, max_sequences=4, max_rows=256):
-        """steps: lists of (sequence, tokens, copies of the last place wanted), or "f": recordings fail from there on"""
+    def call(design, mode, steps, max_sequences=4, max_rows=256, errors=False):
+        """steps: lists of (sequence, tokens, copies of the last place wanted), or a word of the driver"""
         path = at / (design + ".json")
         path.write_text(json.dumps(MANY_WORDS if design == "many_words" else DESIGNS[design]))
         words = ["steps", path, mode, max_sequences, max_rows]
         for s in steps:
-            words += [s] if s == "f" else ["s", len(s), *(w for e in s for w in e)]
+            words += [s] if isinstance(s, str) else ["s", len(s), *(w for e in s for w in e)]
         out = subprocess.run([exe], input=" ".join(str(w) for w in words) + "\n", capture_output=True, text=True, check=True, timeout=60).stdout
         got = json.loads(out)
-        assert "error" not in got, got
+        assert errors or "error" not in got, got
         return got
     return call
 
@@ -78,3 +78,9 @@ def test_rows_that_fit_come_through_pinned_memory(run):
     """16 megabytes of logits have a place in host memory that kernels write, whatever rows all sequences together would take."""
     steps = [[(i, 1, 1) for i in range(n)] for n in (1, 16, 17, 1)]
     assert [s["blocking_copies"] for s in run("many_words", 2, steps, 40, 64)["steps"]] == [0, 0, 1, 0]
+
+
+@pytest.mark.parametrize("mode", [0, 2])
+def test_logits_without_a_place_are_an_error(run, mode):
+    assert run("pimosun", mode, ["n", [(0, 3, 0)]])["steps"]
+    assert "place" in run("pimosun", mode, ["n", [(0, 3, 0)], [(0, 1, 0), (1, 1, 1)]], errors=True)["error"]
