@@ -200,6 +200,8 @@ int m40host_model_release(M40HostModel* model, uint32_t sequence_id);
 int m40host_model_assume_length(M40HostModel* model, uint32_t sequence_id, uint32_t tokens);
 uint32_t m40host_model_length(M40HostModel* model, uint32_t sequence_id);
 uint32_t m40host_model_free_pages(M40HostModel* model);
+/* diagnosis: passes replayed from a graph, graphs recorded, graphs dropped since the model was made */
+int m40host_model_step_counts(M40HostModel* model, uint32_t* replayed, uint32_t* recorded, uint32_t* dropped);
 
 /* ---- continuous-batching decode scheduler (src/server.rs:203-770 without HTTP, tokenizer and channels) ---------- */
 typedef struct M40HostScheduler M40HostScheduler;

@@ -592,6 +592,16 @@ uint32_t m40host_model_length(M40HostModel* m, uint32_t seq) {
 uint32_t m40host_model_free_pages(M40HostModel* m) {
     return guarded([&]() -> uint32_t { return m->layered().sequences().free_pages(); }, 0xffffffffu);
 }
+int m40host_model_step_counts(M40HostModel* m, uint32_t* replayed, uint32_t* recorded, uint32_t* dropped) {
+    return guarded(
+        [&]() -> int {
+            if (!m || !replayed || !recorded || !dropped) throw std::invalid_argument("null argument");
+            const StepCounts& c = m->layered().step_counts();
+            *replayed = c.replayed; *recorded = c.recorded; *dropped = c.dropped;
+            return 0;
+        },
+        -100);
+}
 
 // ---- continuous-batching decode scheduler -----------------------------------------------------------------
 M40HostScheduler* m40host_scheduler_create_for_model(M40HostModel* model, uint32_t sequence_slots) {

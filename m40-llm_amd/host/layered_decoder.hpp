@@ -29,6 +29,9 @@ struct StepEntry {
     uint32_t n_want;
 };
 
+// Passes of a decoder's life: how many were replayed from a graph, how many graphs were recorded, and how many were dropped again.
+struct StepCounts { uint32_t replayed = 0, recorded = 0, dropped = 0; };
+
 // Greedy picks of a step's wanted places, in the order of its logits rows: a row flagged greedy whose two best logits are no near
 // tie is decided on the device (picks, picked = 1), and its logits are not brought back.
 struct StepPicks {
@@ -61,6 +64,7 @@ public:
     const DecoderSpec& spec() const { return spec_; }
     const SequencePages& sequences() const { return seqs_; }
     M40llmCudaContext* ctx() const { return ctx_; }
+    const StepCounts& step_counts() const { return counts_; }
 
     const char* family() const override { return spec_.architecture.c_str(); }
     uint32_t vocab() const override { return spec_.vocab; }
@@ -566,6 +570,7 @@ private:
         if (it != steps_.end() && it->graph) {
             std::rotate(steps_.begin(), it, it + 1);
             M40H_TRY(m40llm_cuda_graph_launch(ctx_, steps_.front().graph, kStream));
+            ++counts_.replayed;
             return;
         }
         launches();
@@ -583,6 +588,7 @@ private:
         if (++f.seen != kRecordAt) return;
         try {
             f.graph = recorded(launches);
+            counts_.recorded += f.graph != nullptr;
         } catch (const std::exception&) {}                // the step itself is launched; so are the next ones
     }
 
@@ -717,9 +723,11 @@ private:
         M40llmCudaGraphExec* graph;
         uint32_t seen;
     };
-    static void drop(StepForm& f) {
-        if (f.graph) m40llm_cuda_graph_destroy(f.graph);
+    void drop(StepForm& f) {
+        if (!f.graph) return;
+        m40llm_cuda_graph_destroy(f.graph);
         f.graph = nullptr;
+        ++counts_.dropped;
     }
     void drop_steps() {
         for (StepForm& f : steps_) drop(f);
@@ -746,6 +754,7 @@ private:
     static constexpr size_t kKeptSteps = 8;
     static constexpr uint32_t kRecordAt = 3;
     std::vector<StepForm> steps_;                     // the latest first
+    StepCounts counts_;
 };
 
 // A folder with config.json and model.safetensors.

@@ -116,6 +116,12 @@ class LayeredModel:
     def free_pages(self):
         return self.H.m40host_model_free_pages(self.h)
 
+    def step_counts(self):
+        """(passes replayed from a graph, graphs recorded, graphs dropped)"""
+        n = (C.c_uint32 * 3)()
+        self._ok(self.H.m40host_model_step_counts(self.h, *(C.byref(n, 4 * i) for i in range(3))), "m40host_model_step_counts")
+        return tuple(n)
+
     def decode_greedy(self, seq, prompt, n_gen, start_pos=0):
         p = np.ascontiguousarray(prompt, dtype=np.uint32)
         ids = np.zeros(len(p) + n_gen, dtype=np.uint32)

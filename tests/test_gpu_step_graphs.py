@@ -42,10 +42,18 @@ def test_replayed_steps_equal_launched_steps(ctx, design, dtype):
     def singles(n, seqs, want=lambda s: [0]):
         for _ in range(n):
             step([(s, 1, want(s)) for s in seqs])
+
+    def counts(since=(0, 0, 0)):
+        assert models[1].step_counts() == (0, 0, 0)
+        return tuple(a - b for a, b in zip(models[0].step_counts(), since))
     step([(0, 5, [4]), (1, 58, [0, 57]), (2, 130, [129])])
     singles(12, (0, 1, 2))                                   # one sequence grows past its first page
+    replayed, recorded, _ = counts()
+    assert replayed >= 3 and 1 <= recorded <= 3              # four steps at least before and behind what the launches are split for anew
     singles(6, (2, 0), lambda s: [0] if s else [])           # another form, one place wanted
-    step([(3, 90, [89]), (0, 1, [0])])                       # a prompt beside a token: buffers may be made anew
+    before = counts()
+    step([(3, 700, [699]), (0, 1, [0])])                     # a prompt beside a token, whose tables are larger than any before
+    assert counts(before)[0] == 0 and models[0].step_counts()[1] == models[0].step_counts()[2]      # every graph went
     singles(5, (0, 1, 2))
     singles(5, (3, 1, 0, 2))
     for m in models:
@@ -53,8 +61,11 @@ def test_replayed_steps_equal_launched_steps(ctx, design, dtype):
     singles(4, (0, 2, 3), lambda s: [])                      # no logits at all
     step([(1, 1, [0])])
     singles(5, (1, 0, 2))
+    before = counts()
     models[0].set_mode(2)
+    assert counts(before)[2] >= 1
     singles(5, (1, 0, 2))
+    assert counts(before)[:2] == (2, 1)
     for n in range(10):                                      # more forms than are kept, and back to the first
         singles(4, [(0, 1, 2, 3)[i] for i in range(4) if n + 1 >> i & 1])
     singles(4, (1, 0, 2))
