@@ -600,7 +600,7 @@ int m40llm_ext_pack_tiles_async(M40llmCudaContext* ctx, const void* d_src_bf16, 
 /* n bf16 values, uniform with mean 0 and the given standard deviation, from a counter-based generator */
 int m40llm_ext_fill_random_bf16_async(M40llmCudaContext* ctx, void* d_dst, uint64_t n, uint64_t seed, float std_dev,
                                       uint32_t stream_kind);
-/* A context whose streams take launches only to record them: streams of its own, ctx's device and scratch.  What is enqueued through it between
+/* A context that takes launches only to record them: a stream of its own (for both kinds), ctx's device and scratch.  What is enqueued through it between
  * m40llm_cuda_graph_begin_capture and m40llm_cuda_graph_end_capture becomes the graph, whatever other threads enqueue on ctx meanwhile; the graph is
  * launched on ctx.  Nothing else is to be enqueued through it.  NULL on failure; given back with m40llm_destroy_context, before ctx is. */
 M40llmCudaContext* m40llm_ext_create_recorder(M40llmCudaContext* ctx);

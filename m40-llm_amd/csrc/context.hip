@@ -157,7 +157,7 @@ void m40llm_destroy_context(M40llmCudaContext* ctx) {
     }
     if (ctx->prefill_waits_decode_event) (void)hipEventDestroy(ctx->prefill_waits_decode_event);
     if (ctx->decode_waits_prefill_event) (void)hipEventDestroy(ctx->decode_waits_prefill_event);
-    if (ctx->prefill_stream) (void)hipStreamDestroy(ctx->prefill_stream);
+    if (ctx->prefill_stream && ctx->prefill_stream != ctx->decode_stream) (void)hipStreamDestroy(ctx->prefill_stream);
     if (ctx->decode_stream) (void)hipStreamDestroy(ctx->decode_stream);
     delete ctx;
 }
@@ -169,13 +169,14 @@ M40llmCudaContext* m40llm_ext_create_recorder(M40llmCudaContext* ctx) {
     rec->recorder_of = ctx;
     rec->prefill_stream = rec->decode_stream = nullptr;
     rec->prefill_waits_decode_event = rec->decode_waits_prefill_event = nullptr;
-    if (hipStreamCreateWithFlags(&rec->prefill_stream, hipStreamNonBlocking) != hipSuccess || hipStreamCreateWithFlags(&rec->decode_stream, hipStreamNonBlocking) != hipSuccess ||
-        hipEventCreateWithFlags(&rec->prefill_waits_decode_event, hipEventDisableTiming) != hipSuccess ||
+    // one stream for both kinds: it never runs anything
+    if (hipStreamCreateWithFlags(&rec->decode_stream, hipStreamNonBlocking) != hipSuccess || hipEventCreateWithFlags(&rec->prefill_waits_decode_event, hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&rec->decode_waits_prefill_event, hipEventDisableTiming) != hipSuccess) {
         (void)hipGetLastError();
         m40llm_destroy_context(rec);
         return nullptr;
     }
+    rec->prefill_stream = rec->decode_stream;
     return rec;
 }
 

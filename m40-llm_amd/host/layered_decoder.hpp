@@ -356,6 +356,7 @@ private:
         pick_parts_ = DeviceBuf(ctx_, (size_t)logits_rows_ * M40LLM_TOP2_PARTS * 16);
         const size_t row = (size_t)spec_.vocab * 4;
         if (const size_t n = std::min<size_t>(std::min(logits_rows_, opt_.max_sequences), kMostPinned / row); n > 0) logits_host_ = PinnedBuf(ctx_, n * row);
+        recorder_ = m40llm_ext_create_recorder(ctx_);      // here and not at the first recording: the process's first takes 3 ms; null: launches only
         for (const SlotState& s : rt_.states) state_bytes_ += s.slot_bytes;
         M40H_TRY(m40llm_stream_synchronize(ctx_, kStream));
     }
@@ -543,8 +544,7 @@ private:
     // another thread enqueues there meanwhile has to run now, and once.
     template <class F>
     M40llmCudaGraphExec* recorded(const F& launches) {
-        if (!recorder_ && !(recorder_ = m40llm_ext_create_recorder(ctx_))) return nullptr;
-        if (m40llm_cuda_graph_begin_capture(recorder_, kStream) != 0) return nullptr;
+        if (!recorder_ || m40llm_cuda_graph_begin_capture(recorder_, kStream) != 0) return nullptr;
         rt_.ctx = recorder_;
         try {
             launches();
@@ -664,8 +664,7 @@ private:
                                                    loop_gaps_.f32(), total, kStream));
         };
         auto run = [&](uint32_t n) {
-            if (mode_ >= 2 && n > 0) {
-                if (!graph_ && !(graph_ = recorded(enqueue))) throw std::runtime_error("a step could not be recorded");
+            if (mode_ >= 2 && n > 0 && (graph_ || (graph_ = recorded(enqueue)))) {
                 for (uint32_t i = 0; i < n; ++i) M40H_TRY(m40llm_cuda_graph_launch(ctx_, graph_, kStream));
             } else {
                 for (uint32_t i = 0; i < n; ++i) enqueue();
@@ -735,7 +734,7 @@ private:
     }
 
     M40llmCudaContext* ctx_;
-    M40llmCudaContext* recorder_ = nullptr;           // made for the first recording
+    M40llmCudaContext* recorder_ = nullptr;
     DecoderSpec spec_;
     LayeredOptions opt_;
     SequencePages seqs_;

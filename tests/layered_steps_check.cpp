@@ -15,7 +15,7 @@ namespace {
 struct World {
     const void* own = nullptr;
     const void* capturing = nullptr;
-    int launched = 0, recorded = 0, replays = 0, recordings = 0, destroyed = 0, blocking_copies = 0;
+    int launched = 0, recorded = 0, replays = 0, recordings = 0, destroyed = 0, blocking_copies = 0, recorders = 0;
     bool captured_shared = false, fail_recording = false;
     std::vector<std::string> head;         // what the head's norms and the last sums of the streams were given, launches only
     std::string order;                     // L a launch, R a recorded one, G a replay, B / E a recording's begin and end, X given up
@@ -70,7 +70,10 @@ int m40llm_ext_stream_update_async(M40llmCudaContext* ctx, const M40llmStreamUpd
     return 0;
 }
 static char recorder;
-M40llmCudaContext* m40llm_ext_create_recorder(M40llmCudaContext* ctx) { return ctx == world.own ? reinterpret_cast<M40llmCudaContext*>(&recorder) : nullptr; }
+M40llmCudaContext* m40llm_ext_create_recorder(M40llmCudaContext* ctx) {
+    ++world.recorders;
+    return ctx == world.own ? reinterpret_cast<M40llmCudaContext*>(&recorder) : nullptr;
+}
 void m40llm_destroy_context(M40llmCudaContext*) {}
 int m40llm_cuda_graph_begin_capture(M40llmCudaContext* ctx, uint32_t) {
     if (ctx == world.own) world.captured_shared = true;
@@ -141,7 +144,7 @@ static void steps(std::istream& in) {
             world.order.clear();
             d.step(entries, place ? logits.data() : nullptr);
             log << (first ? "" : ", ") << "{\"replays\": " << world.replays - before.replays << ", \"recordings\": " << world.recordings - before.recordings
-                << ", \"destroyed\": " << world.destroyed - before.destroyed << ", \"blocking_copies\": " << world.blocking_copies - before.blocking_copies << ", \"order\": " << quoted(world.order) << ", \"head\": [";
+                << ", \"destroyed\": " << world.destroyed - before.destroyed << ", \"recorders\": " << world.recorders - before.recorders << ", \"blocking_copies\": " << world.blocking_copies - before.blocking_copies << ", \"order\": " << quoted(world.order) << ", \"head\": [";
             for (size_t i = 0; i < world.head.size(); ++i) log << (i ? ", " : "") << quoted(world.head[i]);
             log << "]}";
             first = false;

@@ -55,7 +55,7 @@ def test_more_logits_than_one_head_takes(run, design, singles):
 def test_steps_are_recorded_beside_the_contexts_stream(run, design):
     """What another thread enqueues on the context's stream while a step is recorded has to run, so nothing of a recording goes there."""
     got = run(design, 2, [[(0, 1, 1), (1, 1, 1)]] * 6)
-    assert not got["captured_shared"]
+    assert not got["captured_shared"] and not any(s["recorders"] for s in got["steps"])      # that stream is made with the model: 3 ms in a process's first
     assert sum(s["recordings"] for s in got["steps"]) == 1 and sum(s["replays"] for s in got["steps"]) >= 3
     for s in got["steps"]:
         assert ("BRE" in s["order"]) == (s["recordings"] == 1) and s["order"].count("R") == s["recordings"], s["order"]
