@@ -635,8 +635,9 @@ int launch_tiles(hipStream_t stream, const _Float16* hi, const _Float16* lo, con
         tiles_n += (mats.N[i] + BN - 1) / BN;
     }
     mats.tile_start[mats.n] = (int)tiles_n;
-    // M 4096, N 11264, K 2048 on the 128 x 256 tile (32 tile rows), bands of 4 / 6 rows: 357 / 338 us (bands of 2, 4, 8 and 16 are all slower than 5, 6
-    // and 7); M 522, N 2048, K 5632 on 64 x 128 (9 tile rows), bands of 1 / 3 / 5 / 9: 54.2 / 48.1 / 46.7 / 44.4 us
+    // On the 128 x 256 tile, bands of 1 / 2 / 4 / 6 / 7 / 9 / 16 rows: M 4096 (32 tile rows), N 11264, K 2048 413 / 360 / 320 / 310 / 302 / 305 / 314 us; N 2048, K 5632
+    // 157 / 165 / 157 / 146 / 140 / 141 / 141; M 2048, N 11264, K 2048 174 / 200 / 175 / 162 / 163 / 159 / 161.  M 522, N 2048, K 5632 on 64 x 128 (9 tile rows), bands of 1 / 3 / 5 /
+    // 9: 44.7 / 46.8 / 45.9 / 43.7
     const int band = tiles_m <= 9 ? tiles_m : 6;
     gemm_tiled_kernel<MT, NT, KS, kBufs, kBBufs><<<(unsigned)(tiles_m * tiles_n * k_splits), kThreads, bytes, stream>>>(hi, lo, row_scale, mats, M, K, k_splits, band);
     return hipGetLastError() == hipSuccess ? 0 : -2;
@@ -644,11 +645,13 @@ int launch_tiles(hipStream_t stream, const _Float16* hi, const _Float16* lo, con
 
 // Which tile, and into how many parts to cut K.  A launch of t workgroups on c CUs takes, per step of 32 k, about
 // max(least, start * ceil(t / c) + load * t / c): a workgroup alone on its CU is bound by the round trips of a step, more of them by the step's
-// products and LDS traffic, and by caches and clock when the other CUs work too.  Fitted to 50 shapes with weights that no cache holds (M 60 ..
-// 4096 of N 2048, 2560, 11264, K 2048 and 5632), most within 10 %, e.g. N 2048, K 2048 (128 x 256 / 128 x 128 / 64 x 128 / 64 x 64):
-//   60 rows 43.6 / 28.5 / 21.0 / 15.5 us, 522 rows 43.3 / 28.0 / 18.2 / 23.4, 1030 rows 44.1 / 30.4 / 35.0 / 35.6, 4096 rows 62 / 82 / 84 / 110
-// (a 128 x 128 tile staged through registers and cut into four parts of K up to 128 tiles, with the launch that adds them: 23 / 32 / 42.7 / 80).
-// Parts of K cost the launch that adds their sums; K 5632 at 256 rows: 35.9 us whole, 24.7 us in two.
+// products and LDS traffic, and by caches and clock when the other CUs work too.  The constants were fitted to 50 shapes when instructions loaded half lines;
+// with whole lines, weights that no cache holds, N 2048, K 2048 (128 x 256 / 128 x 128 / 64 x 128 / 64 x 64):
+//   60 rows 40.4 / 25.3 / 21.6 / 16.2 us, 522 rows 44.1 / 27.1 / 18.9 / 23.3, 1030 rows 45.9 / 30.7 / 36.0 / 37.1, 2048 rows 49.5 / 35.5 / 44.4 / 60.3, 4096 rows 62.4 / 86.1 /
+//   96.0 / 118.6
+// Of M 60, 101, 250, 522, 1030, 2048 and 4096 with N 2048, 2560 and 11264 at K 2048 and N 2048 at K 5632 the tile chosen for a whole K is the fastest or within 3 % of it but
+// for M 4096, N 2560 (128 x 256, 96 to 100 us, where 128 x 128 takes 90).
+// Parts of K cost the launch that adds their sums; N 2048, K 5632 at 250 rows: 35.9 us whole, 19.7 us and that launch in parts.
 struct TileChoice { int shape, k_splits; };
 constexpr struct { int bm, bn; float least, start, load; } kShapes[4] = {
     {128, 256, 0.66f, 0.62f, 0.28f}, {128, 128, 0.44f, 0.38f, 0.20f}, {64, 128, 0.28f, 0.25f, 0.05f}, {64, 64, 0.235f, 0.17f, 0.03f}};

@@ -401,8 +401,11 @@ int launch_t(hipStream_t stream, const WideArgs& a, int k_parts) {
     rows_wide_kernel<MODE, RT, T><<<dim3((a.tiles + T - 1) / T, k_parts), kThreads, bytes, stream>>>(a);
     return hipGetLastError() == hipSuccess ? 0 : -7;
 }
-// Tiles per workgroup: rounds of workgroups over the CUs (one is resident per CU) times what a workgroup costs, its tiles and about one
-// more for its start.
+// Tiles per workgroup: rounds of workgroups over the CUs times what a workgroup costs, its tiles and about one more for its start.  (Of up to sixteen rows and
+// one tile two workgroups fit a CU; they gain less than the start that they repeat.)  All choices measured, K 2048, in the order 1 / 2 / 3 / 4 / 6 tiles, the rule's
+// in brackets, us: gate and up of 5632, 16 rows 16.0 / 13.8 / [10.8] / 11.6 / 14.1, 32 rows 27.0 / 21.9 / [13.8] / 15.0 / 18.4; of 11008, 16 rows 28.1 / 20.3 /
+// 18.5 / 22.5 / [17.6], 32 rows 52.0 / 32.6 / 25.8 / 28.2 / [21.7]; vocabulary of 32000, 16 rows 39.1 / 30.4 / 30.4 / [30.8] / 35.5, 32 rows 71.8 / 44.4 / 40.6 / [35.3] /
+// 42.7; N 4096, 16 rows [8.2] / 9.2 / 10.2 / 11.0 / 13.6.  Of 24 such launches (12 to 32 rows) the rule's is the fastest or within 7 % of it (12 rows, vocabulary of 128256: 114, three tiles 106).
 int pick_tiles(int tiles, int num_cus) {
     int best = 1, best_cost = 1 << 30;
     for (const int t : {1, 2, 3, 4, 6}) {

@@ -1,5 +1,5 @@
-"""Projections of a decode step for up to 32 rows (m40llm_ext_batched_wide_*): every row count at the edges of its tiles of sixteen, K that ends in the
-middle of a chunk of 512, columns that end in the middle of a tile, every number of column tiles per workgroup, against 64-bit products."""
+"""Projections of a decode step for up to 32 rows (m40llm_ext_batched_wide_*): every row count at the edges of its tiles of sixteen, K that gives
+the eight waves unequal numbers of blocks of 64, columns that end in the middle of a tile, every number of column tiles per workgroup, against 64-bit products."""
 import numpy as np
 import pytest
 
