@@ -2,8 +2,8 @@
 //
 // rows_packed_kernel   a workgroup owns one or two column tiles for up to 64 rows and its waves share out K: weights go
 //                      straight from memory into the matrix instruction's operand registers, one contiguous kilobyte a
-//                      load, each tile read once per 64 rows; the waves' sums meet in LDS.  Decode steps and short
-//                      portions, and every product in f32.
+//                      load, each tile read once per 64 rows; the waves' sums meet in LDS.  17 to 64 rows, and every
+//                      product in f32 (up to 16 bf16 rows: few_rows.hip).
 // tile_packed_kernel   bf16, more rows: tiles of C of 64 x 64 to 128 x 256, both operands staged through LDS by direct
 //                      global-to-LDS loads, five or six stages deep with one barrier a stage.  The buffers hold
 //                      operands in instruction order, so LDS reads are contiguous kilobytes as well.
@@ -149,10 +149,8 @@ int launch_rows(hipStream_t stream, const PackedArgs& g, const M40Epilogue<T>& e
 }
 
 // Waves and column tiles of a workgroup, bf16: a launch is mostly the round trips of its requests, so as many waves share out K as let every
-// workgroup have its place at once (32 waves a CU); more than 16 rows take tiles in pairs, which read the rows once.  K 2048, weights that no cache
+// workgroup have its place at once (32 waves a CU); bf16 tiles go in pairs, which read the rows once.  K 2048, weights that no cache
 // holds, us:
-//   8 rows, 16 / 8 / 4 waves: 192 tiles 5.7 / 6.5 / 8.3, 384 tiles 8.2 / 7.5 / 8.9, 528 tiles 11.3 / 11.7 / 10.3, 644 tiles 11.7 / 13.1 / 10.6, 2000 tiles
-//   29.8 / 27.7 / 25.1;  gate and up in pairs, 352 of them: 13.1 / 13.1 / 11.6
 //   64 rows, 16 waves / pairs and 8 waves / pairs and 4: 192 tiles 8.5 / 11.0 / 12.4, 384 tiles 15.0 / 11.1 / 11.7, 644 tiles 21.8 / 21.1 / 18.8, 2000 tiles
 //   57 / 43 / 36
 template <class T, int MT, int PARTS, int JOBS>
@@ -187,7 +185,8 @@ int launch_rows_m(hipStream_t stream, const PackedArgs& g, const M40Epilogue<T>&
 }
 template <class T, int JOBS>
 int launch_rows_any(hipStream_t stream, const PackedArgs& g, const M40Epilogue<T>& e, int batches, int rows, int num_cus) {
-    if (rows <= 16) return launch_rows_m<T, 1, JOBS>(stream, g, e, batches, num_cus);
+    if constexpr (sizeof(T) == 4)          // (few_rows.hip in bf16)
+        if (rows <= 16) return launch_rows_m<T, 1, JOBS>(stream, g, e, batches, num_cus);
     if (rows <= 32) return launch_rows_m<T, 2, JOBS>(stream, g, e, batches, num_cus);
     return launch_rows_m<T, 4, JOBS>(stream, g, e, batches, num_cus);
 }
@@ -495,6 +494,11 @@ M40Epilogue<T> make_epilogue(const M40llmPackedGemm& p) {
     return e;
 }
 
+int launch_few(hipStream_t stream, const PackedArgs& g, const M40Epilogue<m40_bf16>& e, int batches, int num_cus) {
+    const M40FewRows f{static_cast<const m40_bf16*>(g.a), g.w, g.lda, g.a_batch, g.w_batch, g.n_tiles, g.k_tiles, g.rows, g.k_stride, g.k_total, g.segment, batches, g.jobs ? g.rows : 1, g.jobs, g.gather};
+    return m40_few_rows_product(stream, f, e, num_cus);
+}
+
 // one thread per source element
 __global__ __launch_bounds__(256) void pack_tiles_kernel(const uint16_t* __restrict__ src, uint16_t* __restrict__ dst,
                                                          M40llmPackPlan p, size_t total) {
@@ -642,6 +646,7 @@ int m40llm_ext_packed_gemm_async(M40llmCudaContext* ctx, const M40llmPackedGemm*
         }
         const M40Epilogue<m40_bf16> e = make_epilogue<m40_bf16>(*p);
         if (rows == 128) return launch_tile_any<kSlots>(stream, g, e, 1, ctx->num_cus);
+        if (rows == 16) return launch_few(stream, g, e, 1, ctx->num_cus);
         return p->gather ? launch_rows_any<m40_bf16, kJobGather>(stream, g, e, 1, rows, ctx->num_cus) : launch_rows_any<m40_bf16, kJobSlots>(stream, g, e, 1, rows, ctx->num_cus);
     }
     if (p->act_dtype == M40LLM_ACT_F32) {
@@ -651,6 +656,7 @@ int m40llm_ext_packed_gemm_async(M40llmCudaContext* ctx, const M40llmPackedGemm*
     const M40Epilogue<m40_bf16> e = make_epilogue<m40_bf16>(*p);
     if (p->epilogue == M40LLM_PACKED_KEYS) return launch_tile_any<kPageKeys>(stream, g, e, batches, ctx->num_cus);
     if (p->epilogue == M40LLM_PACKED_VALUES) return launch_tile_any<kPageValues>(stream, g, e, batches, ctx->num_cus);
+    if (g.rows <= 16) return launch_few(stream, g, e, batches, ctx->num_cus);
     // few columns leave most CUs without a wide tile
     if (g.rows <= 64 || (g.n_tiles <= 8 && batches == 1 && g.rows <= 65535 * 16 && p->epilogue != M40LLM_PACKED_PROJECT)) return launch_rows_any<m40_bf16, kAllRows>(stream, g, e, batches, g.rows, ctx->num_cus);
     return launch_tile_any<kPlainRows>(stream, g, e, batches, ctx->num_cus);

@@ -243,4 +243,16 @@ __device__ __forceinline__ void m40_epilogue_pair(const M40Epilogue<T>& e, int r
     }
     m40_store_packed<T>(e.out_act, row, e.act_col + col, e.ld_act, y, 4, true);
 }
+
+// A product of at most 16 bf16 rows (few_rows.hip).  All rows, of one batch or several (heads, parts of K), or products per expert: jobs with packed rows
+// in the order of the list, or with plain rows that `gather` names.
+enum { kFewAll = 0, kFewSlots = 1, kFewGather = 2 };
+struct M40FewRows {
+    const m40_bf16 *a, *w;
+    long lda, a_batch, w_batch;
+    int n_tiles, k_tiles, rows, k_stride, k_total, segment, batches;      // as in a product of any rows
+    int max_jobs;                  // 1 without jobs
+    const uint32_t *jobs, *gather;
+};
+int m40_few_rows_product(hipStream_t stream, const M40FewRows& g, const M40Epilogue<m40_bf16>& e, int num_cus);
 #endif  // __HIPCC__

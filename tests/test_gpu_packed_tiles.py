@@ -66,6 +66,36 @@ def test_waves_and_pairs_change_no_bit(ctx, rows, k):
     assert np.array_equal(got[2][:, last:].view(np.uint32), tail.view(np.uint32))
 
 
+# up to 16 rows: one tile a workgroup and (more than eight rows of more than four tiles a CU) two, gate and up over 8 and (more than one pair a CU, at most
+# two) 4 waves; rows that are not there hold no numbers
+@pytest.mark.parametrize("rows,k", [(1, 2048), (8, 2080), (9, 2048), (15, 2368), (16, 3000), (3, 1000), (9, 96)])
+def test_forms_of_few_rows_change_no_bit(ctx, rows, k):
+    rng, K = np.random.default_rng(rows + k), up32(k)
+    A, W = rng.standard_normal((rows, k)), bf16w(rng, 16 * 1100, k)
+    full = np.full((16, K), np.nan)
+    full[:rows, :k], full[:rows, k:] = A, 0.0
+    want, bufs = rounded(A, "bfloat16") @ W.T.astype(np.float64), [ctx.to_device(pack_tiles(b)) for b in (ld.f32_to_bf16(full), ld.f32_to_bf16(W))]
+
+    def product(tiles, kind):
+        n = 16 * tiles if kind == STORE else 8 * tiles
+        out = ctx.to_device(np.zeros((rows, n), np.float32) if kind == STORE else np.zeros((16, n), np.uint16))
+        g = Gemm(act_dtype=ACT["bfloat16"], epilogue=kind, a=bufs[0].ptr, lda=K, w=bufs[1].ptr, n_tiles=tiles, k_tiles=K // 32, rows=rows, batches=1, activation=1)
+        if kind == STORE:
+            g.out_f32, g.ld_out, g.cols = out.ptr, n, n
+        else:
+            g.out_act, g.ld_act = out.ptr, n
+        call(ctx, "m40llm_ext_packed_gemm_async", C.byref(g), 1)
+        return out.download(np.float32, (rows, n)) if kind == STORE else unpack_tiles(out.download(np.uint16, (16 * n,)), rows, n)
+    wide = product(1100, STORE)
+    close_to(wide, want, "float32", factor=2)
+    assert np.array_equal(wide[:, :64].view(np.uint32), product(4, STORE).view(np.uint32))
+    act = product(1100, PROJECT)                       # 550 pairs, 300, 4
+    gate, up = want.reshape(rows, 550, 2, 16).transpose(2, 0, 1, 3).reshape(2, rows, -1)
+    close_to(from_act(act, "bfloat16"), gate / (1.0 + np.exp(-gate)) * up, "bfloat16", factor=2)
+    for tiles in (600, 8):
+        assert np.array_equal(act[:, :64], product(tiles, PROJECT)[:, :64])
+
+
 # 64 x 64 tiles (two k tiles a stage), 64 x 128, 128 x 128 (one and two a stage), 128 x 256 (long sums)
 @pytest.mark.parametrize("k", [992, 2048, 2112])
 def test_tile_shapes_change_no_bit(ctx, k):
