@@ -277,9 +277,12 @@ __global__ __launch_bounds__(kThreads) void gemv_residual_kernel(const float* __
     }
 }
 
-// hid[j] = silu(Wg[j] . xn) * (Wu[j] . xn),  xn = RMSNorm(x) * w.  A wave owns PAIRS consecutive j (gate and up rows).
-template <int PAIRS>
-__global__ __launch_bounds__(kThreads) void norm_gate_up_swiglu_kernel(const float* __restrict__ x,
+// hid[j] = silu(Wg[j] . xn) * (Wu[j] . xn),  xn = RMSNorm(x) * w.  A wave owns one j (gate and up row).  The row is staged by the first four waves (whose
+// order of sums the norm's own kernel has); four more that only stream weights halve how often it is staged, and keep as many requests in flight as half as many
+// waves with two j each: 46 MB (FFN 5632, K 2048) 10.1 -> 9.5 us a launch, 90 MB (11008) 17.1 -> 16.1; with one j and four waves 10.8 and 17.1, sixteen waves
+// 10.9 and 17.1, eleven (two workgroups on every CU) 9.6 and 16.7.
+template <int WAVES>
+__global__ __launch_bounds__(WAVES * 64) void norm_gate_up_swiglu_kernel(const float* __restrict__ x,
                                                                        const void* __restrict__ norm_w,
                                                                        uint32_t norm_dtype, float eps,
                                                                        const uint16_t* __restrict__ Wg,
@@ -288,31 +291,26 @@ __global__ __launch_bounds__(kThreads) void norm_gate_up_swiglu_kernel(const flo
     extern __shared__ float a_lds[];
     __shared__ float wave_sums[kWavesPerBlock];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int j0 = (blockIdx.x * kWavesPerBlock + wave) * PAIRS;
-    const uint4* bp[2 * PAIRS];
-#pragma unroll
-    for (int q = 0; q < PAIRS; ++q) {
-        const int j = j0 + q < F ? j0 + q : F - 1;
-        bp[2 * q] = reinterpret_cast<const uint4*>(Wg + (size_t)j * K);
-        bp[2 * q + 1] = reinterpret_cast<const uint4*>(Wu + (size_t)j * K);
+    const int j = blockIdx.x * WAVES + wave, row = j < F ? j : F - 1;
+    const uint4* const bp[2] = {reinterpret_cast<const uint4*>(Wg + (size_t)row * K), reinterpret_cast<const uint4*>(Wu + (size_t)row * K)};
+    GemvRegs<2> regs;
+    if (WAVES == kWavesPerBlock || wave < kWavesPerBlock) {
+        StageRegs xr;
+        stage_load(x, norm_w, norm_dtype, K, 0, xr);
+        gemv_prefetch<2>(bp, 0, K >> 3, lane, regs);
+        stage_finish(xr, x, norm_w, norm_dtype, eps, K, a_lds, wave_sums);
+    } else {
+        gemv_prefetch<2>(bp, 0, K >> 3, lane, regs);
+        __syncthreads();                 // as in stage_finish
+        __syncthreads();
     }
-    StageRegs xr;
-    stage_load(x, norm_w, norm_dtype, K, 0, xr);
-    GemvRegs<2 * PAIRS> regs;
-    gemv_prefetch<2 * PAIRS>(bp, 0, K >> 3, lane, regs);
-    stage_finish(xr, x, norm_w, norm_dtype, eps, K, a_lds, wave_sums);
-    float d[2 * PAIRS];
-    gemv_accumulate<2 * PAIRS>(bp, a_lds, 0, K >> 3, lane, regs, d);
-    gemv_finish<2 * PAIRS, 1>(d, nullptr, wave, lane);
-    if (lane == 0) {
-#pragma unroll
-        for (int q = 0; q < PAIRS; ++q) {
-            if (j0 + q < F) {
-                const float g = d[2 * q];
-                const float silu = g / (1.0f + expf(-g));
-                hid[j0 + q] = silu * d[2 * q + 1];
-            }
-        }
+    float d[2];
+    gemv_accumulate<2>(bp, a_lds, 0, K >> 3, lane, regs, d);
+    gemv_finish<2, 1>(d, nullptr, wave, lane);
+    if (lane == 0 && j < F) {
+        const float g = d[0];
+        const float silu = g / (1.0f + expf(-g));
+        hid[j] = silu * d[1];
     }
 }
 
@@ -524,14 +522,10 @@ int m40llm_ext_fused_norm_gate_up_swiglu_async(M40llmCudaContext* ctx, const voi
         (size_t)d_model * 4 > 60 * 1024)
         return -6;
     (void)hipGetLastError();
-    // two (gate, up) row pairs per wave once there are enough rows to fill the chip that way (measured: 3 % faster
-    // than one pair at FFN 5632; four pairs are slower)
-    if (ffn >= 4096)
-    norm_gate_up_swiglu_kernel<2><<<(ffn + 7) / 8, kThreads, (size_t)d_model * 4, ctx->decode_stream>>>(
-        static_cast<const float*>(d_x_f32), d_norm_w, norm_weight_dtype, eps, static_cast<const uint16_t*>(d_wgate_f16),
-        static_cast<const uint16_t*>(d_wup_f16), static_cast<float*>(d_hid_f32), ffn, d_model);
-    else
-    norm_gate_up_swiglu_kernel<1><<<(ffn + 3) / 4, kThreads, (size_t)d_model * 4, ctx->decode_stream>>>(
+    // from two workgroups of eight waves a CU on (measured in the kernel's comment); below, four waves reach more CUs
+    const auto kernel = ffn >= 4096 ? norm_gate_up_swiglu_kernel<8> : norm_gate_up_swiglu_kernel<4>;
+    const int waves = ffn >= 4096 ? 8 : 4;
+    kernel<<<(ffn + waves - 1) / waves, waves * 64, (size_t)d_model * 4, ctx->decode_stream>>>(
         static_cast<const float*>(d_x_f32), d_norm_w, norm_weight_dtype, eps, static_cast<const uint16_t*>(d_wgate_f16),
         static_cast<const uint16_t*>(d_wup_f16), static_cast<float*>(d_hid_f32), ffn, d_model);
     return hipGetLastError() == hipSuccess ? 0 : -7;

@@ -130,6 +130,13 @@ def test_norm_gate_up_swiglu_equals_call_sequence(dev, orc, F, K):
     close(got, want)
 
 
+# four waves a workgroup and (from 4096 rows on) eight, of which four stage the row: a last workgroup that is not full, rows of less than a wave's requests, of more, of two
+# batches of the staging
+@pytest.mark.parametrize("F,K", [(4095, 256), (4096, 512), (4099, 2048), (4101, 2304), (4097, 4352)])
+def test_norm_gate_up_swiglu_of_four_and_eight_waves(dev, orc, F, K):
+    test_norm_gate_up_swiglu_equals_call_sequence(dev, orc, F, K)
+
+
 @pytest.mark.parametrize("V,K", [(32000, 2048), (151936, 2048), (1000, 256), (5, 64)])
 def test_lm_head_top2_and_greedy_step(dev, orc, V, K):
     rng = np.random.default_rng(V)
