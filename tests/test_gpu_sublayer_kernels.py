@@ -217,6 +217,30 @@ def test_choice_of_experts_and_sorted_list(ctx, rows, experts, identity, top, jo
     assert rows_of[:jobs[1]].max(initial=0) < rows
 
 
+# the list of up to 16 rows comes from one workgroup, that of 17 from one an expert; experts that fill their words of bits and not, choices of a whole wave
+@pytest.mark.parametrize("rows", [2, 15, 16, 17])
+@pytest.mark.parametrize("experts,identity,top", [(32, 0, 4), (33, 2, 6), (64, 0, 64), (65, 1, 9), (1000, 24, 33), (1024, 0, 3)])
+def test_list_of_few_rows(ctx, rows, experts, identity, top):
+    rng = np.random.default_rng(rows + experts)
+    n = experts + identity
+    z = (rng.standard_normal((rows, n)) * 2).astype(np.float32)
+    z[:, experts // 2] += 9.0          # everyone's
+    ids, weight, d_rows, d_place, d_jobs, slots, max_jobs, _ = route(ctx, z, np.zeros(n, np.float32), experts, top, 16)
+    order = np.argsort(-z, axis=1, kind="stable")[:, :top]
+    assert np.array_equal(np.sort(ids, axis=1), np.sort(order, axis=1))
+    rows_of, jobs, place = [], [], np.full((rows, top), INPUT, np.uint32)
+    for e in range(experts):
+        r, j = np.nonzero(ids == e)
+        for i in range(0, len(r), 16):
+            jobs.append((e, len(rows_of) + i, min(16, len(r) - i), 0))
+        place[r, j] = len(rows_of) + np.arange(len(r))
+        rows_of += r.tolist() + [0] * (-len(r) % 16)
+    assert np.array_equal(d_place.download(np.uint32, (rows, top)), place)
+    got = d_jobs.download(np.uint32, (4 + 4 * max_jobs,))
+    assert got[0] == len(jobs) and got[1] == len(rows_of) and np.array_equal(got[4:4 + 4 * len(jobs)].reshape(-1, 4), jobs)
+    assert np.array_equal(d_rows.download(np.uint32, (slots,))[:len(rows_of)], rows_of)
+
+
 @pytest.mark.parametrize("dtype,job_rows", [("float32", 16), ("float32", 64), ("bfloat16", 16), ("bfloat16", 32), ("bfloat16", 64), ("bfloat16", 128)])
 @pytest.mark.parametrize("rows,experts,top,width,ff", [(1, 3, 2, 64, 40), (50, 4, 3, 100, 70), (300, 5, 2, 256, 130), (200, 1, 1, 96, 16)])
 def test_products_per_expert(ctx, dtype, job_rows, rows, experts, top, width, ff):
