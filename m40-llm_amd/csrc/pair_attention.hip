@@ -290,11 +290,46 @@ __global__ __launch_bounds__(256, 1) void pair_rows_kernel(PairArgs p) {
         }
     const float c = a.scale * kLog2e;
     const m40_bf16* cache = static_cast<const m40_bf16*>(a.cache) + kv * p.page.head_elements() + lane * 8;
+    // What the end needs is requested now, by the wave that will need it, and found near by then: gates and sink were two round trips behind the last product.
+    m40_float4 gates[M == 1 ? DVT : 1];
+    float sink = 0.0f;
+    if (wave == 0 && a.splits == 1u) {
+        const float* z = static_cast<const float*>(a.gate) + (a.gate ? (size_t)row * a.ld_gate + (M == 1 ? head * a.vdim : head) : 0);
+        const bool vec = M == 1 && a.gate && a.vdim % 4u == 0 && a.ld_gate % 4u == 0 && m40_aligned16(a.gate);
+#pragma unroll
+        for (int j = 0; j < (M == 1 ? DVT : 1); ++j) {
+            gates[j] = m40_float4{0.f, 0.f, 0.f, 0.f};
+            if (vec && j * 16 + 4 * g < (int)a.vdim) gates[j] = *reinterpret_cast<const m40_float4*>(z + j * 16 + 4 * g);
+            else if (M != 1) gates[j][0] = z[0];
+        }
+        if (a.sink) sink = static_cast<const float*>(a.sink)[head];
+    }
+    // a page's keys and values together where they have room: the values behind the scores were one more round trip a page
+    constexpr bool kTogether = M * DKT <= 4 && DVT <= 8;
     for (uint32_t n = page0 + wave; n < page1; n += 4u) {
         const m40_bf16* keys = cache + table[n] * p.page.elements();
         const m40_bf16* values = keys + p.page.key_elements();
         const bool whole = whole_page<X>(a, n, first_pos, last_pos);
-        m40_bf16x8 pf[M][1][2], vf[DVT][2];
+        m40_bf16x8 pf[M][1][2], vf[DVT][2], kf[M][4][kTogether ? DKT : 1];
+        auto key_tile = [&](int m, int t, int k) __attribute__((always_inline)) {
+            return *reinterpret_cast<const m40_bf16x8*>(keys + ((m * 4 + t) * kt + (k < kt ? k : kt - 1)) * kM40Tile);
+        };
+        auto load_values = [&]() __attribute__((always_inline)) {
+#pragma unroll
+            for (int j = 0; j < DVT; ++j)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) vf[j][h] = *reinterpret_cast<const m40_bf16x8*>(values + ((j < vt ? j : vt - 1) * 2 + h) * kM40Tile);
+        };
+        if constexpr (kTogether) {
+#pragma unroll
+            for (int m = 0; m < M; ++m)
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+#pragma unroll
+                    for (int k = 0; k < DKT; ++k) kf[m][t][k] = key_tile(m, t, k);
+            load_values();
+            __builtin_amdgcn_sched_barrier(0);
+        }
 #pragma unroll
         for (int m = 0; m < M; ++m) {
             m40_float4 sc[4][1];
@@ -302,17 +337,10 @@ __global__ __launch_bounds__(256, 1) void pair_rows_kernel(PairArgs p) {
             for (int t = 0; t < 4; ++t) {
                 sc[t][0] = m40_float4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int k = 0; k < DKT; ++k) {
-                    const m40_bf16x8 kf = *reinterpret_cast<const m40_bf16x8*>(keys + ((m * 4 + t) * kt + (k < kt ? k : kt - 1)) * kM40Tile);
-                    sc[t][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, s.q[m][0][k], sc[t][0], 0, 0, 0);
-                }
+                for (int k = 0; k < DKT; ++k)
+                    sc[t][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kTogether ? kf[m][t][kTogether ? k : 0] : key_tile(m, t, k), s.q[m][0][k], sc[t][0], 0, 0, 0);
             }
-            if (m == 0) {
-#pragma unroll
-                for (int j = 0; j < DVT; ++j)
-#pragma unroll
-                    for (int h = 0; h < 2; ++h) vf[j][h] = *reinterpret_cast<const m40_bf16x8*>(values + ((j < vt ? j : vt - 1) * 2 + h) * kM40Tile);
-            }
+            if (!kTogether && m == 0) load_values();
             if constexpr (X >= kBounded) {
                 s.template weigh_bounded<X>(a, slope, sc, whole, n * kPage + 4 * g, pf[m]);
             } else {
@@ -328,7 +356,8 @@ __global__ __launch_bounds__(256, 1) void pair_rows_kernel(PairArgs p) {
                 for (int h = 0; h < 2; ++h) s.o[m][j][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[j][h], pf[m][0][h], s.o[m][j][0], 0, 0, 0);
     }
     constexpr int kFloats = PairState<M, DKT, DVT, 1>::kFloats;
-    if (wave > 0) {
+    const int busy = page1 > page0 + 3u ? 4 : page1 > page0 ? (int)(page1 - page0) : 1;          // waves that had a page
+    if (wave > 0 && wave < busy) {
         float* mine = join_lds + (size_t)(wave - 1) * kFloats * 64 + lane;
         s.put([&](int i, float v) { mine[i * 64] = v; });
     }
@@ -336,9 +365,13 @@ __global__ __launch_bounds__(256, 1) void pair_rows_kernel(PairArgs p) {
     if (wave > 0) return;
 #pragma unroll
     for (int w = 0; w < 3; ++w) {
+        if (w + 1 >= busy) break;
         const float* other = join_lds + (size_t)w * kFloats * 64 + lane;
         s.join([&](int i) { return other[i * 64]; });
     }
+#pragma unroll
+    for (int j = 0; j < (M == 1 ? DVT : 1); ++j) asm volatile("" ::"v"(gates[j]));
+    asm volatile("" ::"v"(sink));
     if (a.splits == 1u) {
         s.finish(p, 0, row, head, live, g);
         return;
