@@ -569,6 +569,27 @@ int m40llm_ext_batched_wide_gemm_residual_onto_zero_async(M40llmCudaContext* ctx
 int m40llm_ext_batched_wide_norm_gemm_async(M40llmCudaContext* ctx, const void* d_x_f32, const void* d_norm_w,
                                             uint32_t norm_weight_dtype, float eps, const void* d_w_f16, void* d_out_f32,
                                             uint32_t rows, int N, int K);
+/* The O and the down projection of up to 32 rows whose producer leaves them as matrix operands (f16 hi + lo parts, a power-of-two scale per eight
+ * elements) in a buffer of m40llm_ext_packed_rows_bytes(rows, K) bytes, 16-byte aligned; rows is the same in the call that writes the buffer and the one that
+ * reads it, and rows that the attention skips are left as they are.  K (q_heads * head_dim, ffn) a multiple of 256.  The feed-forward call takes more than eight
+ * rows of d_model a multiple of 256, or up to eight rows of d_model 2048 (..._supported: 1 / 0).  ..._onto_zero: out HOLDS ZEROS stored by an
+ * earlier call on the decode stream and lies apart from the buffer and the residual.  -6 otherwise, nothing enqueued. */
+size_t m40llm_ext_packed_rows_bytes(uint32_t rows, int K);
+int m40llm_ext_batched_packed_supported(uint32_t rows, int d_model);
+int m40llm_ext_batched_norm_qkv_rope_append_clear_async(
+    M40llmCudaContext* ctx, M40llmKVCache* kv, const uint32_t* seq_ids_dev, const uint32_t* seq_lens_dev, uint32_t rows,
+    const void* d_x_f32, const void* d_norm_w, uint32_t norm_weight_dtype, float eps, const void* d_wq_f16,
+    const void* d_wk_f16, const void* d_wv_f16, const void* d_bq_f32, const void* d_bk_f32, const void* d_bv_f32,
+    uint32_t d_model, uint32_t q_heads, float freq_base, float freq_scale, uint32_t rope_layout, void* d_q_out_f32,
+    void* d_clear_f32, uint32_t clear_floats);
+int m40llm_ext_attention_last_token_f32_gqa_batched_lens_dev_packed_async(M40llmCudaContext* ctx, const M40llmKVCache* kv, const uint32_t* seq_ids_dev,
+                                                                          const uint32_t* seq_lens_dev, uint32_t len_bias, uint32_t batch_size,
+                                                                          uint32_t max_len_hint, const void* q_dev_f32, uint32_t q_heads, void* packed_dev);
+int m40llm_ext_batched_norm_gate_up_swiglu_packed_async(M40llmCudaContext* ctx, const void* d_x_f32, const void* d_norm_w, uint32_t norm_weight_dtype, float eps,
+                                                        const void* d_wgate_f16, const void* d_wup_f16, void* d_packed, uint32_t rows, int ffn, int d_model,
+                                                        void* d_clear_f32, uint32_t clear_floats);
+int m40llm_ext_batched_packed_gemm_residual_onto_zero_async(M40llmCudaContext* ctx, const void* d_packed, const void* d_w_f16, const void* d_residual_f32,
+                                                            void* d_out_f32, uint32_t rows, int N, int K);
 /*   per row: first index of the maximum of logits[row][n] and the top-1/top-2 gap -> ids_dev/gaps_dev[row][step of the
  *   row] (row stride = capacity); seq_lens_dev[row] += 1; embedding row of the pick -> d_x_out_f32[row].
  *   state_dev = {unused, capacity, step of row 0, step of row 1, ...} */

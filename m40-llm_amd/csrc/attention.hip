@@ -204,7 +204,7 @@ __global__ __launch_bounds__(kAttnThreads, 2) void attn_partial_kernel(AttnParam
         const uint32_t qh = qh0 + h;
         if (final_out) {
             const float denom = l > 0.0f ? l : 1.0f;
-            p.Out[((size_t)b * p.q_heads + qh) * HD + d] = v / denom;
+            m40_attn_store<HD>(p, b, qh, d, v / denom);
         } else {
             float* w = p.ws + (((size_t)b * p.q_heads + qh) * p.nchunks + blockIdx.y) * (HD + 2);
             w[2 + d] = v;
@@ -276,7 +276,7 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(AttnParams p) {
             m = nm;
         }
         den = den > 0.0f ? den : 1.0f;
-        p.Out[((size_t)b * p.q_heads + qh) * HD + d] = num / den;
+        m40_attn_store<HD>(p, b, qh, d, num / den);
     }
 }
 
@@ -417,6 +417,7 @@ int m40_launch_dense_attention(M40llmCudaContext* ctx, hipStream_t stream, uint3
                                const M40AttnArgs& a) {
     AttnParams p{};
     p.K = a.K; p.V = a.V; p.Q = a.Q; p.Out = a.Out;
+    p.packed = a.packed; p.packed_pad = (uint32_t)m40_packed_pad((int)a.batch);
     p.seq_ids_dev = a.seq_ids_dev; p.seq_lens_dev = a.seq_lens_dev;
     p.seq_id = a.seq_id; p.seq_len = a.seq_len;
     p.max_seq_len = a.max_seq_len; p.kv_heads = a.kv_heads; p.q_heads = a.q_heads; p.window = a.window;
@@ -439,6 +440,7 @@ int m40_launch_dense_attention(M40llmCudaContext* ctx, hipStream_t stream, uint3
                                         : launch_hd<128>(ctx, stream, partial, partial_bytes, fixed, p, a.batch, group, span);
         if (rc != 0) return rc;
     } else {
+        if (a.packed) return -6;
         p.chunk = span; p.nchunks = 1;
         dim3 grid((a.head_dim + 63) / 64, a.q_heads, a.batch);
         attn_generic_kernel<<<grid, 64, 0, stream>>>(p, a.head_dim);
@@ -655,13 +657,9 @@ static int batched_impl(M40llmCudaContext* ctx, const M40llmKVCache* kv, const u
 
 // Row-batched attention whose ids / lengths stay on the device: nothing is copied back for validation; rows whose
 // id or length (+ len_bias) is out of range are skipped by the kernel.  max_len_hint bounds every row's length.
-int m40llm_ext_attention_last_token_f32_gqa_batched_lens_dev_async(M40llmCudaContext* ctx, const M40llmKVCache* kv,
-                                                                   const uint32_t* seq_ids_dev,
-                                                                   const uint32_t* seq_lens_dev, uint32_t len_bias,
-                                                                   uint32_t batch_size, uint32_t max_len_hint,
-                                                                   const void* q_dev_f32, uint32_t q_heads,
-                                                                   void* out_dev_f32) {
-    if (!ctx || !kv || !seq_ids_dev || !seq_lens_dev || !q_dev_f32 || !out_dev_f32) return -1;
+static int batched_lens_dev(M40llmCudaContext* ctx, const M40llmKVCache* kv, const uint32_t* seq_ids_dev, const uint32_t* seq_lens_dev, uint32_t len_bias,
+                            uint32_t batch_size, uint32_t max_len_hint, const void* q_dev_f32, uint32_t q_heads, void* out_dev_f32, void* packed_dev) {
+    if (!ctx || !kv || !seq_ids_dev || !seq_lens_dev || !q_dev_f32 || (!out_dev_f32 && !packed_dev)) return -1;
     if (batch_size == 0) return -2;
     if (q_heads == 0 || kv->num_heads == 0 || q_heads % kv->num_heads != 0) return -3;
     if (kv->head_dim != 64 && kv->head_dim != 128) return -6;
@@ -671,9 +669,27 @@ int m40llm_ext_attention_last_token_f32_gqa_batched_lens_dev_async(M40llmCudaCon
     a.K = kv->d_k; a.V = kv->d_v; a.max_seq_len = kv->max_seq_len; a.kv_heads = kv->num_heads;
     a.head_dim = kv->head_dim; a.q_heads = q_heads; a.Q = static_cast<const float*>(q_dev_f32);
     a.Out = static_cast<float*>(out_dev_f32); a.batch = batch_size;
+    a.packed = static_cast<uint8_t*>(packed_dev);
     a.seq_ids_dev = seq_ids_dev; a.seq_lens_dev = seq_lens_dev; a.len_bias = len_bias; a.max_len_hint = max_len_hint;
     a.max_batch = kv->max_batch_size;
     return m40_launch_dense_attention(ctx, ctx->decode_stream, 1, a) == 0 ? 0 : -4;
+}
+
+int m40llm_ext_attention_last_token_f32_gqa_batched_lens_dev_async(M40llmCudaContext* ctx, const M40llmKVCache* kv,
+                                                                   const uint32_t* seq_ids_dev,
+                                                                   const uint32_t* seq_lens_dev, uint32_t len_bias,
+                                                                   uint32_t batch_size, uint32_t max_len_hint,
+                                                                   const void* q_dev_f32, uint32_t q_heads,
+                                                                   void* out_dev_f32) {
+    return batched_lens_dev(ctx, kv, seq_ids_dev, seq_lens_dev, len_bias, batch_size, max_len_hint, q_dev_f32, q_heads, out_dev_f32, nullptr);
+}
+
+int m40llm_ext_attention_last_token_f32_gqa_batched_lens_dev_packed_async(M40llmCudaContext* ctx, const M40llmKVCache* kv, const uint32_t* seq_ids_dev,
+                                                                          const uint32_t* seq_lens_dev, uint32_t len_bias, uint32_t batch_size,
+                                                                          uint32_t max_len_hint, const void* q_dev_f32, uint32_t q_heads, void* packed_dev) {
+    if (!packed_dev) return -1;
+    if (batch_size > 32 || !m40_aligned16(packed_dev)) return -6;
+    return batched_lens_dev(ctx, kv, seq_ids_dev, seq_lens_dev, len_bias, batch_size, max_len_hint, q_dev_f32, q_heads, nullptr, packed_dev);
 }
 
 int m40llm_attention_last_token_f32_gqa_batched(M40llmCudaContext* ctx, const M40llmKVCache* kv,

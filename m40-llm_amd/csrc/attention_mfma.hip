@@ -245,7 +245,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_mfma_kernel(AttnParams p) {
         }
         const uint32_t qh = qh0 + h;
         if (final_out) {
-            p.Out[((size_t)b * p.q_heads + qh) * HD + d] = num / (den > 0.0f ? den : 1.0f);
+            m40_attn_store<HD>(p, b, qh, d, num / (den > 0.0f ? den : 1.0f));
         } else {
             float* w = p.ws + (((size_t)b * p.q_heads + qh) * p.nchunks + blockIdx.y) * (HD + 2);
             w[2 + d] = num;

@@ -140,7 +140,7 @@ int m40_rows_norm_qkv(M40llmCudaContext* ctx, hipStream_t stream, const M40llmKV
 float4* m40_rope_cs_cache(M40llmCudaContext* ctx, const float* table);
 bool m40_rows_mfma_supported(int rows, int K);
 int m40_rows_mfma_swiglu(M40llmCudaContext* ctx, hipStream_t stream, const float* x, const void* norm_w, uint32_t norm_dtype,
-                         float eps, const uint16_t* wgate, const uint16_t* wup, float* out, int rows, int ffn, int K,
+                         float eps, const uint16_t* wgate, const uint16_t* wup, float* out, uint8_t* packed, int rows, int ffn, int K,
                          float* zero = nullptr, int zero_count = 0);
 // rows_khalf_mfma.hip: up to eight rows against [N][K] with a long K in one launch: tiles x two halves of K, each
 // workgroup adding its sums (the first half's with the residual) into a result that an earlier launch has cleared
@@ -155,7 +155,7 @@ int m40_rows_mfma_qkv(M40llmCudaContext* ctx, hipStream_t stream, const M40llmKV
                       const uint32_t* lens_dev, uint32_t rows, const float* x, const void* norm_w, uint32_t norm_dtype, float eps,
                       const uint16_t* wq, const uint16_t* wk, const uint16_t* wv, const float* bq, const float* bk,
                       const float* bv, uint32_t d_model, uint32_t q_heads, float rope_base, float rope_scale,
-                      uint32_t rope_layout, float* q_out);
+                      uint32_t rope_layout, float* q_out, float* zero, int zero_count);
 // the projections for 9 to 32 rows, K a multiple of 256 (rows_wide_mfma.hip); zero: zero_count floats cleared on the side.  -6 also where
 // what a launch writes overlaps rows that it reads (a residual may be the result itself)
 bool m40_rows_wide_supported(int rows, int K);
@@ -164,7 +164,7 @@ int m40_rows_wide_qkv(M40llmCudaContext* ctx, hipStream_t stream, const M40llmKV
                       const uint16_t* wv, const float* bq, const float* bk, const float* bv, uint32_t d_model, uint32_t q_heads, float rope_base,
                       float rope_scale, uint32_t rope_layout, float* q_out, float* zero, int zero_count);
 int m40_rows_wide_swiglu(M40llmCudaContext* ctx, hipStream_t stream, const float* x, const void* norm_w, uint32_t norm_dtype, float eps,
-                         const uint16_t* wgate, const uint16_t* wup, float* out, int rows, int ffn, int K, float* zero, int zero_count);
+                         const uint16_t* wgate, const uint16_t* wup, float* out, uint8_t* packed, int rows, int ffn, int K, float* zero, int zero_count);
 int m40_rows_wide_norm(M40llmCudaContext* ctx, hipStream_t stream, const float* x, const void* norm_w, uint32_t norm_dtype, float eps,
                        const uint16_t* W, float* out, int rows, int N, int K);
 int m40_rows_wide_residual(M40llmCudaContext* ctx, hipStream_t stream, const float* x, const uint16_t* W, const float* residual, float* out, int rows,
@@ -202,6 +202,7 @@ struct M40AttnArgs {
     uint32_t max_seq_len, kv_heads, head_dim, q_heads;
     const float* Q;          // [batch][q_heads][hd]
     float* Out;
+    uint8_t* packed;         // not null: the result goes here as operands of the next product (packed_rows.hpp) instead of to Out
     uint32_t batch;
     // one of: fixed (seq_id, seq_len) for batch==1, or device arrays
     uint32_t seq_id, seq_len;

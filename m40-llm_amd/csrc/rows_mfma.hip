@@ -23,7 +23,7 @@
 //
 // Reference semantics: RMSNorm cuda/kernels.cu:770-807, f32 x f16 GGUF product :5037-5052, SwiGLU :869-880; call
 // order of the batched layer src/infer/forward.rs:1831-2136.
-#include "common.hpp"
+#include "packed_rows.hpp"
 
 #include <type_traits>
 
@@ -72,6 +72,7 @@ struct RowsMfmaArgs {
     const uint16_t* W0;        // [N][K]
     const uint16_t* W1;        // SwiGLU: the up matrix
     float* out;                // [rows][N]
+    uint8_t* packed;           // SwiGLU: not null, the result goes here as operands of the next product instead (N a multiple of 8)
     int rows, N, units;        // units: 16-column tiles (plain) or 8-column gate/up tiles (SwiGLU)
     float* zero;               // not null: zero_count floats the launch clears on the side (the result of a following
     int zero_count;            // product whose two K halves are added into it)
@@ -367,6 +368,10 @@ __global__ __launch_bounds__(64 * WAVES, 1) void rows_mfma_kernel(const float* x
         if (SWIGLU) {
             const float up = tile_sum(parity, e_lane + 8) * s;
             v = v / (1.0f + expf(-v)) * up;
+            if (p.packed) {
+                m40_store_packed(p.packed, kRows, N, e_row, col, v);
+                return;
+            }
         }
         p.out[(size_t)e_row * N + col] = v;
     };
@@ -418,12 +423,12 @@ int launch(M40llmCudaContext* ctx, hipStream_t stream, const RowsMfmaArgs& a) {
 bool m40_rows_mfma_supported(int rows, int K) { return rows >= 1 && rows <= kRows && K == kK; }
 
 int m40_rows_mfma_swiglu(M40llmCudaContext* ctx, hipStream_t stream, const float* x, const void* norm_w, uint32_t norm_dtype,
-                         float eps, const uint16_t* wgate, const uint16_t* wup, float* out, int rows, int ffn, int K,
+                         float eps, const uint16_t* wgate, const uint16_t* wup, float* out, uint8_t* packed, int rows, int ffn, int K,
                          float* zero, int zero_count) {
-    if (!m40_rows_mfma_supported(rows, K) || ffn <= 0) return -6;
+    if (!m40_rows_mfma_supported(rows, K) || ffn <= 0 || (packed && ffn % 8 != 0)) return -6;
     if (!m40_aligned16(x) || !m40_aligned16(wgate) || !m40_aligned16(wup) || (norm_w && !m40_aligned16(norm_w))) return -6;
     RowsMfmaArgs a{};
-    a.x = x; a.norm_w = norm_w; a.norm_dtype = norm_dtype; a.eps = eps; a.W0 = wgate; a.W1 = wup; a.out = out;
+    a.x = x; a.norm_w = norm_w; a.norm_dtype = norm_dtype; a.eps = eps; a.W0 = wgate; a.W1 = wup; a.out = out; a.packed = packed;
     a.rows = rows; a.N = ffn; a.units = (ffn + 7) / 8;
     a.zero = zero; a.zero_count = zero_count;
     return launch<1>(ctx, stream, a);
@@ -446,7 +451,7 @@ int m40_rows_mfma_qkv(M40llmCudaContext* ctx, hipStream_t stream, const M40llmKV
                       const uint32_t* lens_dev, uint32_t rows, const float* x, const void* norm_w, uint32_t norm_dtype, float eps,
                       const uint16_t* wq, const uint16_t* wk, const uint16_t* wv, const float* bq, const float* bk,
                       const float* bv, uint32_t d_model, uint32_t q_heads, float rope_base, float rope_scale,
-                      uint32_t rope_layout, float* q_out) {
+                      uint32_t rope_layout, float* q_out, float* zero, int zero_count) {
     if (!m40_rows_mfma_qkv_supported((int)rows, (int)d_model, kv->head_dim)) return -6;
     // one tile per workgroup: the rotation angle of a thread's element is computed once, ahead of the product
     if ((int)((q_heads + 2u * kv->num_heads) * kv->head_dim / 16u) > ctx->num_cus) return -6;
@@ -460,5 +465,6 @@ int m40_rows_mfma_qkv(M40llmCudaContext* ctx, hipStream_t stream, const M40llmKV
     a.head_dim = kv->head_dim; a.rope_layout = rope_layout; a.rope_base = rope_base; a.rope_scale = rope_scale;
     a.rows = (int)rows; a.N = (int)((q_heads + 2u * kv->num_heads) * kv->head_dim);
     a.units = a.N / 16;
+    a.zero = zero; a.zero_count = zero_count;
     return launch<2>(ctx, stream, a);
 }

@@ -18,7 +18,7 @@
 // 31.4 -> 30.5.  Weight loads are whole 128-byte lines (eight lanes a column) and pass through a wave-private LDS tile into operand order, as in
 // rows_mfma.hip.  A product of few columns onto zeros is cut into two halves of K, which meet in the result element by element: two terms, the
 // same bits in either order.
-#include "common.hpp"
+#include "packed_rows.hpp"
 
 #include <type_traits>
 
@@ -53,6 +53,7 @@ struct WideArgs {
     float eps;
     const uint16_t *W0, *W1, *W2; // kSwiglu: gate, up; kQkv: q, k, v
     float* out;                   // [rows][N]
+    uint8_t* packed;              // kSwiglu: not null, the result goes here as operands of the next product instead (N a multiple of 8)
     const float* residual;        // kResidual: added to the product, or null
     int rows, N, K, tiles, blocks;
     float* zero;                  // cleared on the side, or null
@@ -368,6 +369,10 @@ __global__ __launch_bounds__(kThreads, 1) void rows_wide_kernel(WideArgs p) {
             if (MODE == kSwiglu) {
                 const float up = sum(t, r, col_in + 8) * factor_s[r];
                 y = y / (1.0f + expf(-y)) * up;
+                if (p.packed) {
+                    m40_store_packed(p.packed, 16 * RT, p.N, r, col, y);
+                    continue;
+                }
             }
             float* dst = p.out + (size_t)r * p.N + col;
             if (MODE == kResidual) {
@@ -468,13 +473,13 @@ int m40_rows_wide_qkv(M40llmCudaContext* ctx, hipStream_t stream, const M40llmKV
 }
 
 int m40_rows_wide_swiglu(M40llmCudaContext* ctx, hipStream_t stream, const float* x, const void* norm_w, uint32_t norm_dtype, float eps,
-                         const uint16_t* wgate, const uint16_t* wup, float* out, int rows, int ffn, int K, float* zero, int zero_count) {
-    if (!m40_rows_wide_supported(rows, K) || ffn <= 0) return -6;
+                         const uint16_t* wgate, const uint16_t* wup, float* out, uint8_t* packed, int rows, int ffn, int K, float* zero, int zero_count) {
+    if (!m40_rows_wide_supported(rows, K) || ffn <= 0 || (packed && (rows <= 8 || ffn % 8 != 0))) return -6;
     if (!m40_aligned16(x) || !m40_aligned16(norm_w) || !m40_aligned16(wgate) || !m40_aligned16(wup)) return -6;
     WideArgs a{};
-    a.x = x; a.norm_w = norm_w; a.norm_dtype = norm_dtype; a.eps = eps; a.W0 = wgate; a.W1 = wup; a.out = out;
+    a.x = x; a.norm_w = norm_w; a.norm_dtype = norm_dtype; a.eps = eps; a.W0 = wgate; a.W1 = wup; a.out = out; a.packed = packed;
     a.rows = rows; a.N = ffn; a.K = K; a.tiles = (ffn + 7) / 8; a.zero = zero; a.zero_count = zero_count;
-    if (!rows_untouched(a, out, ffn)) return -6;
+    if (!packed && !rows_untouched(a, out, ffn)) return -6;
     return launch<kSwiglu>(ctx, stream, a);
 }
 
@@ -528,7 +533,7 @@ int m40llm_ext_batched_wide_norm_gate_up_swiglu_async(M40llmCudaContext* ctx, co
     if (norm_weight_dtype > 1) return -4;
     (void)hipGetLastError();
     return m40_rows_wide_swiglu(ctx, ctx->decode_stream, static_cast<const float*>(d_x_f32), d_norm_w, norm_weight_dtype, eps,
-                                static_cast<const uint16_t*>(d_wgate_f16), static_cast<const uint16_t*>(d_wup_f16), static_cast<float*>(d_hid_f32),
+                                static_cast<const uint16_t*>(d_wgate_f16), static_cast<const uint16_t*>(d_wup_f16), static_cast<float*>(d_hid_f32), nullptr,
                                 (int)rows, ffn, d_model, clear_floats ? static_cast<float*>(d_clear_f32) : nullptr, (int)clear_floats);
 }
 

@@ -762,10 +762,22 @@ int m40llm_ext_batched_norm_qkv_rope_append_async(
     const void* d_x_f32, const void* d_norm_w, uint32_t norm_weight_dtype, float eps, const void* d_wq_f16,
     const void* d_wk_f16, const void* d_wv_f16, const void* d_bq_f32, const void* d_bk_f32, const void* d_bv_f32,
     uint32_t d_model, uint32_t q_heads, float freq_base, float freq_scale, uint32_t rope_layout, void* d_q_out_f32) {
+    return m40llm_ext_batched_norm_qkv_rope_append_clear_async(ctx, kv, seq_ids_dev, seq_lens_dev, rows, d_x_f32, d_norm_w, norm_weight_dtype, eps, d_wq_f16,
+                                                               d_wk_f16, d_wv_f16, d_bq_f32, d_bk_f32, d_bv_f32, d_model, q_heads, freq_base, freq_scale,
+                                                               rope_layout, d_q_out_f32, nullptr, 0);
+}
+
+int m40llm_ext_batched_norm_qkv_rope_append_clear_async(
+    M40llmCudaContext* ctx, M40llmKVCache* kv, const uint32_t* seq_ids_dev, const uint32_t* seq_lens_dev, uint32_t rows,
+    const void* d_x_f32, const void* d_norm_w, uint32_t norm_weight_dtype, float eps, const void* d_wq_f16,
+    const void* d_wk_f16, const void* d_wv_f16, const void* d_bq_f32, const void* d_bk_f32, const void* d_bv_f32,
+    uint32_t d_model, uint32_t q_heads, float freq_base, float freq_scale, uint32_t rope_layout, void* d_q_out_f32,
+    void* d_clear_f32, uint32_t clear_floats) {
     if (!ctx || !kv || !seq_ids_dev || !seq_lens_dev || !d_x_f32 || !d_norm_w || !d_wq_f16 || !d_wk_f16 || !d_wv_f16 ||
         !d_q_out_f32)
         return -1;
-    if (kv->compressed || !kv->d_k || !kv->d_v) return -2;
+    if (!d_clear_f32) clear_floats = 0;
+    if (kv->compressed || !kv->d_k || !kv->d_v || clear_floats > (1u << 30)) return -2;
     if (norm_weight_dtype > 1) return -4;
     if (kv->head_dim == 0 || kv->head_dim % 2 != 0 || kv->num_heads == 0 || q_heads == 0) return -3;
     if (!rows_ok(ctx, (int)rows, (int)d_model)) return -6;
@@ -779,7 +791,9 @@ int m40llm_ext_batched_norm_qkv_rope_append_async(
                                  static_cast<const uint16_t*>(d_wk_f16), static_cast<const uint16_t*>(d_wv_f16),
                                  static_cast<const float*>(d_bq_f32), static_cast<const float*>(d_bk_f32),
                                  static_cast<const float*>(d_bv_f32), d_model, q_heads, freq_base, freq_scale, rope_layout,
-                                 static_cast<float*>(d_q_out_f32));
+                                 static_cast<float*>(d_q_out_f32),
+                                 clear_floats ? static_cast<float*>(d_clear_f32) : nullptr, (int)clear_floats);
+    if (clear_floats && m40_zero_f32(ctx->decode_stream, static_cast<float*>(d_clear_f32), clear_floats) != 0) return -7;
     // nine rows and more: one launch as well, K in chunks; a result that overlaps the rows takes the two launches below, here and in the other calls
     if (rows > 8 && kv->head_dim % 16 == 0 && m40_aligned16(d_x_f32) && m40_aligned16(d_norm_w) &&
         m40_apart(d_x_f32, (size_t)rows * d_model * 4, d_q_out_f32, (size_t)rows * q_heads * kv->head_dim * 4))
@@ -881,14 +895,14 @@ int m40llm_ext_batched_norm_gate_up_swiglu_clear_async(M40llmCudaContext* ctx, c
     if (m40_rows_mfma_supported((int)rows, d_model) && m40_aligned16(d_x_f32) && m40_aligned16(d_norm_w))
         return m40_rows_mfma_swiglu(ctx, ctx->decode_stream, static_cast<const float*>(d_x_f32), d_norm_w, norm_weight_dtype,
                                     eps, static_cast<const uint16_t*>(d_wgate_f16), static_cast<const uint16_t*>(d_wup_f16),
-                                    static_cast<float*>(d_hid_f32), (int)rows, ffn, d_model,
+                                    static_cast<float*>(d_hid_f32), nullptr, (int)rows, ffn, d_model,
                                     clear_floats ? static_cast<float*>(d_clear_f32) : nullptr, (int)clear_floats);
     const size_t x_bytes = (size_t)rows * d_model * 4, hid_bytes = (size_t)rows * ffn * 4, clear_bytes = (size_t)clear_floats * 4;
     if (rows > 8 && m40_aligned16(d_x_f32) && m40_aligned16(d_norm_w) && m40_apart(d_x_f32, x_bytes, d_hid_f32, hid_bytes) &&
         (!clear_floats || (m40_apart(d_x_f32, x_bytes, d_clear_f32, clear_bytes) && m40_apart(d_hid_f32, hid_bytes, d_clear_f32, clear_bytes))))
         return m40_rows_wide_swiglu(ctx, ctx->decode_stream, static_cast<const float*>(d_x_f32), d_norm_w, norm_weight_dtype, eps,
                                     static_cast<const uint16_t*>(d_wgate_f16), static_cast<const uint16_t*>(d_wup_f16),
-                                    static_cast<float*>(d_hid_f32), (int)rows, ffn, d_model,
+                                    static_cast<float*>(d_hid_f32), nullptr, (int)rows, ffn, d_model,
                                     clear_floats ? static_cast<float*>(d_clear_f32) : nullptr, (int)clear_floats);
     if (clear_floats && m40_zero_f32(ctx->decode_stream, static_cast<float*>(d_clear_f32), clear_floats) != 0) return -7;
     PackSpec pk{static_cast<const float*>(d_x_f32), nullptr, d_norm_w, norm_weight_dtype, eps};

@@ -123,7 +123,7 @@ private:
 struct ForwardWorkspace {
     uint32_t rows = 0;
     uint32_t generation = 0;   // bumped whenever the buffers are reallocated: captured graphs hold their addresses
-    DeviceBuf xn, q, k, v, ctx_out, y_attn, x1, x1n, gate, up, hid, y_mlp, scratch_a, scratch_b, norm_hidden, logits;
+    DeviceBuf xn, q, k, v, ctx_out, y_attn, x1, x1n, gate, up, hid, y_mlp, scratch_a, scratch_b, norm_hidden, logits, packed;
     DeviceBuf argmax_idx, argmax_gap, positions;
     void ensure(M40llmCudaContext* c, const ModelConfig& m, uint32_t want_rows) {
         if (want_rows <= rows) return;
@@ -134,6 +134,8 @@ struct ForwardWorkspace {
         hid = DeviceBuf(c, R * F * 4); y_mlp = DeviceBuf(c, R * D * 4); scratch_a = DeviceBuf(c, R * D * 4);
         scratch_b = DeviceBuf(c, R * D * 4); norm_hidden = DeviceBuf(c, R * D * 4);
         logits = DeviceBuf(c, R * (size_t)m.vocab * 4);
+        const uint32_t fused = want_rows < 32 ? want_rows : 32;
+        packed = DeviceBuf(c, std::max({m40llm_ext_packed_rows_bytes(fused, (int)D), m40llm_ext_packed_rows_bytes(fused, (int)F), (size_t)16}));
         argmax_idx = DeviceBuf(c, R * 4); argmax_gap = DeviceBuf(c, R * 4); positions = DeviceBuf(c, R * 4 * 2);
         rows = want_rows;
         ++generation;
@@ -733,17 +735,18 @@ public:
                              const float* d_x, float* d_out) {
         const LayerWeights& w = layers_[l];
         const uint32_t D = cfg_.d_model, F = cfg_.ffn;
-        if (rows > kNarrowRows) {
-            // x1 and d_out are dead until the O and the down projection write them: the launches before clear them on the side
-            M40H_TRY(m40llm_ext_batched_wide_norm_qkv_rope_append_async(ctx_, kv_, slots_dev, lens_dev, rows, d_x, w.attn_norm, cfg_.norm_weight_dtype,
-                                                                        cfg_.rms_eps, w.wq, w.wk, w.wv, w.bq, w.bk, w.bv, D, cfg_.q_heads, cfg_.rope_base,
-                                                                        cfg_.rope_scale, cfg_.rope_layout, ws_.q.ptr(), ws_.x1.ptr(), rows * D));
-            M40H_TRY(m40llm_ext_attention_last_token_f32_gqa_batched_lens_dev_async(ctx_, kv_, slots_dev, lens_dev, 1, rows, hint, ws_.q.ptr(),
-                                                                                    cfg_.q_heads, ws_.ctx_out.ptr()));
-            M40H_TRY(m40llm_ext_batched_wide_gemm_residual_onto_zero_async(ctx_, ws_.ctx_out.ptr(), w.wo, d_x, ws_.x1.ptr(), rows, (int)D, (int)D));
-            M40H_TRY(m40llm_ext_batched_wide_norm_gate_up_swiglu_async(ctx_, ws_.x1.ptr(), w.ffn_norm, cfg_.norm_weight_dtype, cfg_.rms_eps, w.wgate,
-                                                                       w.wup, ws_.hid.ptr(), rows, (int)F, (int)D, d_out, rows * D));
-            M40H_TRY(m40llm_ext_batched_wide_gemm_residual_onto_zero_async(ctx_, ws_.hid.ptr(), w.wdown, ws_.x1.ptr(), d_out, rows, (int)D, (int)F));
+        // The attention's and the feed-forward's rows are what the O and the down projection multiply: they are left as operands.  x1 and d_out
+        // are dead until those write them: the launches before clear them on the side, and two halves of K meet in them.
+        if (m40llm_ext_batched_packed_supported(rows, (int)D)) {
+            const auto qkv = rows > kNarrowRows ? m40llm_ext_batched_wide_norm_qkv_rope_append_async : m40llm_ext_batched_norm_qkv_rope_append_clear_async;
+            M40H_TRY(qkv(ctx_, kv_, slots_dev, lens_dev, rows, d_x, w.attn_norm, cfg_.norm_weight_dtype, cfg_.rms_eps, w.wq, w.wk, w.wv, w.bq, w.bk, w.bv, D,
+                         cfg_.q_heads, cfg_.rope_base, cfg_.rope_scale, cfg_.rope_layout, ws_.q.ptr(), ws_.x1.ptr(), rows * D));
+            M40H_TRY(m40llm_ext_attention_last_token_f32_gqa_batched_lens_dev_packed_async(ctx_, kv_, slots_dev, lens_dev, 1, rows, hint, ws_.q.ptr(),
+                                                                                           cfg_.q_heads, ws_.packed.ptr()));
+            M40H_TRY(m40llm_ext_batched_packed_gemm_residual_onto_zero_async(ctx_, ws_.packed.ptr(), w.wo, d_x, ws_.x1.ptr(), rows, (int)D, (int)D));
+            M40H_TRY(m40llm_ext_batched_norm_gate_up_swiglu_packed_async(ctx_, ws_.x1.ptr(), w.ffn_norm, cfg_.norm_weight_dtype, cfg_.rms_eps, w.wgate, w.wup,
+                                                                         ws_.packed.ptr(), rows, (int)F, (int)D, d_out, rows * D));
+            M40H_TRY(m40llm_ext_batched_packed_gemm_residual_onto_zero_async(ctx_, ws_.packed.ptr(), w.wdown, ws_.x1.ptr(), d_out, rows, (int)D, (int)F));
             return;
         }
         M40H_TRY(m40llm_ext_batched_norm_qkv_rope_append_async(ctx_, kv_, slots_dev, lens_dev, rows, d_x, w.attn_norm,

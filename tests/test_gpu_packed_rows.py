@@ -1,0 +1,92 @@
+"""O and down projection of rows that the launch before left as matrix operands (m40llm_ext_batched_packed_*, ..._packed_async): every padded row count, K that gives
+the waves unequal numbers of blocks, columns that end in the middle of a tile, K whole and in halves, units of zeros, against 64-bit products of the rows that the
+f32 form of the same call makes."""
+import numpy as np
+import pytest
+
+from gpu_common import Dev, close, f16bits, m40
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def dev():
+    d = Dev()
+    yield d
+    d.ctx.close()
+
+
+def _bytes(rows, K):
+    pad = 8 if rows <= 8 else (16 if rows <= 16 else 32)
+    return pad * K * 4 + pad * K // 8 * 4
+
+
+def _f64(w):
+    return w.view(np.float16).astype(np.float64)
+
+
+def _project(dev, packed, rows64, w, res, rows, N, K):
+    """Residual, no residual and the same bits twice, onto zeros; `rows64`: the rows the buffer holds."""
+    dw, dres = dev.up(w), dev.up(res)
+    want = rows64 @ _f64(w).T
+    # operands exact to 2^-22 of a unit's largest value, f32 sums of K products: a few 2^-24 of the row's largest sum of magnitudes a wave's share
+    bound = np.abs(rows64) @ np.abs(_f64(w)).T * 2.0 ** -21
+    got = []
+    for r in (res, None, res):
+        out = dev.zeros(rows * N * 4)
+        dev.call("m40llm_ext_batched_packed_gemm_residual_onto_zero_async", packed.ptr, dw.ptr, None if r is None else dres.ptr, out.ptr, rows, N, K)
+        dev.sync()
+        got.append(out.download(np.float32, (rows, N)))
+        full = want + (0.0 if r is None else r)
+        assert np.all(np.abs(got[-1] - full) <= bound + np.abs(full) * 2.0 ** -23)
+    assert np.array_equal(got[0], got[2])           # the same bits whichever half of K arrives first
+    dev.call("m40llm_ext_batched_packed_gemm_residual_onto_zero_async", packed.ptr, dw.ptr, dres.ptr, dres.ptr, rows, N, K, expect=-6)
+    dev.call("m40llm_ext_batched_packed_gemm_residual_onto_zero_async", packed.ptr, dw.ptr, dres.ptr, out.ptr, 33, N, K, expect=-6)
+    dev.call("m40llm_ext_batched_packed_gemm_residual_onto_zero_async", packed.ptr, dw.ptr, dres.ptr, out.ptr, rows, N, K - 64, expect=-6)
+
+
+@pytest.mark.parametrize("rows,F,D,N", [(1, 256, 2048, 7), (3, 5632, 2048, 2048), (8, 11008, 2048, 2048), (9, 768, 256, 2063), (16, 5632, 512, 2048), (17, 1024, 256, 4100),
+                                        (32, 2816, 2048, 2048), (25, 4864, 256, 900)])
+def test_feed_forward(dev, rows, F, D, N):
+    rng = np.random.default_rng(rows * 5 + F)
+    x = rng.standard_normal((rows, D)).astype(np.float32)
+    x[rows // 2] *= 3e3
+    x[rows - 1] *= 1e-3
+    nw = np.abs(1 + 0.1 * rng.standard_normal(D)).astype(np.float32)
+    wg, wu = (rng.standard_normal((F, D)) * 0.08 for _ in range(2))
+    wu[8:16] = 0.0                                  # a unit of zeros
+    wu[16:24] *= 1e-4                               # units of very different magnitude that meet in one instruction
+    dx, dnw, dwg, dwu = dev.up(x), dev.up(nw), dev.up(f16bits(wg)), dev.up(f16bits(wu))
+    hid, clear = dev.zeros(rows * F * 4), dev.up(np.full(rows * 99 + 3, 5.0, dtype=np.float32))
+    packed = dev.up(np.full(_bytes(rows, F), 0xFF, dtype=np.uint8))     # rows that are not there: NaN
+    plain = "m40llm_ext_batched_norm_gate_up_swiglu_clear_async" if rows <= 8 else "m40llm_ext_batched_wide_norm_gate_up_swiglu_async"
+    dev.call(plain, dx.ptr, dnw.ptr, 1, 1e-5, dwg.ptr, dwu.ptr, hid.ptr, rows, F, D, None, 0)
+    dev.call("m40llm_ext_batched_norm_gate_up_swiglu_packed_async", dx.ptr, dnw.ptr, 1, 1e-5, dwg.ptr, dwu.ptr, packed.ptr, rows, F, D, clear.ptr, rows * 99)
+    dev.sync()
+    assert np.array_equal(clear.download(np.float32, (rows * 99 + 3,)), [0.0] * (rows * 99) + [5.0] * 3)
+    w = f16bits(rng.standard_normal((N, F)) * 0.03)
+    _project(dev, packed, hid.download(np.float32, (rows, F)).astype(np.float64), w, rng.standard_normal((rows, N)).astype(np.float32), rows, N, F)
+    dev.call("m40llm_ext_batched_norm_gate_up_swiglu_packed_async", dx.ptr, dnw.ptr, 1, 1e-5, dwg.ptr, dwu.ptr, packed.ptr, rows, F - 64, D, None, 0, expect=-6)
+    dev.call("m40llm_ext_batched_norm_gate_up_swiglu_packed_async", dx.ptr, dnw.ptr, 1, 1e-5, dwg.ptr, dwu.ptr, dx.ptr, rows, F, D, None, 0, expect=-6)
+
+
+# one chunk and several, the kernel for short rows and the one on matrix instructions
+@pytest.mark.parametrize("rows,qh,kvh,hd,longest", [(2, 4, 2, 64, 60), (8, 16, 2, 128, 700), (5, 32, 4, 64, 400), (9, 8, 8, 64, 530), (17, 4, 4, 128, 40), (32, 32, 4, 64, 1000)])
+def test_attention(dev, rows, qh, kvh, hd, longest):
+    rng = np.random.default_rng(rows + longest)
+    kv = m40.KVCache(dev.ctx, 1024, rows, kvh, hd)
+    lens = rng.integers(1, longest + 1, rows).astype(np.uint32)
+    lens[0] = longest
+    for r in range(rows):
+        k, v = (f16bits(rng.standard_normal((int(lens[r]), kvh, hd))) for _ in range(2))
+        dev.fill_dense(kv, r, k, v)
+    K, N = qh * hd, 2048 if qh * hd > 512 else 130
+    q = rng.standard_normal((rows, K)).astype(np.float32)
+    dq, out, ids, dlens = dev.up(q), dev.zeros(q.nbytes), dev.up(np.arange(rows, dtype=np.uint32)), dev.up(lens)
+    packed = dev.up(np.full(_bytes(rows, K), 0xFF, dtype=np.uint8))
+    dev.call("m40llm_ext_attention_last_token_f32_gqa_batched_lens_dev_async", kv.h, ids.ptr, dlens.ptr, 0, rows, longest, dq.ptr, qh, out.ptr)
+    dev.call("m40llm_ext_attention_last_token_f32_gqa_batched_lens_dev_packed_async", kv.h, ids.ptr, dlens.ptr, 0, rows, longest, dq.ptr, qh, packed.ptr)
+    dev.sync()
+    w = f16bits(rng.standard_normal((N, K)) * 0.03)
+    _project(dev, packed, out.download(np.float32, (rows, K)).astype(np.float64), w, rng.standard_normal((rows, N)).astype(np.float32), rows, N, K)
+    kv.destroy()
