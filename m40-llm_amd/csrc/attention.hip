@@ -60,8 +60,9 @@ constexpr int kAttnThreads = 512;
 constexpr int kWaves = kAttnThreads / 64;
 
 
-// HD in {64, 128}; G = q heads per workgroup (<= 4); S = token rows per lane group
-template <int HD, int G, int S>
+// HD in {64, 128}; G = q heads per workgroup (<= 4); S = token rows per lane group; PACKED: the result as operands (a launch of one short row has no time to look
+// it up: 4.35 us instead of 4.29)
+template <int HD, int G, int S, bool PACKED>
 __global__ __launch_bounds__(kAttnThreads, 2) void attn_partial_kernel(AttnParams p) {
     constexpr int LPT = HD / 8;      // lanes per token row
     constexpr int TPW = 64 / LPT;    // token rows per wave load
@@ -204,79 +205,77 @@ __global__ __launch_bounds__(kAttnThreads, 2) void attn_partial_kernel(AttnParam
         const uint32_t qh = qh0 + h;
         if (final_out) {
             const float denom = l > 0.0f ? l : 1.0f;
-            m40_attn_store<HD>(p, b, qh, d, v / denom);
+            if constexpr (PACKED) m40_attn_store<HD>(p, b, qh, d, v / denom);
+            else p.Out[((size_t)b * p.q_heads + qh) * HD + d] = v / denom;
         } else {
-            float* w = p.ws + (((size_t)b * p.q_heads + qh) * p.nchunks + blockIdx.y) * (HD + 2);
-            w[2 + d] = v;
-            if (d == 0) {
-                w[0] = mh[h];
-                w[1] = l;
-            }
+            const size_t at = ((size_t)b * p.q_heads + qh) * p.nchunks + blockIdx.y;
+            p.ws[at * HD + d] = v;
+            if (d == 0) reinterpret_cast<float2*>(p.ml)[at] = make_float2(mh[h], l);
         }
     }
 }
 
-// Merge chunk partials: grid (q_heads, batch), 256 threads = 256/HD chunk lanes x HD dims.  Each chunk lane
-// folds chunks lane, lane + n_lanes, ... with a running maximum; the chunk lanes are then folded in order.
+// Merge chunk partials: grid (q_heads, batch), 256 threads.  HD / 4 lanes take a chunk's sums, four columns each; the chunks go round the 1024 / HD such groups.
+//
+// Bound by its round trips to memory: everything of the first 64 chunks -- sums, maxima, denominators, the row's length and id -- is asked for at once, before
+// anything is known; partials of chunks past the row's end are stale values inside the buffer and are left out.  Every wave forms all weights itself, one
+// lane a chunk, so that the waves meet once, with their sums.  (Folding the chunks one after the other under a running maximum, 256 / HD of them side by side:
+// the two launches of 8 rows of up to 4093 tokens, head size 128, 13.3 us, now 12.6; 32 rows of up to 1021, 64, 11.8 / 11.3; 2 rows of up to 3000 10.3 / 8.9; one of
+// 16000, 125 chunks, 19.6 / 11.8.)
 template <int HD>
-__global__ __launch_bounds__(256) void attn_combine_kernel(AttnParams p) {
-    constexpr int NCG = 256 / HD;
-    __shared__ float s_m[NCG], s_den[NCG];
-    __shared__ float s_num[NCG][HD];
+__global__ __launch_bounds__(256) void attn_combine_kernel(const float* ws, const float* ml, const uint32_t* seq_lens_dev, const uint32_t* seq_ids_dev, uint32_t nchunks,
+                                                           uint32_t q_heads, AttnParams p) {
+    constexpr int kLanes = HD / 4, kGroups = 256 / kLanes, kPass = 64, kEach = kPass / kGroups;
+    __shared__ __attribute__((aligned(16))) float sums[4][HD];
     const uint32_t qh = blockIdx.x, b = blockIdx.y;
-    const uint32_t d = threadIdx.x % HD, cg = threadIdx.x / HD;
-    // The lane's first kPre chunk partials are requested together with the row's length and id, before either is
-    // known (one memory round trip instead of a chain of three); partials of chunks past the row's end are stale
-    // values inside the buffer and are never used.  The chunks are folded in the same ascending order either way.
-    constexpr uint32_t kPre = 8;
-    const float* w = p.ws + (((size_t)b * p.q_heads + qh) * p.nchunks) * (HD + 2);
-    float pm[kPre], pl[kPre], pv[kPre];
+    const uint32_t tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, c4 = tid % kLanes, group = tid / kLanes;
+    const size_t first = ((size_t)b * q_heads + qh) * nchunks;
+    const float4* v_at = reinterpret_cast<const float4*>(ws + first * HD) + c4;
+    const float2* ml_at = reinterpret_cast<const float2*>(ml) + first;
+    float4 v[kEach];
+    auto load = [&](uint32_t base) {
 #pragma unroll
-    for (uint32_t u = 0; u < kPre; ++u) {
-        const uint32_t ch = cg + u * NCG;
-        const float* wc = w + (size_t)(ch < p.nchunks ? ch : 0u) * (HD + 2);
-        pm[u] = wc[0]; pl[u] = wc[1]; pv[u] = wc[2 + d];
-    }
-    const uint32_t len = p.seq_lens_dev ? p.seq_lens_dev[b] + p.len_bias : p.seq_len;
-    const uint32_t sid = (p.max_batch != 0 && p.seq_ids_dev) ? p.seq_ids_dev[b] : 0u;
+        for (int u = 0; u < kEach; ++u) {
+            const uint32_t c = base + group + u * kGroups;
+            v[u] = v_at[(size_t)(c < nchunks ? c : 0u) * kLanes];
+        }
+    };
+    const float2 ml0 = ml_at[lane < nchunks ? lane : 0u];
+    load(0);
+    const uint32_t len = seq_lens_dev ? seq_lens_dev[b] + p.len_bias : p.seq_len;
+    const uint32_t sid = (p.max_batch != 0 && seq_ids_dev) ? seq_ids_dev[b] : 0u;
     if (len == 0 || len > p.max_seq_len) return;
-    if (p.max_batch != 0 && p.seq_ids_dev && sid >= p.max_batch) return;
+    if (p.max_batch != 0 && seq_ids_dev && sid >= p.max_batch) return;
     const uint32_t t0 = (p.window != 0 && len > p.window) ? len - p.window : 0;
     if (len - t0 > p.span_limit) return;      // longer than the launch was sized for: the row is skipped
     const uint32_t n = (len - t0 + p.chunk - 1) / p.chunk;
-    float m = -INFINITY, num = 0.0f, den = 0.0f;
-    auto fold = [&](float mc, float lc, float vc) {
-        const float nm = fmaxf(m, mc);
-        const float fa = m == -INFINITY ? 0.0f : expf(m - nm);
-        const float fb = mc == -INFINITY ? 0.0f : expf(mc - nm);
-        num = fmaf(num, fa, vc * fb);
-        den = fmaf(den, fa, lc * fb);
-        m = nm;
-    };
+    float m = lane < n ? ml0.x : -INFINITY;
+    for (uint32_t c = kPass + lane; c < n; c += kPass) m = fmaxf(m, ml_at[c].x);
+    m = m40_max64(m);
+    float den = 0.0f;
+    float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (uint32_t base = 0; base < n; base += kPass) {
+        const float2 x = base == 0 ? ml0 : ml_at[base + lane < n ? base + lane : 0u];
+        if (base != 0) load(base);
+        const float f = base + lane < n && x.x != -INFINITY ? expf(x.x - m) : 0.0f;
+        den = fmaf(base + lane < n ? x.y : 0.0f, f, den);
 #pragma unroll
-    for (uint32_t u = 0; u < kPre; ++u)
-        if (cg + u * NCG < n) fold(pm[u], pl[u], pv[u]);
-#pragma unroll 4
-    for (uint32_t ch = cg + kPre * NCG; ch < n; ch += NCG) {
-        const float* wc = w + (size_t)ch * (HD + 2);
-        fold(wc[0], wc[1], wc[2 + d]);
-    }
-    s_num[cg][d] = num;
-    if (d == 0) { s_m[cg] = m; s_den[cg] = den; }
-    __syncthreads();
-    if (cg == 0) {
-#pragma unroll
-        for (int g = 1; g < NCG; ++g) {
-            const float mc = s_m[g];
-            const float nm = fmaxf(m, mc);
-            const float fa = m == -INFINITY ? 0.0f : expf(m - nm);
-            const float fb = mc == -INFINITY ? 0.0f : expf(mc - nm);
-            num = fmaf(num, fa, s_num[g][d] * fb);
-            den = fmaf(den, fa, s_den[g] * fb);
-            m = nm;
+        for (int u = 0; u < kEach; ++u) {
+            const float w = __shfl(f, (int)(group + u * kGroups), 64);
+            if (base + group + u * kGroups < n) {
+                sum.x = fmaf(v[u].x, w, sum.x); sum.y = fmaf(v[u].y, w, sum.y);
+                sum.z = fmaf(v[u].z, w, sum.z); sum.w = fmaf(v[u].w, w, sum.w);
+            }
         }
-        den = den > 0.0f ? den : 1.0f;
-        m40_attn_store<HD>(p, b, qh, d, num / den);
+    }
+    den = m40_sum64(den);
+    if (HD == 64) { sum.x = m40_add_xor16(sum.x); sum.y = m40_add_xor16(sum.y); sum.z = m40_add_xor16(sum.z); sum.w = m40_add_xor16(sum.w); }
+    sum.x = m40_add_xor32(sum.x); sum.y = m40_add_xor32(sum.y); sum.z = m40_add_xor32(sum.z); sum.w = m40_add_xor32(sum.w);
+    if (lane < kLanes) *reinterpret_cast<float4*>(&sums[wave][4 * lane]) = sum;
+    __syncthreads();
+    if (tid < HD) {
+        const float num = (sums[0][tid] + sums[1][tid]) + (sums[2][tid] + sums[3][tid]);
+        m40_attn_store<HD>(p, b, qh, tid, num / (den > 0.0f ? den : 1.0f));
     }
 }
 
@@ -318,7 +317,8 @@ __global__ __launch_bounds__(64) void attn_generic_kernel(AttnParams p, uint32_t
 template <int HD, int G, int S>
 void launch_partial(hipStream_t stream, const AttnParams& p, uint32_t batch) {
     dim3 grid(p.kv_heads * p.subgroups, p.nchunks, batch);
-    attn_partial_kernel<HD, G, S><<<grid, kAttnThreads, 0, stream>>>(p);
+    if (p.packed && p.nchunks == 1) attn_partial_kernel<HD, G, S, true><<<grid, kAttnThreads, 0, stream>>>(p);
+    else attn_partial_kernel<HD, G, S, false><<<grid, kAttnThreads, 0, stream>>>(p);
 }
 
 template <int HD, int G>
@@ -361,10 +361,11 @@ int launch_hd(M40llmCudaContext* ctx, hipStream_t stream, float* partial, size_t
             chunk *= 2;
         }
         p.ws = partial;
+        p.ml = partial + (size_t)batch * p.q_heads * p.nchunks * HD;
         m40_launch_attn_mfma(stream, p, HD, batch);
         if (p.nchunks > 1) {
             dim3 grid(p.q_heads, batch);
-            attn_combine_kernel<HD><<<grid, 256, 0, stream>>>(p);
+            attn_combine_kernel<HD><<<grid, 256, 0, stream>>>(p.ws, p.ml, p.seq_lens_dev, p.seq_ids_dev, p.nchunks, p.q_heads, p);
         }
         return 0;
     }
@@ -399,6 +400,7 @@ int launch_hd(M40llmCudaContext* ctx, hipStream_t stream, float* partial, size_t
         }
     }
     p.ws = partial;
+    p.ml = partial + (size_t)batch * p.q_heads * p.nchunks * HD;
     switch (G) {
         case 4: launch_g<HD, 4>(stream, p, batch, S); break;
         case 2: launch_g<HD, 2>(stream, p, batch, S); break;
@@ -406,7 +408,7 @@ int launch_hd(M40llmCudaContext* ctx, hipStream_t stream, float* partial, size_t
     }
     if (p.nchunks > 1) {
         dim3 grid(p.q_heads, batch);
-        attn_combine_kernel<HD><<<grid, 256, 0, stream>>>(p);
+        attn_combine_kernel<HD><<<grid, 256, 0, stream>>>(p.ws, p.ml, p.seq_lens_dev, p.seq_ids_dev, p.nchunks, p.q_heads, p);
     }
     return 0;
 }

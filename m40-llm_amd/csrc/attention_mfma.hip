@@ -6,7 +6,8 @@
 //   scores  S[h][t] = sum_d q[h][d] K[t][d]:  A = q (16 rows = up to 8 q heads x {hi, lo} f16 split), B = K rows read
 //           straight from the cache (a lane's 16 bytes are 8 consecutive d of its token);
 //   output  O[h][d] = sum_t P[h][t] V[t][d]:  A = softmax weights (hi/lo split, re-laid out through a 1 KB LDS tile),
-//           B = V, staged row-major in LDS by 16-byte global loads and read back one token column at a time.
+//           B = V, staged row-major in LDS by 16-byte global loads and read back transposed (ds_read_b64_tr_b16; gathering
+//           the sixteen-bit values of a column one by one: 8 rows of up to 4093 tokens, head size 128, 13.5 -> 13.25 us with the merge).
 // A workgroup is four waves on one kv head and one chunk of tokens; a wave walks 32-token tiles with a running
 // maximum (the rows of one head live in one 16-lane row, so the softmax state never leaves that row), the four
 // waves are merged through LDS, and chunks are merged by the same second kernel as the vector-ALU path.
@@ -25,6 +26,13 @@ __device__ __forceinline__ m40_float4 mfma16x16x32(const uint4& a, const uint4& 
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(m40_half8, a),
                                                   __builtin_bit_cast(m40_half8, b), c, 0, 0, 0);
 }
+__device__ __forceinline__ uint4 read_transposed(const uint8_t* p0, const uint8_t* p1) {
+    typedef short s16x4 __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(3))) s16x4* lds4_t;
+    const uint2 a = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4_t)(p0)));
+    const uint2 b = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4_t)(p1)));
+    return make_uint4(a.x, a.y, b.x, b.y);
+}
 __device__ __forceinline__ float max16(float x) {   // over rows of 16 lanes
     x = fmaxf(x, m40_dpp_f<M40_DPP_XOR1>(x));
     x = fmaxf(x, m40_dpp_f<M40_DPP_XOR2>(x));
@@ -34,8 +42,13 @@ __device__ __forceinline__ float max16(float x) {   // over rows of 16 lanes
 }
 __device__ __forceinline__ uint16_t f16_bits(float x) { return __builtin_bit_cast(uint16_t, static_cast<_Float16>(x)); }
 
+// What the first requests need is passed on its own, in registers when a wave starts; the structure is read from memory meanwhile.  q goes out before the row's
+// length and id are known, K and V as soon as they are, K ahead of V: scores and softmax are formed while V is on its way.  (All behind the structure, V waited for
+// ahead of the scores: 8 rows of up to 4093 tokens, head size 128, 12.6 us with the merge, now 12.5; 16 rows of up to 1200 11.9 / 11.4; 2 rows of up to 3000 8.9 / 8.8.
+// Eight waves with a tile each instead of four with two are no faster, 16 rows a quarter slower; K in whole lines through LDS neither, 12.5 -> 13.1 us.)
 template <int HD>
-__global__ __launch_bounds__(kThreads, 2) void attn_mfma_kernel(AttnParams p) {
+__global__ __launch_bounds__(kThreads, 2) void attn_mfma_kernel(const uint16_t* K, const uint16_t* V, const float* Q, const uint32_t* ids_dev, const uint32_t* lens_dev,
+                                                                 uint32_t max_seq_len, uint32_t kv_heads, uint32_t q_heads, uint32_t subgroups, uint32_t chunk, uint32_t len_bias, AttnParams p) {
     constexpr int KS = HD / 32;            // MFMA k-steps of a score tile
     constexpr int DT = HD / 16;            // 16-column output tiles
     constexpr int RS = HD * 2 + 8;         // LDS bytes per V row (8-byte aligned, spreads the row groups over the banks)
@@ -45,35 +58,47 @@ __global__ __launch_bounds__(kThreads, 2) void attn_mfma_kernel(AttnParams p) {
     __shared__ float m_s[kWaves][8], l_s[kWaves][8];
     __shared__ float o_s[kWaves][8][HD];
 
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int c16 = lane & 15, g = lane >> 4;
     const uint32_t b = blockIdx.z;
-    const uint32_t seq_id = p.seq_ids_dev ? p.seq_ids_dev[b] : p.seq_id;
-    const uint32_t len = p.seq_lens_dev ? p.seq_lens_dev[b] + p.len_bias : p.seq_len;
-    if (len == 0 || len > p.max_seq_len) return;
+    const uint32_t kvh = blockIdx.x / subgroups, sub = blockIdx.x % subgroups;
+    const uint32_t group = q_heads / kv_heads;
+    const uint32_t qh0 = kvh * group + sub * 8u;
+    const uint32_t gcount = (sub * 8u + 8u <= group) ? 8u : group - sub * 8u;
+    const float* Qb = Q + ((size_t)b * q_heads + qh0) * HD;      // gcount heads, contiguous
+    // A-operand row rho = c16: head 2*(rho/4) + (rho%4)/2, part rho&1 (0 hi, 1 lo)
+    const uint32_t qhead = 2u * (uint32_t)(c16 >> 2) + (uint32_t)((c16 & 3) >> 1);
+    const bool q_live = qhead < gcount;
+    float4 qraw[KS][2];
+    {
+        const float* qp = Qb + (size_t)(q_live ? qhead : 0u) * HD + 8 * g;
+#pragma unroll
+        for (int i = 0; i < KS; ++i) {
+            qraw[i][0] = *reinterpret_cast<const float4*>(qp + 32 * i);
+            qraw[i][1] = *reinterpret_cast<const float4*>(qp + 32 * i + 4);
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    const uint32_t seq_id = ids_dev ? ids_dev[b] : p.seq_id;
+    const uint32_t len = lens_dev ? lens_dev[b] + len_bias : p.seq_len;
+    if (len == 0 || len > max_seq_len) return;
     if (p.max_batch != 0 && seq_id >= p.max_batch) return;
     const uint32_t t0 = (p.window != 0 && len > p.window) ? len - p.window : 0;
     if (len - t0 > p.span_limit) return;      // longer than the launch was sized for: the row is skipped
-    const uint32_t cbeg = t0 + blockIdx.y * p.chunk;
+    const uint32_t cbeg = t0 + blockIdx.y * chunk;
     if (cbeg >= len) return;
-    const uint32_t cend = cbeg + p.chunk < len ? cbeg + p.chunk : len;
+    const uint32_t cend = cbeg + chunk < len ? cbeg + chunk : len;
     const uint32_t ntok = cend - cbeg;
 
-    const uint32_t kvh = blockIdx.x / p.subgroups, sub = blockIdx.x % p.subgroups;
-    const uint32_t group = p.q_heads / p.kv_heads;
-    const uint32_t qh0 = kvh * group + sub * 8u;
-    const uint32_t gcount = (sub * 8u + 8u <= group) ? 8u : group - sub * 8u;
+    const size_t row_stride = (size_t)kv_heads * HD;
+    const uint16_t* Kb = K + ((size_t)seq_id * max_seq_len) * row_stride + (size_t)kvh * HD;
+    const uint16_t* Vb = V + ((size_t)seq_id * max_seq_len) * row_stride + (size_t)kvh * HD;
 
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int c16 = lane & 15, g = lane >> 4;
-    const size_t row_stride = (size_t)p.kv_heads * HD;
-    const uint16_t* Kb = p.K + ((size_t)seq_id * p.max_seq_len) * row_stride + (size_t)kvh * HD;
-    const uint16_t* Vb = p.V + ((size_t)seq_id * p.max_seq_len) * row_stride + (size_t)kvh * HD;
-    const float* Qb = p.Q + ((size_t)b * p.q_heads + qh0) * HD;      // gcount heads, contiguous
-
-    // ---- weight loads of the first tile go out before anything else ------------------------------------
+    // ---- the first tile's loads
     uint4 kreg[2][KS], vreg[DT];
     const int my_tiles_begin = wave;
     const int ntiles = (int)((ntok + kTile - 1) / kTile);
-    auto issue = [&](int tile) {
+    auto issue_k = [&](int tile) {
 #pragma unroll
         for (int hf = 0; hf < 2; ++hf) {
             uint32_t t = cbeg + (uint32_t)(tile * kTile + 16 * hf + c16);
@@ -82,6 +107,8 @@ __global__ __launch_bounds__(kThreads, 2) void attn_mfma_kernel(AttnParams p) {
             for (int i = 0; i < KS; ++i)
                 kreg[hf][i] = *reinterpret_cast<const uint4*>(Kb + (size_t)t * row_stride + 32 * i + 8 * g);
         }
+    };
+    auto issue_v = [&](int tile) {
 #pragma unroll
         for (int k = 0; k < DT; ++k) {
             const int q = k * 64 + lane;
@@ -90,24 +117,17 @@ __global__ __launch_bounds__(kThreads, 2) void attn_mfma_kernel(AttnParams p) {
             vreg[k] = *reinterpret_cast<const uint4*>(Vb + (size_t)t * row_stride + 8 * (q % PIECES));
         }
     };
-    if (my_tiles_begin < ntiles) issue(my_tiles_begin);
+    if (my_tiles_begin < ntiles) { issue_k(my_tiles_begin); __builtin_amdgcn_sched_barrier(0); issue_v(my_tiles_begin); }
+    __builtin_amdgcn_sched_barrier(0);
 
     // ---- q fragments: power-of-two scaled, split into f16 hi + lo -----------------------------------------
-    // A-operand row rho = c16: head 2*(rho/4) + (rho%4)/2, part rho&1 (0 hi, 1 lo).  Every wave holds each q value
-    // of the group (twice: hi and lo lanes), so the largest magnitude needs no exchange between waves.  All loads
-    // go out together, behind the first tile's.
-    const uint32_t qhead = 2u * (uint32_t)(c16 >> 2) + (uint32_t)((c16 & 3) >> 1);
-    const bool q_live = qhead < gcount;
+    // Every wave holds each q value of the group (twice: hi and lo lanes), so the largest magnitude needs no exchange between waves.
     float qv[KS][8];
-    {
-        const float* qp = Qb + (size_t)(q_live ? qhead : 0u) * HD + 8 * g;
 #pragma unroll
-        for (int i = 0; i < KS; ++i) {
-            const float4 x = *reinterpret_cast<const float4*>(qp + 32 * i);
-            const float4 y = *reinterpret_cast<const float4*>(qp + 32 * i + 4);
-            qv[i][0] = x.x; qv[i][1] = x.y; qv[i][2] = x.z; qv[i][3] = x.w;
-            qv[i][4] = y.x; qv[i][5] = y.y; qv[i][6] = y.z; qv[i][7] = y.w;
-        }
+    for (int i = 0; i < KS; ++i) {
+        const float4 x = qraw[i][0], y = qraw[i][1];
+        qv[i][0] = x.x; qv[i][1] = x.y; qv[i][2] = x.z; qv[i][3] = x.w;
+        qv[i][4] = y.x; qv[i][5] = y.y; qv[i][6] = y.z; qv[i][7] = y.w;
     }
     float qmax = 0.0f;
 #pragma unroll
@@ -151,14 +171,6 @@ __global__ __launch_bounds__(kThreads, 2) void attn_mfma_kernel(AttnParams p) {
     uint8_t* my_v = v_lds[wave];
 
     for (int tile = my_tiles_begin; tile < ntiles; tile += kWaves) {
-        // V tile -> LDS (row-major, two 8-byte stores per piece)
-#pragma unroll
-        for (int k = 0; k < DT; ++k) {
-            const int q = k * 64 + lane;
-            uint2* dst = reinterpret_cast<uint2*>(my_v + (q / PIECES) * RS + 16 * (q % PIECES));
-            dst[0] = make_uint2(vreg[k].x, vreg[k].y);
-            dst[1] = make_uint2(vreg[k].z, vreg[k].w);
-        }
         // scores of the two 16-token halves
         m40_float4 sA = {0.f, 0.f, 0.f, 0.f}, sB = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -166,7 +178,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_mfma_kernel(AttnParams p) {
             sA = mfma16x16x32(qf[i], kreg[0][i], sA);
             sB = mfma16x16x32(qf[i], kreg[1][i], sB);
         }
-        if (tile + kWaves < ntiles) issue(tile + kWaves);      // in flight during the rest of this tile
+        if (tile + kWaves < ntiles) issue_k(tile + kWaves);
         const bool vA = (uint32_t)(tile * kTile + c16) < ntok, vB = (uint32_t)(tile * kTile + 16 + c16) < ntok;
         const float a0 = vA ? (sA[0] + sA[1]) * score_scale : -INFINITY;
         const float a1 = vA ? (sA[2] + sA[3]) * score_scale : -INFINITY;
@@ -201,20 +213,23 @@ __global__ __launch_bounds__(kThreads, 2) void attn_mfma_kernel(AttnParams p) {
             pl[4 * g + 2][16 + c16] = __builtin_bit_cast(uint16_t, hB1);
             pl[4 * g + 3][16 + c16] = f16_bits(pB1 - static_cast<float>(hB1));
         }
-        const uint4 pa = *reinterpret_cast<const uint4*>(&p_lds[wave][c16][8 * g]);
-        // O += P . V, one 16-column tile at a time: lane (column c16, group g) gathers tokens 8g .. 8g+7
+        // V tile -> LDS (row-major, two 8-byte stores per piece)
 #pragma unroll
-        for (int d = 0; d < DT; ++d) {
-            const uint8_t* col = my_v + (8 * g) * RS + 2 * (16 * d + c16);
-            uint32_t w[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const uint32_t lo = *reinterpret_cast<const uint16_t*>(col + (2 * j) * RS);
-                const uint32_t hi = *reinterpret_cast<const uint16_t*>(col + (2 * j + 1) * RS);
-                w[j] = lo | (hi << 16);
-            }
-            O[d] = mfma16x16x32(pa, make_uint4(w[0], w[1], w[2], w[3]), O[d]);
+        for (int k = 0; k < DT; ++k) {
+            const int q = k * 64 + lane;
+            uint2* dst = reinterpret_cast<uint2*>(my_v + (q / PIECES) * RS + 16 * (q % PIECES));
+            dst[0] = make_uint2(vreg[k].x, vreg[k].y);
+            dst[1] = make_uint2(vreg[k].z, vreg[k].w);
         }
+        if (tile + kWaves < ntiles) issue_v(tile + kWaves);
+        const uint4 pa = *reinterpret_cast<const uint4*>(&p_lds[wave][c16][8 * g]);
+        // O += P . V, one 16-column tile at a time: lane (column c16, group g) takes tokens 8g .. 8g+7, transposed by the read: a group of 16 lanes reads four
+        // tokens x 16 columns, eight bytes a lane, and lane i receives column i
+        __builtin_amdgcn_wave_barrier();
+        const uint8_t* rows = my_v + (8 * g + (c16 >> 2)) * RS + 8 * (c16 & 3);
+#pragma unroll
+        for (int d = 0; d < DT; ++d) O[d] = mfma16x16x32(pa, read_transposed(rows + 32 * d, rows + 32 * d + 4 * RS), O[d]);
+        __builtin_amdgcn_wave_barrier();
     }
 
     // ---- merge the four waves --------------------------------------------------------------------------------------
@@ -247,12 +262,9 @@ __global__ __launch_bounds__(kThreads, 2) void attn_mfma_kernel(AttnParams p) {
         if (final_out) {
             m40_attn_store<HD>(p, b, qh, d, num / (den > 0.0f ? den : 1.0f));
         } else {
-            float* w = p.ws + (((size_t)b * p.q_heads + qh) * p.nchunks + blockIdx.y) * (HD + 2);
-            w[2 + d] = num;
-            if (d == 0) {
-                w[0] = M;
-                w[1] = den;
-            }
+            const size_t at = ((size_t)b * p.q_heads + qh) * p.nchunks + blockIdx.y;
+            p.ws[at * HD + d] = num;
+            if (d == 0) reinterpret_cast<float2*>(p.ml)[at] = make_float2(M, den);
         }
     }
 }
@@ -261,6 +273,6 @@ __global__ __launch_bounds__(kThreads, 2) void attn_mfma_kernel(AttnParams p) {
 
 void m40_launch_attn_mfma(hipStream_t stream, const AttnParams& p, uint32_t head_dim, uint32_t batch) {
     dim3 grid(p.kv_heads * p.subgroups, p.nchunks, batch);
-    if (head_dim == 64) attn_mfma_kernel<64><<<grid, kThreads, 0, stream>>>(p);
-    else attn_mfma_kernel<128><<<grid, kThreads, 0, stream>>>(p);
+    const auto kernel = head_dim == 64 ? attn_mfma_kernel<64> : attn_mfma_kernel<128>;
+    kernel<<<grid, kThreads, 0, stream>>>(p.K, p.V, p.Q, p.seq_ids_dev, p.seq_lens_dev, p.max_seq_len, p.kv_heads, p.q_heads, p.subgroups, p.chunk, p.len_bias, p);
 }

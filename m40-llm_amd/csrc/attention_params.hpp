@@ -10,7 +10,8 @@ struct AttnParams {
     float* Out;
     uint8_t* packed;              // not null: rows as operands of the next product (packed_rows.hpp) instead of Out
     uint32_t packed_pad;
-    float* ws;                    // partials: [batch][q_heads][nchunks][hd + 2]
+    float* ws;                    // partials: sums [batch][q_heads][nchunks][hd], behind them
+    float* ml;                    // [batch][q_heads][nchunks][2]: maximum and denominator
     const uint32_t* seq_ids_dev;  // may be null
     const uint32_t* seq_lens_dev; // may be null
     uint32_t seq_id, seq_len;

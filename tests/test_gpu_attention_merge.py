@@ -1,0 +1,43 @@
+"""Merge of chunk partials: one, some and more than 64 chunks a row, rows of one batch with very different numbers of them, and partials of an earlier, longer call
+(infinities) left in the buffer, against 64-bit attention."""
+import numpy as np
+import pytest
+
+from gpu_common import Dev, close, f16bits, m40
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def dev():
+    d = Dev()
+    yield d
+    d.ctx.close()
+
+
+@pytest.mark.parametrize("qh,kvh,hd,lens,hint", [(4, 2, 64, [8192], 8192), (4, 2, 128, [8193], 8704), (2, 1, 128, [16500, 1, 700], 16512), (16, 2, 64, [129, 128, 1000, 3], 1024),
+                                                 (8, 8, 128, [640], 640)])
+def test_merge_of_chunks(dev, qh, kvh, hd, lens, hint):
+    rng = np.random.default_rng(hd + len(lens))
+    B, L = len(lens), max(lens)
+    kv = m40.KVCache(dev.ctx, hint, B + 1, kvh, hd)
+    Kc, Vc = (rng.standard_normal((B, L, kvh, hd)).astype(np.float16) for _ in range(2))
+    for b, n in enumerate(lens): dev.fill_dense(kv, b, Kc[b, :n].view(np.uint16), Vc[b, :n].view(np.uint16))
+    dev.fill_dense(kv, B, f16bits(np.zeros((hint, kvh, hd))), f16bits(np.full((hint, kvh, hd), np.inf)))
+    q = (2.0 * rng.standard_normal((B, qh * hd))).astype(np.float32)
+    dq, out = dev.up(q), dev.zeros(q.nbytes)
+    call = "m40llm_ext_attention_last_token_f32_gqa_batched_lens_dev_async"
+    stale = dev.up(np.full(B, B, dtype=np.uint32)), dev.up(np.full(B, hint, dtype=np.uint32))
+    ids, dlens = dev.up(np.arange(B, dtype=np.uint32)), dev.up(np.asarray(lens, dtype=np.uint32))
+    dev.call(call, kv.h, stale[0].ptr, stale[1].ptr, 0, B, hint, dq.ptr, qh, out.ptr)
+    dev.call(call, kv.h, ids.ptr, dlens.ptr, 0, B, hint, dq.ptr, qh, out.ptr)
+    dev.sync()
+    got = out.download(np.float32, (B, qh, hd)).astype(np.float64)
+    for b, n in enumerate(lens):
+        k, v = (np.repeat(t[b, :n].astype(np.float64), qh // kvh, axis=1) for t in (Kc, Vc))
+        s = np.einsum("hd,thd->ht", q[b].reshape(qh, hd).astype(np.float64), k) / np.sqrt(hd)
+        w = np.exp(s - s.max(axis=1, keepdims=True))
+        want = np.einsum("ht,thd->hd", w / w.sum(axis=1, keepdims=True), v)
+        # q exact to 2^-22 and sums of f32: scores of up to 40 off by a few 2^-20, the weights by as much
+        close(got[b], want, 1e-5, 2e-5)
+    kv.destroy()
