@@ -885,6 +885,12 @@ public:
         }
     }
 
+    // Steps of one attention size from which a batched run records them as a graph.  Recording takes the host 0.2 to 0.55 ms a run, and a launch of the GPU's is
+    // longer than one of the host's at every size measured: steps launch by launch / recorded, us: TinyLlama shape, 32 rows, 4 steps 5084 / 5226, 20 steps 25 094 / 25 371;
+    // 8 rows, 2 steps 1819 / 2093; Qwen2.5-3B shape, 2 rows, 8 steps 15 404 / 15 660; width 256, 22 layers, 8 rows, 48 steps 30 653 / 30 935.  A long run is
+    // recorded all the same: it costs it less than a hundredth and leaves the host free.
+    static constexpr uint32_t kRecordFrom = 48;
+
     // Returns false when a pick was a near-tie (the caller then repeats the decode on the host-sampled path).
     bool decode_batch_device(const uint32_t* seq_ids, const uint32_t* kv_lens, const uint32_t* first_tokens, uint32_t rows,
                              uint32_t warmup, uint32_t steps, uint32_t* ids_out, float* gaps_out, double* elapsed_ms) {
@@ -925,26 +931,25 @@ public:
                 uint32_t n = n_steps - done;
                 if (hint < cfg_.max_seq_len && longest + n > hint) n = hint - longest;
                 uint32_t i = 0;
-                if (mode_ >= 2 && (!bgraph_ || bgraph_rows_ != rows || bgraph_hint_ != hint || bgraph_ws_generation_ != ws_.generation)) {
+                const bool record = mode_ >= 2 && n > kRecordFrom;
+                if (record && (!bgraph_ || bgraph_rows_ != rows || bgraph_hint_ != hint || bgraph_ws_generation_ != ws_.generation)) {
                     if (bgraph_) M40H_TRY(m40llm_stream_synchronize(ctx_, M40LLM_STREAM_DECODE));
                     drop_batch_graph();
                     // the first step goes out launch by launch: the GPU works on it while the host records the graph for those after it
                     enqueue_batched_step(rows, hint, hidden, other);
                     i = 1;
-                    if (n > 1) {
-                        M40H_TRY(m40llm_cuda_graph_begin_capture(ctx_, M40LLM_STREAM_DECODE));
-                        try {
-                            enqueue_batched_step(rows, hint, hidden, other);
-                        } catch (...) {
-                            m40llm_cuda_graph_cancel_capture(ctx_, M40LLM_STREAM_DECODE);
-                            throw;
-                        }
-                        M40H_TRY(m40llm_cuda_graph_end_capture(ctx_, M40LLM_STREAM_DECODE, &bgraph_));
-                        bgraph_rows_ = rows; bgraph_hint_ = hint; bgraph_ws_generation_ = ws_.generation;
+                    M40H_TRY(m40llm_cuda_graph_begin_capture(ctx_, M40LLM_STREAM_DECODE));
+                    try {
+                        enqueue_batched_step(rows, hint, hidden, other);
+                    } catch (...) {
+                        m40llm_cuda_graph_cancel_capture(ctx_, M40LLM_STREAM_DECODE);
+                        throw;
                     }
+                    M40H_TRY(m40llm_cuda_graph_end_capture(ctx_, M40LLM_STREAM_DECODE, &bgraph_));
+                    bgraph_rows_ = rows; bgraph_hint_ = hint; bgraph_ws_generation_ = ws_.generation;
                 }
                 for (; i < n; ++i) {
-                    if (mode_ >= 2) M40H_TRY(m40llm_cuda_graph_launch(ctx_, bgraph_, M40LLM_STREAM_DECODE));
+                    if (record) M40H_TRY(m40llm_cuda_graph_launch(ctx_, bgraph_, M40LLM_STREAM_DECODE));
                     else enqueue_batched_step(rows, hint, hidden, other);
                 }
                 done += n;
