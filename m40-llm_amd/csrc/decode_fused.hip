@@ -27,16 +27,20 @@ constexpr int kWavesPerBlock = 4;
 //
 // In two halves so that the caller can request x and the norm weights first, then the GEMV weights, and only then
 // wait: loads return in issue order, so x arrives ahead of the weight stream and the whole prologue (sum of squares,
-// scaling, LDS, two barriers) runs while the weights are still in flight.  A batch is four 16-byte loads per thread
-// and array (K <= 4096 in one batch); longer rows take further batches inside stage_finish.
-constexpr int kStageBatch = 4;
+// scaling, LDS, two barriers) runs while the weights are still in flight.  A batch is BATCH 16-byte loads per thread
+// and array, two up to K = 2048 and four beyond (K <= 4096 in one batch; longer rows take further batches inside stage_finish): what is asked for here keeps the
+// weights waiting, a request at a time.  (Four of the row and eight halves of the norm's weights whatever K: Q/K/V of
+// 10.5 MB 4.93 us, now 4.44; gate and up of 46 MB 9.53 / 9.25, of 90 MB 16.15 / 15.75; vocabulary of 32000 24.2 / 23.4.)
+template <int BATCH>
 struct StageRegs {
-    float4 x[kStageBatch];
-    uint4 w[kStageBatch];      // raw bits: four f32 norm weights, or four f16 in .x/.y
+    float4 x[BATCH];
+    uint4 w[BATCH];      // raw bits: four f32 norm weights, or the eight f16 that hold the four
 };
+inline int stage_batch(int K) { return K <= 2 * 4 * kThreads ? 2 : 4; }
 
+template <int kStageBatch>
 __device__ __forceinline__ void stage_load(const float* __restrict__ x, const void* __restrict__ w, uint32_t w_dtype,
-                                           int K, int batch, StageRegs& r) {
+                                           int K, int batch, StageRegs<kStageBatch>& r) {
     const int n4 = K >> 2;
     int idx[kStageBatch];
 #pragma unroll
@@ -47,18 +51,15 @@ __device__ __forceinline__ void stage_load(const float* __restrict__ x, const vo
 #pragma unroll
     for (int u = 0; u < kStageBatch; ++u) r.x[u] = reinterpret_cast<const float4*>(x)[idx[u]];
     // One unconditional batch whatever the weights' type: a branch around loads makes the compiler wait for every
-    // load in flight at its join (the rows above).  f32: 16 bytes per index as two halves; f16: 8 bytes, asked for twice.
+    // load in flight at its join (the rows above).  The weights are 16-byte aligned, K a multiple of eight.
     const char* wb = static_cast<const char*>(w);
-    const int stride = w_dtype == 0u ? 8 : 16, hi_off = w_dtype == 0u ? 0 : 8;
+    const int shift = w_dtype == 0u ? 3 : 4;
 #pragma unroll
-    for (int u = 0; u < kStageBatch; ++u) {
-        const uint2 lo = *reinterpret_cast<const uint2*>(wb + (size_t)idx[u] * stride);
-        const uint2 hi = *reinterpret_cast<const uint2*>(wb + (size_t)idx[u] * stride + hi_off);
-        r.w[u].x = lo.x; r.w[u].y = lo.y; r.w[u].z = hi.x; r.w[u].w = hi.y;
-    }
+    for (int u = 0; u < kStageBatch; ++u) r.w[u] = *reinterpret_cast<const uint4*>(wb + (((size_t)idx[u] << shift) & ~(size_t)15));
 }
 
-__device__ __forceinline__ void stage_sumsq(const StageRegs& r, int K, int batch, float& ss) {
+template <int kStageBatch>
+__device__ __forceinline__ void stage_sumsq(const StageRegs<kStageBatch>& r, int K, int batch, float& ss) {
     const int n4 = K >> 2;
 #pragma unroll
     for (int u = 0; u < kStageBatch; ++u) {
@@ -72,7 +73,8 @@ __device__ __forceinline__ void stage_sumsq(const StageRegs& r, int K, int batch
     }
 }
 
-__device__ __forceinline__ void stage_store(const StageRegs& r, uint32_t w_dtype, int K, int batch, float scale,
+template <int kStageBatch>
+__device__ __forceinline__ void stage_store(const StageRegs<kStageBatch>& r, uint32_t w_dtype, int K, int batch, float scale,
                                             float* __restrict__ a_lds) {
     const int n4 = K >> 2;
 #pragma unroll
@@ -82,7 +84,7 @@ __device__ __forceinline__ void stage_store(const StageRegs& r, uint32_t w_dtype
             float4 wv = make_float4(__uint_as_float(r.w[u].x), __uint_as_float(r.w[u].y), __uint_as_float(r.w[u].z),
                                     __uint_as_float(r.w[u].w));
             if (w_dtype == 0u) {
-                const uint32_t h0 = r.w[u].x, h1 = r.w[u].y;
+                const uint32_t h0 = i & 1 ? r.w[u].z : r.w[u].x, h1 = i & 1 ? r.w[u].w : r.w[u].y;
                 wv = make_float4(m40_h2f((uint16_t)(h0 & 0xffffu)), m40_h2f((uint16_t)(h0 >> 16)),
                                  m40_h2f((uint16_t)(h1 & 0xffffu)), m40_h2f((uint16_t)(h1 >> 16)));
             }
@@ -93,7 +95,8 @@ __device__ __forceinline__ void stage_store(const StageRegs& r, uint32_t w_dtype
 }
 
 // `first` holds batch 0, loaded by the caller before its weight prefetch.
-__device__ __forceinline__ void stage_finish(const StageRegs& first, const float* __restrict__ x,
+template <int kStageBatch>
+__device__ __forceinline__ void stage_finish(const StageRegs<kStageBatch>& first, const float* __restrict__ x,
                                              const void* __restrict__ w, uint32_t w_dtype, float eps, int K,
                                              float* __restrict__ a_lds, float* __restrict__ wave_sums) {
     const int tid = threadIdx.x;
@@ -102,7 +105,7 @@ __device__ __forceinline__ void stage_finish(const StageRegs& first, const float
     stage_sumsq(first, K, 0, ss);
     if (nbatch > 1) {       // rows longer than one batch: kept apart so that the usual case has no loop with loads in it
         for (int b = 1; b < nbatch; ++b) {
-            StageRegs r;
+            StageRegs<kStageBatch> r;
             stage_load(x, w, w_dtype, K, b, r);
             stage_sumsq(r, K, b, ss);
         }
@@ -117,7 +120,7 @@ __device__ __forceinline__ void stage_finish(const StageRegs& first, const float
     stage_store(first, w_dtype, K, 0, scale, a_lds);
     if (nbatch > 1) {
         for (int b = 1; b < nbatch; ++b) {
-            StageRegs r;
+            StageRegs<kStageBatch> r;
             stage_load(x, w, w_dtype, K, b, r);
             stage_store(r, w_dtype, K, b, scale, a_lds);
         }
@@ -144,8 +147,9 @@ struct QkvArgs {
 
 // One wave per PAIRS consecutive rotation pairs (two output columns each).  Pair space: Q pairs, then K pairs, then
 // V pairs.  What the first requests need is passed on its own: such arguments lie in registers when a wave starts (a structure is read from memory first).
-template <int PAIRS>
-__global__ __launch_bounds__(kThreads) void norm_qkv_rope_append_kernel(const float* x, const void* norm_w, const uint16_t* wq, const uint32_t* position_dev,
+// The row is staged by the first four waves; six where that leaves no CU a second workgroup (see the launch).
+template <int WAVES, int PAIRS, int BATCH>
+__global__ __launch_bounds__(64 * WAVES) void norm_qkv_rope_append_kernel(const float* x, const void* norm_w, const uint16_t* wq, const uint32_t* position_dev,
                                                                         uint32_t d_model, uint32_t q_heads, uint32_t kv_heads, uint32_t head_dim,
                                                                         uint32_t rope_layout, uint32_t norm_dtype, QkvArgs p) {
     extern __shared__ float a_lds[];
@@ -154,12 +158,12 @@ __global__ __launch_bounds__(kThreads) void norm_qkv_rope_append_kernel(const fl
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     // x and the norm weights are requested before anything else is computed, then (below) the position and the pair's
     // rotation entry, then the GEMV weights; the norm prologue runs while the weights stream in
-    StageRegs xr;
-    stage_load(x, norm_w, norm_dtype, K, 0, xr);
+    StageRegs<BATCH> xr;
+    if (WAVES == kWavesPerBlock || wave < kWavesPerBlock) stage_load(x, norm_w, norm_dtype, K, 0, xr);
     __builtin_amdgcn_sched_barrier(0);
     const uint32_t half = head_dim / 2u;
     const uint32_t q_pairs = q_heads * half, kv_pairs = kv_heads * half;
-    const uint32_t pair0 = (blockIdx.x * kWavesPerBlock + wave) * PAIRS;
+    const uint32_t pair0 = (blockIdx.x * WAVES + wave) * PAIRS;
     bool live[PAIRS];
     int which[PAIRS];       // 0 Q, 1 K, 2 V
     uint32_t local[PAIRS], off[PAIRS];
@@ -218,7 +222,12 @@ __global__ __launch_bounds__(kThreads) void norm_qkv_rope_append_kernel(const fl
             }
         }
     }
-    stage_finish(xr, x, norm_w, norm_dtype, p.eps, K, a_lds, wave_sums);
+    if (WAVES == kWavesPerBlock || wave < kWavesPerBlock) {
+        stage_finish(xr, x, norm_w, norm_dtype, p.eps, K, a_lds, wave_sums);
+    } else {
+        __syncthreads();                 // as in stage_finish
+        __syncthreads();
+    }
     float d[2 * PAIRS];
     gemv_accumulate<2 * PAIRS>(bp, a_lds, 0, K >> 3, lane, regs, d);
     gemv_finish<2 * PAIRS, 1>(d, nullptr, wave, lane);
@@ -279,9 +288,9 @@ __global__ __launch_bounds__(kThreads) void gemv_residual_kernel(const float* __
 
 // hid[j] = silu(Wg[j] . xn) * (Wu[j] . xn),  xn = RMSNorm(x) * w.  A wave owns one j (gate and up row).  The row is staged by the first four waves (whose
 // order of sums the norm's own kernel has); four more that only stream weights halve how often it is staged, and keep as many requests in flight as half as many
-// waves with two j each: 46 MB (FFN 5632, K 2048) 10.1 -> 9.5 us a launch, 90 MB (11008) 17.1 -> 16.1; with one j and four waves 10.8 and 17.1, sixteen waves
-// 10.9 and 17.1, eleven (two workgroups on every CU) 9.6 and 16.7.
-template <int WAVES>
+// waves with two j each: 46 MB (FFN 5632, K 2048) 10.1 -> 9.5 us a launch, 90 MB (11008) 17.1 -> 16.1 (9.25 and 15.75 with fewer requests ahead of the weights); with
+// one j and four waves 10.8 and 17.1, sixteen waves 10.9 and 17.1, eleven (two workgroups on every CU) 9.6 and 16.7.
+template <int WAVES, int BATCH>
 __global__ __launch_bounds__(WAVES * 64) void norm_gate_up_swiglu_kernel(const float* __restrict__ x,
                                                                        const void* __restrict__ norm_w,
                                                                        uint32_t norm_dtype, float eps,
@@ -295,7 +304,7 @@ __global__ __launch_bounds__(WAVES * 64) void norm_gate_up_swiglu_kernel(const f
     const uint4* const bp[2] = {reinterpret_cast<const uint4*>(Wg + (size_t)row * K), reinterpret_cast<const uint4*>(Wu + (size_t)row * K)};
     GemvRegs<2> regs;
     if (WAVES == kWavesPerBlock || wave < kWavesPerBlock) {
-        StageRegs xr;
+        StageRegs<BATCH> xr;
         stage_load(x, norm_w, norm_dtype, K, 0, xr);
         gemv_prefetch<2>(bp, 0, K >> 3, lane, regs);
         stage_finish(xr, x, norm_w, norm_dtype, eps, K, a_lds, wave_sums);
@@ -316,7 +325,7 @@ __global__ __launch_bounds__(WAVES * 64) void norm_gate_up_swiglu_kernel(const f
 
 // logits = W . RMSNorm(x); optionally the workgroup's top-2 (largest, second, first index of largest) goes
 // to blk_top (a | b | idx planes of `top_cap` entries) for the device-side greedy pick.
-template <int COLS>
+template <int COLS, int BATCH>
 __global__ __launch_bounds__(kThreads) void norm_gemv_kernel(const float* __restrict__ x,
                                                              const void* __restrict__ norm_w, uint32_t norm_dtype,
                                                              float eps, const uint16_t* __restrict__ W,
@@ -335,7 +344,7 @@ __global__ __launch_bounds__(kThreads) void norm_gemv_kernel(const float* __rest
         const int col = (live && col0 + c < N) ? col0 + c : N - 1;
         bp[c] = reinterpret_cast<const uint4*>(W + (size_t)col * K);
     }
-    StageRegs xr;
+    StageRegs<BATCH> xr;
     stage_load(x, norm_w, norm_dtype, K, 0, xr);
     GemvRegs<COLS> regs;
     gemv_prefetch<COLS>(bp, 0, K >> 3, lane, regs);
@@ -488,8 +497,13 @@ int m40llm_ext_fused_norm_qkv_rope_append_async(
     p.rope_cs = m40_rope_cs_cache(ctx, p.rope_table);
     const uint32_t pairs = (q_heads + 2u * kv->num_heads) * (kv->head_dim / 2u);
     (void)hipGetLastError();
-    // one pair per wave: two per wave measured 3 % slower on the whole token at 1280 pairs
-    norm_qkv_rope_append_kernel<1><<<(pairs + kWavesPerBlock - 1) / kWavesPerBlock, kThreads, (size_t)D * 4, ctx->decode_stream>>>(
+    // one pair per wave: two per wave measured 3 % slower on the whole token at 1280 pairs.  Six waves a workgroup where four would put two workgroups on some CUs
+    // and six put one on each (4 / 6 waves, us: 1280 pairs of K 2048 4.44 / 4.10, 1536 of 2048 4.63 / 4.37, 1536 of 1024 3.73 / 3.47); fewer pairs leave CUs idle
+    // (768 of 1024 3.01 / 3.06), more gain at some sizes and lose at others (3072 of 2048 6.24 / 6.35, of 4096 10.6 / 9.8, 3584 of 5120 15.4 / 17.3)
+    const uint32_t cus = (uint32_t)ctx->num_cus, waves = pairs > 4u * cus && pairs <= 6u * cus ? 6u : 4u;
+    const auto kernel = stage_batch((int)D) == 2 ? (waves == 6u ? norm_qkv_rope_append_kernel<6, 1, 2> : norm_qkv_rope_append_kernel<4, 1, 2>)
+                                                 : (waves == 6u ? norm_qkv_rope_append_kernel<6, 1, 4> : norm_qkv_rope_append_kernel<4, 1, 4>);
+    kernel<<<(pairs + waves - 1) / waves, 64 * waves, (size_t)D * 4, ctx->decode_stream>>>(
         p.x, p.norm_w, p.wq, p.position_dev, p.d_model, p.q_heads, p.kv_heads, p.head_dim, p.rope_layout, p.norm_dtype, p);
     return hipGetLastError() == hipSuccess ? 0 : -7;
 }
@@ -523,8 +537,9 @@ int m40llm_ext_fused_norm_gate_up_swiglu_async(M40llmCudaContext* ctx, const voi
         return -6;
     (void)hipGetLastError();
     // from two workgroups of eight waves a CU on (measured in the kernel's comment); below, four waves reach more CUs
-    const auto kernel = ffn >= 4096 ? norm_gate_up_swiglu_kernel<8> : norm_gate_up_swiglu_kernel<4>;
     const int waves = ffn >= 4096 ? 8 : 4;
+    const auto kernel = stage_batch(d_model) == 2 ? (waves == 8 ? norm_gate_up_swiglu_kernel<8, 2> : norm_gate_up_swiglu_kernel<4, 2>)
+                                                  : (waves == 8 ? norm_gate_up_swiglu_kernel<8, 4> : norm_gate_up_swiglu_kernel<4, 4>);
     kernel<<<(ffn + waves - 1) / waves, waves * 64, (size_t)d_model * 4, ctx->decode_stream>>>(
         static_cast<const float*>(d_x_f32), d_norm_w, norm_weight_dtype, eps, static_cast<const uint16_t*>(d_wgate_f16),
         static_cast<const uint16_t*>(d_wup_f16), static_cast<float*>(d_hid_f32), ffn, d_model);
@@ -549,9 +564,10 @@ int m40llm_ext_fused_norm_gemv_f32xf16_async(M40llmCudaContext* ctx, const void*
     const int blocks = (N + 4 * cols - 1) / (4 * cols);
     if (top && (uint32_t)blocks > top2_capacity) return -5;
     if (out_n_blocks) *out_n_blocks = (uint32_t)blocks;
-    if (cols == 4) norm_gemv_kernel<4><<<blocks, kThreads, lds, ctx->decode_stream>>>(x, d_norm_w, norm_weight_dtype, eps, W, o, N, K, top, top2_capacity);
-    else if (cols == 2) norm_gemv_kernel<2><<<blocks, kThreads, lds, ctx->decode_stream>>>(x, d_norm_w, norm_weight_dtype, eps, W, o, N, K, top, top2_capacity);
-    else norm_gemv_kernel<1><<<blocks, kThreads, lds, ctx->decode_stream>>>(x, d_norm_w, norm_weight_dtype, eps, W, o, N, K, top, top2_capacity);
+    const bool two = stage_batch(K) == 2;
+    const auto kernel = cols == 4 ? (two ? norm_gemv_kernel<4, 2> : norm_gemv_kernel<4, 4>)
+                                  : (cols == 2 ? (two ? norm_gemv_kernel<2, 2> : norm_gemv_kernel<2, 4>) : (two ? norm_gemv_kernel<1, 2> : norm_gemv_kernel<1, 4>));
+    kernel<<<blocks, kThreads, lds, ctx->decode_stream>>>(x, d_norm_w, norm_weight_dtype, eps, W, o, N, K, top, top2_capacity);
     return hipGetLastError() == hipSuccess ? 0 : -7;
 }
 

@@ -83,6 +83,13 @@ def test_norm_qkv_rope_append_equals_call_sequence(dev, orc, qh, kvh, hd, d_mode
         kv_f.destroy(); kv_u.destroy()
 
 
+# four waves a workgroup and (1025 to 1536 pairs on 256 CUs) six, of which four stage the row: a last workgroup that is not full, either edge; rows of one pass of
+# two requests and of one of four (from K 4096 on the call sequence splits K over the waves)
+@pytest.mark.parametrize("qh,kvh,hd,K", [(30, 1, 64, 512), (31, 1, 64, 2048), (32, 1, 64, 2056), (46, 1, 64, 264), (47, 1, 64, 256), (34, 2, 64, 4088), (6, 2, 32, 3072)])
+def test_norm_qkv_rope_append_of_four_and_six_waves(dev, orc, qh, kvh, hd, K):
+    test_norm_qkv_rope_append_equals_call_sequence(dev, orc, qh, kvh, hd, K, 1, True, 1e4)
+
+
 @pytest.mark.parametrize("N,K", [(2048, 2048), (2048, 5632), (2048, 11008), (8192, 2048), (300, 4096), (33, 64)])
 def test_gemv_residual_equals_call_sequence(dev, orc, N, K):
     rng = np.random.default_rng(N + K)
