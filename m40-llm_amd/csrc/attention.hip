@@ -215,68 +215,23 @@ __global__ __launch_bounds__(kAttnThreads, 2) void attn_partial_kernel(AttnParam
     }
 }
 
-// Merge chunk partials: grid (q_heads, batch), 256 threads.  HD / 4 lanes take a chunk's sums, four columns each; the chunks go round the 1024 / HD such groups.
-//
-// Bound by its round trips to memory: everything of the first 64 chunks -- sums, maxima, denominators, the row's length and id -- is asked for at once, before
-// anything is known; partials of chunks past the row's end are stale values inside the buffer and are left out.  Every wave forms all weights itself, one
-// lane a chunk, so that the waves meet once, with their sums.  (Folding the chunks one after the other under a running maximum, 256 / HD of them side by side:
-// the two launches of 8 rows of up to 4093 tokens, head size 128, 13.3 us, now 12.6; 32 rows of up to 1021, 64, 11.8 / 11.3; 2 rows of up to 3000 10.3 / 8.9; one of
-// 16000, 125 chunks, 19.6 / 11.8.)
+// Merge chunk partials: grid (q_heads, batch), 256 threads
 template <int HD>
 __global__ __launch_bounds__(256) void attn_combine_kernel(const float* ws, const float* ml, const uint32_t* seq_lens_dev, const uint32_t* seq_ids_dev, uint32_t nchunks,
                                                            uint32_t q_heads, AttnParams p) {
-    constexpr int kLanes = HD / 4, kGroups = 256 / kLanes, kPass = 64, kEach = kPass / kGroups;
     __shared__ __attribute__((aligned(16))) float sums[4][HD];
     const uint32_t qh = blockIdx.x, b = blockIdx.y;
-    const uint32_t tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, c4 = tid % kLanes, group = tid / kLanes;
     const size_t first = ((size_t)b * q_heads + qh) * nchunks;
-    const float4* v_at = reinterpret_cast<const float4*>(ws + first * HD) + c4;
-    const float2* ml_at = reinterpret_cast<const float2*>(ml) + first;
-    float4 v[kEach];
-    auto load = [&](uint32_t base) {
-#pragma unroll
-        for (int u = 0; u < kEach; ++u) {
-            const uint32_t c = base + group + u * kGroups;
-            v[u] = v_at[(size_t)(c < nchunks ? c : 0u) * kLanes];
-        }
-    };
-    const float2 ml0 = ml_at[lane < nchunks ? lane : 0u];
-    load(0);
+    M40ChunkMerge<HD> merge;
+    merge.request(ws + first * HD, reinterpret_cast<const float2*>(ml) + first, nchunks);
     const uint32_t len = seq_lens_dev ? seq_lens_dev[b] + p.len_bias : p.seq_len;
     const uint32_t sid = (p.max_batch != 0 && seq_ids_dev) ? seq_ids_dev[b] : 0u;
     if (len == 0 || len > p.max_seq_len) return;
     if (p.max_batch != 0 && seq_ids_dev && sid >= p.max_batch) return;
     const uint32_t t0 = (p.window != 0 && len > p.window) ? len - p.window : 0;
     if (len - t0 > p.span_limit) return;      // longer than the launch was sized for: the row is skipped
-    const uint32_t n = (len - t0 + p.chunk - 1) / p.chunk;
-    float m = lane < n ? ml0.x : -INFINITY;
-    for (uint32_t c = kPass + lane; c < n; c += kPass) m = fmaxf(m, ml_at[c].x);
-    m = m40_max64(m);
-    float den = 0.0f;
-    float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (uint32_t base = 0; base < n; base += kPass) {
-        const float2 x = base == 0 ? ml0 : ml_at[base + lane < n ? base + lane : 0u];
-        if (base != 0) load(base);
-        const float f = base + lane < n && x.x != -INFINITY ? expf(x.x - m) : 0.0f;
-        den = fmaf(base + lane < n ? x.y : 0.0f, f, den);
-#pragma unroll
-        for (int u = 0; u < kEach; ++u) {
-            const float w = __shfl(f, (int)(group + u * kGroups), 64);
-            if (base + group + u * kGroups < n) {
-                sum.x = fmaf(v[u].x, w, sum.x); sum.y = fmaf(v[u].y, w, sum.y);
-                sum.z = fmaf(v[u].z, w, sum.z); sum.w = fmaf(v[u].w, w, sum.w);
-            }
-        }
-    }
-    den = m40_sum64(den);
-    if (HD == 64) { sum.x = m40_add_xor16(sum.x); sum.y = m40_add_xor16(sum.y); sum.z = m40_add_xor16(sum.z); sum.w = m40_add_xor16(sum.w); }
-    sum.x = m40_add_xor32(sum.x); sum.y = m40_add_xor32(sum.y); sum.z = m40_add_xor32(sum.z); sum.w = m40_add_xor32(sum.w);
-    if (lane < kLanes) *reinterpret_cast<float4*>(&sums[wave][4 * lane]) = sum;
-    __syncthreads();
-    if (tid < HD) {
-        const float num = (sums[0][tid] + sums[1][tid]) + (sums[2][tid] + sums[3][tid]);
-        m40_attn_store<HD>(p, b, qh, tid, num / (den > 0.0f ? den : 1.0f));
-    }
+    const float y = merge.finish((len - t0 + p.chunk - 1) / p.chunk, sums);
+    if (threadIdx.x < HD) m40_attn_store<HD>(p, b, qh, threadIdx.x, y);
 }
 
 // Any head_dim: one thread per output element, the reference's three passes verbatim

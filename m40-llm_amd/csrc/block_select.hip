@@ -14,14 +14,14 @@
 //   3. attend : per q head, softmax attention over [tokens of the selected blocks] ++ [recent window], one block per
 //               wave.  Old V is unpacked from 4 bits in registers (value = nibble * scale, rounded through f16 as
 //               the reference does).
-//   4. combine: chunk partials merged in ascending order.
+//   4. combine: chunk partials merged.
 //
 // The compressed cache keeps its old store head-major ([kv head][token][...]), so a selected block is one contiguous
 // run of K rows, of packed V and of scales; the dense cache is token-major ([token][kv head][head_dim]).
 //
 // Reference: kernel cuda/kernels.cu:2832-3096 (compressed) and :1825-1983 (dense), entry points
 // :4504-4577 and :4025-4070.  Only the plain top-k policy and score-rank block order are built.
-#include "common.hpp"
+#include "attention_params.hpp"
 
 #include <cstdlib>
 #include <cstring>
@@ -42,7 +42,7 @@ struct BsParams {
     uint32_t* sel;             // [q_heads][64]   block ids in rank order
     float* sel_scores;         // [q_heads][64]
     uint32_t* counts;          // [q_heads] selected blocks
-    float* partial;            // [q_heads][nchunks][hd+2]
+    float* partial;            // sums [q_heads][nchunks][hd], behind them pairs (maximum, denominator) [q_heads][nchunks]
     size_t old_head_stride;
     uint32_t old_tok_stride;
     uint32_t max_seq_len;
@@ -519,55 +519,25 @@ __global__ __launch_bounds__(kBsThreads, 3) void bs_attend_kernel(BsMulti multi)
         if (p.nchunks == 1) {
             p.Out[(size_t)qh * HD + tid] = v / (l > 0.0f ? l : 1.0f);
         } else {
-            float* w = p.partial + ((size_t)qh * p.nchunks + y) * (HD + 2);
-            w[2 + tid] = v;                 // an empty chunk leaves M = -inf, which the merge skips
-            if (tid == 0) { w[0] = M; w[1] = l; }
+            const size_t at = (size_t)qh * p.nchunks + y;
+            p.partial[at * HD + tid] = v;                 // an empty chunk leaves M = -inf, which the merge skips
+            if (tid == 0) reinterpret_cast<float2*>(p.partial + (size_t)p.q_heads * p.nchunks * HD)[at] = make_float2(M, l);
         }
     }
 }
 
-// Merge the chunk partials of one q head: 1024 threads = 1024/HD chunk lanes x HD dims, each lane folds chunks
-// lane, lane + n_lanes, ... with a running maximum; the lanes are then folded in order.  Empty partials (maximum
-// -inf) are skipped.
+// Merge the chunk partials of one q head, 256 threads.  (1024 threads, 1024 / HD chunks side by side under a running maximum: 4 slots of 20 chunks, head size 128,
+// 88.4 us a call, now 86.8.)
 template <int HD>
-__global__ __launch_bounds__(1024) void bs_combine_kernel(BsMulti multi) {
+__global__ __launch_bounds__(256) void bs_combine_kernel(BsMulti multi) {
     const BsParams& p = multi.slot[blockIdx.z];
     if (p.nchunks <= 1) return;      // the attend kernel wrote the output itself
-    constexpr int NCG = 1024 / HD;
-    __shared__ float s_m[NCG], s_den[NCG];
-    __shared__ float s_num[NCG][HD];
-    const uint32_t qh = blockIdx.x, d = threadIdx.x % HD, cg = threadIdx.x / HD;
-    const uint32_t n = p.nchunks;
-    const float* w = p.partial + (size_t)qh * p.nchunks * (HD + 2);
-    float m = -INFINITY, num = 0.0f, den = 0.0f;
-    for (uint32_t ch = cg; ch < n; ch += NCG) {
-        const float* wc = w + (size_t)ch * (HD + 2);
-        const float mc = wc[0], lc = wc[1], vc = wc[2 + d];
-        if (mc == -INFINITY) continue;
-        const float nm = fmaxf(m, mc);
-        const float fa = m == -INFINITY ? 0.0f : expf(m - nm);
-        const float fb = expf(mc - nm);
-        num = fmaf(num, fa, vc * fb);
-        den = fmaf(den, fa, lc * fb);
-        m = nm;
-    }
-    s_num[cg][d] = num;
-    if (d == 0) { s_m[cg] = m; s_den[cg] = den; }
-    __syncthreads();
-    if (cg == 0) {
-#pragma unroll
-        for (int g = 1; g < NCG; ++g) {
-            const float mc = s_m[g];
-            if (mc == -INFINITY) continue;
-            const float nm = fmaxf(m, mc);
-            const float fa = m == -INFINITY ? 0.0f : expf(m - nm);
-            const float fb = expf(mc - nm);
-            num = fmaf(num, fa, s_num[g][d] * fb);
-            den = fmaf(den, fa, s_den[g] * fb);
-            m = nm;
-        }
-        p.Out[(size_t)qh * HD + d] = num / (den > 0.0f ? den : 1.0f);
-    }
+    __shared__ __attribute__((aligned(16))) float sums[4][HD];
+    const uint32_t qh = blockIdx.x, n = p.nchunks;
+    M40ChunkMerge<HD> merge;
+    merge.request(p.partial + (size_t)qh * n * HD, reinterpret_cast<const float2*>(p.partial + (size_t)p.q_heads * n * HD) + (size_t)qh * n, n);
+    const float y = merge.finish(n, sums);
+    if (threadIdx.x < HD) p.Out[(size_t)qh * HD + threadIdx.x] = y;
 }
 
 uint32_t policy_from_env() {
@@ -665,7 +635,7 @@ int launch_multi(hipStream_t s, const BsMulti& m, uint32_t n, bool selection_onl
     bs_rank_kernel<<<dim3(p0.q_heads, max_nblk ? (max_nblk + kBsRankCand - 1) / kBsRankCand : 1, n), kBsRankThreads, keys_lds, s>>>(m);
     if (!selection_only) {
         bs_attend_kernel<HD><<<dim3(p0.q_heads, max_chunks, n), kBsThreads, 0, s>>>(m);
-        if (max_chunks > 1) bs_combine_kernel<HD><<<dim3(p0.q_heads, 1, n), 1024, 0, s>>>(m);
+        if (max_chunks > 1) bs_combine_kernel<HD><<<dim3(p0.q_heads, 1, n), 256, 0, s>>>(m);
     }
     return hipGetLastError() == hipSuccess ? 0 : -8;
 }
