@@ -437,6 +437,15 @@ int m40llm_ext_prefill_project_norm_project_async(M40llmCudaContext* ctx, const 
                                                   void* d_C0_f32, const void* d_norm_weight, uint32_t norm_weight_dtype, float eps, uint32_t gated, int n_mats,
                                                   const void* d_B1_f16, int N1, void* d_C1_f32, const void* d_B2_f16, int N2, void* d_C2_f32,
                                                   const void* d_B3_f16, int N3, void* d_C3_f32, uint32_t stream_kind);
+/* A layer's prompts from Q, K and V to its feed-forward's hidden rows: m40llm_ext_prefill_attention_rope_append_async with its arguments but for the result, which goes to
+ * m40llm_ext_prefill_project_norm_project_async (d_x_f32 = residual + attention . Wo, gated = 1) without being written as f32 in between.  The sequences' rows lie one behind the
+ * other from 0, `rows` in all.  Returns as those calls (1: nothing was enqueued).  Prefill stream. */
+int m40llm_ext_prefill_attention_project_gate_up_async(M40llmCudaContext* ctx, M40llmKVCache* kv, const void* q_dev_f32, const void* k_dev_f32, const void* v_dev_f32,
+                                                       const uint32_t* offsets_dev, const uint32_t* lens_dev, uint32_t batch, const uint32_t* seq_slots_host,
+                                                       const uint32_t* offsets_host, const uint32_t* lens_host, uint32_t q_heads, uint32_t rope_layout,
+                                                       const void* d_angles, const void* d_bq_f32, const void* d_bk_f32, const void* d_bv_f32, uint32_t rows,
+                                                       const void* d_wo_f16, int d_model, const void* d_residual_f32, void* d_x_f32, const void* d_norm_weight,
+                                                       uint32_t norm_weight_dtype, float eps, const void* d_gate_f16, const void* d_up_f16, int ffn, void* d_hid_f32);
 /* embedding rows of `rows` (<= 65535) token ids held on the device (f16 table [vocab][d_model]) -> f32 [rows][d_model];
  * the row form of m40llm_ext_embed_token_dev_async (src/infer/forward.rs:2241-2250 loads them one blocking call per
  * token).  Decode stream. */

@@ -183,9 +183,16 @@ int m40_launch_gemm_tiled_fused(M40llmCudaContext* ctx, hipStream_t stream, uint
                                 const float* A2, const void* norm_w, uint32_t norm_dtype, float eps, int M, int K, int n_mats,
                                 const uint16_t* const* B, const int* N, float* const* C, const float* const* R, bool pair);
 // C0 [M][N0] = R0 + A [M][K0] . B0, and the products of RMSNorm(C0) with one to three matrices (pair: as above); 1 as above, nothing enqueued
+// Rows as the tiled kernel reads them: f16 high and low planes in tiles of 16 rows x 32 columns, a kilobyte each, the tiles of sixteen rows one behind the other;
+// row = scale (hi + lo), scale a power of two.
+struct M40TiledRows { _Float16 *hi, *lo; float* scale; };
+static inline __host__ __device__ size_t m40_tiled_row(int row, int K) { return (size_t)(row >> 4) * (K / 32) * 512 + (row & 15) * 32; }      // f16 ahead of a row's first column,
+static inline __host__ __device__ size_t m40_tiled_col(int k) { return (size_t)(k >> 5) * 512 + (k & 31); }                                 // and of column k from there
+// produce: not null, A is ignored: called once everything is provided, to enqueue what writes the first product's rows; its error is returned
 int m40_launch_gemm_tiled_chain(M40llmCudaContext* ctx, hipStream_t stream, uint32_t stream_kind, const float* A, int M, int K0, const uint16_t* B0, int N0,
                                 const float* R0, float* C0, const void* norm_w, uint32_t norm_dtype, float eps, int n_mats, const uint16_t* const* B,
-                                const int* N, float* const* C, bool pair);
+                                const int* N, float* const* C, bool pair, int (*produce)(void*, const M40TiledRows&) = nullptr,
+                                void* produce_arg = nullptr);
 bool m40_skinny_supported(const M40llmCudaContext* ctx, uint32_t stream_kind, int M, int N, int K, int fmt);
 int m40_launch_skinny(M40llmCudaContext* ctx, hipStream_t stream, uint32_t stream_kind, int fmt, const float* A,
                       const float* up, const void* W0, float* C0, const void* W1, float* C1, int M, int N, int K);

@@ -53,7 +53,7 @@ struct PackSource {
     float4* sum;
     int k_splits;
 };
-enum { kPackPlain = 0, kPackNorm = 1, kPackSwiglu = 2, kPackSumNorm = 3 };
+enum { kPackPlain = 0, kPackNorm = 1, kPackSwiglu = 2, kPackSumNorm = 3, kPackDone = 4 };      // done: somebody else writes the planes
 
 // A [M][K] f32 -> hi, lo [M][K] f16 planes and one scale per row: a = scale * (hi + lo) up to 2^-22 relative.  The scale is
 // the power of two that brings the row's largest magnitude into [2^10, 2^11) -- any finite f32 row fits the f16 planes,
@@ -104,8 +104,8 @@ __device__ __forceinline__ float4 sum_planes(const float4* planes, int k_splits,
 // The planes lie in tiles of 16 rows x 32 k, a kilobyte each, all k of sixteen rows one after the other: what an instruction of the tiled kernel
 // loads is contiguous.  A row's stores are half lines, which the L2 of the die that has the tile's sixteen rows puts together (4096 rows of 5632: 32.0
 // us as whole rows, 35.1 this way, 39.2 with the rows dealt to the dies in turn).  16-byte chunk of a row's first k, and how far on its chunk c is:
-__device__ __forceinline__ size_t plane_chunk(int row, int K) { return (size_t)(row >> 4) * (K / kBK) * 64 + (row & 15) * 4; }
-__device__ __forceinline__ size_t plane_step(int c) { return (size_t)(c >> 2) * 64 + (c & 3); }
+__device__ __forceinline__ size_t plane_chunk(int row, int K) { return m40_tiled_row(row, K) / 8; }
+__device__ __forceinline__ size_t plane_step(int c) { return m40_tiled_col(8 * c) / 8; }
 
 // ROW_THREADS = 64: a wave per row, four rows per workgroup, no barrier (K <= 4096 keeps the row in registers);
 // 256: a workgroup per row (always for the RMSNorm source, whose sum of squares is formed with the thread layout and
@@ -728,7 +728,7 @@ struct TiledPlan {
 
 int plan_tiled(const M40llmCudaContext* ctx, const TiledCall& c, TiledPlan& plan) {
     const PackSource& src = c.source;
-    if (c.n_mats < 1 || c.n_mats > kMaxMats || c.source_kind < kPackPlain || c.source_kind > kPackSwiglu) return -2;
+    if (c.n_mats < 1 || c.n_mats > kMaxMats || c.source_kind < kPackPlain || (c.source_kind > kPackSwiglu && c.source_kind != kPackDone)) return -2;
     if (c.pair && (c.n_mats != 2 || c.N[0] != c.N[1] || c.N[0] % 16 != 0 || c.N[0] > 0x3fffffff || c.R)) return -2;
     if (c.source_kind == kPackSwiglu && (!src.a2 || !m40_aligned16(src.a2))) return -2;
     if (c.source_kind == kPackNorm && (!src.norm_w || src.norm_dtype > 1u || !m40_aligned16(src.norm_w))) return -2;
@@ -806,7 +806,8 @@ int enqueue_tiled(const M40StreamScratch& sc, hipStream_t stream, const TiledCal
         else if (wave_rows) pack(std::integral_constant<int, 64>(), kind, std::integral_constant<int, kPackChunks>());
         else pack(std::integral_constant<int, 256>(), kind, std::integral_constant<int, kPackChunks>());
     };
-    if (c.source_kind == kPackNorm && source.planes) pack_norm(std::integral_constant<int, kPackSumNorm>());
+    if (c.source_kind == kPackDone) {}
+    else if (c.source_kind == kPackNorm && source.planes) pack_norm(std::integral_constant<int, kPackSumNorm>());
     else if (c.source_kind == kPackNorm) pack_norm(std::integral_constant<int, kPackNorm>());
     else if (c.source_kind == kPackSwiglu) pack_either(std::integral_constant<int, kPackSwiglu>());
     else pack_either(std::integral_constant<int, kPackPlain>());
@@ -867,17 +868,22 @@ int m40_launch_gemm_tiled_fused(M40llmCudaContext* ctx, hipStream_t stream, uint
 // product's packed rows, K0 >= K1 columns of them, so the second product's packed rows do not reach them.
 int m40_launch_gemm_tiled_chain(M40llmCudaContext* ctx, hipStream_t stream, uint32_t stream_kind, const float* A, int M, int K0, const uint16_t* B0, int N0,
                                 const float* R0, float* C0, const void* norm_w, uint32_t norm_dtype, float eps, int n_mats, const uint16_t* const* B,
-                                const int* N, float* const* C, bool pair) {
+                                const int* N, float* const* C, bool pair, int (*produce)(void*, const M40TiledRows&), void* produce_arg) {
     if (!ctx || stream_kind > 1u) return -2;
     float* const C_first[1] = {C0};
     const float* const R_first[1] = {R0};
-    const TiledCall first{kPackPlain, {A, nullptr, nullptr, 0u, 0.0f, nullptr, nullptr, nullptr, 0}, M, K0, 1, &B0, &N0, C_first, R_first, false};
+    const TiledCall first{produce ? kPackDone : kPackPlain, {produce ? nullptr : A, nullptr, nullptr, 0u, 0.0f, nullptr, nullptr, nullptr, 0}, M, K0, 1, &B0, &N0, C_first, R_first, false};
     TiledCall second{kPackNorm, {C0, nullptr, norm_w, norm_dtype, eps, nullptr, nullptr, nullptr, 0}, M, N0, n_mats, B, N, C, nullptr, pair};
     TiledPlan plan0, plan1;
     int rc = plan_tiled(ctx, first, plan0);
     if (rc == 0) rc = plan_tiled(ctx, second, plan1);
     if (rc == 0) rc = provide_pack(ctx->scratch[stream_kind], stream, plan0.need > plan1.need ? plan0.need : plan1.need);
     if (rc != 0) return rc;
+    if (produce) {
+        _Float16* hi = static_cast<_Float16*>(ctx->scratch[stream_kind].tiled_pack);
+        rc = produce(produce_arg, {hi, hi + (size_t)padded_rows(M) * K0, reinterpret_cast<float*>(hi + 2 * (size_t)padded_rows(M) * K0)});
+        if (rc != 0) return rc;
+    }
     rc = enqueue_tiled(ctx->scratch[stream_kind], stream, first, plan0, K0 >= N0 ? &second.source : nullptr);
     return rc != 0 ? rc : enqueue_tiled(ctx->scratch[stream_kind], stream, second, plan1, nullptr);
 }

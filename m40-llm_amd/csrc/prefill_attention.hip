@@ -30,7 +30,6 @@
 #include "common.hpp"
 
 #include <type_traits>
-
 #include <vector>
 
 namespace {
@@ -85,6 +84,8 @@ struct PrefillArgs {
     uint32_t plane_tiles;       // padded tiles in total (sequence b starts at tile kv_offsets[b] / 32 + b ... see pack)
     const uint32_t* q_offsets; const uint32_t* kv_offsets; const uint32_t* q_lens; const uint32_t* kv_lens;
     uint32_t q_heads, kv_heads;
+    float* v_max;               // per padded tile and kv head: largest finite |V| (with a PrefillRope)
+    M40TiledRows rows;          // where the result goes as rows of the next product instead of Out
 };
 
 // Prompts that go in unrotated: rows 0 .. of sequence b are its positions 0 ..; queries are rotated where they are loaded, keys where they are
@@ -123,6 +124,7 @@ __global__ __launch_bounds__(kThreads) void prefill_pack_kv_kernel(PrefillArgs p
     constexpr bool kRope = std::is_same<ROPE, PrefillRope>::value;
     constexpr int kKTile = key_tile_of(HD);
     __shared__ float vt[kKTile][HD + 1];
+    __shared__ float wave_max[kWaves];
     const uint32_t b = blockIdx.z, kvh = blockIdx.y, tile = blockIdx.x;
     const uint32_t kv_len = p.kv_lens[b];
     if (tile * kKTile >= kv_len) return;
@@ -197,6 +199,15 @@ __global__ __launch_bounds__(kThreads) void prefill_pack_kv_kernel(PrefillArgs p
             *reinterpret_cast<ushort4*>(rope.v_cache + to) = make_ushort4(m40_f2h(vx[u].x), m40_f2h(vx[u].y), m40_f2h(vx[u].z), m40_f2h(vx[u].w));
         }
         if (tile == 0 && kvh == 0 && threadIdx.x == 0) rope.seq_map[rope.slot[b]] = kv_len;
+        float mx = 0.0f;
+#pragma unroll
+        for (int u = 0; u < kQuads; ++u) {
+            const float v4[4] = {vx[u].x, vx[u].y, vx[u].z, vx[u].w};
+#pragma unroll
+            for (int i = 0; i < 4; ++i) mx = fmaxf(mx, fabsf(v4[i]) <= 3.402823466e+38f ? fabsf(v4[i]) : 0.0f);      // (keys past the end: the last one's again)
+        }
+        mx = m40_max64(mx);
+        if ((threadIdx.x & 63) == 0) wave_max[threadIdx.x >> 6] = mx;
     }
 #pragma unroll
     for (int u = 0; u < kQuads; ++u) {
@@ -216,6 +227,9 @@ __global__ __launch_bounds__(kThreads) void prefill_pack_kv_kernel(PrefillArgs p
         *reinterpret_cast<half4*>(kl + e) = lo;
     }
     __syncthreads();
+    if constexpr (kRope) {
+        if (threadIdx.x == 0) p.v_max[(size_t)(first_tile_of(p.kv_offsets[b], b, kKTile) + tile) * p.kv_heads + kvh] = fmaxf(fmaxf(wave_max[0], wave_max[1]), fmaxf(wave_max[2], wave_max[3]));
+    }
 #pragma unroll
     for (int u = 0; u < kKTile * HD / 8 / kThreads; ++u) {
         const int e = ((int)threadIdx.x + u * kThreads) * 8, d = e / kKTile, slot = e % kKTile;
@@ -234,7 +248,10 @@ __global__ __launch_bounds__(kThreads) void prefill_pack_kv_kernel(PrefillArgs p
 
 // QB: 16-query blocks per wave.  With two, every K and V fragment a wave reads from LDS serves 32 queries instead of 16:
 // the kernel's LDS traffic (each wave reads the whole K and V tile) was what it spent most of its time on.
-template <int HD, int QB, class ROPE>
+// PLANES (with a PrefillRope): the result goes to the rows of the next product, which a packing pass read and wrote again (4096 rows of 2048 12.9 us, 522 rows
+// 6.0).  A row's scale must be known to the workgroups of all its heads: it follows from the largest |V| of the row's sequence, which no weighted mean of V
+// exceeds, brought into [2^14, 2^15): f16 hi + lo keep 22 bits of every value down to 2^-18 of it.  A value that is not finite goes in as it is.
+template <int HD, int QB, class ROPE, bool PLANES>
 __global__ __launch_bounds__(kThreads) void prefill_attn_kernel(PrefillArgs p, ROPE rope) {
     constexpr bool kRope = std::is_same<ROPE, PrefillRope>::value;
     constexpr int kKTile = key_tile_of(HD);
@@ -265,6 +282,9 @@ __global__ __launch_bounds__(kThreads) void prefill_attn_kernel(PrefillArgs p, R
     if (q0 >= q_len || q_len > kv_len) return;
     const uint32_t kvh = h / (p.q_heads / p.kv_heads);
     const int tid = threadIdx.x, lane = tid & 63;
+    const uint32_t n_max = (kv_len + kKTile - 1) / kKTile * p.kv_heads;
+    const float* v_max = PLANES ? p.v_max + (size_t)first_tile_of(p.kv_offsets[b], b, kKTile) * p.kv_heads : nullptr;
+    float bound = PLANES ? v_max[(uint32_t)tid < n_max ? tid : 0] : 0.0f;        // waited for at the end
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);       // as a scalar: tests on it branch without masks
     const int j = lane & 15, g = lane >> 4;
     const float inv_sqrt = HD == 64 ? 0.125f : 0.08838834764831845f;
@@ -509,6 +529,23 @@ __global__ __launch_bounds__(kThreads) void prefill_attn_kernel(PrefillArgs p, R
     }
 
     // ---- out = O / sum: this lane holds columns 16 d + 4 g .. + 3 of its query
+    float row_scale = 1.0f, row_inv = 1.0f;
+    if constexpr (PLANES) {
+        __shared__ float wave_max[kWaves];
+        for (uint32_t i = tid + kThreads; i < n_max; i += kThreads) bound = fmaxf(bound, v_max[i]);
+        bound = m40_max64(bound);
+        if (lane == 0) wave_max[wave] = bound;
+        __syncthreads();
+        bound = fmaxf(fmaxf(wave_max[0], wave_max[1]), fmaxf(wave_max[2], wave_max[3]));
+        if (bound > 0.0f) {
+            int ex;
+            (void)frexpf(bound, &ex);
+            ex -= 15;
+            ex = ex < -100 ? -100 : (ex > 100 ? 100 : ex);
+            row_scale = ldexpf(1.0f, ex);
+            row_inv = ldexpf(1.0f, -ex);
+        }
+    }
     if (!wave_live) return;
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb) {
@@ -516,7 +553,25 @@ __global__ __launch_bounds__(kThreads) void prefill_attn_kernel(PrefillArgs p, R
         l += __shfl_xor(l, 32);
         const float denom = l > 0.0f ? l : 1.0f;
         const uint32_t q = wq0 + 16u * qb + (uint32_t)j;
-        if (q < q_len) {
+        if constexpr (PLANES) {
+            if (q >= q_len) continue;
+            const int row = (int)(p.q_offsets[b] + q), K = (int)p.q_heads * HD;
+            const size_t first = m40_tiled_row(row, K);
+            if (h == 0 && g == 0) p.rows.scale[row] = row_scale;
+#pragma unroll
+            for (int d = 0; d < DT; ++d) {
+                half4 hi, lo;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float y = O[qb][d][r] / denom * row_inv;
+                    hi[r] = static_cast<_Float16>(y);
+                    lo[r] = fabsf(y) <= 3.402823466e+38f ? static_cast<_Float16>(y - static_cast<float>(hi[r])) : static_cast<_Float16>(0.0f);
+                }
+                const size_t at = first + m40_tiled_col((int)h * HD + 16 * d + 4 * g);
+                *reinterpret_cast<half4*>(p.rows.hi + at) = hi;
+                *reinterpret_cast<half4*>(p.rows.lo + at) = lo;
+            }
+        } else if (q < q_len) {
             float* op = p.Out + ((size_t)(p.q_offsets[b] + q) * p.q_heads + h) * HD + 4 * g;
 #pragma unroll
             for (int d = 0; d < DT; ++d)
@@ -530,8 +585,8 @@ int prefill_impl(M40llmCudaContext* ctx, const void* q, const void* k, const voi
                  const uint32_t* kv_offsets, const uint32_t* q_lens, const uint32_t* kv_lens, uint32_t batch,
                  uint32_t q_heads, uint32_t kv_heads, uint32_t head_dim, void* out, bool synchronize,
                  const uint32_t* kv_offsets_host = nullptr, const uint32_t* q_lens_host = nullptr,
-                 const uint32_t* kv_lens_host = nullptr, const PrefillRope* rope = nullptr) {
-    if (!ctx || !q || !k || !v || !q_offsets || !kv_offsets || !q_lens || !kv_lens || !out) return -1;
+                 const uint32_t* kv_lens_host = nullptr, const PrefillRope* rope = nullptr, const M40TiledRows* rows = nullptr) {
+    if (!ctx || !q || !k || !v || !q_offsets || !kv_offsets || !q_lens || !kv_lens || (!out && !rows)) return -1;
     if (batch == 0) return -2;
     if (q_heads == 0 || kv_heads == 0 || q_heads % kv_heads != 0) return -3;
     if (head_dim != 64 && head_dim != 128) return -9;
@@ -571,7 +626,7 @@ int prefill_impl(M40llmCudaContext* ctx, const void* q, const void* k, const voi
     }
     const uint32_t kKTile = (uint32_t)key_tile_of((int)head_dim);
     const uint64_t plane_tiles = (offs[batch - 1] / kKTile + (batch - 1)) + (host[2 * (size_t)batch - 1] + kKTile - 1) / kKTile;
-    const size_t need = (size_t)plane_tiles * kv_heads * 4 * kKTile * head_dim * sizeof(_Float16);
+    const size_t planes_bytes = (size_t)plane_tiles * kv_heads * 4 * kKTile * head_dim * sizeof(_Float16), need = planes_bytes + (size_t)plane_tiles * kv_heads * sizeof(float);
     M40StreamScratch& sc = ctx->scratch[0];
     if (sc.attn_planes_bytes < need) {
         if (hipStreamSynchronize(ctx->prefill_stream) != hipSuccess) return -5;
@@ -586,6 +641,8 @@ int prefill_impl(M40llmCudaContext* ctx, const void* q, const void* k, const voi
     }
     a.planes = static_cast<const _Float16*>(sc.attn_planes);
     a.plane_tiles = (uint32_t)plane_tiles;
+    a.v_max = reinterpret_cast<float*>(static_cast<char*>(sc.attn_planes) + planes_bytes);
+    if (rows) a.rows = *rows;
     (void)hipGetLastError();
     const dim3 pack_grid((max_kv + kKTile - 1) / kKTile, kv_heads, batch);
     uint64_t long_groups = 0;           // two-block workgroups that the long sequences make
@@ -598,8 +655,15 @@ int prefill_impl(M40llmCudaContext* ctx, const void* q, const void* k, const voi
         constexpr int HD = decltype(hd)::value;
         using R = decltype(r);
         prefill_pack_kv_kernel<HD, R><<<pack_grid, kThreads, 0, ctx->prefill_stream>>>(a, r);
-        if (blocks == 2) prefill_attn_kernel<HD, 2, R><<<grid, kThreads, 0, ctx->prefill_stream>>>(a, r);
-        else prefill_attn_kernel<HD, 1, R><<<grid, kThreads, 0, ctx->prefill_stream>>>(a, r);
+        if constexpr (std::is_same<R, PrefillRope>::value) {
+            if (rows) {
+                if (blocks == 2) prefill_attn_kernel<HD, 2, R, true><<<grid, kThreads, 0, ctx->prefill_stream>>>(a, r);
+                else prefill_attn_kernel<HD, 1, R, true><<<grid, kThreads, 0, ctx->prefill_stream>>>(a, r);
+                return;
+            }
+        }
+        if (blocks == 2) prefill_attn_kernel<HD, 2, R, false><<<grid, kThreads, 0, ctx->prefill_stream>>>(a, r);
+        else prefill_attn_kernel<HD, 1, R, false><<<grid, kThreads, 0, ctx->prefill_stream>>>(a, r);
     };
     const auto launch_rope = [&](auto hd) { rope ? launch(hd, *rope) : launch(hd, NoRope{}); };
     if (head_dim == 64) launch_rope(std::integral_constant<int, 64>());
@@ -644,26 +708,26 @@ int m40llm_ext_attention_prefill_f32_gqa_varlen_host_tables_async(M40llmCudaCont
                         batch_size, q_heads, kv_heads, head_dim, out_dev_f32, false, kv_offsets_host, q_lens_host, kv_lens_host);
 }
 
-int m40llm_ext_prefill_attention_rope_append_async(M40llmCudaContext* ctx, M40llmKVCache* kv, const void* q_dev_f32, const void* k_dev_f32,
+static int rope_append(M40llmCudaContext* ctx, M40llmKVCache* kv, const void* q_dev_f32, const void* k_dev_f32,
                                                    const void* v_dev_f32, const uint32_t* offsets_dev, const uint32_t* lens_dev, uint32_t batch,
                                                    const uint32_t* seq_slots_host, const uint32_t* offsets_host, const uint32_t* lens_host, uint32_t q_heads,
                                                    uint32_t rope_layout, const void* d_angles, const void* d_bq_f32, const void* d_bk_f32,
-                                                   const void* d_bv_f32, void* out_dev_f32) {
-    if (!ctx || !kv || !q_dev_f32 || !k_dev_f32 || !v_dev_f32 || !offsets_dev || !lens_dev || !seq_slots_host || !offsets_host || !lens_host || !d_angles || !out_dev_f32)
+                                                   const void* d_bv_f32, void* out_dev_f32, const M40TiledRows* rows) {
+    if (!ctx || !kv || !q_dev_f32 || !k_dev_f32 || !v_dev_f32 || !offsets_dev || !lens_dev || !seq_slots_host || !offsets_host || !lens_host || !d_angles || (!out_dev_f32 && !rows))
         return -1;
     const int n_bias = (d_bq_f32 != nullptr) + (d_bk_f32 != nullptr) + (d_bv_f32 != nullptr);
     if (batch == 0 || batch > (uint32_t)kM40PrefillSeqs || (n_bias != 0 && n_bias != 3) || rope_layout > M40LLM_ROPE_LAYOUT_NEOX) return -2;
     if (kv->compressed || !kv->d_k || !kv->d_v) return -6;
     PrefillRope r{};
-    uint32_t rows = 0;
+    uint32_t n_rows = 0;
     for (uint32_t i = 0; i < batch; ++i) {
         if (seq_slots_host[i] >= kv->max_batch_size) return -2;
         if (lens_host[i] > kv->max_seq_len) return -5;
         for (uint32_t j = 0; j < i; ++j)
             if (seq_slots_host[j] == seq_slots_host[i]) return -8;   // two sequences of one call would race on a slot
         r.slot[i] = seq_slots_host[i];
-        r.first[i] = rows;
-        rows += lens_host[i];              // at most 64 lengths, which the attention refuses above 8192
+        r.first[i] = n_rows;
+        n_rows += lens_host[i];              // at most 64 lengths, which the attention refuses above 8192
     }
     if (!m40_aligned16(d_angles)) return -4;
     r.angles = static_cast<const float2*>(d_angles);
@@ -671,7 +735,48 @@ int m40llm_ext_prefill_attention_rope_append_async(M40llmCudaContext* ctx, M40ll
     r.layout = rope_layout; r.max_seq_len = kv->max_seq_len;
     r.k_cache = kv->d_k; r.v_cache = kv->d_v; r.seq_map = kv->d_seq_map;
     return prefill_impl(ctx, q_dev_f32, k_dev_f32, v_dev_f32, offsets_dev, offsets_dev, lens_dev, lens_dev, batch, q_heads, kv->num_heads, kv->head_dim, out_dev_f32,
-                        false, offsets_host, lens_host, lens_host, &r);
+                        false, offsets_host, lens_host, lens_host, &r, rows);
+}
+
+int m40llm_ext_prefill_attention_rope_append_async(M40llmCudaContext* ctx, M40llmKVCache* kv, const void* q_dev_f32, const void* k_dev_f32,
+                                                   const void* v_dev_f32, const uint32_t* offsets_dev, const uint32_t* lens_dev, uint32_t batch,
+                                                   const uint32_t* seq_slots_host, const uint32_t* offsets_host, const uint32_t* lens_host, uint32_t q_heads,
+                                                   uint32_t rope_layout, const void* d_angles, const void* d_bq_f32, const void* d_bk_f32,
+                                                   const void* d_bv_f32, void* out_dev_f32) {
+    return rope_append(ctx, kv, q_dev_f32, k_dev_f32, v_dev_f32, offsets_dev, lens_dev, batch, seq_slots_host, offsets_host, lens_host, q_heads, rope_layout, d_angles, d_bq_f32,
+                       d_bk_f32, d_bv_f32, out_dev_f32, nullptr);
+}
+
+int m40llm_ext_prefill_attention_project_gate_up_async(M40llmCudaContext* ctx, M40llmKVCache* kv, const void* q_dev_f32, const void* k_dev_f32, const void* v_dev_f32,
+                                                       const uint32_t* offsets_dev, const uint32_t* lens_dev, uint32_t batch, const uint32_t* seq_slots_host,
+                                                       const uint32_t* offsets_host, const uint32_t* lens_host, uint32_t q_heads, uint32_t rope_layout,
+                                                       const void* d_angles, const void* d_bq_f32, const void* d_bk_f32, const void* d_bv_f32, uint32_t rows,
+                                                       const void* d_wo_f16, int d_model, const void* d_residual_f32, void* d_x_f32, const void* d_norm_weight,
+                                                       uint32_t norm_weight_dtype, float eps, const void* d_gate_f16, const void* d_up_f16, int ffn, void* d_hid_f32) {
+    if (!ctx || !kv || !lens_host || !offsets_host || !d_wo_f16 || !d_residual_f32 || !d_x_f32 || !d_norm_weight || !d_gate_f16 || !d_up_f16 || !d_hid_f32) return -1;
+    if (rows == 0 || d_model <= 0 || ffn <= 0 || norm_weight_dtype > 1u || batch == 0) return -2;
+    // every row of the product is a row of a sequence, one behind the other
+    uint64_t at = 0;
+    for (uint32_t i = 0; i < batch; ++i) {
+        if (offsets_host[i] != at) return 1;
+        at += lens_host[i];
+    }
+    const uint64_t K = (uint64_t)q_heads * kv->head_dim;
+    if (at != rows || rows > 65535u || K == 0 || K > 65536u) return 1;
+    const uint16_t *wo = static_cast<const uint16_t*>(d_wo_f16), *B[2] = {static_cast<const uint16_t*>(d_gate_f16), static_cast<const uint16_t*>(d_up_f16)};
+    float *x = static_cast<float*>(d_x_f32), *C[2] = {static_cast<float*>(d_hid_f32), nullptr};
+    const int N[2] = {ffn, ffn};
+    if (!m40_gemm_tiled_supported(nullptr, wo, (int)rows, d_model, (int)K) || !m40_aligned16(d_norm_weight) || ffn % 16 != 0 || ffn > 0x3fffffff ||
+        !m40_gemm_tiled_supported(x, B[0], (int)rows, ffn, d_model) || !m40_gemm_tiled_supported(x, B[1], (int)rows, ffn, d_model))
+        return 1;
+    if (m40_ensure_device(ctx) != 0) return -2;
+    auto attend = [&](const M40TiledRows& to) {
+        return rope_append(ctx, kv, q_dev_f32, k_dev_f32, v_dev_f32, offsets_dev, lens_dev, batch, seq_slots_host, offsets_host, lens_host, q_heads, rope_layout, d_angles,
+                           d_bq_f32, d_bk_f32, d_bv_f32, nullptr, &to);
+    };
+    return m40_launch_gemm_tiled_chain(ctx, ctx->prefill_stream, 0u, nullptr, (int)rows, (int)K, wo, d_model, static_cast<const float*>(d_residual_f32), x, d_norm_weight,
+                                       norm_weight_dtype, eps, 2, B, N, C, true,
+                                       [](void* f, const M40TiledRows& to) { return (*static_cast<decltype(attend)*>(f))(to); }, &attend);
 }
 
 }  // extern "C"

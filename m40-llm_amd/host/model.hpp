@@ -505,14 +505,21 @@ public:
             if (!have_qkv)
                 prefill_project(1, a, nullptr, w.attn_norm, pws_.xn.f32(), rows, D, 3, w.wq, D, pws_.q.f32(), w.wk, KV, pws_.k.f32(), w.wv, KV,
                                 pws_.v.f32(), nullptr);
-            M40H_TRY(m40llm_ext_prefill_attention_rope_append_async(ctx_, kv_, pws_.q.ptr(), pws_.k.ptr(), pws_.v.ptr(), d_off, d_len, batch, slots.data(),
-                                                                    offsets.data(), lens, cfg_.q_heads, cfg_.rope_layout, pws_.angles.ptr(),
-                                                                    cfg_.has_qkv_bias ? w.bq : nullptr, cfg_.has_qkv_bias ? w.bk : nullptr,
-                                                                    cfg_.has_qkv_bias ? w.bv : nullptr, pws_.att.ptr()));
-            // O projection, norm, gate and up in one call; the down projection, the next layer's norm and Q/K/V likewise
-            int gated = m40llm_ext_prefill_project_norm_project_async(ctx_, pws_.att.ptr(), (int)rows, (int)D, w.wo, (int)D, a, pws_.x1.ptr(), w.ffn_norm,
+            const void *bq = cfg_.has_qkv_bias ? w.bq : nullptr, *bk = cfg_.has_qkv_bias ? w.bk : nullptr, *bv = cfg_.has_qkv_bias ? w.bv : nullptr;
+            // attention, O projection, norm, gate and up in one call; the down projection, the next layer's norm and Q/K/V likewise
+            int gated = m40llm_ext_prefill_attention_project_gate_up_async(ctx_, kv_, pws_.q.ptr(), pws_.k.ptr(), pws_.v.ptr(), d_off, d_len, batch, slots.data(),
+                                                                           offsets.data(), lens, cfg_.q_heads, cfg_.rope_layout, pws_.angles.ptr(), bq, bk, bv, rows, w.wo,
+                                                                           (int)D, a, pws_.x1.ptr(), w.ffn_norm, cfg_.norm_weight_dtype, cfg_.rms_eps, w.wgate, w.wup,
+                                                                           (int)F, pws_.hid.ptr());
+            if (gated != 0 && gated != 1) M40H_TRY(gated);
+            if (gated != 0) {
+                M40H_TRY(m40llm_ext_prefill_attention_rope_append_async(ctx_, kv_, pws_.q.ptr(), pws_.k.ptr(), pws_.v.ptr(), d_off, d_len, batch, slots.data(),
+                                                                        offsets.data(), lens, cfg_.q_heads, cfg_.rope_layout, pws_.angles.ptr(), bq, bk, bv,
+                                                                        pws_.att.ptr()));
+                gated = m40llm_ext_prefill_project_norm_project_async(ctx_, pws_.att.ptr(), (int)rows, (int)D, w.wo, (int)D, a, pws_.x1.ptr(), w.ffn_norm,
                                                                       cfg_.norm_weight_dtype, cfg_.rms_eps, 1u, 2, w.wgate, (int)F, pws_.hid.ptr(), w.wup, (int)F,
                                                                       nullptr, nullptr, 0, nullptr, PRE);
+            }
             if (gated != 0) {
                 if (gated != 1) M40H_TRY(gated);
                 prefill_project(0, pws_.att.f32(), nullptr, nullptr, nullptr, rows, D, 1, w.wo, D, pws_.x1.f32(), nullptr, 0, nullptr, nullptr, 0,

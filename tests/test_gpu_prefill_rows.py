@@ -1,0 +1,73 @@
+"""Prompts from Q, K and V to the feed-forward's hidden rows in one call (m40llm_ext_prefill_attention_project_gate_up_async): the attention leaves its result as the O
+projection's operands.  Against the two calls that write it as f32 in between, and the projection against 64 bits of those f32 rows: ragged lengths that start inside tiles
+of sixteen rows, both head sizes, one and two query blocks a wave, K whole and in parts, values of one sequence fifty times another's and, within one,
+a hundred times the first tokens', values that are not finite."""
+import numpy as np
+import pytest
+
+from gpu_common import Dev, f16bits, m40
+
+pytestmark = pytest.mark.gpu
+u32 = lambda a: np.asarray(a, dtype=np.uint32)
+
+
+@pytest.fixture(scope="module")
+def dev():
+    d = Dev()
+    yield d
+    d.ctx.close()
+
+
+@pytest.mark.parametrize("hd,qh,kvh,D,F,lens,layout,bias", [(64, 4, 1, 256, 512, [1, 63, 64, 65], 0, False), (64, 32, 4, 2048, 512, [23, 187, 90, 61, 161], 0, False),
+                                                            (128, 16, 2, 2048, 256, [130, 700], 1, True), (64, 32, 4, 256, 256, [4096], 0, False), (128, 2, 2, 64, 64, [33], 1, True)])
+def test_attention_project_gate_up(dev, hd, qh, kvh, D, F, lens, layout, bias):
+    rng = np.random.default_rng(sum(lens) + hd)
+    rows, K, n = sum(lens), qh * hd, len(lens)
+    q, k, v = (rng.standard_normal((rows, w)).astype(np.float32) for w in (K, kvh * hd, kvh * hd))
+    offs = u32(np.concatenate([[0], np.cumsum(lens)[:-1]]))
+    v[offs[-1]:] *= 50.0
+    v[offs[-1] + lens[-1] // 2:] *= 1e2
+    if n > 1: v[offs[1] + lens[1] // 2, 0] = np.inf
+    dq, dk, dv = (dev.up(t) for t in (q, k, v))
+    biases = [dev.up(0.1 * rng.standard_normal(w).astype(np.float32)) for w in (K, kvh * hd, kvh * hd)]
+    b = [t.ptr if bias else None for t in biases]
+    wo, wg, wu = (f16bits(0.05 * rng.standard_normal(s)) for s in ((D, K), (F, D), (F, D)))
+    res, nw = rng.standard_normal((rows, D)).astype(np.float32), np.ones(D, np.float32)
+    dwo, dwg, dwu, dres, dnw = (dev.up(t) for t in (wo, wg, wu, res, nw))
+    h_lens, slots = u32(lens), u32(range(n))
+    d_offs, d_lens, angles = dev.up(offs), dev.up(h_lens), dev.zeros(rows * hd // 2 * 8)
+    dev.call("m40llm_ext_prefill_angles_async", n, h_lens.ctypes.data, hd, 1e4, 1.0, angles.ptr, 0)
+    att, got = dev.zeros(rows * K * 4), []
+    for whole in (False, True):
+        kv = m40.KVCache(dev.ctx, max(lens) + 1, n, kvh, hd)
+        x, hid = dev.zeros(rows * D * 4), dev.zeros(rows * F * 4)
+        head = [kv.h, dq.ptr, dk.ptr, dv.ptr, d_offs.ptr, d_lens.ptr, n, slots.ctypes.data, offs.ctypes.data, h_lens.ctypes.data, qh, layout, angles.ptr, *b]
+        if whole:
+            tail = [dwo.ptr, D, dres.ptr, x.ptr, dnw.ptr, 1, 1e-5, dwg.ptr, dwu.ptr, F, hid.ptr]
+            call = "m40llm_ext_prefill_attention_project_gate_up_async"
+            dev.call(call, *head, rows, *tail)
+            dev.call(call, *head, rows + 1, *tail, expect=1)
+            same = u32([0] * n)
+            if n > 1: dev.call(call, *(head[:7] + [same.ctypes.data] + head[8:]), rows, *tail, expect=-8)
+        else:
+            dev.call("m40llm_ext_prefill_attention_rope_append_async", *head, att.ptr)
+            dev.call("m40llm_ext_prefill_project_norm_project_async", att.ptr, rows, K, dwo.ptr, D, dres.ptr, x.ptr, dnw.ptr, 1, 1e-5, 1, 2, dwg.ptr, F, hid.ptr, dwu.ptr, F, None,
+                     None, 0, None, 0)
+        dev.sync()
+        got.append((x.download(np.float32, (rows, D)), hid.download(np.float32, (rows, F)), [kv.read_token(s, lens[s] - 1) for s in range(n)]))
+        kv.destroy()
+    a = att.download(np.float32, (rows, K)).astype(np.float64)
+    fine = np.isfinite(a).all(axis=1)
+    assert fine.all() == (n == 1)
+    w64 = wo.view(np.float16).astype(np.float64)
+    want, bound = a[fine] @ w64.T + res[fine], np.abs(a[fine]) @ np.abs(w64).T * 2.0 ** -20
+    for x, _, _ in got:
+        # operands exact to 2^-22 each, f32 sums of K products in chains of at most K / 32 steps
+        assert np.all(np.abs(x[fine] - want) <= bound + np.abs(want) * 2.0 ** -23)
+    rms = [np.sqrt(np.mean(((x[fine] - want) / np.sqrt(np.mean(want ** 2, axis=1, keepdims=True))) ** 2)) for x, _, _ in got]
+    assert rms[1] <= 1.05 * rms[0], rms
+    assert not np.isfinite(got[1][0][~fine]).any()
+    sc = np.abs(got[0][1][fine]).max(axis=1, keepdims=True)
+    assert np.all(np.abs(got[1][1][fine] - got[0][1][fine]) <= 1e-5 * sc)
+    for s in range(n):
+        for i in range(2): assert np.array_equal(got[0][2][s][i], got[1][2][s][i])
