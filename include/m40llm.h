@@ -439,7 +439,7 @@ int m40llm_ext_prefill_project_norm_project_async(M40llmCudaContext* ctx, const 
                                                   const void* d_B3_f16, int N3, void* d_C3_f32, uint32_t stream_kind);
 /* A layer's prompts from Q, K and V to its feed-forward's hidden rows: m40llm_ext_prefill_attention_rope_append_async with its arguments but for the result, which goes to
  * m40llm_ext_prefill_project_norm_project_async (d_x_f32 = residual + attention . Wo, gated = 1) without being written as f32 in between.  The sequences' rows lie one behind the
- * other from 0, `rows` in all.  Returns as those calls (1: nothing was enqueued).  Prefill stream. */
+ * other from 0; of `rows` those behind them are undefined in the results.  Returns as those calls (1: nothing was enqueued).  Prefill stream. */
 int m40llm_ext_prefill_attention_project_gate_up_async(M40llmCudaContext* ctx, M40llmKVCache* kv, const void* q_dev_f32, const void* k_dev_f32, const void* v_dev_f32,
                                                        const uint32_t* offsets_dev, const uint32_t* lens_dev, uint32_t batch, const uint32_t* seq_slots_host,
                                                        const uint32_t* offsets_host, const uint32_t* lens_host, uint32_t q_heads, uint32_t rope_layout,

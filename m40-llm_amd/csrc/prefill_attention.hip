@@ -755,14 +755,14 @@ int m40llm_ext_prefill_attention_project_gate_up_async(M40llmCudaContext* ctx, M
                                                        uint32_t norm_weight_dtype, float eps, const void* d_gate_f16, const void* d_up_f16, int ffn, void* d_hid_f32) {
     if (!ctx || !kv || !lens_host || !offsets_host || !d_wo_f16 || !d_residual_f32 || !d_x_f32 || !d_norm_weight || !d_gate_f16 || !d_up_f16 || !d_hid_f32) return -1;
     if (rows == 0 || d_model <= 0 || ffn <= 0 || norm_weight_dtype > 1u || batch == 0) return -2;
-    // every row of the product is a row of a sequence, one behind the other
+    // the sequences' rows lie one behind the other; what the product has behind them nobody reads
     uint64_t at = 0;
     for (uint32_t i = 0; i < batch; ++i) {
         if (offsets_host[i] != at) return 1;
         at += lens_host[i];
     }
     const uint64_t K = (uint64_t)q_heads * kv->head_dim;
-    if (at != rows || rows > 65535u || K == 0 || K > 65536u) return 1;
+    if (at > rows || rows > 65535u || K == 0 || K > 65536u) return 1;
     const uint16_t *wo = static_cast<const uint16_t*>(d_wo_f16), *B[2] = {static_cast<const uint16_t*>(d_gate_f16), static_cast<const uint16_t*>(d_up_f16)};
     float *x = static_cast<float*>(d_x_f32), *C[2] = {static_cast<float*>(d_hid_f32), nullptr};
     const int N[2] = {ffn, ffn};

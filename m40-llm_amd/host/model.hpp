@@ -459,6 +459,7 @@ public:
     // every row, RoPE + bias + the f16 KV append run as one launch, and the attention is the packed causal prefill
     // kernel.  Each sequence starts at position 0 of its (cleared) cache slots.  Returns the hidden rows
     // [total rows][d_model] on the device; row offsets are the running sum of `lens`.
+    static constexpr uint32_t kManyRows = 33;
     bool packed_prefill_available() const { return !kvcfg_.is_enabled() && (cfg_.head_dim == 64 || cfg_.head_dim == 128); }
     const float* forward_prefill(const uint32_t* seq_ids, const uint32_t* lens, const uint32_t* tokens, uint32_t batch) {
         if (batch == 0) throw std::invalid_argument("batched prefill requires at least one item");
@@ -476,9 +477,20 @@ public:
             total += lens[i];
         }
         if (total > 65535u) throw std::invalid_argument("batched prefill is limited to 65535 rows per call");
-        const uint32_t rows = (uint32_t)total;
-        for (uint32_t r = 0; r < rows; ++r)
+        for (uint64_t r = 0; r < total; ++r)
             if (tokens[r] >= cfg_.vocab) throw std::out_of_range("token id out of range");
+        // Few rows go through the many-row products as well, which take them from kManyRows on: with rows behind the last that nobody reads (the first token again).  The
+        // products read the weights once either way; the separate launches that fewer rows took go from stream to stream and read the weights once for sixteen rows or
+        // less (us, separate / padded, TinyLlama shape: 1 token 4040 / 1770, 8 4330 / 1750, 16 7840 / 1730, 24 9800 / 1720, 32 12 550 / 1790; Qwen2.5-3B: 8 7930 / 3500,
+        // 32 26 200 / 3510).
+        const bool many = total >= kManyRows || (weights_aligned_ && cfg_.d_model % 64 == 0 && cfg_.ffn % 64 == 0 && cfg_.kv_heads * cfg_.head_dim >= 16u);
+        const uint32_t rows = many && total < kManyRows ? kManyRows : (uint32_t)total;
+        std::vector<uint32_t> padded;
+        if (rows != total) {
+            padded.assign(tokens, tokens + total);
+            padded.resize(rows, tokens[0]);
+            tokens = padded.data();
+        }
         pws_.ensure(ctx_, cfg_, rows, batch);
         const uint32_t D = cfg_.d_model, KV = cfg_.kv_heads * cfg_.head_dim, F = cfg_.ffn;
         const uint32_t PRE = M40LLM_STREAM_PREFILL, DEC = M40LLM_STREAM_DECODE;

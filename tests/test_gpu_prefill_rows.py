@@ -2,12 +2,15 @@
 projection's operands.  Against the two calls that write it as f32 in between, and the projection against 64 bits of those f32 rows: ragged lengths that start inside tiles
 of sixteen rows, both head sizes, one and two query blocks a wave, K whole and in parts, values of one sequence fifty times another's and, within one,
 a hundred times the first tokens', values that are not finite."""
+import importlib
+
 import numpy as np
 import pytest
 
 from gpu_common import Dev, f16bits, m40
 
 pytestmark = pytest.mark.gpu
+syn = importlib.import_module("m40-llm_amd.synthetic")
 u32 = lambda a: np.asarray(a, dtype=np.uint32)
 
 
@@ -46,7 +49,7 @@ def test_attention_project_gate_up(dev, hd, qh, kvh, D, F, lens, layout, bias):
             tail = [dwo.ptr, D, dres.ptr, x.ptr, dnw.ptr, 1, 1e-5, dwg.ptr, dwu.ptr, F, hid.ptr]
             call = "m40llm_ext_prefill_attention_project_gate_up_async"
             dev.call(call, *head, rows, *tail)
-            dev.call(call, *head, rows + 1, *tail, expect=1)
+            dev.call(call, *head, rows - 1, *tail, expect=1)
             same = u32([0] * n)
             if n > 1: dev.call(call, *(head[:7] + [same.ctypes.data] + head[8:]), rows, *tail, expect=-8)
         else:
@@ -71,3 +74,25 @@ def test_attention_project_gate_up(dev, hd, qh, kvh, D, F, lens, layout, bias):
     assert np.all(np.abs(got[1][1][fine] - got[0][1][fine]) <= 1e-5 * sc)
     for s in range(n):
         for i in range(2): assert np.array_equal(got[0][2][s][i], got[1][2][s][i])
+
+
+@pytest.mark.parametrize("lens", [[1], [5, 3], [31, 1], [32], [33], [20, 14]])
+def test_few_rows_of_prompts(dev, lens):
+    """Prompts of fewer rows than the many-row products take go through them with rows behind theirs: the same bits whatever an earlier, longer call left in the buffers,
+    and the hidden rows of the tokens one by one (whose keys and values pass through f16)."""
+    cfg = dict(n_layers=2, d_model=256, q_heads=4, kv_heads=2, head_dim=64, ffn=512, vocab=500, rms_eps=1e-5, rope_base=1e4, rope_scale=1.0, rope_layout=0, qkv_bias=False)
+    W = syn.make_weights(cfg, seed=4, std=0.08, emb_std=1.0)
+    rng = np.random.default_rng(sum(lens))
+    prompts, long = [rng.integers(0, 500, n) for n in lens], [rng.integers(0, 500, 200)]
+    got = []
+    for before in (False, True):
+        dm = syn.DeviceModel(dev.ctx, cfg, W, max_seq_len=256, max_sequences=3)
+        dm.set_mode(2)
+        if before: dm.forward_prefill([2], long)
+        got.append(dm.forward_prefill(range(len(lens)), prompts))
+        for s, p in enumerate(prompts):
+            for t, tok in enumerate(p): h, l = dm.forward_token(2, t, int(tok))
+            for a, b in zip((got[-1][0][s], got[-1][1][s]), (h, l)):
+                assert np.abs(a - b).max() <= 2e-3 * np.abs(b).max()
+        dm.close()
+    assert all(np.array_equal(a, b) for a, b in zip(*got))
