@@ -463,7 +463,7 @@ bool q80_gemv_supported(int M, int N, int K) {
 }
 
 // W1/C1 may be null (one matrix of N columns); otherwise both matrices have N columns.
-int launch_q80_gemv(hipStream_t stream, const float* A, const float* up, const uint8_t* W0, float* C0,
+int launch_q80_gemv(int num_cus, hipStream_t stream, const float* A, const float* up, const uint8_t* W0, float* C0,
                     const uint8_t* W1, float* C1, int M, int N, int K) {
     Q80GemvArgs p;
     p.A = A; p.up = up;
@@ -475,7 +475,10 @@ int launch_q80_gemv(hipStream_t stream, const float* A, const float* up, const u
     p.per = (nblk + p.kw - 1) / p.kw;
     p.per += p.per & 1;
     const int tpw = kQ80GemvWaves / p.kw;
-    const int cols_target = 16;   // columns per team: amortises the activation staging; measured best of 4..32
+    // Columns per team, two at a time: as many as one workgroup a CU leaves, up to sixteen, beyond which more workgroups are better than longer ones.  Feed-forward of one row /
+    // two rows, us, sixteen columns throughout and now: 512 x 1024 19.6 / 28.6 -> 8.0 / 10.4, 1024 x 2816 20.2 / 30.2 -> 10.4 / 14.5, 2048 x 2048 20.1 / 29.2 -> 8.5 / 10.8,
+    // 2048 x 5632 22.0 / 32.2 -> 13.7 / 18.4, one row of 2048 x 11008 23.7 -> 20.4; of 4096 x 14336, sixteen either way, 36.5 (12 columns 41.5, 8 39.2).
+    const int per_cu = (p.N + tpw * num_cus - 1) / (tpw * num_cus), cols_target = per_cu >= 15 ? 16 : (per_cu + 1) / 2 * 2;
     int nteams = (p.N + cols_target - 1) / cols_target;
     int blocks = (nteams + tpw - 1) / tpw;
     if (blocks < 1) blocks = 1;
@@ -581,7 +584,7 @@ static int launch_multi_f32xf16(M40llmCudaContext* ctx, hipStream_t stream, uint
 static int launch_q80(M40llmCudaContext* ctx, hipStream_t stream, uint32_t stream_kind, const float* A, const uint8_t* B,
                       float* C, int M, int N, int K) {
     if (m40_aligned16(B) && m40_aligned16(A) && q80_gemv_supported(M, N, K))
-        return launch_q80_gemv(stream, A, nullptr, B, C, nullptr, nullptr, M, N, K);
+        return launch_q80_gemv(ctx->num_cus, stream, A, nullptr, B, C, nullptr, nullptr, M, N, K);
     if (m40_aligned16(B) && m40_aligned16(A) && m40_q80_i8_supported(ctx, stream_kind, M, N, K))
         return m40_launch_q80_i8(ctx, stream, stream_kind, A, B, C, M, N, K);
     if (m40_aligned16(B) && m40_aligned16(A) && m40_skinny_supported(ctx, stream_kind, M, N, K, 1))
@@ -819,15 +822,16 @@ int m40llm_ext_ffn_swiglu_q80_f32_async(M40llmCudaContext* ctx, const void* d_x_
     float* out = static_cast<float*>(d_out_f32);
     const bool aligned = m40_aligned16(wg) && m40_aligned16(wu) && m40_aligned16(wd) && m40_aligned16(x) &&
                          m40_aligned16(gate) && m40_aligned16(up);
-    // two rows of a large FFN: the int8 form's three launches (52.8 us at 4096 / 14336) beat the two GEMV launches (63.5 us)
-    const bool two_rows_i8 = M == 2 && (size_t)ffn * d_model >= ((size_t)1 << 24) && aligned &&
+    // two rows of a large FFN: the int8 form beats the two GEMV launches (us, int8 / GEMV: 4096 x 14336 40.9 / 51.3, 3072 x 8192 24.5 / 27.9, but 2048 x 11008 28.5 / 27.8,
+    // 2048 x 8192 22.0 / 21.3, 4096 x 4096 24.2 / 19.2)
+    const bool two_rows_i8 = M == 2 && (size_t)ffn * d_model >= ((size_t)3 << 23) && aligned &&
                              m40_q80_i8_supported(ctx, 1, M, ffn, d_model) && m40_q80_i8_supported(ctx, 1, M, d_model, ffn);
     if (!two_rows_i8 && aligned && q80_gemv_supported(M, ffn, d_model) && q80_gemv_supported(M, d_model, ffn)) {
         // gate and up in one launch; SwiGLU is applied while each lane loads its slices for the down projection
         (void)hipGetLastError();
-        int rc = launch_q80_gemv(ctx->decode_stream, x, nullptr, wg, gate, wu, up, M, ffn, d_model);
+        int rc = launch_q80_gemv(ctx->num_cus, ctx->decode_stream, x, nullptr, wg, gate, wu, up, M, ffn, d_model);
         if (rc != 0) return rc;
-        return launch_q80_gemv(ctx->decode_stream, gate, up, wd, out, nullptr, nullptr, M, d_model, ffn);
+        return launch_q80_gemv(ctx->num_cus, ctx->decode_stream, gate, up, wd, out, nullptr, nullptr, M, d_model, ffn);
     }
     if (aligned && m40_q80_i8_supported(ctx, 1, M, ffn, d_model) && m40_q80_i8_supported(ctx, 1, M, d_model, ffn)) {
         // digit planes of x, gate / up / SwiGLU / digit planes of the hidden row, down projection: three launches
