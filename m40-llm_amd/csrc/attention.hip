@@ -291,7 +291,12 @@ template <int HD>
 int launch_hd(M40llmCudaContext* ctx, hipStream_t stream, float* partial, size_t partial_bytes, bool fixed_chunking,
               AttnParams& p, uint32_t batch, uint32_t group, uint32_t span) {
     constexpr uint32_t kRowsPerStep = kWaves * (64 / (HD / 8));   // token rows one workgroup covers per S
-    if (span > 512 && m40_aligned16(p.Q)) {
+    // Short rows of a batch: a launch of the vector-ALU kernel grows with the q heads of all rows, the matrix-core kernel and its merge hardly do.  From 512 of them on (128
+    // where the rows take two launches either way) they are the faster ones; us, vector ALU / matrix cores, 32 q heads to 4 kv of 64, up to 512 tokens: 8 rows of 100
+    // 6.4 / 6.9, of 500 7.8 / 7.2, 16 rows of 100 9.8 / 7.0, of 500 10.9 / 7.8, 32 rows 10.3 / 7.8 and 12.8 / 9.4; 16 to 2 of 128, 250 tokens: 16 rows 7.9 / 8.9, 32 rows
+    // 11.1 / 9.2; 500 tokens: 4 rows 8.2 / 8.8, 8 rows 11.0 / 8.8, 32 rows 16.7 / 10.6; 32 to 8 of 128, 500 tokens: 2 rows 8.2 / 8.4, 4 rows 11.0 / 8.6.
+    const bool many_heads = batch > 1 && batch * p.q_heads >= (span > kRowsPerStep * 8 ? 128u : 512u);
+    if ((span > 512 || many_heads) && m40_aligned16(p.Q)) {
         // long rows: matrix-core kernel (it reads q with 16-byte loads).  Chunks are a multiple of 128 tokens (one
         // 32-token tile per wave and pass) sized for about one workgroup per CU -- measured best at 32 K tokens (256
         // workgroups of 1024 tokens: 32 us against 36 us with twice as many half-sized ones) and on the batch-8 step

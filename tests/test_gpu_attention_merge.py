@@ -41,3 +41,12 @@ def test_merge_of_chunks(dev, qh, kvh, hd, lens, hint):
         # q exact to 2^-22 and sums of f32: scores of up to 40 off by a few 2^-20, the weights by as much
         close(got[b], want, 1e-5, 2e-5)
     kv.destroy()
+
+
+# either side of the number of q heads from which short rows of a batch take the matrix-core kernel: one chunk and several, rows of a token, uneven rows
+@pytest.mark.parametrize("qh,kvh,hd,rows,hint", [(32, 4, 64, 15, 512), (32, 4, 64, 16, 512), (8, 8, 64, 64, 130), (16, 2, 128, 7, 400), (16, 2, 128, 8, 400), (64, 4, 128, 8, 256), (64, 4, 128, 2, 257)])
+def test_short_rows_of_a_batch(dev, qh, kvh, hd, rows, hint):
+    rng = np.random.default_rng(qh + rows)
+    lens = rng.integers(1, hint + 1, rows)
+    lens[0], lens[-1] = hint, 1
+    test_merge_of_chunks(dev, qh, kvh, hd, [int(n) for n in lens], hint)
