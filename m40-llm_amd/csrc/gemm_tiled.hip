@@ -340,7 +340,7 @@ __device__ __forceinline__ void tiled_unrolled(std::integer_sequence<int, I...>,
 // KS: k steps of 32 a stage (what is loaded together, between two barriers); kBufs: LDS buffers of a stage each (one
 // workgroup is resident per CU).  Two steps a stage read whole 128-byte lines of a column: with weights that no cache holds 64 x 64 tiles of N 2048,
 // K 2048 take 15.5 us that way and 21.3 us in stages of one step, 64 x 128 tiles 21.0 and 24.6 us (60 rows).
-template <int MT, int NT, int KS, int kBufs, int kBBufs>
+template <int MT, int NT, int KS, int kBufs, int kBBufs, bool FINE>
 __global__ __launch_bounds__(kThreads, 1) void gemm_tiled_kernel(const _Float16* __restrict__ A_hi, const _Float16* __restrict__ A_lo,
                                                                       const float* __restrict__ row_scale, TiledMats mats, int M, int K,
                                                                       int k_splits, int band) {
@@ -431,15 +431,27 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_tiled_kernel(const _Float16*
     for (int i = 0; i < MT; ++i)
 #pragma unroll
         for (int j = 0; j < NT; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-    // Per accumulator step by step, high part then low part: the two large tiles give the same bits.  The weights are the instruction's first
-    // operand, so a lane's four sums are four neighbouring columns of one row and a store is 16 bytes.
+    // Per accumulator step by step, high part then low part: the two large tiles give the same bits.  (FINE: the low parts' sums apart.)  The weights are the instruction's
+    // first operand, so a lane's four sums are four neighbouring columns of one row and a store is 16 bytes.
+    constexpr bool kBlocked = MT * NT <= 8;
+    static_assert(kBlocked || !FINE);
+    floatx4 low[FINE ? MT : 1][FINE ? NT : 1];
+    if (FINE) {
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int j = 0; j < NT; ++j) low[FINE ? i : 0][FINE ? j : 0] = floatx4{0.f, 0.f, 0.f, 0.f};
+    }
     auto compute = [&](const Frags& f) __attribute__((always_inline)) {
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(f.b[nt], f.hi[mt], acc[mt][nt], 0, 0, 0);
 #pragma unroll
-            for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(f.b[nt], f.lo[mt], acc[mt][nt], 0, 0, 0);
+            for (int nt = 0; nt < NT; ++nt) {
+                floatx4& to = FINE ? low[FINE ? mt : 0][FINE ? nt : 0] : acc[mt][nt];
+                to = __builtin_amdgcn_mfma_f32_16x16x32_f16(f.b[nt], f.lo[mt], to, 0, 0, 0);
+            }
         }
     };
     // The barriers are bare s_barrier instructions with the vector-memory wait written out: __syncthreads() would wait for every
@@ -511,8 +523,9 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_tiled_kernel(const _Float16*
         wait_and_meet(std::integral_constant<int, Flight::at(kEven + decltype(ph_c)::value)>());
     };
     // Small tiles have registers to keep the sums of a period (10 or 12 steps) apart from those before: a fraction of the chain of roundings
-    // that all of K would be (as short as the parts of K that small grids are otherwise cut into).
-    constexpr bool kBlocked = MT * NT <= 8;
+    // that all of K would be (as short as the parts of K that small grids are otherwise cut into).  FINE, for one row of tiles, where that costs a hundredth and
+    // not several: twice a period, so that few rows, which other kernels would take otherwise, are no further from 64-bit products than those leave them.  Errors in units of 1e-7
+    // of a row's mean at K 2048 and 5632: those kernels 1.2-1.3 up to 8 rows and 1.6-1.7 up to 32; a chain a period 1.7-1.9; FINE 1.1-1.2.
     floatx4 total[kBlocked ? MT : 1][kBlocked ? NT : 1];
     if (kBlocked) {
 #pragma unroll
@@ -520,28 +533,37 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_tiled_kernel(const _Float16*
 #pragma unroll
             for (int j = 0; j < NT; ++j) total[kBlocked ? i : 0][kBlocked ? j : 0] = floatx4{0.f, 0.f, 0.f, 0.f};
     }
+    auto set_aside = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < (kBlocked ? MT : 0); ++i)
+#pragma unroll
+            for (int j = 0; j < NT; ++j) {
+                if (FINE) acc[i][j] += low[FINE ? i : 0][FINE ? j : 0];
+                total[kBlocked ? i : 0][kBlocked ? j : 0] += acc[i][j];
+                acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+                if (FINE) low[FINE ? i : 0][FINE ? j : 0] = floatx4{0.f, 0.f, 0.f, 0.f};
+            }
+    };
+    constexpr auto set_aside_behind = [](int ph) { return kBlocked && (ph + 1 == kPeriod || (FINE && ph + 1 == kPeriod / 2)); };
     int s = 0;
     for (; s + kPeriod <= stages; s += kPeriod) {
-        tiled_unrolled(std::make_integer_sequence<int, kPeriod>(),
-                       [&](auto ph_c) __attribute__((always_inline)) { stage(ph_c, s + decltype(ph_c)::value); });
-        if (kBlocked) {
-#pragma unroll
-            for (int i = 0; i < MT; ++i)
-#pragma unroll
-                for (int j = 0; j < NT; ++j) {
-                    total[kBlocked ? i : 0][kBlocked ? j : 0] += acc[i][j];
-                    acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-                }
-        }
+        tiled_unrolled(std::make_integer_sequence<int, kPeriod>(), [&](auto ph_c) __attribute__((always_inline)) {
+            stage(ph_c, s + decltype(ph_c)::value);
+            if constexpr (set_aside_behind(decltype(ph_c)::value)) set_aside();
+        });
     }
     tiled_unrolled(std::make_integer_sequence<int, kPeriod - 1>(), [&](auto ph_c) __attribute__((always_inline)) {
         if (s + decltype(ph_c)::value < stages) stage(ph_c, s + decltype(ph_c)::value);
+        if constexpr (set_aside_behind(decltype(ph_c)::value)) set_aside();
     });
     if (kBlocked) {
 #pragma unroll
         for (int i = 0; i < MT; ++i)
 #pragma unroll
-            for (int j = 0; j < NT; ++j) acc[i][j] += total[kBlocked ? i : 0][kBlocked ? j : 0];
+            for (int j = 0; j < NT; ++j) {
+                if (FINE) acc[i][j] += low[FINE ? i : 0][FINE ? j : 0];
+                acc[i][j] += total[kBlocked ? i : 0][kBlocked ? j : 0];
+            }
     }
     __builtin_amdgcn_s_waitcnt(vmcnt_only(0));      // no write into LDS may be outstanding when the workgroup ends
 
@@ -621,11 +643,11 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_tiled_kernel(const _Float16*
     else store_tile(std::false_type{});
 }
 
-template <int MT, int NT, int KS, int kBufs, int kBBufs = kBufs>
+template <int MT, int NT, int KS, int kBufs, int kBBufs = kBufs, bool FINE = false>
 int launch_tiles(hipStream_t stream, const _Float16* hi, const _Float16* lo, const float* row_scale, TiledMats mats, int M, int K, int k_splits) {
     constexpr int BM = 32 * MT, BN = 32 * NT, bytes = kBufs * 2 * BM * 64 * KS + kBBufs * BN * 128;
     static_assert(bytes <= 160 * 1024);
-    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_tiled_kernel<MT, NT, KS, kBufs, kBBufs>),
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_tiled_kernel<MT, NT, KS, kBufs, kBBufs, FINE>),
                                                        hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
     if (attr != hipSuccess) return -2;
     const int tiles_m = (M + BM - 1) / BM;
@@ -639,7 +661,7 @@ int launch_tiles(hipStream_t stream, const _Float16* hi, const _Float16* lo, con
     // 157 / 165 / 157 / 146 / 140 / 141 / 141; M 2048, N 11264, K 2048 174 / 200 / 175 / 162 / 163 / 159 / 161.  M 522, N 2048, K 5632 on 64 x 128 (9 tile rows), bands of 1 / 3 / 5 /
     // 9: 44.7 / 46.8 / 45.9 / 43.7
     const int band = tiles_m <= 9 ? tiles_m : 6;
-    gemm_tiled_kernel<MT, NT, KS, kBufs, kBBufs><<<(unsigned)(tiles_m * tiles_n * k_splits), kThreads, bytes, stream>>>(hi, lo, row_scale, mats, M, K, k_splits, band);
+    gemm_tiled_kernel<MT, NT, KS, kBufs, kBBufs, FINE><<<(unsigned)(tiles_m * tiles_n * k_splits), kThreads, bytes, stream>>>(hi, lo, row_scale, mats, M, K, k_splits, band);
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 
@@ -824,8 +846,8 @@ int enqueue_tiled(const M40StreamScratch& sc, hipStream_t stream, const TiledCal
     switch (plan.choice.shape) {
         case 0: rc = launch_tiles<4, 8, 1, 4, 3>(stream, hi, lo, row_scale, launch, M, K, k_splits); break;
         case 1: rc = launch_tiles<4, 4, 1, 6, 3>(stream, hi, lo, row_scale, launch, M, K, k_splits); break;
-        case 2: rc = launch_tiles<2, 4, 2, 5>(stream, hi, lo, row_scale, launch, M, K, k_splits); break;
-        case 3: rc = launch_tiles<2, 2, 2, 6>(stream, hi, lo, row_scale, launch, M, K, k_splits); break;
+        case 2: rc = M <= 64 ? launch_tiles<2, 4, 2, 5, 5, true>(stream, hi, lo, row_scale, launch, M, K, k_splits) : launch_tiles<2, 4, 2, 5>(stream, hi, lo, row_scale, launch, M, K, k_splits); break;
+        case 3: rc = M <= 64 ? launch_tiles<2, 2, 2, 6, 6, true>(stream, hi, lo, row_scale, launch, M, K, k_splits) : launch_tiles<2, 2, 2, 6>(stream, hi, lo, row_scale, launch, M, K, k_splits); break;
     }
     if (rc != 0) return rc;
     if (k_splits > 1 && leave) {
