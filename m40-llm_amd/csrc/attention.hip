@@ -15,6 +15,7 @@
 
 #include <atomic>
 #include <mutex>
+#include <type_traits>
 
 // Fixed chunk-partial buffer of m40llm_ext_attention_last_token_f32_gqa_static_scratch_async: device memory that
 // exists from the moment the code object is loaded, so that entry point never allocates.  Every GPU the library
@@ -61,31 +62,36 @@ constexpr int kWaves = kAttnThreads / 64;
 
 
 // HD in {64, 128}; G = q heads per workgroup (<= 4); S = token rows per lane group; PACKED: the result as operands (a launch of one short row has no time to look
-// it up: 4.35 us instead of 4.29)
+// it up: 4.35 us instead of 4.29).
+//
+// Bound by the vector ALU and a launch's round trips: 32 workgroups of two waves a SIMD, on 32 CUs.  One row of 32 q heads to 4 kv of 64, sized for 512 tokens, us in a
+// recorded chain over caches that no cache holds, before / with the kv heads in turn / columns halved in the join, lane groups joined once, clamped loads without a branch /
+// and as many steps as there are: 64 tokens 3.73 / 3.73 / 3.9 / 2.55; 128 4.22 / 3.73 / 3.9 / 2.73; 256 4.53 / 3.89 / 3.9 / 3.11; 512 5.23 / 4.97 / 4.49 / 4.50.
+// 16 q heads to 2 of 128, 256 tokens 5.05 -> 4.56; 32 to 8 5.11 -> 4.53.
 template <int HD, int G, int S, bool PACKED>
 __global__ __launch_bounds__(kAttnThreads, 2) void attn_partial_kernel(AttnParams p) {
     constexpr int LPT = HD / 8;      // lanes per token row
     constexpr int TPW = 64 / LPT;    // token rows per wave load
-    __shared__ float red[kWaves][G][HD];
+    constexpr uint32_t kChunk = kWaves * TPW * S;
+    __shared__ __attribute__((aligned(16))) float red[kWaves][G][HD];
     __shared__ float wmax[kWaves][G];
     __shared__ float wsum[kWaves][G];
 
+    // Neighbouring workgroups take the kv heads in turn: with 2, 4 or 8 of them a die of the eight then reads the rows of one, not of all, for its heads
+    const uint32_t kvh = blockIdx.x % p.kv_heads, sub = blockIdx.x / p.kv_heads;
+    const uint32_t group = p.q_heads / p.kv_heads;
+    const uint32_t qh0 = kvh * group + sub * G;          // first q head of this workgroup
+    const uint32_t gcount = (sub * G + G <= group) ? G : group - sub * G;
     const uint32_t b = blockIdx.z;
     const uint32_t seq_id = p.seq_ids_dev ? p.seq_ids_dev[b] : p.seq_id;
-    const uint32_t len = p.seq_lens_dev ? p.seq_lens_dev[b] + p.len_bias : p.seq_len;
+    const uint32_t len = p.length(b);
     if (len == 0 || len > p.max_seq_len) return;
     if (p.max_batch != 0 && seq_id >= p.max_batch) return;
     const uint32_t t0 = (p.window != 0 && len > p.window) ? len - p.window : 0;
     if (len - t0 > p.span_limit) return;      // longer than the launch was sized for: the row is skipped
-    const uint32_t cbeg = t0 + blockIdx.y * p.chunk;
+    const uint32_t cbeg = t0 + blockIdx.y * kChunk;
     if (cbeg >= len) return;
-    const uint32_t cend = cbeg + p.chunk < len ? cbeg + p.chunk : len;
-
-    const uint32_t kvh = blockIdx.x / p.subgroups;
-    const uint32_t sub = blockIdx.x % p.subgroups;
-    const uint32_t group = p.q_heads / p.kv_heads;
-    const uint32_t qh0 = kvh * group + sub * G;          // first q head of this workgroup
-    const uint32_t gcount = (sub * G + G <= group) ? G : group - sub * G;
+    const uint32_t cend = cbeg + kChunk < len ? cbeg + kChunk : len;
 
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int c = lane % LPT, tg = lane / LPT;
@@ -95,101 +101,114 @@ __global__ __launch_bounds__(kAttnThreads, 2) void attn_partial_kernel(AttnParam
     const uint16_t* Vb = p.V + base;
     const float inv_sqrt = HD == 64 ? 0.125f : 0.08838834764831845f;
 
-    // every load of this lane, issued before anything waits on memory
-    uint4 kw[S], vw[S];
-    bool valid[S];
+    float mh[G], lsum[G], acc[G][8];
+    // One pass over the chunk's rows, with half, a quarter or one of its steps where they fill no more: a recorded step is sized for more tokens than its row has by
+    // now, and arithmetic on rows that are not there took 1.1 us of 3.7.  A test at each step instead keeps the steps of a full chunk from overlapping (5.2 -> 5.5).
+    const auto pass = [&](auto n_steps) {
+        constexpr int NS = decltype(n_steps)::value;
+        // every load of this lane, issued before anything waits on memory
+        uint4 kw[NS], vw[NS];
+        bool valid[NS];
 #pragma unroll
-    for (int s = 0; s < S; ++s) {
-        const uint32_t t = cbeg + (uint32_t)((s * kWaves + wave) * TPW + tg);
-        valid[s] = t < cend;
-        kw[s] = make_uint4(0, 0, 0, 0);
-        vw[s] = make_uint4(0, 0, 0, 0);
-        if (valid[s]) {
-            kw[s] = *reinterpret_cast<const uint4*>(Kb + (size_t)t * row_stride);
-            vw[s] = *reinterpret_cast<const uint4*>(Vb + (size_t)t * row_stride);
+        for (int s = 0; s < NS; ++s) {
+            const uint32_t t = cbeg + (uint32_t)((s * kWaves + wave) * TPW + tg);
+            valid[s] = t < cend;
+            const size_t at = (size_t)(valid[s] ? t : cend - 1u) * row_stride;
+            kw[s] = *reinterpret_cast<const uint4*>(Kb + at);
+            vw[s] = *reinterpret_cast<const uint4*>(Vb + at);
         }
-    }
-    float q[G][8];
-#pragma unroll
-    for (int h = 0; h < G; ++h) {
-        const uint32_t qh = qh0 + (h < (int)gcount ? h : 0);
-        const float* qp = p.Q + ((size_t)b * p.q_heads + qh) * HD + 8 * c;
-        const float4 q0 = *reinterpret_cast<const float4*>(qp);
-        const float4 q1 = *reinterpret_cast<const float4*>(qp + 4);
-        q[h][0] = q0.x; q[h][1] = q0.y; q[h][2] = q0.z; q[h][3] = q0.w;
-        q[h][4] = q1.x; q[h][5] = q1.y; q[h][6] = q1.z; q[h][7] = q1.w;
-    }
-
-    // ---- scores (every lane of a row group ends up with the row's score) -----------------------
-    float sc[S][G];
-    float lmax[G];
-#pragma unroll
-    for (int h = 0; h < G; ++h) lmax[h] = -INFINITY;
-#pragma unroll
-    for (int s = 0; s < S; ++s) {
-        float kf[8];
-        m40_unpack8(kw[s], kf);
+        float q[G][8];
 #pragma unroll
         for (int h = 0; h < G; ++h) {
-            float d = 0.0f;
-#pragma unroll
-            for (int j = 0; j < 8; ++j) d = fmaf(q[h][j], kf[j], d);
-            d = LPT == 8 ? m40_sum8(d) : m40_sum16(d);
-            sc[s][h] = valid[s] ? d * inv_sqrt : -INFINITY;
-            lmax[h] = fmaxf(lmax[h], sc[s][h]);
+            const uint32_t qh = qh0 + (h < (int)gcount ? h : 0);
+            const float* qp = p.Q + ((size_t)b * p.q_heads + qh) * HD + 8 * c;
+            const float4 q0 = *reinterpret_cast<const float4*>(qp);
+            const float4 q1 = *reinterpret_cast<const float4*>(qp + 4);
+            q[h][0] = q0.x; q[h][1] = q0.y; q[h][2] = q0.z; q[h][3] = q0.w;
+            q[h][4] = q1.x; q[h][5] = q1.y; q[h][6] = q1.z; q[h][7] = q1.w;
         }
-    }
-#pragma unroll
-    for (int h = 0; h < G; ++h) {
-        const float m = m40_max64(lmax[h]);
-        if (lane == 0) wmax[wave][h] = m;
-    }
-    __syncthreads();
-    float mh[G];
-#pragma unroll
-    for (int h = 0; h < G; ++h) {
-        float m = wmax[0][h];
-#pragma unroll
-        for (int w = 1; w < kWaves; ++w) m = fmaxf(m, wmax[w][h]);
-        mh[h] = m;
-    }
 
-    // ---- exp, row sums, weighted V -----------------------------------------------------------
-    float lsum[G];
-    float acc[G][8];
+        // ---- scores (every lane of a row group ends up with the row's score) -----------------------
+        float sc[NS][G];
+        float lmax[G];
 #pragma unroll
-    for (int h = 0; h < G; ++h) {
-        lsum[h] = 0.0f;
+        for (int h = 0; h < G; ++h) lmax[h] = -INFINITY;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) acc[h][j] = 0.0f;
-    }
+        for (int s = 0; s < NS; ++s) {
+            float kf[8];
+            m40_unpack8(kw[s], kf);
 #pragma unroll
-    for (int s = 0; s < S; ++s) {
-        float vf[8];
-        m40_unpack8(vw[s], vf);
+            for (int h = 0; h < G; ++h) {
+                float d = 0.0f;
+#pragma unroll
+                for (int j = 0; j < 8; ++j) d = fmaf(q[h][j], kf[j], d);
+                d = LPT == 8 ? m40_sum8(d) : m40_sum16(d);
+                sc[s][h] = valid[s] ? d * inv_sqrt : -INFINITY;
+                lmax[h] = fmaxf(lmax[h], sc[s][h]);
+            }
+        }
 #pragma unroll
         for (int h = 0; h < G; ++h) {
-            const float e = valid[s] ? expf(sc[s][h] - mh[h]) : 0.0f;
-            if (c == 0) lsum[h] += e;
-#pragma unroll
-            for (int j = 0; j < 8; ++j) acc[h][j] = fmaf(e, vf[j], acc[h][j]);
+            const float m = m40_max_lanes_from<LPT>(lmax[h]);
+            if (lane == 0) wmax[wave][h] = m;
         }
-    }
-    // join the TPW token rows of the wave (lanes with equal c), then the waves
+        __syncthreads();
+#pragma unroll
+        for (int h = 0; h < G; ++h) {
+            float m = wmax[0][h];
+#pragma unroll
+            for (int w = 1; w < kWaves; ++w) m = fmaxf(m, wmax[w][h]);
+            mh[h] = m;
+        }
+
+        // ---- exp, row sums, weighted V -----------------------------------------------------------
+#pragma unroll
+        for (int h = 0; h < G; ++h) {
+            lsum[h] = 0.0f;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) acc[h][j] = 0.0f;
+        }
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+            float vf[8];
+            if (!valid[s]) vw[s] = make_uint4(0, 0, 0, 0);      // the last row once more: an infinity there counts once
+            m40_unpack8(vw[s], vf);
+#pragma unroll
+            for (int h = 0; h < G; ++h) {
+                const float e = valid[s] ? expf(sc[s][h] - mh[h]) : 0.0f;
+                lsum[h] += e;
+#pragma unroll
+                for (int j = 0; j < 8; ++j) acc[h][j] = fmaf(e, vf[j], acc[h][j]);
+            }
+        }
+    };
+    const uint32_t steps = (cend - cbeg + kWaves * TPW - 1) / (kWaves * TPW);
+    if (S == 1 || steps > S / 2) pass(std::integral_constant<int, S>());
+    else if (S == 2 || steps > S / 4) pass(std::integral_constant<int, S < 2 ? 1 : S / 2>());
+    else if (S == 8 && steps > 1) pass(std::integral_constant<int, S < 4 ? 1 : S / 4>());
+    else pass(std::integral_constant<int, 1>());
+
+    // Join the TPW token rows of the wave (lanes with equal c): each exchange leaves a lane half of the columns to go on with, at the end two of its eight.
 #pragma unroll
     for (int h = 0; h < G; ++h) {
+        float* a = acc[h];
+        if (LPT == 8) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            acc[h][j] = m40_sum_lanes_from<LPT>(acc[h][j]);
+            for (int j = 0; j < 8; ++j) a[j] += m40_dpp_f<M40_DPP_ROW_ROR8>(a[j]);
         }
-        const float ssum = m40_sum64(lsum[h]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            m40_swap_rows16(a[j], a[j + 4]);
+            a[j] += a[j + 4];
+        }
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            m40_swap_rows32(a[j], a[j + 2]);
+            a[j] += a[j + 2];
+        }
+        const float ssum = m40_sum_lanes_from<LPT>(lsum[h]);
         if (lane == 0) wsum[wave][h] = ssum;
-    }
-    if (tg == 0) {
-#pragma unroll
-        for (int h = 0; h < G; ++h)
-#pragma unroll
-            for (int j = 0; j < 8; ++j) red[wave][h][8 * c + j] = acc[h][j];
+        if (LPT == 16 || (lane & 8) == 0) *reinterpret_cast<float2*>(&red[wave][h][8 * c + ((lane & 16) >> 2) + ((lane & 32) >> 4)]) = make_float2(a[0], a[1]);
     }
     __syncthreads();
 
@@ -206,28 +225,27 @@ __global__ __launch_bounds__(kAttnThreads, 2) void attn_partial_kernel(AttnParam
         if (final_out) {
             const float denom = l > 0.0f ? l : 1.0f;
             if constexpr (PACKED) m40_attn_store<HD>(p, b, qh, d, v / denom);
-            else p.Out[((size_t)b * p.q_heads + qh) * HD + d] = v / denom;
+            else static_cast<float*>(p.out)[((size_t)b * p.q_heads + qh) * HD + d] = v / denom;
         } else {
             const size_t at = ((size_t)b * p.q_heads + qh) * p.nchunks + blockIdx.y;
             p.ws[at * HD + d] = v;
-            if (d == 0) reinterpret_cast<float2*>(p.ml)[at] = make_float2(mh[h], l);
+            if (d == 0) p.ml()[at] = make_float2(mh[h], l);
         }
     }
 }
 
 // Merge chunk partials: grid (q_heads, batch), 256 threads
 template <int HD>
-__global__ __launch_bounds__(256) void attn_combine_kernel(const float* ws, const float* ml, const uint32_t* seq_lens_dev, const uint32_t* seq_ids_dev, uint32_t nchunks,
-                                                           uint32_t q_heads, AttnParams p) {
+__global__ __launch_bounds__(256) void attn_combine_kernel(AttnParams p) {
     __shared__ __attribute__((aligned(16))) float sums[4][HD];
     const uint32_t qh = blockIdx.x, b = blockIdx.y;
-    const size_t first = ((size_t)b * q_heads + qh) * nchunks;
+    const size_t first = ((size_t)b * p.q_heads + qh) * p.nchunks;
     M40ChunkMerge<HD> merge;
-    merge.request(ws + first * HD, reinterpret_cast<const float2*>(ml) + first, nchunks);
-    const uint32_t len = seq_lens_dev ? seq_lens_dev[b] + p.len_bias : p.seq_len;
-    const uint32_t sid = (p.max_batch != 0 && seq_ids_dev) ? seq_ids_dev[b] : 0u;
+    merge.request(p.ws + first * HD, p.ml() + first, p.nchunks);
+    const uint32_t len = p.length(b);
+    const uint32_t sid = (p.max_batch != 0 && p.seq_ids_dev) ? p.seq_ids_dev[b] : 0u;
     if (len == 0 || len > p.max_seq_len) return;
-    if (p.max_batch != 0 && seq_ids_dev && sid >= p.max_batch) return;
+    if (p.max_batch != 0 && p.seq_ids_dev && sid >= p.max_batch) return;
     const uint32_t t0 = (p.window != 0 && len > p.window) ? len - p.window : 0;
     if (len - t0 > p.span_limit) return;      // longer than the launch was sized for: the row is skipped
     const float y = merge.finish((len - t0 + p.chunk - 1) / p.chunk, sums);
@@ -241,7 +259,7 @@ __global__ __launch_bounds__(64) void attn_generic_kernel(AttnParams p, uint32_t
     const uint32_t d = blockIdx.x * 64 + threadIdx.x;
     if (d >= head_dim) return;
     const uint32_t seq_id = p.seq_ids_dev ? p.seq_ids_dev[b] : p.seq_id;
-    const uint32_t len = p.seq_lens_dev ? p.seq_lens_dev[b] + p.len_bias : p.seq_len;
+    const uint32_t len = p.length(b);
     if (len == 0 || len > p.max_seq_len) return;
     const uint32_t t0 = (p.window != 0 && len > p.window) ? len - p.window : 0;
     if (len - t0 > p.span_limit) return;      // longer than the launch was sized for: the row is skipped
@@ -266,7 +284,7 @@ __global__ __launch_bounds__(64) void attn_generic_kernel(AttnParams p, uint32_t
         acc += e * m40_h2f(Vb[(size_t)t * ept + d]);
     }
     den = den > 0.0f ? den : 1.0f;
-    p.Out[((size_t)b * p.q_heads + qh) * head_dim + d] = acc / den;
+    static_cast<float*>(p.out)[((size_t)b * p.q_heads + qh) * head_dim + d] = acc / den;
 }
 
 template <int HD, int G, int S>
@@ -286,16 +304,23 @@ void launch_g(hipStream_t stream, const AttnParams& p, uint32_t batch, int S) {
     }
 }
 
+template <int HD>
+void launch_combine(hipStream_t stream, const AttnParams& p, uint32_t batch) {
+    attn_combine_kernel<HD><<<dim3(p.q_heads, batch), 256, 0, stream>>>(p);
+}
+
 // Chooses rows per lane group (S), q heads per workgroup (G) and the chunking for a span of `span` tokens.
 template <int HD>
 int launch_hd(M40llmCudaContext* ctx, hipStream_t stream, float* partial, size_t partial_bytes, bool fixed_chunking,
               AttnParams& p, uint32_t batch, uint32_t group, uint32_t span) {
     constexpr uint32_t kRowsPerStep = kWaves * (64 / (HD / 8));   // token rows one workgroup covers per S
-    // Short rows of a batch: a launch of the vector-ALU kernel grows with the q heads of all rows, the matrix-core kernel and its merge hardly do.  From 512 of them on (128
-    // where the rows take two launches either way) they are the faster ones; us, vector ALU / matrix cores, 32 q heads to 4 kv of 64, up to 512 tokens: 8 rows of 100
-    // 6.4 / 6.9, of 500 7.8 / 7.2, 16 rows of 100 9.8 / 7.0, of 500 10.9 / 7.8, 32 rows 10.3 / 7.8 and 12.8 / 9.4; 16 to 2 of 128, 250 tokens: 16 rows 7.9 / 8.9, 32 rows
-    // 11.1 / 9.2; 500 tokens: 4 rows 8.2 / 8.8, 8 rows 11.0 / 8.8, 32 rows 16.7 / 10.6; 32 to 8 of 128, 500 tokens: 2 rows 8.2 / 8.4, 4 rows 11.0 / 8.6.
-    const bool many_heads = batch > 1 && batch * p.q_heads >= (span > kRowsPerStep * 8 ? 128u : 512u);
+    // Short rows of a batch: a launch of the vector-ALU kernel grows with the q heads of all rows, the matrix-core kernel and its merge (none up to 128 tokens) hardly do.
+    // us, vector ALU / matrix cores.  Up to 128 tokens, 512 q heads: 32 to 4 kv of 64 5.1 / 4.6, 16 to 2 of 128 6.2 / 6.2, 32 to 8 of 128 6.2 / 5.9 (256 heads: 3.9 / 6.8,
+    // 5.0 / 6.1).  Half the steps of a chunk of head size 64 (250 tokens): 512 6.2 / 7.3, 1024 6.7 / 8.3, 2048 10.3 / 6.2.  A whole chunk: of 64 (500) 256 heads 6.2 / 7.2,
+    // 512 8.8 / 7.8; of 128 (250) 512 9.2 / 9.25 and 10.1 / 10.5, 1024 11.3 / 10.2.  Chunks and a merge either way (128, 500 tokens): 128 heads 8.2 / 8.8 and 7.6 / 8.6,
+    // 256 11.2 / 8.9 and 10.6 / 10.3.
+    const uint32_t many = span <= 128 ? 512u : span <= kRowsPerStep * 4 ? 2048u : span > kRowsPerStep * 8 ? 256u : HD == 64 ? 512u : 1024u;
+    const bool many_heads = batch > 1 && batch * p.q_heads >= many;
     if ((span > 512 || many_heads) && m40_aligned16(p.Q)) {
         // long rows: matrix-core kernel (it reads q with 16-byte loads).  Chunks are a multiple of 128 tokens (one
         // 32-token tile per wave and pass) sized for about one workgroup per CU -- measured best at 32 K tokens (256
@@ -321,11 +346,10 @@ int launch_hd(M40llmCudaContext* ctx, hipStream_t stream, float* partial, size_t
             chunk *= 2;
         }
         p.ws = partial;
-        p.ml = partial + (size_t)batch * p.q_heads * p.nchunks * HD;
+        p.ml_from = (uint32_t)((size_t)batch * p.q_heads * p.nchunks * HD);
         m40_launch_attn_mfma(stream, p, HD, batch);
         if (p.nchunks > 1) {
-            dim3 grid(p.q_heads, batch);
-            attn_combine_kernel<HD><<<grid, 256, 0, stream>>>(p.ws, p.ml, p.seq_lens_dev, p.seq_ids_dev, p.nchunks, p.q_heads, p);
+            launch_combine<HD>(stream, p, batch);
         }
         return 0;
     }
@@ -360,15 +384,14 @@ int launch_hd(M40llmCudaContext* ctx, hipStream_t stream, float* partial, size_t
         }
     }
     p.ws = partial;
-    p.ml = partial + (size_t)batch * p.q_heads * p.nchunks * HD;
+    p.ml_from = (uint32_t)((size_t)batch * p.q_heads * p.nchunks * HD);
     switch (G) {
         case 4: launch_g<HD, 4>(stream, p, batch, S); break;
         case 2: launch_g<HD, 2>(stream, p, batch, S); break;
         default: launch_g<HD, 1>(stream, p, batch, S); break;
     }
     if (p.nchunks > 1) {
-        dim3 grid(p.q_heads, batch);
-        attn_combine_kernel<HD><<<grid, 256, 0, stream>>>(p.ws, p.ml, p.seq_lens_dev, p.seq_ids_dev, p.nchunks, p.q_heads, p);
+        launch_combine<HD>(stream, p, batch);
     }
     return 0;
 }
@@ -378,13 +401,13 @@ int launch_hd(M40llmCudaContext* ctx, hipStream_t stream, float* partial, size_t
 int m40_launch_dense_attention(M40llmCudaContext* ctx, hipStream_t stream, uint32_t stream_kind,
                                const M40AttnArgs& a) {
     AttnParams p{};
-    p.K = a.K; p.V = a.V; p.Q = a.Q; p.Out = a.Out;
-    p.packed = a.packed; p.packed_pad = (uint32_t)m40_packed_pad((int)a.batch);
+    p.K = a.K; p.V = a.V; p.Q = a.Q;
+    p.out = a.packed ? static_cast<void*>(a.packed) : a.Out;
+    p.packed = a.packed ? (uint32_t)m40_packed_pad((int)a.batch) : 0u;
     p.seq_ids_dev = a.seq_ids_dev; p.seq_lens_dev = a.seq_lens_dev;
-    p.seq_id = a.seq_id; p.seq_len = a.seq_len;
+    p.seq_id = a.seq_id; p.len_or_bias = a.seq_lens_dev ? a.len_bias : a.seq_len;
     p.max_seq_len = a.max_seq_len; p.kv_heads = a.kv_heads; p.q_heads = a.q_heads; p.window = a.window;
     p.subgroups = 1;
-    p.len_bias = a.len_bias;
     p.max_batch = a.max_batch;
     (void)hipGetLastError();
     const uint32_t group = a.q_heads / a.kv_heads;

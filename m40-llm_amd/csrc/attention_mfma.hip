@@ -42,13 +42,12 @@ __device__ __forceinline__ float max16(float x) {   // over rows of 16 lanes
 }
 __device__ __forceinline__ uint16_t f16_bits(float x) { return __builtin_bit_cast(uint16_t, static_cast<_Float16>(x)); }
 
-// What the first requests need is passed on its own, in registers when a wave starts; the structure is read from memory meanwhile.  q goes out before the row's
-// length and id are known, K and V as soon as they are, K ahead of V: scores and softmax are formed while V is on its way.  (All behind the structure, V waited for
-// ahead of the scores: 8 rows of up to 4093 tokens, head size 128, 12.6 us with the merge, now 12.5; 16 rows of up to 1200 11.9 / 11.4; 2 rows of up to 3000 8.9 / 8.8.
+// q goes out before the row's length and id are known, K and V as soon as they are, K ahead of V: scores and softmax are formed while V is on its way.  (V waited for
+// ahead of the scores: 8 rows of up to 4093 tokens, head size 128, 12.6 us with the merge, now 12.4; 16 rows of up to 1200 11.9 / 11.4; 2 rows of up to 3000 8.9 / 8.9.
+// What the first requests need as arguments of their own, in registers when a wave starts, saves 0.1 us of these and costs a call of one row 0.5 us on the host.
 // Eight waves with a tile each instead of four with two are no faster, 16 rows a quarter slower; K in whole lines through LDS neither, 12.5 -> 13.1 us.)
 template <int HD>
-__global__ __launch_bounds__(kThreads, 2) void attn_mfma_kernel(const uint16_t* K, const uint16_t* V, const float* Q, const uint32_t* ids_dev, const uint32_t* lens_dev,
-                                                                 uint32_t max_seq_len, uint32_t kv_heads, uint32_t q_heads, uint32_t subgroups, uint32_t chunk, uint32_t len_bias, AttnParams p) {
+__global__ __launch_bounds__(kThreads, 2) void attn_mfma_kernel(AttnParams p) {
     constexpr int KS = HD / 32;            // MFMA k-steps of a score tile
     constexpr int DT = HD / 16;            // 16-column output tiles
     constexpr int RS = HD * 2 + 8;         // LDS bytes per V row (8-byte aligned, spreads the row groups over the banks)
@@ -61,11 +60,11 @@ __global__ __launch_bounds__(kThreads, 2) void attn_mfma_kernel(const uint16_t* 
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int c16 = lane & 15, g = lane >> 4;
     const uint32_t b = blockIdx.z;
-    const uint32_t kvh = blockIdx.x / subgroups, sub = blockIdx.x % subgroups;
-    const uint32_t group = q_heads / kv_heads;
+    const uint32_t kvh = blockIdx.x / p.subgroups, sub = blockIdx.x % p.subgroups;
+    const uint32_t group = p.q_heads / p.kv_heads;
     const uint32_t qh0 = kvh * group + sub * 8u;
     const uint32_t gcount = (sub * 8u + 8u <= group) ? 8u : group - sub * 8u;
-    const float* Qb = Q + ((size_t)b * q_heads + qh0) * HD;      // gcount heads, contiguous
+    const float* Qb = p.Q + ((size_t)b * p.q_heads + qh0) * HD;      // gcount heads, contiguous
     // A-operand row rho = c16: head 2*(rho/4) + (rho%4)/2, part rho&1 (0 hi, 1 lo)
     const uint32_t qhead = 2u * (uint32_t)(c16 >> 2) + (uint32_t)((c16 & 3) >> 1);
     const bool q_live = qhead < gcount;
@@ -79,20 +78,20 @@ __global__ __launch_bounds__(kThreads, 2) void attn_mfma_kernel(const uint16_t* 
         }
     }
     __builtin_amdgcn_sched_barrier(0);
-    const uint32_t seq_id = ids_dev ? ids_dev[b] : p.seq_id;
-    const uint32_t len = lens_dev ? lens_dev[b] + len_bias : p.seq_len;
-    if (len == 0 || len > max_seq_len) return;
+    const uint32_t seq_id = p.seq_ids_dev ? p.seq_ids_dev[b] : p.seq_id;
+    const uint32_t len = p.length(b);
+    if (len == 0 || len > p.max_seq_len) return;
     if (p.max_batch != 0 && seq_id >= p.max_batch) return;
     const uint32_t t0 = (p.window != 0 && len > p.window) ? len - p.window : 0;
     if (len - t0 > p.span_limit) return;      // longer than the launch was sized for: the row is skipped
-    const uint32_t cbeg = t0 + blockIdx.y * chunk;
+    const uint32_t cbeg = t0 + blockIdx.y * p.chunk;
     if (cbeg >= len) return;
-    const uint32_t cend = cbeg + chunk < len ? cbeg + chunk : len;
+    const uint32_t cend = cbeg + p.chunk < len ? cbeg + p.chunk : len;
     const uint32_t ntok = cend - cbeg;
 
-    const size_t row_stride = (size_t)kv_heads * HD;
-    const uint16_t* Kb = K + ((size_t)seq_id * max_seq_len) * row_stride + (size_t)kvh * HD;
-    const uint16_t* Vb = V + ((size_t)seq_id * max_seq_len) * row_stride + (size_t)kvh * HD;
+    const size_t row_stride = (size_t)p.kv_heads * HD;
+    const uint16_t* Kb = p.K + ((size_t)seq_id * p.max_seq_len) * row_stride + (size_t)kvh * HD;
+    const uint16_t* Vb = p.V + ((size_t)seq_id * p.max_seq_len) * row_stride + (size_t)kvh * HD;
 
     // ---- the first tile's loads
     uint4 kreg[2][KS], vreg[DT];
@@ -264,7 +263,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_mfma_kernel(const uint16_t* 
         } else {
             const size_t at = ((size_t)b * p.q_heads + qh) * p.nchunks + blockIdx.y;
             p.ws[at * HD + d] = num;
-            if (d == 0) reinterpret_cast<float2*>(p.ml)[at] = make_float2(M, den);
+            if (d == 0) p.ml()[at] = make_float2(M, den);
         }
     }
 }
@@ -274,5 +273,5 @@ __global__ __launch_bounds__(kThreads, 2) void attn_mfma_kernel(const uint16_t* 
 void m40_launch_attn_mfma(hipStream_t stream, const AttnParams& p, uint32_t head_dim, uint32_t batch) {
     dim3 grid(p.kv_heads * p.subgroups, p.nchunks, batch);
     const auto kernel = head_dim == 64 ? attn_mfma_kernel<64> : attn_mfma_kernel<128>;
-    kernel<<<grid, kThreads, 0, stream>>>(p.K, p.V, p.Q, p.seq_ids_dev, p.seq_lens_dev, p.max_seq_len, p.kv_heads, p.q_heads, p.subgroups, p.chunk, p.len_bias, p);
+    kernel<<<grid, kThreads, 0, stream>>>(p);
 }

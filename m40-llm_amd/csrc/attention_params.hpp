@@ -3,32 +3,35 @@
 
 #include "packed_rows.hpp"
 
+// One argument of 112 bytes for each kernel: launches one by one are bound by the host, and more bytes or the members as arguments of their own cost it time (one row,
+// one launch: 3.6 us, 4.2 with 136 bytes, 4.5 as ten arguments; two launches 7.0, 8.0 with eleven and nine).
 struct AttnParams {
     const uint16_t* K;
     const uint16_t* V;
     const float* Q;
-    float* Out;
-    uint8_t* packed;              // not null: rows as operands of the next product (packed_rows.hpp) instead of Out
-    uint32_t packed_pad;
+    void* out;                    // f32 rows, or with `packed` rows as operands of the next product (packed_rows.hpp)
     float* ws;                    // partials: sums [batch][q_heads][nchunks][hd], behind them
-    float* ml;                    // [batch][q_heads][nchunks][2]: maximum and denominator
     const uint32_t* seq_ids_dev;  // may be null
     const uint32_t* seq_lens_dev; // may be null
-    uint32_t seq_id, seq_len;
+    uint32_t ml_from;             // [batch][q_heads][nchunks][2]: maximum and denominator, that many floats behind ws
+    uint32_t packed;              // 0, or the operands' padded rows
+    uint32_t seq_id;
+    uint32_t len_or_bias;         // the length, or what is added to a device-side one (position -> length)
     uint32_t max_seq_len, kv_heads, q_heads, window;
     uint32_t chunk, nchunks;
     uint32_t subgroups;           // q-head subgroups per kv head
-    uint32_t len_bias;            // added to a device-side length (position -> length)
     uint32_t max_batch;           // device-side sequence ids at or above this are skipped (0 = not checked)
     uint32_t span_limit;          // tokens a row may attend (the length bound the grid and chunking were sized for): rows
                                   // whose device-side length asks for more are skipped
+    __device__ __forceinline__ uint32_t length(uint32_t b) const { return seq_lens_dev ? seq_lens_dev[b] + len_or_bias : len_or_bias; }
+    __device__ __forceinline__ float2* ml() const { return reinterpret_cast<float2*>(ws + ml_from); }
 };
 
 // Element d of q head qh of row b; called by the lanes of whole groups of eight d.
 template <int HD>
 __device__ __forceinline__ void m40_attn_store(const AttnParams& p, uint32_t b, uint32_t qh, uint32_t d, float y) {
-    if (p.packed) m40_store_packed(p.packed, (int)p.packed_pad, (int)p.q_heads * HD, (int)b, (int)(qh * HD + d), y);
-    else p.Out[((size_t)b * p.q_heads + qh) * HD + d] = y;
+    if (p.packed) m40_store_packed(static_cast<uint8_t*>(p.out), (int)p.packed, (int)p.q_heads * HD, (int)b, (int)(qh * HD + d), y);
+    else static_cast<float*>(p.out)[((size_t)b * p.q_heads + qh) * HD + d] = y;
 }
 
 // One head's chunk partials (sums [chunks][HD], pairs of maximum and denominator [chunks]) merged by a workgroup of 256: HD / 4 lanes take a chunk's sums, four

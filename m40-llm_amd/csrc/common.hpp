@@ -344,6 +344,12 @@ __device__ __forceinline__ float m40_max64(float x) {
     x = m40_max_xor32(x);
     return x;
 }
+template <int FROM>
+__device__ __forceinline__ float m40_max_lanes_from(float v) {
+    static_assert(FROM == 8 || FROM == 16, "see m40_sum_lanes_from");
+    if (FROM <= 8) v = fmaxf(v, m40_dpp_f<M40_DPP_ROW_ROR8>(v));
+    return m40_max_xor32(m40_max_xor16(v));
+}
 
 __device__ __forceinline__ float m40_inv_sqrt_head_dim(uint32_t hd) {
     return hd == 64u ? 0.125f : (hd == 128u ? 0.08838834764831845f : 1.0f / sqrtf((float)hd));

@@ -44,9 +44,40 @@ def test_merge_of_chunks(dev, qh, kvh, hd, lens, hint):
 
 
 # either side of the number of q heads from which short rows of a batch take the matrix-core kernel: one chunk and several, rows of a token, uneven rows
-@pytest.mark.parametrize("qh,kvh,hd,rows,hint", [(32, 4, 64, 15, 512), (32, 4, 64, 16, 512), (8, 8, 64, 64, 130), (16, 2, 128, 7, 400), (16, 2, 128, 8, 400), (64, 4, 128, 8, 256), (64, 4, 128, 2, 257)])
+@pytest.mark.parametrize("qh,kvh,hd,rows,hint", [(32, 4, 64, 15, 128), (32, 4, 64, 16, 128), (32, 4, 64, 63, 256), (32, 4, 64, 64, 256), (32, 4, 64, 15, 512), (32, 4, 64, 16, 512),
+                                                 (8, 8, 64, 64, 130), (64, 4, 128, 15, 256), (64, 4, 128, 16, 256), (16, 2, 128, 15, 400), (16, 2, 128, 16, 400), (64, 4, 128, 4, 257)])
 def test_short_rows_of_a_batch(dev, qh, kvh, hd, rows, hint):
     rng = np.random.default_rng(qh + rows)
     lens = rng.integers(1, hint + 1, rows)
     lens[0], lens[-1] = hint, 1
     test_merge_of_chunks(dev, qh, kvh, hd, [int(n) for n in lens], hint)
+
+
+@pytest.mark.parametrize("qh,kvh,hd,hint", [(32, 4, 64, 512), (6, 2, 64, 256), (5, 5, 64, 100), (16, 2, 128, 256), (12, 3, 128, 128), (40, 8, 128, 480)])
+def test_short_row_in_a_launch_for_more(dev, qh, kvh, hd, hint):
+    """Lengths at the edges of the steps of a pass, in a launch sized for `hint` tokens and in one of the row's own size: the same bits; rows behind the end hold NaN, and
+    an infinity in the last one stays an infinity."""
+    rng = np.random.default_rng(hint + hd)
+    L, step = hint + 1, 8 * 512 // hd
+    kv = m40.KVCache(dev.ctx, L, 1, kvh, hd)
+    for n in sorted({1, step - 1, step, step + 1, 2 * step, 2 * step + 1, 4 * step, 4 * step + 1, hint - 1, hint}):
+        if n > hint: continue
+        Kc, Vc = (rng.standard_normal((L, kvh, hd)).astype(np.float16) for _ in range(2))
+        Kc[n:], Vc[n:] = np.nan, np.nan
+        Vc[n - 1, 0, 3] = np.inf
+        dev.fill_dense(kv, 0, Kc.view(np.uint16), Vc.view(np.uint16))
+        q = (2.0 * rng.standard_normal((qh, hd))).astype(np.float32)
+        dq, out, own, pos = dev.up(q), dev.zeros(q.nbytes), dev.zeros(q.nbytes), dev.up(np.array([n - 1], dtype=np.uint32))
+        dev.call("m40llm_ext_attention_last_token_f32_gqa_position_dev_async", kv.h, 0, dq.ptr, qh, pos.ptr, hint, out.ptr)
+        dev.call("m40llm_attention_last_token_f32_gqa_async", kv.h, 0, dq.ptr, qh, n, own.ptr)
+        dev.sync()
+        got = out.download(np.float32, (qh, hd))
+        if hint <= 8 * step: assert np.array_equal(got.view(np.uint32), own.download(np.uint32, (qh, hd)))
+        k, v = (np.repeat(t[:n].astype(np.float64), qh // kvh, axis=1) for t in (Kc, Vc))
+        s = np.einsum("hd,thd->ht", q.astype(np.float64), k) / np.sqrt(hd)
+        w = np.exp(s - s.max(axis=1, keepdims=True))
+        want = np.einsum("ht,thd->hd", w / w.sum(axis=1, keepdims=True), v)
+        # scores of up to 2 hd terms in f32 and sums of n: (hd + n) 2^-24 of values of a few units, with room for exp
+        assert np.array_equal(np.isinf(got), np.isinf(want))
+        keep = np.isfinite(want)
+        assert np.abs(got[keep] - want[keep]).max() <= 4 * (hd + n) * 2.0 ** -24 * np.abs(want[keep]).max() + 1e-6
