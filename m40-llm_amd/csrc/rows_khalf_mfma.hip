@@ -1,5 +1,5 @@
-// Row-batched projection with a long K and few output columns -- the down projection of a batched decode step -- in
-// one launch: out[rows][N] += residual + a[rows][K] . W^T for up to eight activation rows, f16 GGUF weights [N][K].
+// Row-batched projection with a long K and few output columns -- the down projection of a batched decode step whose rows
+// come as f32 (packed_rows.hip takes them as operands) -- in one launch: out[rows][N] += residual + a[rows][K] . W^T for up to eight activation rows, f16 GGUF weights [N][K].
 //
 // A workgroup owns one 16-column tile and one half of K; its eight waves split that half into contiguous runs of
 // MFMA k-steps (32 k each), add their sums in wave order through LDS, and the workgroup ADDS its 16 x rows values

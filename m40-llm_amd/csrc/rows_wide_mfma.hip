@@ -15,7 +15,7 @@
 // four blocks of weights or rows on their way (more code, more registers, waits for what was asked for later) take 0.6 to 1.4 us more a launch.
 // 32 rows, width 2048, feed-forward 5632, against the form that converted chunks of 512 k for all waves between barriers: Q/K/V 13.9 -> 11.5 us, O
 // 7.6 -> 6.7, gate/up 19.0 -> 15.7, down 14.6 -> 11.8, vocabulary of 32000 39.4 -> 35.2; 16 rows 10.1 -> 8.3, 6.2 -> 5.4, 14.6 -> 13.8, 11.4 -> 10.0,
-// 31.4 -> 30.5.  Weight loads are whole 128-byte lines (eight lanes a column) and pass through a wave-private LDS tile into operand order, as in
+// 31.4 -> 30.5.  (O and down of a decode step come as operands and go to packed_rows.hip: 6.0 and 10.8 us; the residual form here is for f32 rows.)  Weight loads are whole 128-byte lines (eight lanes a column) and pass through a wave-private LDS tile into operand order, as in
 // rows_mfma.hip.  A product of few columns onto zeros is cut into two halves of K, which meet in the result element by element: two terms, the
 // same bits in either order.
 #include "packed_rows.hpp"
