@@ -11,6 +11,7 @@
 // Reference semantics: three-pass softmax per q head, kv head = qh / (q_heads / kv_heads),
 // scale literals for head_dim 64 / 128: cuda/kernels.cu:1367-1655, entry points :3837-4023,
 // batched :1740-1823 and :4694-4832.
+#include "attention_chunks.hpp"
 #include "attention_params.hpp"
 
 #include <atomic>
@@ -322,22 +323,13 @@ int launch_hd(M40llmCudaContext* ctx, hipStream_t stream, float* partial, size_t
     const uint32_t many = span <= 128 ? 512u : span <= kRowsPerStep * 4 ? 2048u : span > kRowsPerStep * 8 ? 256u : HD == 64 ? 512u : 1024u;
     const bool many_heads = batch > 1 && batch * p.q_heads >= many;
     if ((span > 512 || many_heads) && m40_aligned16(p.Q)) {
-        // long rows: matrix-core kernel (it reads q with 16-byte loads).  Chunks are a multiple of 128 tokens (one
-        // 32-token tile per wave and pass) sized for about one workgroup per CU -- measured best at 32 K tokens (256
-        // workgroups of 1024 tokens: 32 us against 36 us with twice as many half-sized ones) and on the batch-8 step
-        // -- rounded to the nearest multiple, and up while more than two workgroups would land on a CU.
+        // long rows: matrix-core kernel (it reads q with 16-byte loads)
         p.subgroups = (group + 7) / 8;
         const uint64_t groups = (uint64_t)batch * p.kv_heads * p.subgroups;
-        uint64_t chunk = (((uint64_t)span * groups / ctx->num_cus) + 64) / 128 * 128;
-        // Around half a thousand tokens a chunk two workgroups a CU are better: a wave's tiles follow one another, and two is as many as are worth
-        // waiting for (32 rows of up to 1021 tokens, 4 kv heads of 64: chunks of 512 9.0 us, of 256 7.8 us; 8 rows of up to 4093, 2 kv heads of 128:
-        // chunks of 256 8.8 us, of 128 9.2 us).  One sequence keeps the larger ones where its partials of 256 tokens would not fit the fixed buffer:
-        // with the context's arena and with that buffer the chunks are the same.
+        // One sequence keeps the larger chunks where its partials of 256 tokens would not fit the fixed buffer: with the context's arena and with that buffer the
+        // chunks are the same.
         const size_t need_256 = (size_t)p.q_heads * ((span + 255u) / 256u) * (HD + 2) * sizeof(float);
-        if (chunk > 256 && chunk <= 512 && (batch > 1 || need_256 <= kStaticScratchBytes)) chunk = 256;
-        if (chunk < 128) chunk = 128;
-        while (groups * ((span + chunk - 1) / chunk) > 2ull * ctx->num_cus) chunk += 128;
-        if (chunk > 2048) chunk = 2048;
+        uint64_t chunk = m40_attention_chunk(groups, span, (uint32_t)ctx->num_cus, batch > 1 || need_256 <= kStaticScratchBytes);
         for (;;) {
             p.chunk = (uint32_t)chunk;
             p.nchunks = (span + p.chunk - 1) / p.chunk;

@@ -53,6 +53,14 @@ def test_short_rows_of_a_batch(dev, qh, kvh, hd, rows, hint):
     test_merge_of_chunks(dev, qh, kvh, hd, [int(n) for n in lens], hint)
 
 
+# more rows and kv heads than two workgroups a CU: rows of one chunk, and long rows that then have one as well
+@pytest.mark.parametrize("qh,kvh,hd,rows,hint", [(8, 8, 64, 65, 100), (4, 4, 128, 129, 128), (8, 4, 64, 129, 520), (8, 8, 128, 65, 2100)])
+def test_more_rows_than_the_chip_takes_at_once(dev, qh, kvh, hd, rows, hint):
+    rng = np.random.default_rng(rows + hint)
+    lens = rng.integers(1, min(hint, 600) + 1, rows)
+    lens[0], lens[-1] = hint, 1
+    test_merge_of_chunks(dev, qh, kvh, hd, [int(n) for n in lens], hint)
+
 @pytest.mark.parametrize("qh,kvh,hd,hint", [(32, 4, 64, 512), (6, 2, 64, 256), (5, 5, 64, 100), (16, 2, 128, 256), (12, 3, 128, 128), (40, 8, 128, 480)])
 def test_short_row_in_a_launch_for_more(dev, qh, kvh, hd, hint):
     """Lengths at the edges of the steps of a pass, in a launch sized for `hint` tokens and in one of the row's own size: the same bits; rows behind the end hold NaN, and
