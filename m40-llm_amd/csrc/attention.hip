@@ -315,14 +315,10 @@ template <int HD>
 int launch_hd(M40llmCudaContext* ctx, hipStream_t stream, float* partial, size_t partial_bytes, bool fixed_chunking,
               AttnParams& p, uint32_t batch, uint32_t group, uint32_t span) {
     constexpr uint32_t kRowsPerStep = kWaves * (64 / (HD / 8));   // token rows one workgroup covers per S
-    // Short rows of a batch: a launch of the vector-ALU kernel grows with the q heads of all rows, the matrix-core kernel and its merge (none up to 128 tokens) hardly do.
-    // us, vector ALU / matrix cores.  Up to 128 tokens, 512 q heads: 32 to 4 kv of 64 5.1 / 4.6, 16 to 2 of 128 6.2 / 6.2, 32 to 8 of 128 6.2 / 5.9 (256 heads: 3.9 / 6.8,
-    // 5.0 / 6.1).  Half the steps of a chunk of head size 64 (250 tokens): 512 6.2 / 7.3, 1024 6.7 / 8.3, 2048 10.3 / 6.2.  A whole chunk: of 64 (500) 256 heads 6.2 / 7.2,
-    // 512 8.8 / 7.8; of 128 (250) 512 9.2 / 9.25 and 10.1 / 10.5, 1024 11.3 / 10.2.  Chunks and a merge either way (128, 500 tokens): 128 heads 8.2 / 8.8 and 7.6 / 8.6,
-    // 256 11.2 / 8.9 and 10.6 / 10.3.
-    const uint32_t many = span <= 128 ? 512u : span <= kRowsPerStep * 4 ? 2048u : span > kRowsPerStep * 8 ? 256u : HD == 64 ? 512u : 1024u;
-    const bool many_heads = batch > 1 && batch * p.q_heads >= many;
-    if ((span > 512 || many_heads) && m40_aligned16(p.Q)) {
+    // Rows of up to 512 tokens stay on the vector-ALU kernel in batches too.  Its launch grows with the q heads of all rows, the matrix-core kernel's hardly does (us, vector
+    // ALU / matrix cores, 512 q heads: 32 to 4 kv of 64, 128 tokens 5.1 / 4.6, 500 tokens 8.8 / 7.8), but q and the weights go into the latter as f16 high and low parts: its
+    // errors are 14 to 30 % larger (32 rows of up to 500 tokens 1.16e-7 / 1.36e-7), and an infinite V comes out of it as NaN.
+    if (span > 512 && m40_aligned16(p.Q)) {
         // long rows: matrix-core kernel (it reads q with 16-byte loads)
         p.subgroups = (group + 7) / 8;
         const uint64_t groups = (uint64_t)batch * p.kv_heads * p.subgroups;

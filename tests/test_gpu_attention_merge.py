@@ -43,7 +43,7 @@ def test_merge_of_chunks(dev, qh, kvh, hd, lens, hint):
     kv.destroy()
 
 
-# either side of the number of q heads from which short rows of a batch take the matrix-core kernel: one chunk and several, rows of a token, uneven rows
+# short rows in batches of few and many q heads: one chunk and several, rows of a token, uneven rows
 @pytest.mark.parametrize("qh,kvh,hd,rows,hint", [(32, 4, 64, 15, 128), (32, 4, 64, 16, 128), (32, 4, 64, 63, 256), (32, 4, 64, 64, 256), (32, 4, 64, 15, 512), (32, 4, 64, 16, 512),
                                                  (8, 8, 64, 64, 130), (64, 4, 128, 15, 256), (64, 4, 128, 16, 256), (16, 2, 128, 15, 400), (16, 2, 128, 16, 400), (64, 4, 128, 4, 257)])
 def test_short_rows_of_a_batch(dev, qh, kvh, hd, rows, hint):
@@ -52,6 +52,33 @@ def test_short_rows_of_a_batch(dev, qh, kvh, hd, rows, hint):
     lens[0], lens[-1] = hint, 1
     test_merge_of_chunks(dev, qh, kvh, hd, [int(n) for n in lens], hint)
 
+
+@pytest.mark.parametrize("qh,kvh,hd,rows,hint", [(32, 4, 64, 4, 128), (32, 4, 64, 16, 128), (32, 4, 64, 32, 500), (16, 2, 128, 32, 120), (16, 2, 128, 16, 400), (32, 8, 128, 32, 256)])
+def test_short_rows_of_a_batch_keep_infinities(dev, qh, kvh, hd, rows, hint):
+    """An infinite value of a short row stays an infinity however many rows a call has, and no other element sees it; the error of the finite ones, q four times as
+    large, stays that of f32 sums (a few 2^-24 of scores of up to 40)."""
+    rng = np.random.default_rng(rows + hint)
+    lens = rng.integers(2, hint + 1, rows)
+    kv = m40.KVCache(dev.ctx, hint, rows, kvh, hd)
+    Kc, Vc = (rng.standard_normal((rows, hint, kvh, hd)).astype(np.float16) for _ in range(2))
+    Kc *= np.float16(0.25)
+    for b, n in enumerate(lens):
+        Vc[b, b % n, b % kvh, 3] = np.inf * (-1) ** b
+        dev.fill_dense(kv, b, Kc[b].view(np.uint16), Vc[b].view(np.uint16))
+    q = (4.0 * rng.standard_normal((rows, qh * hd))).astype(np.float32)
+    dq, out, ids, dlens = dev.up(q), dev.zeros(q.nbytes), dev.up(np.arange(rows, dtype=np.uint32)), dev.up(lens.astype(np.uint32))
+    dev.call("m40llm_ext_attention_last_token_f32_gqa_batched_lens_dev_async", kv.h, ids.ptr, dlens.ptr, 0, rows, hint, dq.ptr, qh, out.ptr)
+    dev.sync()
+    got = out.download(np.float32, (rows, qh, hd)).astype(np.float64)
+    for b, n in enumerate(lens):
+        k, v = (np.repeat(t[b, :n].astype(np.float64), qh // kvh, axis=1) for t in (Kc, Vc))
+        s = np.einsum("hd,thd->ht", q[b].reshape(qh, hd).astype(np.float64), k) / np.sqrt(hd)
+        w = np.exp(s - s.max(axis=1, keepdims=True))
+        want = np.einsum("ht,thd->hd", w / w.sum(axis=1, keepdims=True), v)
+        assert np.array_equal(np.isinf(want), np.isinf(got[b])) and np.array_equal(want[np.isinf(want)], got[b][np.isinf(want)])
+        fine = np.isfinite(want)
+        close(got[b][fine], want[fine], 2e-6, 4e-6)
+    kv.destroy()
 
 # more rows and kv heads than two workgroups a CU: rows of one chunk, and long rows that then have one as well
 @pytest.mark.parametrize("qh,kvh,hd,rows,hint", [(8, 8, 64, 65, 100), (4, 4, 128, 129, 128), (8, 4, 64, 129, 520), (8, 8, 128, 65, 2100)])
