@@ -582,7 +582,8 @@ int m40llm_ext_batched_wide_norm_gemm_async(M40llmCudaContext* ctx, const void* 
  * elements) in a buffer of m40llm_ext_packed_rows_bytes(rows, K) bytes, 16-byte aligned; rows is the same in the call that writes the buffer and the one that
  * reads it, and rows that the attention skips are left as they are.  K (q_heads * head_dim, ffn) a multiple of 256.  The feed-forward call takes more than eight
  * rows of d_model a multiple of 256, or up to eight rows of d_model 2048 (..._supported: 1 / 0).  ..._onto_zero: out HOLDS ZEROS stored by an
- * earlier call on the decode stream and lies apart from the buffer and the residual.  -6 otherwise, nothing enqueued. */
+ * earlier call on the decode stream and lies apart from the buffer and the residual; the buffer lies apart from the rows that a call turns into it.  -6 otherwise,
+ * nothing enqueued; ..._bytes then is 0. */
 size_t m40llm_ext_packed_rows_bytes(uint32_t rows, int K);
 int m40llm_ext_batched_packed_supported(uint32_t rows, int d_model);
 int m40llm_ext_batched_norm_qkv_rope_append_clear_async(

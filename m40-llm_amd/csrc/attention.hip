@@ -660,8 +660,12 @@ int m40llm_ext_attention_last_token_f32_gqa_batched_lens_dev_async(M40llmCudaCon
 int m40llm_ext_attention_last_token_f32_gqa_batched_lens_dev_packed_async(M40llmCudaContext* ctx, const M40llmKVCache* kv, const uint32_t* seq_ids_dev,
                                                                           const uint32_t* seq_lens_dev, uint32_t len_bias, uint32_t batch_size,
                                                                           uint32_t max_len_hint, const void* q_dev_f32, uint32_t q_heads, void* packed_dev) {
-    if (!packed_dev) return -1;
-    if (batch_size > 32 || !m40_aligned16(packed_dev)) return -6;
+    if (!ctx || !kv || !seq_ids_dev || !seq_lens_dev || !q_dev_f32 || !packed_dev) return -1;
+    if (batch_size == 0) return -2;
+    if (q_heads == 0 || kv->num_heads == 0 || q_heads % kv->num_heads != 0) return -3;
+    const uint64_t K = (uint64_t)q_heads * kv->head_dim;
+    const size_t bytes = K <= 0x7fffffffu ? m40llm_ext_packed_rows_bytes(batch_size, (int)K) : 0;
+    if (bytes == 0 || !m40_aligned16(packed_dev) || !m40_aligned16(q_dev_f32) || !m40_apart(q_dev_f32, (size_t)batch_size * K * 4, packed_dev, bytes)) return -6;
     return batched_lens_dev(ctx, kv, seq_ids_dev, seq_lens_dev, len_bias, batch_size, max_len_hint, q_dev_f32, q_heads, nullptr, packed_dev);
 }
 

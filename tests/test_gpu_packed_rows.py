@@ -90,3 +90,37 @@ def test_attention(dev, rows, qh, kvh, hd, longest):
     w = f16bits(rng.standard_normal((N, K)) * 0.03)
     _project(dev, packed, out.download(np.float32, (rows, K)).astype(np.float64), w, rng.standard_normal((rows, N)).astype(np.float32), rows, N, K)
     kv.destroy()
+
+
+@pytest.mark.parametrize("rows,qh,kvh,hd", [(2, 14, 2, 64), (9, 1, 1, 64), (32, 5, 5, 64), (4, 1, 1, 128), (33, 4, 4, 64)])
+def test_refused_attention(dev, rows, qh, kvh, hd):
+    """Rows that the buffer has no form for (q heads x head size no multiple of 256, more than 32): its size is 0, the call refuses, and nothing is written."""
+    K = qh * hd
+    kv = m40.KVCache(dev.ctx, 16, rows, kvh, hd)
+    ids, lens, q = dev.up(np.arange(rows, dtype=np.uint32)), dev.up(np.full(rows, 3, dtype=np.uint32)), dev.zeros(rows * K * 4)
+    packed = dev.up(np.full(64, 0xFF, dtype=np.uint8))
+    assert dev.lib.m40llm_ext_packed_rows_bytes(rows, K) == 0
+    dev.call("m40llm_ext_attention_last_token_f32_gqa_batched_lens_dev_packed_async", kv.h, ids.ptr, lens.ptr, 0, rows, 16, q.ptr, qh, packed.ptr, expect=-6)
+    dev.sync()
+    assert (packed.download(np.uint8, (64,)) == 0xFF).all()
+    kv.destroy()
+
+
+def test_refused_buffers(dev):
+    """A buffer, or q, that is not aligned, and one that lies over q; the size is that of the rows' padded number."""
+    rows, qh, hd = 9, 4, 64
+    K = qh * hd
+    kv = m40.KVCache(dev.ctx, 16, rows, qh, hd)
+    ids, lens, q = dev.up(np.arange(rows, dtype=np.uint32)), dev.up(np.full(rows, 3, dtype=np.uint32)), dev.zeros(rows * K * 4 + 16)
+    for r in (1, 8, 9, 16, 17, 32): assert dev.lib.m40llm_ext_packed_rows_bytes(r, K) == _bytes(r, K)
+    packed = dev.zeros(_bytes(rows, K) + 16)
+    call = lambda qp, pp, expect: dev.call("m40llm_ext_attention_last_token_f32_gqa_batched_lens_dev_packed_async", kv.h, ids.ptr, lens.ptr, 0, rows, 16, qp, qh, pp, expect=expect)
+    call(q.ptr, packed.ptr + 4, -6)
+    call(q.ptr + 4, packed.ptr, -6)
+    call(packed.ptr, packed.ptr, -6)
+    call(packed.ptr + _bytes(rows, K) - 16, packed.ptr, -6)
+    call(None, packed.ptr, -1)
+    call(q.ptr, None, -1)
+    call(q.ptr, packed.ptr, 0)
+    dev.sync()
+    kv.destroy()
