@@ -782,6 +782,11 @@ int m40llm_ext_batched_norm_qkv_rope_append_clear_async(
     if (kv->head_dim == 0 || kv->head_dim % 2 != 0 || kv->num_heads == 0 || q_heads == 0) return -3;
     if (!rows_ok(ctx, (int)rows, (int)d_model)) return -6;
     if (!m40_aligned16(d_wq_f16) || !m40_aligned16(d_wk_f16) || !m40_aligned16(d_wv_f16)) return -6;
+    // what is cleared goes while other workgroups still read the rows and store q
+    const size_t x_bytes = (size_t)rows * d_model * 4, q_bytes = (size_t)rows * q_heads * kv->head_dim * 4, clear_bytes = (size_t)clear_floats * 4;
+    if (clear_floats && (!m40_apart(d_x_f32, x_bytes, d_clear_f32, clear_bytes) || !m40_apart(d_q_out_f32, q_bytes, d_clear_f32, clear_bytes))) return -6;
+    float* const clear = clear_floats ? static_cast<float*>(d_clear_f32) : nullptr;
+    const auto clear_behind = [&](int rc) { return rc != 0 || !clear ? rc : (m40_zero_f32(ctx->decode_stream, clear, clear_floats) == 0 ? 0 : -7); };
     (void)hipGetLastError();
     // up to eight rows and K = 2048: persistent matrix-core kernel with the whole epilogue inside
     if (m40_rows_mfma_qkv_supported((int)rows, (int)d_model, kv->head_dim) && m40_aligned16(d_x_f32) && m40_aligned16(d_norm_w) &&
@@ -791,25 +796,23 @@ int m40llm_ext_batched_norm_qkv_rope_append_clear_async(
                                  static_cast<const uint16_t*>(d_wk_f16), static_cast<const uint16_t*>(d_wv_f16),
                                  static_cast<const float*>(d_bq_f32), static_cast<const float*>(d_bk_f32),
                                  static_cast<const float*>(d_bv_f32), d_model, q_heads, freq_base, freq_scale, rope_layout,
-                                 static_cast<float*>(d_q_out_f32),
-                                 clear_floats ? static_cast<float*>(d_clear_f32) : nullptr, (int)clear_floats);
-    if (clear_floats && m40_zero_f32(ctx->decode_stream, static_cast<float*>(d_clear_f32), clear_floats) != 0) return -7;
+                                 static_cast<float*>(d_q_out_f32), clear, (int)clear_floats);
     // nine rows and more: one launch as well, K in chunks; a result that overlaps the rows takes the two launches below, here and in the other calls
     if (rows > 8 && kv->head_dim % 16 == 0 && m40_aligned16(d_x_f32) && m40_aligned16(d_norm_w) &&
-        m40_apart(d_x_f32, (size_t)rows * d_model * 4, d_q_out_f32, (size_t)rows * q_heads * kv->head_dim * 4))
+        m40_apart(d_x_f32, x_bytes, d_q_out_f32, q_bytes))
         return m40_rows_wide_qkv(ctx, ctx->decode_stream, kv, seq_ids_dev, seq_lens_dev, rows, static_cast<const float*>(d_x_f32), d_norm_w,
                                  norm_weight_dtype, eps, static_cast<const uint16_t*>(d_wq_f16), static_cast<const uint16_t*>(d_wk_f16),
                                  static_cast<const uint16_t*>(d_wv_f16), static_cast<const float*>(d_bq_f32),
                                  static_cast<const float*>(d_bk_f32), static_cast<const float*>(d_bv_f32), d_model, q_heads, freq_base,
-                                 freq_scale, rope_layout, static_cast<float*>(d_q_out_f32), nullptr, 0);
+                                 freq_scale, rope_layout, static_cast<float*>(d_q_out_f32), clear, (int)clear_floats);
     // up to eight rows and K <= 2048: vector-ALU kernel with the whole epilogue inside (one launch instead of two)
     if (m40_rows_gemv_supported((int)rows, (int)d_model) && m40_aligned16(d_x_f32) && m40_aligned16(d_norm_w))
-        return m40_rows_norm_qkv(ctx, ctx->decode_stream, kv, seq_ids_dev, seq_lens_dev, rows, static_cast<const float*>(d_x_f32),
-                                 d_norm_w, norm_weight_dtype, eps, static_cast<const uint16_t*>(d_wq_f16),
-                                 static_cast<const uint16_t*>(d_wk_f16), static_cast<const uint16_t*>(d_wv_f16),
-                                 static_cast<const float*>(d_bq_f32), static_cast<const float*>(d_bk_f32),
-                                 static_cast<const float*>(d_bv_f32), d_model, q_heads, freq_base, freq_scale, rope_layout,
-                                 static_cast<float*>(d_q_out_f32));
+        return clear_behind(m40_rows_norm_qkv(ctx, ctx->decode_stream, kv, seq_ids_dev, seq_lens_dev, rows, static_cast<const float*>(d_x_f32),
+                                              d_norm_w, norm_weight_dtype, eps, static_cast<const uint16_t*>(d_wq_f16),
+                                              static_cast<const uint16_t*>(d_wk_f16), static_cast<const uint16_t*>(d_wv_f16),
+                                              static_cast<const float*>(d_bq_f32), static_cast<const float*>(d_bk_f32),
+                                              static_cast<const float*>(d_bv_f32), d_model, q_heads, freq_base, freq_scale, rope_layout,
+                                              static_cast<float*>(d_q_out_f32)));
     const int QN = (int)(q_heads * kv->head_dim), KN = (int)(kv->num_heads * kv->head_dim);
     PackSpec pk{static_cast<const float*>(d_x_f32), nullptr, d_norm_w, norm_weight_dtype, eps};
     const void* W[3] = {d_wq_f16, d_wk_f16, d_wv_f16};
@@ -828,7 +831,7 @@ int m40llm_ext_batched_norm_qkv_rope_append_clear_async(
     e.head_dim = kv->head_dim; e.rope_layout = rope_layout; e.rope_base = freq_base; e.rope_scale = freq_scale;
     const uint32_t pairs = (q_heads + 2u * kv->num_heads) * (kv->head_dim / 2u);
     skinny_qkv_epilogue_kernel<<<dim3((pairs + 255u) / 256u, rows), 256, 0, ctx->decode_stream>>>(e);
-    return hipGetLastError() == hipSuccess ? 0 : -7;
+    return clear_behind(hipGetLastError() == hipSuccess ? 0 : -7);
 }
 
 int m40llm_ext_batched_gemm_residual_f32xf16_async(M40llmCudaContext* ctx, const void* d_a_f32, const void* d_w_f16,

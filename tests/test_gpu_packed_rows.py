@@ -124,3 +124,30 @@ def test_refused_buffers(dev):
     call(q.ptr, packed.ptr, 0)
     dev.sync()
     kv.destroy()
+
+
+# one launch on matrix cores (width 2048, up to eight rows), nine rows and more, the vector-ALU form, product and epilogue
+@pytest.mark.parametrize("rows,qh,kvh,hd,D", [(1, 32, 4, 64, 2048), (8, 16, 2, 128, 2048), (5, 4, 2, 64, 256), (12, 8, 8, 64, 512), (16, 4, 1, 128, 2048), (3, 8, 2, 64, 4096)])
+@pytest.mark.parametrize("floats", [1, 1000])
+def test_clear_beside_qkv(dev, rows, qh, kvh, hd, D, floats):
+    """Q, K and V with a range cleared on the side: the bits of the call without one, zeros in the range and nothing behind it; a range that lies over the rows or q is refused."""
+    rng = np.random.default_rng(rows * 7 + D)
+    x, nw = rng.standard_normal((rows, D)).astype(np.float32), (1 + 0.1 * rng.standard_normal(D)).astype(np.float32)
+    dx, dnw = dev.up(x), dev.up(nw)
+    w = [dev.up(f16bits(rng.standard_normal((n * hd, D)) * 0.05)) for n in (qh, kvh, kvh)]
+    ids, lens = dev.up(np.arange(rows, dtype=np.uint32)), dev.up(rng.integers(0, 8, rows).astype(np.uint32))
+    got = []
+    for name, clear in (("m40llm_ext_batched_norm_qkv_rope_append_async", False), ("m40llm_ext_batched_norm_qkv_rope_append_clear_async", True)):
+        kv, q = m40.KVCache(dev.ctx, 16, rows, kvh, hd), dev.zeros(rows * qh * hd * 4)
+        zone = dev.up(np.full(floats + 3, 5.0, dtype=np.float32))
+        args = lambda *tail: (kv.h, ids.ptr, lens.ptr, rows, dx.ptr, dnw.ptr, 1, 1e-5, *(t.ptr for t in w), None, None, None, D, qh, 1e4, 1.0, 0, q.ptr, *tail)
+        if clear:
+            for at in (dx.ptr, dx.ptr + rows * D * 4 - 4, q.ptr, q.ptr + rows * qh * hd * 4 - 4): dev.call(name, *args(at, floats), expect=-6)
+            dev.sync()
+            assert np.array_equal(dx.download(np.float32, (rows, D)), x) and not q.download(np.uint32, (rows * qh * hd,)).any()
+        dev.call(name, *args(*((zone.ptr, floats) if clear else ())))
+        dev.sync()
+        assert np.array_equal(zone.download(np.float32, (floats + 3,)), ([0.0] if clear else [5.0]) * floats + [5.0] * 3)
+        got.append([q.download(np.uint32, (rows * qh * hd,))] + [t for r in range(rows) for p in range(8) for t in kv.read_token(r, p)])
+        kv.destroy()
+    assert all(np.array_equal(a, b) for a, b in zip(*got))
