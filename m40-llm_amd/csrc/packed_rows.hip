@@ -10,7 +10,8 @@
 //
 // Two halves of K where one tile a workgroup would leave half of the CUs idle, onto a result that holds zeros, as in rows_wide_mfma.hip: no second launch, and no
 // result depends on timing.  Measured in a replayed graph with cold weights, N 2048, f32 rows before / packed now, us: K 2048, 8 rows 5.4 / 4.2, 16 rows
-// 5.1 / 4.5, 32 rows 6.5 / 5.3; K 5632 7.5 / 6.9, 8.5 / 8.1, 11.6 / 9.9; K 11008, 8 rows 13.5 / 11.9.
+// 5.1 / 4.5, 32 rows 6.5 / 5.3; K 5632 7.5 / 6.9, 8.5 / 8.1, 11.6 / 9.9; K 11008, 8 rows 13.5 / 11.9.  (Looking for units far below their block's largest, below,
+// is part of that since: 0.1 us a launch at 8 rows, 0.05 at 16 and 32.)
 #include "packed_rows.hpp"
 
 namespace {
@@ -18,6 +19,7 @@ namespace {
 constexpr int kBlock = 128, kSteps = kBlock / 32;        // k of a wave's block, matrix instructions deep
 constexpr int kRunLanes = kBlock * 2 / 16;              // lanes that cover a column's block with 16 bytes each
 constexpr int kCols = 64 / kRunLanes, kLoads = 16 / kCols;
+constexpr float kFar = 256.0f;                           // a unit that far below the largest of its row and block is multiplied on its own
 constexpr int kStageRow = kBlock * 2 + 16;              // LDS bytes per column: +16 spreads the columns over the banks
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -49,6 +51,14 @@ __global__ __launch_bounds__(64 * WAVES) void packed_rows_kernel(const uint8_t* 
     m40_float4 total[RT];
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) total[rt] = {0.f, 0.f, 0.f, 0.f};
+    const auto scale_at = [&](int kb, int i, int rt) { return scales[(size_t)(kb * 4 * kSteps + 4 * i + g) * PAD + 16 * rt + (PAD > 8 ? j : j & 7)]; };
+    const auto largest = [&](const float (&s)[kSteps]) {         // of a row's sixteen units of the block
+        const float most = m40_max_xor32(m40_max_xor16(fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]))));
+        return most > 0.0f ? most : 1.0f;
+    };
+    // (rows that are not there hold anything)
+    const auto is_far = [&](float s, float most, int rt) { return s > 0.0f && s * kFar < most && 16 * rt + (PAD > 8 ? j : j & 7) < rows; };
+    bool left_out = false;
     for (int kb = b_begin + wave; kb < b_end; kb += WAVES) {
         f16x8 a[RT][PARTS][kSteps];
         float s[RT][kSteps];
@@ -59,23 +69,26 @@ __global__ __launch_bounds__(64 * WAVES) void packed_rows_kernel(const uint8_t* 
             for (int rt = 0; rt < RT; ++rt) {
 #pragma unroll
                 for (int h = 0; h < PARTS; ++h) a[rt][h][i] = *reinterpret_cast<const f16x8*>(from + ((i * RT + rt) * PARTS + h) * 1024);
-                s[rt][i] = scales[(size_t)(kb * 4 * kSteps + 4 * i + g) * PAD + 16 * rt + (PAD > 8 ? j : j & 7)];
+                s[rt][i] = scale_at(kb, i, rt);
             }
         __builtin_amdgcn_sched_barrier(0);      // the rows (cache hits) ahead of the weights: loads return in issue order
         u32x4 b[kLoads];
 #pragma unroll
         for (int li = 0; li < kLoads; ++li) b[li] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(w_tile + (size_t)kb * kBlock + w_at[li]));
         __builtin_amdgcn_sched_barrier(0);
-        // one scale for a row's sixteen units of the block, the largest; the others' parts are multiplied by the power of two between: exact, or off by at most
-        // 2^-25 where the row's largest value is 2^10 and more
+        // One scale for a row's sixteen units of the block, the largest: the others' parts are multiplied by the power of two between, exactly, or off by at most 2^-25 where the
+        // largest value is 2^14 and more.  Of a unit that lies further below, beside an outlier, that would take bits which count once the outlier's weights are small: it is left
+        // out here and added behind the loop.
         float top[RT];
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
-            top[rt] = m40_max_xor32(m40_max_xor16(fmaxf(fmaxf(s[rt][0], s[rt][1]), fmaxf(s[rt][2], s[rt][3]))));
+            top[rt] = largest(s[rt]);
             const float inv = __uint_as_float(0x7f000000u - __float_as_uint(top[rt]));
 #pragma unroll
             for (int i = 0; i < kSteps; ++i) {
-                const _Float16 f = static_cast<_Float16>(s[rt][i] * inv);
+                const bool far = is_far(s[rt][i], top[rt], rt);
+                left_out = left_out || far;
+                const _Float16 f = static_cast<_Float16>(far ? 0.0f : s[rt][i] > 0.0f ? s[rt][i] * inv : 1.0f);
 #pragma unroll
                 for (int h = 0; h < PARTS; ++h) a[rt][h][i] *= f;
             }
@@ -104,6 +117,49 @@ __global__ __launch_bounds__(64 * WAVES) void packed_rows_kernel(const uint8_t* 
                 const float scale = __shfl(top[rt], PAD > 8 ? 4 * g + r : 4 * (g & 1) + r, 64);
                 total[rt][r] = fmaf(scale, acc[rt][1][r], fmaf(scale, acc[rt][0][r], total[rt][r]));
             }
+    }
+    // What was left out: the units of each lane group on their own, the others' parts and weights zero.
+    if (__builtin_expect(__ballot(left_out) != 0, 0)) {
+        for (int kb = b_begin + wave; kb < b_end; kb += WAVES) {
+            float far[RT][kSteps];               // the scale of a unit that was left out, or 0
+            bool any = false;
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) {
+                float s[kSteps];
+#pragma unroll
+                for (int i = 0; i < kSteps; ++i) s[i] = scale_at(kb, i, rt);
+                const float most = largest(s);
+#pragma unroll
+                for (int i = 0; i < kSteps; ++i) {
+                    far[rt][i] = is_far(s[i], most, rt) ? s[i] : 0.0f;
+                    any = any || far[rt][i] > 0.0f;
+                }
+            }
+            if (__ballot(any) == 0) continue;
+            const uint16_t* w_at_j = w_tile + (size_t)(n0 + j < N ? j : N - 1 - n0) * K + (size_t)kb * kBlock + 8 * g;
+            const uint8_t* from = packed + (size_t)kb * (kSteps * PAD * 128) + 16 * lane;
+#pragma unroll
+            for (int i = 0; i < kSteps; ++i) {
+                const uint4 w = *reinterpret_cast<const uint4*>(w_at_j + 32 * i), none = make_uint4(0, 0, 0, 0);
+#pragma unroll 1
+                for (int u = 0; u < 4; ++u) {
+#pragma unroll
+                    for (int rt = 0; rt < RT; ++rt) {
+                        m40_float4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                        for (int h = PARTS - 1; h >= 0; --h) {
+                            const uint4 part = *reinterpret_cast<const uint4*>(from + ((i * RT + rt) * PARTS + h) * 1024);
+                            acc = mfma16x16x32(__builtin_bit_cast(f16x8, g == u ? part : none), g == u ? w : none, acc);
+                        }
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            const float scale = __shfl(far[rt][i], 16 * u + (PAD > 8 ? 4 * g + r : 4 * (g & 1) + r), 64);
+                            if (scale > 0.0f) total[rt][r] = fmaf(scale, acc[r], total[rt][r]);
+                        }
+                    }
+                }
+            }
+        }
     }
     __syncthreads();
     float* red = reinterpret_cast<float*>(lds);          // [waves][RT * 4][64]: nobody reads the staged weights any more

@@ -29,7 +29,8 @@ def _project(dev, packed, rows64, w, res, rows, N, K):
     """Residual, no residual and the same bits twice, onto zeros; `rows64`: the rows the buffer holds."""
     dw, dres = dev.up(w), dev.up(res)
     want = rows64 @ _f64(w).T
-    # operands exact to 2^-22 of a unit's largest value, f32 sums of K products: a few 2^-24 of the row's largest sum of magnitudes a wave's share
+    # operands exact to 2^-22 of themselves and 2^-31 of the largest of their eight; f32 sums of K products: a few 2^-24 of
+    # the row's largest sum of magnitudes a wave's share
     bound = np.abs(rows64) @ np.abs(_f64(w)).T * 2.0 ** -21
     got = []
     for r in (res, None, res):
@@ -151,3 +152,69 @@ def test_clear_beside_qkv(dev, rows, qh, kvh, hd, D, floats):
         got.append([q.download(np.uint32, (rows * qh * hd,))] + [t for r in range(rows) for p in range(8) for t in kv.read_token(r, p)])
         kv.destroy()
     assert all(np.array_equal(a, b) for a, b in zip(*got))
+
+
+# `far`: log2 between the units that meet in an instruction, either side of where each is multiplied on its own
+@pytest.mark.parametrize("rows,F,D,N", [(2, 512, 2048, 40), (8, 2816, 2048, 2048), (13, 1024, 256, 70), (32, 2816, 256, 2048)])
+@pytest.mark.parametrize("far", [4, 8, 12, 20, 25, 30, 39])
+def test_outliers(dev, rows, F, D, N, far):
+    """A unit far above its neighbours, whose columns have no weight: nothing of the small ones is lost beside it."""
+    rng = np.random.default_rng(far + F)
+    x, nw = rng.standard_normal((rows, D)).astype(np.float32), np.ones(D, np.float32)
+    wg, wu = (rng.standard_normal((F, D)) * 0.02 for _ in range(2))
+    unit = np.arange(F) // 8
+    large, low = unit % 8 == unit // 8 % 8, min(far, 24)
+    wu[~large] *= 2.0 ** -(low // 2)
+    wg[~large] *= 2.0 ** -(low - low // 2)
+    wu[large] *= 2.0 ** (far - low)
+    dx, dnw, dwg, dwu = dev.up(x), dev.up(nw), dev.up(f16bits(wg)), dev.up(f16bits(wu))
+    hid, packed = dev.zeros(rows * F * 4), dev.up(np.full(_bytes(rows, F), 0xFF, dtype=np.uint8))
+    plain = "m40llm_ext_batched_norm_gate_up_swiglu_clear_async" if rows <= 8 else "m40llm_ext_batched_wide_norm_gate_up_swiglu_async"
+    dev.call(plain, dx.ptr, dnw.ptr, 1, 1e-5, dwg.ptr, dwu.ptr, hid.ptr, rows, F, D, None, 0)
+    dev.call("m40llm_ext_batched_norm_gate_up_swiglu_packed_async", dx.ptr, dnw.ptr, 1, 1e-5, dwg.ptr, dwu.ptr, packed.ptr, rows, F, D, None, 0)
+    dev.sync()
+    a = hid.download(np.float32, (rows, F)).astype(np.float64)
+    w = rng.standard_normal((N, F)) * 0.03
+    w[:, large] = 0.0
+    w = f16bits(w)
+    dw, out = dev.up(w), dev.zeros(rows * N * 4)
+    dev.call("m40llm_ext_batched_packed_gemm_residual_onto_zero_async", packed.ptr, dw.ptr, None, out.ptr, rows, N, F)
+    dev.sync()
+    most = np.repeat(np.abs(a).reshape(rows, F // 8, 8).max(axis=2), 8, axis=1)
+    # a value is exact to 2^-22 of itself and 2^-31 of its unit's largest; f32 sums of K products (2^-22 of the sum of magnitudes)
+    bound = (np.abs(a) * 2.0 ** -21 + most * 2.0 ** -30) @ np.abs(_f64(w)).T
+    err = np.abs(out.download(np.float32, (rows, N)) - a @ _f64(w).T)
+    assert np.all(err <= bound), (err / bound).max()
+
+
+@pytest.mark.parametrize("rows,qh,kvh,hd,length", [(3, 4, 2, 64, 40), (8, 32, 4, 64, 128), (9, 4, 4, 64, 70), (32, 16, 2, 128, 256)])
+def test_infinities(dev, rows, qh, kvh, hd, length):
+    """A row with one infinity gives infinities, of each weight's sign; rows of very large and very small values beside it keep theirs."""
+    rng = np.random.default_rng(rows + length)
+    K, N = qh * hd, 130
+    kv = m40.KVCache(dev.ctx, length, rows, kvh, hd)
+    for r in range(rows):
+        k, v = (rng.standard_normal((length, kvh, hd)).astype(np.float16) for _ in range(2))
+        v *= np.float16(2.0 ** (13 if r % 3 == 1 else -10))          # |v| < 2^3: within f16
+        if r % 3 == 0: v[r % length, r % kvh, 5] = np.inf
+        dev.fill_dense(kv, r, f16bits(0.1 * k), v.view(np.uint16))
+    q = rng.standard_normal((rows, K)).astype(np.float32)
+    dq, out, ids, dlens = dev.up(q), dev.zeros(q.nbytes), dev.up(np.arange(rows, dtype=np.uint32)), dev.up(np.full(rows, length, dtype=np.uint32))
+    packed, y = dev.up(np.full(_bytes(rows, K), 0xFF, dtype=np.uint8)), dev.zeros(rows * N * 4)
+    dev.call("m40llm_ext_attention_last_token_f32_gqa_batched_lens_dev_async", kv.h, ids.ptr, dlens.ptr, 0, rows, length, dq.ptr, qh, out.ptr)
+    dev.call("m40llm_ext_attention_last_token_f32_gqa_batched_lens_dev_packed_async", kv.h, ids.ptr, dlens.ptr, 0, rows, length, dq.ptr, qh, packed.ptr)
+    w = rng.standard_normal((N, K)) * 0.03
+    w = f16bits(np.where(np.abs(w) < 1e-3, 1e-3, w))
+    # one head of the infinite kv head alone keeps its weight's sign: the heads that share it would add infinities of both
+    group = qh // kvh
+    w64 = _f64(w).reshape(N, kvh, group, hd)
+    w64[:, :, 1:, 5] = np.abs(w64[:, :, :1, 5]) * np.sign(w64[:, :, :1, 5])
+    w = f16bits(w64.reshape(N, K))
+    dw = dev.up(w)
+    dev.call("m40llm_ext_batched_packed_gemm_residual_onto_zero_async", packed.ptr, dw.ptr, None, y.ptr, rows, N, K)
+    dev.sync()
+    a, got = out.download(np.float32, (rows, K)).astype(np.float64), y.download(np.float32, (rows, N))
+    want, fine = a @ _f64(w).T, np.arange(rows) % 3 != 0
+    assert np.isinf(want[~fine]).all() and np.array_equal(got[~fine], want[~fine])
+    assert np.all(np.abs(got[fine] - want[fine]) <= np.abs(a[fine]) @ np.abs(_f64(w)).T * 2.0 ** -21)
+    kv.destroy()
