@@ -84,7 +84,7 @@ struct PrefillArgs {
     uint32_t plane_tiles;       // padded tiles in total (sequence b starts at tile kv_offsets[b] / 32 + b ... see pack)
     const uint32_t* q_offsets; const uint32_t* kv_offsets; const uint32_t* q_lens; const uint32_t* kv_lens;
     uint32_t q_heads, kv_heads;
-    float* v_max;               // per padded tile and kv head: largest finite |V| (with a PrefillRope)
+    float *v_max, *v_key;       // per padded tile and kv head: largest finite |V|, of the tile and of each of its keys (with a PrefillRope)
     M40TiledRows rows;          // where the result goes as rows of the next product instead of Out
 };
 
@@ -200,11 +200,20 @@ __global__ __launch_bounds__(kThreads) void prefill_pack_kv_kernel(PrefillArgs p
         }
         if (tile == 0 && kvh == 0 && threadIdx.x == 0) rope.seq_map[rope.slot[b]] = kv_len;
         float mx = 0.0f;
+        float* const v_key = p.v_key + ((size_t)(first_tile_of(p.kv_offsets[b], b, kKTile) + tile) * p.kv_heads + kvh) * kKTile;
 #pragma unroll
-        for (int u = 0; u < kQuads; ++u) {
-            const float v4[4] = {vx[u].x, vx[u].y, vx[u].z, vx[u].w};
+        for (int u = 0; u < kQuads; u += 2) {
+            const float v8[8] = {vx[u].x, vx[u].y, vx[u].z, vx[u].w, vx[u + 1].x, vx[u + 1].y, vx[u + 1].z, vx[u + 1].w};
+            float of_key = 0.0f;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) mx = fmaxf(mx, fabsf(v4[i]) <= 3.402823466e+38f ? fabsf(v4[i]) : 0.0f);      // (keys past the end: the last one's again)
+            for (int i = 0; i < 8; ++i) of_key = fmaxf(of_key, fabsf(v8[i]) <= 3.402823466e+38f ? fabsf(v8[i]) : 0.0f);      // (keys past the end: the last one's again)
+            // HD / 8 neighbouring lanes hold a key
+            of_key = fmaxf(of_key, m40_dpp_f<M40_DPP_XOR1>(of_key));
+            of_key = fmaxf(of_key, m40_dpp_f<M40_DPP_XOR2>(of_key));
+            of_key = fmaxf(of_key, m40_dpp_f<M40_DPP_HALF_MIRROR>(of_key));
+            if (HD == 128) of_key = fmaxf(of_key, m40_dpp_f<M40_DPP_ROW_ROR8>(of_key));
+            if (threadIdx.x % (HD / 8) == 0) v_key[at[u] / HD] = of_key;
+            mx = fmaxf(mx, of_key);
         }
         mx = m40_max64(mx);
         if ((threadIdx.x & 63) == 0) wave_max[threadIdx.x >> 6] = mx;
@@ -249,8 +258,11 @@ __global__ __launch_bounds__(kThreads) void prefill_pack_kv_kernel(PrefillArgs p
 // QB: 16-query blocks per wave.  With two, every K and V fragment a wave reads from LDS serves 32 queries instead of 16:
 // the kernel's LDS traffic (each wave reads the whole K and V tile) was what it spent most of its time on.
 // PLANES (with a PrefillRope): the result goes to the rows of the next product, which a packing pass read and wrote again (4096 rows of 2048 12.9 us, 522 rows
-// 6.0).  A row's scale must be known to the workgroups of all its heads: it follows from the largest |V| of the row's sequence, which no weighted mean of V
-// exceeds, brought into [2^14, 2^15): f16 hi + lo keep 22 bits of every value down to 2^-18 of it.  A value that is not finite goes in as it is.
+// 6.0).  A row's scale must be known to the workgroups of all its heads: it follows from the largest |V| of the keys that the row sees, which no weighted mean of
+// those exceeds, brought into [2^14, 2^15): f16 hi + lo keep 22 bits of every value down to 2^-17 of it, and no row depends on what comes behind it (the largest of the
+// whole sequence instead took bits from the rows ahead of a large V; a whole prompt of 4096 tokens 21.18 ms
+// so, 21.25 now, five of 522 together 4.66 and 4.69, inside their spread).  Below, an error of
+// 2^-39 of the largest: for |V| up to 2^14 within the 2^-25 that V's own two parts leave.  A value that is not finite goes in as it is.
 template <int HD, int QB, class ROPE, bool PLANES>
 __global__ __launch_bounds__(kThreads) void prefill_attn_kernel(PrefillArgs p, ROPE rope) {
     constexpr bool kRope = std::is_same<ROPE, PrefillRope>::value;
@@ -282,9 +294,12 @@ __global__ __launch_bounds__(kThreads) void prefill_attn_kernel(PrefillArgs p, R
     if (q0 >= q_len || q_len > kv_len) return;
     const uint32_t kvh = h / (p.q_heads / p.kv_heads);
     const int tid = threadIdx.x, lane = tid & 63;
-    const uint32_t n_max = (kv_len + kKTile - 1) / kKTile * p.kv_heads;
-    const float* v_max = PLANES ? p.v_max + (size_t)first_tile_of(p.kv_offsets[b], b, kKTile) * p.kv_heads : nullptr;
-    float bound = PLANES ? v_max[(uint32_t)tid < n_max ? tid : 0] : 0.0f;        // waited for at the end
+    // PLANES: the largest |V| of the keys ahead of the workgroup's queries, by tiles, and of the queries' own, a few heads a thread; the rest is looked at at the end
+    const uint32_t n_ahead = q0 / kKTile * p.kv_heads, own_key = q0 + (uint32_t)(tid % kQGroup) < q_len ? q0 + (uint32_t)(tid % kQGroup) : q_len - 1;
+    const size_t first_max = PLANES ? (size_t)first_tile_of(p.kv_offsets[b], b, kKTile) * p.kv_heads : 0;
+    const float* v_key = PLANES ? p.v_key + (first_max + own_key / kKTile * p.kv_heads) * kKTile + own_key % kKTile : nullptr;
+    float ahead = PLANES && (uint32_t)tid < n_ahead ? p.v_max[first_max + tid] : 0.0f;
+    float own = PLANES && (uint32_t)(tid / kQGroup) < p.kv_heads ? v_key[tid / kQGroup * kKTile] : 0.0f;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);       // as a scalar: tests on it branch without masks
     const int j = lane & 15, g = lane >> 4;
     const float inv_sqrt = HD == 64 ? 0.125f : 0.08838834764831845f;
@@ -529,22 +544,31 @@ __global__ __launch_bounds__(kThreads) void prefill_attn_kernel(PrefillArgs p, R
     }
 
     // ---- out = O / sum: this lane holds columns 16 d + 4 g .. + 3 of its query
-    float row_scale = 1.0f, row_inv = 1.0f;
+    float seen = 0.0f;                 // of the wave's sixty-four queries that hold its own: largest |V| of the keys up to query `lane`
     if constexpr (PLANES) {
-        __shared__ float wave_max[kWaves];
-        for (uint32_t i = tid + kThreads; i < n_max; i += kThreads) bound = fmaxf(bound, v_max[i]);
-        bound = m40_max64(bound);
-        if (lane == 0) wave_max[wave] = bound;
+        __shared__ float wave_max[kWaves], own_max[kThreads];
+        for (uint32_t i = tid + kThreads; i < n_ahead; i += kThreads) ahead = fmaxf(ahead, p.v_max[first_max + i]);
+        for (uint32_t i = tid / kQGroup + kThreads / kQGroup; i < p.kv_heads; i += kThreads / kQGroup) own = fmaxf(own, v_key[i * kKTile]);
+        ahead = m40_max64(ahead);
+        if (lane == 0) wave_max[wave] = ahead;
+        own_max[tid] = own;
         __syncthreads();
-        bound = fmaxf(fmaxf(wave_max[0], wave_max[1]), fmaxf(wave_max[2], wave_max[3]));
-        if (bound > 0.0f) {
-            int ex;
-            (void)frexpf(bound, &ex);
-            ex -= 15;
-            ex = ex < -100 ? -100 : (ex > 100 ? 100 : ex);
-            row_scale = ldexpf(1.0f, ex);
-            row_inv = ldexpf(1.0f, -ex);
+        ahead = fmaxf(fmaxf(wave_max[0], wave_max[1]), fmaxf(wave_max[2], wave_max[3]));
+        const auto of_query = [&](int q) {
+            float m = own_max[q];
+#pragma unroll
+            for (int i = kQGroup; i < kThreads; i += kQGroup) m = fmaxf(m, own_max[q + i]);
+            return m;
+        };
+        const int half = kQWave * wave / 64;
+        seen = of_query(64 * half + lane);
+#pragma unroll
+        for (int d = 1; d < 64; d *= 2) {
+            const float before = __shfl_up(seen, d, 64);
+            if (lane >= d) seen = fmaxf(seen, before);
         }
+        if (half) ahead = fmaxf(ahead, m40_max64(of_query(lane)));
+        seen = fmaxf(seen, ahead);
     }
     if (!wave_live) return;
 #pragma unroll
@@ -554,10 +578,15 @@ __global__ __launch_bounds__(kThreads) void prefill_attn_kernel(PrefillArgs p, R
         const float denom = l > 0.0f ? l : 1.0f;
         const uint32_t q = wq0 + 16u * qb + (uint32_t)j;
         if constexpr (PLANES) {
+            const float bound = __shfl(seen, (kQWave * wave + 16 * qb) % 64 + j, 64);
             if (q >= q_len) continue;
             const int row = (int)(p.q_offsets[b] + q), K = (int)p.q_heads * HD;
             const size_t first = m40_tiled_row(row, K);
-            if (h == 0 && g == 0) p.rows.scale[row] = row_scale;
+            int ex;
+            (void)frexpf(bound, &ex);
+            ex = bound > 0.0f ? (ex < -85 ? -100 : ex - 15) : 0;
+            const float row_inv = __uint_as_float((uint32_t)(127 - ex) << 23);
+            if (h == 0 && g == 0) p.rows.scale[row] = __uint_as_float((uint32_t)(127 + ex) << 23);
 #pragma unroll
             for (int d = 0; d < DT; ++d) {
                 half4 hi, lo;
@@ -626,7 +655,7 @@ int prefill_impl(M40llmCudaContext* ctx, const void* q, const void* k, const voi
     }
     const uint32_t kKTile = (uint32_t)key_tile_of((int)head_dim);
     const uint64_t plane_tiles = (offs[batch - 1] / kKTile + (batch - 1)) + (host[2 * (size_t)batch - 1] + kKTile - 1) / kKTile;
-    const size_t planes_bytes = (size_t)plane_tiles * kv_heads * 4 * kKTile * head_dim * sizeof(_Float16), need = planes_bytes + (size_t)plane_tiles * kv_heads * sizeof(float);
+    const size_t planes_bytes = (size_t)plane_tiles * kv_heads * 4 * kKTile * head_dim * sizeof(_Float16), need = planes_bytes + (size_t)plane_tiles * kv_heads * (1 + kKTile) * sizeof(float);
     M40StreamScratch& sc = ctx->scratch[0];
     if (sc.attn_planes_bytes < need) {
         if (hipStreamSynchronize(ctx->prefill_stream) != hipSuccess) return -5;
@@ -642,6 +671,7 @@ int prefill_impl(M40llmCudaContext* ctx, const void* q, const void* k, const voi
     a.planes = static_cast<const _Float16*>(sc.attn_planes);
     a.plane_tiles = (uint32_t)plane_tiles;
     a.v_max = reinterpret_cast<float*>(static_cast<char*>(sc.attn_planes) + planes_bytes);
+    a.v_key = a.v_max + (size_t)plane_tiles * kv_heads;
     if (rows) a.rows = *rows;
     (void)hipGetLastError();
     const dim3 pack_grid((max_kv + kKTile - 1) / kKTile, kv_heads, batch);

@@ -96,3 +96,37 @@ def test_few_rows_of_prompts(dev, lens):
                 assert np.abs(a - b).max() <= 2e-3 * np.abs(b).max()
         dm.close()
     assert all(np.array_equal(a, b) for a, b in zip(*got))
+
+
+@pytest.mark.parametrize("hd,qh,kvh,D,lens,at", [(64, 4, 1, 256, [300, 65], [77, 1]), (64, 32, 4, 2048, [23, 187, 90, 61, 161], [5, 130, 64, 60, 100]), (128, 16, 2, 256, [130, 700], [129, 33]),
+                                                 (128, 5, 5, 320, [97], [40]), (64, 32, 4, 256, [4096], [2100])])
+def test_rows_do_not_see_what_comes_behind_them(dev, hd, qh, kvh, D, lens, at):
+    """Values a million times larger from a token on: the rows ahead of it have the bits that they have without, and the error against 64 bits that f32 rows have."""
+    rng = np.random.default_rng(sum(lens) + hd)
+    rows, K, n, F = sum(lens), qh * hd, len(lens), 64
+    q, k, v = (rng.standard_normal((rows, w)).astype(np.float32) for w in (K, kvh * hd, kvh * hd))
+    v *= 0.01
+    offs = u32(np.concatenate([[0], np.cumsum(lens)[:-1]]))
+    large, ahead = v.copy(), np.zeros(rows, bool)
+    for o, m, t in zip(offs, lens, at):
+        large[o + t:o + m] *= np.float32(2.0 ** 20)
+        ahead[o:o + t] = True
+    dq, dk = dev.up(q), dev.up(k)
+    wo, wg, wu = (f16bits(0.05 * rng.standard_normal(s)) for s in ((D, K), (F, D), (F, D)))
+    dwo, dwg, dwu, dres, dnw = (dev.up(t) for t in (wo, wg, wu, np.zeros((rows, D), np.float32), np.ones(D, np.float32)))
+    h_lens, slots = u32(lens), u32(range(n))
+    d_offs, d_lens, angles = dev.up(offs), dev.up(h_lens), dev.zeros(rows * hd // 2 * 8)
+    dev.call("m40llm_ext_prefill_angles_async", n, h_lens.ctypes.data, hd, 1e4, 1.0, angles.ptr, 0)
+    kv, att, got = m40.KVCache(dev.ctx, max(lens), n, kvh, hd), dev.zeros(rows * K * 4), []
+    for values in (v, large):
+        dv, x, hid = dev.up(values), dev.zeros(rows * D * 4), dev.zeros(rows * F * 4)
+        head = [kv.h, dq.ptr, dk.ptr, dv.ptr, d_offs.ptr, d_lens.ptr, n, slots.ctypes.data, offs.ctypes.data, h_lens.ctypes.data, qh, 0, angles.ptr, None, None, None]
+        dev.call("m40llm_ext_prefill_attention_project_gate_up_async", *head, rows, dwo.ptr, D, dres.ptr, x.ptr, dnw.ptr, 1, 1e-5, dwg.ptr, dwu.ptr, F, hid.ptr)
+        dev.call("m40llm_ext_prefill_attention_rope_append_async", *head, att.ptr)
+        dev.sync()
+        got.append(x.download(np.float32, (rows, D)))
+    assert np.array_equal(got[0][ahead].view(np.uint32), got[1][ahead].view(np.uint32))
+    a, w64 = att.download(np.float32, (rows, K)).astype(np.float64), wo.view(np.float16).astype(np.float64)
+    # operands exact to 2^-22 each, f32 sums of K products in chains of at most K / 32 steps
+    assert np.all(np.abs(got[1] - a @ w64.T) <= np.abs(a) @ np.abs(w64).T * 2.0 ** -20)
+    kv.destroy()
