@@ -905,7 +905,7 @@ public:
     }
 
     // Steps of one attention size from which a batched run records them as a graph.  Recording takes the host 0.2 to 0.55 ms a run, and a launch of the GPU's is
-    // longer than one of the host's at every size measured: steps launch by launch / recorded, us: TinyLlama shape, 32 rows, 4 steps 5084 / 5226, 20 steps 25 094 / 25 371;
+    // longer than one of the host's at every size measured, on a host with nothing else to do: steps launch by launch / recorded, us: TinyLlama shape, 32 rows, 4 steps 5084 / 5226, 20 steps 25 094 / 25 371;
     // 8 rows, 2 steps 1819 / 2093; Qwen2.5-3B shape, 2 rows, 8 steps 15 404 / 15 660; width 256, 22 layers, 8 rows, 48 steps 30 653 / 30 935.  A long run is
     // recorded all the same: it costs it less than a hundredth and leaves the host free.
     static constexpr uint32_t kRecordFrom = 48;
