@@ -45,6 +45,7 @@ public:
     static constexpr uint32_t kStream = LayerRuntime::kStream;
     static constexpr uint32_t kPage = LayerRuntime::kPage;
     static constexpr size_t kMostPinned = 16u << 20;       // bytes of host memory for a step's logits
+    static constexpr uint32_t kDirectRows = 4;             // most rows of logits that the head stores there itself
 
     LayeredDecoder(M40llmCudaContext* ctx, DecoderSpec spec, TensorSource& tensors, const LayeredOptions& opt)
         : ctx_(ctx), spec_(std::move(spec)), opt_(checked(ctx, opt)), seqs_(round_up(opt.max_tokens, kPage) / kPage, kPage, opt.max_sequences),
@@ -446,8 +447,8 @@ private:
         if (streams_) streams_->begin();
         for (auto& t : rt_.tables) t->enqueue(r);
     }
-    // final norm and head of n of a pass's rows (row_index NULL = all of them)
-    void enqueue_logits(const uint32_t* row_index, uint32_t n, uint32_t rows) {
+    // final norm and head of n of a pass's rows (row_index NULL = all of them), the logits to `to` (NULL = the device's buffer)
+    void enqueue_logits(const uint32_t* row_index, uint32_t n, uint32_t rows, float* to = nullptr) {
         if (streams_) streams_->last_sum(row_index, n);
         M40H_TRY(m40llm_ext_norm_rows_async(rt_.ctx, spec_.norm == NormKind::Rms ? M40LLM_NORM_RMS : M40LLM_NORM_LAYER, rt_.x.ptr(), rt_.planes.ptr(), rt_.pending,
                                             (uint64_t)rows * spec_.width, final_norm_.ptr(), row_index, n, spec_.width, spec_.eps, hn_.ptr(), rt_.d_pad,
@@ -457,7 +458,7 @@ private:
             g.epilogue = M40LLM_PACKED_CAP;
             g.out_scale = spec_.logit_scale; g.out_cap = spec_.logit_cap;
         }
-        g.out_f32 = logits_.ptr(); g.ld_out = spec_.vocab; g.cols = spec_.vocab;
+        g.out_f32 = to ? to : logits_.f32(); g.ld_out = spec_.vocab; g.cols = spec_.vocab;
         rt_.launch(g);
     }
 
@@ -470,13 +471,16 @@ private:
         Upload up;
         std::vector<uint32_t> key;
         const Rows r = provide(plan, tables_, longest, &want, up, &key, (bool)on_layer);
-        // The rows of a step of single tokens come through pinned memory, which a kernel behind the head writes: a blocking copy begins when the
-        // host has seen the head's end, and takes 16 us a row and 66 us for eight of 32000 against 10 and 35 with the wait for the stream.
+        // The rows of a step of single tokens come through pinned memory: a blocking copy begins when the host has seen the head's end, and takes 16 us a
+        // row and 66 us for eight of 32000.  Up to kDirectRows rows the head writes them there itself, while it reads its weights; its stores are 64 bytes a row, which
+        // take twice as long as those of a kernel behind it that copies whole kilobytes.  A step, that kernel / the head: one row 267 -> 262 us, three 296 -> 289, four
+        // 310 -> 307, eight 366 and 366.
         const auto pinned = [&](uint32_t n) { return !picks && (size_t)n * spec_.vocab * 4 <= logits_host_.bytes(); };
         const auto first_logits = [&] {
             const uint32_t n = (uint32_t)std::min<size_t>(logits_rows_, plan.want.size());
-            enqueue_logits(want, n, r.rows);
-            if (pinned(n)) M40H_TRY(m40llm_ext_copy_words_async(rt_.ctx, logits_host_.f32(), logits_.ptr(), (size_t)n * spec_.vocab, kStream));
+            const bool direct = pinned(n) && n <= kDirectRows && rt_.bf16();
+            enqueue_logits(want, n, r.rows, direct ? logits_host_.f32() : nullptr);
+            if (pinned(n) && !direct) M40H_TRY(m40llm_ext_copy_words_async(rt_.ctx, logits_host_.f32(), logits_.ptr(), (size_t)n * spec_.vocab, kStream));
         };
         const auto layers = [&] {
             enqueue_upload(up);
