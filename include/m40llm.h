@@ -696,6 +696,9 @@ typedef struct M40llmPackedGemm {
     const void* row_scale;        /* PROJECT: f32 [rows] (or slots), gate and up are multiplied by it before the activation; NULL = ones */
     float act_alpha, act_limit, out_scale, out_cap;
     uint32_t segment_tiles;       /* column tile t reads columns t / segment_tiles * a_batch on of a (0 = all read the same; else a multiple of 16, one batch) */
+    /* not NULL: an M40llmRoute (host memory) whose ids and weight are there and whose place and jobs this launch makes on the way: up to 64 experts, 16 rows, 64 choices, job_rows
+     * 16, bf16.  jobs, gather and row_scale NULL: the rows of a are plain; with the route's slot_weight (not written) a choice's weight multiplies gate and up.  PROJECT without plain tiles */
+    const void* route;
 } M40llmPackedGemm;
 int m40llm_ext_packed_gemm_async(M40llmCudaContext* ctx, const M40llmPackedGemm* g, uint32_t stream_kind);
 
@@ -752,7 +755,10 @@ typedef struct M40llmNormAdd {
     const void* weight;              /* f32 */
     const void* w;
     void *h, *h_rows;
-    uint32_t ld_h;
+    uint32_t ld_h, router_tiles;
+    /* route not NULL: an M40llmRoute (host memory) whose ids and weight this launch leaves, from the new h (the logits, their place not asked for, are its product with `router`, packed,
+     * router_tiles column tiles; the list is left to the product, M40llmPackedGemm).  bf16, up to 16 rows and 64 experts, ld_h 2048 to 4096, width a multiple of 8 */
+    const void *route, *router;
 } M40llmNormAdd;
 int m40llm_ext_norm_add_rows_async(M40llmCudaContext* ctx, const M40llmNormAdd* n, uint32_t stream_kind);
 /* out[row][c] = y / sqrt(mean(y^2) + eps) * w[c] * sigmoid(gate[row][c]), packed, ld_out columns, zero past cols (f32 rows y, gate) */
@@ -912,6 +918,8 @@ typedef struct M40llmStreamUpdate {
     void *h, *h_rows, *x_out;
     uint32_t ld_h;
     const uint32_t* row_index;
+    const void *route, *router;      /* as in M40llmNormAdd, for one or four streams and with w */
+    uint32_t router_tiles;
 } M40llmStreamUpdate;
 int m40llm_ext_stream_update_async(M40llmCudaContext* ctx, const M40llmStreamUpdate* u, uint32_t stream_kind);
 

@@ -11,24 +11,82 @@
 
 namespace {
 
+struct NoChoices {};
+template <int JOBS> struct ChoicesOf { using type = NoChoices; };
+template <> struct ChoicesOf<kFewIds> { using type = M40FewChoices; };
+
+// The list of experts in use from the choices of up to 64 (row, choice) pairs, a lane a pair: what few_lists_kernel makes, for the one expert that is number `job` of those in use.
+struct ChosenExpert {
+    int jobs, expert, rows;           // experts in use; this one (job < jobs), and how many rows took it
+    int pair, row;                    // of the lane's operand row: lane % 16, or its last row
+    uint32_t own;                     // the lane's choice (0xffffffff: none)
+    unsigned long long hits;          // the pairs that took it
+};
+__device__ __forceinline__ uint32_t or64(uint32_t v) {
+    v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, M40_DPP_XOR1, 0xf, 0xf, false);
+    v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, M40_DPP_XOR2, 0xf, 0xf, false);
+    v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, M40_DPP_HALF_MIRROR, 0xf, 0xf, false);
+    v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, M40_DPP_MIRROR, 0xf, 0xf, false);
+    return (uint32_t)(__builtin_amdgcn_readlane((int)v, 0) | __builtin_amdgcn_readlane((int)v, 16) | __builtin_amdgcn_readlane((int)v, 32) | __builtin_amdgcn_readlane((int)v, 48));
+}
+__device__ __forceinline__ int bits_below(unsigned long long mask) {          // of the lane
+    return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+}
+__device__ __forceinline__ ChosenExpert chosen_expert(const uint32_t* ids, int pairs, int top, uint32_t experts, int job, int lane) {
+    ChosenExpert c;
+    c.own = ids[lane < pairs ? lane : 0];
+    if (lane >= pairs) c.own = 0xffffffffu;
+    const bool real = c.own < experts;                                     // (experts at most 64)
+    const unsigned long long used = (unsigned long long)or64(real && c.own >= 32u ? 1u << (c.own - 32u) : 0u) << 32 | or64(real && c.own < 32u ? 1u << c.own : 0u);
+    c.jobs = __popcll(used);
+    c.expert = __ffsll(__ballot((used >> lane & 1ull) && bits_below(used) == job)) - 1;
+    c.hits = __ballot(real && (int)c.own == c.expert);
+    c.rows = __popcll(c.hits);
+    // pair of the lane's operand row: pairs that took the expert go to the lanes of their rank, the others to one that is not looked at
+    const int at = __builtin_amdgcn_ds_permute(4 * ((c.hits >> lane & 1ull) ? bits_below(c.hits) : 63), lane);
+    c.pair = __shfl(at, (lane & 15) < c.rows ? lane & 15 : (c.rows > 0 ? c.rows - 1 : 0), 64);
+    c.row = c.pair / top;
+    return c;
+}
+// What later launches read of the list: the first expert's job also says how many there are, and where rows go on as they are.
+__device__ __forceinline__ void store_list(const M40FewChoices& l, const ChosenExpert& c, int job, int lane) {
+    if (job < c.jobs && (c.hits >> lane & 1ull)) l.place[lane] = 16u * (uint32_t)job + (uint32_t)bits_below(c.hits);
+    if (job == 0 && lane < l.rows * l.top && c.own >= (uint32_t)l.experts) l.place[lane] = M40LLM_PLACE_INPUT;
+    if (lane != 0) return;
+    if (job < c.jobs) *reinterpret_cast<uint4*>(l.jobs + 4 + 4 * job) = make_uint4((uint32_t)c.expert, 16u * (uint32_t)job, (uint32_t)c.rows, 0u);
+    if (job == 0) *reinterpret_cast<uint2*>(l.jobs) = make_uint2((uint32_t)c.jobs, 16u * (uint32_t)c.jobs);
+}
+
 // The k tiles of a column tile are added up as PARTS sums (k tile i in sum i % PARTS, the sums in order), PARTS following from K alone, so that WAVES
 // changes no bit.  A wave requests U k tiles together, with AHEAD the next U before those are multiplied.  JOBS as in M40FewRows.
 //
 // All that the first requests need stands in plain arguments, which lie in registers when a wave starts (a structure is read from memory first): count is
-// the rows or, with jobs, lda in tiles; p0 the jobs or a_batch in tiles and above it the segment; p1 the gather list or k_total.
+// the rows or, with jobs, lda in tiles; p0 the jobs or a_batch in tiles and above it the segment; p1 the gather list or k_total.  kFewIds: p0 the choices, p1 their number, those
+// of a row and the experts (16, 16 and 32 bits).
 template <int NT, int WAVES, int PARTS, int U, bool AHEAD, int KIND, int JOBS>
 __global__ __launch_bounds__(WAVES * 64) void few_rows_kernel(const m40_bf16* rows_a, const m40_bf16* weights, int n_tiles, int k_tiles_in, int count, int k_stride, uint64_t p0, uint64_t p1,
-                                                                      long w_batch, M40Epilogue<m40_bf16> e) {
+                                                                      long w_batch, M40Epilogue<m40_bf16> e, typename ChoicesOf<JOBS>::type choices) {
     extern __shared__ __align__(16) float red[];       // [PARTS][NT][64][4]
     constexpr int kOwn = PARTS / WAVES;                // sums a wave keeps
     static_assert(PARTS % WAVES == 0 && U % kOwn == 0 && NT <= WAVES);
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), tile0 = (int)blockIdx.x * NT;
     int batch = blockIdx.z, row0 = 0, rows = count, k_tiles = k_tiles_in;
-    const m40_bf16* a = rows_a + (lane >> 4) * (JOBS == kFewGather ? 8 : 128);
+    constexpr bool kPlain = JOBS == kFewGather || JOBS == kFewIds;       // rows of a that a list names
+    float row_scale = 1.0f;
+    const m40_bf16* a = rows_a + (lane >> 4) * (kPlain ? 8 : 128);
     if (JOBS == kFewAll) {
         const int segment = (int)(p0 >> 32), k_total = (int)p1;
         a += (long)(segment ? tile0 / segment : batch) * (long)(uint32_t)p0 * kM40Tile + ((lane & 15) < rows ? lane & 15 : rows - 1) * 8;
         if (k_total && k_total - batch * k_tiles < k_tiles) k_tiles = k_total - batch * k_tiles;
+    } else if constexpr (JOBS == kFewIds) {
+        const ChosenExpert c = chosen_expert(reinterpret_cast<const uint32_t*>(p0), (int)(p1 & 0xffffu), (int)(p1 >> 16 & 0xffffu), (uint32_t)(p1 >> 32), (int)blockIdx.y, lane);
+        if (blockIdx.x == 0 && wave == 0) store_list(choices, c, (int)blockIdx.y, lane);
+        if ((int)blockIdx.y >= c.jobs) return;
+        batch = c.expert;
+        row0 = 16 * (int)blockIdx.y;
+        rows = c.rows;
+        a += (long)c.row * count * 32;
+        if (choices.weight_input) row_scale = static_cast<const float*>(choices.weight)[c.pair];
     } else {
         const uint32_t* jobs = reinterpret_cast<const uint32_t*>(p0);
         if (blockIdx.y >= jobs[0]) return;
@@ -40,7 +98,7 @@ __global__ __launch_bounds__(WAVES * 64) void few_rows_kernel(const m40_bf16* ro
         if (JOBS == kFewGather) a += (long)reinterpret_cast<const uint32_t*>(p1)[row0 + r] * count * 32;
         else a += (long)(row0 >> 4) * count * kM40Tile + r * 8;
     }
-    constexpr long kStep = JOBS == kFewGather ? 32 : kM40Tile;       // elements from k tile to k tile
+    constexpr long kStep = kPlain ? 32 : kM40Tile;       // elements from k tile to k tile
     const m40_bf16* w[NT];
 #pragma unroll
     for (int n = 0; n < NT; ++n) {
@@ -60,9 +118,9 @@ __global__ __launch_bounds__(WAVES * 64) void few_rows_kernel(const m40_bf16* ro
             if (u >= left) break;
 #pragma unroll
             for (int n = 0; n < NT; ++n) b.w[u][n] = m40_load_stream(reinterpret_cast<const uint4*>(w[n] + (long)(k + u * WAVES) * kM40Tile));
-            if (JOBS != kFewGather) b.a[u] = *reinterpret_cast<const m40_bf16x8*>(a + (long)(k + u * WAVES) * kStep);
+            if (!kPlain) b.a[u] = *reinterpret_cast<const m40_bf16x8*>(a + (long)(k + u * WAVES) * kStep);
         }
-        if (JOBS == kFewGather) {          // the rows' numbers are still on their way: all weights first
+        if (kPlain) {          // the rows' numbers are still on their way: all weights first
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 if (u >= left) break;
@@ -112,7 +170,10 @@ __global__ __launch_bounds__(WAVES * 64) void few_rows_kernel(const m40_bf16* ro
         return s;
     };
     if (KIND == M40LLM_PACKED_PROJECT && (JOBS != kFewAll || tile0 >= e.plain_tiles)) {
-        if (wave == 0) m40_epilogue_pair(e, row0, (tile0 - e.plain_tiles) / 2, lane, sum(0), sum(NT - 1));
+        if (wave == 0) {
+            if (JOBS == kFewIds) m40_epilogue_pair(e, row0, (tile0 - e.plain_tiles) / 2, lane, sum(0), sum(NT - 1), row_scale);
+            else m40_epilogue_pair(e, row0, (tile0 - e.plain_tiles) / 2, lane, sum(0), sum(NT - 1));
+        }
     } else if (wave < NT && tile0 + wave < n_tiles) {      // a wave a tile
         m40_epilogue_tile(e, JOBS == kFewAll ? batch : 0, row0, tile0 + wave, lane, sum(wave));
     }
@@ -126,7 +187,12 @@ int launch(hipStream_t stream, const M40FewRows& g, const M40Epilogue<m40_bf16>&
     const bool all = JOBS == kFewAll;
     const uint64_t p0 = all ? (uint64_t)(uint32_t)g.segment << 32 | (uint32_t)(g.a_batch / kM40Tile) : (uint64_t)reinterpret_cast<uintptr_t>(g.jobs);
     const uint64_t p1 = all ? (uint64_t)(uint32_t)g.k_total : (uint64_t)reinterpret_cast<uintptr_t>(g.gather);
-    few_rows_kernel<NT, WAVES, PARTS, U, AHEAD, KIND, JOBS><<<grid, WAVES * 64, lds, stream>>>(g.a, g.w, g.n_tiles, g.k_tiles, all ? g.rows : (int)(g.lda / 32), g.k_stride, p0, p1, g.w_batch, e);
+    if constexpr (JOBS == kFewIds)
+        few_rows_kernel<NT, WAVES, PARTS, U, AHEAD, KIND, JOBS><<<grid, WAVES * 64, lds, stream>>>(
+            g.a, g.w, g.n_tiles, g.k_tiles, (int)(g.lda / 32), g.k_stride, (uint64_t) reinterpret_cast<uintptr_t>(g.choices->ids),
+            (uint64_t)(g.choices->rows * g.choices->top) | (uint64_t)g.choices->top << 16 | (uint64_t)g.choices->experts << 32, g.w_batch, e, *g.choices);
+    else
+        few_rows_kernel<NT, WAVES, PARTS, U, AHEAD, KIND, JOBS><<<grid, WAVES * 64, lds, stream>>>(g.a, g.w, g.n_tiles, g.k_tiles, all ? g.rows : (int)(g.lda / 32), g.k_stride, p0, p1, g.w_batch, e, NoChoices{});
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 
@@ -135,7 +201,7 @@ int launch_kind(hipStream_t stream, const M40FewRows& g, const M40Epilogue<m40_b
     if constexpr (KIND == M40LLM_PACKED_PROJECT) {
         // pairs of tiles, us, 4 waves / 8: 176 pairs 8.3 / 6.3; 352, of which some CUs get one and some two, 9.8 / 10.4; 352 of four experts 10.4 / 11.1; 1056 of
         // twelve 22.4 / 21.4, 2816 of 32 39.7 / 38.4
-        const long long pairs = (long long)(g.n_tiles / 2) * (g.jobs ? g.max_jobs : g.batches);
+        const long long pairs = (long long)(g.n_tiles / 2) * (g.jobs || g.choices ? g.max_jobs : g.batches);
         if (pairs > num_cus && pairs <= 2ll * num_cus) return launch<2, 4, 8, 2, true, KIND, JOBS>(stream, g, e);
         return launch<2, 8, 8, 4, false, KIND, JOBS>(stream, g, e);
     } else {
@@ -152,6 +218,7 @@ int launch_kind(hipStream_t stream, const M40FewRows& g, const M40Epilogue<m40_b
 }  // namespace
 
 int m40_few_rows_product(hipStream_t stream, const M40FewRows& g, const M40Epilogue<m40_bf16>& e, int num_cus) {
+    if (g.choices) return launch_kind<M40LLM_PACKED_PROJECT, kFewIds>(stream, g, e, num_cus);
     if (g.jobs) return g.gather ? launch_kind<M40LLM_PACKED_PROJECT, kFewGather>(stream, g, e, num_cus) : launch_kind<M40LLM_PACKED_STORE_ACT, kFewSlots>(stream, g, e, num_cus);
     switch (e.kind) {
         case M40LLM_PACKED_STORE: return launch_kind<M40LLM_PACKED_STORE, kFewAll>(stream, g, e, num_cus);

@@ -10,6 +10,7 @@
 //
 // Products per expert: both kernels take a list of jobs (expert, rows of the list sorted by expert) made on the device; the rows are
 // gathered from plain rows (few rows, gate and up) or lie packed in list order.
+#include "norm_route.hpp"
 #include "packed_gemm.hpp"
 
 #include <type_traits>
@@ -495,7 +496,14 @@ M40Epilogue<T> make_epilogue(const M40llmPackedGemm& p) {
 }
 
 int launch_few(hipStream_t stream, const PackedArgs& g, const M40Epilogue<m40_bf16>& e, int batches, int num_cus) {
-    const M40FewRows f{static_cast<const m40_bf16*>(g.a), g.w, g.lda, g.a_batch, g.w_batch, g.n_tiles, g.k_tiles, g.rows, g.k_stride, g.k_total, g.segment, batches, g.jobs ? g.rows : 1, g.jobs, g.gather};
+    const M40FewRows f{static_cast<const m40_bf16*>(g.a), g.w, g.lda, g.a_batch, g.w_batch, g.n_tiles, g.k_tiles, g.rows, g.k_stride, g.k_total, g.segment, batches, g.jobs ? g.rows : 1, g.jobs, g.gather, nullptr};
+    return m40_few_rows_product(stream, f, e, num_cus);
+}
+
+// gate and up of the experts that a route's ids name; rows = most jobs
+int launch_choices(hipStream_t stream, const PackedArgs& g, const M40Epilogue<m40_bf16>& e, const M40llmRoute& q, bool weight_input, int num_cus) {
+    const M40FewChoices c{q.ids, q.weight, q.place, q.jobs, (int)q.rows, (int)q.top, (int)q.experts, weight_input};
+    const M40FewRows f{static_cast<const m40_bf16*>(g.a), g.w, g.lda, 0, g.w_batch, g.n_tiles, g.k_tiles, 0, g.k_stride, 0, 0, 1, g.rows, nullptr, nullptr, &c};
     return m40_few_rows_product(stream, f, e, num_cus);
 }
 
@@ -572,6 +580,14 @@ int m40llm_ext_packed_gemm_async(M40llmCudaContext* ctx, const M40llmPackedGemm*
     hipStream_t stream = m40_select_stream(ctx, stream_kind);
     if (!stream || m40_ensure_device(ctx) != 0) return -2;
     const bool paged = p->epilogue == M40LLM_PACKED_KEYS || p->epilogue == M40LLM_PACKED_VALUES;
+    const M40llmRoute* choices = static_cast<const M40llmRoute*>(p->route);
+    if (choices) {
+        if (!choices->ids || !choices->weight || !choices->place || !choices->jobs) return -1;
+        if (p->jobs || p->gather || p->row_scale || p->act_dtype != M40LLM_ACT_BF16 || p->epilogue != M40LLM_PACKED_PROJECT || p->plain_tiles != 0 || p->batches != 1u || p->k_parts > 1u || p->segment_tiles ||
+            m40_route_refused(*choices) || choices->job_rows != 16u || choices->rows * choices->top > 64u || choices->rows > 16u || choices->experts > 64u || !m40_aligned16(choices->jobs) ||
+            p->w_batch % 8 != 0)
+            return -3;
+    }
     const uint32_t k_parts = p->k_parts > 1u ? p->k_parts : 1u, part_tiles = (p->k_tiles + k_parts - 1) / k_parts;
     if (p->act_dtype > 1u || p->epilogue > M40LLM_PACKED_CAP || p->activation > M40LLM_LIMITED_GATE || p->rows == 0 || p->batches == 0 || p->batches > 65535u ||
         p->n_tiles == 0 || p->k_tiles == 0 || !m40_aligned16(p->a) || !m40_aligned16(p->w) || p->rows > 0x3fffffffu ||
@@ -636,6 +652,10 @@ int m40llm_ext_packed_gemm_async(M40llmCudaContext* ctx, const M40llmPackedGemm*
         batches = (int)k_parts;
     }
     (void)hipGetLastError();
+    if (choices) {
+        g.rows = (int)m40llm_ext_expert_max_jobs(choices->rows, choices->experts, choices->top, 16u);
+        return launch_choices(stream, g, make_epilogue<m40_bf16>(*p), *choices, choices->slot_weight != nullptr, ctx->num_cus);
+    }
     if (p->jobs) {
         g.jobs = p->jobs; g.gather = p->gather;
         g.rows = (int)p->max_jobs;

@@ -226,11 +226,10 @@ __device__ __forceinline__ void m40_epilogue_values(const M40Epilogue<m40_bf16>&
 // PROJECT, columns from plain_tiles on: tiles come in pairs (gate, up); pair p gives 16 activated columns
 template <class T>
 __device__ __forceinline__ void m40_epilogue_pair(const M40Epilogue<T>& e, int row0, int pair, int lane, const m40_float4& g,
-                                                  const m40_float4& u) {
+                                                  const m40_float4& u, float f) {
     const int col = pair * 16 + 4 * (lane >> 4), row = row0 + (lane & 15);
     if (row >= e.rows) return;
     m40_float4 y;
-    const float f = e.row_scale ? e.row_scale[row] : 1.0f;
     if (e.activation == M40LLM_LIMITED_GATE) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -244,15 +243,29 @@ __device__ __forceinline__ void m40_epilogue_pair(const M40Epilogue<T>& e, int r
     m40_store_packed<T>(e.out_act, row, e.act_col + col, e.ld_act, y, 4, true);
 }
 
+template <class T>
+__device__ __forceinline__ void m40_epilogue_pair(const M40Epilogue<T>& e, int row0, int pair, int lane, const m40_float4& g, const m40_float4& u) {
+    const int row = row0 + (lane & 15);
+    m40_epilogue_pair(e, row0, pair, lane, g, u, e.row_scale && row < e.rows ? e.row_scale[row] : 1.0f);
+}
+
 // A product of at most 16 bf16 rows (few_rows.hip).  All rows, of one batch or several (heads, parts of K), or products per expert: jobs with packed rows
-// in the order of the list, or with plain rows that `gather` names.
-enum { kFewAll = 0, kFewSlots = 1, kFewGather = 2 };
+// in the order of the list, or with plain rows that `gather` names, or that follow from the rows' choices, whose list the launch makes.
+enum { kFewAll = 0, kFewSlots = 1, kFewGather = 2, kFewIds = 3 };
+struct M40FewChoices {
+    const uint32_t* ids;           // [rows][top], rows * top at most 64
+    const void* weight;            // of the choices, f32
+    uint32_t *place, *jobs;        // written
+    int rows, top, experts;        // experts at most 64
+    bool weight_input;
+};
 struct M40FewRows {
     const m40_bf16 *a, *w;
     long lda, a_batch, w_batch;
     int n_tiles, k_tiles, rows, k_stride, k_total, segment, batches;      // as in a product of any rows
     int max_jobs;                  // 1 without jobs
     const uint32_t *jobs, *gather;
+    const M40FewChoices* choices;  // not null: jobs and gather are
 };
 int m40_few_rows_product(hipStream_t stream, const M40FewRows& g, const M40Epilogue<m40_bf16>& e, int num_cus);
 #endif  // __HIPCC__

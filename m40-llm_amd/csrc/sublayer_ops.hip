@@ -1,8 +1,9 @@
 // Row-wise steps of layers whose sublayers have their norm on the output: norm + residual add, norm + gate, and the step between an
 // attention's projections and its attention (short convolution, query and key norms, cache append).
-#include "packed_gemm.hpp"
+#include "norm_route.hpp"
 #include "pair_cache.hpp"
 #include "short_conv.hpp"
+#include "sublayer_rows.hpp"
 
 namespace {
 
@@ -19,104 +20,10 @@ __device__ __forceinline__ float block_sum(float v, float* scratch) {
     return s;
 }
 template <class T, bool VEC>
-__device__ __forceinline__ void load_group(const T* src, uint32_t at, uint32_t width, float (&v)[8]) {
-    if (VEC) {
-        const typename M40Act<T>::vec8 t = M40Act<T>::load8(src + at);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) v[i] = M40Act<T>::to(t[i]);
-    } else {
-#pragma unroll
-        for (uint32_t i = 0; i < 8; ++i) v[i] = at + i < width ? M40Act<T>::to(src[at + i]) : 0.0f;
-    }
-}
-
-// A thread takes groups of eight neighbouring elements and keeps two of them in registers (width up to 4096); beyond, sums are formed again.
-template <class T, bool VEC>
 __global__ __launch_bounds__(kThreads) void norm_add_rows_kernel(M40llmNormAdd a) {
     __shared__ float scratch[kThreads / 64];
-    constexpr uint32_t kGroups = 2;
-    const uint32_t row = m40_tile_row(blockIdx.x, a.rows), width = a.width, groups = a.ld_h / 8u;
-    float* x = static_cast<float*>(a.x) + (size_t)row * width;
-    const float* w = static_cast<const float*>(a.w);
-    auto value = [&](uint32_t g, float (&y)[8]) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) y[i] = 0.0f;
-        if (g * 8u >= width) return;
-        if (a.place) {
-            for (uint32_t j = 0; j < a.top; ++j) {
-                const uint32_t at = a.place[(size_t)row * a.top + j];
-                const float f = static_cast<const float*>(a.weight)[(size_t)row * a.top + j];
-                float v[8];
-                if (at == M40LLM_PLACE_INPUT) load_group<float, VEC>(x, g * 8u, width, v);
-                else load_group<T, VEC>(static_cast<const T*>(a.expert_out) + (size_t)at * a.ld_expert, g * 8u, width, v);
-#pragma unroll
-                for (int i = 0; i < 8; ++i) y[i] = fmaf(f, v[i], y[i]);
-            }
-        } else {
-            for (uint32_t p = 0; p < a.n_planes; ++p) {
-                float v[8];
-                load_group<float, VEC>(static_cast<const float*>(a.planes) + p * (size_t)a.plane_stride + (size_t)row * width, g * 8u, width, v);
-#pragma unroll
-                for (int i = 0; i < 8; ++i) y[i] += v[i];
-            }
-        }
-    };
-    // a row's old values and the weights, requested ahead of the sums
-    auto old_and_weights = [&](uint32_t g, float (&v)[8], float (&u)[8]) __attribute__((always_inline)) {
-        const uint32_t c = g * 8u < width ? g * 8u : 0u;
-        load_group<float, VEC>(x, c, width, v);
-        load_group<float, VEC>(w, c, width, u);
-    };
-    float keep[kGroups][8], keep_x[kGroups][8], keep_w[kGroups][8];
-    float q = 0.0f;
-    auto sq8 = [&](const float (&y)[8]) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) q = fmaf(y[i], y[i], q);
-    };
-#pragma unroll
-    for (uint32_t j = 0; j < kGroups; ++j) {
-        old_and_weights(threadIdx.x + j * kThreads, keep_x[j], keep_w[j]);
-        value(threadIdx.x + j * kThreads, keep[j]);
-        sq8(keep[j]);
-    }
-    for (uint32_t g = threadIdx.x + kGroups * kThreads; g < groups; g += kThreads) {
-        float y[8];
-        value(g, y);
-        sq8(y);
-    }
-    const float f = a.mult / sqrtf(block_sum(q, scratch) / (float)width + a.eps);
-    auto finish = [&](uint32_t g, const float (&y)[8], const float (&old)[8], const float (&u)[8]) __attribute__((always_inline)) {
-        float v[8];
-        if (g * 8u < width) {
-#pragma unroll
-            for (uint32_t i = 0; i < 8; ++i) v[i] = VEC || g * 8u + i < width ? fmaf(y[i] * f, u[i], old[i]) : 0.0f;
-            if (VEC) {
-                reinterpret_cast<float4*>(x + g * 8u)[0] = make_float4(v[0], v[1], v[2], v[3]);
-                reinterpret_cast<float4*>(x + g * 8u)[1] = make_float4(v[4], v[5], v[6], v[7]);
-            } else {
-#pragma unroll
-                for (uint32_t i = 0; i < 8; ++i)
-                    if (g * 8u + i < width) x[g * 8u + i] = v[i];
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < 8; ++i) v[i] = 0.0f;
-        }
-        const m40_float4 lo = {v[0], v[1], v[2], v[3]}, hi = {v[4], v[5], v[6], v[7]};
-        m40_store8<T>(static_cast<T*>(a.h) + m40_packed_at(row, g * 8u, a.ld_h >> 5), lo, hi);
-        if (a.h_rows) m40_store8<T>(static_cast<T*>(a.h_rows) + (size_t)row * a.ld_h + g * 8u, lo, hi);
-    };
-#pragma unroll
-    for (uint32_t j = 0; j < kGroups; ++j) {
-        const uint32_t g = threadIdx.x + j * kThreads;
-        if (g < groups) finish(g, keep[j], keep_x[j], keep_w[j]);
-    }
-    for (uint32_t g = threadIdx.x + kGroups * kThreads; g < groups; g += kThreads) {
-        float y[8], v[8], u[8];
-        old_and_weights(g, v, u);
-        value(g, y);
-        finish(g, y, v, u);
-    }
+    const uint32_t row = m40_tile_row(blockIdx.x, a.rows);
+    m40_norm_add_row<T, VEC>(a, row, threadIdx.x, scratch, [&](uint32_t g, const m40_float4& lo, const m40_float4& hi) { m40_store_input<T>(a, row, g, lo, hi); });
 }
 
 template <class T, bool VEC>
@@ -129,7 +36,7 @@ __global__ __launch_bounds__(kThreads) void norm_gate_rows_kernel(const float* _
     float q = 0.0f;
     for (uint32_t g = threadIdx.x; g * 8u < cols; g += kThreads) {
         float v[8];
-        load_group<float, VEC>(src, g * 8u, cols, v);
+        m40_load_group<float, VEC>(src, g * 8u, cols, v);
 #pragma unroll
         for (int i = 0; i < 8; ++i) q = fmaf(v[i], v[i], q);
     }
@@ -140,9 +47,9 @@ __global__ __launch_bounds__(kThreads) void norm_gate_rows_kernel(const float* _
         for (int i = 0; i < 8; ++i) v[i] = 0.0f;
         if (g * 8u < cols) {
             float z[8], u[8];
-            load_group<float, VEC>(src, g * 8u, cols, v);
-            load_group<float, VEC>(gt, g * 8u, cols, z);
-            load_group<float, VEC>(w, g * 8u, cols, u);
+            m40_load_group<float, VEC>(src, g * 8u, cols, v);
+            m40_load_group<float, VEC>(gt, g * 8u, cols, z);
+            m40_load_group<float, VEC>(w, g * 8u, cols, u);
 #pragma unroll
             for (uint32_t i = 0; i < 8; ++i) v[i] = VEC || g * 8u + i < cols ? v[i] * inv * u[i] * m40_sigmoid(z[i]) : 0.0f;
         }
@@ -240,6 +147,13 @@ int m40llm_ext_norm_add_rows_async(M40llmCudaContext* ctx, const M40llmNormAdd* 
     if (n->rows == 0 || n->width == 0 || n->ld_h < n->width || n->ld_h % 32u != 0 || n->act_dtype > 1u || !m40_aligned16(n->h) || (n->h_rows && !m40_aligned16(n->h_rows)))
         return -3;
     const bool vec = n->width % 8u == 0 && m40_aligned16(n->x) && m40_aligned16(n->w) && (n->place ? n->ld_expert % 8u == 0 && m40_aligned16(n->expert_out) : n->plane_stride % 4u == 0 && m40_aligned16(n->planes));
+    if (n->route) {
+        const M40llmRoute* q = static_cast<const M40llmRoute*>(n->route);
+        if (!q->ids || !q->weight || !q->rows_of || !q->place || !q->jobs) return -1;
+        if (!vec || m40_route_refused(*q)) return -3;
+        (void)hipGetLastError();
+        return m40_norm_add_route(stream, *n);
+    }
     if (n->act_dtype == M40LLM_ACT_F32) {
         if (vec) norm_add_rows_kernel<float, true><<<n->rows, kThreads, 0, stream>>>(*n);
         else norm_add_rows_kernel<float, false><<<n->rows, kThreads, 0, stream>>>(*n);

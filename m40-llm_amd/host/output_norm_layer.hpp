@@ -297,9 +297,19 @@ struct SublayerOut {
     }
 };
 
+// The router's product and the choice of experts as part of the launch that makes the rows; none where route is null.
+struct Routing {
+    const M40llmRoute* route = nullptr;
+    const void* router = nullptr;
+    uint32_t tiles = 0;
+    template <class N>
+    void put(N& n) const { n.route = route; n.router = router; n.router_tiles = tiles; }
+};
+
 class FeedForward {
 public:
     virtual ~FeedForward() = default;
+    virtual Routing routing(const Rows&) { return {}; }          // for the launch before enqueue, which leaves it to that launch
     virtual SublayerOut enqueue(const Rows& r) = 0;
     virtual bool reads_plain_rows() const { return false; }      // it wants its input as plain rows (h_rows) as well
 };
@@ -415,22 +425,19 @@ public:
         if (m.weight_input) sh_->slot_weight.want((size_t)slots * 4);
     }
     bool reads_plain_rows() const override { return true; }
+    Routing routing(const Rows& r) override {
+        if (!beside_norm(r)) return {};
+        route_ = route(r);
+        return {&route_, w_router_.ptr(), router_tiles_};
+    }
     SublayerOut enqueue(const Rows& r) override {
         SublayerOut n;
-        {
+        const uint32_t job_rows = rows_a_job(r.rows), max_jobs = m40llm_ext_expert_max_jobs(r.rows, m_.experts, m_.top, job_rows);
+        if (!beside_norm(r)) {
             M40llmPackedGemm g = rt_.product(rt_.h.ptr(), rt_.d_pad, w_router_, router_tiles_, rt_.d_pad / 32, r.rows, M40LLM_PACKED_STORE);
             g.out_f32 = sh_->logits.ptr(); g.ld_out = router_tiles_ * 16; g.cols = router_tiles_ * 16;
             rt_.launch(g);
-        }
-        const uint32_t job_rows = rows_a_job(r.rows), max_jobs = m40llm_ext_expert_max_jobs(r.rows, m_.experts, m_.top, job_rows);
-        {
-            M40llmRoute q{};
-            q.rows = r.rows; q.experts = m_.experts; q.identity = m_.identity; q.top = m_.top; q.job_rows = job_rows; q.groups = m_.groups; q.keep = m_.keep; q.scale = m_.scale;
-            q.logits = sh_->logits.ptr(); q.ld_logits = router_tiles_ * 16; q.correction = correction_.ptr();
-            q.ids = sh_->ids.u32(); q.weight = sh_->weight.ptr();
-            q.rows_of = sh_->rows_of.u32(); q.place = sh_->place.u32(); q.jobs = sh_->jobs.u32();
-            q.score = m_.score == RouterScore::Sigmoid ? M40LLM_SCORE_SIGMOID : M40LLM_SCORE_SOFTMAX;
-            if (m_.weight_input) q.slot_weight = sh_->slot_weight.ptr();
+            const M40llmRoute q = route(r);
             M40H_TRY(m40llm_ext_route_rows_async(rt_.ctx, &q, rt_.kStream));
         }
         const uint32_t d_tiles = rt_.d_pad / 32, down_tiles = round_up(rt_.spec.width, 16) / 16;
@@ -438,15 +445,19 @@ public:
             M40llmPackedGemm g = rt_.product(rt_.h_rows.ptr(), rt_.d_pad, w_in_, 2 * tiles_, d_tiles, r.rows, M40LLM_PACKED_PROJECT);
             g.activation = activation_code(m_.activation);
             g.act_limit = m_.limit; g.act_alpha = m_.alpha;
-            if (m_.weight_input) g.row_scale = sh_->slot_weight.ptr();      // gate and up are linear in the input
-            if (job_rows == 128) {
-                M40H_TRY(m40llm_ext_gather_rows_async(rt_.ctx, rt_.h_rows.ptr(), rt_.d_pad, sh_->rows_of.u32(), sh_->jobs.u32(),
-                                                      m40llm_ext_expert_slots(r.rows, m_.experts, m_.top), sh_->rows.ptr(), rt_.kStream));
-                g.a = sh_->rows.ptr();
+            if (beside_norm(r)) {
+                g.route = &route_;
             } else {
-                g.gather = sh_->rows_of.u32();
+                if (m_.weight_input) g.row_scale = sh_->slot_weight.ptr();      // gate and up are linear in the input
+                if (job_rows == 128) {
+                    M40H_TRY(m40llm_ext_gather_rows_async(rt_.ctx, rt_.h_rows.ptr(), rt_.d_pad, sh_->rows_of.u32(), sh_->jobs.u32(),
+                                                          m40llm_ext_expert_slots(r.rows, m_.experts, m_.top), sh_->rows.ptr(), rt_.kStream));
+                    g.a = sh_->rows.ptr();
+                } else {
+                    g.gather = sh_->rows_of.u32();
+                }
+                g.jobs = sh_->jobs.u32(); g.max_jobs = max_jobs; g.job_rows = job_rows;
             }
-            g.jobs = sh_->jobs.u32(); g.max_jobs = max_jobs; g.job_rows = job_rows;
             g.w_batch = (uint64_t)2 * tiles_ * d_tiles * 512;
             g.out_act = sh_->act.ptr(); g.ld_act = pad_;
             rt_.launch(g);
@@ -472,9 +483,25 @@ private:
         if (rt_.bf16() && rows > 64 && mean >= 48) return 128;
         return mean <= 24 ? 32 : 64;
     }
+    M40llmRoute route(const Rows& r) const {
+        M40llmRoute q{};
+        q.rows = r.rows; q.experts = m_.experts; q.identity = m_.identity; q.top = m_.top; q.job_rows = rows_a_job(r.rows); q.groups = m_.groups; q.keep = m_.keep; q.scale = m_.scale;
+        q.logits = sh_->logits.ptr(); q.ld_logits = router_tiles_ * 16; q.correction = correction_.ptr();
+        q.ids = sh_->ids.u32(); q.weight = sh_->weight.ptr();
+        q.rows_of = sh_->rows_of.u32(); q.place = sh_->place.u32(); q.jobs = sh_->jobs.u32();
+        q.score = m_.score == RouterScore::Sigmoid ? M40LLM_SCORE_SIGMOID : M40LLM_SCORE_SOFTMAX;
+        if (m_.weight_input) q.slot_weight = sh_->slot_weight.ptr();
+        return q;
+    }
+    // The choice beside the norm and the list beside gate and up, where both have a form for it: up to 16 rows of 2048 to 4096 and 64 choices of up to 64 experts.
+    bool beside_norm(const Rows& r) const {
+        const bool streams = rt_.spec.block == BlockKind::OutputNorm || rt_.spec.streams == 1 || rt_.spec.streams == 4;
+        return rt_.bf16() && r.rows <= 16 && streams && rt_.spec.width % 8 == 0 && rt_.d_pad >= 2048 && rt_.d_pad <= 4096 && router_tiles_ <= 4 && r.rows * m_.top <= 64;
+    }
     LayerRuntime& rt_;
     std::shared_ptr<ExpertShared> sh_;
     ExpertMlpSpec m_;
+    M40llmRoute route_{};
     uint32_t tiles_, pad_, out_cols_, router_tiles_;
     DeviceBuf w_router_, correction_, w_in_, w_out_;
 };
@@ -500,6 +527,7 @@ public:
         m.planes = rt_.planes.ptr(); m.plane_stride = (uint64_t)r.rows * rt_.spec.width;
         m.w = norm1_.ptr();
         m.h_rows = ff_ && ff_->reads_plain_rows() ? rt_.h_rows.ptr() : nullptr;
+        if (ff_) ff_->routing(r).put(m);
         M40H_TRY(m40llm_ext_norm_add_rows_async(rt_.ctx, &m, rt_.kStream));
         if (!ff_) return;
         ff_->enqueue(r).put(n);

@@ -32,11 +32,12 @@ public:
     }
     void begin() { fresh_ = true; pending_ = nullptr; }          // all streams are the embedding's rows
     // what the sublayer of these weights reads, as packed (and plain) rows
-    void read(const Rows& r, const StreamWeights& w, bool plain_rows) {
+    void read(const Rows& r, const StreamWeights& w, bool plain_rows, const Routing& routing = {}) {
         M40llmStreamUpdate u = update(r.rows);
         u.take = w.take.ptr(); u.w = w.norm.ptr();
         u.h = rt_.h.ptr(); u.ld_h = rt_.d_pad;
         u.h_rows = plain_rows ? rt_.h_rows.ptr() : nullptr;
+        routing.put(u);
         M40H_TRY(m40llm_ext_stream_update_async(rt_.ctx, &u, rt_.kStream));
         taken();
     }
@@ -487,7 +488,7 @@ public:
         y.planes = rt_.planes.ptr(); y.plane_stride = (uint64_t)r.rows * rt_.spec.width;
         streams_.write(w_->mix, y);
         if (w_->ff) {
-            streams_.read(r, w_->feed, w_->ff->reads_plain_rows());
+            streams_.read(r, w_->feed, w_->ff->reads_plain_rows(), w_->ff->routing(r));
             streams_.write(w_->feed, w_->ff->enqueue(r));
         }
         if (r.in_place) streams_.sum(r);

@@ -1,0 +1,120 @@
+"""The norm before a routed feed-forward with the router's product and the choice of experts in its launch, and the experts' first product with the list of rows by expert in its,
+beside the launches one by one: the same bits everywhere."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+from pimosun_common import c_struct, ld, m40, pack_tiles, up32  # noqa: E402
+from test_gpu_layer_kernels import PROJECT, call  # noqa: E402
+
+NormAdd, Update, Route, Gemm = (c_struct("M40llm" + n) for n in ("NormAdd", "StreamUpdate", "Route", "PackedGemm"))
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    yield m40.Context(0)
+
+
+def run(ctx, fused, rows, width, streams, experts, identity, top, groups, sigmoid, weighted, source, odd=False, times=3):
+    rng, keep = np.random.default_rng(rows * width + experts), []
+    f32 = lambda *s: rng.standard_normal(s).astype(np.float32)          # noqa: E731
+
+    def put(a):
+        keep.append(ctx.to_device(np.ascontiguousarray(a)))
+        return keep[-1]
+    all_, ldh, tiles = experts + identity, up32(width), (experts + identity + 15) // 16
+    W = np.zeros((tiles * 16, ldh), np.float32)
+    W[:all_, :width] = 3 * f32(all_, width) / np.sqrt(width)
+    router = put(pack_tiles(ld.f32_to_bf16(W)))
+    correction = put(0.1 * f32(all_))
+    planes = f32(3, rows, width)
+    if odd:
+        planes[0, 0, 5] = np.nan
+        planes[1, -1, 7] = np.inf
+    sub = dict(act_dtype=0, rows=rows, width=width, eps=1e-5, mult=0.7, ld_h=ldh, w=put(1 + 0.2 * f32(width)).ptr)
+    if source == "planes":
+        sub.update(planes=put(planes).ptr, n_planes=3, plane_stride=rows * width)
+    else:
+        place = rng.permutation(rows * 3).astype(np.uint32).reshape(rows, 3)
+        if not streams:
+            place[0, 1] = 0xffffffff
+        sub.update(expert_out=put(ld.f32_to_bf16(f32(rows * 3, width))).ptr, ld_expert=width, place=put(place).ptr, weight=put(np.abs(f32(rows, 3))).ptr, top=3)
+    if streams:
+        x, stride = put(f32(streams, rows, width)), rows * width
+        sub.update(streams=streams, streams_x=x.ptr, stream_stride=stride, mix=put(f32(streams, streams)).ptr, share=put(f32(streams)).ptr, take=put(f32(streams)).ptr)
+    else:
+        x = put(f32(rows, width))
+        sub.update(x=x.ptr)
+    slots = ctx.lib.m40llm_ext_expert_slots(rows, experts, top)
+    jobs_n = 4 + 4 * ctx.lib.m40llm_ext_expert_max_jobs(rows, experts, top, 16)
+    gate_up = put(ld.f32_to_bf16(f32(experts * 96 * ldh) / np.sqrt(width)))      # any numbers in the order of the tiles: six column tiles an expert
+    out = dict(act=put(np.zeros((slots, 64), np.uint16)), h=put(np.zeros(16 * ldh, np.uint16)), h_rows=put(np.zeros((rows, ldh), np.uint16)), ids=put(np.full(rows * top, 77, np.uint32)), weight=put(f32(rows * top)),
+               place=put(np.zeros(rows * top, np.uint32)), jobs=put(np.zeros(jobs_n, np.uint32)), x=x)
+    rows_of, slot_weight = put(np.full(slots, 99, np.uint32)), put(np.zeros(slots, np.float32))
+    logits = put(np.zeros((rows, tiles * 16), np.float32))
+    q = Route(rows=rows, experts=experts, identity=identity, top=top, job_rows=16, groups=groups, keep=max(1, groups // 2), score=int(sigmoid), scale=1.5, logits=logits.ptr, ld_logits=tiles * 16,
+              correction=correction.ptr, ids=out["ids"].ptr, weight=out["weight"].ptr, rows_of=rows_of.ptr, place=out["place"].ptr, jobs=out["jobs"].ptr,
+              slot_weight=slot_weight.ptr if weighted else None)
+    sub.update(h=out["h"].ptr, h_rows=out["h_rows"].ptr)
+    name, struct = ("m40llm_ext_stream_update_async", Update) if streams else ("m40llm_ext_norm_add_rows_async", NormAdd)
+    got = []
+    for _ in range(times):       # the streams go on from time to time; the rows' count is to be zero again
+        if fused:
+            call(ctx, name, C.byref(struct(**sub, route=C.addressof(q), router=router.ptr, router_tiles=tiles)), 1)
+        else:
+            call(ctx, name, C.byref(struct(**sub)), 1)
+            g = Gemm(act_dtype=0, epilogue=0, a=out["h"].ptr, lda=ldh, w=router.ptr, n_tiles=tiles, k_tiles=ldh // 32, rows=rows, batches=1, out_f32=logits.ptr, ld_out=tiles * 16, cols=tiles * 16)
+            call(ctx, "m40llm_ext_packed_gemm_async", C.byref(g), 1)
+            call(ctx, "m40llm_ext_route_rows_async", C.byref(q), 1)
+        g = Gemm(act_dtype=0, epilogue=PROJECT, a=out["h_rows"].ptr, lda=ldh, w=gate_up.ptr, n_tiles=6, k_tiles=ldh // 32, rows=rows, batches=1, w_batch=96 * ldh, out_act=out["act"].ptr, ld_act=64, activation=1)
+        if fused:
+            g.route = C.addressof(q)
+        else:
+            g.jobs, g.gather, g.max_jobs, g.job_rows, g.row_scale = out["jobs"].ptr, rows_of.ptr, (jobs_n - 4) // 4, 16, slot_weight.ptr if weighted else None
+        call(ctx, "m40llm_ext_packed_gemm_async", C.byref(g), 1)
+        ctx.sync(1)
+        got.append({n: b.download(np.uint8, (b.nbytes,)) for n, b in out.items()})
+    return got
+
+
+@pytest.mark.parametrize("rows,width,streams,experts,identity,top,groups,sigmoid,weighted,source", [
+    (1, 2048, 0, 32, 2, 4, 0, False, False, "planes"), (8, 2048, 0, 32, 2, 4, 0, False, False, "experts"), (10, 4096, 0, 62, 2, 6, 0, True, True, "planes"),
+    (1, 2048, 1, 32, 0, 4, 0, True, True, "planes"), (5, 2072, 1, 20, 0, 2, 0, False, True, "experts"), (1, 2048, 1, 48, 0, 48, 0, True, False, "planes"),
+    (1, 2048, 4, 32, 0, 4, 8, False, False, "planes"), (3, 4064, 4, 64, 0, 4, 8, False, False, "experts"), (16, 2048, 4, 8, 0, 1, 0, True, True, "planes"), (16, 2048, 0, 33, 31, 4, 0, False, False, "planes"),
+    (2, 2080, 0, 1, 0, 1, 0, False, False, "planes")])
+@pytest.mark.parametrize("odd", [False, True])
+def test_norm_with_the_router_behind_it(ctx, odd, rows, width, streams, experts, identity, top, groups, sigmoid, weighted, source):
+    want, got = (run(ctx, fused, rows, width, streams, experts, identity, top, groups, sigmoid, weighted, source, odd) for fused in (False, True))
+    for i, (a, b) in enumerate(zip(want, got)):
+        for n in a:
+            assert np.array_equal(a[n], b[n]), (i, n)
+
+
+def test_what_the_launch_has_no_form_for_is_refused(ctx):
+    x = ctx.to_device(np.zeros(4096 * 32, np.float32))
+    p = x.ptr
+
+    def rc(rows=2, width=2048, streams=0, tiles=2, experts=32, job_rows=16, top=4, router=p, dtype=0, ids=p, ld=None):
+        q = Route(rows=rows, experts=experts, top=top, job_rows=job_rows, ids=ids, weight=p, rows_of=p, place=p, jobs=p)
+        both = dict(act_dtype=dtype, rows=rows, width=width, ld_h=ld or up32(width), planes=p, n_planes=1, plane_stride=width, w=p, h=p, route=C.addressof(q), router=router, router_tiles=tiles)
+        if streams:
+            return ctx.lib.m40llm_ext_stream_update_async(ctx.h, C.byref(Update(streams=streams, streams_x=p, stream_stride=width, mix=p, share=p, take=p, **both)), 1)
+        return ctx.lib.m40llm_ext_norm_add_rows_async(ctx.h, C.byref(NormAdd(x=p, **both)), 1)
+    for streams in (0, 1):
+        assert rc(streams=streams, ids=None) == -1
+        for bad in (dict(rows=17), dict(width=2016), dict(width=4128), dict(width=2044), dict(tiles=0), dict(tiles=5), dict(tiles=1), dict(router=None), dict(router=p + 4), dict(dtype=1),
+                    dict(top=33)):
+            assert rc(streams=streams, **bad) == -3, bad
+    assert rc(streams=2) == rc(streams=16) == -3
+    route = dict(experts=32, job_rows=16, top=4, ids=p, weight=p, rows_of=p, place=p, jobs=p)
+    gemm = dict(act_dtype=0, epilogue=PROJECT, a=p, lda=2048, w=p, n_tiles=2, k_tiles=64, batches=1, out_act=p, ld_act=32)
+
+    def product(more={}, **kw):
+        q = Route(**dict(dict(route, rows=2), **kw))
+        return ctx.lib.m40llm_ext_packed_gemm_async(ctx.h, C.byref(Gemm(**dict(gemm, rows=2, route=C.addressof(q), **more))), 1)
+    assert product(dict(jobs=p)) == product(dict(gather=p)) == product(dict(row_scale=p)) == product(dict(plain_tiles=2, out_f32=p)) == -3
+    assert [product(**dict(dict(route, rows=2), **bad)) for bad in (dict(rows=17), dict(job_rows=32), dict(top=33), dict(experts=65), dict(rows=16, top=5), dict(rows=0))] == [-3] * 6
+    assert product(**dict(route, ids=None)) == -1
