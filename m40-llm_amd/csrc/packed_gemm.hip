@@ -193,8 +193,8 @@ int launch_rows_any(hipStream_t stream, const PackedArgs& g, const M40Epilogue<T
 }
 
 // ---- many rows, bf16 ---------------------------------------------------------------------------------------------------
-// Workgroup of four waves (2 x 2), wave tile 16 MTW x 16 NTW: C tile 32 MTW x 32 NTW.  A stage is KS k tiles of every operand
-// tile: 2 (MTW + NTW) KS KB, filled by global_load_lds (a wave's instruction moves one 16 x 32 operand tile, a contiguous kilobyte).
+// Workgroup of WM x WN waves, wave tile 16 MTW x 16 NTW: C tile 16 WM MTW x 16 WN NTW.  A stage is KS k tiles of every operand
+// tile: (WM MTW + WN NTW) KS KB, filled by global_load_lds (a wave's instruction moves one 16 x 32 operand tile, a contiguous kilobyte).
 //
 // Memory instructions are issued under matrix instructions: the fragments of the next step and the loads of a stage kBufs - 1
 // ahead go out one at a time between the current step's products (sched_group_barrier), so that no wave waits for an address
@@ -214,20 +214,21 @@ template <int... I, class F>
 __device__ __forceinline__ void unrolled(std::integer_sequence<int, I...>, F&& f) { (f(std::integral_constant<int, I>{}), ...); }
 
 // rows of tiles of a wave whose sums fit into the buffers at a time
-constexpr int tile_part(int mtw, int ntw, int ks, int bufs) {
+constexpr int tile_part(int mtw, int ntw, int wm, int wn, int ks, int bufs) {
     int part = mtw;
-    while (4 * part * ntw > 2 * (mtw + ntw) * ks * bufs) part /= 2;
+    while (wm * wn * part * ntw > (wm * mtw + wn * ntw) * ks * bufs) part /= 2;
     return part;
 }
 
-template <int MTW, int NTW, int KS, int kBufs, int FORM>
-__global__ __launch_bounds__(256, 1) void tile_packed_kernel(PackedArgs g, M40Epilogue<m40_bf16> e, int band) {
+template <int MTW, int NTW, int WM, int WN, int KS, int kBufs, int FORM>
+__global__ __launch_bounds__(64 * WM * WN, 1) void tile_packed_kernel(PackedArgs g, M40Epilogue<m40_bf16> e, int band) {
     typedef __attribute__((address_space(3))) void* lds_dst_t;
     typedef const __attribute__((address_space(1))) void* global_src_t;
     extern __shared__ __align__(16) uint8_t stage_lds[];
-    constexpr int kATiles = 2 * MTW, kBTiles = 2 * NTW, kRows = 16 * kATiles;      // 16-row operand tiles of the workgroup
+    constexpr int kWaves = WM * WN, kATiles = WM * MTW, kBTiles = WN * NTW, kRows = 16 * kATiles;      // 16-row operand tiles of the workgroup
     constexpr int kStageBytes = (kATiles + kBTiles) * KS * 1024;
-    constexpr int kALoads = kATiles * KS / 4, kLoads = (kATiles + kBTiles) * KS / 4;      // per wave and stage
+    static_assert(kATiles * KS % kWaves == 0 && kBTiles * KS % kWaves == 0);
+    constexpr int kALoads = kATiles * KS / kWaves, kLoads = (kATiles + kBTiles) * KS / kWaves;      // per wave and stage
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     constexpr bool kJobs = FORM == kSlots, kPaged = FORM == kPageKeys || FORM == kPageValues;
     const int tiles_n = (g.n_tiles + kBTiles - 1) / kBTiles, tiles_m = kJobs ? (int)g.jobs[0] : (g.rows + kRows - 1) / kRows;
@@ -248,14 +249,14 @@ __global__ __launch_bounds__(256, 1) void tile_packed_kernel(PackedArgs g, M40Ep
     }
     const int stages = g.k_count(batch) / KS;
     // A scalar address that walks k, and per lane a 32-bit offset from it that does not change (cache pages lie anywhere: whole addresses).
-    // This wave's pieces of a stage: operand tiles' k tiles wave, wave + 4, ... of A, then of the weights.
+    // This wave's pieces of a stage: operand tiles' k tiles wave, wave + kWaves, ... of A, then of the weights.
     const uint8_t* a_base = static_cast<const uint8_t*>(g.a) + ((kJobs ? 0 : (g.segment ? t0 / g.segment : batch) * g.a_batch) + (long)m0 * g.lda) * 2;
     const uint8_t* w_base = reinterpret_cast<const uint8_t*>(g.w + batch * g.w_batch + (long)t0 * g.k_stride * kM40Tile);
     const uint8_t* page[kPaged ? kALoads : 1];
     uint32_t off[kLoads];
 #pragma unroll
     for (int i = 0; i < kLoads; ++i) {
-        const int piece = wave + 4 * i, sub = piece % KS, t = piece / KS;
+        const int piece = wave + kWaves * i, sub = piece % KS, t = piece / KS;
         if (i >= kALoads) {
             const int n = t0 + t - kATiles;
             off[i] = (uint32_t)((n < g.n_tiles ? n : g.n_tiles - 1) - t0) * (uint32_t)g.k_stride * 1024u + sub * 1024u + lane * 16u;
@@ -274,10 +275,10 @@ __global__ __launch_bounds__(256, 1) void tile_packed_kernel(PackedArgs g, M40Ep
 #pragma unroll
         for (int i = 0; i < kLoads; ++i) {
             const uint8_t* src = i >= kALoads ? w_base + k + off[i] : kPaged ? page[kPaged ? i : 0] + k : a_base + k + off[i];
-            __builtin_amdgcn_global_load_lds((global_src_t)src, (lds_dst_t)(base + i * 4096), 16, 0, 0);
+            __builtin_amdgcn_global_load_lds((global_src_t)src, (lds_dst_t)(base + i * (kWaves * 1024)), 16, 0, 0);
         }
     };
-    const int wm = wave >> 1, wn = wave & 1;
+    const int wm = wave / WN, wn = wave % WN;
     m40_float4 acc[MTW][NTW];
 #pragma unroll
     for (int i = 0; i < MTW; ++i)
@@ -373,7 +374,7 @@ __global__ __launch_bounds__(256, 1) void tile_packed_kernel(PackedArgs g, M40Ep
     }
     // The sums go through LDS (each wave its own, as many rows of tiles at a time as fit) so that the last step is a loop of a few instructions
     // and not MTW NTW copies of it: run once per workgroup, those would be fetched cold.
-    constexpr int kPart = tile_part(MTW, NTW, KS, kBufs);
+    constexpr int kPart = tile_part(MTW, NTW, WM, WN, KS, kBufs);
     m40_float4* mine = reinterpret_cast<m40_float4*>(stage_lds) + wave * kPart * NTW * 64 + lane;
 #pragma unroll 1
     for (int part = 0; part < MTW / kPart; ++part) {
@@ -404,63 +405,73 @@ __global__ __launch_bounds__(256, 1) void tile_packed_kernel(PackedArgs g, M40Ep
     }
 }
 
-template <int MTW, int NTW, int KS, int kBufs, int FORM>
+template <int MTW, int NTW, int KS, int kBufs, int FORM, int WM = 2, int WN = 2>
 int launch_tile(hipStream_t stream, const PackedArgs& g, const M40Epilogue<m40_bf16>& e, int batches) {
-    constexpr int lds = 2 * (MTW + NTW) * KS * 1024 * kBufs;
+    constexpr int lds = (WM * MTW + WN * NTW) * KS * 1024 * kBufs;
     static_assert(lds <= 160 * 1024);
-    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(tile_packed_kernel<MTW, NTW, KS, kBufs, FORM>),
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(tile_packed_kernel<MTW, NTW, WM, WN, KS, kBufs, FORM>),
                                                        hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     if (attr != hipSuccess) return -2;
     constexpr bool kJobs = FORM == kSlots;        // g.rows: the most jobs there can be
-    const long long tiles_m = kJobs ? g.rows : (g.rows + 32 * MTW - 1) / (32 * MTW), tiles = tiles_m * ((g.n_tiles + 2 * NTW - 1) / (2 * NTW));
+    const long long tiles_m = kJobs ? g.rows : (g.rows + 16 * WM * MTW - 1) / (16 * WM * MTW), tiles = tiles_m * ((g.n_tiles + WN * NTW - 1) / (WN * NTW));
     // blocks of 5 to 7 rows of tiles measure alike, larger and smaller ones up to a tenth slower (4096 rows, K 2048, N 11264, 128 x 128 tiles, blocks of
     // 4 / 6 / 8 / 16 / 32: 188 / 178 / 185 / 187 / 214 us); few rows are one block
     const int band = kJobs ? 4 : tiles_m <= 9 ? (int)tiles_m : 6;
-    tile_packed_kernel<MTW, NTW, KS, kBufs, FORM><<<dim3((unsigned)tiles, 1, (unsigned)batches), 256, lds, stream>>>(g, e, band);
+    tile_packed_kernel<MTW, NTW, WM, WN, KS, kBufs, FORM><<<dim3((unsigned)tiles, 1, (unsigned)batches), 64 * WM * WN, lds, stream>>>(g, e, band);
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }
-// Which tile: sums are the same whichever it is.  A launch of t workgroups on c CUs takes, per k tile, about max(least, start + load * t / c): one
-// workgroup alone waits for the round trips of a stage, the second on its CU fills those waits.  Measured with weights that no cache holds, bf16, K 2048 (128 x 256 / 128 x 128 / 64 x 128 / 64 x 64, us):
-//   N 2048:  77 rows 31 / 17.3 / 12.0 / 8.3, 300 rows 31 / 17.7 / 12.0 / 9.2, 700 rows 31 / 18.2 / 13.5 / 15.0, 4096 rows 39.7 / 38.5 / - / -
-//   N 11264: 77 rows 36 / 24 / 17.7 / 18.2, 300 rows 35 / 30 / 29 / 33, 1300 rows 73 / 71 / 82 / 95, 2600 rows 139 / 125 / - / -, 4096 rows 212 / 178 / - / -
-//   N 2048, K 5632: 77 rows 77 / 51 / 36 / 21, 700 rows 75 / 51 / 38 / 41, 4096 rows 85 / 91 / - / -
-// (4096 rows before, with the first tile alone on its CU and addresses and buffers worked out at run time: 230 us at N 11264, 121 at K 5632.)
-constexpr struct { int rows, cols; float least, start, load; } kTileShapes[4] = {
-    {128, 256, 0.48f, 0.50f, 0.0f}, {128, 128, 0.28f, 0.13f, 0.245f}, {64, 128, 0.20f, 0.10f, 0.165f}, {64, 64, 0.13f, 0.10f, 0.10f}};
+// Which tile: sums are the same whichever it is.  Of the three small ones a launch of t workgroups on c CUs takes, per k tile, about max(least, start + load * t / c): one workgroup
+// alone waits for the round trips of a stage, the second on its CU fills those waits.  Measured with weights that no cache holds, bf16, K 2048 (128 x 128 / 64 x 128 / 64 x 64, us):
+//   N 2048:  77 rows 17.3 / 12.0 / 8.3, 300 rows 17.7 / 12.0 / 9.2, 700 rows 18.2 / 13.5 / 15.0, 4096 rows 38.5 / - / -
+//   N 11264: 77 rows 24 / 17.7 / 18.2, 300 rows 30 / 29 / 33, 1300 rows 71 / 82 / 95, 4096 rows 178 / - / -
+//   N 2048, K 5632: 77 rows 51 / 36 / 21, 700 rows 51 / 38 / 41, 4096 rows 91 / - / -
+constexpr struct { int rows, cols; float least, start, load; } kTileShapes[3] = {{128, 128, 0.28f, 0.13f, 0.245f}, {64, 128, 0.20f, 0.10f, 0.165f}, {64, 64, 0.13f, 0.10f, 0.10f}};
+// The two large ones are eight waves alone on their CU, and what counts is rounds of the CUs: a k tile of one takes `start` us, a round `fixed` besides, and a round that not all CUs
+// have `least` of a full one and more the fuller it is.  Two waves a SIMD fill each other's waits, and of the larger one an operand byte from L2 serves 128 products instead of 64
+// (1240 TFLOP/s with every CU busy, more than a large product of the library's).  us, 256 x 256 / 128 x 256 / 128 x 128 (in brackets: four waves to a tile of 128 x 256, as before):
+//   4096 rows, K 2048: N 2048 53 / 36 / 39, N 12048 184 / 199 / 206, N 12624 217 / 220 / 221; K 7680, N 2048: 148 / 108 [114] / -; K 4096: N 4096 111 / 121 / 132, N 11008 292 / 322 / 338
+//   2048 rows, N 11264, K 2048: 113 / 105 / 108; N 11008, K 4096: 188 / 175 / 186; N 2048, K 7680: - / 98 / 71; 1024 rows, N 11264, K 2048: 58 / 70 / 61; N 11008, K 4096: 95 / 116 / 106
+//   3000 rows, K 2048, N 12048: 168 / 164 / 168; 2567 rows, N 4096: 56 / 59 / 51; 1500 rows, N 12624: 105 / 98 / 94; 500 rows: - / 36 / 43; 4096 rows, N 3072, K 768: 34 / - / 30
+constexpr struct { int rows, cols; float start, fixed, least; } kLargeTiles[2] = {{128, 256, 0.45f, 5.0f, 0.9f}, {256, 256, 0.86f, 7.0f, 0.6f}};
+constexpr int kLargeFrom = 48;           // k tiles
 
 template <int FORM>
 int launch_tile_any(hipStream_t stream, const PackedArgs& g, const M40Epilogue<m40_bf16>& e, int batches, int num_cus) {
     if constexpr (FORM == kSlots) {
-        // a job is one row of tiles; long sums take the wider tile, which reads a job's rows half as often (32 experts of 4096 x 5504, 512 rows of four
-        // choices: 302 us against 316; of 2048 x 2816 the narrow one's two workgroups a CU are faster)
-        if (g.k_tiles > 64) return launch_tile<4, 8, 1, 6, FORM>(stream, g, e, batches);
+        // A job is one row of tiles.  Long sums take the wider tile, which reads a job's rows half as often (32 experts of 4096 x 2752, gate and up / down, us: 2048 rows 281 / 152, four
+        // waves to such a tile 289 / 160; 8192 rows 558 / 298, 571 / 309); of 2048 x 1408 the narrow one's two workgroups a CU are faster (10 268 rows 174, wide 189).
+        if (g.k_tiles > 64) return launch_tile<4, 4, 1, 6, FORM, 2, 4>(stream, g, e, batches);
         return launch_tile<4, 4, 1, 5, FORM>(stream, g, e, batches);
     } else {
         const bool pairs = g.k_tiles % 2 == 0 && g.k_total % 2 == 0;          // two k tiles a stage
-        int best = 1;
-        float best_cost = 3.0e38f;
-        long long t[4];
-        for (int c = 0; c < 4; ++c) {
-            t[c] = (long long)((g.rows + kTileShapes[c].rows - 1) / kTileShapes[c].rows) * ((g.n_tiles * 16 + kTileShapes[c].cols - 1) / kTileShapes[c].cols) * batches;
-            // the largest tile pays for long sums, where its tiles fill the CUs just once or their rounds better (below)
-            if ((c == 0 && (g.k_tiles <= 64 || t[0] > num_cus)) || (c == 3 && !pairs)) continue;
+        const auto count = [&](int rows, int cols) { return (long long)((g.rows + rows - 1) / rows) * ((g.n_tiles * 16 + cols - 1) / cols) * batches; };
+        int best = 0;
+        float best_cost = 3.0e38f, best_us = 0.0f;
+        long long t[3];
+        for (int c = 0; c < 3; ++c) {
+            t[c] = count(kTileShapes[c].rows, kTileShapes[c].cols);
+            if (c == 2 && !pairs) continue;
             const float u = (float)t[c] / (float)num_cus, cost = kTileShapes[c].start + kTileShapes[c].load * u;
             const float at_least = cost > kTileShapes[c].least ? cost : kTileShapes[c].least;
-            if (at_least < best_cost) { best_cost = at_least; best = c; }
+            // (what a tile takes besides its k tiles, which counts beside the large ones)
+            if (at_least < best_cost) { best_cost = at_least; best = c; best_us = at_least * (float)g.k_tiles + 1.5f * u * (float)(kTileShapes[c].rows * kTileShapes[c].cols) / 16384.0f; }
         }
-        // long sums over more tiles than CUs: what counts is how many the fullest CU has (K 4096, 128 x 256 / 128 x 128: 512 rows, N 26752 131 / 147 us;
-        // 1500 rows, N 4096 67 / 78, N 6144 116 / 102, N 12800 188 / 174)
-        if (best == 1 && g.k_tiles > 64 && t[1] > num_cus) {
-            const auto most = [&](int c) { return (float)((t[c] + num_cus - 1) / num_cus); };
-            if (kTileShapes[0].start * most(0) < kTileShapes[1].start + kTileShapes[1].load * most(1)) best = 0;
+        int large = -1;
+        for (int c = 0; c < 2 && g.k_tiles >= kLargeFrom; ++c) {
+            const long long n = count(kLargeTiles[c].rows, kLargeTiles[c].cols), full = n / num_cus, rest = n % num_cus;
+            if (2 * n < num_cus || g.lda > 1 << 23) continue;            // (a tile's operand rows lie within 32-bit offsets)
+            const float part = rest ? kLargeTiles[c].least + (1.0f - kLargeTiles[c].least) * (float)rest / (float)num_cus : 0.0f;
+            const float us = kLargeTiles[c].start * (float)g.k_tiles * ((float)full + part) + kLargeTiles[c].fixed * (float)(full + (rest != 0));
+            if (us < best_us) { best_us = us; large = c; }
         }
+        if (large == 0) return launch_tile<4, 4, 1, 6, FORM, 2, 4>(stream, g, e, batches);
+        if (large == 1) return launch_tile<4, 8, 1, 4, FORM, 4, 2>(stream, g, e, batches);
         // alone on its CU a workgroup takes the memory of two for deeper buffers: N 2048, K 5632 at 77 rows 21.2 us (64 x 64) against 24.4, at
         // 1300 rows 43.6 us (128 x 128) against 50.7
         const bool alone = pairs && t[best] <= num_cus;
         switch (best) {
-            case 0: return launch_tile<4, 8, 1, 6, FORM>(stream, g, e, batches);
-            case 1: return alone ? launch_tile<4, 4, 2, 5, FORM>(stream, g, e, batches) : launch_tile<4, 4, 1, 5, FORM>(stream, g, e, batches);
-            case 2: return launch_tile<2, 4, 1, 6, FORM>(stream, g, e, batches);
+            case 0: return alone ? launch_tile<4, 4, 2, 5, FORM>(stream, g, e, batches) : launch_tile<4, 4, 1, 5, FORM>(stream, g, e, batches);
+            case 1: return launch_tile<2, 4, 1, 6, FORM>(stream, g, e, batches);
             default: return alone ? launch_tile<2, 2, 2, 6, FORM>(stream, g, e, batches) : launch_tile<2, 2, 2, 5, FORM>(stream, g, e, batches);
         }
     }

@@ -7,7 +7,7 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 from pimosun_common import c_struct, close_to, from_act, ld, m40, pack_tiles, unpack_tiles, up32  # noqa: E402
-from test_gpu_layer_kernels import ACT, ADD, PROJECT, STORE, STORE_ACT, bf16w, call, gemm, rounded  # noqa: E402
+from test_gpu_layer_kernels import ACT, ADD, KEYS, PROJECT, STORE, STORE_ACT, VALUES, bf16w, call, gemm, rounded  # noqa: E402
 
 Gemm = c_struct("M40llmPackedGemm")
 
@@ -144,3 +144,57 @@ def test_expert_jobs_of_short_and_long_sums(ctx, n, k):
     got = from_act(out.download(np.uint16, (slots, n)), "bfloat16")
     for e, first, m, _ in jobs:
         close_to(got[first:first + m], rounded(A[first:first + m], "bfloat16") @ W[e].T.astype(np.float64), "bfloat16")
+
+
+# 128 x 256 and 256 x 256 tiles of eight waves: one round of the CUs and a part of a next one, rows and columns that fill no tile, an even and an odd number of k tiles, the fewest that
+# they take and one less; every part of the result against a narrower tile's
+@pytest.mark.parametrize("rows,n,k", [(4090, 2040, 1536), (500, 12600, 1568), (4090, 3990, 1536), (4000, 4000, 1568), (700, 16400, 1568), (4090, 2040, 1504), (2050, 11010, 2048)])
+def test_large_tiles_change_no_bit(ctx, rows, n, k):
+    rng = np.random.default_rng(rows + n + k)
+    A, W = rng.standard_normal((rows, k)), bf16w(rng, n, k)
+    old = rng.standard_normal((rows, n)).astype(np.float32)
+    store = lambda first, m: gemm(ctx, "bfloat16", STORE, A[first:first + m], W, out_f32=np.zeros((m, n), np.float32), ld_out=n, cols=n)["out_f32"]
+    whole = store(0, rows)
+    some = np.array([0, 15, 127, 128, 255, 256, rows - 1])
+    close_to(whole[some], rounded(A[some], "bfloat16") @ W.T.astype(np.float64), "float32", factor=2)
+    for first in (0, 120, 256, rows // 2, rows - 77):
+        assert np.array_equal(store(first, 77).view(np.uint32), whole[first:first + 77].view(np.uint32)), first
+    added = gemm(ctx, "bfloat16", ADD, A, W, out_f32=old, ld_out=n, cols=n)["out_f32"]
+    assert np.array_equal(added, old + whole)
+    act = gemm(ctx, "bfloat16", STORE_ACT, A, W, out_act=np.zeros((rows, up32(n)), np.uint16), ld_act=up32(n), cols=n)["out_act"]
+    assert np.array_equal(act[:, :n], ld.f32_to_bf16(whole))
+
+
+@pytest.mark.parametrize("rows,tiles,k", [(4090, 128, 1536), (700, 1026, 1568), (500, 790, 1536)])
+def test_large_tiles_gated_pairs(ctx, rows, tiles, k):
+    """Two plain tiles and pairs of gate and up behind it; rows of the result against a launch of few rows."""
+    rng = np.random.default_rng(tiles)
+    A, W, width = rng.standard_normal((rows, k)), bf16w(rng, tiles * 16, k), up32((tiles - 2) * 8)
+    def project(first, m):
+        out = gemm(ctx, "bfloat16", PROJECT, A[first:first + m], W, out_f32=np.zeros((m, 32), np.float32), ld_out=32, plain_tiles=2, cols=W.shape[0],
+                   out_act=np.zeros((m + 15) // 16 * 16 * width, np.uint16), ld_act=width)
+        return out["out_f32"].view(np.uint32), unpack_tiles(out["out_act"], m, width)[:, :(tiles - 2) * 8]
+    whole = project(0, rows)
+    for first, m in ((0, 65), (112, 70), (240, 77), (rows - 70, 70)):
+        for a, b in zip(project(first, m), whole):
+            assert np.array_equal(a, b[first:first + m]), first
+
+
+@pytest.mark.parametrize("kind", [KEYS, VALUES])
+@pytest.mark.parametrize("tiles", [128, 256])
+def test_large_tiles_over_pages(ctx, kind, tiles):
+    """Scattered pages of 50 k tiles, of which the product takes 48; the results of a page are one piece."""
+    rng, pages = np.random.default_rng(tiles), 63
+    cache, W = rng.standard_normal((pages + 2, 64, 1600)), bf16w(rng, tiles * 16, 1536)
+    order = rng.permutation(pages + 2)[:pages].astype(np.uint32)
+    dc, dw = ctx.to_device(np.concatenate([pack_tiles(ld.f32_to_bf16(p)).reshape(-1) for p in cache])), ctx.to_device(pack_tiles(ld.f32_to_bf16(W)))
+    def product(first, n):
+        out, dl = ctx.to_device(np.zeros((n, 64 * tiles * 16), np.uint16)), ctx.to_device(order[first:first + n])
+        g = Gemm(act_dtype=ACT["bfloat16"], epilogue=kind, a=dc.ptr, w=dw.ptr, n_tiles=tiles, k_tiles=48, rows=64 * n, batches=1, out_act=out.ptr, pages=dl.ptr, page_k_tiles=50)
+        call(ctx, "m40llm_ext_packed_gemm_async", C.byref(g), 1)
+        return out.download(np.uint16, (n, 64 * tiles * 16))
+    whole = product(0, pages)
+    for first, n in ((0, 1), (3, 3), (30, 5), (61, 2)):
+        assert np.array_equal(product(first, n), whole[first:first + n])
+    want = rounded(cache[order[5]][:, :1536], "bfloat16") @ W.T.astype(np.float64)
+    close_to(np.sort(from_act(whole[5], "bfloat16")), np.sort(want.reshape(-1)), "bfloat16", factor=2)
