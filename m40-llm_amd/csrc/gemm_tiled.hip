@@ -23,7 +23,6 @@ namespace {
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 constexpr int kBK = 32;
-constexpr int kThreads = 256;
 constexpr int kMaxMats = 3;
 
 // Up to three weight matrices that share the activations (Q/K/V, gate/up): their column tiles are laid side by side.
@@ -277,7 +276,7 @@ __global__ __launch_bounds__(256) void pack_hilo_planes_kernel(PackSource src_ar
     }
 }
 
-// ---- tiles of 32 MT x 32 NT per workgroup of four waves (2 x 2, wave tile 16 MT x 16 NT) -----------------------------------
+// ---- tiles of 16 WM MT x 16 WN NT per workgroup of WM x WN waves (wave tile 16 MT x 16 NT) ---------------------------------
 //
 // Measured on a 128 x 128 kernel that staged through registers with parts of it switched off (M 4096, N 2048, K 2048): arithmetic alone
 // 46 us, loads + LDS traffic + barriers alone 45 us, everything 87 us -- the two did not overlap.  A wave issues in order, and a
@@ -295,8 +294,10 @@ __global__ __launch_bounds__(256) void pack_hilo_planes_kernel(PackSource src_ar
 //    buffers of those, asked for in every second step).  With 16 rows of 64 bytes an instruction, half lines of both, the launches below took, on
 //    one card, 378 us (N 11264), 175 (K 5632) and 112 (N 2560); with both as they are 351, 162 and 105 (whole lines of A alone: 1 to 2 % more than
 //    that);
-//  * in the 128 x 256 tile the wave tile is 64 x 128: per matrix instruction two thirds of the fragment bytes of a 64 x 64 tile (the
-//    activation rows, read twice -- high and low part -- are the short side).
+//  * a workgroup is eight waves, two to a SIMD, which fill each other's waits (behind the barrier, between fragments and the first products).  With four, wave tiles twice as large
+//    read a quarter to two fifths fewer fragment bytes a product and were slower all the same (us, four / eight waves): 128 x 256 tiles, K 2048, M 4096, N 11264 341 / 331, M 522
+//    58.0 / 55.5; 128 x 128, M 2000, N 2048 66.6 / 62.4 (median of K 2048 and 5632), M 1000, N 2560 34.7 / 33.0; 64 x 128, M 522, N 2048 in parts of K 5632 22.9 / 20.7, N 2560
+//    22.1 / 20.1; 64 x 64, M 60, N 2048, K 11008 in parts 16.4 / 16.0.
 // M 4096, N 2048, K 2048: 79 (128 x 128, through registers) -> 63 us; N 11264: 479 -> 338 us; K 5632: 232 -> 155 us (before the whole lines).  Under this load the part lowers
 // its clock (1.4-1.9 GHz measured inside the kernel, against 2.0-2.2 GHz in short or memory-bound launches), and a form
 // with fewer issue cycles (32 x 32 x 16 instructions: 1370 instead of 1500 cycles per step) ran at a lower clock
@@ -340,13 +341,13 @@ __device__ __forceinline__ void tiled_unrolled(std::integer_sequence<int, I...>,
 // KS: k steps of 32 a stage (what is loaded together, between two barriers); kBufs: LDS buffers of a stage each (one
 // workgroup is resident per CU).  Two steps a stage read whole 128-byte lines of a column: with weights that no cache holds 64 x 64 tiles of N 2048,
 // K 2048 take 15.5 us that way and 21.3 us in stages of one step, 64 x 128 tiles 21.0 and 24.6 us (60 rows).
-template <int MT, int NT, int KS, int kBufs, int kBBufs, bool FINE>
-__global__ __launch_bounds__(kThreads, 1) void gemm_tiled_kernel(const _Float16* __restrict__ A_hi, const _Float16* __restrict__ A_lo,
+template <int MT, int NT, int WM, int WN, int KS, int kBufs, int kBBufs, bool FINE>
+__global__ __launch_bounds__(64 * WM * WN, 1) void gemm_tiled_kernel(const _Float16* __restrict__ A_hi, const _Float16* __restrict__ A_lo,
                                                                       const float* __restrict__ row_scale, TiledMats mats, int M, int K,
                                                                       int k_splits, int band) {
     typedef __attribute__((address_space(3))) void* lds_dst_t;
     typedef const __attribute__((address_space(1))) void* global_src_t;
-    constexpr int BM = 32 * MT, BN = 32 * NT;
+    constexpr int kThreads = 64 * WM * WN, BM = 16 * WM * MT, BN = 16 * WN * NT;
     constexpr int kRow = 64 * KS, kLoadRows = kThreads / (4 * KS);           // bytes of a row of A in a stage; rows the workgroup loads at a time
     constexpr int kRowB = 128, kLoadRowsB = kThreads / 8;                    // of B, always two steps
     constexpr int kPlane = BM * kRow, kBuf = 2 * kPlane, kBufB = BN * kRowB, kB0 = kBufs * kBuf;      // bytes: a plane of a stage, both, B of two steps; where B starts
@@ -357,7 +358,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_tiled_kernel(const _Float16*
     at.m0 = __builtin_amdgcn_readfirstlane(at.m0); at.n0 = __builtin_amdgcn_readfirstlane(at.n0);      // the same in every lane: divisions leave them in vector registers
     at.mat = __builtin_amdgcn_readfirstlane(at.mat); at.split = __builtin_amdgcn_readfirstlane(at.split);
     const int N = mats.N[at.mat], m0 = at.m0, n0 = at.n0;
-    // in a pair a wave's eight rows of a load are one matrix's
+    // in a pair a wave's eight rows of a load are one matrix's (the next ones an even number of sixteens further)
     const uint16_t* __restrict__ B = mats.B[mats.pair ? (wave >> 1) & 1 : at.mat];
     // loader: thread -> row lrow (+ kLoadRows i) of a plane and a 16-byte place in that row's bytes, which holds the row's chunk of that number
     // xor-ed with bits of the row: the fragment reads of rows that share banks fall into different ones
@@ -388,8 +389,8 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_tiled_kernel(const _Float16*
         uint8_t* dst = tile_lds + buf * kBuf + wave * 1024;
 #pragma unroll
         for (int i = 0; i < AL; ++i) {
-            __builtin_amdgcn_global_load_lds((global_src_t)(hi_base + k + a_off[i]), (lds_dst_t)(dst + i * 4096), 16, 0, 0);
-            __builtin_amdgcn_global_load_lds((global_src_t)(lo_base + k + a_off[i]), (lds_dst_t)(dst + kPlane + i * 4096), 16, 0, 0);
+            __builtin_amdgcn_global_load_lds((global_src_t)(hi_base + k + a_off[i]), (lds_dst_t)(dst + i * (16 * kThreads)), 16, 0, 0);
+            __builtin_amdgcn_global_load_lds((global_src_t)(lo_base + k + a_off[i]), (lds_dst_t)(dst + kPlane + i * (16 * kThreads)), 16, 0, 0);
         }
     };
     // B of the steps 2 pair and 2 pair + 1 (one stage where a stage is two steps); of an odd number of steps the last one is read twice
@@ -404,9 +405,9 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_tiled_kernel(const _Float16*
         uint8_t* dst = tile_lds + kB0 + buf * kBufB + wave * 1024;
 #pragma unroll
         for (int i = 0; i < BL; ++i)
-            __builtin_amdgcn_global_load_lds((global_src_t)(b_base + k + (KS == 1 ? b_off[i] - back : b_off[i])), (lds_dst_t)(dst + i * 4096), 16, 0, 0);
+            __builtin_amdgcn_global_load_lds((global_src_t)(b_base + k + (KS == 1 ? b_off[i] - back : b_off[i])), (lds_dst_t)(dst + i * (16 * kThreads)), 16, 0, 0);
     };
-    const int wm = wave >> 1, wn = wave & 1, frag_row = lane & 15;
+    const int wm = wave / WN, wn = wave % WN, frag_row = lane & 15;
     float scale[MT];                   // of the rows this lane will store, requested ahead of everything else
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
@@ -433,7 +434,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_tiled_kernel(const _Float16*
         for (int j = 0; j < NT; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
     // Per accumulator step by step, high part then low part: the two large tiles give the same bits.  (FINE: the low parts' sums apart.)  The weights are the instruction's
     // first operand, so a lane's four sums are four neighbouring columns of one row and a store is 16 bytes.
-    constexpr bool kBlocked = MT * NT <= 8;
+    constexpr bool kBlocked = BM * BN <= 64 * 128;
     static_assert(kBlocked || !FINE);
     floatx4 low[FINE ? MT : 1][FINE ? NT : 1];
     if (FINE) {
@@ -643,11 +644,11 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_tiled_kernel(const _Float16*
     else store_tile(std::false_type{});
 }
 
-template <int MT, int NT, int KS, int kBufs, int kBBufs = kBufs, bool FINE = false>
+template <int MT, int NT, int WM, int WN, int KS, int kBufs, int kBBufs, bool FINE = false>
 int launch_tiles(hipStream_t stream, const _Float16* hi, const _Float16* lo, const float* row_scale, TiledMats mats, int M, int K, int k_splits) {
-    constexpr int BM = 32 * MT, BN = 32 * NT, bytes = kBufs * 2 * BM * 64 * KS + kBBufs * BN * 128;
+    constexpr int BM = 16 * WM * MT, BN = 16 * WN * NT, bytes = kBufs * 2 * BM * 64 * KS + kBBufs * BN * 128;
     static_assert(bytes <= 160 * 1024);
-    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_tiled_kernel<MT, NT, KS, kBufs, kBBufs, FINE>),
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_tiled_kernel<MT, NT, WM, WN, KS, kBufs, kBBufs, FINE>),
                                                        hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
     if (attr != hipSuccess) return -2;
     const int tiles_m = (M + BM - 1) / BM;
@@ -661,7 +662,7 @@ int launch_tiles(hipStream_t stream, const _Float16* hi, const _Float16* lo, con
     // 157 / 165 / 157 / 146 / 140 / 141 / 141; M 2048, N 11264, K 2048 174 / 200 / 175 / 162 / 163 / 159 / 161.  M 522, N 2048, K 5632 on 64 x 128 (9 tile rows), bands of 1 / 3 / 5 /
     // 9: 44.7 / 46.8 / 45.9 / 43.7
     const int band = tiles_m <= 9 ? tiles_m : 6;
-    gemm_tiled_kernel<MT, NT, KS, kBufs, kBBufs, FINE><<<(unsigned)(tiles_m * tiles_n * k_splits), kThreads, bytes, stream>>>(hi, lo, row_scale, mats, M, K, k_splits, band);
+    gemm_tiled_kernel<MT, NT, WM, WN, KS, kBufs, kBBufs, FINE><<<(unsigned)(tiles_m * tiles_n * k_splits), 64 * WM * WN, bytes, stream>>>(hi, lo, row_scale, mats, M, K, k_splits, band);
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 
@@ -671,12 +672,12 @@ int launch_tiles(hipStream_t stream, const _Float16* hi, const _Float16* lo, con
 // with whole lines, weights that no cache holds, N 2048, K 2048 (128 x 256 / 128 x 128 / 64 x 128 / 64 x 64):
 //   60 rows 40.4 / 25.3 / 21.6 / 16.2 us, 522 rows 44.1 / 27.1 / 18.9 / 23.3, 1030 rows 45.9 / 30.7 / 36.0 / 37.1, 2048 rows 49.5 / 35.5 / 44.4 / 60.3, 4096 rows 62.4 / 86.1 /
 //   96.0 / 118.6
-// Of M 60, 101, 250, 522, 1030, 2048 and 4096 with N 2048, 2560 and 11264 at K 2048 and N 2048 at K 5632 the tile chosen for a whole K is the fastest or within 3 % of it but
-// for M 4096, N 2560 (128 x 256, 96 to 100 us, where 128 x 128 takes 90).
+// (four waves a workgroup).  The constants of 128 x 128 were fitted again for eight, K 2048 (128 x 256 / 128 x 128): N 2560 2000 rows 57.2 / 63.2, 3000 59.4 / 67.4, 4000 103.2 / 90.3; N 11264
+//   1000 rows 110.3 / 101.1, 2000 171.5 / 191.1, 3000 261.6 / 273.4, 4000 324.7 / 340.0; N 22016, 1200 rows 204.3 / 213.7.  Of these the faster one is chosen.
 // Parts of K cost the launch that adds their sums; N 2048, K 5632 at 250 rows: 35.9 us whole, 19.7 us and that launch in parts.
 struct TileChoice { int shape, k_splits; };
 constexpr struct { int bm, bn; float least, start, load; } kShapes[4] = {
-    {128, 256, 0.66f, 0.62f, 0.28f}, {128, 128, 0.44f, 0.38f, 0.20f}, {64, 128, 0.28f, 0.25f, 0.05f}, {64, 64, 0.235f, 0.17f, 0.03f}};
+    {128, 256, 0.66f, 0.62f, 0.28f}, {128, 128, 0.44f, 0.37f, 0.13f}, {64, 128, 0.28f, 0.25f, 0.05f}, {64, 64, 0.235f, 0.17f, 0.03f}};
 // The two large tiles add up all of their part of K in one chain: in small grids they are taken for four parts only (K 2048 is where a chain's error
 // shows: 64 steps and more).  The two small tiles, which add up blocks of k, are for small grids and for one row of tiles; past
 // that the larger ones are faster (above, 1030 rows), and a row's sums do not depend on how many rows come with it.
@@ -844,10 +845,10 @@ int enqueue_tiled(const M40StreamScratch& sc, hipStream_t stream, const TiledCal
     }
     int rc = -2;
     switch (plan.choice.shape) {
-        case 0: rc = launch_tiles<4, 8, 1, 4, 3>(stream, hi, lo, row_scale, launch, M, K, k_splits); break;
-        case 1: rc = launch_tiles<4, 4, 1, 6, 3>(stream, hi, lo, row_scale, launch, M, K, k_splits); break;
-        case 2: rc = M <= 64 ? launch_tiles<2, 4, 2, 5, 5, true>(stream, hi, lo, row_scale, launch, M, K, k_splits) : launch_tiles<2, 4, 2, 5>(stream, hi, lo, row_scale, launch, M, K, k_splits); break;
-        case 3: rc = M <= 64 ? launch_tiles<2, 2, 2, 6, 6, true>(stream, hi, lo, row_scale, launch, M, K, k_splits) : launch_tiles<2, 2, 2, 6>(stream, hi, lo, row_scale, launch, M, K, k_splits); break;
+        case 0: rc = launch_tiles<4, 4, 2, 4, 1, 4, 3>(stream, hi, lo, row_scale, launch, M, K, k_splits); break;
+        case 1: rc = launch_tiles<2, 4, 4, 2, 1, 6, 3>(stream, hi, lo, row_scale, launch, M, K, k_splits); break;
+        case 2: rc = M <= 64 ? launch_tiles<2, 2, 2, 4, 2, 5, 5, true>(stream, hi, lo, row_scale, launch, M, K, k_splits) : launch_tiles<2, 2, 2, 4, 2, 5, 5>(stream, hi, lo, row_scale, launch, M, K, k_splits); break;
+        case 3: rc = M <= 64 ? launch_tiles<1, 2, 4, 2, 2, 6, 6, true>(stream, hi, lo, row_scale, launch, M, K, k_splits) : launch_tiles<1, 2, 4, 2, 2, 6, 6>(stream, hi, lo, row_scale, launch, M, K, k_splits); break;
     }
     if (rc != 0) return rc;
     if (k_splits > 1 && leave) {
