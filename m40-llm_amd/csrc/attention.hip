@@ -236,12 +236,12 @@ __global__ __launch_bounds__(kAttnThreads, 2) void attn_partial_kernel(AttnParam
 }
 
 // Merge chunk partials: grid (q_heads, batch), 256 threads
-template <int HD>
+template <int HD, int PASS>
 __global__ __launch_bounds__(256) void attn_combine_kernel(AttnParams p) {
     __shared__ __attribute__((aligned(16))) float sums[4][HD];
     const uint32_t qh = blockIdx.x, b = blockIdx.y;
     const size_t first = ((size_t)b * p.q_heads + qh) * p.nchunks;
-    M40ChunkMerge<HD> merge;
+    M40ChunkMerge<HD, PASS> merge;
     merge.request(p.ws + first * HD, p.ml() + first, p.nchunks);
     const uint32_t len = p.length(b);
     const uint32_t sid = (p.max_batch != 0 && p.seq_ids_dev) ? p.seq_ids_dev[b] : 0u;
@@ -307,7 +307,12 @@ void launch_g(hipStream_t stream, const AttnParams& p, uint32_t batch, int S) {
 
 template <int HD>
 void launch_combine(hipStream_t stream, const AttnParams& p, uint32_t batch) {
-    attn_combine_kernel<HD><<<dim3(p.q_heads, batch), 256, 0, stream>>>(p);
+    // What is asked for beyond the chunks there can be is asked for in vain, 32 KB a head of 128 columns.  us a step, 64 chunks / as many as there can be: Qwen2.5-3B, 8 rows of up
+    // to 4000 tokens 2147 / 2133, of 600 2061 / 2045, one of 600 1990 / 1978; TinyLlama, 32 of 900 1273 / 1270
+    const dim3 grid(p.q_heads, batch);
+    if (p.nchunks <= 16) attn_combine_kernel<HD, 16><<<grid, 256, 0, stream>>>(p);
+    else if (p.nchunks <= 32) attn_combine_kernel<HD, 32><<<grid, 256, 0, stream>>>(p);
+    else attn_combine_kernel<HD, 64><<<grid, 256, 0, stream>>>(p);
 }
 
 // Chooses rows per lane group (S), q heads per workgroup (G) and the chunking for a span of `span` tokens.

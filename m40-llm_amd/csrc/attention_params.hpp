@@ -37,14 +37,16 @@ __device__ __forceinline__ void m40_attn_store(const AttnParams& p, uint32_t b, 
 // One head's chunk partials (sums [chunks][HD], pairs of maximum and denominator [chunks]) merged by a workgroup of 256: HD / 4 lanes take a chunk's sums, four
 // columns each; the chunks go round the 1024 / HD such groups.
 //
-// Bound by its round trips to memory: everything of the first 64 chunks is asked for at once, before it is known how many there are; partials of chunks past
+// Bound by its round trips to memory: everything of the first PASS chunks is asked for at once, before it is known how many there are; partials of chunks past
 // the row's end are stale values inside the buffer and are left out; an empty chunk (maximum -inf, sums of 0) has no weight.  Every wave forms all weights itself, one
 // lane a chunk, so that the waves meet once, with their sums.  (Folding the chunks one after the other under a running maximum, 256 / HD of them side by side:
 // the two launches of 8 rows of up to 4093 tokens, head size 128, 13.3 us, now 12.6; 32 rows of up to 1021, 64, 11.8 / 11.3; 2 rows of up to 3000 10.3 / 8.9; one of
 // 16000, 125 chunks, 19.6 / 11.8.)
-template <int HD>
+//
+// PASS: how many chunks are asked for at once; 64 go on to the next ones, with fewer there must be no more.
+template <int HD, int PASS>
 struct M40ChunkMerge {
-    static constexpr int kLanes = HD / 4, kGroups = 256 / kLanes, kPass = 64, kEach = kPass / kGroups;
+    static constexpr int kLanes = HD / 4, kGroups = 256 / kLanes, kPass = PASS, kEach = kPass / kGroups;
     const float4* v_at;
     const float2* ml_at;
     uint32_t stored, lane, group;
@@ -67,11 +69,12 @@ struct M40ChunkMerge {
     // element threadIdx.x of the result, in the first HD threads; n <= stored
     __device__ __forceinline__ float finish(uint32_t n, float (*sums)[HD]) {
         float m = lane < n ? ml0.x : -INFINITY;
-        for (uint32_t c = kPass + lane; c < n; c += kPass) m = fmaxf(m, ml_at[c].x);
+        if (kPass == 64)
+            for (uint32_t c = kPass + lane; c < n; c += kPass) m = fmaxf(m, ml_at[c].x);
         m = m40_max64(m);
         float den = 0.0f;
         float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
-        for (uint32_t base = 0; base < n; base += kPass) {
+        for (uint32_t base = 0; base < (kPass == 64 ? n : 1u); base += kPass) {
             const float2 x = base == 0 ? ml0 : ml_at[base + lane < n ? base + lane : 0u];
             if (base != 0) load(base);
             const bool live = base + lane < n && x.x != -INFINITY;

@@ -534,7 +534,7 @@ __global__ __launch_bounds__(256) void bs_combine_kernel(BsMulti multi) {
     if (p.nchunks <= 1) return;      // the attend kernel wrote the output itself
     __shared__ __attribute__((aligned(16))) float sums[4][HD];
     const uint32_t qh = blockIdx.x, n = p.nchunks;
-    M40ChunkMerge<HD> merge;
+    M40ChunkMerge<HD, 64> merge;
     merge.request(p.partial + (size_t)qh * n * HD, reinterpret_cast<const float2*>(p.partial + (size_t)p.q_heads * n * HD) + (size_t)qh * n, n);
     const float y = merge.finish(n, sums);
     if (threadIdx.x < HD) p.Out[(size_t)qh * HD + threadIdx.x] = y;

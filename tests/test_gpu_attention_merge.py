@@ -43,6 +43,13 @@ def test_merge_of_chunks(dev, qh, kvh, hd, lens, hint):
     kv.destroy()
 
 
+# 16, 17, 32 and 33 chunks of 128 tokens: what a merge asks for at once, and one more
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("hint", [2048, 2049, 4096, 4097])
+def test_merge_at_the_edges_of_a_request(dev, hd, hint):
+    test_merge_of_chunks(dev, 4, 2, hd, [hint, 129], hint)
+
+
 # short rows in batches of few and many q heads: one chunk and several, rows of a token, uneven rows
 @pytest.mark.parametrize("qh,kvh,hd,rows,hint", [(32, 4, 64, 15, 128), (32, 4, 64, 16, 128), (32, 4, 64, 63, 256), (32, 4, 64, 64, 256), (32, 4, 64, 15, 512), (32, 4, 64, 16, 512),
                                                  (8, 8, 64, 64, 130), (64, 4, 128, 15, 256), (64, 4, 128, 16, 256), (16, 2, 128, 15, 400), (16, 2, 128, 16, 400), (64, 4, 128, 4, 257)])
