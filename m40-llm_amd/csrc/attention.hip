@@ -62,6 +62,20 @@ constexpr int kAttnThreads = 512;
 constexpr int kWaves = kAttnThreads / 64;
 
 
+// Steps of a chunk are rows' scores that all lanes of a row hold; lane c goes on with step c % P (P: the steps, rounded up to a power of two), so that a lane works out
+// one weight and not all of them, and hands it to the others.  Of eight lanes, step s is in lane s, which quad s / 4 reads itself; in the other quad the mirrored values have it.
+template <int... I, class F>
+__device__ __forceinline__ void attn_unrolled(std::integer_sequence<int, I...>, F&& f) { (f(std::integral_constant<int, I>{}), ...); }
+
+template <int NS>
+__device__ __forceinline__ constexpr int attn_step_mask() { return NS > 4 ? 7 : (NS > 2 ? 3 : NS - 1); }
+template <int S, bool EIGHT>
+__device__ __forceinline__ float attn_from_step(float own, float mirrored) {
+    constexpr int kQuad = (S & 3) * 0x55, kMirror = (3 - (S & 3)) * 0x55, kOther = S & 4 ? 0x5 : 0xa;
+    const int here = __builtin_amdgcn_mov_dpp(__float_as_int(own), kQuad, 0xf, 0xf, true);
+    return __int_as_float(EIGHT ? __builtin_amdgcn_update_dpp(here, __float_as_int(mirrored), kMirror, 0xf, kOther, false) : here);
+}
+
 // HD in {64, 128}; G = q heads per workgroup (<= 4); S = token rows per lane group; PACKED: the result as operands (a launch of one short row has no time to look
 // it up: 4.35 us instead of 4.29).
 //
@@ -69,6 +83,9 @@ constexpr int kWaves = kAttnThreads / 64;
 // recorded chain over caches that no cache holds, before / with the kv heads in turn / columns halved in the join, lane groups joined once, clamped loads without a branch /
 // and as many steps as there are: 64 tokens 3.73 / 3.73 / 3.9 / 2.55; 128 4.22 / 3.73 / 3.9 / 2.73; 256 4.53 / 3.89 / 3.9 / 3.11; 512 5.23 / 4.97 / 4.49 / 4.50.
 // 16 q heads to 2 of 128, 256 tokens 5.05 -> 4.56; 32 to 8 5.11 -> 4.53.
+// With a weight worked out by one lane a row instead of by all, and six and three steps beside eight, four, two and one, us a step of 8 tokens, before / now: TinyLlama, one row of 310
+// 822 / 812, of 490 836 / 826, four of 310 835 / 823, eight 879 / 844; Qwen2.5-3B, one row of 200 1854 / 1836.  (All requests ahead of the first product, with scalar addresses and a third
+// fewer instructions, give half of that back: 846 with one row of Qwen, 855 with eight of TinyLlama; K's come later behind V's.)
 template <int HD, int G, int S, bool PACKED>
 __global__ __launch_bounds__(kAttnThreads, 2) void attn_partial_kernel(AttnParams p) {
     constexpr int LPT = HD / 8;      // lanes per token row
@@ -103,17 +120,18 @@ __global__ __launch_bounds__(kAttnThreads, 2) void attn_partial_kernel(AttnParam
     const float inv_sqrt = HD == 64 ? 0.125f : 0.08838834764831845f;
 
     float mh[G], lsum[G], acc[G][8];
-    // One pass over the chunk's rows, with half, a quarter or one of its steps where they fill no more: a recorded step is sized for more tokens than its row has by
+    // One pass over the chunk's rows, with as many steps as they fill, five and seven rounded up: a recorded step is sized for more tokens than its row has by
     // now, and arithmetic on rows that are not there took 1.1 us of 3.7.  A test at each step instead keeps the steps of a full chunk from overlapping (5.2 -> 5.5).
-    const auto pass = [&](auto n_steps) {
+    const auto pass = [&](auto n_steps) __attribute__((always_inline)) {
         constexpr int NS = decltype(n_steps)::value;
+        constexpr int kSure = NS == 8 ? 6 : (NS == 6 ? 4 : NS - 1);      // of fewer steps' rows this pass is not taken
         // every load of this lane, issued before anything waits on memory
         uint4 kw[NS], vw[NS];
         bool valid[NS];
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
             const uint32_t t = cbeg + (uint32_t)((s * kWaves + wave) * TPW + tg);
-            valid[s] = t < cend;
+            valid[s] = s < kSure || t < cend;
             const size_t at = (size_t)(valid[s] ? t : cend - 1u) * row_stride;
             kw[s] = *reinterpret_cast<const uint4*>(Kb + at);
             vw[s] = *reinterpret_cast<const uint4*>(Vb + at);
@@ -130,27 +148,26 @@ __global__ __launch_bounds__(kAttnThreads, 2) void attn_partial_kernel(AttnParam
         }
 
         // ---- scores (every lane of a row group ends up with the row's score) -----------------------
-        float sc[NS][G];
-        float lmax[G];
+        const int own_step = c & attn_step_mask<NS>();
+        const bool own_valid = cbeg + (uint32_t)((own_step * kWaves + wave) * TPW + tg) < cend && own_step < NS;
+        float own[G], mirrored[G];
 #pragma unroll
-        for (int h = 0; h < G; ++h) lmax[h] = -INFINITY;
+        for (int h = 0; h < G; ++h) {
+            float x = 0.0f;
 #pragma unroll
-        for (int s = 0; s < NS; ++s) {
-            float kf[8];
-            m40_unpack8(kw[s], kf);
-#pragma unroll
-            for (int h = 0; h < G; ++h) {
-                float d = 0.0f;
+            for (int s = 0; s < NS; ++s) {
+                float kf[8], d = 0.0f;
+                m40_unpack8(kw[s], kf);
 #pragma unroll
                 for (int j = 0; j < 8; ++j) d = fmaf(q[h][j], kf[j], d);
                 d = LPT == 8 ? m40_sum8(d) : m40_sum16(d);
-                sc[s][h] = valid[s] ? d * inv_sqrt : -INFINITY;
-                lmax[h] = fmaxf(lmax[h], sc[s][h]);
+                x = s == 0 || own_step == s ? d : x;
             }
+            own[h] = own_valid ? x * inv_sqrt : -INFINITY;
         }
 #pragma unroll
         for (int h = 0; h < G; ++h) {
-            const float m = m40_max_lanes_from<LPT>(lmax[h]);
+            const float m = m40_max64(own[h]);
             if (lane == 0) wmax[wave][h] = m;
         }
         __syncthreads();
@@ -168,26 +185,35 @@ __global__ __launch_bounds__(kAttnThreads, 2) void attn_partial_kernel(AttnParam
             lsum[h] = 0.0f;
 #pragma unroll
             for (int j = 0; j < 8; ++j) acc[h][j] = 0.0f;
+            own[h] = own_valid ? expf(own[h] - mh[h]) : 0.0f;
+            mirrored[h] = m40_dpp_f<M40_DPP_HALF_MIRROR>(own[h]);
         }
-#pragma unroll
-        for (int s = 0; s < NS; ++s) {
+        attn_unrolled(std::make_integer_sequence<int, NS>(), [&](auto s_c) __attribute__((always_inline)) {
+            constexpr int s = decltype(s_c)::value;
             float vf[8];
-            if (!valid[s]) vw[s] = make_uint4(0, 0, 0, 0);      // the last row once more: an infinity there counts once
+            if (s >= kSure) {      // the last row once more: an infinity there counts once
+                const uint32_t keep = valid[s] ? ~0u : 0u;
+                vw[s] = make_uint4(vw[s].x & keep, vw[s].y & keep, vw[s].z & keep, vw[s].w & keep);
+            }
             m40_unpack8(vw[s], vf);
 #pragma unroll
             for (int h = 0; h < G; ++h) {
-                const float e = valid[s] ? expf(sc[s][h] - mh[h]) : 0.0f;
+                const float e = NS == 1 ? own[h] : attn_from_step<s, (NS > 4)>(own[h], mirrored[h]);
                 lsum[h] += e;
 #pragma unroll
                 for (int j = 0; j < 8; ++j) acc[h][j] = fmaf(e, vf[j], acc[h][j]);
             }
-        }
+        });
     };
     const uint32_t steps = (cend - cbeg + kWaves * TPW - 1) / (kWaves * TPW);
-    if (S == 1 || steps > S / 2) pass(std::integral_constant<int, S>());
-    else if (S == 2 || steps > S / 4) pass(std::integral_constant<int, S < 2 ? 1 : S / 2>());
-    else if (S == 8 && steps > 1) pass(std::integral_constant<int, S < 4 ? 1 : S / 4>());
-    else pass(std::integral_constant<int, 1>());
+    const auto at_most = [&](auto n_steps) __attribute__((always_inline)) {
+        constexpr int NS = decltype(n_steps)::value;
+        if (NS > S || steps > NS) return false;
+        pass(std::integral_constant<int, NS <= S ? NS : S>());
+        return true;
+    };
+    at_most(std::integral_constant<int, 1>()) || at_most(std::integral_constant<int, 2>()) || at_most(std::integral_constant<int, 3>()) || at_most(std::integral_constant<int, 4>()) ||
+        at_most(std::integral_constant<int, 6>()) || at_most(std::integral_constant<int, 8>());
 
     // Join the TPW token rows of the wave (lanes with equal c): each exchange leaves a lane half of the columns to go on with, at the end two of its eight.
 #pragma unroll

@@ -123,3 +123,25 @@ def test_short_row_in_a_launch_for_more(dev, qh, kvh, hd, hint):
         assert np.array_equal(np.isinf(got), np.isinf(want))
         keep = np.isfinite(want)
         assert np.abs(got[keep] - want[keep]).max() <= 4 * (hd + n) * 2.0 ** -24 * np.abs(want[keep]).max() + 1e-6
+
+
+# a row of every number of steps (64 tokens each, 32 with heads of 128), full and with one token more; one and four q heads a workgroup; an infinity in the last
+# token's values, whose rows past the end repeat it
+@pytest.mark.parametrize("qh,kvh,hd", [(4, 2, 64), (4, 2, 128), (32, 8, 64), (32, 8, 128)])
+def test_every_number_of_steps(dev, qh, kvh, hd):
+    step = 64 if hd == 64 else 32
+    lens = [k * step + o for k in range(1, 8) for o in (0, 1)] + [1, 8 * step]
+    test_merge_of_chunks(dev, qh, kvh, hd, lens, 8 * step)
+    rng, rows, hint = np.random.default_rng(hd), len(lens), 8 * step
+    kv = m40.KVCache(dev.ctx, hint, rows, kvh, hd)
+    K, V = (rng.standard_normal((rows, hint, kvh, hd)).astype(np.float16) for _ in range(2))
+    for b, n in enumerate(lens):
+        V[b, n - 1, :, 5] = np.inf
+        dev.fill_dense(kv, b, K[b].view(np.uint16), V[b].view(np.uint16))
+    q = rng.standard_normal((rows, qh * hd)).astype(np.float32)
+    dq, out, ids, dlens = dev.up(q), dev.zeros(q.nbytes), dev.up(np.arange(rows, dtype=np.uint32)), dev.up(np.asarray(lens, dtype=np.uint32))
+    dev.call("m40llm_ext_attention_last_token_f32_gqa_batched_lens_dev_async", kv.h, ids.ptr, dlens.ptr, 0, rows, hint, dq.ptr, qh, out.ptr)
+    dev.sync()
+    got = out.download(np.float32, (rows, qh, hd))
+    assert np.all(got[:, :, 5] == np.inf) and np.all(np.isfinite(np.delete(got, 5, axis=2)))
+    kv.destroy()
