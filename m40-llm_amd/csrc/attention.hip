@@ -84,8 +84,8 @@ __device__ __forceinline__ float attn_from_step(float own, float mirrored) {
 // and as many steps as there are: 64 tokens 3.73 / 3.73 / 3.9 / 2.55; 128 4.22 / 3.73 / 3.9 / 2.73; 256 4.53 / 3.89 / 3.9 / 3.11; 512 5.23 / 4.97 / 4.49 / 4.50.
 // 16 q heads to 2 of 128, 256 tokens 5.05 -> 4.56; 32 to 8 5.11 -> 4.53.
 // With a weight worked out by one lane a row instead of by all, and six and three steps beside eight, four, two and one, us a step of 8 tokens, before / now: TinyLlama, one row of 310
-// 822 / 812, of 490 836 / 826, four of 310 835 / 823, eight 879 / 844; Qwen2.5-3B, one row of 200 1854 / 1836.  (All requests ahead of the first product, with scalar addresses and a third
-// fewer instructions, give half of that back: 846 with one row of Qwen, 855 with eight of TinyLlama; K's come later behind V's.)
+// 822 / 812, of 490 836 / 826, four of 310 835 / 823, eight 879 / 844; Qwen2.5-3B, one row of 200 1854 / 1836.  Then with scalar addresses, a third fewer instructions: eight rows of 490
+// 878 / 863, others as they were (and 855 instead of 840 with eight of 310 where V's requests may go out between K's, or must be out before the first product).
 template <int HD, int G, int S, bool PACKED>
 __global__ __launch_bounds__(kAttnThreads, 2) void attn_partial_kernel(AttnParams p) {
     constexpr int LPT = HD / 8;      // lanes per token row
@@ -113,10 +113,10 @@ __global__ __launch_bounds__(kAttnThreads, 2) void attn_partial_kernel(AttnParam
 
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int c = lane % LPT, tg = lane / LPT;
-    const size_t row_stride = (size_t)p.kv_heads * HD;
-    const size_t base = ((size_t)seq_id * p.max_seq_len) * row_stride + (size_t)kvh * HD + 8 * c;
-    const uint16_t* Kb = p.K + base;
-    const uint16_t* Vb = p.V + base;
+    const uint32_t row_bytes = p.kv_heads * HD * 2u, row = (uint32_t)(wave * TPW + tg);
+    const size_t base = ((size_t)seq_id * p.max_seq_len + cbeg) * row_bytes + (size_t)kvh * (2 * HD);
+    const uint8_t* Kb = reinterpret_cast<const uint8_t*>(p.K) + base;
+    const uint8_t* Vb = reinterpret_cast<const uint8_t*>(p.V) + base;
     const float inv_sqrt = HD == 64 ? 0.125f : 0.08838834764831845f;
 
     float mh[G], lsum[G], acc[G][8];
@@ -125,17 +125,7 @@ __global__ __launch_bounds__(kAttnThreads, 2) void attn_partial_kernel(AttnParam
     const auto pass = [&](auto n_steps) __attribute__((always_inline)) {
         constexpr int NS = decltype(n_steps)::value;
         constexpr int kSure = NS == 8 ? 6 : (NS == 6 ? 4 : NS - 1);      // of fewer steps' rows this pass is not taken
-        // every load of this lane, issued before anything waits on memory
-        uint4 kw[NS], vw[NS];
-        bool valid[NS];
-#pragma unroll
-        for (int s = 0; s < NS; ++s) {
-            const uint32_t t = cbeg + (uint32_t)((s * kWaves + wave) * TPW + tg);
-            valid[s] = s < kSure || t < cend;
-            const size_t at = (size_t)(valid[s] ? t : cend - 1u) * row_stride;
-            kw[s] = *reinterpret_cast<const uint4*>(Kb + at);
-            vw[s] = *reinterpret_cast<const uint4*>(Vb + at);
-        }
+        // every load of this lane, issued before anything waits on memory: scalar addresses that walk the steps, and of a lane 32 bits that do not change
         float q[G][8];
 #pragma unroll
         for (int h = 0; h < G; ++h) {
@@ -146,10 +136,26 @@ __global__ __launch_bounds__(kAttnThreads, 2) void attn_partial_kernel(AttnParam
             q[h][0] = q0.x; q[h][1] = q0.y; q[h][2] = q0.z; q[h][3] = q0.w;
             q[h][4] = q1.x; q[h][5] = q1.y; q[h][6] = q1.z; q[h][7] = q1.w;
         }
+        __builtin_amdgcn_sched_barrier(0);
+        uint4 kw[NS], vw[NS];
+        bool valid[NS];
+        uint32_t off[NS];
+        const size_t step_bytes = (size_t)(kWaves * TPW) * row_bytes;
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+            const uint32_t r = (uint32_t)(s * kWaves * TPW) + row, last = cend - 1u - cbeg;
+            valid[s] = s < kSure || r <= last;
+            off[s] = s < kSure ? row * row_bytes + 16u * c : ((valid[s] ? r : last) - (uint32_t)(kSure * kWaves * TPW)) * row_bytes + 16u * c;
+        }
+#pragma unroll
+        for (int s = 0; s < NS; ++s) kw[s] = *reinterpret_cast<const uint4*>(Kb + (s < kSure ? s : kSure) * step_bytes + off[s]);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int s = 0; s < NS; ++s) vw[s] = *reinterpret_cast<const uint4*>(Vb + (s < kSure ? s : kSure) * step_bytes + off[s]);
 
         // ---- scores (every lane of a row group ends up with the row's score) -----------------------
         const int own_step = c & attn_step_mask<NS>();
-        const bool own_valid = cbeg + (uint32_t)((own_step * kWaves + wave) * TPW + tg) < cend && own_step < NS;
+        const bool own_valid = cbeg + (uint32_t)(own_step * kWaves * TPW) + row < cend && own_step < NS;
         float own[G], mirrored[G];
 #pragma unroll
         for (int h = 0; h < G; ++h) {
