@@ -405,7 +405,7 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void tile_packed_kernel(PackedArgs
     }
 }
 
-template <int MTW, int NTW, int KS, int kBufs, int FORM, int WM = 2, int WN = 2>
+template <int MTW, int NTW, int KS, int kBufs, int FORM, int WM, int WN>
 int launch_tile(hipStream_t stream, const PackedArgs& g, const M40Epilogue<m40_bf16>& e, int batches) {
     constexpr int lds = (WM * MTW + WN * NTW) * KS * 1024 * kBufs;
     static_assert(lds <= 160 * 1024);
@@ -425,6 +425,10 @@ int launch_tile(hipStream_t stream, const PackedArgs& g, const M40Epilogue<m40_b
 //   N 2048:  77 rows 17.3 / 12.0 / 8.3, 300 rows 17.7 / 12.0 / 9.2, 700 rows 18.2 / 13.5 / 15.0, 4096 rows 38.5 / - / -
 //   N 11264: 77 rows 24 / 17.7 / 18.2, 300 rows 30 / 29 / 33, 1300 rows 71 / 82 / 95, 4096 rows 178 / - / -
 //   N 2048, K 5632: 77 rows 51 / 36 / 21, 700 rows 51 / 38 / 41, 4096 rows 91 / - / -
+// (four waves a workgroup).  Tiles of 128 x 128 and 64 x 64 are eight waves now, half the wave tile each: more waves a SIMD that fill each other's waits, for more fragment bytes a product.  us,
+// four / eight: 128 x 128: 1200 rows, K 2048, N 2048 21.9 / 18.7; 2048 rows, K 1408, N 2048 19.7 / 17.2; 4096 rows, K 768, N 3072 29.9 / 28.1; 2567 rows, K 2048, N 4096 50.5 / 49.2;
+// 4096 rows, N 12624 219.3 / 219.9; experts of 2048 x 1408, gate and up / down, 2000 rows 74.5 / 36.1, 73.7 / 34.2, 10 268 rows 168.8 / 85.0, 166.5 / 86.5, of 1024 x 704, 8000 rows 41.6 / 28.1,
+// 38.7 / 26.0.  64 x 64: K 2048, N 2048, 77 rows 9.0 / 8.4, 300 rows 9.6 / 9.1.  (64 x 128 in stages of one k tile has no eight shares of its rows.)
 constexpr struct { int rows, cols; float least, start, load; } kTileShapes[3] = {{128, 128, 0.28f, 0.13f, 0.245f}, {64, 128, 0.20f, 0.10f, 0.165f}, {64, 64, 0.13f, 0.10f, 0.10f}};
 // The two large ones are eight waves alone on their CU, and what counts is rounds of the CUs: a k tile of one takes `start` us, a round `fixed` besides, and a round that not all CUs
 // have `least` of a full one and more the fuller it is.  Two waves a SIMD fill each other's waits, and of the larger one an operand byte from L2 serves 128 products instead of 64
@@ -441,7 +445,7 @@ int launch_tile_any(hipStream_t stream, const PackedArgs& g, const M40Epilogue<m
         // A job is one row of tiles.  Long sums take the wider tile, which reads a job's rows half as often (32 experts of 4096 x 2752, gate and up / down, us: 2048 rows 281 / 152, four
         // waves to such a tile 289 / 160; 8192 rows 558 / 298, 571 / 309); of 2048 x 1408 the narrow one's two workgroups a CU are faster (10 268 rows 174, wide 189).
         if (g.k_tiles > 64) return launch_tile<4, 4, 1, 6, FORM, 2, 4>(stream, g, e, batches);
-        return launch_tile<4, 4, 1, 5, FORM>(stream, g, e, batches);
+        return launch_tile<2, 4, 1, 5, FORM, 4, 2>(stream, g, e, batches);
     } else {
         const bool pairs = g.k_tiles % 2 == 0 && g.k_total % 2 == 0;          // two k tiles a stage
         const auto count = [&](int rows, int cols) { return (long long)((g.rows + rows - 1) / rows) * ((g.n_tiles * 16 + cols - 1) / cols) * batches; };
@@ -470,9 +474,9 @@ int launch_tile_any(hipStream_t stream, const PackedArgs& g, const M40Epilogue<m
         // 1300 rows 43.6 us (128 x 128) against 50.7
         const bool alone = pairs && t[best] <= num_cus;
         switch (best) {
-            case 0: return alone ? launch_tile<4, 4, 2, 5, FORM>(stream, g, e, batches) : launch_tile<4, 4, 1, 5, FORM>(stream, g, e, batches);
-            case 1: return launch_tile<2, 4, 1, 6, FORM>(stream, g, e, batches);
-            default: return alone ? launch_tile<2, 2, 2, 6, FORM>(stream, g, e, batches) : launch_tile<2, 2, 2, 5, FORM>(stream, g, e, batches);
+            case 0: return alone ? launch_tile<2, 4, 2, 5, FORM, 4, 2>(stream, g, e, batches) : launch_tile<2, 4, 1, 5, FORM, 4, 2>(stream, g, e, batches);
+            case 1: return launch_tile<2, 4, 1, 6, FORM, 2, 2>(stream, g, e, batches);
+            default: return alone ? launch_tile<1, 2, 2, 6, FORM, 4, 2>(stream, g, e, batches) : launch_tile<1, 2, 2, 5, FORM, 4, 2>(stream, g, e, batches);
         }
     }
 }
