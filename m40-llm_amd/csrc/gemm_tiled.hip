@@ -2,7 +2,7 @@
 // matrix cores.  Same contract as the reference's gemm_f32xf16_gguf_f32 (cuda/kernels.cu:5037-5052); used when M is
 // beyond what the skinny kernels serve in one pass, where they would stream the weights once per 16 rows.
 //
-// Tiling: a workgroup of 4 waves owns a tile of C and walks K in steps of 32.  The rows of A are split into an f16 high part and an f16
+// Tiling: a workgroup of eight waves owns a tile of C and walks K in steps of 32.  The rows of A are split into an f16 high part and an f16
 // low part under a per-row power-of-two scale (a = scale (hi + lo) up to 2^-22 relative; the scale multiplies the row of C at the end);
 // v_mfma_f32_16x16x32_f16 runs once with the high and once with the low part, so the products carry the f32 activations' precision.
 // Four tile shapes, from 128 x 256 (most products per byte of LDS traffic) to 64 x 64 (most workgroups for few rows), and parts of K where
@@ -672,7 +672,7 @@ int launch_tiles(hipStream_t stream, const _Float16* hi, const _Float16* lo, con
 // with whole lines, weights that no cache holds, N 2048, K 2048 (128 x 256 / 128 x 128 / 64 x 128 / 64 x 64):
 //   60 rows 40.4 / 25.3 / 21.6 / 16.2 us, 522 rows 44.1 / 27.1 / 18.9 / 23.3, 1030 rows 45.9 / 30.7 / 36.0 / 37.1, 2048 rows 49.5 / 35.5 / 44.4 / 60.3, 4096 rows 62.4 / 86.1 /
 //   96.0 / 118.6
-// (four waves a workgroup).  The constants of 128 x 128 were fitted again for eight, K 2048 (128 x 256 / 128 x 128): N 2560 2000 rows 57.2 / 63.2, 3000 59.4 / 67.4, 4000 103.2 / 90.3; N 11264
+// (four waves a workgroup).  The constants of 128 x 128 were fitted again for eight, K 2048 (128 x 256 / 128 x 128): N 2560 2000 rows 57.2 / 63.2, 3000 59.4 / 67.4; N 11264
 //   1000 rows 110.3 / 101.1, 2000 171.5 / 191.1, 3000 261.6 / 273.4, 4000 324.7 / 340.0; N 22016, 1200 rows 204.3 / 213.7.  Of these the faster one is chosen.
 // Parts of K cost the launch that adds their sums; N 2048, K 5632 at 250 rows: 35.9 us whole, 19.7 us and that launch in parts.
 struct TileChoice { int shape, k_splits; };
@@ -697,7 +697,11 @@ TileChoice pick_tile(int M, int n_mats, const int* N, int steps, int num_cus, bo
             if (c < 2 && may_split && s < 4 && per >= 32) continue;
             if (c < 2 && small_grid && !may_split && steps >= 64 && steps % 2 == 0) continue;
             const long long units = (tiles * s + num_cus - 1) / num_cus;
-            const float a = kShapes[c].start * (float)units + kShapes[c].load * (float)(tiles * s) / (float)num_cus;
+            // Thousands of rows run at the part's power, where a tile that reads more bytes a product slows down what comes next: alone, Q/K/V of 4000 rows takes 90 us in 128 x 128
+            // tiles and 103 in 128 x 256, but whole prompts of 3500 and 4096 tokens 17.68 and 20.15 ms with the former, 17.26 and 19.69 with the latter (up to 1500 rows, gate and up in
+            // 128 x 128: 800 tokens 5.54 ms against 5.65, 1000 5.96 / 6.08, 1500 8.10 / 8.18).
+            const float load = c == 1 && M > 2048 ? 0.20f : kShapes[c].load;
+            const float a = kShapes[c].start * (float)units + load * (float)(tiles * s) / (float)num_cus;
             float us = (float)per * (a > kShapes[c].least ? a : kShapes[c].least);
             if (s > 1) us += 6.0f + (float)(s + 1) * out_mb / 5.0f;       // MB over TB/s are us
             if (us < best_us) { best_us = us; best = {c, s}; }
