@@ -698,9 +698,9 @@ TileChoice pick_tile(int M, int n_mats, const int* N, int steps, int num_cus, bo
             if (c < 2 && small_grid && !may_split && steps >= 64 && steps % 2 == 0) continue;
             const long long units = (tiles * s + num_cus - 1) / num_cus;
             // Thousands of rows run at the part's power, where a tile that reads more bytes a product slows down what comes next: alone, Q/K/V of 4000 rows takes 90 us in 128 x 128
-            // tiles and 103 in 128 x 256, but whole prompts of 3500 and 4096 tokens 17.68 and 20.15 ms with the former, 17.26 and 19.69 with the latter (up to 1500 rows, gate and up in
+            // tiles and 103 in 128 x 256, but whole prompts of 3300, 3500 and 4096 tokens 17.14, 17.68 and 20.15 ms with the former, 16.93, 17.26 and 19.69 with the latter (up to 1500 rows, gate and up in
             // 128 x 128: 800 tokens 5.54 ms against 5.65, 1000 5.96 / 6.08, 1500 8.10 / 8.18).
-            const float load = c == 1 && M > 2048 ? 0.20f : kShapes[c].load;
+            const float load = c == 1 && M > 2048 ? 0.22f : kShapes[c].load;
             const float a = kShapes[c].start * (float)units + load * (float)(tiles * s) / (float)num_cus;
             float us = (float)per * (a > kShapes[c].least ? a : kShapes[c].least);
             if (s > 1) us += 6.0f + (float)(s + 1) * out_mb / 5.0f;       // MB over TB/s are us

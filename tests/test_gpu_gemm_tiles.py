@@ -35,6 +35,16 @@ def test_many_rows_tiles_vs_float64(dev, M, N, K):
     assert (err <= bound).all(), (i // N, i % N, float(err.flat[i]), float(bound.flat[i]))
 
 
+# where the tile of thousands of rows changes over: the same bits as the rows of a call that takes 128 x 128 tiles, and as those of one row of tiles more or less
+@pytest.mark.parametrize("M,N,K", [(2048, 2560, 320), (2049, 2560, 320), (3333, 2560, 288), (3500, 2304, 64)])
+def test_rows_of_the_large_tiles_are_the_same(dev, M, N, K):
+    rng = np.random.default_rng(M)
+    A, B = rng.standard_normal((M, K)).astype(np.float32), f16bits(rng.standard_normal((N, K)) * 0.05)
+    got = dev.gemm_gguf(A, B, M, N, K).view(np.uint32)
+    for first, rows in ((0, 1100), (M - 1100, 1100), (0, M - 128), (1, M - 1)):
+        assert np.array_equal(dev.gemm_gguf(np.ascontiguousarray(A[first:first + rows]), B, rows, N, K).view(np.uint32), got[first:first + rows]), (first, rows)
+
+
 @pytest.mark.parametrize("norm_dtype", [0, 1])
 @pytest.mark.parametrize("M,F,K", [(33, 16, 64), (65, 48, 128), (100, 5632, 2048), (129, 1024, 320), (300, 5632, 256), (522, 272, 2048), (1030, 2816, 96), (2049, 1040, 160)])
 def test_gate_up_swiglu_equals_separate_calls(dev, M, F, K, norm_dtype):
