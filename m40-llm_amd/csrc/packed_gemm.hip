@@ -599,7 +599,7 @@ int m40llm_ext_packed_gemm_async(M40llmCudaContext* ctx, const M40llmPackedGemm*
     if (choices) {
         if (!choices->ids || !choices->weight || !choices->place || !choices->jobs) return -1;
         if (p->jobs || p->gather || p->row_scale || p->act_dtype != M40LLM_ACT_BF16 || p->epilogue != M40LLM_PACKED_PROJECT || p->plain_tiles != 0 || p->batches != 1u || p->k_parts > 1u || p->segment_tiles ||
-            m40_route_refused(*choices) || choices->job_rows != 16u || choices->rows * choices->top > 64u || choices->rows > 16u || choices->experts > 64u || !m40_aligned16(choices->jobs) ||
+            m40_route_refused(*choices) || choices->job_rows != 16u || choices->rows * choices->top > 64u || choices->rows > 16u || p->rows < choices->rows || choices->experts > 64u || !m40_aligned16(choices->jobs) ||
             p->w_batch % 8 != 0)
             return -3;
     }

@@ -118,3 +118,6 @@ def test_what_the_launch_has_no_form_for_is_refused(ctx):
     assert product(dict(jobs=p)) == product(dict(gather=p)) == product(dict(row_scale=p)) == product(dict(plain_tiles=2, out_f32=p)) == -3
     assert [product(**dict(dict(route, rows=2), **bad)) for bad in (dict(rows=17), dict(job_rows=32), dict(top=33), dict(experts=65), dict(rows=16, top=5), dict(rows=0))] == [-3] * 6
     assert product(**dict(route, ids=None)) == -1
+    for rows, of_route in ((1, 2), (2, 3), (15, 16)):          # fewer rows than the route has choices of: none past the end of a is read
+        q = Route(**dict(route, rows=of_route))
+        assert ctx.lib.m40llm_ext_packed_gemm_async(ctx.h, C.byref(Gemm(**dict(gemm, rows=rows, route=C.addressof(q)))), 1) == -3
