@@ -698,7 +698,7 @@ typedef struct M40llmPackedGemm {
     uint32_t segment_tiles;       /* column tile t reads columns t / segment_tiles * a_batch on of a (0 = all read the same; else a multiple of 16, one batch) */
     /* not NULL: an M40llmRoute (host memory) whose ids and weight are there and whose place and jobs this launch makes on the way: up to 64 experts, 16 rows (no more than this product's),
      * 64 choices, job_rows 16, bf16.  jobs, gather and row_scale NULL: the rows of a are plain; with the route's slot_weight (not written) a choice's weight multiplies gate and up.
-     * PROJECT without plain tiles */
+     * PROJECT without plain tiles.  A row's ids are different ones below experts + identity: of more than 16 pairs that name one expert only the first 16 are multiplied */
     const void* route;
 } M40llmPackedGemm;
 int m40llm_ext_packed_gemm_async(M40llmCudaContext* ctx, const M40llmPackedGemm* g, uint32_t stream_kind);

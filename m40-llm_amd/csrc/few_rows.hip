@@ -16,6 +16,7 @@ template <int JOBS> struct ChoicesOf { using type = NoChoices; };
 template <> struct ChoicesOf<kFewIds> { using type = M40FewChoices; };
 
 // The list of experts in use from the choices of up to 64 (row, choice) pairs, a lane a pair: what few_lists_kernel makes, for the one expert that is number `job` of those in use.
+// A row's choices are different experts, so that none has more than 16 rows.  Ids are the caller's memory: of some that repeat an expert, pairs past its 16 slots share the last one.
 struct ChosenExpert {
     int jobs, expert, rows;           // experts in use; this one (job < jobs), and how many rows took it
     int pair, row;                    // of the lane's operand row: lane % 16, or its last row
@@ -41,7 +42,7 @@ __device__ __forceinline__ ChosenExpert chosen_expert(const uint32_t* ids, int p
     c.jobs = __popcll(used);
     c.expert = __ffsll(__ballot((used >> lane & 1ull) && bits_below(used) == job)) - 1;
     c.hits = __ballot(real && (int)c.own == c.expert);
-    c.rows = __popcll(c.hits);
+    c.rows = min(__popcll(c.hits), 16);
     // pair of the lane's operand row: pairs that took the expert go to the lanes of their rank, the others to one that is not looked at
     const int at = __builtin_amdgcn_ds_permute(4 * ((c.hits >> lane & 1ull) ? bits_below(c.hits) : 63), lane);
     c.pair = __shfl(at, (lane & 15) < c.rows ? lane & 15 : (c.rows > 0 ? c.rows - 1 : 0), 64);
@@ -50,7 +51,7 @@ __device__ __forceinline__ ChosenExpert chosen_expert(const uint32_t* ids, int p
 }
 // What later launches read of the list: the first expert's job also says how many there are, and where rows go on as they are.
 __device__ __forceinline__ void store_list(const M40FewChoices& l, const ChosenExpert& c, int job, int lane) {
-    if (job < c.jobs && (c.hits >> lane & 1ull)) l.place[lane] = 16u * (uint32_t)job + (uint32_t)bits_below(c.hits);
+    if (job < c.jobs && (c.hits >> lane & 1ull)) l.place[lane] = 16u * (uint32_t)job + (uint32_t)min(bits_below(c.hits), 15);
     if (job == 0 && lane < l.rows * l.top && c.own >= (uint32_t)l.experts) l.place[lane] = M40LLM_PLACE_INPUT;
     if (lane != 0) return;
     if (job < c.jobs) *reinterpret_cast<uint4*>(l.jobs + 4 + 4 * job) = make_uint4((uint32_t)c.expert, 16u * (uint32_t)job, (uint32_t)c.rows, 0u);

@@ -7,8 +7,8 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
-from pimosun_common import c_struct, ld, m40, pack_tiles, up32  # noqa: E402
-from test_gpu_layer_kernels import PROJECT, call  # noqa: E402
+from pimosun_common import c_struct, close_to, from_act, ld, m40, pack_tiles, unpack_tiles, up32  # noqa: E402
+from test_gpu_layer_kernels import PROJECT, bf16w, call, rounded  # noqa: E402
 
 NormAdd, Update, Route, Gemm = (c_struct("M40llm" + n) for n in ("NormAdd", "StreamUpdate", "Route", "PackedGemm"))
 
@@ -121,3 +121,36 @@ def test_what_the_launch_has_no_form_for_is_refused(ctx):
     for rows, of_route in ((1, 2), (2, 3), (15, 16)):          # fewer rows than the route has choices of: none past the end of a is read
         q = Route(**dict(route, rows=of_route))
         assert ctx.lib.m40llm_ext_packed_gemm_async(ctx.h, C.byref(Gemm(**dict(gemm, rows=rows, route=C.addressof(q)))), 1) == -3
+
+
+@pytest.mark.parametrize("rows,top,expert", [(16, 4, 5), (5, 4, 0), (16, 4, None)])
+def test_repeated_ids_stay_in_their_experts_slots(ctx, rows, top, expert):
+    """Ids that a caller wrote: one expert for all pairs (64 and 20), or the same two in every row; the list names slots of the expert's own job alone, and the first 16 pairs'
+    products are those of the rows."""
+    rng, ldh, experts = np.random.default_rng(rows), 2048, 8
+    ids = np.full((rows, top), expert) if expert is not None else np.tile([3, 6, 3, 6], (rows, 1))
+    A, W = rng.standard_normal((rows, ldh)), bf16w(rng, experts * 32, ldh)           # 16 rows of gate, 16 of up an expert
+    x, w = ld.f32_to_bf16(A.astype(np.float32)), pack_tiles(ld.f32_to_bf16(W))
+    slots, n_jobs = ctx.lib.m40llm_ext_expert_slots(rows, experts, top), ctx.lib.m40llm_ext_expert_max_jobs(rows, experts, top, 16)
+    bufs = [ctx.to_device(a) for a in (ids.astype(np.uint32), np.ones((rows, top), np.float32), np.full(rows * top, 9999, np.uint32), np.zeros(4 + 4 * n_jobs, np.uint32), x, w)]
+    dids, weight, place, jobs, dx, dw = bufs
+    act = ctx.to_device(np.full((slots, 32), 0x4242, np.uint16))
+    q = Route(rows=rows, experts=experts, top=top, job_rows=16, ids=dids.ptr, weight=weight.ptr, rows_of=place.ptr, place=place.ptr, jobs=jobs.ptr)
+    g = Gemm(act_dtype=0, epilogue=PROJECT, a=dx.ptr, lda=ldh, w=dw.ptr, n_tiles=2, k_tiles=ldh // 32, rows=rows, batches=1, w_batch=32 * ldh, out_act=act.ptr, ld_act=32, activation=1)
+    g.route = C.addressof(q)
+    call(ctx, "m40llm_ext_packed_gemm_async", C.byref(g), 1)
+    ctx.sync(1)
+    used = sorted(set(ids.ravel().tolist()))
+    want = np.zeros(rows * top, np.uint32)
+    for job, e in enumerate(used):
+        mine = np.flatnonzero(ids.ravel() == e)
+        want[mine] = 16 * job + np.minimum(np.arange(len(mine)), 15)
+    assert np.array_equal(place.download(np.uint32, (rows * top,)), want)
+    j = jobs.download(np.uint32, (4 + 4 * n_jobs,))
+    assert j[0] == len(used) and j[4:4 + 4 * len(used)].reshape(-1, 4).tolist() == [[e, 16 * i, 16, 0] for i, e in enumerate(used)]
+    got = act.download(np.uint16, (slots * 32,))
+    assert np.all(got[512 * len(used):] == 0x4242)
+    y = (rounded(A, "bfloat16") @ W.T.astype(np.float64)).reshape(rows, experts, 2, 16)
+    gate, up = y[:, :, 0], y[:, :, 1]
+    y, first = gate / (1.0 + np.exp(-gate)) * up, [np.flatnonzero(want == s)[0] for s in range(16 * len(used))]
+    close_to(from_act(unpack_tiles(got, 16 * len(used), 32)[:, :16], "bfloat16"), np.stack([y[p // top, ids.ravel()[p]] for p in first]), "bfloat16", factor=2)
