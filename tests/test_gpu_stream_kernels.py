@@ -85,6 +85,31 @@ def test_streams_take_the_output_and_the_next_sublayer_reads_them(ctx, dtype, ro
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("streams,width,weighted", [(1, 40, True), (4, 2048, True), (4, 36, False), (6, 100, True)])
+@pytest.mark.parametrize("top", [1, 3, 4, 5, 6, 7])
+def test_infinite_results_of_experts_stay_infinite(ctx, dtype, streams, width, weighted, top):
+    """Experts' rows are read four at a time, the first of the last four again where fewer are left; an infinity in any of them counts once."""
+    rng, keep, rows = np.random.default_rng(top * width), [], 9
+    X, mix, share = (rng.standard_normal(s).astype(np.float32) for s in ((streams, rows, width), (streams, streams), streams))
+    out = rng.standard_normal((rows * top, (width + 7) // 8 * 8))
+    place, weight = rng.permutation(rows * top).reshape(rows, top), (0.1 + rng.random((rows, top))).astype(np.float32)
+    for r in range(rows):
+        out[place[r, r % top], 3 * r] = np.inf * (-1) ** r
+    y = np.einsum("rj,rjw->rw", weight.astype(np.float64) if weighted else np.ones((rows, top)), rounded(out, dtype)[place][..., :width])
+    dx = ctx.to_device(X)
+    xo = ctx.to_device(np.zeros((rows, width), np.float32))
+    call(ctx, "m40llm_ext_stream_update_async", C.byref(Update(act_dtype=ACT[dtype], rows=rows, width=width, streams=streams, eps=1e-5, mult=0.6, streams_x=dx.ptr, stream_stride=rows * width,
+                                                               mix=dev(ctx, keep, mix), share=dev(ctx, keep, share), expert_out=dev(ctx, keep, as_act(out, dtype)), ld_expert=out.shape[1],
+                                                               place=u32(ctx, keep, place), weight=dev(ctx, keep, weight) if weighted else None, top=top, x_out=xo.ptr)), 1)
+    got, fine = dx.download(np.float32, X.shape), np.isfinite(y)
+    assert (~fine).sum() == rows and not np.isnan(got).any()
+    with np.errstate(invalid="ignore"):
+        want = sd.write_streams(X.astype(np.float64), mix.astype(np.float64), share.astype(np.float64), y, 0.6)
+    assert np.array_equal(got[:, ~fine], want[:, ~fine].astype(np.float32))
+    close_to(got[:, fine], want[:, fine], "float32", factor=2)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("rows", [1, 30, 129])
 def test_projection_with_columns_as_operand(ctx, dtype, rows):
     rng = np.random.default_rng(rows)
