@@ -86,8 +86,11 @@ __device__ __forceinline__ float attn_from_step(float own, float mirrored) {
 // With a weight worked out by one lane a row instead of by all, and six and three steps beside eight, four, two and one, us a step of 8 tokens, before / now: TinyLlama, one row of 310
 // 822 / 812, of 490 836 / 826, four of 310 835 / 823, eight 879 / 844; Qwen2.5-3B, one row of 200 1854 / 1836.  Then with scalar addresses, a third fewer instructions: eight rows of 490
 // 878 / 863, others as they were (and 855 instead of 840 with eight of 310 where V's requests may go out between K's, or must be out before the first product).
-template <int HD, int G, int S, bool PACKED>
+//
+// WIDE: offsets from a step's address in 64 bits, for more kv heads than 32 bits have room for (kMostNarrowHeads).
+template <int HD, int G, int S, bool PACKED, bool WIDE = false>
 __global__ __launch_bounds__(kAttnThreads, 2) void attn_partial_kernel(AttnParams p) {
+    using Offset = std::conditional_t<WIDE, size_t, uint32_t>;
     constexpr int LPT = HD / 8;      // lanes per token row
     constexpr int TPW = 64 / LPT;    // token rows per wave load
     constexpr uint32_t kChunk = kWaves * TPW * S;
@@ -113,7 +116,8 @@ __global__ __launch_bounds__(kAttnThreads, 2) void attn_partial_kernel(AttnParam
 
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int c = lane % LPT, tg = lane / LPT;
-    const uint32_t row_bytes = p.kv_heads * HD * 2u, row = (uint32_t)(wave * TPW + tg);
+    const Offset row_bytes = (Offset)p.kv_heads * (HD * 2u);
+    const uint32_t row = (uint32_t)(wave * TPW + tg);
     const size_t base = ((size_t)seq_id * p.max_seq_len + cbeg) * row_bytes + (size_t)kvh * (2 * HD);
     const uint8_t* Kb = reinterpret_cast<const uint8_t*>(p.K) + base;
     const uint8_t* Vb = reinterpret_cast<const uint8_t*>(p.V) + base;
@@ -125,7 +129,7 @@ __global__ __launch_bounds__(kAttnThreads, 2) void attn_partial_kernel(AttnParam
     const auto pass = [&](auto n_steps) __attribute__((always_inline)) {
         constexpr int NS = decltype(n_steps)::value;
         constexpr int kSure = NS == 8 ? 6 : (NS == 6 ? 4 : NS - 1);      // of fewer steps' rows this pass is not taken
-        // every load of this lane, issued before anything waits on memory: scalar addresses that walk the steps, and of a lane 32 bits that do not change
+        // every load of this lane, issued before anything waits on memory: scalar addresses that walk the steps, and of a lane an offset that does not change
         float q[G][8];
 #pragma unroll
         for (int h = 0; h < G; ++h) {
@@ -139,7 +143,7 @@ __global__ __launch_bounds__(kAttnThreads, 2) void attn_partial_kernel(AttnParam
         __builtin_amdgcn_sched_barrier(0);
         uint4 kw[NS], vw[NS];
         bool valid[NS];
-        uint32_t off[NS];
+        Offset off[NS];
         const size_t step_bytes = (size_t)(kWaves * TPW) * row_bytes;
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
@@ -320,6 +324,9 @@ __global__ __launch_bounds__(64) void attn_generic_kernel(AttnParams p, uint32_t
     static_cast<float*>(p.out)[((size_t)b * p.q_heads + qh) * head_dim + d] = acc / den;
 }
 
+// The last step of a full chunk (six of eight steps have addresses of their own) reads up to 2 * 8 * 512 / HD - 1 rows past its address: 2^14 bytes a kv head
+constexpr uint32_t kMostNarrowHeads = 1u << 18;
+
 template <int HD, int G, int S>
 void launch_partial(hipStream_t stream, const AttnParams& p, uint32_t batch) {
     dim3 grid(p.kv_heads * p.subgroups, p.nchunks, batch);
@@ -410,7 +417,11 @@ int launch_hd(M40llmCudaContext* ctx, hipStream_t stream, float* partial, size_t
     }
     p.ws = partial;
     p.ml_from = (uint32_t)((size_t)batch * p.q_heads * p.nchunks * HD);
-    switch (G) {
+    if (p.kv_heads > kMostNarrowHeads) {
+        const dim3 grid(p.q_heads, p.nchunks, batch);
+        if (p.packed && p.nchunks == 1) attn_partial_kernel<HD, 1, 8, true, true><<<grid, kAttnThreads, 0, stream>>>(p);
+        else attn_partial_kernel<HD, 1, 8, false, true><<<grid, kAttnThreads, 0, stream>>>(p);
+    } else switch (G) {
         case 4: launch_g<HD, 4>(stream, p, batch, S); break;
         case 2: launch_g<HD, 2>(stream, p, batch, S); break;
         default: launch_g<HD, 1>(stream, p, batch, S); break;

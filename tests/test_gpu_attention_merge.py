@@ -145,3 +145,19 @@ def test_every_number_of_steps(dev, qh, kvh, hd):
     got = out.download(np.float32, (rows, qh, hd))
     assert np.all(got[:, :, 5] == np.inf) and np.all(np.isfinite(np.delete(got, 5, axis=2)))
     kv.destroy()
+
+
+# rows of a step that are 2^32 bytes and more from its address (64 rows of 64 columns, 32 of 128), and as many kv heads as have 32-bit offsets
+@pytest.mark.parametrize("kvh,hd,n", [(540_672, 64, 64), (540_672, 64, 70), (541_300, 128, 32), (1 << 18, 64, 70)])
+def test_rows_far_apart(dev, kvh, hd, n):
+    """A key that takes nearly all weight in the last token, none in the others; a value there that says whose head it is."""
+    kv = m40.KVCache(dev.ctx, n, 1, kvh, hd)
+    value = np.repeat((np.arange(kvh) % 7 + 1).astype(np.float32), hd)
+    zero, ones, dvalue, out = dev.zeros(value.nbytes), dev.up(np.ones(kvh * hd, np.float32)), dev.up(value), dev.zeros(value.nbytes)
+    for t in range(n): dev.call("m40llm_kvcache_append_token_f32_async", kv.h, 0, (ones if t == n - 1 else zero).ptr, (dvalue if t == n - 1 else zero).ptr)
+    dev.call("m40llm_attention_last_token_f32_gqa_async", kv.h, 0, ones.ptr, kvh, n, out.ptr)
+    dev.sync()
+    weight = np.exp(np.sqrt(hd)) / (np.exp(np.sqrt(hd)) + n - 1)
+    # scores exact, a weight and a division in f32: a few 2^-24
+    assert np.abs(out.download(np.float32, value.shape) / value - weight).max() <= 2e-6
+    kv.destroy()
