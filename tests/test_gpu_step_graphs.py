@@ -120,3 +120,17 @@ def test_a_recording_leaves_the_contexts_stream_alone(ctx):
     lib.m40llm_destroy_context(rec)
     m40.check(lib.m40llm_ext_copy_words_async(ctx.h, theirs.ptr, src.ptr, 64, 1), "after the recorder is gone")
     ctx.sync(1)
+
+
+@pytest.mark.parametrize("design,vocab", [("gulidra", 1000), ("pimosun", 1001)])
+def test_rows_of_logits_that_the_head_stores_itself_and_one_more(ctx, design, vocab):
+    """Up to four rows of logits are written to the host's memory by the head, five go there by a copy: the same bits, launched and replayed."""
+    models = [layered.LayeredModel.random(ctx, dict(config(design), vocab=vocab), seed=3, std=0.05, max_tokens=2048, max_sequences=5, max_rows=256) for _ in range(3)]
+    models[2].set_mode(0)
+    rng = np.random.default_rng(4)
+    for n in [7] + 9 * [1]:
+        tokens = rng.integers(0, vocab, (5, n))
+        five, four, launched = ([m.step([(s, tokens[s], [n - 1] if s < k else []) for s in range(5)])] for m, k in zip(models, (5, 4, 5)))
+        assert five[0].shape == (5, vocab) and np.isfinite(five[0]).all()
+        assert np.array_equal(five[0][:4].view(np.uint32), four[0].view(np.uint32)) and np.array_equal(five[0].view(np.uint32), launched[0].view(np.uint32)), n
+    assert all(m.step_counts()[0] >= 4 for m in models[:2])
