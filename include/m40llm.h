@@ -28,7 +28,10 @@
  * all of them still links.  They are listed at the end of this header.
  *
  * Entry points that have no counterpart in the reference are prefixed
- * `m40llm_ext_` and say so.
+ * `m40llm_ext_` and say so.  Their structures are read whole, at the size this
+ * header gives them, and members are added at their ends: clear a structure
+ * before filling it (a member that is zero is as good as not there), and build a
+ * program with the header of the library it loads.
  */
 #ifndef M40LLM_H
 #define M40LLM_H
@@ -758,7 +761,8 @@ typedef struct M40llmNormAdd {
     void *h, *h_rows;
     uint32_t ld_h, router_tiles;
     /* route not NULL: an M40llmRoute (host memory) whose ids and weight this launch leaves, from the new h (the logits, their place not asked for, are its product with `router`, packed,
-     * router_tiles column tiles; the list is left to the product, M40llmPackedGemm).  bf16, up to 16 rows and 64 experts, ld_h 2048 to 4096, width a multiple of 8 */
+     * router_tiles column tiles; the list is left to the product, M40llmPackedGemm).  bf16, up to 16 rows and 64 experts, ld_h 2048 to 4096, width a multiple of 8.  The rest of the route is
+     * what m40llm_ext_route_rows_async takes and is checked like there, also what this launch does not touch (rows_of, place, jobs) */
     const void *route, *router;
 } M40llmNormAdd;
 int m40llm_ext_norm_add_rows_async(M40llmCudaContext* ctx, const M40llmNormAdd* n, uint32_t stream_kind);

@@ -502,14 +502,14 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void gemm_tiled_kernel(const _Floa
         if constexpr (sub == 0) issue_a((ph + kBufs - 1) % kBufs, s + kBufs - 1);
         if constexpr (loads_b) issue_b(Flight::pair(ph) % kBBufs, Flight::pair(s));
         compute(f[set]);
-        constexpr int kReads = 2 * MT + NT, kProducts = 2 * MT * NT, kPerRead = NT == 8 ? 2 : 1, kLoads = (sub == 0 ? 2 * AL : 0) + (loads_b ? BL : 0);
+        constexpr int kReads = 2 * MT + NT, kProducts = 2 * MT * NT, kLoads = (sub == 0 ? 2 * AL : 0) + (loads_b ? BL : 0);
 #pragma unroll
         for (int i = 0; i < kReads; ++i) {
-            __builtin_amdgcn_sched_group_barrier(0x008, kPerRead, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
             __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
         }
         if constexpr (kLoads > 0) {
-            constexpr int kPerLoad = (kProducts - kPerRead * kReads) / kLoads > 0 ? (kProducts - kPerRead * kReads) / kLoads : 1;
+            constexpr int kPerLoad = (kProducts - kReads) / kLoads > 0 ? (kProducts - kReads) / kLoads : 1;
 #pragma unroll
             for (int i = 0; i < kLoads; ++i) {
                 __builtin_amdgcn_sched_group_barrier(0x008, kPerLoad, 0);

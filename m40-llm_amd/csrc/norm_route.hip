@@ -36,9 +36,10 @@ __global__ __launch_bounds__(kThreads) void norm_route_kernel(const m40_bf16* we
     __shared__ __align__(16) float sums[kParts][TILES * 16];
     const uint32_t tid = threadIdx.x, lane = tid & 63u, row = blockIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), part = wave - kRowWaves;
-    // The row's waves and the product's go separate ways to two barriers each (left in one way the weights' registers would not fit beside the row's).
+    // The row's waves and the product's go separate ways to as many barriers each, those within the row and one behind it (left in one way the weights' registers would not fit beside
+    // the row's).
     if (part < 0) {
-        Row::make(a, row, tid, scratch, [&](uint32_t g, const m40_float4& lo, const m40_float4& hi) {        // a barrier inside
+        Row::make(a, row, tid, scratch, [&](uint32_t g, const m40_float4& lo, const m40_float4& hi) {        // kM40RowBarriers inside
             m40_store8<m40_bf16>(row_s + g * 8u, lo, hi);
             m40_store_input<m40_bf16>(a, row, g, lo, hi);
         });
@@ -55,8 +56,8 @@ __global__ __launch_bounds__(kThreads) void norm_route_kernel(const m40_bf16* we
             }
         };
         request(part);
-        __syncthreads();
-        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < kM40RowBarriers + 1; ++i) __syncthreads();
         m40_float4 acc[2][TILES];            // k tiles part, part + 16, ... and part + 8, part + 24, ...
 #pragma unroll
         for (int h = 0; h < 2; ++h)

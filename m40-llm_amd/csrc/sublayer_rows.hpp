@@ -6,7 +6,8 @@
 
 constexpr uint32_t kM40RowThreads = 256;
 
-// over 256 threads, whose waves' sums are added in order; once a workgroup (waves with other work meet them at the barrier)
+// Over 256 threads, whose waves' sums are added in order; once a row, which therefore has as many barriers as this has: waves with other work meet a row's at that many (norm_route.hip)
+constexpr int kM40RowBarriers = 1;
 __device__ __forceinline__ float m40_row_sum(float v, uint32_t tid, float* scratch) {
     v = m40_sum64(v);
     if ((tid & 63u) == 0u) scratch[tid >> 6] = v;

@@ -386,7 +386,7 @@ private:
 struct ExpertShared { Scratch logits, ids, weight, rows_of, place, jobs, rows, act, out, slot_weight; };
 
 // Launches: product (router logits) | choice and sorted list (two launches above 64 rows) | (many rows: rows in list order) | gate and up per
-// expert | down per expert
+// expert | down per expert.  Where beside_norm says so: the router's product and the choice are part of the launch before (routing), the list of gate and up | down per expert
 class ExpertFeedForward : public FeedForward {
 public:
     ExpertFeedForward(LayerRuntime& rt, std::shared_ptr<ExpertShared> shared, TensorSource& t, const std::string& layer, const ExpertMlpSpec& m)

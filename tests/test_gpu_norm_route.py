@@ -61,7 +61,7 @@ def run(ctx, fused, rows, width, streams, experts, identity, top, groups, sigmoi
     sub.update(h=out["h"].ptr, h_rows=out["h_rows"].ptr)
     name, struct = ("m40llm_ext_stream_update_async", Update) if streams else ("m40llm_ext_norm_add_rows_async", NormAdd)
     got = []
-    for _ in range(times):       # the streams go on from time to time; the rows' count is to be zero again
+    for _ in range(times):       # the rows and streams go on from time to time, over the list of the time before
         if fused:
             call(ctx, name, C.byref(struct(**sub, route=C.addressof(q), router=router.ptr, router_tiles=tiles)), 1)
         else:
