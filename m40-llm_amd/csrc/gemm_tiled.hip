@@ -668,12 +668,13 @@ int launch_tiles(hipStream_t stream, const _Float16* hi, const _Float16* lo, con
 
 // Which tile, and into how many parts to cut K.  A launch of t workgroups on c CUs takes, per step of 32 k, about
 // max(least, start * ceil(t / c) + load * t / c): a workgroup alone on its CU is bound by the round trips of a step, more of them by the step's
-// products and LDS traffic, and by caches and clock when the other CUs work too.  The constants were fitted to 50 shapes when instructions loaded half lines;
-// with whole lines, weights that no cache holds, N 2048, K 2048 (128 x 256 / 128 x 128 / 64 x 128 / 64 x 64):
-//   60 rows 40.4 / 25.3 / 21.6 / 16.2 us, 522 rows 44.1 / 27.1 / 18.9 / 23.3, 1030 rows 45.9 / 30.7 / 36.0 / 37.1, 2048 rows 49.5 / 35.5 / 44.4 / 60.3, 4096 rows 62.4 / 86.1 /
-//   96.0 / 118.6
-// (four waves a workgroup).  The constants of 128 x 128 were fitted again for eight, K 2048 (128 x 256 / 128 x 128): N 2560 2000 rows 57.2 / 63.2, 3000 59.4 / 67.4; N 11264
-//   1000 rows 110.3 / 101.1, 2000 171.5 / 191.1, 3000 261.6 / 273.4, 4000 324.7 / 340.0; N 22016, 1200 rows 204.3 / 213.7.  Of these the faster one is chosen.
+// products and LDS traffic, and by caches and clock when the other CUs work too.  The constants were fitted to 50 shapes in tiles of four waves, those of 128 x 128 again for eight.  us with
+// eight, the whole of K, weights that no cache holds (128 x 256 / 128 x 128 / 64 x 128 / 64 x 64, in brackets what is chosen where K is not cut):
+//   K 2048, N 2048: 60 rows 40.2 / 26.2 / 24.0 / 18.2, 250 rows 41.1 / 25.0 / 17.4 / 13.7, 522 rows 41.8 / 24.7 / [16.8] / 21.4, 1030 rows 44.4 / [28.5] / 32.3 / 35.4, 2048 rows
+//     47.7 / [33.5] / 41.9 / 55.1, 4096 rows [56.3] / 62.9 / 72.5 / 96.6, 4300 rows [92.3] / 82.6 / 90 / 108;  K 5632: 4096 rows [142] / 161 / 186 / 276, 4300 rows [237] / 212 / 226 / 285
+//   N 2560: 522 rows 42.0 / 25.9 / [17.9] / 24.4, 2000 rows [49.0] / 54.2 / 51.7 / 59.7, 3000 rows [54.6] / 62.1 / 80 / 103, 3500 rows [93.1] / 84.5 / 90 / 109, 4096 rows [95.4] / 86.2 / 92 / 120
+//   N 11264: 522 rows [53.2] / 59.9 / 66.2 / 85.9, 1000 rows 101.5 / [95.4] / 117 / 150, 1500 rows 146.7 / [145.1] / 163 / 219, 2000 rows [165] / 178 / 231 / 299, 3000 rows [283] / 290 / 358 / 451,
+//     4096 rows [352] / 400 / 464 / 610
 // Parts of K cost the launch that adds their sums; N 2048, K 5632 at 250 rows: 35.9 us whole, 19.7 us and that launch in parts.
 struct TileChoice { int shape, k_splits; };
 constexpr struct { int bm, bn; float least, start, load; } kShapes[4] = {
@@ -697,9 +698,12 @@ TileChoice pick_tile(int M, int n_mats, const int* N, int steps, int num_cus, bo
             if (c < 2 && may_split && s < 4 && per >= 32) continue;
             if (c < 2 && small_grid && !may_split && steps >= 64 && steps % 2 == 0) continue;
             const long long units = (tiles * s + num_cus - 1) / num_cus;
-            // Thousands of rows run at the part's power, where a tile that reads more bytes a product slows down what comes next: alone, Q/K/V of 4000 rows takes 90 us in 128 x 128
-            // tiles and 103 in 128 x 256, but whole prompts of 3300, 3500 and 4096 tokens 17.14, 17.68 and 20.15 ms with the former, 16.93, 17.26 and 19.69 with the latter (up to 1500 rows, gate and up in
-            // 128 x 128: 800 tokens 5.54 ms against 5.65, 1000 5.96 / 6.08, 1500 8.10 / 8.18).
+            // Past 2048 rows 128 x 128 keeps about the price that it had with four waves, which leaves every choice for the two dense models as it was.  Alone it is the faster one where
+            // 128 x 256 has just begun another round (above, 3500, 4096 and 4300 rows).  But thousands of rows run at the part's power, where a tile that reads more bytes a product slows down
+            // what comes next, and how much depends on the card.  Whole prompts, ms, with 128 x 128 there / with 128 x 256: TinyLlama on one card, 3300 tokens 17.14 / 16.93, 3500 17.68 /
+            // 17.26, 4096 20.15 / 19.69; on another 3300 16.24 / 16.43, 3500 17.06 / 17.30, 4096 19.10 / 19.30, 4300 22.66 / 23.12, 4800 25.26 / 25.49, 5500 28.72 / 28.84, 7600 41.39 / 41.25,
+            // Qwen2.5-3B 3300 39.5 / 39.9, 4600 61.2 / 61.9, 5500 72.2 / 71.9, 6700 90.1 / 89.1 (four waves, 128 x 256: TinyLlama 4096 19.96 and 19.54, Qwen2.5-3B 4600 63.3).  From 2049
+            // to 3200 rows both prices choose alike there.  Up to 2048 rows the fitted price: gate and up in 128 x 128 tiles, 800 tokens 5.54 ms against 5.65, 1000 5.96 / 6.08, 1500 8.10 / 8.18.
             const float load = c == 1 && M > 2048 ? 0.22f : kShapes[c].load;
             const float a = kShapes[c].start * (float)units + load * (float)(tiles * s) / (float)num_cus;
             float us = (float)per * (a > kShapes[c].least ? a : kShapes[c].least);

@@ -421,21 +421,30 @@ int launch_tile(hipStream_t stream, const PackedArgs& g, const M40Epilogue<m40_b
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 // Which tile: sums are the same whichever it is.  Of the three small ones a launch of t workgroups on c CUs takes, per k tile, about max(least, start + load * t / c): one workgroup
-// alone waits for the round trips of a stage, the second on its CU fills those waits.  Measured with weights that no cache holds, bf16, K 2048 (128 x 128 / 64 x 128 / 64 x 64, us):
-//   N 2048:  77 rows 17.3 / 12.0 / 8.3, 300 rows 17.7 / 12.0 / 9.2, 700 rows 18.2 / 13.5 / 15.0, 4096 rows 38.5 / - / -
-//   N 11264: 77 rows 24 / 17.7 / 18.2, 300 rows 30 / 29 / 33, 1300 rows 71 / 82 / 95, 4096 rows 178 / - / -
-//   N 2048, K 5632: 77 rows 51 / 36 / 21, 700 rows 51 / 38 / 41, 4096 rows 91 / - / -
-// (four waves a workgroup).  Tiles of 128 x 128 and 64 x 64 are eight waves now, half the wave tile each: more waves a SIMD that fill each other's waits, for more fragment bytes a product.  us,
-// four / eight: 128 x 128: 1200 rows, K 2048, N 2048 21.9 / 18.7; 2048 rows, K 1408, N 2048 19.7 / 17.2; 4096 rows, K 768, N 3072 29.9 / 28.1; 2567 rows, K 2048, N 4096 50.5 / 49.2;
-// 4096 rows, N 12624 219.3 / 219.9; experts of 2048 x 1408, gate and up / down, 2000 rows 74.5 / 36.1, 73.7 / 34.2, 10 268 rows 168.8 / 85.0, 166.5 / 86.5, of 1024 x 704, 8000 rows 41.6 / 28.1,
-// 38.7 / 26.0.  64 x 64: K 2048, N 2048, 77 rows 9.0 / 8.4, 300 rows 9.6 / 9.1.  (64 x 128 in stages of one k tile has no eight shares of its rows.)
+// alone waits for the round trips of a stage, the second on its CU fills those waits.  Tiles of 128 x 128 and 64 x 64 are eight waves, half the wave tile of four: more waves a SIMD that
+// fill each other's waits, for more fragment bytes a product (64 x 128 in stages of one k tile has no eight shares of its rows).  us, four waves / eight: 1200 rows, K 2048, N 2048 22.4 /
+// 18.9; 2048 rows, K 1408, N 2048 20.4 / 17.1; 4096 rows, K 768, N 3072 29.3 / 27.6; 1500 rows, K 4096, N 2048 35.9 / 30.9; 4096 rows, N 12624 217 / 219; 77 rows, K 2048, N 2048 9.2 / 8.5;
+// experts of 2048 x 1408, gate and up / down, 2000 rows 74.5 / 36.1, 73.7 / 34.2, 10 268 rows 168.8 / 85.0, 166.5 / 86.5, of 1024 x 704, 8000 rows 41.6 / 28.1, 38.7 / 26.0.
+// The constants were fitted to four waves.  What they choose now, with the two large tiles below (128 x 128 / 64 x 128 / 64 x 64 / 128 x 256 / 256 x 256, the chosen one in brackets; us,
+// bf16, weights that no cache holds):
+//   K 2048, N 2048:  77 rows 15.7 / 12.7 / [8.5] / 24.7 / 44, 300 rows 16.6 / 13.1 / [9.2] / 25.8 / 46, 700 rows 17.5 / [14.1] / 15.4 / 26.7 / 47, 1200 rows [18.8] / 22.5 / 22.1 / 27.8 / 48,
+//     2048 rows [21.1] / 25.0 / 29.8 / 29.5 / 50, 4096 rows 35.7 / 44.8 / 55.5 / [34.9] / 54;  N 4096: 1500 rows 31.8 / 35.0 / 42.5 / [31.9] / 50, 2567 rows [49.0] / 63 / 73 / 58 / 56
+//   N 11264: 77 rows 22.8 / [18.4] / 18.8 / 31.7 / 48, 300 rows [31.8] / 30.6 / 35.4 / 32.9 / 52, 700 rows [50.9] / 52.9 / 64 / 58 / 55, 1024 rows 60 / 74 / 88 / 69 / [58], 1300 rows 73 / 91 /
+//     109 / [69] / 104, 2048 rows 106 / 130 / 159 / [101] / 112, 2600 rows 137 / 160 / 190 / 127 / [119], 4096 rows 193 / 234 / 284 / 187 / [170]
+//   N 12624: 500 rows 40.7 / 49 / 56 / [36.5] / 54, 1300 rows [84] / 102 / 121 / 90 / 103, 1500 rows [90] / - / - / 97 / 103, 4096 rows [218] / - / - / 213 / 212;  N 12048: 2000 rows 107 / - /
+//     - / [103] / 113, 3000 rows [164] / - / - / 161 / 163
+//   K 5632, N 2048: 77 rows 34.5 / 27.4 / [17.5] / 56 / 99, 700 rows 39.4 / [34.8] / 38.4 / 59 / 103, 1300 rows [41.4] / 52 / 56 / 61 / 104, 4096 rows 90 / 115 / 143 / [82] / 113
+//   4096 rows, K 768, N 3072 [27.7] / 35.7 / 43.4 / 34.4 / 33.0; 2048 rows, K 1408, N 2048 [17.2] / 20.3 / 23.4 / 24.1 / 39.4; K 7680, N 2048 [67] / 87 / 105 / 97 / 146; K 4096, N 4096 69.7 /
+//     88 / 111 / [62.5] / 91; 1200 rows, K 4096, N 11008 130 / 156 / 182 / 116 / [104]
+// Of 80 shapes of 1100 to 2600 rows (N 2048 to 12624, K 2048 to 7680) 128 x 128, the one chosen and the two large ones were timed as well: the chosen one is the fastest or within 3 % of
+// it in 70 and at most 8 % behind in the others (128 x 128 where 128 x 256 is faster: 2200 to 2600 rows, K 5632, N 2048 69 to 75 against 64 to 70; 1250 rows, K 4096, N 4096 62 / 58), and
+// never more than half a per cent slower than what four waves took.
 constexpr struct { int rows, cols; float least, start, load; } kTileShapes[3] = {{128, 128, 0.28f, 0.13f, 0.245f}, {64, 128, 0.20f, 0.10f, 0.165f}, {64, 64, 0.13f, 0.10f, 0.10f}};
 // The two large ones are eight waves alone on their CU, and what counts is rounds of the CUs: a k tile of one takes `start` us, a round `fixed` besides, and a round that not all CUs
 // have `least` of a full one and more the fuller it is.  Two waves a SIMD fill each other's waits, and of the larger one an operand byte from L2 serves 128 products instead of 64
-// (1240 TFLOP/s with every CU busy, more than a large product of the library's).  us, 256 x 256 / 128 x 256 / 128 x 128 (in brackets: four waves to a tile of 128 x 256, as before):
-//   4096 rows, K 2048: N 2048 53 / 36 / 39, N 12048 184 / 199 / 206, N 12624 217 / 220 / 221; K 7680, N 2048: 148 / 108 [114] / -; K 4096: N 4096 111 / 121 / 132, N 11008 292 / 322 / 338
-//   2048 rows, N 11264, K 2048: 113 / 105 / 108; N 11008, K 4096: 188 / 175 / 186; N 2048, K 7680: - / 98 / 71; 1024 rows, N 11264, K 2048: 58 / 70 / 61; N 11008, K 4096: 95 / 116 / 106
-//   3000 rows, K 2048, N 12048: 168 / 164 / 168; 2567 rows, N 4096: 56 / 59 / 51; 1500 rows, N 12624: 105 / 98 / 94; 500 rows: - / 36 / 43; 4096 rows, N 3072, K 768: 34 / - / 30
+// (1240 TFLOP/s with every CU busy, more than a large product of the library's).  us, 256 x 256 / 128 x 256 (in brackets: four waves to a tile of 128 x 256):
+//   4096 rows, K 2048: N 2048 53 / 36, N 12048 184 / 199, N 12624 217 / 220 (a whole prompt with the former in place of 128 x 128 2235, with 128 x 128 2202); K 7680, N 2048: 148 / 108 [114];
+//   K 4096: N 4096 111 / 121, N 11008 292 / 322;  2048 rows, N 11264, K 2048: 113 / 105; N 11008, K 4096: 188 / 175; 1024 rows, N 11008, K 4096: 95 / 116;  3000 rows, K 2048, N 12048 168 / 164
 constexpr struct { int rows, cols; float start, fixed, least; } kLargeTiles[2] = {{128, 256, 0.45f, 5.0f, 0.9f}, {256, 256, 0.86f, 7.0f, 0.6f}};
 constexpr int kLargeFrom = 48;           // k tiles
 
