@@ -181,16 +181,15 @@ __device__ __forceinline__ void m40_stream_update_row(const M40llmStreamUpdate& 
                 for (uint32_t j = 0; j < 4; ++j) {
                     const size_t pick = (size_t)row * a.top + (j0 + j < a.top ? j0 + j : j0);
                     at[j] = a.place[pick];
-                    f[j] = a.weight ? static_cast<const float*>(a.weight)[pick] : 1.0f;
+                    f[j] = j0 + j >= a.top ? 0.0f : a.weight ? static_cast<const float*>(a.weight)[pick] : 1.0f;
                 }
 #pragma unroll
                 for (uint32_t j = 0; j < 4; ++j) m40_load_group<T, VEC>(static_cast<const T*>(a.expert_out) + (size_t)at[j] * a.ld_expert, g * 8u, width, v[j]);
+                // (past top zeros times zero: times a repeated row's infinity it would be a NaN.  Selected and not branched over: three Natatar prompts, four streams, mean of a launch 18.6 us and 19.4)
 #pragma unroll
-                for (uint32_t j = 0; j < 4; ++j) {
-                    if (j0 + j >= a.top) break;          // (the repeated row with a weight of 0 would make a NaN of an infinity)
+                for (uint32_t j = 0; j < 4; ++j)
 #pragma unroll
-                    for (int i = 0; i < 8; ++i) y[i] = fmaf(f[j], v[j][i], y[i]);
-                }
+                    for (int i = 0; i < 8; ++i) y[i] = fmaf(f[j], j == 0 || j0 + j < a.top ? v[j][i] : 0.0f, y[i]);
             }
         } else {
             const float* plane = static_cast<const float*>(a.planes) + (size_t)row * width;
