@@ -45,7 +45,7 @@ public:
     static constexpr uint32_t kStream = LayerRuntime::kStream;
     static constexpr uint32_t kPage = LayerRuntime::kPage;
     static constexpr size_t kMostPinned = 16u << 20;       // bytes of host memory for a step's logits
-    static constexpr uint32_t kDirectRows = 4;             // most rows of logits that the head stores there itself
+    static constexpr uint32_t kDirectRows = 4, kDirectWidth = 2048, kDirectWords = 128u << 10;      // rows of logits that the head stores there itself (run_pass)
 
     LayeredDecoder(M40llmCudaContext* ctx, DecoderSpec spec, TensorSource& tensors, const LayeredOptions& opt)
         : ctx_(ctx), spec_(std::move(spec)), opt_(checked(ctx, opt)), seqs_(round_up(opt.max_tokens, kPage) / kPage, kPage, opt.max_sequences),
@@ -474,11 +474,14 @@ private:
         // The rows of a step of single tokens come through pinned memory: a blocking copy begins when the host has seen the head's end, and takes 16 us a
         // row and 66 us for eight of 32000.  Up to kDirectRows rows the head writes them there itself, while it reads its weights; its stores are 64 bytes a row, which
         // take twice as long as those of a kernel behind it that copies whole kilobytes.  A step, that kernel / the head: one row 267 -> 262 us, three 296 -> 289, four
-        // 310 -> 307, eight 366 and 366.
+        // 310 -> 307, eight 366 and 366 (2048 wide, 32000 words).  From kDirectWidth columns on the head's form of more waves hides the stores whatever the vocabulary: two layers of 2048,
+        // one / four rows of 32000 147.9 / 167.4 -> 145.6 / 166.4, of 128000 219.4 / 313.3 -> 214.4 / 300.5, of 256000 324 / 505 -> 304 / 440.  Narrower heads hide kDirectWords of them: 256
+        // columns, three rows of 32000 105.2 -> 104.8, four 111.8 -> 111.7, one of 128000 113.0 and 113.0, but two 137.9 -> 139.2, four 208.3 -> 212.8; 1536 columns, one of 128000 189.7 ->
+        // 188.8, four 277.4 -> 282.9.
         const auto pinned = [&](uint32_t n) { return !picks && (size_t)n * spec_.vocab * 4 <= logits_host_.bytes(); };
         const auto first_logits = [&] {
             const uint32_t n = (uint32_t)std::min<size_t>(logits_rows_, plan.want.size());
-            const bool direct = pinned(n) && n <= kDirectRows && rt_.bf16();
+            const bool direct = pinned(n) && n <= kDirectRows && (rt_.d_pad >= kDirectWidth || (size_t)n * spec_.vocab <= kDirectWords) && rt_.bf16();
             enqueue_logits(want, n, r.rows, direct ? logits_host_.f32() : nullptr);
             if (pinned(n) && !direct) M40H_TRY(m40llm_ext_copy_words_async(rt_.ctx, logits_host_.f32(), logits_.ptr(), (size_t)n * spec_.vocab, kStream));
         };

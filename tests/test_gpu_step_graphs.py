@@ -122,15 +122,20 @@ def test_a_recording_leaves_the_contexts_stream_alone(ctx):
     ctx.sync(1)
 
 
-@pytest.mark.parametrize("design,vocab", [("gulidra", 1000), ("pimosun", 1001)])
-def test_rows_of_logits_that_the_head_stores_itself_and_one_more(ctx, design, vocab):
-    """Up to four rows of logits are written to the host's memory by the head, five go there by a copy: the same bits, launched and replayed."""
-    models = [layered.LayeredModel.random(ctx, dict(config(design), vocab=vocab), seed=3, std=0.05, max_tokens=2048, max_sequences=5, max_rows=256) for _ in range(3)]
-    models[2].set_mode(0)
+NARROW = bench.pimosun_config(dict(bench.SHAPES["2k"], width=256, heads=2, kv_rank=64, q_rank=64, ff=704, layers=2))
+
+
+@pytest.mark.parametrize("cfg,vocab", [(config("gulidra"), 1000), (config("pimosun"), 1001), (config("pimosun"), 40_000), (NARROW, 30_000), (NARROW, 40_000), (NARROW, 1001)],
+                         ids=["gulidra", "pimosun", "pimosun wide vocabulary", "narrow", "narrow wide vocabulary", "narrow few words"])
+def test_rows_of_logits_that_the_head_stores_itself_and_one_more(ctx, cfg, vocab):
+    """Up to four rows of logits (of narrow models up to 128 k words) are written to the host's memory by the head, more go there by a copy: the same bits, launched and replayed."""
+    models = [layered.LayeredModel.random(ctx, dict(cfg, vocab=vocab), seed=3, std=0.05, max_tokens=2048, max_sequences=5, max_rows=256) for _ in range(4)]
+    models[3].set_mode(0)
     rng = np.random.default_rng(4)
     for n in [7] + 9 * [1]:
         tokens = rng.integers(0, vocab, (5, n))
-        five, four, launched = ([m.step([(s, tokens[s], [n - 1] if s < k else []) for s in range(5)])] for m, k in zip(models, (5, 4, 5)))
-        assert five[0].shape == (5, vocab) and np.isfinite(five[0]).all()
-        assert np.array_equal(five[0][:4].view(np.uint32), four[0].view(np.uint32)) and np.array_equal(five[0].view(np.uint32), launched[0].view(np.uint32)), n
-    assert all(m.step_counts()[0] >= 4 for m in models[:2])
+        five, four, three, launched = (m.step([(s, tokens[s], [n - 1] if s < k else []) for s in range(5)]) for m, k in zip(models, (5, 4, 3, 5)))
+        assert five.shape == (5, vocab) and np.isfinite(five).all()
+        for other in (four, three, launched):
+            assert np.array_equal(five[:len(other)].view(np.uint32), other.view(np.uint32)), (n, len(other))
+    assert all(m.step_counts()[0] >= 4 for m in models[:3])
