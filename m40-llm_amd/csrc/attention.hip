@@ -177,7 +177,7 @@ __global__ __launch_bounds__(kAttnThreads, 2) void attn_partial_kernel(AttnParam
         }
 #pragma unroll
         for (int h = 0; h < G; ++h) {
-            const float m = m40_max64(own[h]);
+            const float m = NS == 1 ? m40_max_lanes_from<LPT>(own[h]) : m40_max64(own[h]);          // (of one step all lanes of a row have the score)
             if (lane == 0) wmax[wave][h] = m;
         }
         __syncthreads();
