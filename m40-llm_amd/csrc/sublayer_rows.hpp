@@ -174,23 +174,27 @@ __device__ __forceinline__ void m40_stream_update_row(const M40llmStreamUpdate& 
 #pragma unroll
         for (int i = 0; i < 8; ++i) y[i] = 0.0f;
         if (a.place) {
-            for (uint32_t j0 = 0; j0 < a.top; j0 += 4u) {                 // places, then rows of four experts at a time
+            // places, then rows of four experts at a time; of the last ones (fewer than four) the first again, of which zeros are taken
+            const auto rows = [&](uint32_t j0, auto all_c) __attribute__((always_inline)) {
+                constexpr bool kAll = decltype(all_c)::value;
                 uint32_t at[4];
                 float f[4], v[4][8];
 #pragma unroll
                 for (uint32_t j = 0; j < 4; ++j) {
-                    const size_t pick = (size_t)row * a.top + (j0 + j < a.top ? j0 + j : j0);
+                    const size_t pick = (size_t)row * a.top + (kAll || j0 + j < a.top ? j0 + j : j0);
                     at[j] = a.place[pick];
-                    f[j] = j0 + j >= a.top ? 0.0f : a.weight ? static_cast<const float*>(a.weight)[pick] : 1.0f;
+                    f[j] = !kAll && j0 + j >= a.top ? 0.0f : a.weight ? static_cast<const float*>(a.weight)[pick] : 1.0f;
                 }
 #pragma unroll
                 for (uint32_t j = 0; j < 4; ++j) m40_load_group<T, VEC>(static_cast<const T*>(a.expert_out) + (size_t)at[j] * a.ld_expert, g * 8u, width, v[j]);
-                // (past top zeros times zero: times a repeated row's infinity it would be a NaN.  Selected and not branched over: three Natatar prompts, four streams, mean of a launch 18.6 us and 19.4)
 #pragma unroll
                 for (uint32_t j = 0; j < 4; ++j)
 #pragma unroll
-                    for (int i = 0; i < 8; ++i) y[i] = fmaf(f[j], j == 0 || j0 + j < a.top ? v[j][i] : 0.0f, y[i]);
-            }
+                    for (int i = 0; i < 8; ++i) y[i] = fmaf(f[j], kAll || j == 0 || j0 + j < a.top ? v[j][i] : 0.0f, y[i]);
+            };
+            uint32_t j0 = 0;
+            for (; j0 + 4u <= a.top; j0 += 4u) rows(j0, std::true_type());
+            if (j0 < a.top) rows(j0, std::false_type());
         } else {
             const float* plane = static_cast<const float*>(a.planes) + (size_t)row * width;
             for (uint32_t p = 0; p < a.n_planes; p += 2u) {
