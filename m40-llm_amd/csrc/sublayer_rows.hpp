@@ -196,13 +196,19 @@ __device__ __forceinline__ void m40_stream_update_row(const M40llmStreamUpdate& 
             if (j0 < a.top) rows(j0, std::false_type());
         } else {
             const float* plane = static_cast<const float*>(a.planes) + (size_t)row * width;
-            for (uint32_t p = 0; p < a.n_planes; p += 2u) {
+            uint32_t p = 0;
+            for (; p + 1u < a.n_planes; p += 2u) {
                 float v[2][8];
-                const bool both = p + 1u < a.n_planes;
                 m40_load_group<float, VEC>(plane + p * (size_t)a.plane_stride, g * 8u, width, v[0]);
-                m40_load_group<float, VEC>(plane + (both ? p + 1u : p) * (size_t)a.plane_stride, g * 8u, width, v[1]);
+                m40_load_group<float, VEC>(plane + (p + 1u) * (size_t)a.plane_stride, g * 8u, width, v[1]);
 #pragma unroll
-                for (int i = 0; i < 8; ++i) y[i] += both ? v[0][i] + v[1][i] : v[0][i];
+                for (int i = 0; i < 8; ++i) y[i] += v[0][i] + v[1][i];
+            }
+            if (p < a.n_planes) {
+                float v[8];
+                m40_load_group<float, VEC>(plane + p * (size_t)a.plane_stride, g * 8u, width, v);
+#pragma unroll
+                for (int i = 0; i < 8; ++i) y[i] += v[i];
             }
         }
     };
