@@ -54,7 +54,7 @@ __device__ __forceinline__ void m40_norm_add_row(const M40llmNormAdd& a, uint32_
     const uint32_t width = a.width, groups = a.ld_h / 8u;
     float* x = static_cast<float*>(a.x) + (size_t)row * width;
     const float* w = static_cast<const float*>(a.w);
-    // Planes two at a time: one by one each waited for the one before (3 rows of 2048 that the launch before wrote, two planes 4.44 -> 4.28 us, three 4.72 -> 4.62).  Experts' rows one by
+    // Planes two at a time: one by one each waited for the one before (a row of 2048, planes that the launch before wrote, with that launch: two 4.23 -> 4.00 us, three 4.52 -> 4.31).  Experts' rows one by
     // one: four at a time they are 0.5 to 3 % slower (four of a row of 2048 4.91 / 5.01).
     auto value = [&](uint32_t g, const float (&old)[8], float (&y)[8]) __attribute__((always_inline)) {
 #pragma unroll
